@@ -1,0 +1,54 @@
+// gemm_impl.hpp — what the prefill GEMMs share (k_gemm.hip, k_gemm_mid.hip): operands, LDS-DMA, the split-K workspace.
+#pragma once
+
+#include "qie_common.hpp"
+#include "../../include/qie/qie_ops.h"
+
+namespace qie {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+struct GemmParams {
+    const uint16_t* A;
+    int64_t lda;
+    const uint16_t* w0;
+    const uint16_t* w1;
+    const uint16_t* w2;
+    const uint16_t* b0;
+    const uint16_t* b1;
+    const uint16_t* b2;
+    int64_t n0, n01;
+    int64_t M, K, N;     // N = output columns
+    int64_t wrows;       // total weight rows addressable (for clamping)
+    uint16_t* C;
+    int64_t ldc;
+    int vec = 0;         // rows of C take 4-element vector stores (set by the kernel's launcher)
+};
+
+__device__ __forceinline__ void glds16(const void* src, void* lds) {
+    __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)(src),
+                                     (__attribute__((address_space(3))) void*)(lds), 16, 0, 0);
+}
+
+// chunk swizzle of 128-B LDS rows: the 16-B chunk c of row r sits at c ^ g8_swz(r)
+__device__ __forceinline__ int g8_swz(int r) { return (r >> 1) & 7; }
+
+typedef unsigned int u32x4_g8 __attribute__((ext_vector_type(4)));
+
+// split-K workspace of one launch (gemm8_kernel has the protocol)
+struct G8Split {
+    int splitk;
+    float* slab;       // [tiles][splitk][256 * 256] fp32
+    unsigned* cnt;     // [tiles], zero at rest
+};
+
+// Slabs of 65,536 floats and zeroed tickets of stream `st`, grown on demand; non-zero: they would have to grow during a
+// graph capture (the caller runs unsplit).
+int g8_workspace(hipStream_t st, int slabs, int tiles, G8Split* out);
+
+// k_gemm_mid.hip: the GEMM of a few dozen to about a thousand rows.  other_us: the expected time of the caller's kernel for
+// this shape; *launched = false: not a shape for this one, or the other is expected to be faster.
+int gemm_mid(const qie_linear_args* a, const GemmParams& q, float other_us, hipStream_t st, bool* launched);
+
+}  // namespace qie

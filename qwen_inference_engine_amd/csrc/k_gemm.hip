@@ -14,32 +14,12 @@
 //     rows of the same output column inside one wave).
 //   * blockIdx.x runs over M tiles so the blocks sharing a weight tile are
 //     adjacent in dispatch order (weights streamed ~once, activations L2/MALL).
-#include "qie_common.hpp"
-#include "../../include/qie/qie_ops.h"
+#include "gemm_impl.hpp"
 
 #include <map>
 #include <mutex>
 
 namespace qie {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-struct GemmParams {
-    const uint16_t* A;
-    int64_t lda;
-    const uint16_t* w0;
-    const uint16_t* w1;
-    const uint16_t* w2;
-    const uint16_t* b0;
-    const uint16_t* b1;
-    const uint16_t* b2;
-    int64_t n0, n01;
-    int64_t M, K, N;     // N = output columns
-    int64_t wrows;       // total weight rows addressable (for clamping)
-    uint16_t* C;
-    int64_t ldc;
-};
 
 constexpr int BM = 128, BN = 128, BK = 64;
 
@@ -261,11 +241,6 @@ constexpr int slot_bytes(int bn) { return (BM + bn) * BK * 2; }
 // rows fr (and chunk g) of a 16-row fragment land on 16 distinct bank slots.
 __device__ __forceinline__ int big_swz(int r) { return ((r >> 2) & 1) * 3; }
 
-__device__ __forceinline__ void glds16(const void* src, void* lds) {
-    __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)(src),
-                                     (__attribute__((address_space(3))) void*)(lds), 16, 0, 0);
-}
-
 // weight row feeding tile column c (0..255) of column tile nt; SwiGLU tiles interleave
 // 32 gate rows and the 32 up rows of the same outputs per 64-column wave slice
 template <int EPI, int BNT>
@@ -448,13 +423,10 @@ __global__ __launch_bounds__(512) void gemm_big_kernel(GemmParams p, int n_mt) {
 // last two tiles.  Waves 4-7 run one barrier behind waves 0-3 (an extra s_barrier before the
 // loop, waves 0-3 one after it), so on every SIMD one wave's MFMAs overlap the other
 // wave's reads and DMA issue.  Accumulation order per output = k order (as gemm_big).
-typedef unsigned int u32x4_g8 __attribute__((ext_vector_type(4)));
 namespace g8 {
 constexpr int BM = 256, BN = 256, BK = 64;
 constexpr int BUF = (BM + BN) * BK * 2;   // 64 KB: A rows [0, 256) then W rows, 128 B each
 }  // namespace g8
-
-__device__ __forceinline__ int g8_swz(int r) { return (r >> 1) & 7; }
 
 // Split-K (tiles < CUs: Qwen2-7B O / down at 2,048 rows have 112 256x256 tiles, QKV 144): the
 // k-tiles of a tile are cut into `splitk` consecutive parts, one workgroup each (the remap
@@ -463,12 +435,6 @@ __device__ __forceinline__ int g8_swz(int r) { return (r >> 1) & 7; }
 // order), drains, and adds to the tile's ticket; the part whose add comes last sums the slabs
 // in PART order (sc1 loads: cdna_hip_programming.md §5 'Projection GEMM' item 2), so the result
 // does not depend on arrival order, runs the epilogue and resets the ticket.
-struct G8Split {
-    int splitk;
-    float* slab;       // [tiles][splitk][256 * 256] fp32
-    unsigned* cnt;     // [tiles], zero at rest
-};
-
 template <int EPI>
 __global__ __launch_bounds__(512) void gemm8_kernel(GemmParams p, int n_mt, G8Split sk) {
 #pragma clang fp contract(off)
@@ -1011,7 +977,7 @@ struct G8Ws {
 static std::mutex g8_mu;
 static std::map<hipStream_t, G8Ws> g8_ws;
 
-static int g8_workspace(hipStream_t st, int slabs, int tiles, G8Split* out) {
+int g8_workspace(hipStream_t st, int slabs, int tiles, G8Split* out) {
     std::lock_guard<std::mutex> lk(g8_mu);
     G8Ws& w = g8_ws[st];
     const size_t need = (size_t)slabs * 65536 * 4;
@@ -1092,6 +1058,13 @@ static int g8_splitk(int64_t tiles, int64_t cus, int nk) {
         }
     }
     return best;
+}
+
+// expected time of gemm8_kernel, us: 1.45 a k-tile and 5 a round of the chip (fitted as k_gemm_mid.hip's tiles)
+static float g8_us(int64_t tiles, int64_t cus, int nk) {
+    const int s = tiles < cus ? g8_splitk(tiles, cus, nk) : 1;
+    if (s == 1 && 2 * tiles < cus) return 1e30f;   // not its launch (gemm() below)
+    return (float)cdiv(tiles * s, cus) * (nk / (float)s * 1.45f + 5.f) + 5.f + (s > 1 ? 8.f * s : 0.f);
 }
 
 template <int EPI, int BNT>
@@ -1578,6 +1551,13 @@ int gemm(const qie_linear_args* a, hipStream_t st) {
         // phase-interleaved 256x256 kernel (K a multiple of 64, >= 4 k-tiles): Qwen2-7B gate/up at 2,048
         // rows 612 -> 488 us, bit-identical to gemm_big; down split-K 2: 309 -> 247 us
         const bool g8ok = a->K % g8::BK == 0 && a->K >= 4 * g8::BK;
+        // rows that do not fill the 256x256 tiles: k_gemm_mid.hip, unless the phase-interleaved kernel below is expected
+        // to be faster (Qwen2-7B gate/up: 301 rows 161 -> 119 us, 700 rows 183 against 229)
+        if (dev_env("QIE_MID", 1) && force < 0 && !(a->flags & QIE_LINEAR_STREAMK)) {
+            bool launched = false;
+            const int rc = gemm_mid(a, p, g8ok && a->M >= big::BM ? g8_us(t256, cus, (int)(a->K / g8::BK)) : 1e30f, st, &launched);
+            if (rc || launched) return rc;
+        }
         const int g8mode = dev_env("QIE_GEMM8", 2);   // 2 (default): + split-K below; 1: full-chip grids only; 0: off
         // stream-K (QIE_GEMM8 = 3; args.flags QIE_LINEAR_STREAMK): any tile count, one workgroup per CU
         if (g8ok && ((a->flags & QIE_LINEAR_STREAMK) || (g8mode == 3 && force < 0 && a->M >= big::BM))) {

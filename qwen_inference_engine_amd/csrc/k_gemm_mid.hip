@@ -1,0 +1,406 @@
+// k_gemm_mid.hip — MFMA bf16 GEMM for prompts of a few dozen to about a thousand rows.
+//
+//   C[M, N] = A[M, K] . W[N, K]^T, fp32 accumulation, the epilogues of k_gemm.hip.
+//
+// At these row counts the weights come from HBM once and the 256x256 tiles of the long-prompt kernels leave most of the
+// chip idle (Qwen2-7B, 301 rows: 2 x 14 tiles for the O and down projections), while the register-staged 128x128 kernel
+// holds one k-tile in flight and waits a memory round trip (about 1 us) for every 64 of K.  Here:
+//   * a BM x BN tile (128x128, 128x64, 64x128, 64x64), BK = 64, in a ring of LDS slots filled by LDS-DMA: all slots but
+//     one are in flight, so a CU keeps 48-96 KB of loads outstanding; one barrier per k-tile;
+//   * 8 waves as 2 (M) x 2 (N) x 2 (K halves of every k-tile): a wave's tile is half the block's in both directions, which
+//     reads LDS as often as four waves would, and two waves a SIMD cover each other's fragment reads.  The K halves meet in
+//     LDS once, behind the loop;
+//   * split-K over workgroups where the tiles do not fill the chip (fp32 slabs, the last arriver sums them in part order:
+//     gemm8_kernel's protocol, the result does not depend on arrival order);
+//   * workgroups that share a weight tile are neighbours in one XCD, parts are the slowest index: an XCD's L2 holds one K
+//     range of A.
+#include "gemm_impl.hpp"
+
+#include <algorithm>
+
+namespace qie {
+
+namespace mid {
+constexpr int BK = 64;
+}
+
+// weight row of tile column c of column tile nt; SwiGLU tiles hold, per wave slice of BN / 2 columns, a half of gate rows
+// and the same outputs' up rows
+template <int EPI, int BN>
+__device__ __forceinline__ const uint16_t* mid_wrow(const GemmParams& p, int64_t nt, int c) {
+    if constexpr (EPI == QIE_EPI_SWIGLU) {
+        constexpr int TN = BN / 2, HALF = TN / 2;
+        const int64_t j = nt * TN + (c / TN) * HALF + (c % HALF);
+        const int64_t jj = j < p.N ? j : p.N - 1;
+        return (c % TN >= HALF ? p.w1 : p.w0) + jj * p.K;
+    } else {
+        const int64_t r = nt * BN + c;
+        const int64_t rr = r < p.N ? r : p.N - 1;
+        if (rr < p.n0) return p.w0 + rr * p.K;
+        if (rr < p.n01) return p.w1 + (rr - p.n0) * p.K;
+        return p.w2 + (rr - p.n01) * p.K;
+    }
+}
+
+template <int EPI, int BM, int BN, int SLOTS>
+__global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, int whole, G8Split sk) {
+#pragma clang fp contract(off)
+    constexpr int TM = BM / 2, TN = BN / 2, FI = TM / 16, FJ = TN / 16, FH = FI / 2;
+    constexpr int SLOT = (BM + BN) * 128;      // A rows, then W rows, 128 B each
+    constexpr int IPW = (BM + BN) / 64;        // LDS-DMA instructions (8 rows each) per wave and k-tile
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wk = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+    const int fr = lane & 15, g = lane >> 4;
+    // workgroups [0, whole): a tile each; behind them the other tiles, splitk parts each.  Within either range the
+    // bijective XCD remap keeps neighbours (the M tiles of a weight tile) on one XCD
+    const bool cut = (int)blockIdx.x >= whole;
+    const int nwg = cut ? gridDim.x - whole : whole, orig = cut ? blockIdx.x - whole : blockIdx.x;
+    const int q8 = nwg >> 3, r8 = nwg & 7, xcd = orig & 7;
+    const int wid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (orig >> 3);
+    const int parts = cut ? sk.splitk : 1, cuts = nwg / parts;   // cut tiles: part-major, so an XCD's parts share a K range of A
+    const int part = cut ? wid / cuts : 0, ct = cut ? wid % cuts : 0, tile = cut ? whole + ct : wid;
+    const int64_t mt = tile % n_mt, nt = tile / n_mt, m0 = mt * BM;
+
+    const int nk_all = (int)(p.K / mid::BK);
+    const int kb = (int)((int64_t)part * nk_all / parts);        // this part's k-tiles [kb, kb + nk)
+    const int nk = (int)((int64_t)(part + 1) * nk_all / parts) - kb;
+
+    // instruction i of this wave fills the slot's rows 8 b .. 8 b + 7, b = 8 i + wave: lane -> row 8 b + (lane >> 3),
+    // LDS chunk lane & 7, which holds the source's chunk (lane & 7) ^ swz(row)
+    const uint16_t* src[IPW];
+#pragma unroll
+    for (int i = 0; i < IPW; i++) {
+        const int r = 8 * (8 * i + wave) + (lane >> 3);
+        const int cs = (lane & 7) ^ g8_swz(r);
+        if (r < BM) {   // uniform over the wave: BM is a multiple of 8
+            int64_t ar = m0 + r;
+            ar = ar < p.M ? ar : p.M - 1;   // rows past M: re-read row M - 1, never stored
+            src[i] = p.A + ar * p.lda + (int64_t)kb * mid::BK + cs * 8;
+        } else {
+            src[i] = mid_wrow<EPI, BN>(p, nt, r - BM) + (int64_t)kb * mid::BK + cs * 8;
+        }
+    }
+    auto stage = [&](int kt, int slot) {
+        unsigned char* dst = smem + slot * SLOT + wave * 1024;
+#pragma unroll
+        for (int i = 0; i < IPW; i++) glds16(src[i] + (int64_t)kt * mid::BK, dst + i * 8192);
+    };
+
+    f32x4 acc[FI][FJ];
+#pragma unroll
+    for (int i = 0; i < FI; i++)
+#pragma unroll
+        for (int j = 0; j < FJ; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    for (int t = 0; t < SLOTS - 1 && t < nk; t++) stage(t, t);
+    int slot = 0, fill = SLOTS - 1;
+    for (int t = 0; t < nk; t++) {
+        // k-tile t has landed (the SLOTS - 2 younger ones may still fly), and every wave is done with the slot of t - 1
+        if (t + SLOTS - 1 <= nk) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(IPW * (SLOTS - 2)) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        if (t + SLOTS - 1 < nk) stage(t + SLOTS - 1, fill);
+        const unsigned char* buf = smem + slot * SLOT;
+        bf16x8 fa[FI], fb[FJ];
+#pragma unroll
+        for (int j = 0; j < FJ; j++) {
+            const int row = BM + wn * TN + j * 16 + fr;
+            fb[j] = *reinterpret_cast<const bf16x8*>(buf + row * 128 + (((4 * wk + g) ^ g8_swz(row)) * 16));
+        }
+#pragma unroll
+        for (int i = 0; i < FI; i++) {
+            const int row = wm * TM + i * 16 + fr;
+            fa[i] = *reinterpret_cast<const bf16x8*>(buf + row * 128 + (((4 * wk + g) ^ g8_swz(row)) * 16));
+        }
+#pragma unroll
+        for (int i = 0; i < FI; i++)
+#pragma unroll
+            for (int j = 0; j < FJ; j++)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);   // W Aᵀ
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave's reads of the slot are done
+        __builtin_amdgcn_sched_barrier(0);
+        slot = slot + 1 == SLOTS ? 0 : slot + 1;
+        fill = fill + 1 == SLOTS ? 0 : fill + 1;
+    }
+
+    // ---------------- the two K halves: wave w and w ^ 4 hold the same tile; each keeps half of its rows
+    f32x4 res[FH][FJ];
+    {
+        f32x4* ex = reinterpret_cast<f32x4*>(smem);
+        constexpr int FIT = SLOTS * SLOT / (8 * FH * 1024), JN = FIT < FJ ? FIT : FJ;   // fragment columns the LDS takes at once
+        static_assert(JN >= 1 && FJ % JN == 0, "exchange area");
+#pragma unroll
+        for (int j0 = 0; j0 < FJ; j0 += JN) {
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < FH; i++)
+#pragma unroll
+                for (int j = j0; j < j0 + JN; j++) {
+                    if (wk == 0) {
+                        ex[((wave * FH + i) * JN + j - j0) * 64 + lane] = acc[FH + i][j];
+                        res[i][j] = acc[i][j];
+                    } else {
+                        ex[((wave * FH + i) * JN + j - j0) * 64 + lane] = acc[i][j];
+                        res[i][j] = acc[FH + i][j];
+                    }
+                }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < FH; i++)
+#pragma unroll
+                for (int j = j0; j < j0 + JN; j++) res[i][j] = res[i][j] + ex[(((wave ^ 4) * FH + i) * JN + j - j0) * 64 + lane];
+        }
+    }
+
+    if (parts > 1) {   // uniform
+        constexpr int SLAB = BM * BN;   // floats
+        const int64_t tb = (int64_t)ct * parts;
+        const auto rs = __builtin_amdgcn_make_buffer_rsrc(sk.slab + (tb + part) * SLAB, (short)0, SLAB * 4, 0x00020000);
+#pragma unroll
+        for (int i = 0; i < FH; i++)
+#pragma unroll
+            for (int j = 0; j < FJ; j++)
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_g8, res[i][j]), rs,
+                                                       (((wave * FH + i) * FJ + j) * 64 + lane) * 16, 0, 16);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every storing wave drains
+        __syncthreads();
+        int* flag = reinterpret_cast<int*>(smem);
+        if (tid == 0) {
+            const unsigned old = __hip_atomic_fetch_add(sk.cnt + ct, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            *flag = old == (unsigned)parts - 1 ? 1 : 0;
+        }
+        __syncthreads();
+        if (*flag == 0) return;   // uniform
+        // part order: independent of who arrived last; QN parts' loads in flight (one after the other cost 0.75 us each)
+        constexpr int QN = FH * FJ >= 16 ? 1 : 16 / (FH * FJ);
+        for (int q0 = 0; q0 < parts; q0 += QN) {
+            f32x4 v[QN][FH][FJ];
+#pragma unroll
+            for (int u = 0; u < QN; u++) {
+                const int q = q0 + u < parts ? q0 + u : parts - 1;
+                const auto rq = __builtin_amdgcn_make_buffer_rsrc(sk.slab + (tb + q) * SLAB, (short)0, SLAB * 4, 0x00020000);
+#pragma unroll
+                for (int i = 0; i < FH; i++)
+#pragma unroll
+                    for (int j = 0; j < FJ; j++)
+                        v[u][i][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                                   rq, (((wave * FH + i) * FJ + j) * 64 + lane) * 16, 0, 16));
+            }
+#pragma unroll
+            for (int u = 0; u < QN; u++) {
+                if (q0 + u >= parts) break;
+#pragma unroll
+                for (int i = 0; i < FH; i++)
+#pragma unroll
+                    for (int j = 0; j < FJ; j++) res[i][j] = q0 + u == 0 ? v[u][i][j] : res[i][j] + v[u][i][j];
+            }
+        }
+        if (tid == 0) __hip_atomic_store(sk.cnt + ct, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+
+    // ---------------- epilogue.  D = W Aᵀ: a lane holds row m = lane & 15 and the columns 4 g .. 4 g + 3 of a fragment, one
+    // 8- (fp32: 16-) byte store where C's rows allow it
+    const bool vec = p.vec != 0;
+    const int64_t row0 = m0 + wm * TM + wk * (FH * 16) + fr;
+    if constexpr (EPI == QIE_EPI_SWIGLU) {
+#pragma unroll
+        for (int jj = 0; jj < FJ / 2; jj++) {
+            const int64_t col = nt * TN + (TN / 2) * wn + 16 * jj + 4 * g;
+#pragma unroll
+            for (int i = 0; i < FH; i++) {
+                const int64_t row = row0 + i * 16;
+                if (row >= p.M) continue;
+                float h[4];
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float gg = rbf(res[i][jj][r]);
+                    const float uu = rbf(res[i][jj + FJ / 2][r]);
+                    h[r] = uu * rbf(gg * (1.0f / (1.0f + expf(-gg))));
+                }
+                uint16_t* dst = p.C + row * p.ldc + col;
+                if (vec && col + 4 <= p.N) {
+                    *reinterpret_cast<uint2*>(dst) = make_uint2(pack2(h[0], h[1]), pack2(h[2], h[3]));
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        if (col + r < p.N) dst[r] = f2bf(h[r]);
+                }
+            }
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < FJ; j++) {
+            const int64_t col = nt * BN + wn * TN + j * 16 + 4 * g;
+            float bias[4] = {0.f, 0.f, 0.f, 0.f};
+            if constexpr (EPI == QIE_EPI_STORE) {
+                if (p.b0 || p.b1 || p.b2) {
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const int64_t c = col + r < p.N ? col + r : p.N - 1;
+                        const uint16_t* b = c < p.n0 ? p.b0 : (c < p.n01 ? p.b1 : p.b2);
+                        if (b) bias[r] = bf2f(b[c < p.n0 ? c : (c < p.n01 ? c - p.n0 : c - p.n01)]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < FH; i++) {
+                const int64_t row = row0 + i * 16;
+                if (row >= p.M) continue;
+                const f32x4 v = res[i][j];
+                if constexpr (EPI == QIE_EPI_F32) {
+                    float* dst = reinterpret_cast<float*>(p.C) + row * p.ldc + col;
+                    if (vec && col + 4 <= p.N) {
+                        *reinterpret_cast<f32x4*>(dst) = v;
+                    } else {
+#pragma unroll
+                        for (int r = 0; r < 4; r++)
+                            if (col + r < p.N) dst[r] = v[r];
+                    }
+                    continue;
+                }
+                uint16_t* dst = p.C + row * p.ldc + col;
+                if (vec && col + 4 <= p.N) {
+                    float o[4];
+                    if constexpr (EPI == QIE_EPI_RESIDUAL) {
+                        const uint2 x = *reinterpret_cast<const uint2*>(dst);
+                        o[0] = bf_lo(x.x) + rbf(v[0]);
+                        o[1] = bf_hi(x.x) + rbf(v[1]);
+                        o[2] = bf_lo(x.y) + rbf(v[2]);
+                        o[3] = bf_hi(x.y) + rbf(v[3]);
+                    } else {
+#pragma unroll
+                        for (int r = 0; r < 4; r++) o[r] = v[r] + bias[r];
+                    }
+                    *reinterpret_cast<uint2*>(dst) = make_uint2(pack2(o[0], o[1]), pack2(o[2], o[3]));
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        if (col + r >= p.N) continue;
+                        if constexpr (EPI == QIE_EPI_RESIDUAL) dst[r] = f2bf(bf2f(dst[r]) + rbf(v[r]));
+                        else dst[r] = f2bf(v[r] + bias[r]);
+                    }
+                }
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------- the plan
+namespace {
+// Times of a tile, us, fitted to the Qwen2-0.5B / 7B and Qwen3-14B projections at 20 to 2,048 rows (168 shapes; what the
+// rule below picks is 1 % over the best of all tiles, splits and the 256x256 kernel on the average, 17 % at most):
+// up to one workgroup a CU a1 + s1 per k-tile, more a2 + (rounds of the chip) * (f2 + s2 per k-tile).  A k-tile costs what its
+// lines take through one CU (about 50 GB/s where they come from HBM or another die, 120 GB/s from L2), not its matrix work,
+// which is why the tall tiles win as soon as the rows fill them.
+struct MidTile {
+    int bm, bn, slots, per_cu;   // per_cu: workgroups that fit a CU's LDS
+    float a1, s1, a2, f2, s2;
+};
+constexpr MidTile MID_TILES[] = {
+    {64, 64, 5, 2, 3.2f, .285f, 5.f, .7f, .487f},   {64, 128, 3, 2, 2.6f, .475f, 5.4f, 1.1f, .74f},
+    {128, 64, 3, 2, 3.3f, .43f, 4.7f, 1.8f, .70f},  {128, 128, 4, 1, 5.9f, .54f, 7.5f, 3.9f, .575f},
+    {192, 128, 4, 1, 8.f, .65f, 5.f, 6.f, .72f},    {256, 128, 3, 1, 9.9f, .90f, 12.f, 2.5f, 1.037f},
+    {320, 64, 3, 1, 6.9f, .70f, 6.5f, 3.f, .787f},  {320, 128, 2, 1, 9.4f, 1.11f, 14.f, 2.f, 1.2f},
+};
+constexpr int MID_N = sizeof(MID_TILES) / sizeof(MID_TILES[0]);
+struct MidPlan {
+    int tile, whole, splitk, n_mt, n_nt;
+    float us;
+};
+
+// the last round of a launch costs nearly a whole one
+float mid_rounds(float x) {
+    const float f = (float)(int)x;
+    return f + (x > f ? std::max(.8f, x - f + .3f) : 0.f);
+}
+
+// Tile and split: the tiles run whole round by round of the chip; the last, partial round's tiles may be cut into `splitk`
+// K ranges (3 us a part for 128x128 outputs: slab out, slab in).
+MidPlan mid_plan(int64_t M, int64_t cols, int64_t K, int64_t cus) {
+    MidPlan best{-1, 0, 1, 0, 0, 1e30f};
+    const int nk = (int)(K / mid::BK);
+    const float floor_us = (float)cols * K * 2 / 5.3e6f + 4.f;   // the weights at the rate they stream here
+    for (int c = 0; c < MID_N; c++) {
+        const MidTile& t = MID_TILES[c];
+        const int64_t n_mt = cdiv(M, t.bm), n_nt = cdiv(cols, t.bn), tiles = n_mt * n_nt;
+        if (tiles > (1 << 22)) continue;   // (of 32-bit workgroup counts)
+        const float room = (float)(cus * t.per_cu);
+        for (int s = 1; s <= 12 && s <= nk; s++) {
+            const int64_t whole = s == 1 ? tiles : tiles / (cus * t.per_cu) * (cus * t.per_cu), cut = (tiles - whole) * s;
+            float us;
+            if (s == 1) {
+                us = tiles <= cus ? t.a1 + nk * t.s1 : t.a2 + mid_rounds(tiles / room) * (t.f2 + nk * t.s2);
+            } else {
+                if (cut == 0) break;
+                const float len = (float)((nk + s - 1) / s);
+                us = whole / room * (t.f2 + nk * t.s2) + 3.f * s * (t.bm * t.bn) / 16384.f + 1.f;
+                us += cut <= cus ? t.a1 + len * t.s1 : t.a2 + mid_rounds(cut / room) * (t.f2 + len * t.s2);
+            }
+            us = std::max(us, floor_us);
+            if (us < best.us) best = {c, (int)whole, s, (int)n_mt, (int)n_nt, us};
+        }
+    }
+    return best;
+}
+
+template <int EPI, int BM, int BN, int SLOTS>
+int launch_mid_t(const GemmParams& p, const MidPlan& pl, const G8Split& sk, hipStream_t st) {
+    const void* fn = (const void*)gemm_mid_kernel<EPI, BM, BN, SLOTS>;
+    constexpr size_t shm = (size_t)SLOTS * (BM + BN) * 128;
+    static bool raised = false;
+    if (!raised) {
+        QIE_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
+        raised = true;
+    }
+    const int tiles = pl.n_mt * pl.n_nt, whole = sk.splitk > 1 ? pl.whole : tiles;
+    hipLaunchKernelGGL((gemm_mid_kernel<EPI, BM, BN, SLOTS>), dim3((unsigned)(whole + (tiles - whole) * sk.splitk)), dim3(512), shm,
+                       st, p, pl.n_mt, whole, sk);
+    QIE_LAUNCH_CHECK();
+    return 0;
+}
+
+template <int EPI>
+int launch_mid(const GemmParams& p, const MidPlan& pl, const G8Split& sk, hipStream_t st) {
+    switch (pl.tile) {
+        case 0: return launch_mid_t<EPI, 64, 64, 5>(p, pl, sk, st);
+        case 1: return launch_mid_t<EPI, 64, 128, 3>(p, pl, sk, st);
+        case 2: return launch_mid_t<EPI, 128, 64, 3>(p, pl, sk, st);
+        case 3: return launch_mid_t<EPI, 128, 128, 4>(p, pl, sk, st);
+        case 4: return launch_mid_t<EPI, 192, 128, 4>(p, pl, sk, st);
+        case 5: return launch_mid_t<EPI, 256, 128, 3>(p, pl, sk, st);
+        case 6: return launch_mid_t<EPI, 320, 64, 3>(p, pl, sk, st);
+        default: return launch_mid_t<EPI, 320, 128, 2>(p, pl, sk, st);
+    }
+}
+}  // namespace
+
+// other_us: what the caller's other kernel for this shape takes
+int gemm_mid(const qie_linear_args* a, const GemmParams& q, float other_us, hipStream_t st, bool* launched) {
+    *launched = false;
+    GemmParams p = q;
+    p.vec = a->ldy % 4 == 0 && ((uintptr_t)a->y) % (a->epilogue == QIE_EPI_F32 ? 16 : 8) == 0;
+    // LDS-DMA moves 16-byte pieces of the weights' rows (x's rows are on that grid: qie_linear)
+    if (a->K % mid::BK != 0 || (((uintptr_t)a->w[0] | (uintptr_t)a->w[1] | (uintptr_t)a->w[2]) % 16) != 0) return 0;
+    const int64_t cols = a->epilogue == QIE_EPI_SWIGLU ? 2 * a->N : a->N;
+    const MidPlan pl = mid_plan(a->M, cols, a->K, device_cu_count());
+    if (pl.tile < 0 || pl.us >= 0.88f * other_us) return 0;   // 12 %: what the two fits are off by on long prompts
+    G8Split sk{1, nullptr, nullptr};
+    const int64_t cut = (int64_t)pl.n_mt * pl.n_nt - pl.whole;
+    if (pl.splitk > 1 && cut > 0) {
+        const int64_t floats = cut * pl.splitk * MID_TILES[pl.tile].bm * MID_TILES[pl.tile].bn;
+        if (g8_workspace(st, (int)cdiv(floats, 65536), (int)cut, &sk) == 0) sk.splitk = pl.splitk;
+    }
+    *launched = true;
+    switch (a->epilogue) {
+        case QIE_EPI_SWIGLU: return launch_mid<QIE_EPI_SWIGLU>(p, pl, sk, st);
+        case QIE_EPI_RESIDUAL: return launch_mid<QIE_EPI_RESIDUAL>(p, pl, sk, st);
+        case QIE_EPI_F32: return launch_mid<QIE_EPI_F32>(p, pl, sk, st);
+        default: return launch_mid<QIE_EPI_STORE>(p, pl, sk, st);
+    }
+}
+
+}  // namespace qie
