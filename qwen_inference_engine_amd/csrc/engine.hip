@@ -27,6 +27,7 @@ int gemv_rope(const qie_linear_args* a, const int32_t* pos, const float* cs, con
               hipStream_t st);
 int gemm(const qie_linear_args* a, hipStream_t st);
 bool dec8_applies(const qie_linear_args* a);
+bool dec_bf16_applies(const qie_linear_args* a);
 int dec8_reserve(hipStream_t st);
 bool persist_supported(const qie_model_spec& s, int B, int tp, bool fp8, bool paged, int ncu, const char** why);
 size_t persist_attn_table_bytes(int n_layers);
@@ -440,7 +441,7 @@ static int row_parallel(qie_batch* b, qie_linear_args& a, uint16_t* x, float* pa
     return e->comm->allreduce_residual_bf16(part, x, n, e->stream);   // one kernel on the peer backend
 }
 
-// Batched rows (2 <= M <= 16, the skinny MFMA kernel): RMSNorm the M rows once into b->xn
+// Batched rows (2 <= M <= 16) of the skinny MFMA kernel (shapes k_decode_bf16.hip and k_decode_fp8.hip do not take): RMSNorm the M rows once into b->xn
 // (qie_rmsnorm, normalization.cu:5-25 semantics) and feed the projection plain rows.  The
 // skinny kernel's fused norm prologue recomputed every row's norm in every workgroup and
 // cost 13-16 us per launch at B = 8 (tools/ubench_b8.py, QIE_SKINNY_DBG); M = 1 keeps the
@@ -448,7 +449,8 @@ static int row_parallel(qie_batch* b, qie_linear_args& a, uint16_t* x, float* pa
 static int prenorm(qie_batch* b, qie_linear_args& a, int64_t M) {
     static const int on = dev_env("QIE_PRENORM", 1);
     if (!on || M < 2 || M > 16 || !a.norm_w) return 0;
-    if (dec8_applies(&a) && dev_env("QIE_DEC8_PRENORM", 0) == 0) return 0;   // the fp8 batched-decode kernel fuses the norm
+    if (dec8_applies(&a) && dev_env("QIE_DEC8_PRENORM", 0) == 0) return 0;   // the batched-decode kernels fuse the norm
+    if (dec_bf16_applies(&a)) return 0;
     QIE_TRY(qie_rmsnorm(a.x, a.norm_w, b->xn, M, a.K, a.norm_eps, a.numerics, b->e->stream));
     a.x = b->xn;
     a.ldx = a.K;
@@ -1761,8 +1763,8 @@ int qie_batch_time_kernel(qie_batch* b, int32_t which, int32_t iters, double* av
             a.argmax_keys = (uint64_t*)(((uintptr_t)(scratch + B * V) + 7) & ~(uintptr_t)7);   // as the greedy step runs it
             *by = (double)V * H * wb + B * H * 2 + B * (double)V * 2;
         }
-        // as prenorm() decides for the real step: the fp8 batched-decode kernel keeps its fused norm
-        const bool fused8 = dec8_applies(&a) && dev_env("QIE_DEC8_PRENORM", 0) == 0;
+        // as prenorm() decides for the real step: the batched-decode kernels keep their fused norm
+        const bool fused8 = (dec8_applies(&a) && dev_env("QIE_DEC8_PRENORM", 0) == 0) || dec_bf16_applies(&a);
         if (batched_norm && a.norm_w && !fused8) {
             a.x = b->xn;   // as the batched step runs it: rows normed once by prenorm(), plain GEMV
             a.ldx = a.K;

@@ -1,0 +1,444 @@
+// k_decode_bf16.hip — batched decode projections on bf16 weights (2 <= M <= 16 rows).
+//
+//   Y[M, N] = X[M, K] . W[N, K]^T with the RMSNorm of X in front where it is asked for, and the epilogues of qie_linear.
+//
+// The weights are all the traffic.  The register-fed skinny kernel (k_gemv.hip) loads its fragments as 16 rows x 64 B and
+// waits for them at every step: 4.7 TB/s for Qwen2-7B's gate/up at 4 rows.  Here a workgroup of 8 waves owns whole tiles of
+// 16 weight rows, and every wave streams the 128-k chunks of its own share of K (256 contiguous bytes of each row, 4 KB) by
+// LDS-DMA through a ring of its own, with no barrier: the loads of R - 1 chunks fly while one is multiplied
+// (v_mfma_f32_16x16x32_bf16, D = W Xᵀ, so a lane ends with four neighbouring columns of one row).
+//   * X lies in LDS for the whole launch (normed once a workgroup by the waves themselves, under the first chunks' loads);
+//     where M rows of K do not fit (the down projection) its chunks travel through the ring beside the weights'.
+//   * The 8 partial tiles meet in LDS, one barrier a tile; the wave that sums them and runs the epilogue rotates.
+//   * SwiGLU: a tile is 8 gate rows and the same outputs' 8 up rows, met across lane halves.
+// One workgroup a CU: LDS holds 64 to 128 KB of chunks.  Sums: per wave over its K share in fp32, the shares in wave order.
+#include "qie_common.hpp"
+#include "../../include/qie/qie_ops.h"
+
+#include <algorithm>
+#include <type_traits>
+
+namespace qie {
+
+typedef __bf16 db_bf16x8 __attribute__((ext_vector_type(8)));
+typedef float db_f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int db_u32x4 __attribute__((ext_vector_type(4)));
+
+namespace db {
+constexpr int NW = 8;          // waves
+constexpr int CH = 128;        // k of a chunk
+constexpr int WCH = 16 * 256;  // bytes of a weight chunk
+}
+
+struct DecBfParams {
+    const uint16_t* x;
+    int64_t ldx;
+    const uint16_t* norm_w;
+    float eps;
+    int numerics;
+    const uint16_t* w[3];
+    const uint16_t* bias[3];
+    int64_t n0, n01;           // rows of segment 0, of segments 0 and 1
+    int K, N, M;
+    int n_tiles;
+    uint16_t* y;
+    int64_t ldy;
+    int vec;                   // 8- (fp32: 16-) byte stores
+    unsigned long long* keys;
+    int64_t key_col0;
+    int xstride;               // bytes of a row of the X image (K * 2 + 16: 16 rows' same chunk in different banks)
+};
+
+__device__ __forceinline__ void db_glds16(const void* src, void* lds) {
+    __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)(src),
+                                     (__attribute__((address_space(3))) void*)(lds), 16, 0, 0);
+}
+
+// XM: 0 = X in LDS; 8, 16 = X's chunks (of 8 or 16 rows) through the ring.  NV: 16-byte vectors of a row per lane while X is
+// normed (K <= 512 NV); R: ring slots a wave.
+template <int EPI, int XM, int NV, int R>
+__global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
+#pragma clang fp contract(off)
+    constexpr int SLOT = db::WCH + XM * 256;
+    constexpr int IPC = 4 + XM / 4;   // LDS-DMA instructions of a chunk (4 rows of 256 B each)
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int fr = lane & 15, g = lane >> 4;
+    unsigned char* ring = smem + wave * (R * SLOT);
+    const int M = p.M, K = p.K;
+    // partial tiles [2][NW][RS]: all 64 lanes' quads, or those of X rows 0 .. 7
+    const int RS = M <= 8 ? 32 : 64, rl = M <= 8 ? g * 8 + (fr & 7) : lane;
+    db_f32x4* red = reinterpret_cast<db_f32x4*>(smem + db::NW * R * SLOT);
+    unsigned char* xs = smem + db::NW * R * SLOT + 2 * db::NW * RS * 16;
+    const int chunks = K / db::CH;
+    const int c0 = wave * chunks / db::NW, cnt = (wave + 1) * chunks / db::NW - c0;   // this wave's share of K
+    const int T = p.n_tiles, G = gridDim.x;
+    const int mine = ((int)blockIdx.x < T) ? (T - 1 - (int)blockIdx.x) / G + 1 : 0;
+    const int items = mine * cnt;   // (tile, chunk) in order
+
+    // ---- X rows for the norm (or the copy), loaded ahead of the first weight chunks: P waves a row (8, 4, 2 rows at a time), so
+    // that few rows keep every wave busy
+    const db_u32x4 zero = {0u, 0u, 0u, 0u};
+    const int P = M <= 2 ? 4 : M <= 4 ? 2 : 1, rows_at = db::NW / P, sub = wave % P;
+    db_u32x4 xv[NV], nv[NV];
+    auto load_row = [&](int m) {
+#pragma unroll
+        for (int v = 0; v < NV; v++) {
+            if (v * P * 512 >= K) break;   // uniform
+            const int k = ((v * P + sub) * 64 + lane) * 8;
+            xv[v] = k < K ? *reinterpret_cast<const db_u32x4*>(p.x + (int64_t)m * p.ldx + k) : zero;
+            if (p.norm_w) nv[v] = k < K ? *reinterpret_cast<const db_u32x4*>(p.norm_w + k) : zero;
+        }
+    };
+    if constexpr (XM == 0) {
+        if (wave / P < M) load_row(wave / P);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+
+    // ---- the weight stream: lane -> row 4 i + (lane >> 4) of the tile, LDS piece lane & 15 of its 256 B, which holds the
+    // source's piece (lane & 15) ^ row (the fragment reads below are then free of bank conflicts)
+    const uint16_t* wsrc[4];
+    const uint16_t* xsrc[XM ? XM / 4 : 1];
+    if constexpr (XM != 0) {
+#pragma unroll
+        for (int i = 0; i < XM / 4; i++) {
+            const int m = 4 * i + (lane >> 4);
+            xsrc[i] = p.x + (int64_t)(m < M ? m : M - 1) * p.ldx + ((lane & 15) ^ m) * 8;
+        }
+    }
+    auto aim = [&](int tile) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int row = 4 * i + (lane >> 4);
+            const uint16_t* base;
+            if constexpr (EPI == QIE_EPI_SWIGLU) {
+                int64_t j = (int64_t)tile * 8 + (row & 7);
+                j = j < p.N ? j : p.N - 1;
+                base = (row < 8 ? p.w[0] : p.w[1]) + j * K;
+            } else {
+                int64_t r = (int64_t)tile * 16 + row;
+                r = r < p.N ? r : p.N - 1;
+                base = r < p.n0 ? p.w[0] + r * K : (r < p.n01 ? p.w[1] + (r - p.n0) * K : p.w[2] + (r - p.n01) * K);
+            }
+            wsrc[i] = base + ((lane & 15) ^ row) * 8;
+        }
+    };
+    int n_tile = blockIdx.x, n_c = 0, n_slot = 0;   // the next chunk to ask for
+    auto issue = [&]() {
+        unsigned char* dst = ring + n_slot * SLOT;
+        const int64_t k = (int64_t)(c0 + n_c) * db::CH;
+#pragma unroll
+        for (int i = 0; i < 4; i++) db_glds16(wsrc[i] + k, dst + i * 1024);
+        if constexpr (XM != 0) {
+#pragma unroll
+            for (int i = 0; i < XM / 4; i++) db_glds16(xsrc[i] + k, dst + db::WCH + i * 1024);
+        }
+        n_slot = n_slot + 1 == R ? 0 : n_slot + 1;
+        if (++n_c == cnt) {
+            n_c = 0;
+            n_tile += G;
+            aim(n_tile < T ? n_tile : T - 1);
+        }
+    };
+    if (items > 0) aim(n_tile);
+    for (int i = 0; i < R && i < items; i++) issue();
+    __builtin_amdgcn_sched_barrier(0);
+
+    if constexpr (XM == 0) {
+        auto store_row = [&](int m) {
+#pragma unroll
+            for (int v = 0; v < NV; v++) {
+                if (v * P * 512 >= K) break;
+                const int k = ((v * P + sub) * 64 + lane) * 8;
+                if (k < K) *reinterpret_cast<db_u32x4*>(xs + m * p.xstride + k * 2) = xv[v];
+            }
+        };
+        if (p.norm_w) {   // M <= 8: one pass
+            const int m = wave / P;
+            float* ssq = reinterpret_cast<float*>(red);
+            float ss = 0.f;
+#pragma unroll
+            for (int v = 0; v < NV; v++) {
+                if (v * P * 512 >= K) break;
+                const uint32_t e[4] = {xv[v].x, xv[v].y, xv[v].z, xv[v].w};
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float a = bf_lo(e[j]), b = bf_hi(e[j]);
+                    ss += a * a + b * b;
+                }
+            }
+            ss = wave_sum(ss);
+            if (lane == 0) ssq[wave] = ss;
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (not __syncthreads: the chunks in flight stay there)
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            float tot = 0.f;
+            for (int q = 0; q < P; q++) tot += ssq[wave - sub + q];
+            const float rms = sqrtf((tot / (float)K) + p.eps), inv = 1.0f / rms, rr = rms < INFINITY ? rms : 0.f;
+            auto apply = [&](auto hf) {
+                constexpr bool HF = decltype(hf)::value;
+#pragma unroll
+                for (int v = 0; v < NV; v++) {
+                    if (v * P * 512 >= K) break;
+                    xv[v].x = rms_pair<HF>(xv[v].x, nv[v].x, rr, inv);
+                    xv[v].y = rms_pair<HF>(xv[v].y, nv[v].y, rr, inv);
+                    xv[v].z = rms_pair<HF>(xv[v].z, nv[v].z, rr, inv);
+                    xv[v].w = rms_pair<HF>(xv[v].w, nv[v].w, rr, inv);
+                }
+            };
+            if (m < M) {
+                if (p.numerics == QIE_NUMERICS_HF) apply(std::true_type{});
+                else apply(std::false_type{});
+                store_row(m);
+            }
+        } else {
+            for (int m = wave / P; m < M; m += rows_at) {
+                if (m >= rows_at) load_row(m);
+                store_row(m);
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    }
+
+    const int arow = fr < M ? fr : M - 1;   // rows past M: copies of row M - 1, never stored
+    unsigned long long kbest = 0ull;
+    int done = 0, slot = 0;
+    for (int it = 0; it < mine; it++) {
+        const int tile = blockIdx.x + it * G;
+        db_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        for (int c = 0; c < cnt; c++) {
+            // the oldest chunk has landed: R - 1 younger ones may fly (fewer at the end of the stream)
+            if (done + R <= items) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(IPC * (R - 1)) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            const unsigned char* buf = ring + slot * SLOT;
+            db_bf16x8 wf[4], xf[4];
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                wf[s] = *reinterpret_cast<const db_bf16x8*>(buf + fr * 256 + (((4 * s + g) ^ fr) * 16));
+                if constexpr (XM == 0)
+                    xf[s] = *reinterpret_cast<const db_bf16x8*>(xs + arow * p.xstride + (c0 + c) * 256 + (4 * s + g) * 16);
+                else
+                    xf[s] = *reinterpret_cast<const db_bf16x8*>(buf + db::WCH + (fr & (XM - 1)) * 256 + (((4 * s + g) ^ (fr & (XM - 1))) * 16));
+            }
+#pragma unroll
+            for (int s = 0; s < 4; s++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[s], xf[s], acc, 0, 0, 0);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the slot's reads are done
+            __builtin_amdgcn_sched_barrier(0);
+            if (done + R < items) issue();
+            done++;
+            slot = slot + 1 == R ? 0 : slot + 1;
+        }
+        if (fr < 8 || M > 8) red[((it & 1) * db::NW + wave) * RS + rl] = acc;
+        // one barrier a tile: a slot of `red` is written again two tiles on, behind the next tile's barrier, which the summing
+        // wave reaches only after its reads.  (No vmcnt wait: the ring's loads stay in flight.)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        if (wave != it % db::NW) continue;   // wave-uniform
+        db_f32x4 v = red[(it & 1) * db::NW * RS + rl];
+#pragma unroll
+        for (int w = 1; w < db::NW; w++) v = v + red[((it & 1) * db::NW + w) * RS + rl];
+        // lane: row m = fr of X, columns 4 g .. 4 g + 3 of the tile (SwiGLU: g = 0, 1 gate, g = 2, 3 the same outputs' up)
+        const int m = fr;
+        if constexpr (EPI == QIE_EPI_SWIGLU) {
+            float h[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                float a = v[r], b = v[r];
+                lane_swap<32>(a, b);   // lanes 0..31: a = own (gate), b = lane + 32's (up)
+                const float gg = rbf(a), uu = rbf(b);
+                h[r] = uu * rbf(gg * (1.0f / (1.0f + expf(-gg))));
+            }
+            const int64_t col = (int64_t)tile * 8 + 4 * g;
+            if (g < 2 && m < M) {
+                uint16_t* dst = p.y + (int64_t)m * p.ldy + col;
+                if (p.vec && col + 4 <= p.N) {
+                    *reinterpret_cast<uint2*>(dst) = make_uint2(pack2(h[0], h[1]), pack2(h[2], h[3]));
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        if (col + r < p.N) dst[r] = f2bf(h[r]);
+                }
+            }
+        } else if (m < M) {
+            const int64_t col = (int64_t)tile * 16 + 4 * g;
+            if constexpr (EPI == QIE_EPI_F32) {
+                float* dst = reinterpret_cast<float*>(p.y) + (int64_t)m * p.ldy + col;
+                if (p.vec && col + 4 <= p.N) {
+                    *reinterpret_cast<db_f32x4*>(dst) = v;
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        if (col + r < p.N) dst[r] = v[r];
+                }
+            } else {
+                uint16_t* dst = p.y + (int64_t)m * p.ldy + col;
+                const bool whole = p.vec && col + 4 <= p.N;
+                float o[4];
+                if constexpr (EPI == QIE_EPI_RESIDUAL) {
+                    if (whole) {
+                        const uint2 x = *reinterpret_cast<const uint2*>(dst);
+                        o[0] = bf_lo(x.x);
+                        o[1] = bf_hi(x.x);
+                        o[2] = bf_lo(x.y);
+                        o[3] = bf_hi(x.y);
+                    } else {
+#pragma unroll
+                        for (int r = 0; r < 4; r++) o[r] = col + r < p.N ? bf2f(dst[r]) : 0.f;
+                    }
+#pragma unroll
+                    for (int r = 0; r < 4; r++) o[r] += rbf(v[r]);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const int64_t c = col + r < p.N ? col + r : p.N - 1;
+                        const uint16_t* b = c < p.n0 ? p.bias[0] : (c < p.n01 ? p.bias[1] : p.bias[2]);
+                        o[r] = v[r] + (b ? bf2f(b[c < p.n0 ? c : (c < p.n01 ? c - p.n0 : c - p.n01)]) : 0.f);
+                    }
+                }
+                const uint32_t lo = pack2(o[0], o[1]), hi = pack2(o[2], o[3]);
+                if (whole) {
+                    *reinterpret_cast<uint2*>(dst) = make_uint2(lo, hi);
+                } else {
+                    const uint16_t q[4] = {(uint16_t)lo, (uint16_t)(lo >> 16), (uint16_t)hi, (uint16_t)(hi >> 16)};
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        if (col + r < p.N) dst[r] = q[r];
+                }
+                if (EPI == QIE_EPI_STORE && p.keys) {
+                    const uint32_t q[4] = {lo & 0xffffu, lo >> 16, hi & 0xffffu, hi >> 16};
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        if (col + r >= p.N) continue;
+                        const unsigned long long kk = sel_key(bf2f(q[r]), (uint32_t)(col + r + p.key_col0));
+                        kbest = kk > kbest ? kk : kbest;
+                    }
+                }
+            }
+        }
+    }
+    if (EPI == QIE_EPI_STORE && p.keys) {   // the best key of every row: over the lanes and waves, then one atomic a workgroup
+        __syncthreads();
+        unsigned long long* kb = reinterpret_cast<unsigned long long*>(red);
+        kb[wave * 64 + lane] = kbest;
+        __syncthreads();
+        if (tid < M) {
+            unsigned long long b = 0ull;
+            for (int w = 0; w < db::NW; w++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const unsigned long long k = kb[w * 64 + q * 16 + tid];
+                    b = k > b ? k : b;
+                }
+            if (b) atomicMax(p.keys + tid, b);
+        }
+    }
+}
+
+// ---------------------------------------------------------------- dispatch
+namespace {
+constexpr int64_t kDbLds = 160 * 1024;
+
+// X in LDS beside a ring of R slots a wave
+int64_t db_red_bytes(int64_t M) { return 2 * db::NW * (M <= 8 ? 512 : 1024); }
+int64_t db_image_bytes(int64_t M, int64_t K, int R) { return db::NW * R * db::WCH + db_red_bytes(M) + M * (K * 2 + 16); }
+
+struct DbPlan {
+    int xm, nv, r;
+    size_t lds;
+};
+bool db_plan(const qie_linear_args* a, DbPlan* out) {
+    if (dev_env("QIE_DEC_BF16", 1) == 0) return false;
+    if ((a->flags & QIE_LINEAR_FP8) || a->M < 2 || a->M > 16 || a->K % db::CH != 0 || a->K / db::CH < db::NW / 2) return false;
+    if (a->norm_w && (a->M > db::NW || ((uintptr_t)a->norm_w) % 16 != 0)) return false;
+    if (a->K <= 5120) {
+        for (int r = 4; r >= 2; r--)
+            if (db_image_bytes(a->M, a->K, r) <= kDbLds) {
+                *out = {0, a->K <= 1024 ? 2 : a->K <= 2048 ? 4 : a->K <= 3584 ? 7 : 10, r, (size_t)db_image_bytes(a->M, a->K, r)};
+                return true;
+            }
+    }
+    if (a->norm_w) return false;
+    const int xm = a->M <= 8 ? 8 : 16;
+    *out = {xm, 1, 2, (size_t)(db::NW * 2 * (db::WCH + xm * 256) + db_red_bytes(a->M))};
+    return true;
+}
+
+template <int EPI, int XM, int NV, int R>
+int db_launch(const DecBfParams& p, size_t lds, hipStream_t st) {
+    const void* fn = (const void*)dec_bf16_kernel<EPI, XM, NV, R>;
+    static bool raised = false;
+    if (!raised) {
+        QIE_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDbLds));
+        raised = true;
+    }
+    const int grid = std::max(1, std::min(p.n_tiles, (int)device_cu_count()));
+    hipLaunchKernelGGL((dec_bf16_kernel<EPI, XM, NV, R>), dim3((unsigned)grid), dim3(512), lds, st, p);
+    QIE_LAUNCH_CHECK();
+    return 0;
+}
+template <int EPI, int R>
+int db_launch_nv(const DecBfParams& p, const DbPlan& pl, hipStream_t st) {
+    switch (pl.nv) {
+        case 2: return db_launch<EPI, 0, 2, R>(p, pl.lds, st);
+        case 4: return db_launch<EPI, 0, 4, R>(p, pl.lds, st);
+        case 7: return db_launch<EPI, 0, 7, R>(p, pl.lds, st);
+        default: return db_launch<EPI, 0, 10, R>(p, pl.lds, st);
+    }
+}
+template <int EPI>
+int db_launch_plan(const DecBfParams& p, const DbPlan& pl, hipStream_t st) {
+    if (pl.xm == 8) return db_launch<EPI, 8, 1, 2>(p, pl.lds, st);
+    if (pl.xm == 16) return db_launch<EPI, 16, 1, 2>(p, pl.lds, st);
+    if (pl.r == 4) return db_launch_nv<EPI, 4>(p, pl, st);
+    if (pl.r == 3) return db_launch_nv<EPI, 3>(p, pl, st);
+    return db_launch_nv<EPI, 2>(p, pl, st);
+}
+}  // namespace
+
+// whether dec_bf16_linear takes this projection as it stands, its norm included
+bool dec_bf16_applies(const qie_linear_args* a) {
+    DbPlan pl;
+    return db_plan(a, &pl);
+}
+
+int dec_bf16_linear(const qie_linear_args* a, hipStream_t st, bool* done) {
+    DbPlan pl;
+    *done = db_plan(a, &pl);
+    if (!*done) return 0;
+    DecBfParams p{};
+    p.x = (const uint16_t*)a->x;
+    p.ldx = a->ldx;
+    p.norm_w = (const uint16_t*)a->norm_w;
+    p.eps = a->norm_eps;
+    p.numerics = a->numerics;
+    for (int i = 0; i < 3; i++) {
+        p.w[i] = (const uint16_t*)a->w[i];
+        p.bias[i] = (const uint16_t*)a->bias[i];
+    }
+    p.n0 = a->seg_rows[0];
+    p.n01 = a->seg_rows[0] + a->seg_rows[1];
+    p.K = (int)a->K;
+    p.N = (int)a->N;
+    p.M = (int)a->M;
+    p.n_tiles = (int)(a->epilogue == QIE_EPI_SWIGLU ? (a->N + 7) / 8 : (a->N + 15) / 16);
+    p.y = (uint16_t*)a->y;
+    p.ldy = a->ldy;
+    p.vec = a->ldy % 4 == 0 && ((uintptr_t)a->y) % (a->epilogue == QIE_EPI_F32 ? 16 : 8) == 0;
+    p.keys = (unsigned long long*)a->argmax_keys;
+    p.key_col0 = a->key_col0;
+    p.xstride = (int)a->K * 2 + 16;
+    switch (a->epilogue) {
+        case QIE_EPI_SWIGLU: return db_launch_plan<QIE_EPI_SWIGLU>(p, pl, st);
+        case QIE_EPI_RESIDUAL: return db_launch_plan<QIE_EPI_RESIDUAL>(p, pl, st);
+        case QIE_EPI_F32: return db_launch_plan<QIE_EPI_F32>(p, pl, st);
+        default: return db_launch_plan<QIE_EPI_STORE>(p, pl, st);
+    }
+}
+
+}  // namespace qie

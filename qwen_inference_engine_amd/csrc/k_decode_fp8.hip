@@ -15,7 +15,7 @@
 //   * the RMSNorm is fused: the block's waves together hold every row's whole K range, so
 //     the sum of squares is one wave reduction + one LDS exchange, and each wave
 //     normalises its own fragments in registers (no qie_rmsnorm launch in front; the norm
-//     weights are staged in LDS, the quotient is a Markstein step, see d8_rms_pair);
+//     weights are staged in LDS, the quotient is a Markstein step, see rms_pair);
 //   * weights: one 16-B buffer load per lane per 64-k unit (16 e4m3 codes of one row;
 //     lanes 16g..16g+15 = rows, g = k quarter), non-temporal, in half-tile steps with
 //     the next step always in flight (two register sets); one v_cvt_scalef32_pk_bf16_fp8 per code pair, two
@@ -65,27 +65,6 @@ struct Dec8Params {
     float* slab;
     unsigned* cnt;
 };
-
-// One bf16 pair of qie_rmsnorm's rms_apply8 (k_misc.hip, normalization.cu:18-23).
-// REF: x / rms as q = x * (1 / rms) plus one FMA residual step (Markstein) — the correctly
-// rounded quotient whenever nothing underflows, i.e. for every |x / rms| above 2^-100
-// (smaller non-zero activations may land 1 fp32 ulp off before the bf16 rounding); three
-// VALU ops instead of the ~10 of the IEEE division sequence, which made the fused prologue
-// VALU-bound (13 µs per launch at config 4).  rms = +inf enters as rr = 0, inv = 0, so the
-// quotient is 0 for finite x and NaN for infinite x, as the division gives.
-// HF: w * bf16(x * (1 / rms)).
-template <bool HF>
-__device__ __forceinline__ uint32_t d8_rms_pair(uint32_t xv, uint32_t wv, float rr, float inv) {
-#pragma clang fp contract(off)
-    const float a[2] = {bf_lo(xv), bf_hi(xv)}, w[2] = {bf_lo(wv), bf_hi(wv)};
-    float y[2];
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const float q = a[j] * inv;
-        y[j] = HF ? w[j] * rbf(q) : fmaf(fmaf(-q, rr, a[j]), inv, q) * w[j];
-    }
-    return pack2(y[0], y[1]);
-}
 
 // (split-K: two blocks per CU — at most 128 VGPRs; one block per CU ran the down projection
 // at 24.8 instead of 18.5 µs)
@@ -282,10 +261,10 @@ __global__ __launch_bounds__(KS * 64, SPL ? 4 : 1) void dec8_kernel(Dec8Params p
                 const float ij = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, inv), j));
                 const float rj = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, rr), j));
                 d8_u32x4 y;
-                y.x = d8_rms_pair<HF>(xc[j].x, nwv.x, rj, ij);
-                y.y = d8_rms_pair<HF>(xc[j].y, nwv.y, rj, ij);
-                y.z = d8_rms_pair<HF>(xc[j].z, nwv.z, rj, ij);
-                y.w = d8_rms_pair<HF>(xc[j].w, nwv.w, rj, ij);
+                y.x = rms_pair<HF>(xc[j].x, nwv.x, rj, ij);
+                y.y = rms_pair<HF>(xc[j].y, nwv.y, rj, ij);
+                y.z = rms_pair<HF>(xc[j].z, nwv.z, rj, ij);
+                y.w = rms_pair<HF>(xc[j].w, nwv.w, rj, ij);
                 *reinterpret_cast<d8_u32x4*>(xs + (int64_t)j * K + 8 * tid) = y;
             }
         };
@@ -329,10 +308,10 @@ __global__ __launch_bounds__(KS * 64, SPL ? 4 : 1) void dec8_kernel(Dec8Params p
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
                     const d8_u32x4 nv = nw_s[wave][8 * u + 2 * g + h];   // k = kw + 64 u + 16 g + 8 h
-                    av[u][h].x = d8_rms_pair<HF>(av[u][h].x, nv.x, rr, inv);
-                    av[u][h].y = d8_rms_pair<HF>(av[u][h].y, nv.y, rr, inv);
-                    av[u][h].z = d8_rms_pair<HF>(av[u][h].z, nv.z, rr, inv);
-                    av[u][h].w = d8_rms_pair<HF>(av[u][h].w, nv.w, rr, inv);
+                    av[u][h].x = rms_pair<HF>(av[u][h].x, nv.x, rr, inv);
+                    av[u][h].y = rms_pair<HF>(av[u][h].y, nv.y, rr, inv);
+                    av[u][h].z = rms_pair<HF>(av[u][h].z, nv.z, rr, inv);
+                    av[u][h].w = rms_pair<HF>(av[u][h].w, nv.w, rr, inv);
                     // one fragment at a time: left alone the scheduler hoists every
                     // product of the prologue first and spills
                     __builtin_amdgcn_sched_barrier(0);
@@ -685,10 +664,10 @@ __global__ __launch_bounds__(KS * 64) void dec8r_kernel(Dec8Params p) {
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
                     const d8_u32x4 nv = nw_s[wave][8 * u + 2 * g + h];
-                    av[u][h].x = d8_rms_pair<HF>(av[u][h].x, nv.x, rr, inv);
-                    av[u][h].y = d8_rms_pair<HF>(av[u][h].y, nv.y, rr, inv);
-                    av[u][h].z = d8_rms_pair<HF>(av[u][h].z, nv.z, rr, inv);
-                    av[u][h].w = d8_rms_pair<HF>(av[u][h].w, nv.w, rr, inv);
+                    av[u][h].x = rms_pair<HF>(av[u][h].x, nv.x, rr, inv);
+                    av[u][h].y = rms_pair<HF>(av[u][h].y, nv.y, rr, inv);
+                    av[u][h].z = rms_pair<HF>(av[u][h].z, nv.z, rr, inv);
+                    av[u][h].w = rms_pair<HF>(av[u][h].w, nv.w, rr, inv);
                     __builtin_amdgcn_sched_barrier(0);
                 }
         };

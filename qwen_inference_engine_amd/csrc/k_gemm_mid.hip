@@ -383,8 +383,7 @@ int gemm_mid(const qie_linear_args* a, const GemmParams& q, float other_us, hipS
     *launched = false;
     GemmParams p = q;
     p.vec = a->ldy % 4 == 0 && ((uintptr_t)a->y) % (a->epilogue == QIE_EPI_F32 ? 16 : 8) == 0;
-    // LDS-DMA moves 16-byte pieces of the weights' rows (x's rows are on that grid: qie_linear)
-    if (a->K % mid::BK != 0 || (((uintptr_t)a->w[0] | (uintptr_t)a->w[1] | (uintptr_t)a->w[2]) % 16) != 0) return 0;
+    if (a->K % mid::BK != 0) return 0;   // (rows of x and weights are on the 16-byte grid of LDS-DMA: qie_linear)
     const int64_t cols = a->epilogue == QIE_EPI_SWIGLU ? 2 * a->N : a->N;
     const MidPlan pl = mid_plan(a->M, cols, a->K, device_cu_count());
     if (pl.tile < 0 || pl.us >= 0.88f * other_us) return 0;   // 12 %: what the two fits are off by on long prompts

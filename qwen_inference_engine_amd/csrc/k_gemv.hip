@@ -1390,12 +1390,18 @@ int gemv_rope(const qie_linear_args* a, const int32_t* pos, const float* cs, con
 
 bool dec8_applies(const qie_linear_args* a);
 int dec8_linear(const qie_linear_args* a, hipStream_t st, bool* done);
+int dec_bf16_linear(const qie_linear_args* a, hipStream_t st, bool* done);
 
 int gemv(const qie_linear_args* a, hipStream_t st) {
     // fp8 weights, 2..16 rows, K a whole number of per-wave slices (or split-K): k_decode_fp8.hip
     if (dec8_applies(a)) {
         bool done = false;
         const int rc = dec8_linear(a, st, &done);
+        if (done) return rc;
+    }
+    {   // bf16 weights, 2..16 rows, K a multiple of 128: k_decode_bf16.hip
+        bool done = false;
+        const int rc = dec_bf16_linear(a, st, &done);
         if (done) return rc;
     }
     GemvParams p;

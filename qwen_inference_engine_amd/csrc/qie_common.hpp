@@ -242,6 +242,27 @@ __device__ __forceinline__ unsigned long long wave_max(unsigned long long v) {
     return v;
 }
 
+// One bf16 pair of qie_rmsnorm's rms_apply8 (k_misc.hip, normalization.cu:18-23).
+// REF: x / rms as q = x * (1 / rms) plus one FMA residual step (Markstein) — the correctly
+// rounded quotient whenever nothing underflows, i.e. for every |x / rms| above 2^-100
+// (smaller non-zero activations may land 1 fp32 ulp off before the bf16 rounding); three
+// VALU ops instead of the ~10 of the IEEE division sequence, which made the fused prologue
+// VALU-bound (13 µs per launch at config 4).  rms = +inf enters as rr = 0, inv = 0, so the
+// quotient is 0 for finite x and NaN for infinite x, as the division gives.
+// HF: w * bf16(x * (1 / rms)).
+template <bool HF>
+__device__ __forceinline__ uint32_t rms_pair(uint32_t xv, uint32_t wv, float rr, float inv) {
+#pragma clang fp contract(off)
+    const float a[2] = {bf_lo(xv), bf_hi(xv)}, w[2] = {bf_lo(wv), bf_hi(wv)};
+    float y[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const float q = a[j] * inv;
+        y[j] = HF ? w[j] * rbf(q) : fmaf(fmaf(-q, rr, a[j]), inv, q) * w[j];
+    }
+    return pack2(y[0], y[1]);
+}
+
 // Selection key of the reference's arg-max / top-k (logit_decode.cu:15-33,
 // 149-274): larger value wins; among equal values the winner maximises
 // bitrev8(idx mod 256), then minimises idx.  0 means "no candidate"
