@@ -8,12 +8,15 @@
 //     selection order (value, then bitrev8(idx mod 256), then -idx; see
 //     qie_common.hpp sel_key) — greedy is a parallel max over keys (also fused
 //     into the lm_head GEMV epilogue, k_gemv.hip);
-//   * top-k = per-4096-slice bitonic sort (LDS) + a merge sort of the slice
-//     winners; the sorted keys reproduce the reference's k rounds exactly;
-//   * softmax + draw on one lane with the reference's sequential order and a
-//     cuRAND-XORWOW restatement (curand_init(seed, 0, 0); curand_uniform).
+//   * top-k = a radix selection per 4096-slice, one over the slices' winners, and a sort of
+//     the k that are left; the sorted keys reproduce the reference's k rounds exactly;
+//   * softmax + draw in one wave: exponentials a lane each, sums in the reference's
+//     sequential order lane by lane, and a cuRAND-XORWOW restatement (curand_init(seed, 0, 0);
+//     curand_uniform).
 #include "qie_common.hpp"
 #include "../../include/qie/qie_ops.h"
+
+#include <algorithm>
 
 namespace qie {
 
@@ -67,21 +70,93 @@ __device__ void bitonic_desc(unsigned long long* k, int n) {
     }
 }
 
+// The k largest of a block's keys (KPT a thread, in registers), unordered, into out[0, k) (LDS or memory; zeros behind the
+// last where fewer than k keys are non-zero).  Radix selection from the top byte: a histogram of the keys that still share the
+// threshold's prefix, until the bin of the k-th holds just what is needed: three to six passes of about 1.5 us where the
+// bitonic sort of 4,096 keys makes 78.  (Bits 47..32 are the low half of a bf16's fp32 pattern: known from its sign.)
+template <int KPT>
+__device__ void radix_top(const unsigned long long (&key)[KPT], int k, unsigned long long* out) {
+    __shared__ unsigned hist[256];
+    __shared__ unsigned pick[3];   // digit, keys above it, keys in it
+    __shared__ unsigned n_out;
+    unsigned long long prefix = 0ull, mask = 0ull;
+    int need = k;
+    for (int shift = 56; shift >= 0; shift -= 8) {
+        if (shift == 40) {
+            const unsigned hi = (unsigned)(prefix >> 48);
+            prefix |= (hi != 0 && !(hi & 0x8000u)) ? 0xffffull << 32 : 0ull;
+            mask |= 0xffffull << 32;
+            shift = 24;
+        }
+        hist[threadIdx.x] = 0u;   // 256 threads
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < KPT; i++)
+            if ((key[i] & mask) == prefix) atomicAdd(&hist[(key[i] >> shift) & 255], 1u);
+        __syncthreads();
+        if (threadIdx.x < 64) {   // lane l holds the bins 255 - 4 l .. 252 - 4 l: counts above them by a scan over the lanes
+            const int l = threadIdx.x;
+            unsigned c[4], own = 0u;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                c[j] = hist[255 - 4 * l - j];
+                own += c[j];
+            }
+            unsigned upto = own;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const unsigned t = __shfl_up(upto, o, 64);
+                if (l >= o) upto += t;
+            }
+            unsigned above = upto - own;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if (above < (unsigned)need && above + c[j] >= (unsigned)need) {   // one bin of one lane
+                    pick[0] = (unsigned)(255 - 4 * l - j);
+                    pick[1] = above;
+                    pick[2] = c[j];
+                }
+                above += c[j];
+            }
+        }
+        __syncthreads();
+        prefix |= (unsigned long long)pick[0] << shift;
+        mask |= 255ull << shift;
+        need -= (int)pick[1];
+        const bool done = pick[2] == (unsigned)need;
+        __syncthreads();
+        if (done) break;   // block-uniform
+    }
+    if (threadIdx.x == 0) n_out = 0u;
+    for (int i = threadIdx.x; i < k; i += 256) out[i] = 0ull;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < KPT; i++)
+        if (key[i] != 0ull && (key[i] & mask) >= prefix) out[atomicAdd(&n_out, 1u)] = key[i];
+    __syncthreads();
+}
+
 __global__ __launch_bounds__(256) void topk_slice_kernel(const uint16_t* __restrict__ logits, int64_t V,
                                                          int64_t ld, int k,
                                                          unsigned long long* __restrict__ cand) {
-    __shared__ unsigned long long keys[kSlice];
+    constexpr int KPT = kSlice / 256;
     const int64_t m = blockIdx.y;
     const int64_t base = (int64_t)blockIdx.x * kSlice;
     const uint16_t* row = logits + m * ld;
-    for (int i = threadIdx.x; i < kSlice; i += 256) {
-        const int64_t idx = base + i;
-        keys[i] = idx < V ? sel_key(bf2f(row[idx]), (uint32_t)idx) : 0ull;
+    unsigned long long key[KPT];
+    uint16_t v[KPT];
+#pragma unroll
+    for (int i = 0; i < KPT; i++) {
+        const int64_t idx = base + threadIdx.x + 256 * i;
+        v[i] = row[idx < V ? idx : V - 1];
     }
-    __syncthreads();
-    bitonic_desc(keys, kSlice);
-    unsigned long long* out = cand + (m * gridDim.x + blockIdx.x) * (int64_t)k;
-    for (int i = threadIdx.x; i < k; i += 256) out[i] = keys[i];
+#pragma unroll
+    for (int i = 0; i < KPT; i++) {
+        const int64_t idx = base + threadIdx.x + 256 * i;
+        key[i] = idx < V ? sel_key(bf2f(v[i]), (uint32_t)idx) : 0ull;
+    }
+    // (at least k keys: k <= kMaxTopK <= kSlice)
+    radix_top<KPT>(key, k, cand + (m * gridDim.x + blockIdx.x) * (int64_t)k);
 }
 
 // cuRAND XORWOW, curand_init(seed, subsequence = 0, offset = 0) (no skip-ahead)
@@ -100,56 +175,75 @@ __device__ __forceinline__ float xorwow_uniform_first(uint64_t seed) {
     return x * 2.3283064e-10f + (2.3283064e-10f / 2.0f);
 }
 
+// One block per row: the k best of the slices' candidates, sorted, then temperature, softmax and one draw
+// (logit_decode.cu:225-272) by one wave that holds candidate i in lane i % 64: the exponentials side by side, the sums in the
+// reference's order.  k2: the power of two >= max(k, 2).
+template <int KPT>
 __global__ __launch_bounds__(256) void topk_merge_sample_kernel(const unsigned long long* __restrict__ cand,
-                                                                int nb, int k, int n2, float temperature,
+                                                                int nb, int k, int k2, float temperature,
                                                                 float top_p, uint64_t seed,
                                                                 const int32_t* step, int32_t* ids) {
 #pragma clang fp contract(off)
-    extern __shared__ __attribute__((aligned(16))) unsigned long long sk[];
+    __shared__ unsigned long long sk[kMaxTopK];
     const int64_t m = blockIdx.x;
     const int total = nb * k;
-    for (int i = threadIdx.x; i < n2; i += 256) sk[i] = i < total ? cand[m * total + i] : 0ull;
+    unsigned long long key[KPT];
+#pragma unroll
+    for (int i = 0; i < KPT; i++) {
+        const int j = threadIdx.x + 256 * i;
+        const unsigned long long c = cand[m * total + (j < total ? j : total - 1)];
+        key[i] = j < total ? c : 0ull;
+    }
+    for (int i = threadIdx.x; i < k2; i += 256) sk[i] = 0ull;
     __syncthreads();
-    bitonic_desc(sk, n2);
-    if (threadIdx.x != 0) return;
-    // logit_decode.cu:225-272 (thread 0): temperature, softmax, one draw.
+    radix_top<KPT>(key, k, sk);
+    bitonic_desc(sk, k2);
+    if (threadIdx.x >= 64) return;
+    const int lane = threadIdx.x;
+    constexpr int J = kMaxTopK / 64;
     int n = 0;
-    while (n < k && sk[n] != 0ull) n++;
-    if (n == 0) { ids[m] = -1; return; }
-    float vals[kMaxTopK];
-    float T = temperature > 0.0f ? temperature : 1.0f;
-    float max_val = key_val(sk[0]) / T;
-    for (int i = 1; i < n; i++) {
-        float v = key_val(sk[i]) / T;
-        if (v > max_val) max_val = v;
-        vals[i] = v;
+    float e[J];
+    const float T = temperature > 0.0f ? temperature : 1.0f;
+    const float max_val = key_val(sk[0]) / T;   // the keys are sorted by value
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        const int i = 64 * j + lane;
+        const unsigned long long c = i < k ? sk[i] : 0ull;
+        n += __popcll(__ballot(c != 0ull));
+        e[j] = c != 0ull ? expf(key_val(c) / T - max_val) : 0.f;
     }
-    vals[0] = key_val(sk[0]) / T;
+    if (n == 0) {
+        if (lane == 0) ids[m] = -1;
+        return;
+    }
+    auto at = [&](int i) {   // candidate i's weight (i uniform)
+        float v = e[0];
+#pragma unroll
+        for (int j = 1; j < J; j++) v = i >= 64 * j ? e[j] : v;
+        return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), i & 63));
+    };
     float sum = 0.0f;
-    for (int i = 0; i < n; i++) {
-        vals[i] = expf(vals[i] - max_val);
-        sum += vals[i];
-    }
+    for (int i = 0; i < n; i++) sum += at(i);
     if (top_p > 0.0f && top_p < 1.0f) {
         float cum = 0.0f;
         int keep = n;
         for (int i = 0; i < n; i++) {
-            cum += vals[i];
+            cum += at(i);
             if (cum >= top_p * sum) { keep = i + 1; break; }
         }
         n = keep;
         sum = 0.0f;
-        for (int i = 0; i < n; i++) sum += vals[i];
+        for (int i = 0; i < n; i++) sum += at(i);
     }
     const uint64_t sd = seed + (step ? (uint64_t)(int64_t)step[m] : 0ull);
     float u = xorwow_uniform_first(sd) * sum;
     float cum = 0.0f;
-    int picked = key_idx(sk[n - 1]);
+    int picked = n - 1;
     for (int i = 0; i < n; i++) {
-        cum += vals[i];
-        if (u <= cum) { picked = key_idx(sk[i]); break; }
+        cum += at(i);
+        if (u <= cum) { picked = i; break; }
     }
-    ids[m] = picked;
+    if (lane == 0) ids[m] = key_idx(sk[picked]);
 }
 
 static int pow2_at_least(int x) {
@@ -200,18 +294,11 @@ int qie_sample(const void* logits, int64_t M, int64_t V, int64_t ld, const qie_s
     hipLaunchKernelGGL(topk_slice_kernel, dim3(nb, (unsigned)M), dim3(256), 0, st,
                        (const uint16_t*)logits, V, ld, k, cand);
     QIE_LAUNCH_CHECK();
-    const int n2 = pow2_at_least(nb * k);
-    const size_t shm = (size_t)n2 * 8;
-    QIE_REQUIRE(shm <= 160 * 1024, "qie_sample: top-k merge exceeds LDS (V=%lld k=%d)", (long long)V, k);
-    if (shm > 65536) {
-        static bool raised = false;
-        if (!raised) {
-            QIE_HIP(hipFuncSetAttribute((const void*)topk_merge_sample_kernel,
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-            raised = true;
-        }
-    }
-    hipLaunchKernelGGL(topk_merge_sample_kernel, dim3((unsigned)M), dim3(256), shm, st, cand, nb, k, n2,
+    const int total = nb * k;
+    QIE_REQUIRE(pow2_at_least(total) <= 64 * 256, "qie_sample: top-k merge exceeds LDS (V=%lld k=%d)", (long long)V, k);
+    const auto fn = total <= 8 * 256 ? topk_merge_sample_kernel<8> : total <= 40 * 256 ? topk_merge_sample_kernel<40>
+                                                                                       : topk_merge_sample_kernel<64>;
+    hipLaunchKernelGGL(fn, dim3((unsigned)M), dim3(256), 0, st, cand, nb, k, std::max(2, pow2_at_least(k)),
                        s->temperature, s->top_p, (uint64_t)s->seed, step_dev, out_ids);
     QIE_LAUNCH_CHECK();
     return 0;
