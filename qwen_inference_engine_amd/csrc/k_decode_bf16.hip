@@ -14,6 +14,7 @@
 // One workgroup a CU: LDS holds 64 to 128 KB of chunks.  Sums: per wave over its K share in fp32, the shares in wave order.
 #include "qie_common.hpp"
 #include "../../include/qie/qie_ops.h"
+#include "k_layered.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -56,7 +57,9 @@ __device__ __forceinline__ void db_glds16(const void* src, void* lds) {
 
 // XM: 0 = X in LDS; 8, 16 = X's chunks (of 8 or 16 rows) through the ring.  NV: 16-byte vectors of a row per lane while X is
 // normed (K <= 512 NV); R: ring slots a wave.
-template <int EPI, int XM, int NV, int R>
+// F32: rows of fp32 instead (p.K, p.ldx in 16-bit units; the fp32 epilogue, no norm): a 16-byte piece is 4 k, four
+// v_mfma_f32_16x16x4f32 instead of one v_mfma_f32_16x16x32_bf16.
+template <int EPI, int XM, int NV, int R, bool F32 = false>
 __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
 #pragma clang fp contract(off)
     constexpr int SLOT = db::WCH + XM * 256;
@@ -225,7 +228,15 @@ __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
                     xf[s] = *reinterpret_cast<const db_bf16x8*>(buf + db::WCH + (fr & (XM - 1)) * 256 + (((4 * s + g) ^ (fr & (XM - 1))) * 16));
             }
 #pragma unroll
-            for (int s = 0; s < 4; s++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[s], xf[s], acc, 0, 0, 0);
+            for (int s = 0; s < 4; s++) {
+                if constexpr (F32) {
+                    const db_f32x4 a = __builtin_bit_cast(db_f32x4, wf[s]), b = __builtin_bit_cast(db_f32x4, xf[s]);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], acc, 0, 0, 0);
+                } else {
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[s], xf[s], acc, 0, 0, 0);
+                }
+            }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the slot's reads are done
             __builtin_amdgcn_sched_barrier(0);
             if (done + R < items) issue();
@@ -369,16 +380,16 @@ bool db_plan(const qie_linear_args* a, DbPlan* out) {
     return true;
 }
 
-template <int EPI, int XM, int NV, int R>
+template <int EPI, int XM, int NV, int R, bool F32 = false>
 int db_launch(const DecBfParams& p, size_t lds, hipStream_t st) {
-    const void* fn = (const void*)dec_bf16_kernel<EPI, XM, NV, R>;
+    const void* fn = (const void*)dec_bf16_kernel<EPI, XM, NV, R, F32>;
     static bool raised = false;
     if (!raised) {
         QIE_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDbLds));
         raised = true;
     }
     const int grid = std::max(1, std::min(p.n_tiles, (int)device_cu_count()));
-    hipLaunchKernelGGL((dec_bf16_kernel<EPI, XM, NV, R>), dim3((unsigned)grid), dim3(512), lds, st, p);
+    hipLaunchKernelGGL((dec_bf16_kernel<EPI, XM, NV, R, F32>), dim3((unsigned)grid), dim3(512), lds, st, p);
     QIE_LAUNCH_CHECK();
     return 0;
 }
@@ -439,6 +450,31 @@ int dec_bf16_linear(const qie_linear_args* a, hipStream_t st, bool* done) {
         case QIE_EPI_F32: return db_launch_plan<QIE_EPI_F32>(p, pl, st);
         default: return db_launch_plan<QIE_EPI_STORE>(p, pl, st);
     }
+}
+
+// y = X W^T in fp32 for up to 16 rows (lay::linear's plain form): *done false: not its shape
+int dec_f32_linear(const lay::LinearP& q, hipStream_t st, bool* done) {
+    *done = q.batch == 1 && !q.grp_off && !q.round_a && q.M <= 16 && q.K % 64 == 0 && q.K >= 256 && q.ldw == q.K && q.lda % 4 == 0 &&
+            (((uintptr_t)q.A | (uintptr_t)q.W) % 16) == 0;
+    if (!*done) return 0;
+    DecBfParams p{};
+    p.x = (const uint16_t*)q.A;
+    p.ldx = q.lda * 2;
+    p.w[0] = (const uint16_t*)q.W;
+    p.n0 = p.n01 = q.N;
+    p.K = q.K * 2;
+    p.N = q.N;
+    p.M = q.M;
+    p.n_tiles = (q.N + 15) / 16;
+    p.y = (uint16_t*)q.Y;
+    p.ldy = q.ldy;
+    p.vec = q.ldy % 4 == 0 && ((uintptr_t)q.Y) % 16 == 0;
+    p.xstride = p.K * 2 + 16;
+    constexpr int E = QIE_EPI_F32;
+    if (p.K <= 5120 && db_image_bytes(p.M, p.K, 2) <= kDbLds) return db_launch<E, 0, 10, 2, true>(p, (size_t)db_image_bytes(p.M, p.K, 2), st);
+    const int xm = p.M <= 8 ? 8 : 16;
+    const size_t lds = (size_t)(db::NW * 2 * (db::WCH + xm * 256) + db_red_bytes(p.M));
+    return xm == 8 ? db_launch<E, 8, 1, 2, true>(p, lds, st) : db_launch<E, 16, 1, 2, true>(p, lds, st);
 }
 
 }  // namespace qie

@@ -22,6 +22,7 @@
 #include "k_layered.hpp"
 
 namespace qie {
+int dec_f32_linear(const lay::LinearP& q, hipStream_t st, bool* done);   // k_decode_bf16.hip
 namespace lay {
 
 template <typename T> __device__ __forceinline__ float ldf(const T* p, int64_t i);
@@ -241,6 +242,13 @@ static bool al16p(const void* q) { return ((uintptr_t)q & 15) == 0; }
 int linear(const LinearP& p, bool w_f32, hipStream_t st) {
     QIE_REQUIRE(p.A && p.W && p.Y && p.M > 0 && p.N > 0 && p.K > 0 && p.batch > 0, "layered linear: bad arguments");
     const bool a_vec = p.lda % 4 == 0 && p.sA % 4 == 0 && al16p(p.A);
+    if (w_f32 && dev_env("QIE_LIN_F32", 1)) {   // fp32 on the matrix cores: k_decode_bf16.hip (up to 16 rows), k_linear_f32.hip
+        bool done = false;
+        int rc = dec_f32_linear(p, st, &done);
+        if (done) return rc;
+        rc = linear_f32(p, st, &done);
+        if (done) return rc;
+    }
     if (p.M <= 32) {
         const bool vec = a_vec && p.K % 8 == 0 && p.ldw % 8 == 0 && p.sW % 8 == 0 && al16p(p.W);
         dim3 grid((unsigned)((p.N + 3) / 4), (unsigned)((p.M + 15) / 16), (unsigned)p.batch);

@@ -27,6 +27,8 @@ struct LinearP {
     int mfma;   // bf16 weights, many rows: the direct MFMA kernel may take the product (batched / grouped forms)
 };
 int linear(const LinearP& p, bool w_f32, hipStream_t st);
+// k_linear_f32.hip: fp32 operands, more than 16 rows, on the fp32 matrix cores; *done false: not its shape
+int linear_f32(const LinearP& p, hipStream_t st, bool* done);
 
 // Paged latent cache: page p at pool + p * page_stride elements; inside a page the rows of one
 // caching layer start at layer_off and are D = R + rot wide: [c (R) | rotated shared key (rot)].

@@ -1,0 +1,205 @@
+// k_linear_f32.hip — fp32 products of more than a handful of rows for the layered models' fp32 engine.
+//
+//   Y[m, n] = sum_k A[m, k] W[n, k], plain, per head (batch) or per expert (grp_off: rows by group), on the fp32 matrix cores
+//   (v_mfma_f32_16x16x4f32: fp32 products and sums).
+//
+// The FMA kernel it replaces (k_layered.hip linear_kernel) keeps nothing in flight and fills 32 to 80 of 256 CUs at a few
+// hundred rows: 145 to 230 us for 1 to 2 GFLOP.  Here a 64 x 64 tile goes through an LDS-DMA ring of 32-k tiles (128-byte rows,
+// as k_gemm_mid.hip), 8 waves as 2 x 2 x 2 K halves, and tiles that do not fill the chip are split over K (slabs summed in part
+// order by the last part, gemm8_kernel's protocol).  Bound: the fp32 matrix rate (157 TFLOP/s) or, at few rows, the weights.
+#include "gemm_impl.hpp"
+#include "k_layered.hpp"
+
+#include <algorithm>
+
+namespace qie {
+namespace lay {
+
+namespace lf {
+constexpr int BM = 64, BN = 64, BK = 32, SLOTS = 4;
+constexpr int SLOT = (BM + BN) * BK * 4;   // A rows, then W rows, 128 B each
+}
+
+struct LinF32P {
+    LinearP q;
+    int parts;          // K ranges per tile
+    int n_nt, n_mt;     // tiles of N; tiles of M per group (of the most rows a group may have)
+    int vec;            // rows of Y take 16-byte stores
+    float* slab;        // [tile][part][64 * 64]
+    unsigned* cnt;      // [tile], zero at rest
+};
+
+__global__ __launch_bounds__(512) void linear_f32_kernel(LinF32P p) {
+#pragma clang fp contract(off)
+    using namespace lf;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wk = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+    const int fr = lane & 15, g = lane >> 4;
+    const int z = blockIdx.z, nt = blockIdx.x % p.n_nt, part = blockIdx.x / p.n_nt, mt = blockIdx.y;
+    int m_lo = 0, m_hi = p.q.M;
+    if (p.q.grp_off) {
+        m_lo = p.q.grp_off[z];
+        m_hi = p.q.grp_off[z + 1];
+    }
+    const int m0 = m_lo + mt * BM, n0 = nt * BN;
+    if (m0 >= m_hi) return;   // block-uniform
+    const float* A = p.q.A + (int64_t)z * p.q.sA;
+    const float* W = (const float*)p.q.W + (int64_t)z * p.q.sW;
+    const int nk_all = p.q.K / BK;
+    const int kb = (int)((int64_t)part * nk_all / p.parts), nk = (int)((int64_t)(part + 1) * nk_all / p.parts) - kb;
+
+    // LDS-DMA: instruction i of this wave fills rows 8 b .. 8 b + 7, b = 8 i + wave (i = 0: A, 1: W)
+    const float* src[2];
+    {
+        const int r = 8 * wave + (lane >> 3), cs = (lane & 7) ^ g8_swz(r);
+        const int ar = m0 + r < m_hi ? m0 + r : m_hi - 1;         // rows past the group: its last again, never stored
+        const int wr = n0 + r < p.q.N ? n0 + r : p.q.N - 1;
+        src[0] = A + (int64_t)ar * p.q.lda + (int64_t)kb * BK + cs * 4;
+        src[1] = W + (int64_t)wr * p.q.ldw + (int64_t)kb * BK + ((lane & 7) ^ g8_swz(BM + r)) * 4;
+    }
+    auto stage = [&](int kt, int slot) {
+        unsigned char* dst = smem + slot * SLOT + wave * 1024;
+        glds16(src[0] + (int64_t)kt * BK, dst);
+        glds16(src[1] + (int64_t)kt * BK, dst + 8192);
+    };
+    f32x4 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < SLOTS - 1 && t < nk; t++) stage(t, t);
+    int slot = 0, fill = SLOTS - 1;
+    for (int t = 0; t < nk; t++) {
+        if (t + SLOTS - 1 <= nk) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (SLOTS - 2)) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        if (t + SLOTS - 1 < nk) stage(t + SLOTS - 1, fill);
+        const unsigned char* buf = smem + slot * SLOT;
+        // this K half: 16 k as four pieces; element e of piece 4 wk + g is k = 4 (4 wk + g) + e in both operands
+        f32x4 fa[2], fb[2];
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int row = BM + wn * 32 + j * 16 + fr;
+            fb[j] = *reinterpret_cast<const f32x4*>(buf + row * 128 + (((4 * wk + g) ^ g8_swz(row)) * 16));
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int row = wm * 32 + i * 16 + fr;
+            fa[i] = *reinterpret_cast<const f32x4*>(buf + row * 128 + (((4 * wk + g) ^ g8_swz(row)) * 16));
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[j][e], fa[i][e], acc[i][j], 0, 0, 0);   // W Aᵀ
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        slot = slot + 1 == SLOTS ? 0 : slot + 1;
+        fill = fill + 1 == SLOTS ? 0 : fill + 1;
+    }
+    // the two K halves: wave w and w ^ 4 hold the same tile, each keeps one of its two row fragments
+    f32x4 res[2];
+    {
+        f32x4* ex = reinterpret_cast<f32x4*>(smem);
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            ex[(wave * 2 + j) * 64 + lane] = wk == 0 ? acc[1][j] : acc[0][j];
+            res[j] = wk == 0 ? acc[0][j] : acc[1][j];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const f32x4 o = ex[((wave ^ 4) * 2 + j) * 64 + lane];
+            res[j] = wk == 0 ? res[j] + o : o + res[j];
+        }
+    }
+    if (p.parts > 1) {
+        const int64_t tile = ((int64_t)z * p.n_mt + mt) * p.n_nt + nt;
+        const auto rs = __builtin_amdgcn_make_buffer_rsrc(p.slab + (tile * p.parts + part) * 4096, (short)0, 16384, 0x00020000);
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_g8, res[j]), rs, ((wave * 2 + j) * 64 + lane) * 16, 0, 16);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        int* flag = reinterpret_cast<int*>(smem);
+        if (tid == 0) {
+            const unsigned old = __hip_atomic_fetch_add(p.cnt + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            *flag = old == (unsigned)p.parts - 1 ? 1 : 0;
+        }
+        __syncthreads();
+        if (*flag == 0) return;   // uniform
+        constexpr int QN = 8;     // parts in flight
+        for (int q0 = 0; q0 < p.parts; q0 += QN) {
+            f32x4 v[QN][2];
+#pragma unroll
+            for (int u = 0; u < QN; u++) {
+                const int q = q0 + u < p.parts ? q0 + u : p.parts - 1;
+                const auto rq = __builtin_amdgcn_make_buffer_rsrc(p.slab + (tile * p.parts + q) * 4096, (short)0, 16384, 0x00020000);
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    v[u][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rq, ((wave * 2 + j) * 64 + lane) * 16, 0, 16));
+            }
+#pragma unroll
+            for (int u = 0; u < QN; u++) {
+                if (q0 + u >= p.parts) break;
+#pragma unroll
+                for (int j = 0; j < 2; j++) res[j] = q0 + u == 0 ? v[u][j] : res[j] + v[u][j];
+            }
+        }
+        if (tid == 0) __hip_atomic_store(p.cnt + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    const int m = m0 + wm * 32 + wk * 16 + fr;
+    if (m >= m_hi) return;
+    float* Y = p.q.Y + (int64_t)z * p.q.sY + (int64_t)m * p.q.ldy;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int n = n0 + wn * 32 + j * 16 + 4 * g;
+        if (p.vec && n + 4 <= p.q.N) {
+            *reinterpret_cast<f32x4*>(Y + n) = res[j];
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (n + r < p.q.N) Y[n + r] = res[j][r];
+        }
+    }
+}
+
+int linear_f32(const LinearP& q, hipStream_t st, bool* done) {
+    using namespace lf;
+    const int64_t a16 = (uintptr_t)q.A % 16 + (uintptr_t)q.W % 16;
+    *done = !q.round_a && q.M > 16 && (!q.grp_off || q.M > 32) && q.K % BK == 0 && q.lda % 4 == 0 && q.ldw % 4 == 0 && q.sA % 4 == 0 &&
+            q.sW % 4 == 0 && a16 == 0;
+    if (!*done) return 0;
+    LinF32P p{};
+    p.q = q;
+    p.n_nt = (q.N + BN - 1) / BN;
+    p.n_mt = (q.M + BM - 1) / BM;   // (grouped: one group may hold every row; the other groups' blocks leave at once)
+    p.vec = q.ldy % 4 == 0 && q.sY % 4 == 0 && (uintptr_t)q.Y % 16 == 0;
+    // K ranges: until about 512 workgroups (two a CU) have work, each keeping 4 k-tiles.  Grouped: rows spread over the groups
+    const int64_t mts = q.grp_off ? std::max<int64_t>(q.batch, (q.M + BM - 1) / BM + q.batch / 2) : (int64_t)p.n_mt * q.batch;
+    const int64_t tiles = (int64_t)p.n_nt * p.n_mt * q.batch;   // of the grid
+    int parts = (int)std::max<int64_t>(1, std::min<int64_t>({16, 2 * (int64_t)device_cu_count() / (mts * p.n_nt), q.K / BK / 4}));
+    if (parts > 1) {
+        G8Split ws{1, nullptr, nullptr};
+        const int64_t slabs = (tiles * parts * 4096 + 65535) / 65536;
+        if (tiles > (1 << 20) || slabs > 2048 || g8_workspace(st, (int)slabs, (int)tiles, &ws) != 0) parts = 1;   // 512 MB at most
+        p.slab = ws.slab;
+        p.cnt = ws.cnt;
+    }
+    p.parts = parts;
+    constexpr size_t shm = (size_t)SLOTS * SLOT;
+    static_assert(shm <= 65536, "linear_f32: default LDS");
+    hipLaunchKernelGGL(linear_f32_kernel, dim3((unsigned)(p.n_nt * parts), (unsigned)p.n_mt, (unsigned)q.batch), dim3(512), shm, st, p);
+    QIE_LAUNCH_CHECK();
+    return 0;
+}
+
+}  // namespace lay
+}  // namespace qie
