@@ -334,7 +334,10 @@ int gqa_post(const GqaPostP& p, bool cache_f32, int T, hipStream_t st) {
 
 // ------------------------------------------------------------------ attention, exact form
 // One block per (head, row): the visible keys go through in chunks of GA_CHUNK with a running
-// maximum and sum; a wave scores a key, a thread owns value coordinates.
+// maximum and sum.  16 lanes score a key (16 bytes of it each at a time where its rows are on that
+// grid), four keys' loads in flight a lane; then the waves take every fourth key's value row, a lane
+// per coordinate, and their sums meet at the end.  (A wave per key and a thread per coordinate over
+// all keys, one load behind the other: 97 us for 3 rows of 16 heads over 160 keys of 64 in fp32.)
 constexpr int GA_CHUNK = 256;
 constexpr int GA_MAXV = 4;   // vdim <= 256 * GA_MAXV
 
@@ -344,19 +347,28 @@ __device__ __forceinline__ int first_visible(int mask, int size, int pos) {
     return 0;
 }
 
+__device__ __forceinline__ float4 key4(const float* p) { return *reinterpret_cast<const float4*>(p); }
+__device__ __forceinline__ float4 key4(const uint16_t* p) {
+    const uint2 u = *reinterpret_cast<const uint2*>(p);
+    return make_float4(bf_lo(u.x), bf_hi(u.x), bf_lo(u.y), bf_hi(u.y));
+}
+
 template <typename TC>
 __global__ __launch_bounds__(256) void gqa_attention_kernel(GqaAttnP p) {
-    extern __shared__ float sm[];
+    constexpr int VC = 4 * GA_MAXV, KU = 4;
+    extern __shared__ __attribute__((aligned(16))) float sm[];
+    const int dimp = (p.dim + 3) & ~3;
     float* q = sm;                 // [dim]
-    float* sc = sm + p.dim;        // [GA_CHUNK]
-    float* ob = sc + GA_CHUNK;     // [vdim]
+    float* sc = sm + dimp;         // [GA_CHUNK]
+    float* ob = sc + GA_CHUNK;     // [4][vdim]
     __shared__ float red[4];
+    __shared__ int64_t kbase[GA_CHUNK];   // a key's page, elements into the pool
+    __shared__ int ktok[GA_CHUNK];        // its token in the page
     const int h = blockIdx.x, t = blockIdx.y, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int slot = p.row_slot[t], pos = p.row_pos[t];
-    const int dim = p.dim, vdim = p.vdim, G = p.kv_heads, g = h / (p.heads / G);
+    const int dim = p.dim, vdim = p.vdim, G = p.kv_heads, g = h / (p.heads / G), PT = p.cache.page_tokens;
     const float* qr = p.proj + (int64_t)t * p.ld + p.q_col + h * dim;
     for (int i = tid; i < dim; i += 256) q[i] = qr[i];
-    __syncthreads();
     const int lo = first_visible(p.mask, p.mask_size, pos);
     const float b1 = p.r1 ? p.r1[h] : 0.f, b2 = p.r1 ? p.r2[h] : 0.f;
     const float slope = p.slopes ? p.slopes[h] : 0.f;
@@ -364,87 +376,112 @@ __global__ __launch_bounds__(256) void gqa_attention_kernel(GqaAttnP p) {
     const float pbh = sig ? p.pb[h] : 0.f;
     // a sink is a score without key or value: the running maximum and sum start from it
     float m_run = p.sink ? p.sink[h] : -INFINITY, l_run = p.sink ? 1.f : 0.f;
-    float acc[GA_MAXV] = {};
+    float acc[VC] = {};
     // the visible keys in order: the kept first ones that lie before the window, then the window's
     const int kept = min(p.mask_keep, lo), n_vis = kept + pos + 1 - lo;
     auto key_of = [&](int i) { return i < kept ? i : lo + i - kept; };
+    const TC* pool = (const TC*)p.cache.pool;
+    // a key's row on the grid of four elements
+    const bool vec = dim % 4 == 0 && p.k_off % 4 == 0 && p.cache.page_stride % 4 == 0 && ((uintptr_t)pool) % 16 == 0;
+    const int gl = tid & 15, gi = tid >> 4;
     for (int j0 = 0; j0 < n_vis; j0 += GA_CHUNK) {
         const int nk = min(GA_CHUNK, n_vis - j0);
-        for (int jj = wave; jj < nk; jj += 4) {
-            const int j = key_of(j0 + jj);
-            const TC* k = (const TC*)p.cache.pool + page_base(p.cache, slot, j) + p.k_off +
-                          ((int64_t)(j % p.cache.page_tokens) * G + g) * dim;
-            float s = 0.f;
-            for (int i = lane; i < dim; i += 64) s = fmaf(q[i], ldc<TC>(k, i), s);
-            s = wsum(s);
-            if (lane == 0) {
-                s *= p.scale;
-                if (p.softcap > 0.f) s = p.softcap * tanhf(s / p.softcap);
-                if (p.r1) s -= b1 * log1pf(b2 * (float)(pos - j));
-                if (p.slopes) s -= slope * (float)(pos - j);
-                sc[jj] = sig ? 1.0f / (1.0f + expf(-(s + pbh))) : s;
-            }
+        __syncthreads();   // q is there; the chunk before is done with
+        if (tid < nk) {
+            const int j = key_of(j0 + tid);
+            kbase[tid] = page_base(p.cache, slot, j);
+            ktok[tid] = j % PT;
         }
         __syncthreads();
-        if (sig) {   // the weights are final: no running maximum, no normalisation
-            for (int jj = 0; jj < nk; jj++) {
-                const int j = key_of(j0 + jj);
-                const int pt = j % p.cache.page_tokens;
-                const TC* v = (const TC*)p.cache.pool + page_base(p.cache, slot, j) + p.v_off;
-                const float w = sc[jj];
+        for (int jb = 0; jb < nk; jb += 16 * KU) {   // (uniform: every lane takes part in the sums over 16 lanes)
+            float s[KU];
 #pragma unroll
-                for (int i = 0; i < GA_MAXV; i++) {
-                    const int r = tid + i * 256;
-                    if (r < vdim)
-                        acc[i] = fmaf(w, ldc<TC>(v, p.v_transposed ? ((int64_t)g * vdim + r) * p.cache.page_tokens + pt
-                                                                     : ((int64_t)pt * G + g) * vdim + r), acc[i]);
+            for (int u = 0; u < KU; u++) {
+                const int jj = min(jb + 16 * u + gi, nk - 1);
+                const TC* k = pool + kbase[jj] + p.k_off + ((int64_t)ktok[jj] * G + g) * dim;
+                s[u] = 0.f;
+                if (vec) {
+                    for (int i = 4 * gl; i < dim; i += 64) {
+                        const float4 kv = key4(k + i), qv = key4(q + i);
+                        s[u] = fmaf(qv.x, kv.x, fmaf(qv.y, kv.y, fmaf(qv.z, kv.z, fmaf(qv.w, kv.w, s[u]))));
+                    }
+                } else {
+                    for (int i = gl; i < dim; i += 16) s[u] = fmaf(q[i], ldc<TC>(k, i), s[u]);
                 }
             }
-            __syncthreads();
-            continue;
-        }
-        float mx = -INFINITY;
-        for (int jj = tid; jj < nk; jj += 256) mx = fmaxf(mx, sc[jj]);
-        mx = wmax(mx);
-        if (lane == 0) red[wave] = mx;
-        __syncthreads();
-        mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-        const float m_new = fmaxf(m_run, mx);
-        const float alpha = expf(m_run - m_new);   // 0 on the first chunk
-        __syncthreads();
-        float ls = 0.f;
-        for (int jj = tid; jj < nk; jj += 256) {
-            const float e = expf(sc[jj] - m_new);
-            sc[jj] = e;
-            ls += e;
-        }
-        ls = bsum256(ls, red);
-        l_run = l_run * alpha + ls;
-        m_run = m_new;
 #pragma unroll
-        for (int i = 0; i < GA_MAXV; i++) acc[i] *= alpha;
-        for (int jj = 0; jj < nk; jj++) {
-            const int j = key_of(j0 + jj);
-            const int pt = j % p.cache.page_tokens;
-            const TC* v = (const TC*)p.cache.pool + page_base(p.cache, slot, j) + p.v_off;
-            const float w = sc[jj];
-#pragma unroll
-            for (int i = 0; i < GA_MAXV; i++) {
-                const int r = tid + i * 256;
-                if (r < vdim)
-                    acc[i] = fmaf(w, ldc<TC>(v, p.v_transposed ? ((int64_t)g * vdim + r) * p.cache.page_tokens + pt
-                                                                 : ((int64_t)pt * G + g) * vdim + r), acc[i]);
+            for (int u = 0; u < KU; u++) {
+                const float v = group_sum<16>(s[u]);
+                s[0] = gl == u ? v : s[0];   // lane u of the group finishes its key u
+            }
+            const int jj = jb + 16 * gl + gi;
+            if (gl < KU && jj < nk) {
+                const int j = key_of(j0 + jj);
+                float v = s[0] * p.scale;
+                if (p.softcap > 0.f) v = p.softcap * tanhf(v / p.softcap);
+                if (p.r1) v -= b1 * log1pf(b2 * (float)(pos - j));
+                if (p.slopes) v -= slope * (float)(pos - j);
+                sc[jj] = sig ? 1.0f / (1.0f + expf(-(v + pbh))) : v;
             }
         }
         __syncthreads();
+        if (!sig) {   // (sigmoid weights are final: no running maximum, no normalisation)
+            float mx = -INFINITY;
+            for (int jj = tid; jj < nk; jj += 256) mx = fmaxf(mx, sc[jj]);
+            mx = wmax(mx);
+            if (lane == 0) red[wave] = mx;
+            __syncthreads();
+            mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+            const float m_new = fmaxf(m_run, mx);
+            const float alpha = expf(m_run - m_new);   // 0 on the first chunk
+            __syncthreads();
+            float ls = 0.f;
+            for (int jj = tid; jj < nk; jj += 256) {
+                const float e = expf(sc[jj] - m_new);
+                sc[jj] = e;
+                ls += e;
+            }
+            ls = bsum256(ls, red);
+            l_run = l_run * alpha + ls;
+            m_run = m_new;
+#pragma unroll
+            for (int i = 0; i < VC; i++) acc[i] *= alpha;
+        }
+        // a wave's keys: jj = wave, wave + 4, ...; a lane's coordinates r = lane + 64 c
+        auto value = [&](int jj, int r) {
+            const int pt = ktok[jj];
+            return ldc<TC>(pool + kbase[jj] + p.v_off, p.v_transposed ? ((int64_t)g * vdim + r) * PT + pt : ((int64_t)pt * G + g) * vdim + r);
+        };
+        int jj = wave;
+        for (; jj + 4 * (KU - 1) < nk; jj += 4 * KU)
+#pragma unroll
+            for (int c = 0; c < VC; c++) {
+                if (64 * c >= vdim) break;   // uniform
+                const int r = min(lane + 64 * c, vdim - 1);
+                float v[KU];
+#pragma unroll
+                for (int u = 0; u < KU; u++) v[u] = value(jj + 4 * u, r);
+#pragma unroll
+                for (int u = 0; u < KU; u++) acc[c] = fmaf(sc[jj + 4 * u], v[u], acc[c]);
+            }
+        for (; jj < nk; jj += 4)
+#pragma unroll
+            for (int c = 0; c < VC; c++) {
+                if (64 * c >= vdim) break;
+                acc[c] = fmaf(sc[jj], value(jj, min(lane + 64 * c, vdim - 1)), acc[c]);
+            }
     }
+#pragma unroll
+    for (int c = 0; c < VC; c++)
+        if (lane + 64 * c < vdim) ob[wave * vdim + lane + 64 * c] = acc[c];
+    __syncthreads();
     float inv = sig ? 1.0f : 1.0f / l_run;
     if (p.gate_col >= 0 && !p.gate_elem) inv *= 1.0f / (1.0f + expf(-p.proj[(int64_t)t * p.ld + p.gate_col + h]));
 #pragma unroll
     for (int i = 0; i < GA_MAXV; i++) {
         const int r = tid + i * 256;
         if (r < vdim) {
-            float o = acc[i] * inv;
+            float o = ((ob[r] + ob[vdim + r]) + (ob[2 * vdim + r] + ob[3 * vdim + r])) * inv;
             if (p.gate_col >= 0 && p.gate_elem) o *= 1.0f / (1.0f + expf(-p.proj[(int64_t)t * p.ld + p.gate_col + h * vdim + r]));
             ob[r] = o;
         }
@@ -465,8 +502,8 @@ int gqa_attention(const GqaAttnP& p, bool cache_f32, int T, hipStream_t st) {
     QIE_REQUIRE(p.mask == 0 || p.mask_size >= 1, "gqa attention: mask size %d", p.mask_size);
     QIE_REQUIRE(p.mask_keep >= 0 && (p.mask_keep == 0 || p.mask == 1), "gqa attention: kept first keys go with the window mask");
     QIE_REQUIRE(p.heads % p.kv_heads == 0, "gqa attention: %d query heads over %d key heads", p.heads, p.kv_heads);
-    const size_t shm = (size_t)(p.dim + GA_CHUNK + p.vdim) * 4;
-    QIE_REQUIRE(shm <= 48 * 1024, "gqa attention: head size above the kernel's staging");
+    QIE_REQUIRE((size_t)(p.dim + GA_CHUNK + p.vdim) * 4 <= 48 * 1024, "gqa attention: head size above the kernel's staging");
+    const size_t shm = (size_t)((p.dim + 3) / 4 * 4 + GA_CHUNK + 4 * p.vdim) * 4;
     if (cache_f32)
         hipLaunchKernelGGL(gqa_attention_kernel<float>, dim3(p.heads, T), dim3(256), shm, st, p);
     else

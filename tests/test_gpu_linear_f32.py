@@ -1,0 +1,35 @@
+"""fp32 products of the layered models on the matrix cores at the sizes where they can go wrong: 1 to 16 rows (k_decode_bf16.hip's
+fp32 form: X in LDS and through the ring), 17 to 300 (k_linear_f32.hip: whole and split tiles, ragged rows and columns, experts of
+few and of no rows), widths off their grid (the plain kernels); and the exact attention at head sizes on and off four elements."""
+import numpy as np
+import pytest
+
+from lugipel_oracle import attn, dense, gru, moe
+from test_gpu_lugipel import feed, model, rel  # noqa: F401  (model: a fixture)
+
+pytestmark = pytest.mark.gpu
+
+TOL = 5e-5   # of the logits' spread: fp32 sums of up to 2,816 terms over three layers
+
+LAYERS = {
+    "dense": [attn(heads=4, kv_heads=2, dim=64, vdim=64, size=70, mlp=dense(2816)), gru(width=320, mlp=dense(96))],
+    "routed": [gru(width=256, mlp=moe(experts=7, identity=1, top=2, count=2, keep=1, ff=64)), attn(heads=4, kv_heads=1, dim=32, vdim=96, size=300, mlp=None)],
+    "odd heads": [attn(heads=3, kv_heads=3, dim=30, vdim=65, size=33, mlp=dense(72)), attn(heads=2, kv_heads=1, dim=130, vdim=257, size=9, mlp=None)],
+}
+
+
+@pytest.mark.parametrize("width", [256, 272])   # 272: off the 64 grid, on the 16 grid
+@pytest.mark.parametrize("layers", sorted(LAYERS))
+def test_rows(model, layers, width):  # noqa: F811
+    m = model(LAYERS[layers], seed=7, vocab=1003, width=width, slots=6, max_ctx=512)
+    toks = m.tokens(302)
+    want = m.ref(toks)
+    sizes = [1, 2, 8, 9, 15, 16, 17, 33, 64, 65, 72]      # 302 rows in all
+    assert sum(sizes) == 302 and rel(feed(m, 0, toks, sizes), want) < TOL
+    assert rel(feed(m, 1, toks, [302]), want) < TOL
+    # sixteen rows as single tokens and short portions of several slots
+    a, b = [m.tokens(5) for _ in range(4)], m.tokens(12)
+    out = m.batch.step([(2 + i, t[:1]) for i, t in enumerate(a)] + [(0, b)], range(16))
+    for i, t in enumerate(a):
+        assert rel(out[i:i + 1], m.ref(t[:1])) < TOL
+    assert rel(out[4:], m.ref(toks + b)[302:]) < TOL
