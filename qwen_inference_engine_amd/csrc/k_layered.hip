@@ -309,6 +309,24 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(const TW* E, const int3
         if (out_bf) out_bf[(int64_t)t * W + w] = f2bf(v);
     }
 }
+// Reads past the caches: the host writes the same memory again for the next step.
+__global__ __launch_bounds__(256) void send_kernel(SendP p) {
+    const uint32_t* src = p.src[blockIdx.y];
+    uint32_t* dst = p.dst[blockIdx.y];
+    const int64_t n = p.words[blockIdx.y];
+    for (int64_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
+        dst[i] = __hip_atomic_load(src + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+int send(const SendP& p, hipStream_t st) {
+    int64_t most = 0;
+    for (int i = 0; i < p.n; i++) most = std::max(most, p.words[i]);
+    QIE_REQUIRE(p.n > 0 && p.n <= SendP::kMax && most > 0, "send: nothing to send, or too many arrays");
+    hipLaunchKernelGGL(send_kernel, dim3((unsigned)std::min<int64_t>((most + 255) / 256, 256), (unsigned)p.n), dim3(256), 0, st, p);
+    QIE_LAUNCH_CHECK();
+    return 0;
+}
+
 int embed_rows(const void* E, bool w_f32, const int32_t* tok, float* out, uint16_t* out_bf, int T, int W, int vocab,
                hipStream_t st, float scale, const int32_t* pos, const double* freq) {
     QIE_REQUIRE(!pos || freq, "embed_rows: positions without their frequencies");

@@ -7,6 +7,16 @@
 namespace qie {
 namespace lay {
 
+// Arrays of 32-bit words from pinned host memory to their buffers, one launch
+struct SendP {
+    static constexpr int kMax = 24;
+    const uint32_t* src[kMax];
+    uint32_t* dst[kMax];
+    int64_t words[kMax];
+    int n;
+};
+int send(const SendP& p, hipStream_t st);
+
 // y[m, n] = sum_k A[m, k] W[n, k] (+ batch z: A + z sA, W + z sW, Y + z sY).  A fp32, rounded to
 // bf16 on load when round_a; W fp32 or bf16 words; Y fp32.  grp_off (device, batch + 1 entries):
 // batch z covers rows [grp_off[z], grp_off[z + 1]) of A and Y (M is then the largest row count a

@@ -300,7 +300,7 @@ class Batch:
         counts = np.asarray([len(t) for _, t in entries], dtype=np.int32)
         toks = np.ascontiguousarray(np.concatenate([np.asarray(t, dtype=np.int32).reshape(-1) for _, t in entries]))
         w = np.ascontiguousarray(np.asarray(list(want), dtype=np.int32))
-        out = np.zeros((len(w), self.e.spec.vocab), dtype=np.float32) if fetch and len(w) else None
+        out = np.empty((len(w), self.e.spec.vocab), dtype=np.float32) if fetch and len(w) else None
         p32 = C.POINTER(C.c_int32)
         _lib.check(self.lib.qie_batch_step(
             self.h, len(slots), slots.ctypes.data_as(p32), counts.ctypes.data_as(p32), toks.ctypes.data_as(p32),
@@ -374,7 +374,7 @@ class Batch:
         return out[:n_steps] if want_ids else None
 
     def logits(self) -> np.ndarray:
-        out = np.zeros((self.B, self.e.spec.vocab), dtype=np.uint16)
+        out = np.empty((self.B, self.e.spec.vocab), dtype=np.uint16)
         _lib.check(self.lib.qie_batch_logits(self.h, out.ctypes.data), "qie_batch_logits")
         return out
 
