@@ -1142,7 +1142,7 @@ __global__ __launch_bounds__(NW * 64) void skinny_mfma_kernel(GemvParams p) {
     }
 }
 
-// block size bound of the one-block-per-CU GEMV variant (9 waves: Qwen2-7B QKV; O / down use 7)
+// block size bound of the one-block-per-CU GEMV variant (Qwen2-7B's down projection: 7 waves)
 constexpr int kGemvBalancedThreads = 576;
 
 static int env_int_gemv(const char* name, int dflt) { return dev_env(name, dflt); }
@@ -1196,14 +1196,13 @@ static int launch_gemv_t(const GemvParams& p, hipStream_t st, int blocks_per_cu)
         const int64_t rounds = (p.n_tasks + 4 * cap - 1) / (4 * cap);
         grid64 = std::max<int64_t>(1, (p.n_tasks + 4 * rounds - 1) / (4 * rounds));
     }
-    // One block per CU for mid-sized GEMVs (4..16 row tasks per CU: Qwen2-7B QKV 2,304, O and
+    // One block per CU for mid-sized GEMVs (4..9 row tasks per CU: Qwen2-7B
     // down 1,792): 448 four-wave blocks on 256 CUs left 64 CUs with half the waves, and the
     // whole launch waited for the doubly loaded CUs.  Block = ceil(tasks / CUs) waves, so every
     // CU streams the same rows.  (SwiGLU and lm_head have > 9 tasks per CU: grid-stride.)
     int threads = 256;
     const int64_t cus = device_cu_count();
-    // one row per wave: up to 16 waves per block (Qwen2-7B O / down: 14 one-row waves per CU)
-    constexpr int LBB = RPW == 1 ? 1024 : kGemvBalancedThreads;
+    constexpr int LBB = kGemvBalancedThreads;
     if (MT == 1 && WT == 0 && EPI != QIE_EPI_SWIGLU && blocks_per_cu < 0 && p.n_tasks > 4 * cus &&
         p.n_tasks <= (LBB / 64) * cus &&
         env_int_gemv("QIE_GEMV_BALANCED", 1) != 0) {
@@ -1234,10 +1233,6 @@ static int launch_gemv_t(const GemvParams& p, hipStream_t st, int blocks_per_cu)
 
 template <int MT, int XCH, int WT = 0, int UO = 0>
 static int launch_gemv_m(const GemvParams& p, int rpw, int epi, hipStream_t st, int bpc) {
-    if constexpr (MT == 1 && XCH == 1 && WT == 0) {   // one row per wave (O / down, x beside the weights)
-        if (rpw == 1 && epi == QIE_EPI_RESIDUAL) return launch_gemv_t<1, 1, QIE_EPI_RESIDUAL, 1, 0, UO>(p, st, bpc);
-        if (rpw == 1 && epi == QIE_EPI_STORE) return launch_gemv_t<1, 1, QIE_EPI_STORE, 1, 0, UO>(p, st, bpc);
-    }
     if (epi == QIE_EPI_SWIGLU) {
         return rpw >= 4 ? launch_gemv_t<MT, 4, QIE_EPI_SWIGLU, XCH, WT, UO>(p, st, bpc)
                         : launch_gemv_t<MT, 2, QIE_EPI_SWIGLU, XCH, WT, UO>(p, st, bpc);
@@ -1279,7 +1274,6 @@ static int launch_gemv_1(const GemvParams& p, int rpw, int epi, hipStream_t st, 
     // K <= 20,480 without a norm (Qwen3-14B O at K = 5,120: 2 x 5; down at K = 17,408: 5 x 7)
     if (xch == 10 && ub == 5 && !vocab) return launch_gemv_m<1, 10, 0, 5>(p, rpw, epi, st, bpc);
     if (xch == 10 && ub == 7 && !vocab) return launch_gemv_m<1, 10, 0, 7>(p, rpw, epi, st, bpc);
-    if (xch == 1 && n == 7) return launch_gemv_m<1, 1, 0, 7>(p, rpw, epi, st, bpc);
     if (xch == 1) return launch_gemv_m<1, 1>(p, rpw, epi, st, bpc);
     if (xch == 2) return launch_gemv_m<1, 2>(p, rpw, epi, st, bpc);
     if (xch == 5) return launch_gemv_m<1, 5>(p, rpw, epi, st, bpc);
@@ -1391,6 +1385,7 @@ int gemv_rope(const qie_linear_args* a, const int32_t* pos, const float* cs, con
 bool dec8_applies(const qie_linear_args* a);
 int dec8_linear(const qie_linear_args* a, hipStream_t st, bool* done);
 int dec_bf16_linear(const qie_linear_args* a, hipStream_t st, bool* done);
+int gemv_row(const qie_linear_args* a, hipStream_t st, bool* done);
 
 int gemv(const qie_linear_args* a, hipStream_t st) {
     // fp8 weights, 2..16 rows, K a whole number of per-wave slices (or split-K): k_decode_fp8.hip
@@ -1402,6 +1397,12 @@ int gemv(const qie_linear_args* a, hipStream_t st) {
     {   // bf16 weights, 2..16 rows, K a multiple of 128: k_decode_bf16.hip
         bool done = false;
         const int rc = dec_bf16_linear(a, st, &done);
+        if (done) return rc;
+    }
+    if (g_rope.rows == 0 && !(g_push && a->epilogue == QIE_EPI_F32) && env_int("QIE_GEMV_ROW", 1) != 0) {
+        // one row, few weight rows of up to 5,120: k_gemv_row.hip
+        bool done = false;
+        const int rc = gemv_row(a, st, &done);
         if (done) return rc;
     }
     GemvParams p;
@@ -1557,39 +1558,20 @@ int gemv(const qie_linear_args* a, hipStream_t st) {
     }
     if (vocab_rows && MT == 1 && bpc < 0)
         bpc = env_int("QIE_GEMV_LM_BPC", a->K <= 1024 ? 5 : (a->K <= 4096 ? 2 : -1));
-    // The normed STORE projection (QKV), Qwen2-7B (K 3,584, 9 row tasks per CU): 2 blocks of 4
-    // waves per CU instead of one 9-wave block, 9.77 -> 9.26 µs, 367.4 -> 369.4 tok/s (1: 357.2,
-    // 3: 364.8, 4: 364.8).  The fused norm's sum of squares is then reduced over 256 threads
-    // instead of 576 (another fp32 order of the same sum; the parity tests bound it).
-    // Qwen2-0.5B's QKV: equal at 1-3 per CU, kept.
     // (dev A/B) residual projections (O, down): caps 3 / 5 / 6 / 8 per CU all ran Qwen2-7B at
     // 363.4-363.5 vs 369.6 tok/s on their one-block-per-CU layout; 0.5B equal
 
     if (MT == 1 && a->epilogue == QIE_EPI_RESIDUAL && bpc < 0) bpc = env_int("QIE_GEMV_RES_BPC", -1);
-    if (!vocab_rows && MT == 1 && p.norm_w && a->epilogue == QIE_EPI_STORE && bpc < 0) {
-        const int64_t tpc = p.n_tasks / cus;
-        bpc = env_int("QIE_GEMV_QKV_BPC", a->K >= 3072 && a->K <= 4096 && tpc >= 6 && tpc <= 12 ? 2 : -1);
-    }
-    // Batch-1 GEMVs without a fused norm on the one-block-per-CU grid (one row task per
-    // wave: Qwen2-7B O, down) read x from L2 beside each weight chunk (XCH = 1) instead of
-    // staging it in LDS behind a barrier: Qwen2-7B decode 355 -> 358 tok/s (two A/B rounds),
-    // in-graph down 24.5 -> 23.5 us, O 7.3 -> 7.05.  Where a wave walks several row tasks
-    // (Qwen3-14B O / down, 10 per CU; Qwen2-0.5B) x would be re-read per task: O 13.1 ->
-    // 16.5, down 32.9 -> 39.7 us at 14B, so those keep the staged copy.
+    // Batch-1 GEMVs without a fused norm on the one-block-per-CU grid (one task of two long rows per wave: Qwen2-7B's down
+    // projection; rows of up to 5,120 are k_gemv_row.hip's) read x from L2 beside each weight chunk (XCH = 1) instead of
+    // staging it in LDS behind a barrier: in-graph down 24.5 -> 23.5 us.  Where a wave walks several row tasks
+    // (Qwen3-14B down, 10 per CU) x would be re-read per task (32.9 -> 39.7 us), so those keep the staged copy.
     // (the condition is launch_gemv_t's one-block-per-CU grid)
     if (MT == 1 && p.M == 1 && !p.norm_w && !(a->flags & QIE_LINEAR_FP8) && a->epilogue != QIE_EPI_SWIGLU &&
         a->K % 8 == 0 && bpc < 0 && p.n_tasks > 4 * (int64_t)cus &&
         p.n_tasks <= (kGemvBalancedThreads / 64) * (int64_t)cus && env_int_gemv("QIE_GEMV_BALANCED", 1) != 0) {
         xch = 1;
         p.xlds = 0;
-        // one row per wave, up to 16 waves per CU, where x is short (each wave re-reads all of x
-        // from L2): Qwen2-7B O 6.68 -> 6.45 us; down (x 37.9 KB, K = 18,944) doubled its L2
-        // traffic for x that way (23.3 -> 25.1 us), so it keeps two rows per wave
-        if ((a->epilogue == QIE_EPI_RESIDUAL || a->epilogue == QIE_EPI_STORE) && rows <= 16 * (int64_t)cus &&
-            a->K <= 4096 && env_int("QIE_GEMV_RPW1", 1) != 0) {
-            rpw = 1;
-            p.n_tasks = rows;
-        }
     }
     QIE_REQUIRE(!(xch == 10 && p.norm_w), "qie_linear: internal: fused norm routed to a variant without one");
     switch (MT) {
