@@ -7,8 +7,13 @@
 // 16 weight rows, and every wave streams the 128-k chunks of its own share of K (256 contiguous bytes of each row, 4 KB) by
 // LDS-DMA through a ring of its own, with no barrier: the loads of R - 1 chunks fly while one is multiplied
 // (v_mfma_f32_16x16x32_bf16, D = W Xᵀ, so a lane ends with four neighbouring columns of one row).
-//   * X lies in LDS for the whole launch (normed once a workgroup by the waves themselves, under the first chunks' loads);
-//     where M rows of K do not fit (the down projection) its chunks travel through the ring beside the weights'.
+//   * X lies in LDS for the whole launch: normed once a workgroup by the waves themselves, under the first chunks' loads, or sent
+//     there as it is by LDS-DMA; where M rows of K do not fit (the down projection) its chunks travel through the ring beside the
+//     weights'.
+//   * Launches of 5 to 15 us feel every instruction and trip to memory ahead of the first product: loads are buffer loads (scalar
+//     offsets, no bounds tests), a tile lies in one weight segment so its base is scalar, the first tile's residuals or biases are
+//     loaded ahead of the weights, and the wait for X is a counted one.  us before -> with that, Qwen2-7B at 4 rows: QKV 13.2 ->
+//     11.1, O 8.8 -> 7.5, gate/up 50.2 -> 48.4; Qwen2-0.5B at 7 rows: QKV 6.4 -> 5.3, O and down 6.5 -> 6.1 a launch.
 //   * The 8 partial tiles meet in LDS, one barrier a tile; the wave that sums them and runs the epilogue rotates.
 //   * SwiGLU: a tile is 8 gate rows and the same outputs' 8 up rows, met across lane halves.
 // One workgroup a CU: LDS holds 64 to 128 KB of chunks.  Sums: per wave over its K share in fp32, the shares in wave order.
@@ -24,6 +29,7 @@ namespace qie {
 typedef __bf16 db_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float db_f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int db_u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int db_u32x2 __attribute__((ext_vector_type(2)));
 
 namespace db {
 constexpr int NW = 8;          // waves
@@ -39,7 +45,8 @@ struct DecBfParams {
     int numerics;
     const uint16_t* w[3];
     const uint16_t* bias[3];
-    int64_t n0, n01;           // rows of segment 0, of segments 0 and 1
+    int rows[3];               // of the segments (SwiGLU: N, N)
+    int t0, t01;               // tiles of segment 0, of segments 0 and 1: a tile lies in one segment
     int K, N, M;
     int n_tiles;
     uint16_t* y;
@@ -47,16 +54,23 @@ struct DecBfParams {
     int vec;                   // 8- (fp32: 16-) byte stores
     unsigned long long* keys;
     int64_t key_col0;
-    int xstride;               // bytes of a row of the X image (K * 2 + 16: 16 rows' same chunk in different banks)
+    int xstride;               // bytes of a row of the X image (whole 1,024 and 16: 16 rows' same chunk in different banks)
 };
 
-__device__ __forceinline__ void db_glds16(const void* src, void* lds) {
-    __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void*)(src),
-                                     (__attribute__((address_space(3))) void*)(lds), 16, 0, 0);
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t db_rsrc(const void* base, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
+}
+// 16 bytes a lane into LDS: lane l at lds + 16 l
+__device__ __forceinline__ void db_lds16(__amdgpu_buffer_rsrc_t rs, void* lds, uint32_t voff, uint32_t soff) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(lds), 16, voff, soff, 0, 0);
+#else
+    (void)rs; (void)lds; (void)voff; (void)soff;
+#endif
 }
 
 // XM: 0 = X in LDS; 8, 16 = X's chunks (of 8 or 16 rows) through the ring.  NV: 16-byte vectors of a row per lane while X is
-// normed (K <= 512 NV); R: ring slots a wave.
+// normed (K <= 512 NV), 0: not normed, its rows go to LDS as they are; R: ring slots a wave.
 // F32: rows of fp32 instead (p.K, p.ldx in 16-bit units; the fp32 epilogue, no norm): a 16-byte piece is 4 k, four
 // v_mfma_f32_16x16x4f32 instead of one v_mfma_f32_16x16x32_bf16.
 template <int EPI, int XM, int NV, int R, bool F32 = false>
@@ -81,61 +95,103 @@ __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
     const int items = mine * cnt;   // (tile, chunk) in order
 
     // ---- X rows for the norm (or the copy), loaded ahead of the first weight chunks: P waves a row (8, 4, 2 rows at a time), so
-    // that few rows keep every wave busy
-    const db_u32x4 zero = {0u, 0u, 0u, 0u};
+    // that few rows keep every wave busy.  (Buffer loads throughout: a load is one instruction with its offset in a scalar register,
+    // and what lies past K reads zeros.  With 64-bit addresses and a bounds test a lane the prologue was ~2,000 instructions.)
     const int P = M <= 2 ? 4 : M <= 4 ? 2 : 1, rows_at = db::NW / P, sub = wave % P;
-    db_u32x4 xv[NV], nv[NV];
+    db_u32x4 xv[NV ? NV : 1], nv[NV ? NV : 1];
     auto load_row = [&](int m) {
+        const auto rx = db_rsrc(p.x + (int64_t)m * p.ldx, (uint32_t)K * 2), rn = db_rsrc(p.norm_w, (uint32_t)K * 2);
 #pragma unroll
         for (int v = 0; v < NV; v++) {
-            if (v * P * 512 >= K) break;   // uniform
-            const int k = ((v * P + sub) * 64 + lane) * 8;
-            xv[v] = k < K ? *reinterpret_cast<const db_u32x4*>(p.x + (int64_t)m * p.ldx + k) : zero;
-            if (p.norm_w) nv[v] = k < K ? *reinterpret_cast<const db_u32x4*>(p.norm_w + k) : zero;
+            if ((v * P + sub) * 512 >= K) break;   // uniform
+            xv[v] = __builtin_amdgcn_raw_buffer_load_b128(rx, lane * 16, (v * P + sub) * 1024, 0);
+            nv[v] = __builtin_amdgcn_raw_buffer_load_b128(rn, lane * 16, (v * P + sub) * 1024, 0);
         }
     };
-    if constexpr (XM == 0) {
+    if constexpr (XM == 0 && NV > 0) {
         if (wave / P < M) load_row(wave / P);
+    } else if constexpr (XM == 0) {
+        for (int m = wave; m < M; m += db::NW) {
+            const auto rx = db_rsrc(p.x + (int64_t)m * p.ldx, (uint32_t)K * 2);
+            for (int c = 0; c * 512 < K; c++) db_lds16(rx, xs + m * p.xstride + c * 1024, lane * 16, c * 1024);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- tiles: segment, first row in it, rows left, first column (uniform)
+    struct Tile {
+        int seg, row0, left, col;
+    };
+    auto tile_at = [&](int tile) {
+        Tile t;
+        if constexpr (EPI == QIE_EPI_SWIGLU) {
+            t.seg = 0;
+            t.row0 = t.col = tile * 8;
+        } else {
+            t.seg = tile < p.t0 ? 0 : tile < p.t01 ? 1 : 2;
+            t.row0 = (tile - (t.seg == 0 ? 0 : t.seg == 1 ? p.t0 : p.t01)) * 16;
+            t.col = t.row0 + (t.seg == 0 ? 0 : t.seg == 1 ? p.rows[0] : p.rows[0] + p.rows[1]);
+        }
+        t.left = (t.seg == 0 ? p.rows[0] : t.seg == 1 ? p.rows[1] : p.rows[2]) - t.row0;
+        return t;
+    };
+    // the epilogue's operands: old values (whole quads), or biases.  The first tile's are loaded by the wave that will need them ahead of
+    // its chunks: behind the reduction they cost another trip to memory, and most launches have one tile a block.
+    db_u32x2 old = {0u, 0u};
+    uint32_t bias[4] = {0u, 0u, 0u, 0u};
+    auto load_old = [&](const Tile& t, bool on) {
+        const auto ry = db_rsrc(p.y, on && p.vec ? (uint32_t)(((int64_t)(M - 1) * p.ldy + p.N) * 2) : 0u);
+        old = __builtin_amdgcn_raw_buffer_load_b64(ry, (int)((fr * (int)p.ldy + t.col + 4 * g) * 2), 0, 0);
+    };
+    auto load_bias = [&](const Tile& t, bool on) {
+        const uint16_t* b = t.seg == 0 ? p.bias[0] : t.seg == 1 ? p.bias[1] : p.bias[2];
+        const auto rb = db_rsrc(b ? b : p.x, b && on ? (uint32_t)(t.row0 + t.left) * 2 : 0u);   // none: zeros
+#pragma unroll
+        for (int r = 0; r < 4; r++) bias[r] = __builtin_amdgcn_raw_buffer_load_b16(rb, (t.row0 + 4 * g + r) * 2, 0, 0);
+    };
+    {
+        const Tile t = tile_at(mine > 0 ? (int)blockIdx.x : 0);
+        if constexpr (EPI == QIE_EPI_RESIDUAL) load_old(t, wave == 0);
+        if constexpr (EPI == QIE_EPI_STORE) load_bias(t, wave == 0);
         __builtin_amdgcn_sched_barrier(0);
     }
 
     // ---- the weight stream: lane -> row 4 i + (lane >> 4) of the tile, LDS piece lane & 15 of its 256 B, which holds the
     // source's piece (lane & 15) ^ row (the fragment reads below are then free of bank conflicts)
-    const uint16_t* wsrc[4];
-    const uint16_t* xsrc[XM ? XM / 4 : 1];
+    uint32_t wsrc[4], xsrc[XM ? XM / 4 : 1];
+    const uint32_t xbytes = (uint32_t)(((int64_t)(M - 1) * p.ldx + K) * 2);
     if constexpr (XM != 0) {
 #pragma unroll
         for (int i = 0; i < XM / 4; i++) {
             const int m = 4 * i + (lane >> 4);
-            xsrc[i] = p.x + (int64_t)(m < M ? m : M - 1) * p.ldx + ((lane & 15) ^ m) * 8;
+            xsrc[i] = (uint32_t)((m < M ? m : M - 1) * (int)p.ldx * 2 + ((lane & 15) ^ m) * 16);
         }
     }
+    const uint16_t *wb0 = nullptr, *wb1 = nullptr;   // the tile's first row (SwiGLU: of gate and up)
+    uint32_t wbytes = 0;
     auto aim = [&](int tile) {
+        const Tile t = tile_at(tile);
+        const int64_t at = (int64_t)t.row0 * K;
+        wb0 = (t.seg == 0 ? p.w[0] : t.seg == 1 ? p.w[1] : p.w[2]) + at;
+        if constexpr (EPI == QIE_EPI_SWIGLU) wb1 = p.w[1] + at;
+        constexpr int TR = EPI == QIE_EPI_SWIGLU ? 8 : 16;
+        wbytes = (uint32_t)(t.left < TR ? t.left : TR) * (uint32_t)K * 2;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const int row = 4 * i + (lane >> 4);
-            const uint16_t* base;
-            if constexpr (EPI == QIE_EPI_SWIGLU) {
-                int64_t j = (int64_t)tile * 8 + (row & 7);
-                j = j < p.N ? j : p.N - 1;
-                base = (row < 8 ? p.w[0] : p.w[1]) + j * K;
-            } else {
-                int64_t r = (int64_t)tile * 16 + row;
-                r = r < p.N ? r : p.N - 1;
-                base = r < p.n0 ? p.w[0] + r * K : (r < p.n01 ? p.w[1] + (r - p.n0) * K : p.w[2] + (r - p.n01) * K);
-            }
-            wsrc[i] = base + ((lane & 15) ^ row) * 8;
+            const int row = 4 * i + (lane >> 4), r = row & (TR - 1);
+            wsrc[i] = (uint32_t)((r < t.left ? r : t.left - 1) * K * 2 + ((lane & 15) ^ row) * 16);
         }
     };
     int n_tile = blockIdx.x, n_c = 0, n_slot = 0;   // the next chunk to ask for
-    auto issue = [&]() {
+    auto issue = [&](bool on) {   // off: nothing is read
         unsigned char* dst = ring + n_slot * SLOT;
-        const int64_t k = (int64_t)(c0 + n_c) * db::CH;
+        const uint32_t k = (uint32_t)(c0 + n_c) * 256;
+        const auto r0 = db_rsrc(wb0, on ? wbytes : 0u), r1 = EPI == QIE_EPI_SWIGLU ? db_rsrc(wb1, on ? wbytes : 0u) : r0;
 #pragma unroll
-        for (int i = 0; i < 4; i++) db_glds16(wsrc[i] + k, dst + i * 1024);
+        for (int i = 0; i < 4; i++) db_lds16(i < 2 ? r0 : r1, dst + i * 1024, wsrc[i], k);
         if constexpr (XM != 0) {
 #pragma unroll
-            for (int i = 0; i < XM / 4; i++) db_glds16(xsrc[i] + k, dst + db::WCH + i * 1024);
+            for (int i = 0; i < XM / 4; i++) db_lds16(db_rsrc(p.x, on ? xbytes : 0u), dst + db::WCH + i * 1024, xsrc[i], k);
         }
         n_slot = n_slot + 1 == R ? 0 : n_slot + 1;
         if (++n_c == cnt) {
@@ -144,26 +200,20 @@ __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
             aim(n_tile < T ? n_tile : T - 1);
         }
     };
-    if (items > 0) aim(n_tile);
-    for (int i = 0; i < R && i < items; i++) issue();
+    aim(n_tile);
+    // R chunks whatever there are, so that the wait for X is a counted one that leaves them in flight
+#pragma unroll
+    for (int i = 0; i < R; i++) issue(i < items);
     __builtin_amdgcn_sched_barrier(0);
 
     if constexpr (XM == 0) {
-        auto store_row = [&](int m) {
-#pragma unroll
-            for (int v = 0; v < NV; v++) {
-                if (v * P * 512 >= K) break;
-                const int k = ((v * P + sub) * 64 + lane) * 8;
-                if (k < K) *reinterpret_cast<db_u32x4*>(xs + m * p.xstride + k * 2) = xv[v];
-            }
-        };
-        if (p.norm_w) {   // M <= 8: one pass
+        if constexpr (NV > 0) {   // M <= 8: one pass
             const int m = wave / P;
             float* ssq = reinterpret_cast<float*>(red);
             float ss = 0.f;
 #pragma unroll
             for (int v = 0; v < NV; v++) {
-                if (v * P * 512 >= K) break;
+                if ((v * P + sub) * 512 >= K) break;
                 const uint32_t e[4] = {xv[v].x, xv[v].y, xv[v].z, xv[v].w};
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
@@ -183,7 +233,7 @@ __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
                 constexpr bool HF = decltype(hf)::value;
 #pragma unroll
                 for (int v = 0; v < NV; v++) {
-                    if (v * P * 512 >= K) break;
+                    if ((v * P + sub) * 512 >= K) break;
                     xv[v].x = rms_pair<HF>(xv[v].x, nv[v].x, rr, inv);
                     xv[v].y = rms_pair<HF>(xv[v].y, nv[v].y, rr, inv);
                     xv[v].z = rms_pair<HF>(xv[v].z, nv[v].z, rr, inv);
@@ -193,19 +243,22 @@ __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
             if (m < M) {
                 if (p.numerics == QIE_NUMERICS_HF) apply(std::true_type{});
                 else apply(std::false_type{});
-                store_row(m);
+#pragma unroll
+                for (int v = 0; v < NV; v++) {
+                    if ((v * P + sub) * 512 >= K) break;
+                    *reinterpret_cast<db_u32x4*>(xs + m * p.xstride + (v * P + sub) * 1024 + lane * 16) = xv[v];
+                }
             }
         } else {
-            for (int m = wave / P; m < M; m += rows_at) {
-                if (m >= rows_at) load_row(m);
-                store_row(m);
-            }
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(IPC * R) : "memory");   // X is there; the chunks fly on
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
     }
 
+    // (the wait for them belongs here, not into the loop of counted waits)
+    asm volatile("" : "+v"(old), "+v"(bias[0]), "+v"(bias[1]), "+v"(bias[2]), "+v"(bias[3]));
     const int arow = fr < M ? fr : M - 1;   // rows past M: copies of row M - 1, never stored
     unsigned long long kbest = 0ull;
     int done = 0, slot = 0;
@@ -239,7 +292,7 @@ __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the slot's reads are done
             __builtin_amdgcn_sched_barrier(0);
-            if (done + R < items) issue();
+            if (done + R < items) issue(true);
             done++;
             slot = slot + 1 == R ? 0 : slot + 1;
         }
@@ -254,6 +307,7 @@ __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
         db_f32x4 v = red[(it & 1) * db::NW * RS + rl];
 #pragma unroll
         for (int w = 1; w < db::NW; w++) v = v + red[((it & 1) * db::NW + w) * RS + rl];
+        const Tile t = tile_at(tile);
         // lane: row m = fr of X, columns 4 g .. 4 g + 3 of the tile (SwiGLU: g = 0, 1 gate, g = 2, 3 the same outputs' up)
         const int m = fr;
         if constexpr (EPI == QIE_EPI_SWIGLU) {
@@ -265,7 +319,7 @@ __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
                 const float gg = rbf(a), uu = rbf(b);
                 h[r] = uu * rbf(gg * (1.0f / (1.0f + expf(-gg))));
             }
-            const int64_t col = (int64_t)tile * 8 + 4 * g;
+            const int64_t col = t.col + 4 * g;
             if (g < 2 && m < M) {
                 uint16_t* dst = p.y + (int64_t)m * p.ldy + col;
                 if (p.vec && col + 4 <= p.N) {
@@ -277,40 +331,40 @@ __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
                 }
             }
         } else if (m < M) {
-            const int64_t col = (int64_t)tile * 16 + 4 * g;
+            const int64_t col = t.col + 4 * g, end = t.col + t.left;   // the segment's end
+            const bool whole = p.vec && t.col % 4 == 0 && col + 4 <= end;
             if constexpr (EPI == QIE_EPI_F32) {
                 float* dst = reinterpret_cast<float*>(p.y) + (int64_t)m * p.ldy + col;
-                if (p.vec && col + 4 <= p.N) {
+                if (whole) {
                     *reinterpret_cast<db_f32x4*>(dst) = v;
                 } else {
 #pragma unroll
                     for (int r = 0; r < 4; r++)
-                        if (col + r < p.N) dst[r] = v[r];
+                        if (col + r < end) dst[r] = v[r];
                 }
             } else {
                 uint16_t* dst = p.y + (int64_t)m * p.ldy + col;
-                const bool whole = p.vec && col + 4 <= p.N;
                 float o[4];
                 if constexpr (EPI == QIE_EPI_RESIDUAL) {
                     if (whole) {
-                        const uint2 x = *reinterpret_cast<const uint2*>(dst);
-                        o[0] = bf_lo(x.x);
-                        o[1] = bf_hi(x.x);
-                        o[2] = bf_lo(x.y);
-                        o[3] = bf_hi(x.y);
+                        if (it > 0) {
+                            const uint2 x = *reinterpret_cast<const uint2*>(dst);
+                            old = db_u32x2{x.x, x.y};
+                        }
+                        o[0] = bf_lo(old.x);
+                        o[1] = bf_hi(old.x);
+                        o[2] = bf_lo(old.y);
+                        o[3] = bf_hi(old.y);
                     } else {
 #pragma unroll
-                        for (int r = 0; r < 4; r++) o[r] = col + r < p.N ? bf2f(dst[r]) : 0.f;
+                        for (int r = 0; r < 4; r++) o[r] = col + r < end ? bf2f(dst[r]) : 0.f;
                     }
 #pragma unroll
                     for (int r = 0; r < 4; r++) o[r] += rbf(v[r]);
                 } else {
+                    if (it > 0) load_bias(t, true);
 #pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const int64_t c = col + r < p.N ? col + r : p.N - 1;
-                        const uint16_t* b = c < p.n0 ? p.bias[0] : (c < p.n01 ? p.bias[1] : p.bias[2]);
-                        o[r] = v[r] + (b ? bf2f(b[c < p.n0 ? c : (c < p.n01 ? c - p.n0 : c - p.n01)]) : 0.f);
-                    }
+                    for (int r = 0; r < 4; r++) o[r] = v[r] + bf2f((uint16_t)bias[r]);
                 }
                 const uint32_t lo = pack2(o[0], o[1]), hi = pack2(o[2], o[3]);
                 if (whole) {
@@ -319,13 +373,13 @@ __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
                     const uint16_t q[4] = {(uint16_t)lo, (uint16_t)(lo >> 16), (uint16_t)hi, (uint16_t)(hi >> 16)};
 #pragma unroll
                     for (int r = 0; r < 4; r++)
-                        if (col + r < p.N) dst[r] = q[r];
+                        if (col + r < end) dst[r] = q[r];
                 }
                 if (EPI == QIE_EPI_STORE && p.keys) {
                     const uint32_t q[4] = {lo & 0xffffu, lo >> 16, hi & 0xffffu, hi >> 16};
 #pragma unroll
                     for (int r = 0; r < 4; r++) {
-                        if (col + r >= p.N) continue;
+                        if (col + r >= end) continue;
                         const unsigned long long kk = sel_key(bf2f(q[r]), (uint32_t)(col + r + p.key_col0));
                         kbest = kk > kbest ? kk : kbest;
                     }
@@ -357,7 +411,7 @@ constexpr int64_t kDbLds = 160 * 1024;
 
 // X in LDS beside a ring of R slots a wave
 int64_t db_red_bytes(int64_t M) { return 2 * db::NW * (M <= 8 ? 512 : 1024); }
-int64_t db_image_bytes(int64_t M, int64_t K, int R) { return db::NW * R * db::WCH + db_red_bytes(M) + M * (K * 2 + 16); }
+int64_t db_image_bytes(int64_t M, int64_t K, int R) { return db::NW * R * db::WCH + db_red_bytes(M) + M * ((K + 511) / 512 * 1024 + 16); }
 
 struct DbPlan {
     int xm, nv, r;
@@ -366,17 +420,21 @@ struct DbPlan {
 bool db_plan(const qie_linear_args* a, DbPlan* out) {
     if (dev_env("QIE_DEC_BF16", 1) == 0) return false;
     if ((a->flags & QIE_LINEAR_FP8) || a->M < 2 || a->M > 16 || a->K % db::CH != 0 || a->K / db::CH < db::NW / 2) return false;
+    if (a->M * a->ldx >= (int64_t)1 << 30 || a->M * a->ldy >= (int64_t)1 << 29) return false;   // 32-bit offsets
     if (a->norm_w && (a->M > db::NW || ((uintptr_t)a->norm_w) % 16 != 0)) return false;
     if (a->K <= 5120) {
-        for (int r = 4; r >= 2; r--)
+        // chunks that a wave of the busiest block streams: a slot beyond them is issued for nothing
+        const int64_t cus = device_cu_count(), tiles = a->epilogue == QIE_EPI_SWIGLU ? (a->N + 7) / 8 : (a->N + 15) / 16 + 2;
+        const int64_t items = (tiles + cus - 1) / cus * ((a->K / db::CH + db::NW - 1) / db::NW);
+        for (int r = (int)std::max<int64_t>(2, std::min<int64_t>(4, items)); r >= 2; r--)
             if (db_image_bytes(a->M, a->K, r) <= kDbLds) {
-                *out = {0, a->K <= 1024 ? 2 : a->K <= 2048 ? 4 : a->K <= 3584 ? 7 : 10, r, (size_t)db_image_bytes(a->M, a->K, r)};
+                *out = {0, !a->norm_w ? 0 : a->K <= 1024 ? 2 : a->K <= 2048 ? 4 : a->K <= 3584 ? 7 : 10, r, (size_t)db_image_bytes(a->M, a->K, r)};
                 return true;
             }
     }
     if (a->norm_w) return false;
     const int xm = a->M <= 8 ? 8 : 16;
-    *out = {xm, 1, 2, (size_t)(db::NW * 2 * (db::WCH + xm * 256) + db_red_bytes(a->M))};
+    *out = {xm, 0, 2, (size_t)(db::NW * 2 * (db::WCH + xm * 256) + db_red_bytes(a->M))};
     return true;
 }
 
@@ -396,6 +454,7 @@ int db_launch(const DecBfParams& p, size_t lds, hipStream_t st) {
 template <int EPI, int R>
 int db_launch_nv(const DecBfParams& p, const DbPlan& pl, hipStream_t st) {
     switch (pl.nv) {
+        case 0: return db_launch<EPI, 0, 0, R>(p, pl.lds, st);
         case 2: return db_launch<EPI, 0, 2, R>(p, pl.lds, st);
         case 4: return db_launch<EPI, 0, 4, R>(p, pl.lds, st);
         case 7: return db_launch<EPI, 0, 7, R>(p, pl.lds, st);
@@ -404,8 +463,8 @@ int db_launch_nv(const DecBfParams& p, const DbPlan& pl, hipStream_t st) {
 }
 template <int EPI>
 int db_launch_plan(const DecBfParams& p, const DbPlan& pl, hipStream_t st) {
-    if (pl.xm == 8) return db_launch<EPI, 8, 1, 2>(p, pl.lds, st);
-    if (pl.xm == 16) return db_launch<EPI, 16, 1, 2>(p, pl.lds, st);
+    if (pl.xm == 8) return db_launch<EPI, 8, 0, 2>(p, pl.lds, st);
+    if (pl.xm == 16) return db_launch<EPI, 16, 0, 2>(p, pl.lds, st);
     if (pl.r == 4) return db_launch_nv<EPI, 4>(p, pl, st);
     if (pl.r == 3) return db_launch_nv<EPI, 3>(p, pl, st);
     return db_launch_nv<EPI, 2>(p, pl, st);
@@ -432,18 +491,19 @@ int dec_bf16_linear(const qie_linear_args* a, hipStream_t st, bool* done) {
         p.w[i] = (const uint16_t*)a->w[i];
         p.bias[i] = (const uint16_t*)a->bias[i];
     }
-    p.n0 = a->seg_rows[0];
-    p.n01 = a->seg_rows[0] + a->seg_rows[1];
+    for (int i = 0; i < 3; i++) p.rows[i] = (int)(a->epilogue == QIE_EPI_SWIGLU ? a->N : a->seg_rows[i]);
+    p.t0 = (p.rows[0] + 15) / 16;
+    p.t01 = p.t0 + (p.rows[1] + 15) / 16;
     p.K = (int)a->K;
     p.N = (int)a->N;
     p.M = (int)a->M;
-    p.n_tiles = (int)(a->epilogue == QIE_EPI_SWIGLU ? (a->N + 7) / 8 : (a->N + 15) / 16);
+    p.n_tiles = a->epilogue == QIE_EPI_SWIGLU ? (p.N + 7) / 8 : p.t01 + (p.rows[2] + 15) / 16;
     p.y = (uint16_t*)a->y;
     p.ldy = a->ldy;
     p.vec = a->ldy % 4 == 0 && ((uintptr_t)a->y) % (a->epilogue == QIE_EPI_F32 ? 16 : 8) == 0;
     p.keys = (unsigned long long*)a->argmax_keys;
     p.key_col0 = a->key_col0;
-    p.xstride = (int)a->K * 2 + 16;
+    p.xstride = (p.K + 511) / 512 * 1024 + 16;
     switch (a->epilogue) {
         case QIE_EPI_SWIGLU: return db_launch_plan<QIE_EPI_SWIGLU>(p, pl, st);
         case QIE_EPI_RESIDUAL: return db_launch_plan<QIE_EPI_RESIDUAL>(p, pl, st);
@@ -455,26 +515,27 @@ int dec_bf16_linear(const qie_linear_args* a, hipStream_t st, bool* done) {
 // y = X W^T in fp32 for up to 16 rows (lay::linear's plain form): *done false: not its shape
 int dec_f32_linear(const lay::LinearP& q, hipStream_t st, bool* done) {
     *done = q.batch == 1 && !q.grp_off && !q.round_a && q.M <= 16 && q.K % 64 == 0 && q.K >= 256 && q.ldw == q.K && q.lda % 4 == 0 &&
-            (((uintptr_t)q.A | (uintptr_t)q.W) % 16) == 0;
+            (int64_t)q.M * q.lda < (int64_t)1 << 29 && (int64_t)q.M * q.ldy < (int64_t)1 << 29 && (((uintptr_t)q.A | (uintptr_t)q.W) % 16) == 0;
     if (!*done) return 0;
     DecBfParams p{};
     p.x = (const uint16_t*)q.A;
     p.ldx = q.lda * 2;
     p.w[0] = (const uint16_t*)q.W;
-    p.n0 = p.n01 = q.N;
+    p.rows[0] = q.N;
+    p.t0 = p.t01 = (q.N + 15) / 16;
     p.K = q.K * 2;
     p.N = q.N;
     p.M = q.M;
-    p.n_tiles = (q.N + 15) / 16;
+    p.n_tiles = p.t0;
     p.y = (uint16_t*)q.Y;
     p.ldy = q.ldy;
     p.vec = q.ldy % 4 == 0 && ((uintptr_t)q.Y) % 16 == 0;
-    p.xstride = p.K * 2 + 16;
+    p.xstride = (p.K + 511) / 512 * 1024 + 16;
     constexpr int E = QIE_EPI_F32;
-    if (p.K <= 5120 && db_image_bytes(p.M, p.K, 2) <= kDbLds) return db_launch<E, 0, 10, 2, true>(p, (size_t)db_image_bytes(p.M, p.K, 2), st);
+    if (p.K <= 5120 && db_image_bytes(p.M, p.K, 2) <= kDbLds) return db_launch<E, 0, 0, 2, true>(p, (size_t)db_image_bytes(p.M, p.K, 2), st);
     const int xm = p.M <= 8 ? 8 : 16;
     const size_t lds = (size_t)(db::NW * 2 * (db::WCH + xm * 256) + db_red_bytes(p.M));
-    return xm == 8 ? db_launch<E, 8, 1, 2, true>(p, lds, st) : db_launch<E, 16, 1, 2, true>(p, lds, st);
+    return xm == 8 ? db_launch<E, 8, 0, 2, true>(p, lds, st) : db_launch<E, 16, 0, 2, true>(p, lds, st);
 }
 
 }  // namespace qie
