@@ -420,7 +420,7 @@ struct DbPlan {
 bool db_plan(const qie_linear_args* a, DbPlan* out) {
     if (dev_env("QIE_DEC_BF16", 1) == 0) return false;
     if ((a->flags & QIE_LINEAR_FP8) || a->M < 2 || a->M > 16 || a->K % db::CH != 0 || a->K / db::CH < db::NW / 2) return false;
-    if (a->M * a->ldx >= (int64_t)1 << 30 || a->M * a->ldy >= (int64_t)1 << 29) return false;   // 32-bit offsets
+    if (a->K >= 1 << 26 || a->M * a->ldx >= 1 << 30 || a->M * a->ldy >= 1 << 29) return false;   // 32-bit offsets
     if (a->norm_w && (a->M > db::NW || ((uintptr_t)a->norm_w) % 16 != 0)) return false;
     if (a->K <= 5120) {
         // chunks that a wave of the busiest block streams: a slot beyond them is issued for nothing
@@ -514,7 +514,7 @@ int dec_bf16_linear(const qie_linear_args* a, hipStream_t st, bool* done) {
 
 // y = X W^T in fp32 for up to 16 rows (lay::linear's plain form): *done false: not its shape
 int dec_f32_linear(const lay::LinearP& q, hipStream_t st, bool* done) {
-    *done = q.batch == 1 && !q.grp_off && !q.round_a && q.M <= 16 && q.K % 64 == 0 && q.K >= 256 && q.ldw == q.K && q.lda % 4 == 0 &&
+    *done = q.batch == 1 && !q.grp_off && !q.round_a && q.M <= 16 && q.K % 64 == 0 && q.K >= 256 && q.K < 1 << 25 && q.ldw == q.K && q.lda % 4 == 0 &&
             (int64_t)q.M * q.lda < (int64_t)1 << 29 && (int64_t)q.M * q.ldy < (int64_t)1 << 29 && (((uintptr_t)q.A | (uintptr_t)q.W) % 16) == 0;
     if (!*done) return 0;
     DecBfParams p{};
