@@ -1,9 +1,9 @@
 // k_layered.hip — kernels of the layered-model engine tier (engine_layered.hip): the
 // mechanisms that the Qwen decoder does not have, each with its constants as parameters.
 //
-//   lay::linear            y = A W^T, fp32 accumulation in k order; A fp32 (optionally rounded to
-//                          bf16 on load), W fp32 or bf16; batched (per head) and grouped (per
-//                          expert) forms
+//   lay::linear            y = A W^T, fp32 accumulation; A fp32 (optionally rounded to bf16 on
+//                          load), W fp32 or bf16; batched (per head) and grouped (per expert)
+//                          forms; the kernels here and those it hands to (k_layered.hpp)
 //   lay::latent_post       latent KV: RMS norm of the compressed row, rotate-half rotary of the
 //                          shared key part and of every head's rotated query part, paged append
 //   lay::latent_attention  sliding-window attention over the latent cache in absorbed form
@@ -17,8 +17,8 @@
 //   lay::silu_mul, embed_rows, final_rows, rows_to_bf16
 //
 // Everything the residual stream, a norm, a router, a score or a softmax touches is fp32.  No
-// result depends on which other rows are in the launch: every output element is reduced in an
-// order fixed by its own sizes.
+// result depends on what other rows are in the launch: every output element is reduced in an
+// order fixed by the launch's sizes.
 #include "k_layered.hpp"
 
 namespace qie {
