@@ -29,6 +29,7 @@ int gemm(const qie_linear_args* a, hipStream_t st);
 bool dec8_applies(const qie_linear_args* a);
 bool dec_bf16_applies(const qie_linear_args* a);
 int dec8_reserve(hipStream_t st);
+void g8_release(hipStream_t st);
 bool persist_supported(const qie_model_spec& s, int B, int tp, bool fp8, bool paged, int ncu, const char** why);
 size_t persist_attn_table_bytes(int n_layers);
 int persist_attn_table(const qie_model_spec& s, const qie_layer_weights* h_layers, const void* qkv_scratch,
@@ -1063,7 +1064,10 @@ void qie_engine_destroy(qie_engine* e) {
     if (e->rope_cos) hipFree(e->rope_cos);
     if (e->rope_sin) hipFree(e->rope_sin);
     if (e->index) qie_index_destroy(e->index);
-    if (e->stream) hipStreamDestroy(e->stream);
+    if (e->stream) {
+        g8_release(e->stream);
+        hipStreamDestroy(e->stream);
+    }
     delete e;
 }
 

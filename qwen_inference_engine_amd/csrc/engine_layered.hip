@@ -24,6 +24,7 @@
 #include <string>
 
 namespace qie {
+void g8_release(hipStream_t st);   // k_gemm.hip
 
 struct HostTensor {
     int dtype = 0;   // 0 bf16 words, 1 int32, 2 fp32
@@ -2565,7 +2566,10 @@ void layered_batch_destroy(qie_batch* b) {
     for (int i = 0; i < LayeredBatch::kSide; i++) {
         if (s->side[i]) hipStreamSynchronize(s->side[i]);
         if (s->ev_join[i]) hipEventDestroy(s->ev_join[i]);
-        if (s->side[i]) hipStreamDestroy(s->side[i]);
+        if (s->side[i]) {
+            g8_release(s->side[i]);
+            hipStreamDestroy(s->side[i]);
+        }
     }
     if (s->ev_fork) hipEventDestroy(s->ev_fork);
     delete s;

@@ -3,6 +3,7 @@
 
 #include "qie_common.hpp"
 #include "../../include/qie/qie_ops.h"
+#include "split_pool.hpp"
 
 namespace qie {
 
@@ -44,8 +45,10 @@ struct G8Split {
 };
 
 // Slabs of 65,536 floats and zeroed tickets of stream `st`, grown on demand; non-zero: they would have to grow during a
-// graph capture (the caller runs unsplit).
+// graph capture, or there is no memory (the caller runs unsplit).  What a capture was given stays valid until g8_release.
 int g8_workspace(hipStream_t st, int slabs, int tiles, G8Split* out);
+// Gives a stream's split-K memory back: before the engine that owns the stream destroys it, its batches' graphs gone.
+void g8_release(hipStream_t st);
 
 // k_gemm_mid.hip: the GEMM of a few dozen to about a thousand rows.  other_us: the expected time of the caller's kernel for
 // this shape; *launched = false: not a shape for this one, or the other is expected to be faster.

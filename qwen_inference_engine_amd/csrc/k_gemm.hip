@@ -967,37 +967,43 @@ static int launch_gemm8(int epi, const GemmParams& p, int n_mt, int n_tiles, con
     return launch_gemm8_t<QIE_EPI_STORE>(p, n_mt, n_tiles, sk, st);
 }
 
-// Split-K slabs + tickets, one set per stream (streams of one device may run GEMMs at the same
+// Split-K slabs + tickets, one pool per stream (streams of one device may run GEMMs at the same
 // time: tensor-parallel ranks on one GPU in the tests), grown on demand outside graph capture.
-struct G8Ws {
-    float* slab = nullptr;
-    unsigned* cnt = nullptr;
-    size_t slab_bytes = 0, cnt_n = 0;
-};
 static std::mutex g8_mu;
-static std::map<hipStream_t, G8Ws> g8_ws;
+static std::map<hipStream_t, SplitPool> g8_pools;
 
 int g8_workspace(hipStream_t st, int slabs, int tiles, G8Split* out) {
     std::lock_guard<std::mutex> lk(g8_mu);
-    G8Ws& w = g8_ws[st];
+    SplitPool& w = g8_pools[st];
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    bool capturing = hipStreamIsCapturing(st, &cs) != hipSuccess;
+    if (capturing) (void)hipGetLastError();   // (the null stream beside another stream's capture)
+    capturing = capturing || cs != hipStreamCaptureStatusNone;
     const size_t need = (size_t)slabs * 65536 * 4;
-    if (need > w.slab_bytes || (size_t)tiles > w.cnt_n) {
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return 1;   // no split
+    if (!w.fits(need, (size_t)tiles)) {
+        if (capturing) return 1;   // no split
         QIE_HIP(hipStreamSynchronize(st));
-        const size_t sb = std::max(need, w.slab_bytes), cn = std::max((size_t)tiles, w.cnt_n);   // never shrink
-        if (w.slab) hipFree(w.slab);
-        if (w.cnt) hipFree(w.cnt);
-        w = G8Ws{};
-        QIE_HIP(hipMalloc((void**)&w.slab, sb));
-        QIE_HIP(hipMalloc((void**)&w.cnt, cn * 4));
-        QIE_HIP(hipMemsetAsync(w.cnt, 0, cn * 4, st));   // ordered before this stream's GEMMs
-        w.slab_bytes = sb;
-        w.cnt_n = cn;
+        const bool ok = w.grow(need, (size_t)tiles, [](size_t n) -> void* {
+            void* p = nullptr;
+            if (hipMalloc(&p, n) == hipSuccess) return p;
+            (void)hipGetLastError();
+            return nullptr;
+        }, [](void* p) { hipFree(p); });
+        if (!ok) return 1;
+        QIE_HIP(hipMemsetAsync(w.cnt, 0, w.cnt_n * 4, st));   // ordered before this stream's GEMMs
     }
+    w.held = w.held || capturing;
     out->slab = w.slab;
     out->cnt = w.cnt;
     return 0;
+}
+
+void g8_release(hipStream_t st) {
+    std::lock_guard<std::mutex> lk(g8_mu);
+    const auto it = g8_pools.find(st);
+    if (it == g8_pools.end()) return;
+    it->second.release([](void* p) { hipFree(p); });
+    g8_pools.erase(it);
 }
 
 template <int EPI>

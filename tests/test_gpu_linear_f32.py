@@ -33,3 +33,36 @@ def test_rows(model, layers, width):  # noqa: F811
     for i, t in enumerate(a):
         assert rel(out[i:i + 1], m.ref(t[:1])) < TOL
     assert rel(out[4:], m.ref(toks + b)[302:]) < TOL
+
+
+def test_replay_after_larger_steps(model):  # noqa: F811
+    """Captured steps keep their split-K memory: steps of 16 rows with four experts each replay after a portion of 60 rows, and
+    after a prompt of another batch on the same engine, made that memory grow."""
+    layers = [gru(width=256, mlp=moe(experts=8, identity=0, top=4, count=1, keep=1, ff=256)), attn(heads=4, kv_heads=2, dim=64, vdim=64, size=40, mlp=None)]
+    m = model(layers, seed=3, vocab=1003, width=256, slots=4, max_ctx=512)
+    seqs = [[], []]
+
+    def small():
+        t = [m.tokens(8), m.tokens(8)]
+        out = m.batch.step([(0, t[0]), (1, t[1])], range(16))
+        for i in range(2):
+            seqs[i] += t[i]
+            assert rel(out[8 * i:8 * i + 8], m.ref(seqs[i])[-8:]) < TOL
+    for _ in range(8):
+        small()
+    graphs, before = m.batch.graph_stats()
+    assert graphs > 0 and before > 0
+    for n in (60, 64):
+        t = m.tokens(n)
+        assert rel(m.batch.step([(2, t)], range(n)), m.ref(t)) < TOL
+        m.batch.release(2)
+        for _ in range(3):
+            small()
+    other = m.eng.batch(1, 512, page_tokens=16)
+    t = m.tokens(300)
+    assert rel(other.step([(0, t)], range(300)), m.ref(t)) < TOL
+    for _ in range(3):
+        small()
+    other.close()
+    small()
+    assert m.batch.graph_stats()[1] > before + 6
