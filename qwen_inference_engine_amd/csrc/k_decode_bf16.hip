@@ -16,7 +16,8 @@
 //     11.1, O 8.8 -> 7.5, gate/up 50.2 -> 48.4; Qwen2-0.5B at 7 rows: QKV 6.4 -> 5.3, O and down 6.5 -> 6.1 a launch.
 //   * The 8 partial tiles meet in LDS, one barrier a tile; the wave that sums them and runs the epilogue rotates.
 //   * SwiGLU: a tile is 8 gate rows and the same outputs' 8 up rows, met across lane halves.
-// One workgroup a CU: LDS holds 64 to 128 KB of chunks.  Sums: per wave over its K share in fp32, the shares in wave order.
+// One workgroup a CU: LDS holds 64 to 128 KB of chunks.  Sums: per wave over its K share in fp32, the shares in wave order (fp32
+// operands: 16 sums a wave, met in pairs).
 #include "qie_common.hpp"
 #include "../../include/qie/qie_ops.h"
 #include "k_layered.hpp"
@@ -72,7 +73,9 @@ __device__ __forceinline__ void db_lds16(__amdgpu_buffer_rsrc_t rs, void* lds, u
 // XM: 0 = X in LDS; 8, 16 = X's chunks (of 8 or 16 rows) through the ring.  NV: 16-byte vectors of a row per lane while X is
 // normed (K <= 512 NV), 0: not normed, its rows go to LDS as they are; R: ring slots a wave.
 // F32: rows of fp32 instead (p.K, p.ldx in 16-bit units; the fp32 epilogue, no norm): a 16-byte piece is 4 k, four
-// v_mfma_f32_16x16x4f32 instead of one v_mfma_f32_16x16x32_bf16.
+// v_mfma_f32_16x16x4f32 instead of one v_mfma_f32_16x16x32_bf16.  Each of a chunk's 16 instructions has a sum of its own, and
+// these and the waves' meet in pairs: a sum is a chain of K / 128 terms at most, not of K / 8 (the Lugipel design at width 1,024,
+// decode steps against 64 bits: 4.5e-7 to 5.6e-7 of the logits with one chain a wave, 2.5e-7 to 3.2e-7 so; the column-per-wave kernel 3.4e-7 to 4.2e-7).
 template <int EPI, int XM, int NV, int R, bool F32 = false>
 __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
 #pragma clang fp contract(off)
@@ -264,7 +267,11 @@ __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
     int done = 0, slot = 0;
     for (int it = 0; it < mine; it++) {
         const int tile = blockIdx.x + it * G;
-        db_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        db_f32x4 acc = {0.f, 0.f, 0.f, 0.f}, af[F32 ? 16 : 1];
+        if constexpr (F32) {
+#pragma unroll
+            for (int i = 0; i < 16; i++) af[i] = acc;
+        }
         for (int c = 0; c < cnt; c++) {
             // the oldest chunk has landed: R - 1 younger ones may fly (fewer at the end of the stream)
             if (done + R <= items) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(IPC * (R - 1)) : "memory");
@@ -285,7 +292,7 @@ __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
                 if constexpr (F32) {
                     const db_f32x4 a = __builtin_bit_cast(db_f32x4, wf[s]), b = __builtin_bit_cast(db_f32x4, xf[s]);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], acc, 0, 0, 0);
+                    for (int e = 0; e < 4; e++) af[4 * s + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], af[4 * s + e], 0, 0, 0);
                 } else {
                     acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[s], xf[s], acc, 0, 0, 0);
                 }
@@ -296,6 +303,13 @@ __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
             done++;
             slot = slot + 1 == R ? 0 : slot + 1;
         }
+        if constexpr (F32) {
+#pragma unroll
+            for (int o = 8; o >= 1; o >>= 1)
+#pragma unroll
+                for (int i = 0; i < o; i++) af[i] = af[i] + af[i + o];
+            acc = af[0];
+        }
         if (fr < 8 || M > 8) red[((it & 1) * db::NW + wave) * RS + rl] = acc;
         // one barrier a tile: a slot of `red` is written again two tiles on, behind the next tile's barrier, which the summing
         // wave reaches only after its reads.  (No vmcnt wait: the ring's loads stay in flight.)
@@ -305,8 +319,15 @@ __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
         __builtin_amdgcn_sched_barrier(0);
         if (wave != it % db::NW) continue;   // wave-uniform
         db_f32x4 v = red[(it & 1) * db::NW * RS + rl];
+        if constexpr (F32) {
+            db_f32x4 u[db::NW];
 #pragma unroll
-        for (int w = 1; w < db::NW; w++) v = v + red[((it & 1) * db::NW + w) * RS + rl];
+            for (int w = 0; w < db::NW; w++) u[w] = red[((it & 1) * db::NW + w) * RS + rl];
+            v = ((u[0] + u[1]) + (u[2] + u[3])) + ((u[4] + u[5]) + (u[6] + u[7]));
+        } else {
+#pragma unroll
+            for (int w = 1; w < db::NW; w++) v = v + red[((it & 1) * db::NW + w) * RS + rl];
+        }
         const Tile t = tile_at(tile);
         // lane: row m = fr of X, columns 4 g .. 4 g + 3 of the tile (SwiGLU: g = 0, 1 gate, g = 2, 3 the same outputs' up)
         const int m = fr;

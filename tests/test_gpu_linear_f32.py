@@ -66,3 +66,23 @@ def test_replay_after_larger_steps(model):  # noqa: F811
     other.close()
     small()
     assert m.batch.graph_stats()[1] > before + 6
+
+
+@pytest.mark.parametrize("width", [2048, 3072])   # X in LDS, through the ring
+def test_sums_of_equal_terms(model, width):  # noqa: F811
+    """Few rows, every product of a sum the same: a serial chain of fp32 additions drifts off by up to half an ulp of the running
+    sum each (width / 8 terms: 60 to 90 units of 2^-24), sums of width / 128 terms that meet in pairs cannot."""
+    def tweak(T, cfg):
+        T["l0.mix.o"][:] = 0                                             # the row stays what the embedding makes it
+        T["embed"][:] = np.where(np.arange(width) % 2 == 0, 2.0, 0.0)    # with position 0's sines and cosines: ones
+        T["final.norm"][:] = 1.0
+        T["head"][:] = (1.0 + np.arange(8) / 64.0)[np.arange(503) % 8, None]
+    m = model([gru(width=64, mlp=None)], seed=5, vocab=503, width=width, slots=16, max_ctx=64, tweak=tweak)
+    want = width * m.W64["head"][:, 0] / np.sqrt(1.0 + 1e-5)
+    # a chain's terms and the seven pairings of 16 x 8 sums, a rounding each; four more for the norm's quotient, its root and its products
+    bound = (width // 128 + 7 + 4) * 2.0 ** -24
+    for rows in (1, 5, 16):
+        got = m.batch.step([(i, m.tokens(1)) for i in range(rows)], range(rows))
+        assert (np.abs(got / want - 1.0) <= bound).all()
+        for i in range(rows):
+            m.batch.release(i)
