@@ -17,8 +17,9 @@
 //   lay::silu_mul, embed_rows, final_rows, rows_to_bf16
 //
 // Everything the residual stream, a norm, a router, a score or a softmax touches is fp32.  No
-// result depends on what other rows are in the launch: every output element is reduced in an
-// order fixed by the launch's sizes.
+// result depends on which other rows are in the launch: every output element is reduced in an
+// order fixed by its own sizes, by the kernel that its product takes (how many rows there are
+// decides between kernels, k_layered.hpp) and by nothing else.
 #include "k_layered.hpp"
 
 namespace qie {

@@ -5,8 +5,11 @@
 //
 // The FMA kernel it replaces (k_layered.hip linear_kernel) keeps nothing in flight and fills 32 to 80 of 256 CUs at a few
 // hundred rows: 145 to 230 us for 1 to 2 GFLOP.  Here a 64 x 64 tile goes through an LDS-DMA ring of 32-k tiles (128-byte rows,
-// as k_gemm_mid.hip), 8 waves as 2 x 2 x 2 K halves, and tiles that do not fill the chip are split over K (slabs summed in part
-// order by the last part, gemm8_kernel's protocol).  Bound: the fp32 matrix rate (157 TFLOP/s) or, at few rows, the weights.
+// as k_gemm_mid.hip), 8 waves as 2 x 2 x 2 K halves, and tiles that do not fill the chip are split over K (slabs summed by the
+// last part, gemm8_kernel's protocol).  Bound: the fp32 matrix rate (157 TFLOP/s) or, at few rows, the weights.
+//   * The order of a sum depends on K alone: K is cut into 1 to 16 segments (a power of two), a wave's segment sums meet in pairs,
+//     pairs of pairs and so on, and at last the two K halves.  A workgroup owns an aligned group of segments, one node of that tree,
+//     so how many workgroups share a tile (by the rows of the launch and the memory there is for slabs) changes no bit.
 #include "gemm_impl.hpp"
 #include "k_layered.hpp"
 
@@ -18,16 +21,41 @@ namespace lay {
 namespace lf {
 constexpr int BM = 64, BN = 64, BK = 32, SLOTS = 4;
 constexpr int SLOT = (BM + BN) * BK * 4;   // A rows, then W rows, 128 B each
+constexpr int LEVELS = 4;                  // of the tree of segments: 16 at most
+constexpr int SLAB = 2 * BM * BN;          // floats of a part: both K halves
 }
 
 struct LinF32P {
     LinearP q;
-    int parts;          // K ranges per tile
+    int log_segs;       // K segments, as a power of two
+    int log_parts;      // workgroups per tile
     int n_nt, n_mt;     // tiles of N; tiles of M per group (of the most rows a group may have)
     int vec;            // rows of Y take 16-byte stores
-    float* slab;        // [tile][part][64 * 64]
+    float* slab;        // [tile][part][K half][64 * 64]
     unsigned* cnt;      // [tile], zero at rest
 };
+
+// Node `i` (0, 1, 2, ... of its level) of a binary tree of 2^log_n nodes arrives in v; lvl[l] holds a left node that waits for its
+// right sibling.  true: it was the last one, v is the tree's root.
+template <int L = 0>
+__device__ __forceinline__ bool lf_meet(f32x4 (&v)[2][2], f32x4 (&lvl)[lf::LEVELS][2][2], int i, int log_n) {
+    if constexpr (L < lf::LEVELS) {
+        if (L == log_n) return true;
+        if (!((i >> L) & 1)) {
+#pragma unroll
+            for (int a = 0; a < 2; a++)
+#pragma unroll
+                for (int b = 0; b < 2; b++) lvl[L][a][b] = v[a][b];
+            return false;
+        }
+#pragma unroll
+        for (int a = 0; a < 2; a++)
+#pragma unroll
+            for (int b = 0; b < 2; b++) v[a][b] = lvl[L][a][b] + v[a][b];
+        return lf_meet<L + 1>(v, lvl, i, log_n);
+    }
+    return true;
+}
 
 __global__ __launch_bounds__(512) void linear_f32_kernel(LinF32P p) {
 #pragma clang fp contract(off)
@@ -47,8 +75,9 @@ __global__ __launch_bounds__(512) void linear_f32_kernel(LinF32P p) {
     if (m0 >= m_hi) return;   // block-uniform
     const float* A = p.q.A + (int64_t)z * p.q.sA;
     const float* W = (const float*)p.q.W + (int64_t)z * p.q.sW;
-    const int nk_all = p.q.K / BK;
-    const int kb = (int)((int64_t)part * nk_all / p.parts), nk = (int)((int64_t)(part + 1) * nk_all / p.parts) - kb;
+    const int nk_all = p.q.K / BK, log_own = p.log_segs - p.log_parts, parts = 1 << p.log_parts;
+    auto seg_at = [&](int seg) { return (int)(((int64_t)seg * nk_all) >> p.log_segs); };   // first k-tile of a segment
+    const int seg0 = part << log_own, kb = seg_at(seg0), nk = seg_at((part + 1) << log_own) - kb;
 
     // LDS-DMA: instruction i of this wave fills rows 8 b .. 8 b + 7, b = 8 i + wave (i = 0: A, 1: W)
     const float* src[2];
@@ -64,11 +93,15 @@ __global__ __launch_bounds__(512) void linear_f32_kernel(LinF32P p) {
         glds16(src[0] + (int64_t)kt * BK, dst);
         glds16(src[1] + (int64_t)kt * BK, dst + 8192);
     };
-    f32x4 acc[2][2];
+    f32x4 acc[2][2], lvl[LEVELS][2][2];
+    auto clear = [&]() {
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+        for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < 2; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    };
+    clear();
+    int seg = 0, seg_end = seg_at(seg0 + 1) - kb;
     for (int t = 0; t < SLOTS - 1 && t < nk; t++) stage(t, t);
     int slot = 0, fill = SLOTS - 1;
     for (int t = 0; t < nk; t++) {
@@ -102,6 +135,53 @@ __global__ __launch_bounds__(512) void linear_f32_kernel(LinF32P p) {
         __builtin_amdgcn_sched_barrier(0);
         slot = slot + 1 == SLOTS ? 0 : slot + 1;
         fill = fill + 1 == SLOTS ? 0 : fill + 1;
+        if (t + 1 == seg_end) {   // uniform
+            if (!lf_meet(acc, lvl, seg, log_own)) clear();   // (the last segment's: acc is this workgroup's node)
+            seg++;
+            seg_end = seg_at(seg0 + seg + 1) - kb;
+        }
+    }
+    if (parts > 1) {
+        const int64_t tile = ((int64_t)z * p.n_mt + mt) * p.n_nt + nt;
+        const auto rs = __builtin_amdgcn_make_buffer_rsrc(p.slab + ((tile << p.log_parts) + part) * SLAB, (short)0, SLAB * 4, 0x00020000);
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_g8, acc[i][j]), rs, ((wave * 4 + i * 2 + j) * 64 + lane) * 16, 0, 16);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        int* flag = reinterpret_cast<int*>(smem);
+        if (tid == 0) {
+            const unsigned old = __hip_atomic_fetch_add(p.cnt + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            *flag = old == (unsigned)parts - 1 ? 1 : 0;
+        }
+        __syncthreads();
+        if (*flag == 0) return;   // uniform
+        constexpr int QN = 4;     // parts in flight
+        for (int q0 = 0; q0 < parts; q0 += QN) {
+            f32x4 v[QN][2][2];
+#pragma unroll
+            for (int u = 0; u < QN; u++) {
+                const int q = q0 + u < parts ? q0 + u : parts - 1;
+                const auto rq = __builtin_amdgcn_make_buffer_rsrc(p.slab + ((tile << p.log_parts) + q) * SLAB, (short)0, SLAB * 4, 0x00020000);
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++)
+                        v[u][i][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rq, ((wave * 4 + i * 2 + j) * 64 + lane) * 16, 0, 16));
+            }
+            // the tree's first two levels here, the others by their waiting nodes
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    const f32x4 lo = v[0][i][j] + v[1][i][j];
+                    acc[i][j] = parts == 2 ? lo : lo + (v[2][i][j] + v[3][i][j]);
+                }
+            if (parts > 2) lf_meet<2>(acc, lvl, q0, p.log_parts);
+        }
+        if (tid == 0) __hip_atomic_store(p.cnt + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     // the two K halves: wave w and w ^ 4 hold the same tile, each keeps one of its two row fragments
     f32x4 res[2];
@@ -119,41 +199,6 @@ __global__ __launch_bounds__(512) void linear_f32_kernel(LinF32P p) {
             const f32x4 o = ex[((wave ^ 4) * 2 + j) * 64 + lane];
             res[j] = wk == 0 ? res[j] + o : o + res[j];
         }
-    }
-    if (p.parts > 1) {
-        const int64_t tile = ((int64_t)z * p.n_mt + mt) * p.n_nt + nt;
-        const auto rs = __builtin_amdgcn_make_buffer_rsrc(p.slab + (tile * p.parts + part) * 4096, (short)0, 16384, 0x00020000);
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_g8, res[j]), rs, ((wave * 2 + j) * 64 + lane) * 16, 0, 16);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        int* flag = reinterpret_cast<int*>(smem);
-        if (tid == 0) {
-            const unsigned old = __hip_atomic_fetch_add(p.cnt + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            *flag = old == (unsigned)p.parts - 1 ? 1 : 0;
-        }
-        __syncthreads();
-        if (*flag == 0) return;   // uniform
-        constexpr int QN = 8;     // parts in flight
-        for (int q0 = 0; q0 < p.parts; q0 += QN) {
-            f32x4 v[QN][2];
-#pragma unroll
-            for (int u = 0; u < QN; u++) {
-                const int q = q0 + u < p.parts ? q0 + u : p.parts - 1;
-                const auto rq = __builtin_amdgcn_make_buffer_rsrc(p.slab + (tile * p.parts + q) * 4096, (short)0, 16384, 0x00020000);
-#pragma unroll
-                for (int j = 0; j < 2; j++)
-                    v[u][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rq, ((wave * 2 + j) * 64 + lane) * 16, 0, 16));
-            }
-#pragma unroll
-            for (int u = 0; u < QN; u++) {
-                if (q0 + u >= p.parts) break;
-#pragma unroll
-                for (int j = 0; j < 2; j++) res[j] = q0 + u == 0 ? v[u][j] : res[j] + v[u][j];
-            }
-        }
-        if (tid == 0) __hip_atomic_store(p.cnt + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     const int m = m0 + wm * 32 + wk * 16 + fr;
     if (m >= m_hi) return;
@@ -182,21 +227,22 @@ int linear_f32(const LinearP& q, hipStream_t st, bool* done) {
     p.n_nt = (q.N + BN - 1) / BN;
     p.n_mt = (q.M + BM - 1) / BM;   // (grouped: one group may hold every row; the other groups' blocks leave at once)
     p.vec = q.ldy % 4 == 0 && q.sY % 4 == 0 && (uintptr_t)q.Y % 16 == 0;
-    // K ranges: until about 512 workgroups (two a CU) have work, each keeping 4 k-tiles.  Grouped: rows spread over the groups
+    // Workgroups a tile: until about 512 (two a CU) have work, each keeping 4 k-tiles.  Grouped: rows spread over the groups
     const int64_t mts = q.grp_off ? std::max<int64_t>(q.batch, (q.M + BM - 1) / BM + q.batch / 2) : (int64_t)p.n_mt * q.batch;
     const int64_t tiles = (int64_t)p.n_nt * p.n_mt * q.batch;   // of the grid
-    int parts = (int)std::max<int64_t>(1, std::min<int64_t>({16, 2 * (int64_t)device_cu_count() / (mts * p.n_nt), q.K / BK / 4}));
-    if (parts > 1) {
+    const int64_t want = std::min<int64_t>(2 * (int64_t)device_cu_count() / (mts * p.n_nt), q.K / BK / 4);
+    while (p.log_segs < LEVELS && (q.K / BK / 4) >> (p.log_segs + 1)) p.log_segs++;
+    while (p.log_parts < p.log_segs && want >> (p.log_parts + 1)) p.log_parts++;
+    if (p.log_parts > 0) {
         G8Split ws{1, nullptr, nullptr};
-        const int64_t slabs = (tiles * parts * 4096 + 65535) / 65536;
-        if (tiles > (1 << 20) || slabs > 2048 || g8_workspace(st, (int)slabs, (int)tiles, &ws) != 0) parts = 1;   // 512 MB at most
+        const int64_t slabs = ((tiles << p.log_parts) * SLAB + 65535) / 65536;
+        if (tiles > (1 << 20) || slabs > 2048 || g8_workspace(st, (int)slabs, (int)tiles, &ws) != 0) p.log_parts = 0;   // 512 MB at most
         p.slab = ws.slab;
         p.cnt = ws.cnt;
     }
-    p.parts = parts;
     constexpr size_t shm = (size_t)SLOTS * SLOT;
     static_assert(shm <= 65536, "linear_f32: default LDS");
-    hipLaunchKernelGGL(linear_f32_kernel, dim3((unsigned)(p.n_nt * parts), (unsigned)p.n_mt, (unsigned)q.batch), dim3(512), shm, st, p);
+    hipLaunchKernelGGL(linear_f32_kernel, dim3((unsigned)(p.n_nt << p.log_parts), (unsigned)p.n_mt, (unsigned)q.batch), dim3(512), shm, st, p);
     QIE_LAUNCH_CHECK();
     return 0;
 }

@@ -86,3 +86,19 @@ def test_sums_of_equal_terms(model, width):  # noqa: F811
         assert (np.abs(got / want - 1.0) <= bound).all()
         for i in range(rows):
             m.batch.release(i)
+
+
+def test_rows_beside_others(model):  # noqa: F811
+    """A prompt's logits are the same bits alone and beside other prompts (more rows: fewer workgroups share a tile's sums)."""
+    layers = [attn(heads=4, kv_heads=2, dim=64, vdim=64, size=70, mlp=dense(1440)), attn(heads=4, kv_heads=2, dim=64, vdim=64, size=70, mlp=moe(experts=6, identity=2, top=2, ff=352))]
+    m = model(layers, seed=9, vocab=1003, width=512, slots=3, max_ctx=512)
+    t, others = m.tokens(40), [m.tokens(30), m.tokens(400)]
+    want = m.batch.step([(0, t)], range(40))
+    assert rel(want, m.ref(t)) < TOL
+    for o in others:
+        m.batch.release(0)
+        m.batch.release(1)
+        assert np.array_equal(m.batch.step([(1, o), (0, t)], range(len(o), len(o) + 40)), want)
+        m.batch.release(0)
+        m.batch.release(1)
+        assert np.array_equal(m.batch.step([(0, t), (1, o)], range(40 + len(o)))[:40], want)
