@@ -19,8 +19,8 @@ int send(const SendP& p, hipStream_t st);
 
 // y[m, n] = sum_k A[m, k] W[n, k] (+ batch z: A + z sA, W + z sW, Y + z sY).  A fp32, rounded to
 // bf16 on load when round_a; W fp32 or bf16 words; Y fp32.  grp_off (device, batch + 1 entries):
-// batch z covers rows [grp_off[z], grp_off[z + 1]) of A and Y (M is then the largest row count a
-// group can have).  By shape: fp32 weights on the 16-byte grid take the fp32 matrix cores (up to 16 rows streamed,
+// batch z covers rows [grp_off[z], grp_off[z + 1]) of A and Y, all inside [0, M) (M is the largest
+// row count a group can have).  By shape: fp32 weights on the 16-byte grid take the fp32 matrix cores (up to 16 rows streamed,
 // k_decode_bf16.hip; else tiles through an LDS-DMA ring, k_linear_f32.hip; grouped rows from 33 on), up to 32 rows a
 // column-per-wave kernel, many rows of a bf16 model (mfma) MFMA tiles from memory, else 64 x 64 fp32 tiles through LDS; an
 // element's sum never depends on what else the launch holds, only on which of them ran.

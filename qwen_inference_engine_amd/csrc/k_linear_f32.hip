@@ -11,6 +11,7 @@
 //     pairs of pairs and so on, and at last the two K halves.  A workgroup owns an aligned group of segments, one node of that tree,
 //     so how many workgroups share a tile (by the rows of the launch and the memory there is for slabs) changes no bit.
 #include "gemm_impl.hpp"
+#include "gemm_plan.hpp"
 #include "k_layered.hpp"
 
 #include <algorithm>
@@ -19,17 +20,14 @@ namespace qie {
 namespace lay {
 
 namespace lf {
-constexpr int BM = 64, BN = 64, BK = 32, SLOTS = 4;
+using namespace qie::lf;                   // gemm_plan.hpp
+constexpr int SLOTS = 4;
 constexpr int SLOT = (BM + BN) * BK * 4;   // A rows, then W rows, 128 B each
-constexpr int LEVELS = 4;                  // of the tree of segments: 16 at most
-constexpr int SLAB = 2 * BM * BN;          // floats of a part: both K halves
 }
 
 struct LinF32P {
     LinearP q;
-    int log_segs;       // K segments, as a power of two
-    int log_parts;      // workgroups per tile
-    int n_nt, n_mt;     // tiles of N; tiles of M per group (of the most rows a group may have)
+    lf::Plan pl;
     int vec;            // rows of Y take 16-byte stores
     float* slab;        // [tile][part][K half][64 * 64]
     unsigned* cnt;      // [tile], zero at rest
@@ -65,7 +63,7 @@ __global__ __launch_bounds__(512) void linear_f32_kernel(LinF32P p) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wk = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
     const int fr = lane & 15, g = lane >> 4;
-    const int z = blockIdx.z, nt = blockIdx.x % p.n_nt, part = blockIdx.x / p.n_nt, mt = blockIdx.y;
+    const int z = blockIdx.z, nt = blockIdx.x % p.pl.n_nt, part = blockIdx.x / p.pl.n_nt, mt = blockIdx.y;
     int m_lo = 0, m_hi = p.q.M;
     if (p.q.grp_off) {
         m_lo = p.q.grp_off[z];
@@ -75,8 +73,8 @@ __global__ __launch_bounds__(512) void linear_f32_kernel(LinF32P p) {
     if (m0 >= m_hi) return;   // block-uniform
     const float* A = p.q.A + (int64_t)z * p.q.sA;
     const float* W = (const float*)p.q.W + (int64_t)z * p.q.sW;
-    const int nk_all = p.q.K / BK, log_own = p.log_segs - p.log_parts, parts = 1 << p.log_parts;
-    auto seg_at = [&](int seg) { return (int)(((int64_t)seg * nk_all) >> p.log_segs); };   // first k-tile of a segment
+    const int nk_all = p.q.K / BK, log_own = p.pl.log_segs - p.pl.log_parts, parts = 1 << p.pl.log_parts;
+    auto seg_at = [&](int seg) { return (int)(((int64_t)seg * nk_all) >> p.pl.log_segs); };   // first k-tile of a segment
     const int seg0 = part << log_own, kb = seg_at(seg0), nk = seg_at((part + 1) << log_own) - kb;
 
     // LDS-DMA: instruction i of this wave fills rows 8 b .. 8 b + 7, b = 8 i + wave (i = 0: A, 1: W)
@@ -142,8 +140,8 @@ __global__ __launch_bounds__(512) void linear_f32_kernel(LinF32P p) {
         }
     }
     if (parts > 1) {
-        const int64_t tile = ((int64_t)z * p.n_mt + mt) * p.n_nt + nt;
-        const auto rs = __builtin_amdgcn_make_buffer_rsrc(p.slab + ((tile << p.log_parts) + part) * SLAB, (short)0, SLAB * 4, 0x00020000);
+        const int64_t tile = row_tile(p.q.grp_off != nullptr, m0, z, mt, p.pl.n_mt) * p.pl.n_nt + nt;
+        const auto rs = __builtin_amdgcn_make_buffer_rsrc(p.slab + ((tile << p.pl.log_parts) + part) * SLAB, (short)0, SLAB * 4, 0x00020000);
 #pragma unroll
         for (int i = 0; i < 2; i++)
 #pragma unroll
@@ -164,7 +162,7 @@ __global__ __launch_bounds__(512) void linear_f32_kernel(LinF32P p) {
 #pragma unroll
             for (int u = 0; u < QN; u++) {
                 const int q = q0 + u < parts ? q0 + u : parts - 1;
-                const auto rq = __builtin_amdgcn_make_buffer_rsrc(p.slab + ((tile << p.log_parts) + q) * SLAB, (short)0, SLAB * 4, 0x00020000);
+                const auto rq = __builtin_amdgcn_make_buffer_rsrc(p.slab + ((tile << p.pl.log_parts) + q) * SLAB, (short)0, SLAB * 4, 0x00020000);
 #pragma unroll
                 for (int i = 0; i < 2; i++)
 #pragma unroll
@@ -179,7 +177,7 @@ __global__ __launch_bounds__(512) void linear_f32_kernel(LinF32P p) {
                     const f32x4 lo = v[0][i][j] + v[1][i][j];
                     acc[i][j] = parts == 2 ? lo : lo + (v[2][i][j] + v[3][i][j]);
                 }
-            if (parts > 2) lf_meet<2>(acc, lvl, q0, p.log_parts);
+            if (parts > 2) lf_meet<2>(acc, lvl, q0, p.pl.log_parts);
         }
         if (tid == 0) __hip_atomic_store(p.cnt + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -224,25 +222,19 @@ int linear_f32(const LinearP& q, hipStream_t st, bool* done) {
     if (!*done) return 0;
     LinF32P p{};
     p.q = q;
-    p.n_nt = (q.N + BN - 1) / BN;
-    p.n_mt = (q.M + BM - 1) / BM;   // (grouped: one group may hold every row; the other groups' blocks leave at once)
+    // (grouped: one group may hold every row; the other groups' blocks leave at once)
+    p.pl = lf::plan(q.M, q.N, q.K, q.batch, q.grp_off != nullptr, device_cu_count());
     p.vec = q.ldy % 4 == 0 && q.sY % 4 == 0 && (uintptr_t)q.Y % 16 == 0;
-    // Workgroups a tile: until about 512 (two a CU) have work, each keeping 4 k-tiles.  Grouped: rows spread over the groups
-    const int64_t mts = q.grp_off ? std::max<int64_t>(q.batch, (q.M + BM - 1) / BM + q.batch / 2) : (int64_t)p.n_mt * q.batch;
-    const int64_t tiles = (int64_t)p.n_nt * p.n_mt * q.batch;   // of the grid
-    const int64_t want = std::min<int64_t>(2 * (int64_t)device_cu_count() / (mts * p.n_nt), q.K / BK / 4);
-    while (p.log_segs < LEVELS && (q.K / BK / 4) >> (p.log_segs + 1)) p.log_segs++;
-    while (p.log_parts < p.log_segs && want >> (p.log_parts + 1)) p.log_parts++;
-    if (p.log_parts > 0) {
+    if (p.pl.log_parts > 0) {
         G8Split ws{1, nullptr, nullptr};
-        const int64_t slabs = ((tiles << p.log_parts) * SLAB + 65535) / 65536;
-        if (tiles > (1 << 20) || slabs > 2048 || g8_workspace(st, (int)slabs, (int)tiles, &ws) != 0) p.log_parts = 0;   // 512 MB at most
+        const int64_t tiles = p.pl.row_tiles * p.pl.n_nt, slabs = ((tiles << p.pl.log_parts) * SLAB + 65535) / 65536;
+        if (g8_workspace(st, (int)slabs, (int)tiles, &ws) != 0) p.pl.log_parts = 0;
         p.slab = ws.slab;
         p.cnt = ws.cnt;
     }
     constexpr size_t shm = (size_t)SLOTS * SLOT;
     static_assert(shm <= 65536, "linear_f32: default LDS");
-    hipLaunchKernelGGL(linear_f32_kernel, dim3((unsigned)(p.n_nt << p.log_parts), (unsigned)p.n_mt, (unsigned)q.batch), dim3(512), shm, st, p);
+    hipLaunchKernelGGL(linear_f32_kernel, dim3((unsigned)(p.pl.n_nt << p.pl.log_parts), (unsigned)p.pl.n_mt, (unsigned)q.batch), dim3(512), shm, st, p);
     QIE_LAUNCH_CHECK();
     return 0;
 }
