@@ -100,7 +100,7 @@ __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
     // ---- X rows for the norm (or the copy), loaded ahead of the first weight chunks: P waves a row (8, 4, 2 rows at a time), so
     // that few rows keep every wave busy.  (Buffer loads throughout: a load is one instruction with its offset in a scalar register,
     // and what lies past K reads zeros.  With 64-bit addresses and a bounds test a lane the prologue was ~2,000 instructions.)
-    const int P = M <= 2 ? 4 : M <= 4 ? 2 : 1, rows_at = db::NW / P, sub = wave % P;
+    const int P = M <= 2 ? 4 : M <= 4 ? 2 : 1, sub = wave % P;
     db_u32x4 xv[NV ? NV : 1], nv[NV ? NV : 1];
     auto load_row = [&](int m) {
         const auto rx = db_rsrc(p.x + (int64_t)m * p.ldx, (uint32_t)K * 2), rn = db_rsrc(p.norm_w, (uint32_t)K * 2);
@@ -211,26 +211,35 @@ __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
 
     if constexpr (XM == 0) {
         if constexpr (NV > 0) {   // M <= 8: one pass
+            // The sum of squares in qie_rmsnorm's order, whatever P is: a row's 512-k pieces go to four sums in turn, each over a wave.
             const int m = wave / P;
-            float* ssq = reinterpret_cast<float*>(red);
-            float ss = 0.f;
+            float* ssq = reinterpret_cast<float*>(red);   // [row][4]
+            auto squares = [&](auto pc) {
+                constexpr int PP = decltype(pc)::value, S = 4 / PP;   // this wave's sums: pieces v PP + sub, v = j, j + S, ...
+                float ss[S] = {};
 #pragma unroll
-            for (int v = 0; v < NV; v++) {
-                if ((v * P + sub) * 512 >= K) break;
-                const uint32_t e[4] = {xv[v].x, xv[v].y, xv[v].z, xv[v].w};
+                for (int v = 0; v < NV; v++) {
+                    if ((v * PP + sub) * 512 >= K) break;
+                    const uint32_t e[4] = {xv[v].x, xv[v].y, xv[v].z, xv[v].w};
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const float a = bf_lo(e[j]), b = bf_hi(e[j]);
-                    ss += a * a + b * b;
+                    for (int j = 0; j < 4; j++) {
+                        const float a = bf_lo(e[j]), b = bf_hi(e[j]);
+                        ss[v % S] += a * a + b * b;
+                    }
                 }
-            }
-            ss = wave_sum(ss);
-            if (lane == 0) ssq[wave] = ss;
+#pragma unroll
+                for (int j = 0; j < S; j++) {
+                    const float t = wave_sum(ss[j]);
+                    if (lane == 0) ssq[m * 4 + j * PP + sub] = t;
+                }
+            };
+            if (P == 1) squares(std::integral_constant<int, 1>{});
+            else if (P == 2) squares(std::integral_constant<int, 2>{});
+            else squares(std::integral_constant<int, 4>{});
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (not __syncthreads: the chunks in flight stay there)
             __builtin_amdgcn_s_barrier();
             __builtin_amdgcn_sched_barrier(0);
-            float tot = 0.f;
-            for (int q = 0; q < P; q++) tot += ssq[wave - sub + q];
+            const float tot = ssq[m * 4] + ssq[m * 4 + 1] + ssq[m * 4 + 2] + ssq[m * 4 + 3];
             const float rms = sqrtf((tot / (float)K) + p.eps), inv = 1.0f / rms, rr = rms < INFINITY ? rms : 0.f;
             auto apply = [&](auto hf) {
                 constexpr bool HF = decltype(hf)::value;

@@ -88,3 +88,25 @@ def test_norm_and_keys(qlib, oracle, M, K, num):
     ids = G.zeros((M,), np.int32)
     G.check(qlib.qie_keys_to_ids(G.p(keys), M, G.p(ids), None), "keys")
     assert [int(i) for i in ids.numpy()] == [oracle.argmax(got[m]) for m in range(M)]
+
+
+@pytest.mark.parametrize("K", [512, 896, 2048, 2560, 3584, 5120])
+@pytest.mark.parametrize("num", [0, 1])
+def test_fused_norm_is_the_separate_one(qlib, K, num):
+    """The norm inside the projection gives qie_rmsnorm's bits, so a row's result does not hang on how many rows share the step."""
+    N, eps = 40, 1e-6
+    nw, w = bf16((K,), 1.0, 22), bf16((N, K), K ** -0.5, 23)
+    dn, dw, xn = G.dev(nw), G.dev(w), G.zeros_bf16(8, K)
+    r = np.random.default_rng(K)
+    for _ in range(24):   # (an ulp of the root moves one element in 2^15 to another bf16 or so: rows enough to meet some)
+        dx = G.dev(G.to_bf16(r.standard_normal((8, K)) * 2.0 ** r.uniform(-6, 6, (8, K))))
+        G.check(qlib.qie_rmsnorm(G.p(dx), G.p(dn), G.p(xn), 8, K, eps, num, None), "rmsnorm")
+        want = G.zeros((8, N), np.float32)
+        linear(xn, [dw], [], 8, K, N, want, _lib.QIE_EPI_F32)
+        want = want.numpy()
+        for M in range(2, 9):
+            y, a = G.zeros((M, N), np.float32), _lib.LinearArgsC()
+            a.x, a.ldx, a.w[0], a.seg_rows[0], a.M, a.K, a.N = G.p(dx), K, G.p(dw), N, M, K, N
+            a.y, a.ldy, a.epilogue, a.numerics, a.norm_w, a.norm_eps = G.p(y), N, _lib.QIE_EPI_F32, num, G.p(dn), eps
+            G.check(qlib.qie_linear(C.byref(a), None), "qie_linear")
+            assert np.array_equal(y.numpy(), want[:M]), M
