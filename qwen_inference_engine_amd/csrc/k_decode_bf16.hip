@@ -447,11 +447,24 @@ struct DbPlan {
     int xm, nv, r;
     size_t lds;
 };
+// Plain rows where the skinny kernel stays ahead, at fewer than 8 rows: its waves divide K of 512, 1,024 and 2,048 without a rest, and
+// here half of them have no chunk at 512.  us, skinny | this one, at 2 and 4 rows: 512 x 8,192 gated 6.1 6.9 | 7.9 7.9, 512 x 2,048
+// 3.4 3.5 | 3.7 3.8, 1,024 x 8,192 gated 9.1 9.7 | 10.6 10.8, 2,048 x 8,192 9.3 9.7 | 11.2 11.7, 2,048 x 48,000 37.0 39.3 | 41.6 42.4;
+// but 512 x 14,336 8.7 9.1 | 7.0 7.1, 640 x 8,192 6.3 6.5 | 5.5 5.6, 2,176 x 8,192 11.3 11.8 | 9.9 9.7, and fp32 outputs (layered
+// models) 2,048 x 14,336 15.9 15.4 | 14.4 14.6.  With a norm the skinny kernel needs another launch.
+bool db_skinny_ahead(const qie_linear_args* a) {
+    if (a->norm_w || a->M >= 8) return false;
+    const bool gated = a->epilogue == QIE_EPI_SWIGLU;
+    const int64_t rows = gated ? 2 * a->N : a->N;
+    if (a->K == 512) return gated || rows <= 8192;
+    return (a->K == 1024 || a->K == 2048) && rows >= 8192 && a->epilogue != QIE_EPI_F32;
+}
 bool db_plan(const qie_linear_args* a, DbPlan* out) {
     if (dev_env("QIE_DEC_BF16", 1) == 0) return false;
     if ((a->flags & QIE_LINEAR_FP8) || a->M < 2 || a->M > 16 || a->K % db::CH != 0 || a->K / db::CH < db::NW / 2) return false;
     if (a->K >= 1 << 26 || a->M * a->ldx >= 1 << 30 || a->M * a->ldy >= 1 << 29) return false;   // 32-bit offsets
     if (a->norm_w && (a->M > db::NW || ((uintptr_t)a->norm_w) % 16 != 0)) return false;
+    if (db_skinny_ahead(a)) return false;
     if (a->K <= 5120) {
         // chunks that a wave of the busiest block streams: a slot beyond them is issued for nothing
         const int64_t cus = device_cu_count(), tiles = a->epilogue == QIE_EPI_SWIGLU ? (a->N + 7) / 8 : (a->N + 15) / 16 + 2;

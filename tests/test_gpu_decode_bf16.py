@@ -110,3 +110,13 @@ def test_fused_norm_is_the_separate_one(qlib, K, num):
             a.y, a.ldy, a.epilogue, a.numerics, a.norm_w, a.norm_eps = G.p(y), N, _lib.QIE_EPI_F32, num, G.p(dn), eps
             G.check(qlib.qie_linear(C.byref(a), None), "qie_linear")
             assert np.array_equal(y.numpy(), want[:M]), M
+
+
+# the sizes where plain rows go back to the skinny kernel, either side of each line
+@pytest.mark.parametrize("M,K,N", [(7, 512, 8192), (7, 512, 8193), (8, 512, 130), (2, 640, 130), (3, 1024, 8191), (3, 1024, 8192), (8, 2048, 8192), (5, 2048, 8193)])
+def test_lines_to_the_skinny_kernel(qlib, M, K, N):
+    x, w = bf16((M, K), 1.0, 31), bf16((N, K), K ** -0.5, 32)
+    y = G.zeros_bf16(M, N)
+    linear(G.dev(x), [G.dev(w)], [], M, K, N, y, _lib.QIE_EPI_STORE)
+    want, scale = products(x, w)
+    assert (np.abs(G.bf(G.host_bf16(y)) - want) <= 2.0 ** -8 * np.abs(want) + 1e-5 * scale).all()   # half an ulp of bf16, two orders of one fp32 sum
