@@ -1052,7 +1052,7 @@ static int g8_splitk(int64_t tiles, int64_t cus, int nk) {
     int best = 1;
     double best_t = 1e30;
     // k-tiles per part at least QIE_GEMM8_SK_MINK (dev A/B; default 64: K >= 4,096 per part).
-    // Round 5: split-K 2 for the O projection at P = 2,048 (112 tiles -> 224, K = 3,584) ran
+    // Split-K 2 for the O projection at P = 2,048 (112 tiles -> 224, K = 3,584) ran
     // 94-98 vs 84 µs for the 256x128 kernel; QKV at 3 parts 114 vs 89 — the slab round trip
     // costs more than the idle CUs at this K
     const int mink = std::max(4, dev_env("QIE_GEMM8_SK_MINK", 64));
@@ -1542,12 +1542,15 @@ int gemm(const qie_linear_args* a, hipStream_t st) {
     const unsigned gm = (unsigned)cdiv(a->M, BM);
     QIE_REQUIRE(a->K % 8 == 0, "qie_linear: GEMM needs K %% 8 == 0");
     if (!(a->flags & QIE_LINEAR_FP8) && a->K % big::BK == 0 && a->ldx % 8 == 0) {
-        // LDS-DMA kernel: 256x256 tiles when they fill the chip at least once (config 4's
-        // O / down at 8,192 rows: 448 tiles; the generic 128x128 kernel took them before), else
-        // 256x128 when those fill >= 3/4 of it in one round (Qwen2-7B O and down projections
-        // at 2,048 rows: 112 vs 224 tiles on 256 CUs), else 256x256 in one round (below).
-        // args.flags QIE_LINEAR_TILE256 / TILE128 force a tile (tests; dev builds also
-        // QIE_GEMM_BIG = 1 / 2, 0 disables the kernel for A/B timing).
+        // In this order:
+        //   1. K a multiple of 64: k_gemm_mid.hip, unless the next is expected to be faster (g8_us);
+        //   2. K a multiple of 64 from 256 on, 256 rows: the phase-interleaved 256x256 kernel, whole where its tiles fill the chip,
+        //      or half of it when K is too short to split; split over K otherwise;
+        //   3. K an odd multiple of 32, or a split that gets no memory for its slabs, 256 rows: the LDS-DMA kernel, with 256x256 tiles
+        //      when they fill the chip at least once, 256x128 when those fill >= 3/4 of it in one round, 256x256 in one round;
+        //   4. fewer rows at such K: the register-staged kernel.
+        // args.flags QIE_LINEAR_TILE256 / TILE128 / STREAMK force a kernel (tests; dev builds also
+        // QIE_GEMM_BIG = 1 / 2, 0 disables 3 for A/B timing).
         const int64_t cols = a->epilogue == QIE_EPI_SWIGLU ? 2 * a->N : a->N;
         const int64_t n_mt = cdiv(a->M, big::BM);
         const int64_t t256 = n_mt * cdiv(cols, 256), t128 = n_mt * cdiv(cols, 128);
@@ -1557,8 +1560,7 @@ int gemm(const qie_linear_args* a, hipStream_t st) {
         // phase-interleaved 256x256 kernel (K a multiple of 64, >= 4 k-tiles): Qwen2-7B gate/up at 2,048
         // rows 612 -> 488 us, bit-identical to gemm_big; down split-K 2: 309 -> 247 us
         const bool g8ok = a->K % g8::BK == 0 && a->K >= 4 * g8::BK;
-        // rows that do not fill the 256x256 tiles: k_gemm_mid.hip, unless the phase-interleaved kernel below is expected
-        // to be faster (Qwen2-7B gate/up: 301 rows 161 -> 119 us, 700 rows 183 against 229)
+        // (Qwen2-7B gate/up, us: 301 rows 161 with the 256x256 kernel, 119 with k_gemm_mid.hip; 700 rows 183 against 229)
         if (dev_env("QIE_MID", 1) && force < 0 && !(a->flags & QIE_LINEAR_STREAMK)) {
             bool launched = false;
             const int rc = gemm_mid(a, p, g8ok && a->M >= big::BM ? g8_us(t256, cus, (int)(a->K / g8::BK)) : 1e30f, st, &launched);
@@ -1587,8 +1589,8 @@ int gemm(const qie_linear_args* a, hipStream_t st) {
             return launch_gemm_big<256>(a->epilogue, p, (int)n_mt, (int)t256, st);
         if (force == 2 || (force < 0 && a->M >= big::BM && t128 >= (3 * cus) / 4 && t128 <= cus))
             return launch_gemm_big<128>(a->epilogue, p, (int)n_mt, (int)t128, st);
-        // 256-column tiles in ONE round when 128-column ones would take two (Qwen2-7B QKV at
-        // 2,048 rows: 144 vs 288 tiles on 256 CUs): 124 -> 99 us against the generic kernel
+        // 256-column tiles in ONE round when 128-column ones would take two (4,608 columns at 2,048 rows:
+        // 144 vs 288 tiles on 256 CUs): 124 -> 99 us against the generic kernel at K = 3,584
         if (force < 0 && a->M >= big::BM && t256 >= cus / 2 && t256 <= cus && t128 > cus)
             return launch_gemm_big<256>(a->epilogue, p, (int)n_mt, (int)t256, st);
     }
