@@ -46,4 +46,67 @@ inline Plan plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool grouped, i
 }
 }  // namespace lf
 
+// ---------------------------------------------------------------- k_gemm_mid.hip
+namespace mid {
+constexpr int BK = 64;
+
+// Times of a tile, us, fitted to the Qwen2-0.5B / 7B and Qwen3-14B projections at 20 to 2,048 rows (168 shapes; what the
+// rule below picks is 1 % over the best of all tiles, splits and the 256x256 kernel on the average, 17 % at most):
+// up to one workgroup a CU a1 + s1 per k-tile, more a2 + (rounds of the chip) * (f2 + s2 per k-tile).  A k-tile costs what its
+// lines take through one CU (about 50 GB/s where they come from HBM or another die, 120 GB/s from L2), not its matrix work,
+// which is why the tall tiles win as soon as the rows fill them.  The constants are an MI355X's, whole (256 CUs): `cus` moves
+// the rounds, but the slopes hold the bandwidth that 256 CUs share, so a part with fewer would still get a correct plan, not
+// the fastest one.
+struct Tile {
+    int bm, bn, slots, per_cu;   // per_cu: workgroups that fit a CU's LDS
+    float a1, s1, a2, f2, s2;
+};
+constexpr Tile TILES[] = {
+    {64, 64, 5, 2, 3.2f, .285f, 5.f, .7f, .487f},   {64, 128, 3, 2, 2.6f, .475f, 5.4f, 1.1f, .74f},
+    {128, 64, 3, 2, 3.3f, .43f, 4.7f, 1.8f, .70f},  {128, 128, 4, 1, 5.9f, .54f, 7.5f, 3.9f, .575f},
+    {192, 128, 4, 1, 8.f, .65f, 5.f, 6.f, .72f},    {256, 128, 3, 1, 9.9f, .90f, 12.f, 2.5f, 1.037f},
+    {320, 64, 3, 1, 6.9f, .70f, 6.5f, 3.f, .787f},  {320, 128, 2, 1, 9.4f, 1.11f, 14.f, 2.f, 1.2f},
+};
+constexpr int N_TILES = sizeof(TILES) / sizeof(TILES[0]);
+struct Plan {
+    int tile, whole, splitk, n_mt, n_nt;
+    float us;
+};
+
+// the last round of a launch costs nearly a whole one
+inline float rounds(float x) {
+    const float f = (float)(int)x;
+    return f + (x > f ? std::max(.8f, x - f + .3f) : 0.f);
+}
+
+// Tile and split: the tiles run whole round by round of the chip; the last, partial round's tiles may be cut into `splitk`
+// K ranges (3 us a part for 128x128 outputs: slab out, slab in).
+inline Plan plan(int64_t M, int64_t cols, int64_t K, int64_t cus) {
+    Plan best{-1, 0, 1, 0, 0, 1e30f};
+    const int nk = (int)(K / BK);
+    const float floor_us = (float)cols * K * 2 / 5.3e6f + 4.f;   // the weights at the rate they stream here
+    for (int c = 0; c < N_TILES; c++) {
+        const Tile& t = TILES[c];
+        const int64_t n_mt = (M + t.bm - 1) / t.bm, n_nt = (cols + t.bn - 1) / t.bn, tiles = n_mt * n_nt;
+        if (tiles > (1 << 22)) continue;   // (of 32-bit workgroup counts)
+        const float room = (float)(cus * t.per_cu);
+        for (int s = 1; s <= 12 && s <= nk; s++) {
+            const int64_t whole = s == 1 ? tiles : tiles / (cus * t.per_cu) * (cus * t.per_cu), cut = (tiles - whole) * s;
+            float us;
+            if (s == 1) {
+                us = tiles <= cus ? t.a1 + nk * t.s1 : t.a2 + rounds(tiles / room) * (t.f2 + nk * t.s2);
+            } else {
+                if (cut == 0) break;
+                const float len = (float)((nk + s - 1) / s);
+                us = whole / room * (t.f2 + nk * t.s2) + 3.f * s * (t.bm * t.bn) / 16384.f + 1.f;
+                us += cut <= cus ? t.a1 + len * t.s1 : t.a2 + rounds(cut / room) * (t.f2 + len * t.s2);
+            }
+            us = std::max(us, floor_us);
+            if (us < best.us) best = {c, (int)whole, s, (int)n_mt, (int)n_nt, us};
+        }
+    }
+    return best;
+}
+}  // namespace mid
+
 }  // namespace qie

@@ -15,14 +15,11 @@
 //   * workgroups that share a weight tile are neighbours in one XCD, parts are the slowest index: an XCD's L2 holds one K
 //     range of A.
 #include "gemm_impl.hpp"
+#include "gemm_plan.hpp"
 
 #include <algorithm>
 
 namespace qie {
-
-namespace mid {
-constexpr int BK = 64;
-}
 
 // weight row of tile column c of column tile nt; SwiGLU tiles hold, per wave slice of BN / 2 columns, a half of gate rows
 // and the same outputs' up rows
@@ -291,64 +288,8 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
 
 // ---------------------------------------------------------------- the plan
 namespace {
-// Times of a tile, us, fitted to the Qwen2-0.5B / 7B and Qwen3-14B projections at 20 to 2,048 rows (168 shapes; what the
-// rule below picks is 1 % over the best of all tiles, splits and the 256x256 kernel on the average, 17 % at most):
-// up to one workgroup a CU a1 + s1 per k-tile, more a2 + (rounds of the chip) * (f2 + s2 per k-tile).  A k-tile costs what its
-// lines take through one CU (about 50 GB/s where they come from HBM or another die, 120 GB/s from L2), not its matrix work,
-// which is why the tall tiles win as soon as the rows fill them.
-struct MidTile {
-    int bm, bn, slots, per_cu;   // per_cu: workgroups that fit a CU's LDS
-    float a1, s1, a2, f2, s2;
-};
-constexpr MidTile MID_TILES[] = {
-    {64, 64, 5, 2, 3.2f, .285f, 5.f, .7f, .487f},   {64, 128, 3, 2, 2.6f, .475f, 5.4f, 1.1f, .74f},
-    {128, 64, 3, 2, 3.3f, .43f, 4.7f, 1.8f, .70f},  {128, 128, 4, 1, 5.9f, .54f, 7.5f, 3.9f, .575f},
-    {192, 128, 4, 1, 8.f, .65f, 5.f, 6.f, .72f},    {256, 128, 3, 1, 9.9f, .90f, 12.f, 2.5f, 1.037f},
-    {320, 64, 3, 1, 6.9f, .70f, 6.5f, 3.f, .787f},  {320, 128, 2, 1, 9.4f, 1.11f, 14.f, 2.f, 1.2f},
-};
-constexpr int MID_N = sizeof(MID_TILES) / sizeof(MID_TILES[0]);
-struct MidPlan {
-    int tile, whole, splitk, n_mt, n_nt;
-    float us;
-};
-
-// the last round of a launch costs nearly a whole one
-float mid_rounds(float x) {
-    const float f = (float)(int)x;
-    return f + (x > f ? std::max(.8f, x - f + .3f) : 0.f);
-}
-
-// Tile and split: the tiles run whole round by round of the chip; the last, partial round's tiles may be cut into `splitk`
-// K ranges (3 us a part for 128x128 outputs: slab out, slab in).
-MidPlan mid_plan(int64_t M, int64_t cols, int64_t K, int64_t cus) {
-    MidPlan best{-1, 0, 1, 0, 0, 1e30f};
-    const int nk = (int)(K / mid::BK);
-    const float floor_us = (float)cols * K * 2 / 5.3e6f + 4.f;   // the weights at the rate they stream here
-    for (int c = 0; c < MID_N; c++) {
-        const MidTile& t = MID_TILES[c];
-        const int64_t n_mt = cdiv(M, t.bm), n_nt = cdiv(cols, t.bn), tiles = n_mt * n_nt;
-        if (tiles > (1 << 22)) continue;   // (of 32-bit workgroup counts)
-        const float room = (float)(cus * t.per_cu);
-        for (int s = 1; s <= 12 && s <= nk; s++) {
-            const int64_t whole = s == 1 ? tiles : tiles / (cus * t.per_cu) * (cus * t.per_cu), cut = (tiles - whole) * s;
-            float us;
-            if (s == 1) {
-                us = tiles <= cus ? t.a1 + nk * t.s1 : t.a2 + mid_rounds(tiles / room) * (t.f2 + nk * t.s2);
-            } else {
-                if (cut == 0) break;
-                const float len = (float)((nk + s - 1) / s);
-                us = whole / room * (t.f2 + nk * t.s2) + 3.f * s * (t.bm * t.bn) / 16384.f + 1.f;
-                us += cut <= cus ? t.a1 + len * t.s1 : t.a2 + mid_rounds(cut / room) * (t.f2 + len * t.s2);
-            }
-            us = std::max(us, floor_us);
-            if (us < best.us) best = {c, (int)whole, s, (int)n_mt, (int)n_nt, us};
-        }
-    }
-    return best;
-}
-
 template <int EPI, int BM, int BN, int SLOTS>
-int launch_mid_t(const GemmParams& p, const MidPlan& pl, const G8Split& sk, hipStream_t st) {
+int launch_mid_t(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, hipStream_t st) {
     const void* fn = (const void*)gemm_mid_kernel<EPI, BM, BN, SLOTS>;
     constexpr size_t shm = (size_t)SLOTS * (BM + BN) * 128;
     static bool raised = false;
@@ -364,7 +305,7 @@ int launch_mid_t(const GemmParams& p, const MidPlan& pl, const G8Split& sk, hipS
 }
 
 template <int EPI>
-int launch_mid(const GemmParams& p, const MidPlan& pl, const G8Split& sk, hipStream_t st) {
+int launch_mid(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, hipStream_t st) {
     switch (pl.tile) {
         case 0: return launch_mid_t<EPI, 64, 64, 5>(p, pl, sk, st);
         case 1: return launch_mid_t<EPI, 64, 128, 3>(p, pl, sk, st);
@@ -385,12 +326,12 @@ int gemm_mid(const qie_linear_args* a, const GemmParams& q, float other_us, hipS
     p.vec = a->ldy % 4 == 0 && ((uintptr_t)a->y) % (a->epilogue == QIE_EPI_F32 ? 16 : 8) == 0;
     if (a->K % mid::BK != 0) return 0;   // (rows of x and weights are on the 16-byte grid of LDS-DMA: qie_linear)
     const int64_t cols = a->epilogue == QIE_EPI_SWIGLU ? 2 * a->N : a->N;
-    const MidPlan pl = mid_plan(a->M, cols, a->K, device_cu_count());
+    const mid::Plan pl = mid::plan(a->M, cols, a->K, device_cu_count());
     if (pl.tile < 0 || pl.us >= 0.88f * other_us) return 0;   // 12 %: what the two fits are off by on long prompts
     G8Split sk{1, nullptr, nullptr};
     const int64_t cut = (int64_t)pl.n_mt * pl.n_nt - pl.whole;
     if (pl.splitk > 1 && cut > 0) {
-        const int64_t floats = cut * pl.splitk * MID_TILES[pl.tile].bm * MID_TILES[pl.tile].bn;
+        const int64_t floats = cut * pl.splitk * mid::TILES[pl.tile].bm * mid::TILES[pl.tile].bn;
         if (g8_workspace(st, (int)cdiv(floats, 65536), (int)cut, &sk) == 0) sk.splitk = pl.splitk;
     }
     *launched = true;

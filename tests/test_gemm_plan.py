@@ -5,18 +5,24 @@ import subprocess
 
 import pytest
 
+from test_gpu_gemm_mid import PLANS
+
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "qwen_inference_engine_amd", "csrc")
 
 DRIVER = r"""
 #include "gemm_plan.hpp"
 #include <cstdio>
 #include <vector>
-// "f M N K batch grouped cus": plan of k_linear_f32.hip; "t M N K groups off[0] .. off[groups]": its row tiles' indices
+// "m M columns K cus": plan of k_gemm_mid.hip; "f M N K batch grouped cus": k_linear_f32.hip; "t M N K groups off[0] .. off[groups]": its row tiles' indices
 int main() {
     char op;
     while (std::scanf(" %c", &op) == 1) {
         long M, N, K, batch, x, cus;
-        if (op == 'f') {
+        if (op == 'm') {
+            if (std::scanf("%ld %ld %ld %ld", &M, &N, &K, &cus) != 4) return 2;
+            const qie::mid::Plan p = qie::mid::plan(M, N, K, cus);
+            std::printf("%d %d %d %d\n", p.tile, p.whole, p.splitk, p.n_mt * p.n_nt);
+        } else if (op == 'f') {
             if (std::scanf("%ld %ld %ld %ld %ld %ld", &M, &N, &K, &batch, &x, &cus) != 6) return 2;
             const qie::lf::Plan p = qie::lf::plan(M, N, K, batch, x != 0, cus);
             std::printf("%d %d %d %d %ld\n", p.n_nt, p.n_mt, p.log_segs, p.log_parts, (long)p.row_tiles);
@@ -48,6 +54,22 @@ def plan(tmp_path_factory):
         out = subprocess.run([str(d / "drive")], input="\n".join(lines), text=True, capture_output=True, check=True).stdout
         return [[int(v) for v in line.split()] for line in out.splitlines()]
     return run
+
+
+def test_gemm_mid_shapes_take_every_tile(plan):
+    """The shapes that the GPU test multiplies have the plans it says, every tile among them whole, split and both."""
+    got = [(p[0], "whole" if p[2] == 1 else "split" if p[1] == 0 else "mixed") for p in plan([f"m {M} {N} {K} 256" for M, N, K, _, _ in PLANS])]
+    assert got == [(t, kind) for _, _, _, t, kind in PLANS]
+    assert set(got) == {(t, kind) for t in range(8) for kind in ("whole", "split", "mixed")}
+
+
+def test_gemm_mid_plans_are_sound(plan):
+    """Whole tiles are whole rounds of the chip or all of them, and a split leaves every part a k-tile."""
+    r = random.Random(3)
+    cases = [(int(2 ** r.uniform(4.1, 13)), int(2 ** r.uniform(3, 18)), 64 * int(2 ** r.uniform(0, 9)), r.choice([256, 256, 304, 64])) for _ in range(3000)]
+    for (M, N, K, cus), (tile, whole, splitk, tiles) in zip(cases, plan(["m %d %d %d %d" % c for c in cases])):
+        assert tile in range(8) and 1 <= splitk <= min(12, K // 64) and 0 <= whole <= tiles
+        assert whole == tiles if splitk == 1 else whole < tiles and whole % cus == 0
 
 
 @pytest.mark.parametrize("seed", range(6))

@@ -38,11 +38,17 @@ def linear(x, ws, biases, M, K, N, y, epi, ldx=None, ldy=None):
     G.check(_lib.load().qie_linear(C.byref(a), None), "qie_linear")
 
 
-# rows, columns, K and the tile that the plan gives on 256 CUs (w whole tiles, s all split, m whole rounds and split rest)
-SHAPES = [(17, 72, 64), (33, 72, 2048), (17, 40000, 128), (17, 16500, 64), (64, 8200, 4096), (65, 40000, 128), (65, 8200, 1024),
-          (129, 4000, 4096), (65, 33000, 2048), (127, 16500, 64), (128, 8200, 4096), (193, 40000, 2048), (500, 8200, 128),
-          (129, 33000, 1024), (640, 8200, 448), (193, 70000, 512), (640, 4000, 4096), (257, 40000, 1024), (257, 16500, 1024),
-          (320, 33000, 2048), (321, 130, 192)]
+# rows, columns, K; the tile that the plan gives them on 256 CUs, and whether tiles run whole, are all split over K, or both
+# (tests/test_gemm_plan.py holds the plan to this, and every tile to all three)
+PLANS = [(17, 72, 64, 0, "whole"), (33, 72, 2048, 0, "split"), (17, 40000, 128, 0, "mixed"), (17, 16500, 64, 1, "whole"),
+         (64, 8200, 4096, 1, "split"), (65, 40000, 128, 1, "mixed"), (65, 8200, 1024, 2, "whole"), (129, 4000, 4096, 2, "split"),
+         (65, 33000, 2048, 2, "mixed"), (127, 16500, 64, 3, "whole"), (128, 8200, 4096, 3, "split"), (193, 40000, 2048, 3, "mixed"),
+         (500, 8200, 128, 4, "whole"), (129, 33000, 1024, 1, "whole"), (640, 8200, 448, 5, "whole"), (193, 70000, 512, 1, "whole"),
+         (640, 4000, 4096, 6, "split"), (257, 40000, 1024, 1, "mixed"), (257, 16500, 1024, 7, "whole"), (320, 33000, 2048, 1, "whole"),
+         (321, 130, 192, 1, "whole"), (140, 38660, 2624, 4, "mixed"), (131, 11014, 3712, 4, "split"), (200, 45648, 1792, 5, "mixed"),
+         (210, 9278, 6464, 5, "split"), (273, 38147, 1792, 6, "mixed"), (259, 12692, 64, 6, "whole"), (1064, 11882, 1728, 7, "mixed"),
+         (257, 8338, 11264, 7, "split")]
+SHAPES = [p[:3] for p in PLANS]
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES)

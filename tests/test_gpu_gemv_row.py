@@ -1,4 +1,4 @@
-"""One-row projections with a whole weight row in a wave's registers (k_gemv_row.hip) through qie_linear, against fp64 products:
+"""One-row projections with a whole weight row in a wave's registers (k_gemv_row.hip) through qie_linear, against fp32 products:
 K at the edges of the register forms, rows from one to 32 a CU, segments, every epilogue it takes, the fused norm in both numerics."""
 import ctypes as C
 
