@@ -295,7 +295,8 @@ int qie_sample(const void* logits, int64_t M, int64_t V, int64_t ld, const qie_s
                        (const uint16_t*)logits, V, ld, k, cand);
     QIE_LAUNCH_CHECK();
     const int total = nb * k;
-    QIE_REQUIRE(pow2_at_least(total) <= 64 * 256, "qie_sample: top-k merge exceeds LDS (V=%lld k=%d)", (long long)V, k);
+    // a thread of the merge holds up to 64 candidates in registers
+    QIE_REQUIRE(total <= 64 * 256, "qie_sample: top-k of %d over %lld logits leaves %d candidates, more than %d", k, (long long)V, total, 64 * 256);
     const auto fn = total <= 8 * 256 ? topk_merge_sample_kernel<8> : total <= 40 * 256 ? topk_merge_sample_kernel<40>
                                                                                        : topk_merge_sample_kernel<64>;
     hipLaunchKernelGGL(fn, dim3((unsigned)M), dim3(256), 0, st, cand, nb, k, std::max(2, pow2_at_least(k)),
