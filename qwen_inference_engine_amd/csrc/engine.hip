@@ -29,6 +29,7 @@ int gemm(const qie_linear_args* a, hipStream_t st);
 bool dec8_applies(const qie_linear_args* a);
 bool dec_bf16_applies(const qie_linear_args* a);
 int dec8_reserve(hipStream_t st);
+void g8_reserve(hipStream_t st);
 void g8_release(hipStream_t st);
 bool persist_supported(const qie_model_spec& s, int B, int tp, bool fp8, bool paged, int ncu, const char** why);
 size_t persist_attn_table_bytes(int n_layers);
@@ -766,6 +767,7 @@ int qie_engine_create(const qie_model_spec* spec, const qie_engine_opts* opts, q
         delete e;
         return fail((int)he, "hipStreamCreate: %s", hipGetErrorString(he));
     }
+    g8_reserve(e->stream);
     int rc = build_rope(e);
     if (rc) {
         qie_engine_destroy(e);

@@ -24,7 +24,8 @@
 #include <string>
 
 namespace qie {
-void g8_release(hipStream_t st);   // k_gemm.hip
+void g8_reserve(hipStream_t st);   // k_gemm.hip
+void g8_release(hipStream_t st);
 
 struct HostTensor {
     int dtype = 0;   // 0 bf16 words, 1 int32, 2 fp32
@@ -2528,6 +2529,7 @@ int layered_batch_create(qie_engine* e, int32_t batch, int32_t max_ctx, int32_t 
         hipError_t he = hipEventCreateWithFlags(&s->ev_fork, hipEventDisableTiming);
         for (int i = 0; i < LayeredBatch::kSide && he == hipSuccess; i++) {
             he = hipStreamCreateWithFlags(&s->side[i], hipStreamNonBlocking);
+            if (he == hipSuccess) g8_reserve(s->side[i]);
             if (he == hipSuccess) he = hipEventCreateWithFlags(&s->ev_join[i], hipEventDisableTiming);
         }
         for (int i = 0; i < 2 && he == hipSuccess; i++) {
@@ -2776,6 +2778,7 @@ int qie_engine_create_layered(const qie_arch_desc* arch, const qie_engine_opts* 
         qie_engine_destroy(e);
         return fail((int)he, "qie_engine_create_layered: %s", hipGetErrorString(he));
     }
+    g8_reserve(e->stream);
     *out = e;
     return 0;
 }

@@ -47,6 +47,8 @@ struct G8Split {
 // Slabs of 65,536 floats and zeroed tickets of stream `st`, grown on demand; non-zero: they would have to grow during a
 // graph capture, or there is no memory (the caller runs unsplit).  What a capture was given stays valid until g8_release.
 int g8_workspace(hipStream_t st, int slabs, int tiles, G8Split* out);
+// Makes room ahead of the first launch, where a stream is made that will run them.
+void g8_reserve(hipStream_t st);
 // Gives a stream's split-K memory back: before the engine that owns the stream destroys it, its batches' graphs gone.
 void g8_release(hipStream_t st);
 

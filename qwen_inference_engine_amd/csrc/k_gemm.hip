@@ -998,6 +998,13 @@ int g8_workspace(hipStream_t st, int slabs, int tiles, G8Split* out) {
     return 0;
 }
 
+// One 256x256 partial tile a CU: what nearly every split launch needs at most, so that a first pass does not stop to allocate
+// (64 MB; growing step by step inside it took 0.3 to 1.1 ms).
+void g8_reserve(hipStream_t st) {
+    G8Split ws;
+    (void)g8_workspace(st, device_cu_count(), 4096, &ws);   // no memory: a later launch asks again, or runs unsplit
+}
+
 void g8_release(hipStream_t st) {
     std::lock_guard<std::mutex> lk(g8_mu);
     const auto it = g8_pools.find(st);
