@@ -122,6 +122,12 @@ __global__ __launch_bounds__(512) void linear_f32_kernel(LinF32P p) {
             const int row = wm * 32 + i * 16 + fr;
             fa[i] = *reinterpret_cast<const f32x4*>(buf + row * 128 + (((4 * wk + g) ^ g8_swz(row)) * 16));
         }
+        if (t == seg_end) {   // uniform; a segment is summed: here, while the fragments are on their way
+            lf_meet(acc, lvl, seg, log_own);
+            clear();
+            seg++;
+            seg_end = seg_at(seg0 + seg + 1) - kb;
+        }
 #pragma unroll
         for (int e = 0; e < 4; e++)
 #pragma unroll
@@ -133,12 +139,8 @@ __global__ __launch_bounds__(512) void linear_f32_kernel(LinF32P p) {
         __builtin_amdgcn_sched_barrier(0);
         slot = slot + 1 == SLOTS ? 0 : slot + 1;
         fill = fill + 1 == SLOTS ? 0 : fill + 1;
-        if (t + 1 == seg_end) {   // uniform
-            if (!lf_meet(acc, lvl, seg, log_own)) clear();   // (the last segment's: acc is this workgroup's node)
-            seg++;
-            seg_end = seg_at(seg0 + seg + 1) - kb;
-        }
     }
+    lf_meet(acc, lvl, seg, log_own);   // the last segment: acc is this workgroup's node
     if (parts > 1) {
         const int64_t tile = row_tile(p.q.grp_off != nullptr, m0, z, mt, p.pl.n_mt) * p.pl.n_nt + nt;
         const auto rs = __builtin_amdgcn_make_buffer_rsrc(p.slab + ((tile << p.pl.log_parts) + part) * SLAB, (short)0, SLAB * 4, 0x00020000);

@@ -92,7 +92,7 @@ def test_slabs_are_bounded(plan):
     cases += [(2048, 256, 1024, 8, 1), (240, 1408, 1024, 8, 1), (240, 1024, 704, 8, 1)]
     for c, (n_nt, n_mt, segs, parts, row_tiles) in zip(cases, plan([f"f {' '.join(map(str, c))} 256" for c in cases])):
         assert 0 <= parts <= segs <= 4
-        assert segs == 0 or c[2] // 32 >> segs >= 4      # a segment keeps four k-tiles
+        assert segs == 0 or c[2] // 32 >> segs >= 8      # a segment keeps eight k-tiles
         if parts:
             assert (row_tiles * n_nt << parts) * 8192 * 4 <= 32 << 20
 
