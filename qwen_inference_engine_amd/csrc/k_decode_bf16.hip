@@ -227,11 +227,25 @@ __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
                         ss[v % S] += a * a + b * b;
                     }
                 }
+                // wave_sum of all of them at once: a lane exchange takes two values, and row r of 16 lanes ends with sum r
 #pragma unroll
-                for (int j = 0; j < S; j++) {
-                    const float t = wave_sum(ss[j]);
-                    if (lane == 0) ssq[m * 4 + j * PP + sub] = t;
+                for (int j = 0; j < S; j++) ss[j] = group_sum<16>(ss[j]);
+                float t;
+                if constexpr (S == 1) {
+                    t = xor32_sum(xor16_sum(ss[0]));
+                } else {
+                    lane_swap<16>(ss[0], ss[1]);
+                    t = ss[0] + ss[1];
+                    if constexpr (S == 4) {
+                        lane_swap<16>(ss[2], ss[3]);
+                        float u = ss[2] + ss[3];
+                        lane_swap<32>(t, u);
+                        t = t + u;
+                    } else {
+                        t = xor32_sum(t);
+                    }
                 }
+                if ((lane & 15) == 0 && lane < 16 * S) ssq[m * 4 + (lane >> 4) * PP + sub] = t;
             };
             if (P == 1) squares(std::integral_constant<int, 1>{});
             else if (P == 2) squares(std::integral_constant<int, 2>{});
