@@ -352,7 +352,7 @@ __device__ __forceinline__ bool attn_decode_mfma2_body(const DecodeAttnParams& a
     // Without the pre-rotation the same holds when the engine keeps the current position's
     // RoPE row (a.rc, tagged with the position): the prologue's loads then need no position
     // either, and a stale tag (a position set some other way) reloads the table row.
-    // (Paged, measured in round 5: the step's page from the block-table entry of (row,
+    // (Paged, measured: the step's page from the block-table entry of (row,
     // 128 s) needs no position either, but the speculative form ran config 4 at 3,563 vs
     // 3,624 tok/s for the plain one — the table round trip still precedes the K / V loads.)
     constexpr bool SPEC = !PG;
@@ -612,8 +612,8 @@ __device__ __forceinline__ bool attn_decode_mfma2_body(const DecodeAttnParams& a
     }
     __syncthreads();
     if (!last_flag || QIE_DBG(a.dbg & 128)) return false;   // (dev timing exit 128: ticket taken, no combine)
-    // Default: 16-B sc1 buffer loads on a uniform (SGPR) resource instead of the acquire
-    // (MI355X_MICROARCH.md hand-off row 1): 9.79 -> 9.56 us per launch.  (Round 2 measured
+    // Default: 16-B sc1 buffer loads on a uniform (SGPR) resource instead of the acquire:
+    // 9.79 -> 9.56 us per launch.  (Measured as well:
     // 8-B agent-scope atomic loads at 11.4 vs 10.7 us, and 16-B sc1 loads at 73 us — that
     // form put the resource in VGPRs, a waterfall loop per load.)
     if (!a.sc1) {

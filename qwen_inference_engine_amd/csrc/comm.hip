@@ -315,7 +315,7 @@ __global__ __launch_bounds__(256) void peer_kernel(PeerArgs A, const void* src, 
 // handed to the next communicator instead of back to the allocator: physical pages that were
 // mapped uncached are never recycled into ordinary (cached) allocations of the process — a
 // weight arena placed on them after the peer tests read back 40 whole 128-B lines of a
-// freshly written tensor as stale zeros (test_tp_weights_bin_equals_synthetic, r06).
+// freshly written tensor as stale zeros (test_tp_weights_bin_equals_synthetic).
 static std::mutex g_peer_pool_mu;
 static std::vector<char*> g_peer_pool;
 static char* peer_pool_get() {

@@ -677,8 +677,8 @@ static int ensure_prefill_scratch(qie_batch* b, int64_t n) {
 }
 
 // The ids and (tensor parallel, peer backend) the exchange error word come back in ONE
-// stream-ordered batch with one synchronisation — not a second blocking round trip per token
-// (ADVICE r05); a backend without the word keeps comm_check's own read.
+// stream-ordered batch with one synchronisation — not a second blocking round trip per token;
+// a backend without the word keeps comm_check's own read.
 // The persistent step's error word (a bounded hand-off wait that gave up): the step's outputs
 // are garbage and the call fails loudly (never a hang; k_persist.hip)
 static int pk_fail(unsigned w) {
@@ -733,7 +733,7 @@ int qie_engine_create(const qie_model_spec* spec, const qie_engine_opts* opts, q
                 "(use replicas for this model at this size)", tp);
     // prefill_fp8 is a numerics choice (every projection input quantised to e4m3): refuse it
     // where the engine could not honour it, instead of silently running bf16 activations
-    // against a caller (and an oracle) that expects the fp8-activation model (ADVICE r05)
+    // against a caller (and an oracle) that expects the fp8-activation model
     if (opts && opts->prefill_fp8) {
         const int64_t qd = (int64_t)probe.nq * s.head_dim, ffl = s.ffn / tp;
         QIE_REQUIRE(opts->weight_fp8, "qie_engine_create: prefill_fp8 needs weight_fp8 (fp8 weights are the "

@@ -296,7 +296,7 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_prefill_mfma2_kernel(Pre
     // 128); rows past kmax re-read row kmax (same page) and are masked by position.
     constexpr int RPI = 512 / HD;                 // key rows per 1 KiB wave-instruction
     constexpr int IPW = KT / RPI / NW;            // wave-instructions per wave per operand
-    // Buffer loads to LDS on a per-tile resource (round 5): the lane byte offsets inside a
+    // Buffer loads to LDS on a per-tile resource: the lane byte offsets inside a
     // tile are constants of the launch and the tile base is scalar, so a tile's DMAs cost no
     // VALU (the flat form recomputed 64-bit addresses and the row clamp per tile: ~40 VALU).
     // The resource covers the tile's rows up to kmax only: rows past it read as zeros (their

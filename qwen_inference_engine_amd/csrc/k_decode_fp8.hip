@@ -102,7 +102,7 @@ __global__ __launch_bounds__(KS * 64, SPL ? 4 : 1) void dec8_kernel(Dec8Params p
     // the buffer range (0) — wave-uniform, and no load sits under a branch
     const int kval = SPL ? (K - kw) / 64 : KU;   // valid units (may be <= 0 or > KU)
 
-    // LDS form of the fused RMSNorm (round 5; M <= 8, one block of KS waves holding whole
+    // LDS form of the fused RMSNorm (M <= 8, one block of KS waves holding whole
     // rows: K = KS x 512): thread t loads chunk t (8 values) of every REAL row once, the
     // rows' sums of squares meet by a transposed butterfly + one LDS exchange, each thread
     // normalises its chunks into an LDS image of the M rows (aliasing the partial-tile area,
@@ -543,7 +543,7 @@ __global__ __launch_bounds__(KS * 64, SPL ? 4 : 1) void dec8_kernel(Dec8Params p
 }
 
 // ---------------------------------------------------------------------------
-// dec8r (round 4): dec8 with the A fragments in LDS and a 4-deep register ring of weight
+// dec8r: dec8 with the A fragments in LDS and a 4-deep register ring of weight
 // steps.  In dec8 the A fragments (16 rows x the wave's K slice, rows >= M padding) held 64
 // VGPRs per wave for the whole launch, leaving room for only two half-tile steps in flight
 // (~112 KB per CU at config 4's gate/up, 4.0 TB/s, where the bf16 GEMV keeps ~200 KB in
@@ -916,7 +916,7 @@ static int dec8_epi(const Dec8Params& p, int epi, hipStream_t st) {
 // Long K without such a shape (the down projection's 18,944 = 296 units): split-K over
 // parts of 8 waves x 4 units (10 parts at 18,944, the last one ragged; 128 VGPRs, two blocks
 // per CU), single-segment epilogues without a fused norm only (a norm needs the whole row in
-// one block).  Config 4 (fp8, B = 8), same box: the general skinny kernel 2,895 tok/s (down
+// one block).  Qwen2-7B, fp8, B = 8: the general skinny kernel 2,895 tok/s (down
 // 24.9 µs live), split 8 x 8 units 2,990 (23.4), 8 x 4 units 3,010 (23.0); the first form,
 // which published each tile's parts as it finished it, stalled every wave on its ticket
 // round trip behind the per-tile barrier: 2,760 (31.5).

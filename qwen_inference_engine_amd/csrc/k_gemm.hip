@@ -405,8 +405,7 @@ __global__ __launch_bounds__(512) void gemm_big_kernel(GemmParams p, int n_mt) {
 }
 
 // ---------------------------------------------------------------------------
-// Prefill GEMM, phase-interleaved (round 4; cdna_hip_programming.md §5 "The 256² 8-phase
-// template", written for this NT layout).  256x256 block tile, BK = 64, 8 waves as 2 (M) x 4
+// Prefill GEMM, phase-interleaved (the 256² 8-phase template, written for this NT layout).  256x256 block tile, BK = 64, 8 waves as 2 (M) x 4
 // (N), 128x64 per wave = 8x4 accumulators; LDS = two 64-KB k-tile buffers (A rows then W
 // rows, 128-B rows, 16-B chunk c of row r at c ^ ((r >> 1) & 7): conflict-free
 // ds_read_b128 for the 16x16x32 fragments).  A k-tile is consumed in FOUR phases, one C
@@ -1119,7 +1118,7 @@ static int launch_gemm(int epi, unsigned gm, const GemmParams& p, size_t shm, hi
 }
 
 // ---------------------------------------------------------------------------
-// Block-scaled fp8 prefill GEMM (round 5; BASELINE config 4's "CDNA4 fp8 MFMA", numerics flag
+// Block-scaled fp8 prefill GEMM (numerics flag
 // QIE_LINEAR_ACT_FP8):  C[m, n] = sum_k (2^ea[m] qa[m, k]) (sw[n] qw[n, k])  with e4m3
 // activation codes qa and per-row power-of-two exponents ea (qie_quantize_rows_fp8), e4m3
 // weight codes qw with power-of-two row scales sw (the engine's fp8 arena, plain or 16-row
@@ -1505,7 +1504,7 @@ static int gemm_mx(const qie_linear_args* a, hipStream_t st) {
     const int64_t cus = device_cu_count();
     const int nk = (int)(a->K / mx::BK);
     G8Split sk{1, nullptr, nullptr};
-    // split only below half the chip (r05, same box, 2,048 rows): O (112 tiles) 91.0 unsplit
+    // split only below half the chip (2,048 rows): O (112 tiles) 91.0 unsplit
     // vs 78.0 split 3, down (112) 307 vs 188; QKV (144 tiles) 69.4 unsplit vs 93.9 split 3
     if (2 * tiles <= cus) {
         int best = 1;

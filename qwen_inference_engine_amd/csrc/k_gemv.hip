@@ -1169,7 +1169,7 @@ static int launch_gemv_t(const GemvParams& p, hipStream_t st, int blocks_per_cu)
         // Full-residency grid-stride grid (the SwiGLU default): every CU holds the same number
         // of blocks for the whole launch.  The balanced grid below gives every WAVE the same
         // task count but leaves CUs with 3 and 4 blocks (948 blocks at 4 per CU for Qwen2-7B
-        // gate/up): in-graph gate/up 43.0 -> 42.2 us, 358.9 -> 361.5 tok/s (same box, A/B)
+        // gate/up): in-graph gate/up 43.0 -> 42.2 us, 358.9 -> 361.5 tok/s (A/B in one run)
         static size_t cached_shm2 = 0;
         static int cached_nb2 = 0;
         int nb = cached_shm2 == shm ? cached_nb2 : 0;
@@ -1456,7 +1456,7 @@ int gemv(const qie_linear_args* a, hipStream_t st) {
             const int64_t n_tiles = (a->N + 15) / 16;
             p.xlds = lds_ok && (a->norm_w || n_tiles > 2 * (int64_t)device_cu_count()) ? 1 : 0;
             // Without a fused norm the staged copy is only an optimisation: keep the launch's
-            // dynamic LDS within the default 64 KiB (no raised kernel attribute).  r02's config-4
+            // dynamic LDS within the default 64 KiB (no raised kernel attribute).  An fp8 batch-8
             // gate/up node (8 rows x 3,592 + two 4-KiB reduction tiles per wave = 65,664 B) was
             // the one decode-graph node above it, and rocprofv3's kernel trace crashed on that
             // graph only; with NW - 1 reduction tiles it is 63,616 B and stays staged.
@@ -1539,7 +1539,7 @@ int gemv(const qie_linear_args* a, hipStream_t st) {
     // gate/up grid: full residency, grid-stride (-2, launch_gemv_t); QIE_GEMV_SWIGLU_BPC = N > 0
     // caps N blocks per CU, -1 the balanced grid (dev A/B)
     //
-    // Round 5, grid caps measured per shape (same box, interleaved, in the graph: tools/ab_decode.py;
+    // Grid caps measured per shape (interleaved, in the graph: tools/ab_decode.py;
     // outputs bit-identical — the grid only changes which wave takes which row task):
     //  * gate/up, Qwen2-7B (K 3,584, 74 row tasks per CU; 198 VGPRs, 2 resident blocks per CU):
     //    6 blocks per CU 42.7 -> 41.3 µs, 361.8 -> 366.7 tok/s — a sharp optimum (5: 357.4,

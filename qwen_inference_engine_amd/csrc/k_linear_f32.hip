@@ -6,7 +6,8 @@
 // The FMA kernel it replaces (k_layered.hip linear_kernel) keeps nothing in flight and fills 32 to 80 of 256 CUs at a few
 // hundred rows: 145 to 230 us for 1 to 2 GFLOP.  Here a 64 x 64 tile goes through an LDS-DMA ring of 32-k tiles (128-byte rows,
 // as k_gemm_mid.hip), 8 waves as 2 x 2 x 2 K halves, and tiles that do not fill the chip are split over K (slabs summed by the
-// last part, gemm8_kernel's protocol).  Bound: the fp32 matrix rate (157 TFLOP/s) or, at few rows, the weights.
+// last part, gemm8_kernel's protocol).  Bound: the fp32 matrix rate (157 TFLOP/s) or, at few rows, the weights.  us: 275 rows x 1,024 x
+// 2,816 230 -> 22, eight experts of some 69 rows (1,024 x 1,408 and 704 x 1,024) 189 and 174 -> 41 and 21.
 //   * The order of a sum depends on K alone: K is cut into 1 to 16 segments (a power of two), a wave's segment sums meet in pairs,
 //     pairs of pairs and so on, and at last the two K halves.  A workgroup owns an aligned group of segments, one node of that tree,
 //     so how many workgroups share a tile (by the rows of the launch and the memory there is for slabs) changes no bit.

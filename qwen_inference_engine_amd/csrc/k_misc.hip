@@ -186,7 +186,7 @@ struct QkvPostArgs {
     uint16_t* q_out;
 };
 
-// Round 6: the wave's heads are taken in batches of kQkvBatch whose source pairs are all
+// The wave's heads are taken in batches of kQkvBatch whose source pairs are all
 // loaded before the first store (the row-at-a-time form waited one memory round trip per head,
 // nine in a row per wave at Qwen2-7B widths); the arithmetic per element is unchanged.
 constexpr int kQkvBatch = 10;

@@ -145,7 +145,7 @@ __device__ __forceinline__ void st_granule(unsigned long long* g, unsigned tag, 
 // sc1 buffer loads (two granules per load: each granule still validates itself by its tag).
 // Whole sweeps: every granule still missing is re-loaded in ONE batch per pass — one memory round
 // trip per pass, never one dependent re-poll per granule (the first form spun on each missing
-// granule in turn: 6-10 us per gather, tools/pk_trace.py r06).  The byte offset is made opaque
+// granule in turn: 6-10 us per gather, tools/pk_trace.py).  The byte offset is made opaque
 // each pass, so the loads are re-issued, not hoisted out of the poll loop.  A failure (timeout,
 // or another block's error word) marks the block dead (LDS flag, read after the next barrier).
 template <int M>

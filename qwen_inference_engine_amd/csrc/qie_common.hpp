@@ -120,7 +120,7 @@ __host__ __device__ inline float e4m3_row_scale(float amax) {
     if (ldexpf(1.f, e - 1) * 448.f >= amax) s = ldexpf(1.f, e - 1);
     if (s * 448.f < amax) s *= 2.f;                       // exact checks: the division rounded
     // never below the smallest normal: the scale's exponent field is the MFMA's e8m0 operand
-    // (read from the float bits), and a subnormal s would read as exponent 0 (ADVICE r05)
+    // (read from the float bits), and a subnormal s would read as exponent 0
     const float smin = ldexpf(1.f, -126);
     return s < smin ? smin : s;
 }
