@@ -218,7 +218,7 @@ __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
                 constexpr int PP = decltype(pc)::value, S = 4 / PP;   // this wave's sums: pieces v PP + sub, v = j, j + S, ...
                 float ss[S] = {};
 #pragma unroll
-                for (int v = 0; v < NV; v++) {
+                for (int v = 0; v < (NV + PP - 1) / PP; v++) {
                     if ((v * PP + sub) * 512 >= K) break;
                     const uint32_t e[4] = {xv[v].x, xv[v].y, xv[v].z, xv[v].w};
 #pragma unroll
