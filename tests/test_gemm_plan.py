@@ -5,7 +5,7 @@ import subprocess
 
 import pytest
 
-from test_gpu_gemm_mid import PLANS
+from test_gpu_gemm_mid import GROWS, PLANS
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "qwen_inference_engine_amd", "csrc")
 
@@ -61,6 +61,12 @@ def test_gemm_mid_shapes_take_every_tile(plan):
     got = [(p[0], "whole" if p[2] == 1 else "split" if p[1] == 0 else "mixed") for p in plan([f"m {M} {N} {K} 256" for M, N, K, _, _ in PLANS])]
     assert got == [(t, kind) for _, _, _, t, kind in PLANS]
     assert set(got) == {(t, kind) for t in range(8) for kind in ("whole", "split", "mixed")}
+
+
+def test_a_shape_whose_slabs_outgrow_the_reserve(plan):
+    (tile, whole, splitk, tiles), = plan(["m %d %d %d 256" % GROWS])
+    bm, bn = [(64, 64), (64, 128), (128, 64), (128, 128), (192, 128), (256, 128), (320, 64), (320, 128)][tile]
+    assert splitk > 1 and (tiles - whole) * splitk * bm * bn * 4 > 64 << 20
 
 
 def test_gemm_mid_plans_are_sound(plan):

@@ -49,6 +49,7 @@ PLANS = [(17, 72, 64, 0, "whole"), (33, 72, 2048, 0, "split"), (17, 40000, 128, 
          (210, 9278, 6464, 5, "split"), (273, 38147, 1792, 6, "mixed"), (259, 12692, 64, 6, "whole"), (1064, 11882, 1728, 7, "mixed"),
          (257, 8338, 11264, 7, "split")]
 SHAPES = [p[:3] for p in PLANS]
+GROWS = (292, 18768, 15168)   # partial tiles of more than the 64 MB that a stream has from the start
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES)

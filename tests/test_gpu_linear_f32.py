@@ -1,10 +1,15 @@
 """fp32 products of the layered models on the matrix cores at the sizes where they can go wrong: 1 to 16 rows (k_decode_bf16.hip's
 fp32 form: X in LDS and through the ring), 17 to 300 (k_linear_f32.hip: whole and split tiles, ragged rows and columns, experts of
 few and of no rows), widths off their grid (the plain kernels); and the exact attention at head sizes on and off four elements."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
+import gpu_util as G
 from lugipel_oracle import attn, dense, gru, moe
+from qwen_inference_engine_amd import _lib
+from test_gpu_gemm_mid import GROWS
 from test_gpu_lugipel import feed, model, rel  # noqa: F401  (model: a fixture)
 
 pytestmark = pytest.mark.gpu
@@ -36,8 +41,8 @@ def test_rows(model, layers, width):  # noqa: F811
 
 
 def test_replay_after_larger_steps(model):  # noqa: F811
-    """Captured steps keep their split-K memory: steps of 16 rows with four experts each replay after a portion of 60 rows, and
-    after a prompt of another batch on the same engine, made that memory grow."""
+    """Captured steps keep their split-K memory: steps of 16 rows with four experts each replay after larger steps, a prompt of another
+    batch on the same engine, and a product on its stream that outgrows the memory the capture has seen."""
     layers = [gru(width=256, mlp=moe(experts=8, identity=0, top=4, count=1, keep=1, ff=256)), attn(heads=4, kv_heads=2, dim=64, vdim=64, size=40, mlp=None)]
     m = model(layers, seed=3, vocab=1003, width=256, slots=4, max_ctx=512)
     seqs = [[], []]
@@ -64,8 +69,15 @@ def test_replay_after_larger_steps(model):  # noqa: F811
     for _ in range(3):
         small()
     other.close()
-    small()
-    assert m.batch.graph_stats()[1] > before + 6
+    M, N, K = GROWS
+    a, x, w, y = _lib.LinearArgsC(), G.zeros_bf16(M, K), G.zeros_bf16(N, K), G.dev(np.full((M, N), 7.0, np.float32))
+    a.x, a.ldx, a.w[0], a.seg_rows[0], a.M, a.K, a.N, a.y, a.ldy, a.epilogue = G.p(x), K, G.p(w), N, M, K, N, G.p(y), N, _lib.QIE_EPI_F32
+    for _ in range(2):
+        G.check(_lib.load().qie_linear(C.byref(a), m.eng.stream), "qie_linear")
+        for _ in range(3):
+            small()
+    assert not y.numpy().any()
+    assert m.batch.graph_stats()[1] > before + 12
 
 
 @pytest.mark.parametrize("width", [2048, 3072])   # X in LDS, through the ring
