@@ -47,6 +47,32 @@ inline Plan plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool grouped, i
 }
 }  // namespace lf
 
+// ---------------------------------------------------------------- order of the tiles of the split GEMMs
+// Workgroup numbers run down bands of `gm` row tiles, column tile by column tile: the workgroups that an XCD runs at a time (32 CUs,
+// neighbours in number) cover about as many rows as columns, which is the least that its L2 has to fetch for them.  One band of all
+// row tiles fetched A anew for every column tile.  Qwen2-7B at 8,192 rows, one band / bands: gate and up 1,800 / 1,690 us, down
+// 950 / 885, QKV 263 / 256, O 234 / 228; Qwen2-0.5B down at 6,000 rows 68 / 60.  Up to 8 row tiles are one band as before.
+QIE_PLAN_HD inline void banded(int wid, int n_mt, int n_nt, int gm, int* mt, int* nt) {
+    if (gm >= n_mt) {
+        *mt = wid % n_mt;
+        *nt = wid / n_mt;
+        return;
+    }
+    const int band = gm * n_nt, b = wid / band, at = wid - b * band;
+    const int h = n_mt - b * gm < gm ? n_mt - b * gm : gm;
+    *mt = b * gm + at % h;
+    *nt = at / h;
+}
+
+// height of even bands, up to about twice as tall as wide (`at_once` tiles of bm x bn outputs): fewer bands read the weights less often,
+// and bands of 4 row tiles of 256 x 128 where 8 or 12 fit one band lost 4 %
+inline int band_height(int n_mt, int bm, int bn, int at_once) {
+    int h = 1;
+    while ((h + 1) * (h + 1) * bm <= 2 * at_once * bn) h++;
+    const int bands = std::max(1, n_mt / h);
+    return (n_mt + bands - 1) / bands;
+}
+
 // ---------------------------------------------------------------- k_gemm_mid.hip
 namespace mid {
 constexpr int BK = 64;

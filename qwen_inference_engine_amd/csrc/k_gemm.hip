@@ -15,6 +15,7 @@
 //   * blockIdx.x runs over M tiles so the blocks sharing a weight tile are
 //     adjacent in dispatch order (weights streamed ~once, activations L2/MALL).
 #include "gemm_impl.hpp"
+#include "gemm_plan.hpp"
 
 #include <map>
 #include <mutex>
@@ -435,7 +436,7 @@ constexpr int BUF = (BM + BN) * BK * 2;   // 64 KB: A rows [0, 256) then W rows,
 // in PART order (sc1 loads: cdna_hip_programming.md §5 'Projection GEMM' item 2), so the result
 // does not depend on arrival order, runs the epilogue and resets the ticket.
 template <int EPI>
-__global__ __launch_bounds__(512) void gemm8_kernel(GemmParams p, int n_mt, G8Split sk) {
+__global__ __launch_bounds__(512) void gemm8_kernel(GemmParams p, int n_mt, int n_nt, int gm, G8Split sk) {
 #pragma clang fp contract(off)
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -446,7 +447,9 @@ __global__ __launch_bounds__(512) void gemm8_kernel(GemmParams p, int n_mt, G8Sp
     const int q8 = nwg >> 3, r8 = nwg & 7, xcd = orig & 7;
     const int wid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (orig >> 3);
     const int tile = wid / sk.splitk, part = wid % sk.splitk;
-    const int64_t mt = tile % n_mt, nt = tile / n_mt;
+    int mti, nti;
+    banded(tile, n_mt, n_nt, gm, &mti, &nti);
+    const int64_t mt = mti, nt = nti;
     const int64_t m0 = mt * g8::BM;
 
     // DMA sources: unit u (0 UA0, 1 UB0, 2 UB1, 3 UA1), instruction i of this wave moves the
@@ -955,7 +958,8 @@ static int launch_gemm8_t(const GemmParams& p, int n_mt, int n_tiles, const G8Sp
         QIE_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
         raised = true;
     }
-    hipLaunchKernelGGL((gemm8_kernel<EPI>), dim3((unsigned)(n_tiles * sk.splitk)), dim3(512), shm, st, p, n_mt, sk);
+    hipLaunchKernelGGL((gemm8_kernel<EPI>), dim3((unsigned)(n_tiles * sk.splitk)), dim3(512), shm, st, p, n_mt,
+                       n_tiles / n_mt, band_height(n_mt, g8::BM, g8::BN, 32), sk);
     QIE_LAUNCH_CHECK();
     return 0;
 }

@@ -40,7 +40,7 @@ __device__ __forceinline__ const uint16_t* mid_wrow(const GemmParams& p, int64_t
 }
 
 template <int EPI, int BM, int BN, int SLOTS>
-__global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, int whole, G8Split sk) {
+__global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, int n_nt, int gm, int whole, G8Split sk) {
 #pragma clang fp contract(off)
     constexpr int TM = BM / 2, TN = BN / 2, FI = TM / 16, FJ = TN / 16, FH = FI / 2;
     constexpr int SLOT = (BM + BN) * 128;      // A rows, then W rows, 128 B each
@@ -58,7 +58,9 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
     const int wid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (orig >> 3);
     const int parts = cut ? sk.splitk : 1, cuts = nwg / parts;   // cut tiles: part-major, so an XCD's parts share a K range of A
     const int part = cut ? wid / cuts : 0, ct = cut ? wid % cuts : 0, tile = cut ? whole + ct : wid;
-    const int64_t mt = tile % n_mt, nt = tile / n_mt, m0 = mt * BM;
+    int mti, nti;
+    banded(tile, n_mt, n_nt, gm, &mti, &nti);
+    const int64_t mt = mti, nt = nti, m0 = mt * BM;
 
     const int nk_all = (int)(p.K / mid::BK);
     const int kb = (int)((int64_t)part * nk_all / parts);        // this part's k-tiles [kb, kb + nk)
@@ -299,7 +301,7 @@ int launch_mid_t(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, hi
     }
     const int tiles = pl.n_mt * pl.n_nt, whole = sk.splitk > 1 ? pl.whole : tiles;
     hipLaunchKernelGGL((gemm_mid_kernel<EPI, BM, BN, SLOTS>), dim3((unsigned)(whole + (tiles - whole) * sk.splitk)), dim3(512), shm,
-                       st, p, pl.n_mt, whole, sk);
+                       st, p, pl.n_mt, pl.n_nt, band_height(pl.n_mt, BM, BN, 32 * mid::TILES[pl.tile].per_cu), whole, sk);
     QIE_LAUNCH_CHECK();
     return 0;
 }
