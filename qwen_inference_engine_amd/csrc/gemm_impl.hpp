@@ -24,7 +24,7 @@ struct GemmParams {
     int64_t wrows;       // total weight rows addressable (for clamping)
     uint16_t* C;
     int64_t ldc;
-    int vec = 0;         // rows of C take 4-element vector stores (set by the kernel's launcher)
+    int vec = 0;         // rows of C take 4-element vector stores
 };
 
 __device__ __forceinline__ void glds16(const void* src, void* lds) {
@@ -34,6 +34,51 @@ __device__ __forceinline__ void glds16(const void* src, void* lds) {
 
 // chunk swizzle of 128-B LDS rows: the 16-B chunk c of row r sits at c ^ g8_swz(r)
 __device__ __forceinline__ int g8_swz(int r) { return (r >> 1) & 7; }
+
+// ---------------------------------------------------------------- epilogues of four columns a lane
+// dst: C at the first of them; `left` columns of the row from there on, the others are not stored.
+
+__device__ __forceinline__ void store_quad(uint16_t* dst, const float (&v)[4], bool vec, int64_t left) {
+    if (vec && left >= 4) {
+        *reinterpret_cast<uint2*>(dst) = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            if (r < left) dst[r] = f2bf(v[r]);
+    }
+}
+__device__ __forceinline__ void store_quad_f32(float* dst, f32x4 v, bool vec, int64_t left) {
+    if (vec && left >= 4) {
+        *reinterpret_cast<f32x4*>(dst) = v;
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            if (r < left) dst[r] = v[r];
+    }
+}
+// residual: C = bf16(x + bf16(v)), x what quad_before read there
+__device__ __forceinline__ uint2 quad_before(const uint16_t* src, bool vec, int64_t left) {
+    if (vec && left >= 4) return *reinterpret_cast<const uint2*>(src);
+    uint32_t h[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+        if (r < left) h[r] = src[r];
+    return make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+}
+__device__ __forceinline__ void add_quad(uint16_t* dst, uint2 x, f32x4 v, bool vec, int64_t left) {
+    const float o[4] = {bf_lo(x.x) + rbf(v[0]), bf_hi(x.x) + rbf(v[1]), bf_lo(x.y) + rbf(v[2]), bf_hi(x.y) + rbf(v[3])};
+    store_quad(dst, o, vec, left);
+}
+// biases of columns col .. col + 3 (zero where a segment has none)
+__device__ __forceinline__ void quad_bias(const GemmParams& p, int64_t col, float (&bias)[4]) {
+    if (!(p.b0 || p.b1 || p.b2)) return;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int64_t c = col + r < p.N ? col + r : p.N - 1;
+        const uint16_t* b = c < p.n0 ? p.b0 : (c < p.n01 ? p.b1 : p.b2);
+        if (b) bias[r] = bf2f(b[c < p.n0 ? c : (c < p.n01 ? c - p.n0 : c - p.n01)]);
+    }
+}
 
 typedef unsigned int u32x4_g8 __attribute__((ext_vector_type(4)));
 

@@ -47,21 +47,29 @@ inline Plan plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool grouped, i
 }
 }  // namespace lf
 
+// a / b of tile counts (below 2^22), uniform over a wave.  On the device by a float's reciprocal and one step of correction: an
+// integer division is some forty instructions of a kernel's start, which cost short products 0.2 us
+QIE_PLAN_HD inline int quotient(int a, int b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    int q = (int)((float)a * __builtin_amdgcn_rcpf((float)b));
+    const int r = a - q * b;
+    q += r >= b ? 1 : r < 0 ? -1 : 0;
+    return __builtin_amdgcn_readfirstlane(q);
+#else
+    return a / b;
+#endif
+}
+
 // ---------------------------------------------------------------- order of the tiles of the split GEMMs
 // Workgroup numbers run down bands of `gm` row tiles, column tile by column tile: the workgroups that an XCD runs at a time (32 CUs,
 // neighbours in number) cover about as many rows as columns, which is the least that its L2 has to fetch for them.  One band of all
 // row tiles fetched A anew for every column tile.  Qwen2-7B at 8,192 rows, one band / bands: gate and up 1,800 / 1,690 us, down
 // 950 / 885, QKV 263 / 256, O 234 / 228; Qwen2-0.5B down at 6,000 rows 68 / 60.  Up to 8 row tiles are one band as before.
 QIE_PLAN_HD inline void banded(int wid, int n_mt, int n_nt, int gm, int* mt, int* nt) {
-    if (gm >= n_mt) {
-        *mt = wid % n_mt;
-        *nt = wid / n_mt;
-        return;
-    }
-    const int band = gm * n_nt, b = wid / band, at = wid - b * band;
-    const int h = n_mt - b * gm < gm ? n_mt - b * gm : gm;
-    *mt = b * gm + at % h;
-    *nt = at / h;
+    const int band = gm * n_nt, b = quotient(wid, band), at = wid - b * band;
+    const int h = n_mt - b * gm < gm ? n_mt - b * gm : gm, c = quotient(at, h);
+    *mt = b * gm + at - c * h;
+    *nt = c;
 }
 
 // height of even bands, up to about twice as tall as wide (`at_once` tiles of bm x bn outputs): fewer bands read the weights less often,

@@ -523,7 +523,7 @@ __global__ __launch_bounds__(512) void gemm8_kernel(GemmParams p, int n_mt, int 
 #pragma unroll
                 for (int j = 0; j < 2; j++)
                     acc[4 * qa + i][2 * qb + j] =
-                        __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i][s2], fb[j][s2], acc[4 * qa + i][2 * qb + j], 0, 0, 0);
+                        __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j][s2], fa[i][s2], acc[4 * qa + i][2 * qb + j], 0, 0, 0);   // W Aᵀ
         __builtin_amdgcn_s_setprio(0);
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -617,51 +617,58 @@ __global__ __launch_bounds__(512) void gemm8_kernel(GemmParams p, int n_mt, int 
         if (tid == 0) __hip_atomic_store(sk.cnt + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 
-    // ---------------- epilogue (as gemm_big_kernel at BNT = 256)
-    constexpr int NJ = 4;
+    // ---------------- epilogue.  D = W Aᵀ: a lane holds row lane & 15 and columns 4 g .. 4 g + 3 of a fragment, one 8- (fp32: 16-)
+    // byte store where C's rows allow it
+    const bool vec = p.vec != 0;
+    const int64_t row0 = m0 + wm * 128 + fr;
     if constexpr (EPI == QIE_EPI_SWIGLU) {
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
+        for (int jj = 0; jj < 2; jj++) {
+            const int64_t col = nt * 128 + 32 * wn + 16 * jj + 4 * g;
 #pragma unroll
-            for (int jj = 0; jj < NJ / 2; jj++) {
-                const int64_t col = nt * 128 + 32 * wn + 16 * jj + fr;
-                if (col >= p.N) continue;
+            for (int i = 0; i < 8; i++) {
+                const int64_t row = row0 + i * 16;
+                if (row >= p.M) continue;
+                float h[4];
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
-                    const int64_t row = m0 + wm * 128 + i * 16 + g * 4 + r;
-                    if (row >= p.M) continue;
                     const float gg = rbf(acc[i][jj][r]);
-                    const float uu = rbf(acc[i][jj + NJ / 2][r]);
-                    const float av = rbf(gg * (1.0f / (1.0f + expf(-gg))));
-                    p.C[row * p.ldc + col] = f2bf(uu * av);
+                    const float uu = rbf(acc[i][jj + 2][r]);
+                    h[r] = uu * rbf(gg * (1.0f / (1.0f + expf(-gg))));
                 }
+                store_quad(p.C + row * p.ldc + col, h, vec, p.N - col);
             }
         }
     } else {
+        uint2 before[8][4];
+        if constexpr (EPI == QIE_EPI_RESIDUAL) {   // all on their way at once: loads between the stores would each wait for memory
 #pragma unroll
-        for (int j = 0; j < NJ; j++) {
-            const int64_t col = nt * 256 + wn * 64 + j * 16 + fr;
-            if (col >= p.N) continue;
-            float bias = 0.f;
-            if constexpr (EPI == QIE_EPI_STORE) {
-                const uint16_t* b = col < p.n0 ? p.b0 : (col < p.n01 ? p.b1 : p.b2);
-                if (b) bias = bf2f(b[col < p.n0 ? col : (col < p.n01 ? col - p.n0 : col - p.n01)]);
+            for (int j = 0; j < 4; j++) {
+                const int64_t col = nt * 256 + wn * 64 + j * 16 + 4 * g;
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    const int64_t row = row0 + i * 16;
+                    before[i][j] = row < p.M && col < p.N ? quad_before(p.C + row * p.ldc + col, vec, p.N - col) : make_uint2(0u, 0u);
+                }
             }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int64_t col = nt * 256 + wn * 64 + j * 16 + 4 * g;
+            float bias[4] = {0.f, 0.f, 0.f, 0.f};
+            if constexpr (EPI == QIE_EPI_STORE) quad_bias(p, col, bias);
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int64_t row = m0 + wm * 128 + i * 16 + g * 4 + r;
-                    if (row >= p.M) continue;
-                    if constexpr (EPI == QIE_EPI_F32) {
-                        reinterpret_cast<float*>(p.C)[row * p.ldc + col] = acc[i][j][r];
-                        continue;
-                    }
-                    uint16_t* dst = p.C + row * p.ldc + col;
-                    if constexpr (EPI == QIE_EPI_RESIDUAL)
-                        *dst = f2bf(bf2f(*dst) + rbf(acc[i][j][r]));
-                    else
-                        *dst = f2bf(acc[i][j][r] + bias);
+                const int64_t row = row0 + i * 16;
+                if (row >= p.M) continue;
+                const f32x4 v = acc[i][j];
+                if constexpr (EPI == QIE_EPI_F32) {
+                    store_quad_f32(reinterpret_cast<float*>(p.C) + row * p.ldc + col, v, vec, p.N - col);
+                } else if constexpr (EPI == QIE_EPI_RESIDUAL) {
+                    add_quad(p.C + row * p.ldc + col, before[i][j], v, vec, p.N - col);
+                } else {
+                    const float o[4] = {v[0] + bias[0], v[1] + bias[1], v[2] + bias[2], v[3] + bias[3]};
+                    store_quad(p.C + row * p.ldc + col, o, vec, p.N - col);
                 }
             }
         }
@@ -1548,6 +1555,7 @@ int gemm(const qie_linear_args* a, hipStream_t st) {
     p.wrows = 0;
     p.C = (uint16_t*)a->y;
     p.ldc = a->ldy;
+    p.vec = a->ldy % 4 == 0 && ((uintptr_t)a->y) % (a->epilogue == QIE_EPI_F32 ? 16 : 8) == 0;
     const size_t shm = (size_t)2 * (BM + BN) * BK * 2;
     const unsigned gm = (unsigned)cdiv(a->M, BM);
     QIE_REQUIRE(a->K % 8 == 0, "qie_linear: GEMM needs K %% 8 == 0");

@@ -56,8 +56,8 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
     const int nwg = cut ? gridDim.x - whole : whole, orig = cut ? blockIdx.x - whole : blockIdx.x;
     const int q8 = nwg >> 3, r8 = nwg & 7, xcd = orig & 7;
     const int wid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (orig >> 3);
-    const int parts = cut ? sk.splitk : 1, cuts = nwg / parts;   // cut tiles: part-major, so an XCD's parts share a K range of A
-    const int part = cut ? wid / cuts : 0, ct = cut ? wid % cuts : 0, tile = cut ? whole + ct : wid;
+    const int parts = cut ? sk.splitk : 1, cuts = quotient(nwg, parts);   // cut tiles: part-major, so an XCD's parts share a K range of A
+    const int part = quotient(wid, cuts), ct = wid - part * cuts, tile = cut ? whole + ct : wid;
     int mti, nti;
     banded(tile, n_mt, n_nt, gm, &mti, &nti);
     const int64_t mt = mti, nt = nti, m0 = mt * BM;
@@ -105,21 +105,27 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
         if (t + SLOTS - 1 < nk) stage(t + SLOTS - 1, fill);
         const unsigned char* buf = smem + slot * SLOT;
         bf16x8 fa[FI], fb[FJ];
+        auto read_a = [&](int i) {
+            const int row = wm * TM + i * 16 + fr;
+            fa[i] = *reinterpret_cast<const bf16x8*>(buf + row * 128 + (((4 * wk + g) ^ g8_swz(row)) * 16));
+        };
 #pragma unroll
         for (int j = 0; j < FJ; j++) {
             const int row = BM + wn * TN + j * 16 + fr;
             fb[j] = *reinterpret_cast<const bf16x8*>(buf + row * 128 + (((4 * wk + g) ^ g8_swz(row)) * 16));
         }
+        constexpr int AHEAD = BM >= 256 ? 2 : FI;   // tall tiles: two A fragments on their way while one is multiplied
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) read_a(i);
 #pragma unroll
         for (int i = 0; i < FI; i++) {
-            const int row = wm * TM + i * 16 + fr;
-            fa[i] = *reinterpret_cast<const bf16x8*>(buf + row * 128 + (((4 * wk + g) ^ g8_swz(row)) * 16));
-        }
-#pragma unroll
-        for (int i = 0; i < FI; i++)
+            if (i + AHEAD < FI) read_a(i + AHEAD);
+            if (AHEAD < FI) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int j = 0; j < FJ; j++)
                 acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);   // W Aᵀ
+            if (AHEAD < FI) __builtin_amdgcn_sched_barrier(0);
+        }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave's reads of the slot are done
         __builtin_amdgcn_sched_barrier(0);
         slot = slot + 1 == SLOTS ? 0 : slot + 1;
@@ -220,14 +226,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
                     const float uu = rbf(res[i][jj + FJ / 2][r]);
                     h[r] = uu * rbf(gg * (1.0f / (1.0f + expf(-gg))));
                 }
-                uint16_t* dst = p.C + row * p.ldc + col;
-                if (vec && col + 4 <= p.N) {
-                    *reinterpret_cast<uint2*>(dst) = make_uint2(pack2(h[0], h[1]), pack2(h[2], h[3]));
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        if (col + r < p.N) dst[r] = f2bf(h[r]);
-                }
+                store_quad(p.C + row * p.ldc + col, h, vec, p.N - col);
             }
         }
     } else {
@@ -235,53 +234,20 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
         for (int j = 0; j < FJ; j++) {
             const int64_t col = nt * BN + wn * TN + j * 16 + 4 * g;
             float bias[4] = {0.f, 0.f, 0.f, 0.f};
-            if constexpr (EPI == QIE_EPI_STORE) {
-                if (p.b0 || p.b1 || p.b2) {
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const int64_t c = col + r < p.N ? col + r : p.N - 1;
-                        const uint16_t* b = c < p.n0 ? p.b0 : (c < p.n01 ? p.b1 : p.b2);
-                        if (b) bias[r] = bf2f(b[c < p.n0 ? c : (c < p.n01 ? c - p.n0 : c - p.n01)]);
-                    }
-                }
-            }
+            if constexpr (EPI == QIE_EPI_STORE) quad_bias(p, col, bias);
 #pragma unroll
             for (int i = 0; i < FH; i++) {
                 const int64_t row = row0 + i * 16;
                 if (row >= p.M) continue;
                 const f32x4 v = res[i][j];
                 if constexpr (EPI == QIE_EPI_F32) {
-                    float* dst = reinterpret_cast<float*>(p.C) + row * p.ldc + col;
-                    if (vec && col + 4 <= p.N) {
-                        *reinterpret_cast<f32x4*>(dst) = v;
-                    } else {
-#pragma unroll
-                        for (int r = 0; r < 4; r++)
-                            if (col + r < p.N) dst[r] = v[r];
-                    }
-                    continue;
-                }
-                uint16_t* dst = p.C + row * p.ldc + col;
-                if (vec && col + 4 <= p.N) {
-                    float o[4];
-                    if constexpr (EPI == QIE_EPI_RESIDUAL) {
-                        const uint2 x = *reinterpret_cast<const uint2*>(dst);
-                        o[0] = bf_lo(x.x) + rbf(v[0]);
-                        o[1] = bf_hi(x.x) + rbf(v[1]);
-                        o[2] = bf_lo(x.y) + rbf(v[2]);
-                        o[3] = bf_hi(x.y) + rbf(v[3]);
-                    } else {
-#pragma unroll
-                        for (int r = 0; r < 4; r++) o[r] = v[r] + bias[r];
-                    }
-                    *reinterpret_cast<uint2*>(dst) = make_uint2(pack2(o[0], o[1]), pack2(o[2], o[3]));
+                    store_quad_f32(reinterpret_cast<float*>(p.C) + row * p.ldc + col, v, vec, p.N - col);
+                } else if constexpr (EPI == QIE_EPI_RESIDUAL) {
+                    uint16_t* dst = p.C + row * p.ldc + col;
+                    add_quad(dst, quad_before(dst, vec, p.N - col), v, vec, p.N - col);
                 } else {
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        if (col + r >= p.N) continue;
-                        if constexpr (EPI == QIE_EPI_RESIDUAL) dst[r] = f2bf(bf2f(dst[r]) + rbf(v[r]));
-                        else dst[r] = f2bf(v[r] + bias[r]);
-                    }
+                    const float o[4] = {v[0] + bias[0], v[1] + bias[1], v[2] + bias[2], v[3] + bias[3]};
+                    store_quad(p.C + row * p.ldc + col, o, vec, p.N - col);
                 }
             }
         }
@@ -324,8 +290,7 @@ int launch_mid(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, hipS
 // other_us: what the caller's other kernel for this shape takes
 int gemm_mid(const qie_linear_args* a, const GemmParams& q, float other_us, hipStream_t st, bool* launched) {
     *launched = false;
-    GemmParams p = q;
-    p.vec = a->ldy % 4 == 0 && ((uintptr_t)a->y) % (a->epilogue == QIE_EPI_F32 ? 16 : 8) == 0;
+    const GemmParams& p = q;
     if (a->K % mid::BK != 0) return 0;   // (rows of x and weights are on the 16-byte grid of LDS-DMA: qie_linear)
     const int64_t cols = a->epilogue == QIE_EPI_SWIGLU ? 2 * a->N : a->N;
     const mid::Plan pl = mid::plan(a->M, cols, a->K, device_cu_count());

@@ -25,3 +25,32 @@ def test_products(qlib, M, N, K, flags):
     want, scale = products(x, w)
     # two fp32 sums of K products in different orders
     assert (np.abs(y.numpy() - want) <= 1e-5 * scale).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 261, 256), (511, 520, 320)])   # scalar stores and a row stride of its own; vector stores
+@pytest.mark.parametrize("epi", ["store", "residual", "swiglu"])
+def test_epilogues_of_256_tiles(qlib, oracle, M, N, K, epi):
+    ld = N + N % 2 * 2
+    x, res = bf16((M, K), 1.0, 3), bf16((M, ld), 1.0, 5)
+    ws = [bf16((N, K), (1.5 - 0.5 * i) * K ** -0.5, 4 + i) for i in range(2 if epi == "swiglu" else 1)]
+    y, dx, dw, db = G.dev(res), G.dev(x), [G.dev(w) for w in ws], G.dev(bf16((N,), 0.5, 7))
+    a = _lib.LinearArgsC()
+    a.x, a.ldx, a.M, a.K, a.N, a.y, a.ldy, a.flags = G.p(dx), K, M, K, N, G.p(y), ld, _lib.QIE_LINEAR_TILE256
+    for i, w in enumerate(dw):
+        a.w[i], a.seg_rows[i] = G.p(w), N
+    a.epilogue = {"store": _lib.QIE_EPI_STORE, "residual": _lib.QIE_EPI_RESIDUAL, "swiglu": _lib.QIE_EPI_SWIGLU}[epi]
+    if epi == "store":
+        a.bias[0] = G.p(db)
+    G.check(_lib.load().qie_linear(C.byref(a), None), "qie_linear")
+    got = G.host_bf16(y)
+    assert np.array_equal(got[:, N:], res[:, N:])   # nothing behind the row's columns
+    got, (v, scale) = G.bf(got)[:, :N], products(x, ws[0])
+    if epi == "swiglu":
+        u, us = products(x, ws[1])
+        want = u / (1.0 + np.exp(-v)) * v
+        # |silu'| <= 1.1; three bf16 roundings (gate, silu, product) and one of the up sum
+        tol = 2.0 ** -7 * (np.abs(want) + 1.1 * np.abs(u) * np.abs(v)) + 1e-5 * (1.1 * np.abs(u) * scale + np.abs(v) * us)
+    else:
+        want = v + G.bf(bf16((N,), 0.5, 7)) if epi == "store" else G.bf(res)[:, :N] + G.bf(oracle.f32_to_bf16(v))
+        tol = 2.0 ** -7 * (np.abs(v) + np.abs(want)) + 1e-5 * scale   # an ulp of either rounding
+    assert (np.abs(got - want) <= tol).all()
