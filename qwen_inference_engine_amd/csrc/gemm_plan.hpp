@@ -103,6 +103,16 @@ constexpr Tile TILES[] = {
     {320, 64, 3, 1, 6.9f, .70f, 6.5f, 3.f, .787f},  {320, 128, 2, 1, 9.4f, 1.11f, 14.f, 2.f, 1.2f},
 };
 constexpr int N_TILES = sizeof(TILES) / sizeof(TILES[0]);
+// Tiles of 160 columns, numbered on from TILES: where the columns of 128-column tiles start a round of the chip that they hardly fill
+// (37,888 columns: 296 tiles, 237 of these), and so many rows of the workgroups' own (weights) that a tile of fewer columns loads more
+// for the same outputs.  Whole only.  Fitted to rounds that are nearly full.
+constexpr Tile WIDE[] = {
+    {128, 160, 4, 1, 3.f, 1.f, 14.3f, -1.3f, .69f}, {192, 160, 3, 1, 6.6f, 1.1f, 7.1f, 6.3f, .825f},
+    {256, 160, 3, 1, 8.8f, 1.29f, 0.f, 10.f, 1.f}, {320, 160, 2, 1, 9.6f, 1.56f, 0.f, 13.f, 1.17f},
+};
+constexpr int N_WIDE = sizeof(WIDE) / sizeof(WIDE[0]);
+inline const Tile& shape(int tile) { return tile < N_TILES ? TILES[tile] : WIDE[tile - N_TILES]; }
+
 struct Plan {
     int tile, whole, splitk, n_mt, n_nt;
     float us;
@@ -139,6 +149,20 @@ inline Plan plan(int64_t M, int64_t cols, int64_t K, int64_t cus) {
             us = std::max(us, floor_us);
             if (us < best.us) best = {c, (int)whole, s, (int)n_mt, (int)n_nt, us};
         }
+    }
+    return best;
+}
+
+// The plan among tiles of 160 columns.
+inline Plan plan_wide(int64_t M, int64_t cols, int64_t K, int64_t cus) {
+    Plan best{-1, 0, 1, 0, 0, 1e30f};
+    const int nk = (int)(K / BK);
+    for (int c = 0; c < N_WIDE; c++) {
+        const Tile& t = WIDE[c];
+        const int64_t n_mt = (M + t.bm - 1) / t.bm, n_nt = (cols + t.bn - 1) / t.bn, tiles = n_mt * n_nt;
+        if (tiles > (1 << 22)) continue;
+        const float us = tiles <= cus ? t.a1 + nk * t.s1 : t.a2 + rounds(tiles / (float)cus) * (t.f2 + nk * t.s2);
+        if (us < best.us) best = {N_TILES + c, (int)tiles, 1, (int)n_mt, (int)n_nt, us};
     }
     return best;
 }

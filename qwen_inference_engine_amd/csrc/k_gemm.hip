@@ -1578,7 +1578,7 @@ int gemm(const qie_linear_args* a, hipStream_t st) {
         // phase-interleaved 256x256 kernel (K a multiple of 64, >= 4 k-tiles): Qwen2-7B gate/up at 2,048
         // rows 612 -> 488 us, bit-identical to gemm_big; down split-K 2: 309 -> 247 us
         const bool g8ok = a->K % g8::BK == 0 && a->K >= 4 * g8::BK;
-        // (Qwen2-7B gate/up, us: 301 rows 161 with the 256x256 kernel, 119 with k_gemm_mid.hip; 700 rows 183 against 229)
+        // (Qwen2-7B gate/up, us: 301 rows 161 with the 256x256 kernel, 97 with k_gemm_mid.hip; 700 rows 183 against 229)
         if (dev_env("QIE_MID", 1) && force < 0 && !(a->flags & QIE_LINEAR_STREAMK)) {
             bool launched = false;
             const int rc = gemm_mid(a, p, g8ok && a->M >= big::BM ? g8_us(t256, cus, (int)(a->K / g8::BK)) : 1e30f, st, &launched);

@@ -5,8 +5,13 @@
 // At these row counts the weights come from HBM once and the 256x256 tiles of the long-prompt kernels leave most of the
 // chip idle (Qwen2-7B, 301 rows: 2 x 14 tiles for the O and down projections), while the register-staged 128x128 kernel
 // holds one k-tile in flight and waits a memory round trip (about 1 us) for every 64 of K.  Here:
-//   * a BM x BN tile (128x128, 128x64, 64x128, 64x64), BK = 64, in a ring of LDS slots filled by LDS-DMA: all slots but
-//     one are in flight, so a CU keeps 48-96 KB of loads outstanding; one barrier per k-tile;
+//   * a BM x BN tile (64x64 to 320x160), BK = 64, in a ring of LDS slots filled by LDS-DMA: all slots but one are in flight,
+//     one barrier per k-tile;
+//   * what bounds it: one CU fills its LDS at 130-140 GB/s with lines of its L2, 97 of the Infinity Cache, 54-64 of HBM (some 40 KB of
+//     requests in flight at their latency; rings of 2 to 9 slots, split roles of waves and prefetches into L2 by the same CUs all
+//     measured the same), so the time follows the rows of A and W that a CU stages for its outputs: tall tiles, and columns in tiles
+//     that fill rounds of the chip.  Qwen2-7B gate / up, 128 / 160 columns a tile: 113 rows 71 / 58 us, 200 rows 97 / 78, 301 rows 120 /
+//     97, 512 rows 171 / 143;
 //   * 8 waves as 2 (M) x 2 (N) x 2 (K halves of every k-tile): a wave's tile is half the block's in both directions, which
 //     reads LDS as often as four waves would, and two waves a SIMD cover each other's fragment reads.  The K halves meet in
 //     LDS once, behind the loop;
@@ -21,15 +26,17 @@
 
 namespace qie {
 
-// weight row of tile column c of column tile nt; SwiGLU tiles hold, per wave slice of BN / 2 columns, a half of gate rows
-// and the same outputs' up rows
+// weight row of tile column c of column tile nt.  SwiGLU: a lane of the epilogue holds columns 4 g .. 4 g + 3 of every fragment, so
+// those are two gate rows and the same outputs' up rows; two fragments give it four outputs side by side (a last odd one two)
 template <int EPI, int BN>
 __device__ __forceinline__ const uint16_t* mid_wrow(const GemmParams& p, int64_t nt, int c) {
     if constexpr (EPI == QIE_EPI_SWIGLU) {
-        constexpr int TN = BN / 2, HALF = TN / 2;
-        const int64_t j = nt * TN + (c / TN) * HALF + (c % HALF);
+        constexpr int TN = BN / 2, FJ = TN / 16;
+        const int cs = c % TN, f = cs / 16, g = (cs % 16) / 4, r = cs % 4;
+        const int jl = f / 2 * 16 + (f == FJ - 1 && FJ % 2 ? 2 * g : 4 * g + 2 * (f % 2)) + (r & 1);
+        const int64_t j = nt * TN + (c / TN) * (TN / 2) + jl;
         const int64_t jj = j < p.N ? j : p.N - 1;
-        return (c % TN >= HALF ? p.w1 : p.w0) + jj * p.K;
+        return (r >= 2 ? p.w1 : p.w0) + jj * p.K;
     } else {
         const int64_t r = nt * BN + c;
         const int64_t rr = r < p.N ? r : p.N - 1;
@@ -44,7 +51,8 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
 #pragma clang fp contract(off)
     constexpr int TM = BM / 2, TN = BN / 2, FI = TM / 16, FJ = TN / 16, FH = FI / 2;
     constexpr int SLOT = (BM + BN) * 128;      // A rows, then W rows, 128 B each
-    constexpr int IPW = (BM + BN) / 64;        // LDS-DMA instructions (8 rows each) per wave and k-tile
+    // LDS-DMA instructions (8 rows each) per wave and k-tile; where the waves don't share them evenly, the first MORE have one more
+    constexpr int BLOCKS = (BM + BN) / 8, IPW = (BLOCKS + 7) / 8, MORE = BLOCKS % 8;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -71,6 +79,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
     const uint16_t* src[IPW];
 #pragma unroll
     for (int i = 0; i < IPW; i++) {
+        if (MORE && i == IPW - 1 && wave >= MORE) break;   // uniform
         const int r = 8 * (8 * i + wave) + (lane >> 3);
         const int cs = (lane & 7) ^ g8_swz(r);
         if (r < BM) {   // uniform over the wave: BM is a multiple of 8
@@ -84,7 +93,10 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
     auto stage = [&](int kt, int slot) {
         unsigned char* dst = smem + slot * SLOT + wave * 1024;
 #pragma unroll
-        for (int i = 0; i < IPW; i++) glds16(src[i] + (int64_t)kt * mid::BK, dst + i * 8192);
+        for (int i = 0; i < IPW; i++) {
+            if (MORE && i == IPW - 1 && wave >= MORE) break;
+            glds16(src[i] + (int64_t)kt * mid::BK, dst + i * 8192);
+        }
     };
 
     f32x4 acc[FI][FJ];
@@ -97,7 +109,8 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
     int slot = 0, fill = SLOTS - 1;
     for (int t = 0; t < nk; t++) {
         // k-tile t has landed (the SLOTS - 2 younger ones may still fly), and every wave is done with the slot of t - 1
-        if (t + SLOTS - 1 <= nk) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(IPW * (SLOTS - 2)) : "memory");
+        if (t + SLOTS - 1 <= nk && (MORE == 0 || wave < MORE)) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(IPW * (SLOTS - 2)) : "memory");
+        else if (t + SLOTS - 1 <= nk) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((IPW - 1) * (SLOTS - 2)) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_barrier();
@@ -137,14 +150,14 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
     {
         f32x4* ex = reinterpret_cast<f32x4*>(smem);
         constexpr int FIT = SLOTS * SLOT / (8 * FH * 1024), JN = FIT < FJ ? FIT : FJ;   // fragment columns the LDS takes at once
-        static_assert(JN >= 1 && FJ % JN == 0, "exchange area");
+        static_assert(JN >= 1, "exchange area");
 #pragma unroll
         for (int j0 = 0; j0 < FJ; j0 += JN) {
             __syncthreads();
 #pragma unroll
             for (int i = 0; i < FH; i++)
 #pragma unroll
-                for (int j = j0; j < j0 + JN; j++) {
+                for (int j = j0; j < j0 + JN && j < FJ; j++) {
                     if (wk == 0) {
                         ex[((wave * FH + i) * JN + j - j0) * 64 + lane] = acc[FH + i][j];
                         res[i][j] = acc[i][j];
@@ -157,7 +170,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
 #pragma unroll
             for (int i = 0; i < FH; i++)
 #pragma unroll
-                for (int j = j0; j < j0 + JN; j++) res[i][j] = res[i][j] + ex[(((wave ^ 4) * FH + i) * JN + j - j0) * 64 + lane];
+                for (int j = j0; j < j0 + JN && j < FJ; j++) res[i][j] = res[i][j] + ex[(((wave ^ 4) * FH + i) * JN + j - j0) * 64 + lane];
         }
     }
 
@@ -213,20 +226,31 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
     const int64_t row0 = m0 + wm * TM + wk * (FH * 16) + fr;
     if constexpr (EPI == QIE_EPI_SWIGLU) {
 #pragma unroll
-        for (int jj = 0; jj < FJ / 2; jj++) {
-            const int64_t col = nt * TN + (TN / 2) * wn + 16 * jj + 4 * g;
+        for (int m = 0; m < (FJ + 1) / 2; m++) {
+            constexpr int PAIRS = FJ / 2;
+            const int n = m < PAIRS ? 4 : 2;   // outputs
+            const int64_t col = nt * TN + (TN / 2) * wn + 16 * m + n * g;
 #pragma unroll
             for (int i = 0; i < FH; i++) {
                 const int64_t row = row0 + i * 16;
                 if (row >= p.M) continue;
                 float h[4];
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const float gg = rbf(res[i][jj][r]);
-                    const float uu = rbf(res[i][jj + FJ / 2][r]);
+                for (int r = 0; r < n; r++) {
+                    const f32x4 v = res[i][2 * m + r / 2];
+                    const float gg = rbf(v[r & 1]);
+                    const float uu = rbf(v[2 + (r & 1)]);
                     h[r] = uu * rbf(gg * (1.0f / (1.0f + expf(-gg))));
                 }
-                store_quad(p.C + row * p.ldc + col, h, vec, p.N - col);
+                uint16_t* dst = p.C + row * p.ldc + col;
+                if (vec && col + n <= p.N) {
+                    if (n == 4) *reinterpret_cast<uint2*>(dst) = make_uint2(pack2(h[0], h[1]), pack2(h[2], h[3]));
+                    else *reinterpret_cast<uint32_t*>(dst) = pack2(h[0], h[1]);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < n; r++)
+                        if (col + r < p.N) dst[r] = f2bf(h[r]);
+                }
             }
         }
     } else {
@@ -267,7 +291,7 @@ int launch_mid_t(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, hi
     }
     const int tiles = pl.n_mt * pl.n_nt, whole = sk.splitk > 1 ? pl.whole : tiles;
     hipLaunchKernelGGL((gemm_mid_kernel<EPI, BM, BN, SLOTS>), dim3((unsigned)(whole + (tiles - whole) * sk.splitk)), dim3(512), shm,
-                       st, p, pl.n_mt, pl.n_nt, band_height(pl.n_mt, BM, BN, 32 * mid::TILES[pl.tile].per_cu), whole, sk);
+                       st, p, pl.n_mt, pl.n_nt, band_height(pl.n_mt, BM, BN, 32 * mid::shape(pl.tile).per_cu), whole, sk);
     QIE_LAUNCH_CHECK();
     return 0;
 }
@@ -282,7 +306,11 @@ int launch_mid(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, hipS
         case 4: return launch_mid_t<EPI, 192, 128, 4>(p, pl, sk, st);
         case 5: return launch_mid_t<EPI, 256, 128, 3>(p, pl, sk, st);
         case 6: return launch_mid_t<EPI, 320, 64, 3>(p, pl, sk, st);
-        default: return launch_mid_t<EPI, 320, 128, 2>(p, pl, sk, st);
+        case 7: return launch_mid_t<EPI, 320, 128, 2>(p, pl, sk, st);
+        case 8: return launch_mid_t<EPI, 128, 160, 4>(p, pl, sk, st);
+        case 9: return launch_mid_t<EPI, 192, 160, 3>(p, pl, sk, st);
+        case 10: return launch_mid_t<EPI, 256, 160, 3>(p, pl, sk, st);
+        default: return launch_mid_t<EPI, 320, 160, 2>(p, pl, sk, st);
     }
 }
 }  // namespace
@@ -293,12 +321,16 @@ int gemm_mid(const qie_linear_args* a, const GemmParams& q, float other_us, hipS
     const GemmParams& p = q;
     if (a->K % mid::BK != 0) return 0;   // (rows of x and weights are on the 16-byte grid of LDS-DMA: qie_linear)
     const int64_t cols = a->epilogue == QIE_EPI_SWIGLU ? 2 * a->N : a->N;
-    const mid::Plan pl = mid::plan(a->M, cols, a->K, device_cu_count());
-    if (pl.tile < 0 || pl.us >= 0.88f * other_us) return 0;   // 12 %: what the two fits are off by on long prompts
+    mid::Plan pl = mid::plan(a->M, cols, a->K, device_cu_count());
+    const mid::Plan wide = mid::plan_wide(a->M, cols, a->K, device_cu_count());
+    // (split plans of gate / up's many columns take 10 to 30 % longer than the fit says)
+    const bool to_wide = a->M > 64 && wide.us < (pl.splitk > 1 ? 1.1f : 1.f) * pl.us && wide.us < 0.97f * other_us;
+    if (to_wide) pl = wide;
+    if (pl.tile < 0 || (!to_wide && pl.us >= 0.88f * other_us)) return 0;   // 12 %: what the two fits are off by on long prompts
     G8Split sk{1, nullptr, nullptr};
     const int64_t cut = (int64_t)pl.n_mt * pl.n_nt - pl.whole;
     if (pl.splitk > 1 && cut > 0) {
-        const int64_t floats = cut * pl.splitk * mid::TILES[pl.tile].bm * mid::TILES[pl.tile].bn;
+        const int64_t floats = cut * pl.splitk * mid::shape(pl.tile).bm * mid::shape(pl.tile).bn;
         if (g8_workspace(st, (int)cdiv(floats, 65536), (int)cut, &sk) == 0) sk.splitk = pl.splitk;
     }
     *launched = true;
