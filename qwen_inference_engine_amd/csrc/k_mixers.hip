@@ -804,6 +804,7 @@ __global__ __launch_bounds__(256) void gqa_attn_mfma_kernel(GqaAttnMfmaP P) {
         return;
     }
     const int64_t unit = ((int64_t)blockIdx.x * (gridDim.y * 4) + tile) * S + z;
+    if (!valid) return;   // (the second pass reads the columns that exist)
     float* po = P.part_o + (unit * 16 + n) * vdim + 4 * g;
 #pragma unroll
     for (int dv = 0; dv < DV; dv++) *reinterpret_cast<float4*>(po + 16 * dv) = make_float4(acc[dv][0], acc[dv][1], acc[dv][2], acc[dv][3]);
@@ -813,54 +814,94 @@ __global__ __launch_bounds__(256) void gqa_attn_mfma_kernel(GqaAttnMfmaP P) {
     }
 }
 
-// Second pass of a split launch: one wave per (group, tile), the same lane layout as the first.
+// Second pass of a split launch: one wave per column (token and head), a lane per 64th value coordinate, so that a column's parts are
+// rows of 256 bytes and more, all on their way at once: two trips to memory (the group, then everything else).  With the first pass's
+// lane layout a decode step's columns kept four lanes of a wave busy and a part was a trip of its own: 10.4 us where this takes 4.7 (5 slots, 16 heads, Nukizen 2k).
+// At most 64 parts.
 template <int DV>
 __global__ __launch_bounds__(256) void gqa_attn_combine_kernel(GqaAttnMfmaP P, int tiles) {
     const GqaAttnP& a = P.a;
-    constexpr int vdim = 16 * DV;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+    constexpr int vdim = 16 * DV, VPL = (vdim + 63) / 64, ZB = VPL <= 2 ? 16 : 8;   // ZB: parts a trip
+    __shared__ float turn[4][vdim];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, n = blockIdx.z;
     const int4 grp = P.groups[blockIdx.x];
     const int n_tok = grp.y, pos0 = grp.w;
     const int hpt = P.pack ? heads_per_token(n_tok, a.heads, a.kv_heads) : 1;
-    const int tile = blockIdx.y * 4 + wave, h0 = tile * hpt;
-    if (h0 >= a.heads) return;
-    const int tI = n / hpt, hh = h0 + n % hpt;
-    if (tI >= n_tok) return;
+    const int tile = blockIdx.y * 4 + wave, h0 = tile * hpt, tI = n / hpt, hh = h0 + n % hpt;
+    if (h0 >= a.heads || tI >= n_tok) return;   // uniform over the wave
+    const int row = grp.x + tI;
     const int64_t u0 = ((int64_t)blockIdx.x * tiles + tile) * P.S;
-    const float* ml = P.part_ml + (u0 * 16 + n) * 2;          // part z at ml + 32 z
-    float M = -1e30f;
-    for (int z = 0; z < P.S; z++) M = fmaxf(M, ml[32 * z]);
-    float L = 0.f;
-    gf32x4_t acc[DV];
+    const float2* ml = reinterpret_cast<const float2*>(P.part_ml) + u0 * 16 + n;   // part z at ml + 16 z
+    const float* po = P.part_o + (u0 * 16 + n) * vdim;                             // ... at po + 16 vdim z
+    const float2 mine = lane < P.S ? ml[16 * lane] : make_float2(-1e30f, 0.f);
+    int v[VPL];
+    bool in[VPL];
 #pragma unroll
-    for (int dv = 0; dv < DV; dv++) acc[dv] = gf32x4_t{0.f, 0.f, 0.f, 0.f};
-    // several parts a turn (a turn is one trip to memory), every load of the turn issued before its first use; a
-    // part that saw no key of the column has l = 0 and zero sums
-    constexpr int PT = DV <= 8 ? 4 : 2;
-    for (int z0 = 0; z0 < P.S; z0 += PT) {
-        float w[PT];
-        float4 o[PT][DV];
-#pragma unroll
-        for (int k = 0; k < PT; k++) {
-            const int zk = min(z0 + k, P.S - 1);
-            const float l = ml[32 * zk + 1];
-            w[k] = (z0 + k >= P.S || l == 0.f) ? 0.f : __expf(ml[32 * zk] - M);
-            L += l * w[k];
-            const float* pk = P.part_o + ((u0 + zk) * 16 + n) * vdim + 4 * g;
-#pragma unroll
-            for (int dv = 0; dv < DV; dv++) o[k][dv] = *reinterpret_cast<const float4*>(pk + 16 * dv);
-        }
-#pragma unroll
-        for (int k = 0; k < PT; k++)
-#pragma unroll
-            for (int dv = 0; dv < DV; dv++) {
-                acc[dv][0] += o[k][dv].x * w[k];
-                acc[dv][1] += o[k][dv].y * w[k];
-                acc[dv][2] += o[k][dv].z * w[k];
-                acc[dv][3] += o[k][dv].w * w[k];
-            }
+    for (int k = 0; k < VPL; k++) {
+        in[k] = lane + 64 * k < vdim;
+        v[k] = in[k] ? lane + 64 * k : vdim - 1;
     }
-    gqa_store<DV>(a, acc, gqa_out_factor(a, L, M, grp.x + tI, hh), grp.x + tI, hh, pos0 + tI, g);
+    const bool gated = a.gate_col >= 0 && a.gate_elem;
+    float gf[VPL];
+    if (gated) {
+        const float* gp = a.proj + (int64_t)row * a.ld + a.gate_col + hh * vdim;
+#pragma unroll
+        for (int k = 0; k < VPL; k++) gf[k] = gp[v[k]];
+    }
+    float o[ZB][VPL];
+    auto load = [&](int z0) {
+#pragma unroll
+        for (int z = 0; z < ZB; z++) {
+            const int zz = min(z0 + z, P.S - 1);
+#pragma unroll
+            for (int k = 0; k < VPL; k++) o[z][k] = po[(int64_t)16 * vdim * zz + v[k]];
+        }
+    };
+    load(0);
+    float M = mine.x;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) M = fmaxf(M, __shfl_xor(M, d, 64));
+    const float w = mine.y == 0.f ? 0.f : __expf(mine.x - M);   // a part that saw no key of the column has l = 0 and zero sums
+    float L = mine.y * w;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) L += __shfl_xor(L, d, 64);
+    float acc[VPL];
+#pragma unroll
+    for (int k = 0; k < VPL; k++) acc[k] = 0.f;
+    for (int z0 = 0; z0 < P.S; z0 += ZB) {
+        if (z0 > 0) load(z0);
+#pragma unroll
+        for (int z = 0; z < ZB; z++) {
+            const float wz = z0 + z < P.S ? __shfl(w, z0 + z, 64) : 0.f;
+#pragma unroll
+            for (int k = 0; k < VPL; k++) acc[k] += o[z][k] * wz;
+        }
+    }
+    const float inv = gqa_out_factor(a, L, M, row, hh);
+    if (a.rot_values) {   // uniform; a wave's own LDS
+#pragma unroll
+        for (int k = 0; k < VPL; k++)
+            if (in[k]) turn[wave][v[k]] = acc[k] * inv;
+        __builtin_amdgcn_wave_barrier();
+    }
+    const int64_t o0 = (int64_t)row * a.ld_out + a.out_col + (int64_t)hh * vdim;
+#pragma unroll
+    for (int k = 0; k < VPL; k++) {
+        float y = acc[k] * inv;
+        if (a.rot_values) {   // turned back by the column's position: the angle negated
+            const int64_t c0 = (int64_t)(pos0 + tI) * (vdim / 2);
+            const bool pairs = a.rot_layout == 1, low = pairs ? v[k] % 2 == 0 : v[k] < vdim / 2;
+            const int pi = pairs ? v[k] / 2 : low ? v[k] : v[k] - vdim / 2;
+            const float other = turn[wave][pairs ? v[k] ^ 1 : low ? v[k] + vdim / 2 : v[k] - vdim / 2];
+            const float c = a.vrope_cos[c0 + pi], sn = a.vrope_sin[c0 + pi];
+            y = low ? y * c + other * sn : y * c - other * sn;
+        }
+        y *= a.out_scale;
+        if (gated) y *= 1.0f / (1.0f + __expf(-gf[k]));
+        if (!in[k]) continue;
+        if (a.out) a.out[o0 + v[k]] = y;
+        if (a.out_bf) a.out_bf[o0 + v[k]] = f2bf(y);
+    }
 }
 
 bool gqa_attention_mfma_fits(int dim, int vdim, int page_tokens) {
@@ -874,7 +915,7 @@ static void gqa_mfma_launch2(const GqaAttnMfmaP& p, dim3 grid, hipStream_t st) {
         hipLaunchKernelGGL((gqa_attn_mfma_kernel<DK, DV, false>), grid, dim3(256), 0, st, p);
     else
         hipLaunchKernelGGL((gqa_attn_mfma_kernel<DK, DV, true>), grid, dim3(256), 0, st, p);
-    if (p.S > 1) hipLaunchKernelGGL(gqa_attn_combine_kernel<DV>, dim3(grid.x, grid.y, 1), dim3(256), 0, st, p, (int)grid.y * 4);
+    if (p.S > 1) hipLaunchKernelGGL(gqa_attn_combine_kernel<DV>, dim3(grid.x, grid.y, 16), dim3(256), 0, st, p, (int)grid.y * 4);
 }
 template <int DK>
 static int gqa_mfma_launch(const GqaAttnMfmaP& p, dim3 grid, hipStream_t st) {
@@ -894,7 +935,7 @@ int gqa_attention_mfma(const GqaAttnMfmaP& p, hipStream_t st) {
     const GqaAttnP& a = p.a;
     QIE_REQUIRE(gqa_attention_mfma_fits(a.dim, a.vdim, a.cache.page_tokens) && a.v_transposed,
                 "gqa attention: sizes %d / %d, pages of %d tokens do not fit the matrix-core form", a.dim, a.vdim, a.cache.page_tokens);
-    QIE_REQUIRE(p.n_groups > 0 && p.S >= 1 && (p.S == 1 || (p.part_o && p.part_ml)), "gqa attention: bad launch");
+    QIE_REQUIRE(p.n_groups > 0 && p.S >= 1 && p.S <= 64 && (p.S == 1 || (p.part_o && p.part_ml)), "gqa attention: bad launch");
     QIE_REQUIRE(a.heads % a.kv_heads == 0, "gqa attention: %d query heads over %d key heads", a.heads, a.kv_heads);
     QIE_REQUIRE(a.mask_keep >= 0 && (a.mask_keep == 0 || a.mask == 1), "gqa attention: kept first keys go with the window mask");
     QIE_REQUIRE(p.pack == ((a.heads / a.kv_heads) % 4 != 0), "gqa attention: packing goes with head ratios that are no multiple of 4");
