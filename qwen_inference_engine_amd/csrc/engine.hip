@@ -131,6 +131,14 @@ __global__ void set_state_kernel(int m, int32_t pos_v, int32_t step_v, int32_t t
         for (int64_t i = threadIdx.x; i < H8; i += blockDim.x) x_res[(int64_t)m * H8 + i] = E[(int64_t)tok * H8 + i];
 }
 
+// ids of n_steps decode steps, [n_steps][B], to pinned host memory: sequence m's from history position at[m] on
+__global__ void fetch_ids_kernel(const int32_t* hist, int hist_stride, const int32_t* at, int B, int n_steps, int32_t* out) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n_steps * B) return;
+    const int m = i % B;
+    out[i] = hist[(int64_t)m * hist_stride + at[m] + i / B];
+}
+
 // positions of n_seqs equal-length prompts laid end to end: row i sits at i % len
 __global__ void iota_kernel(int32_t* p, int n, int len) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1133,6 +1141,8 @@ static int batch_create(qie_engine* e, int32_t batch, int32_t max_ctx, int32_t p
         A((void**)&b->logits_full, batch * (int64_t)s.vocab * 2);
         A((void**)&b->gather_tmp, batch * (int64_t)s.vocab * 2);
     }
+    if (!rc && hipHostMalloc((void**)&b->h_ids, (size_t)batch * (max_ctx + 1) * 4, hipHostMallocDefault) != hipSuccess)
+        rc = fail(-2, "qie_batch_create: no pinned memory for the ids");
     if (!rc) {
         hipMemsetAsync(b->dec_ws, 0, (size_t)dec_ws, e->stream);
         hipMemsetAsync(b->kc, 0, (size_t)n_runs * b->seq_stride * 2, e->stream);
@@ -1225,6 +1235,7 @@ void qie_batch_destroy(qie_batch* b) {
                   b->gather_tmp, b->pf_part, b->xn, b->pf_q8, b->pf_e8, b->pk_mem, b->d_layers, b->d_attp, b->pk_ts};
     for (void* p : ps)
         if (p) hipFree(p);
+    if (b->h_ids) hipHostFree(b->h_ids);
     delete b;
 }
 
@@ -1479,21 +1490,22 @@ int qie_decode(qie_batch* b, int32_t n_steps, const qie_sampling* smp, int32_t* 
     QIE_REQUIRE(!b || !b->lb, "%s: not for a batch of a layered engine (qie_batch_step drives it)", __func__);
     QIE_REQUIRE(b && n_steps >= 0, "qie_decode: bad arguments");
     QIE_TRY(prepare_steps(b, n_steps, "qie_decode"));
-    std::vector<int32_t> p0 = b->h_pos;
+    const bool want = out_ids && n_steps > 0;
+    if (want)
+        for (int m = 0; m < b->B; m++) b->h_ids[m] = b->h_pos[m] + 1;   // (no call leaves a launch behind that reads or writes h_ids)
     for (int i = 0; i < n_steps; i++) {
         QIE_TRY(launch_step(b, smp));
         for (int m = 0; m < b->B; m++) b->h_pos[m] += 1;
     }
+    if (want) {   // one launch behind the steps, and the wait that there is anyway (a copy and a wait a sequence took 15 us each)
+        hipLaunchKernelGGL(fetch_ids_kernel, dim3((unsigned)cdiv(n_steps * b->B, 256)), dim3(256), 0, b->e->stream, b->d_hist, b->max_ctx, b->h_ids,
+                           b->B, n_steps, b->h_ids + b->B);
+        QIE_LAUNCH_CHECK();
+    }
     QIE_HIP(hipStreamSynchronize(b->e->stream));
     QIE_TRY(comm_check(b->e, "qie_decode"));
     QIE_TRY(pk_check(b));
-    if (out_ids && n_steps > 0) {
-        std::vector<int32_t> row(b->max_ctx);
-        for (int m = 0; m < b->B; m++) {
-            QIE_HIP(d2h(b->e, row.data(), b->d_hist + (int64_t)m * b->max_ctx, (size_t)b->max_ctx * 4));
-            for (int i = 0; i < n_steps; i++) out_ids[(int64_t)i * b->B + m] = row[p0[m] + 1 + i];
-        }
-    }
+    if (want) memcpy(out_ids, b->h_ids + b->B, (size_t)n_steps * b->B * 4);
     return 0;
 }
 
@@ -1545,7 +1557,6 @@ int qie_batch_set_position(qie_batch* b, int32_t seq, int32_t pos, int32_t token
                        b->d_hist, b->max_ctx, (const uint4*)e->w.embed, (uint4*)b->x_res,
                        (int64_t)e->spec.hidden / 8, 1, rope_cur_args(b));
     QIE_LAUNCH_CHECK();
-    QIE_HIP(hipStreamSynchronize(e->stream));
     b->h_pos[seq] = pos;
     return 0;
 }
