@@ -838,6 +838,221 @@ static int dec8_launch(const Dec8Params& p, hipStream_t st) {
     return 0;
 }
 
+// ---------------------------------------------------------------------------
+// dec8s: long K (the down projection), plain rows: nobody else's sums.  The split-K form above shares a tile among ten workgroups that
+// meet through memory: a ticket, a drain and a second trip behind every launch, 3.6 TB/s.  Here a workgroup of 8 waves owns whole
+// 16-row tiles and every wave streams the 128-k chunks of its own share of K by LDS-DMA through a ring of its own, X's rows beside
+// the weights' (they come from L2; all of them do not fit LDS), with no barrier until the waves' partial tiles meet in LDS.
+// D = W Xᵀ: a lane ends with four neighbouring columns of one row.  XR: rows of X a chunk carries (X is as many bytes as the weights at
+// 8 rows, and they cost about 2 us).  us at 18,944 x 3,584, split-K form -> this one: 1 row 18.3 -> 13.5, 4 rows 19.2 -> 14.3, 8 rows
+// 19.7 -> 15.8 (weights read without the non-temporal hint: 14.7, -, 16.5); 16 rows 20.8 -> 22.7 and stay there.
+namespace d8s {
+constexpr int NW = 8;
+constexpr int CH = 128;         // k of a chunk
+constexpr int WCH = 16 * CH;    // bytes of its weights
+constexpr int slots(int xr) { return xr == 8 ? 4 : 5; }   // of a wave's ring
+constexpr int lds(int xr) { return NW * slots(xr) * (WCH + xr * CH * 2) + 2 * NW * 512; }
+}  // namespace d8s
+
+// 16 bytes a lane into LDS: lane l at lds + 16 l.  NT: lines that nobody reads again
+template <bool NT>
+__device__ __forceinline__ void d8_lds16(__amdgpu_buffer_rsrc_t rs, void* lds, uint32_t voff, uint32_t soff) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(lds), 16, voff, soff, 0, NT ? 2 : 0);
+#else
+    (void)rs; (void)lds; (void)voff; (void)soff;
+#endif
+}
+
+template <int EPI, bool T16, int XR>
+__global__ __launch_bounds__(512) void dec8s_kernel(Dec8Params p) {
+#pragma clang fp contract(off)
+    constexpr int R = d8s::slots(XR), SLOT = d8s::WCH + XR * d8s::CH * 2, IPC = 2 + XR / 4;
+    constexpr int RS = 32;   // quads of a partial tile: those of X rows 0 .. 7
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int fr = lane & 15, g = lane >> 4, rl = g * 8 + (fr & 7);
+    unsigned char* ring = smem + wave * (R * SLOT);
+    d8_f32x4* red = reinterpret_cast<d8_f32x4*>(smem + d8s::NW * R * SLOT);   // [2][NW][RS]
+    const int M = p.M, K = p.K, rows = p.seg_rows[0], T = p.n_tiles, G = gridDim.x;
+    const int chunks = K / d8s::CH;
+    const int c0 = wave * chunks / d8s::NW, cnt = (wave + 1) * chunks / d8s::NW - c0;   // this wave's share of K
+    const int mine = (int)blockIdx.x < T ? (T - 1 - (int)blockIdx.x) / G + 1 : 0;
+    const int items = mine * cnt;   // (tile, chunk) in order
+
+    const auto rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.w[0]), (short)0, (int)((int64_t)rows * (K + 4)), 0x00020000);
+    const auto none = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.w[0]), (short)0, 0, 0x00020000);
+    const auto rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.x), (short)0, (int)(((int64_t)(M - 1) * p.ldx + K) * 2), 0x00020000);
+    // the epilogue's operands: row scales, and old values or biases.  Those of the block's first tile are loaded ahead of its chunks.
+    d8_u32x4 sc = {0u, 0u, 0u, 0u};
+    uint32_t ep[4] = {0u, 0u, 0u, 0u};
+    auto load_epi = [&](int tile, bool on) {   // off: zeros
+        const int col = tile * 16 + 4 * g;
+        sc = __builtin_amdgcn_raw_buffer_load_b128(on ? rw : none, rows * K + col * 4, 0, 0);
+        if constexpr (EPI == QIE_EPI_RESIDUAL) {
+            const auto ry = __builtin_amdgcn_make_buffer_rsrc(p.y, (short)0, on ? (int)(((int64_t)(M - 1) * p.ldy + p.N) * 2) : 0, 0x00020000);
+#pragma unroll
+            for (int r = 0; r < 4; r++) ep[r] = __builtin_amdgcn_raw_buffer_load_b16(ry, (fr * (int)p.ldy + col + r) * 2, 0, 0);
+        } else if constexpr (EPI == QIE_EPI_STORE) {
+            const uint16_t* b = p.bias[0];
+            const auto rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(b ? b : p.x), (short)0, b && on ? rows * 2 : 0, 0x00020000);
+#pragma unroll
+            for (int r = 0; r < 4; r++) ep[r] = __builtin_amdgcn_raw_buffer_load_b16(rb, (col + r) * 2, 0, 0);
+        }
+    };
+    load_epi(blockIdx.x, wave == 0 && mine > 0);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // X: lane -> row 4 i + (lane >> 4) (rows past M: row M - 1 again), LDS piece lane & 15 of its 256 bytes, which holds the source's
+    // piece (lane & 15) ^ row: the fragment reads are free of bank conflicts
+    uint32_t xsrc[XR / 4];
+#pragma unroll
+    for (int i = 0; i < XR / 4; i++) {
+        const int m = 4 * i + (lane >> 4);
+        xsrc[i] = (uint32_t)((m < M ? m : M - 1) * (int)p.ldx * 2 + ((lane & 15) ^ m) * 16);
+    }
+    // weights: lane (fr, g) takes codes 16 g .. 16 g + 15 of a 64-k unit of row fr, in the plain layout (a gather of 64-byte
+    // pieces) as in the tiled one (the unit's 1 KB in order)
+    uint32_t wv = 0, ws = 0;
+    auto aim = [&](int tile) {
+        if constexpr (T16) {
+            wv = lane * 16;
+            ws = (uint32_t)(tile * 16 * K);
+        } else {
+            const int r = tile * 16 + fr;
+            wv = (uint32_t)((r < rows ? r : rows - 1) * K + 16 * g);
+            ws = 0;
+        }
+    };
+    int n_tile = blockIdx.x, n_c = 0, n_slot = 0;   // the next chunk to ask for
+    auto issue = [&](bool on) {                     // off: nothing is read
+        unsigned char* dst = ring + n_slot * SLOT;
+        const int c = c0 + n_c;
+#pragma unroll
+        for (int u = 0; u < 2; u++) d8_lds16<true>(on ? rw : none, dst + u * 1024, wv, ws + (uint32_t)(2 * c + u) * (T16 ? 1024 : 64));
+#pragma unroll
+        for (int i = 0; i < XR / 4; i++) d8_lds16<false>(on ? rx : none, dst + d8s::WCH + i * 1024, xsrc[i], (uint32_t)c * 256);
+        n_slot = n_slot + 1 == R ? 0 : n_slot + 1;
+        if (++n_c == cnt) {
+            n_c = 0;
+            n_tile += G;
+            aim(n_tile < T ? n_tile : T - 1);
+        }
+    };
+    aim(n_tile);
+#pragma unroll
+    for (int i = 0; i < R; i++) issue(i < items);
+    __builtin_amdgcn_sched_barrier(0);
+    // (the wait for them belongs here, not into the loop of counted waits)
+    asm volatile("" : "+v"(sc), "+v"(ep[0]), "+v"(ep[1]), "+v"(ep[2]), "+v"(ep[3]));
+
+    const int xm = fr & (XR - 1);
+    unsigned long long kbest = 0ull;
+    int done = 0, slot = 0;
+    for (int it = 0; it < mine; it++) {
+        const int tile = blockIdx.x + it * G;
+        d8_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        for (int c = 0; c < cnt; c++) {
+            // the oldest chunk has landed: R - 1 younger ones may fly (fewer at the end of the stream)
+            if (done + R <= items) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(IPC * (R - 1)) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            const unsigned char* buf = ring + slot * SLOT;
+            d8_u32x4 wf[2];
+            d8_bf16x8 xf[4];
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                wf[u] = *reinterpret_cast<const d8_u32x4*>(buf + u * 1024 + lane * 16);
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+                    xf[2 * u + h] = *reinterpret_cast<const d8_bf16x8*>(buf + d8s::WCH + xm * 256 + (((8 * u + 2 * g + h) ^ xm) * 16));
+            }
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const uint2 q0 = fp8x4_to_bf16x4(wf[u].x), q1 = fp8x4_to_bf16x4(wf[u].y);
+                const uint2 q2 = fp8x4_to_bf16x4(wf[u].z), q3 = fp8x4_to_bf16x4(wf[u].w);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(d8_bf16x8, d8_u32x4{q0.x, q0.y, q1.x, q1.y}), xf[2 * u], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(d8_bf16x8, d8_u32x4{q2.x, q2.y, q3.x, q3.y}), xf[2 * u + 1], acc, 0, 0, 0);
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the slot's reads are done
+            __builtin_amdgcn_sched_barrier(0);
+            if (done + R < items) issue(true);
+            done++;
+            slot = slot + 1 == R ? 0 : slot + 1;
+        }
+        if (fr < 8) red[((it & 1) * d8s::NW + wave) * RS + rl] = acc;
+        // one barrier a tile: a slot of `red` is written again two tiles on, behind the next tile's barrier, which the summing
+        // wave reaches only after its reads.  (No vmcnt wait: the ring's loads stay in flight.)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        if (wave != it % d8s::NW) continue;   // wave-uniform
+        d8_f32x4 v = red[(it & 1) * d8s::NW * RS + rl];
+#pragma unroll
+        for (int w = 1; w < d8s::NW; w++) v = v + red[((it & 1) * d8s::NW + w) * RS + rl];
+        if (it > 0) load_epi(tile, true);
+        if (fr < M) {
+            const int col = tile * 16 + 4 * g;
+            const uint32_t s4[4] = {sc.x, sc.y, sc.z, sc.w};
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                if (col + r >= p.N) continue;
+                const float c = v[r] * __uint_as_float(s4[r]);
+                const int64_t at = (int64_t)fr * p.ldy + col + r;
+                if constexpr (EPI == QIE_EPI_F32) {
+                    reinterpret_cast<float*>(p.y)[at] = c;
+                } else if constexpr (EPI == QIE_EPI_RESIDUAL) {
+                    p.y[at] = f2bf(bf2f((uint16_t)ep[r]) + rbf(c));
+                } else {
+                    const uint16_t o = f2bf(c + bf2f((uint16_t)ep[r]));
+                    p.y[at] = o;
+                    if (p.keys) {
+                        const unsigned long long kk = sel_key(bf2f(o), (uint32_t)(col + r + p.key_col0));
+                        kbest = kk > kbest ? kk : kbest;
+                    }
+                }
+            }
+        }
+    }
+    if constexpr (EPI == QIE_EPI_STORE) {
+        if (p.keys && fr < M && kbest) atomicMax(p.keys + fr, kbest);
+    }
+}
+
+template <int EPI, bool T16, int XR>
+static int dec8s_launch(const Dec8Params& p, hipStream_t st) {
+    const void* fn = (const void*)dec8s_kernel<EPI, T16, XR>;
+    static bool raised = false;
+    if (!raised) {
+        QIE_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, d8s::lds(XR)));
+        raised = true;
+    }
+    const int grid = std::max(1, std::min(p.n_tiles, (int)device_cu_count()));
+    hipLaunchKernelGGL((dec8s_kernel<EPI, T16, XR>), dim3((unsigned)grid), dim3(512), d8s::lds(XR), st, p);
+    QIE_LAUNCH_CHECK();
+    return 0;
+}
+template <int EPI, bool T16>
+static int dec8s_rows(const Dec8Params& p, hipStream_t st) {
+    return p.M <= 4 ? dec8s_launch<EPI, T16, 4>(p, st) : dec8s_launch<EPI, T16, 8>(p, st);
+}
+template <bool T16>
+static int dec8s(const Dec8Params& p, int epi, hipStream_t st) {
+    switch (epi) {
+        case QIE_EPI_RESIDUAL: return dec8s_rows<QIE_EPI_RESIDUAL, T16>(p, st);
+        case QIE_EPI_F32: return dec8s_rows<QIE_EPI_F32, T16>(p, st);
+        default: return dec8s_rows<QIE_EPI_STORE, T16>(p, st);
+    }
+}
+// Where the tiles keep most CUs busy (below that the split-K form spreads K over the others), up to 8 rows.
+static bool dec8s_applies(const qie_linear_args* a) {
+    const int64_t tiles = (a->N + 15) / 16;
+    return a->M <= 8 && a->K % d8s::CH == 0 && a->K / d8s::CH >= d8s::NW && tiles * 4 >= device_cu_count() * 3 &&
+           a->M * a->ldx < 1 << 30 && a->M * a->ldy < 1 << 29;   // 32-bit offsets
+}
+
 // Split-K workspace (slabs + tickets), one per stream — streams of one device may run
 // projections at the same time (tensor-parallel ranks on one GPU in the tests) — reserved by
 // qie_batch_create (dec8_reserve) so that the captured decode step finds it; tickets are
@@ -1019,6 +1234,7 @@ int dec8_linear(const qie_linear_args* a, hipStream_t st, bool* done) {
     int ku = 0, ks = 0;
     if (!dec8_shape(a->K, &ku, &ks)) {
         p.parts = dec8_split_parts(a, &ku);
+        if (dec8s_applies(a)) return t16 ? dec8s<true>(p, a->epilogue, st) : dec8s<false>(p, a->epilogue, st);
         if (!dec8_workspace(st, &p)) {
             *done = false;
             return 0;

@@ -1,0 +1,63 @@
+"""fp8 projections of long plain rows, up to 8 rows of X (k_decode_fp8.hip dec8s_kernel): uneven shares of K, a block's second tile, a ragged
+last tile, either layout of the weights, every epilogue, either number of X rows that a chunk carries."""
+import numpy as np
+import pytest
+
+import gpu_util as G
+from qwen_inference_engine_amd import _lib
+from test_gpu_fp8 import _fp8_dev, _tiled
+from test_gpu_ops import _abs_scale, _linear, rand_bf16
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("tiled", [False, True])
+@pytest.mark.parametrize("M,K,N", [(1, 2176, 3072), (3, 2176, 4112), (4, 3712, 3077), (5, 2176, 4112), (8, 2176, 8200), (8, 18944, 3584)])
+def test_long_rows(oracle, qlib, M, K, N, tiled):
+    if tiled:
+        N -= N % 16   # (the tiled layout has whole tiles)
+    elif M == 1:
+        pytest.skip("one row of plain weights is the row GEMV's")
+    x = rand_bf16(oracle, (M, K), seed=M + K)
+    d, dq = _fp8_dev(qlib, rand_bf16(oracle, (N, K), 0.05, seed=N))
+    w = [(_tiled(qlib, d, N, K) if tiled else d, N)]
+    flags = _lib.QIE_LINEAR_FP8 | (_lib.QIE_LINEAR_FP8_T16 if tiled else 0)
+    ldy, scale = N + 7, _abs_scale(oracle, x, dq)
+    exact = oracle.bf16_to_f32(x).astype(np.float64) @ oracle.bf16_to_f32(dq).astype(np.float64).T
+
+    def run(epi, y0, **kw):
+        y = G.dev(y0.copy())
+        _linear(qlib, G.dev(x), w, kw.pop("biases", []), M, K, N, y, epi, ldy=ldy, flags=flags, **kw)
+        return y
+
+    # fp32: each of at most 2,432 products of a chain and the 8 waves' sums rounds once, sqrt of that many on the average; 1e-5 is the
+    # repository's bound for such sums
+    y = G.host(run(_lib.QIE_EPI_F32, np.full((M, ldy), 3.0, np.float32)))
+    assert (np.abs(y[:, :N] - exact) <= 1e-5 * scale).all() and (y[:, N:] == 3.0).all()
+    res = rand_bf16(oracle, (M, ldy), seed=5)
+    y = G.host_bf16(run(_lib.QIE_EPI_RESIDUAL, res))
+    want = oracle.f32_to_bf16((oracle.bf16_to_f32(res[:, :N]) + oracle.bf16_to_f32(oracle.matmul(x, dq))).astype(np.float32))
+    # (a last bit of the product, and of the sum it goes into)
+    ulp = 2.0 ** -7 * (np.abs(exact) + np.abs(oracle.bf16_to_f32(want).astype(np.float64)))
+    diff = np.abs(oracle.bf16_to_f32(y[:, :N]).astype(np.float64) - oracle.bf16_to_f32(want))
+    assert (diff <= np.maximum(ulp, 1e-5 * scale)).all() and np.array_equal(y[:, N:], res[:, N:])
+    b = rand_bf16(oracle, (N,), 0.1, seed=9)
+    keys = G.dev(np.zeros(M, np.uint64))
+    y = G.host_bf16(run(_lib.QIE_EPI_STORE, res, biases=[G.dev(b)], keys=keys))
+    G.assert_sum_close(y[:, :N], oracle.matmul(x, dq, b), scale, what=f"M={M} K={K} N={N}")
+    ids = G.zeros((M,), np.int32)
+    G.check(qlib.qie_keys_to_ids(G.p(keys), M, G.p(ids), None))
+    for m in range(M):
+        assert G.host(ids)[m] == oracle.argmax(np.ascontiguousarray(y[m, :N]))
+
+
+def test_a_row_does_not_depend_on_its_neighbours(oracle, qlib):
+    K, N = 2176, 3072
+    x = rand_bf16(oracle, (8, K), seed=3)
+    w = _tiled(qlib, _fp8_dev(qlib, rand_bf16(oracle, (N, K), 0.05, seed=4))[0], N, K)
+    rows = []
+    for M in (1, 4, 8):
+        y = G.zeros((M, N), np.float32)
+        _linear(qlib, G.dev(x[:M].copy()), [(w, N)], [], M, K, N, y, _lib.QIE_EPI_F32, flags=_lib.QIE_LINEAR_FP8 | _lib.QIE_LINEAR_FP8_T16)
+        rows.append(G.host(y))
+    assert np.array_equal(rows[0], rows[2][:1]) and np.array_equal(rows[1], rows[2][:4])
