@@ -26,6 +26,8 @@ int gemv(const qie_linear_args* a, hipStream_t st);
 int gemv_rope(const qie_linear_args* a, const int32_t* pos, const float* cs, const float* sn, int hd, int64_t rows,
               hipStream_t st);
 int gemm(const qie_linear_args* a, hipStream_t st);
+int gemm_qkv(const qie_linear_args* a, const qie_kv_cache* cache, int32_t layer, int32_t len, const float* turns, uint16_t* q,
+             hipStream_t st, bool* done);
 bool dec8_applies(const qie_linear_args* a);
 bool dec_bf16_applies(const qie_linear_args* a);
 int dec8_reserve(hipStream_t st);
@@ -232,6 +234,16 @@ static int build_rope(qie_engine* e) {
     QIE_TRY(dmalloc((void**)&e->rope_sin, s.size() * 4));
     QIE_HIP(hipMemcpyAsync(e->rope_cos, c.data(), c.size() * 4, hipMemcpyHostToDevice, e->stream));
     QIE_HIP(hipMemcpyAsync(e->rope_sin, s.data(), s.size() * 4, hipMemcpyHostToDevice, e->stream));
+    std::vector<float> turns;   // both, pair by pair: a lane of the QKV product's epilogue reads two pairs at once
+    if (e->spec.numerics == QIE_NUMERICS_REF) {
+        turns.resize(2 * c.size());
+        for (size_t i = 0; i < c.size(); i++) {
+            turns[2 * i] = c[i];
+            turns[2 * i + 1] = s[i];
+        }
+        QIE_TRY(dmalloc((void**)&e->rope_turns, turns.size() * 4));
+        QIE_HIP(hipMemcpyAsync(e->rope_turns, turns.data(), turns.size() * 4, hipMemcpyHostToDevice, e->stream));
+    }
     QIE_HIP(hipStreamSynchronize(e->stream));   // the host tables go out of scope
     e->rope_rows = rows;
     return 0;
@@ -1071,6 +1083,7 @@ void qie_engine_destroy(qie_engine* e) {
     layered_engine_destroy(e);
     if (e->arena) hipFree(e->arena);
     if (e->fp8_arena) hipFree(e->fp8_arena);
+    if (e->rope_turns) hipFree(e->rope_turns);
     if (e->rope_cos) hipFree(e->rope_cos);
     if (e->rope_sin) hipFree(e->rope_sin);
     if (e->index) qie_index_destroy(e->index);
@@ -1239,6 +1252,8 @@ void qie_batch_destroy(qie_batch* b) {
     delete b;
 }
 
+static int linear_check(const qie_linear_args* a);
+
 // Prefill of n_seqs prompts of len ids each into slots seq0 .. seq0+n_seqs-1 (ids laid end
 // to end): every GEMM runs once over all n_seqs * len rows, attention and the KV append see
 // the prompts as sequences of rows_per_seq = len, and the head samples the n_seqs last rows
@@ -1339,9 +1354,16 @@ static int prefill_rows(qie_batch* b, int seq0, int n_seqs, const int32_t* ids, 
         a.bias[0] = L.bq; a.bias[1] = L.bk; a.bias[2] = L.bv;
         a.seg_rows[0] = QD; a.seg_rows[1] = KD; a.seg_rows[2] = KD;
         a.M = n; a.K = H; a.N = QKVD; a.y = b->pf_qkv; a.ldy = QKVD; a.epilogue = QIE_EPI_STORE;
-        QIE_TRY(qie_linear(&a, st));
-        QIE_TRY(qie_qkv_post(b->pf_qkv, n, b->pf_pos, len, L.q_norm, L.k_norm, e->rope_cos, e->rope_sin, sh.nq,
-                             &cache, l, s.rms_eps, s.numerics, b->pf_q, st));
+        bool post = false;   // rotation and cache rows by the product's epilogue
+        if (n > 16 && !L.q_norm && !L.k_norm && s.numerics == QIE_NUMERICS_REF) {
+            QIE_TRY(linear_check(&a));
+            QIE_TRY(gemm_qkv(&a, &cache, l, len, e->rope_turns, b->pf_q, st, &post));
+        } else {
+            QIE_TRY(qie_linear(&a, st));
+        }
+        if (!post)
+            QIE_TRY(qie_qkv_post(b->pf_qkv, n, b->pf_pos, len, L.q_norm, L.k_norm, e->rope_cos, e->rope_sin, sh.nq,
+                                 &cache, l, s.rms_eps, s.numerics, b->pf_q, st));
         QIE_TRY(qie_attention(b->pf_q, n, b->pf_pos, len, &cache, l, sh.nq, b->pf_att, b->pf_attn_ws, st));
         a = pf_base();
         a.x = b->pf_att; a.ldx = QD; a.w[0] = L.wo; a.seg_rows[0] = H;
@@ -1855,7 +1877,7 @@ int qie_batch_debug_step(qie_batch* b, const qie_sampling* smp, int32_t* next_id
     return sync_ids(b, next_ids);
 }
 
-int qie_linear(const qie_linear_args* a, void* stream) {
+static int linear_check(const qie_linear_args* a) {
     QIE_REQUIRE(a && a->x && a->y && a->w[0] && a->M > 0 && a->K > 0 && a->N > 0, "qie_linear: bad arguments");
     QIE_REQUIRE(a->K % 8 == 0 && a->ldx >= a->K && a->ldx % 8 == 0, "qie_linear: K and ldx must be multiples of 8");
     QIE_REQUIRE(((uintptr_t)a->x % 16) == 0, "qie_linear: x must be 16-byte aligned");
@@ -1874,9 +1896,7 @@ int qie_linear(const qie_linear_args* a, void* stream) {
     QIE_REQUIRE(a->epilogue != QIE_EPI_F32 || (a->bias[0] == nullptr && a->bias[1] == nullptr && a->bias[2] == nullptr),
                 "qie_linear: F32 (partial-sum) epilogue takes no bias");
     QIE_REQUIRE(a->argmax_keys == nullptr || a->epilogue == QIE_EPI_STORE, "qie_linear: arg-max needs STORE");
-    const bool act_fp8 = (a->flags & QIE_LINEAR_ACT_FP8) != 0;
-    hipStream_t st = (hipStream_t)stream;
-    if (act_fp8) return gemm(a, st);   // fp8 activations: the block-scaled MFMA GEMM at every M
+    if (a->flags & QIE_LINEAR_ACT_FP8) return 0;
     QIE_REQUIRE(!(a->flags & QIE_LINEAR_FP8_T16) ||
                     ((a->flags & QIE_LINEAR_FP8) && a->M >= 1 && a->M <= 16 && a->K % 64 == 0 &&
                      (a->epilogue == QIE_EPI_SWIGLU ? a->N % 16 == 0
@@ -1884,6 +1904,13 @@ int qie_linear(const qie_linear_args* a, void* stream) {
                                                           a->seg_rows[2] % 16 == 0)),
                 "qie_linear: 16-row tiled fp8 weights are read by the batched-decode kernels only (M <= 16, K %% 64 == 0, "
                 "segments of whole 16-row tiles) and, with fp8 activations, the block-scaled GEMM");
+    return 0;
+}
+
+int qie_linear(const qie_linear_args* a, void* stream) {
+    QIE_TRY(linear_check(a));
+    hipStream_t st = (hipStream_t)stream;
+    if (a->flags & QIE_LINEAR_ACT_FP8) return gemm(a, st);   // fp8 activations: the block-scaled MFMA GEMM at every M
     if (a->M <= 16) return gemv(a, st);   // GEMV (M = 1..8) or the skinny MFMA kernel (2..16)
     return gemm(a, st);
 }

@@ -54,6 +54,7 @@ struct qie_engine {
     void* fp8_arena = nullptr;
     float* rope_cos = nullptr;
     float* rope_sin = nullptr;
+    float* rope_turns = nullptr;       // [position][head_dim / 2][cos, sin]; interleaved pairs only
     int rope_rows = 0;
     qie::LayeredModel* lm = nullptr;   // layered engines (engine_layered.hip): architecture + weights
 };

@@ -11,6 +11,19 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
+// What follows a QKV projection of prompts laid end to end, each from position 0 on, without q / k norms and with rotary pairs
+// (2 i, 2 i + 1): q and k turned, q to its rows, k and v to the cache (qkv_post_kernel's results)
+struct QkvTail {
+    uint16_t* q;             // [M][qd]; null: no such tail
+    uint16_t *k, *v;         // the layer's first run
+    const float* turns;      // [position][hd / 2][cos, sin]
+    int len;                 // rows of a prompt
+    int qd, kd;              // columns of q, of k and of v
+    int hd_log2;
+    KvMap km;
+};
+constexpr int kEpiQkv = 4;   // the epilogue that does this: k_gemm.hip's 256x256 kernel and k_gemm_mid.hip's have it
+
 struct GemmParams {
     const uint16_t* A;
     int64_t lda;
@@ -26,6 +39,7 @@ struct GemmParams {
     uint16_t* C;
     int64_t ldc;
     int vec = 0;         // rows of C take 4-element vector stores
+    QkvTail qkv{};
 };
 
 __device__ __forceinline__ void glds16(const void* src, void* lds) {
@@ -78,6 +92,68 @@ __device__ __forceinline__ void quad_bias(const GemmParams& p, int64_t col, floa
         const int64_t c = col + r < p.N ? col + r : p.N - 1;
         const uint16_t* b = c < p.n0 ? p.b0 : (c < p.n01 ? p.b1 : p.b2);
         if (b) bias[r] = bf2f(b[c < p.n0 ? c : (c < p.n01 ? c - p.n0 : c - p.n01)]);
+    }
+}
+
+// What the epilogue kEpiQkv loads for a quad of columns at `at`: biases; (cos, sin) of its two pairs in each of the lane's rows
+template <int NI>
+struct QkvOps {
+    float bias[4];
+    float4 turn[NI];
+};
+template <int NI>
+__device__ __forceinline__ void qkv_load(const GemmParams& p, int64_t row0, int64_t col, QkvOps<NI>& o) {
+    const QkvTail& t = p.qkv;
+    const int hd = 1 << t.hd_log2, at = (int)(col < p.N ? col : p.N - 4);
+    o.bias[0] = o.bias[1] = o.bias[2] = o.bias[3] = 0.f;
+    quad_bias(p, at, o.bias);
+#pragma unroll
+    for (int i = 0; i < NI; i++) {   // (no bounds tests: every row's clamped position has them)
+        const uint32_t row = (uint32_t)(row0 + 16 * i < p.M ? row0 + 16 * i : p.M - 1);
+        o.turn[i] = *reinterpret_cast<const float4*>(t.turns + (int64_t)(row % (uint32_t)t.len) * hd + (at & (hd - 1)));
+    }
+}
+// The epilogue of rows row0 + 16 i, columns col0 + 16 j .. + 3 (whole quads: heads are multiples of 8).  `early`: operands loaded
+// ahead, where they are few enough to hold.  A kernel of its own for this (10 us at 2,048 rows, 4 at 113) read the projection back and
+// cost a launch.  A layer with this is shorter by: Qwen2-0.5B at 113 rows 2.6 us, Qwen2-7B at 301 rows 5.0, at 2,048 rows 6.3 (there the
+// epilogue takes some of it back: with the two tables apart, twice the loads, nothing was left), at 8,192 rows nothing.
+template <int NI, int NJ, bool EARLY>
+__device__ __forceinline__ void qkv_tail(const GemmParams& p, int64_t row0, int64_t col0, const f32x4 (&acc)[NI][NJ],
+                                         const QkvOps<NI> (&early)[EARLY ? NJ : 1]) {
+#pragma clang fp contract(off)
+    const QkvTail& t = p.qkv;
+    const int hd = 1 << t.hd_log2, turned = t.qd + t.kd;
+    int64_t kv[NI];   // where the row's token lies in a run
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+        const uint32_t row = (uint32_t)(row0 + 16 * i < p.M ? row0 + 16 * i : p.M - 1), seq = row / (uint32_t)t.len;
+        const int pos = (int)(row - seq * (uint32_t)t.len);
+        kv[i] = t.km.table ? kv_tok<true>(t.km, seq, pos, hd) : kv_tok<false>(t.km, seq, pos, hd);
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        const int64_t col = col0 + 16 * j;
+        const int at = (int)(col < p.N ? col : p.N - 4);
+        QkvOps<NI> late;
+        if constexpr (!EARLY) qkv_load(p, row0, col, late);
+        const QkvOps<NI>& o = EARLY ? early[EARLY ? j : 0] : late;
+        const int in_kv = at < t.qd ? 0 : at < turned ? at - t.qd : at - turned;
+        uint16_t* run = (at < turned ? t.k : t.v) + kv_run_off(t.km, in_kv >> t.hd_log2, hd) + (in_kv & (hd - 1));
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            const int64_t row = row0 + 16 * i;
+            const float4 w = o.turn[i];
+            float x[4], y[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) x[r] = rbf(acc[i][j][r] + o.bias[r]);
+            y[0] = x[0] * w.x - x[1] * w.y;
+            y[1] = x[1] * w.x + x[0] * w.y;
+            y[2] = x[2] * w.z - x[3] * w.w;
+            y[3] = x[3] * w.z + x[2] * w.w;
+            uint2 out = make_uint2(pack2(y[0], y[1]), pack2(y[2], y[3]));
+            if (at >= turned) out = make_uint2(pack2(x[0], x[1]), pack2(x[2], x[3]));
+            if (row < p.M && col < p.N) *reinterpret_cast<uint2*>(at < t.qd ? t.q + row * t.qd + at : run + kv[i]) = out;
+        }
     }
 }
 

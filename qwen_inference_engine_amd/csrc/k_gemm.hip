@@ -639,6 +639,9 @@ __global__ __launch_bounds__(512) void gemm8_kernel(GemmParams p, int n_mt, int 
                 store_quad(p.C + row * p.ldc + col, h, vec, p.N - col);
             }
         }
+    } else if constexpr (EPI == kEpiQkv) {
+        const QkvOps<8> none[1] = {};
+        qkv_tail<8, 4, false>(p, row0, nt * 256 + wn * 64 + 4 * g, acc, none);
     } else {
         uint2 before[8][4];
         if constexpr (EPI == QIE_EPI_RESIDUAL) {   // all on their way at once: loads between the stores would each wait for memory
@@ -971,6 +974,7 @@ static int launch_gemm8_t(const GemmParams& p, int n_mt, int n_tiles, const G8Sp
     return 0;
 }
 static int launch_gemm8(int epi, const GemmParams& p, int n_mt, int n_tiles, const G8Split& sk, hipStream_t st) {
+    if (p.qkv.q) return launch_gemm8_t<kEpiQkv>(p, n_mt, n_tiles, sk, st);
     if (epi == QIE_EPI_SWIGLU) return launch_gemm8_t<QIE_EPI_SWIGLU>(p, n_mt, n_tiles, sk, st);
     if (epi == QIE_EPI_RESIDUAL) return launch_gemm8_t<QIE_EPI_RESIDUAL>(p, n_mt, n_tiles, sk, st);
     if (epi == QIE_EPI_F32) return launch_gemm8_t<QIE_EPI_F32>(p, n_mt, n_tiles, sk, st);
@@ -1534,7 +1538,8 @@ static int gemm_mx(const qie_linear_args* a, hipStream_t st) {
                : launch_gemm8mx<false>(a->epilogue, p, (int)n_mt, (int)tiles, sk, st);
 }
 
-int gemm(const qie_linear_args* a, hipStream_t st) {
+// tail: to follow the product where the kernel that takes it can (*done)
+static int gemm_with(const qie_linear_args* a, const QkvTail* tail, bool* done, hipStream_t st) {
     if (a->flags & QIE_LINEAR_ACT_FP8) return gemm_mx(a, st);
     QIE_REQUIRE(a->norm_w == nullptr, "qie_linear: fused RMSNorm is GEMV-only (M <= 8)");
     QIE_REQUIRE(a->argmax_keys == nullptr, "qie_linear: fused arg-max is GEMV-only (M <= 8)");
@@ -1581,7 +1586,9 @@ int gemm(const qie_linear_args* a, hipStream_t st) {
         // (Qwen2-7B gate/up, us: 301 rows 161 with the 256x256 kernel, 97 with k_gemm_mid.hip; 700 rows 183 against 229)
         if (dev_env("QIE_MID", 1) && force < 0 && !(a->flags & QIE_LINEAR_STREAMK)) {
             bool launched = false;
+            if (tail) p.qkv = *tail;
             const int rc = gemm_mid(a, p, g8ok && a->M >= big::BM ? g8_us(t256, cus, (int)(a->K / g8::BK)) : 1e30f, st, &launched);
+            if (done) *done = launched && tail;
             if (rc || launched) return rc;
         }
         const int g8mode = dev_env("QIE_GEMM8", 2);   // 2 (default): + split-K below; 1: full-chip grids only; 0: off
@@ -1593,6 +1600,7 @@ int gemm(const qie_linear_args* a, hipStream_t st) {
         }
         if (g8ok && g8mode != 0 && force != 2 && (force == 1 || (force < 0 && a->M >= big::BM && t256 >= cus))) {
             G8Split sk{1, nullptr, nullptr};
+            if (done) *done = p.qkv.q != nullptr;
             return launch_gemm8(a->epilogue, p, (int)n_mt, (int)t256, sk, st);
         }
         if (g8ok && g8mode == 2 && force < 0 && a->M >= big::BM && t256 < cus) {
@@ -1600,8 +1608,10 @@ int gemm(const qie_linear_args* a, hipStream_t st) {
             G8Split sk{1, nullptr, nullptr};
             // unsplit, 256x256 tiles must still cover half the chip: QKV at 144 tiles 101.7 ->
             // 87.8 us, but O at 112 tiles 78 -> 103 us (its 256x128 kernel fills 224 CUs)
-            if ((s == 1 && 2 * t256 >= cus) || (s > 1 && g8_workspace(st, (int)t256 * s, (int)t256, &sk) == 0 && (sk.splitk = s) > 1))
+            if ((s == 1 && 2 * t256 >= cus) || (s > 1 && g8_workspace(st, (int)t256 * s, (int)t256, &sk) == 0 && (sk.splitk = s) > 1)) {
+                if (done) *done = p.qkv.q != nullptr;
                 return launch_gemm8(a->epilogue, p, (int)n_mt, (int)t256, sk, st);
+            }
         }
         if (force == 1 || (force < 0 && a->M >= big::BM && t256 >= cus))
             return launch_gemm_big<256>(a->epilogue, p, (int)n_mt, (int)t256, st);
@@ -1614,6 +1624,30 @@ int gemm(const qie_linear_args* a, hipStream_t st) {
     }
     if (a->flags & QIE_LINEAR_FP8) return launch_gemm<1>(a->epilogue, gm, p, shm, st);
     return launch_gemm<0>(a->epilogue, gm, p, shm, st);
+}
+
+int gemm(const qie_linear_args* a, hipStream_t st) { return gemm_with(a, nullptr, nullptr, st); }
+
+// The QKV projection `a` (STORE) of M > 16 rows and, where its kernel has the epilogue, all that follows it up to the attention: *done;
+// else the product alone, in a->y.  cache: of the prompts' first slot.
+int gemm_qkv(const qie_linear_args* a, const qie_kv_cache* cache, int32_t layer, int32_t len, const float* turns, uint16_t* q,
+             hipStream_t st, bool* done) {
+    *done = false;
+    const int64_t hd = cache->head_dim;
+    QkvTail t{};
+    QIE_TRY(kv_map_make(cache, &t.km, "qie_prefill"));
+    t.q = q;
+    t.k = (uint16_t*)cache->k + kv_run_off(t.km, (int64_t)layer * cache->n_kv_heads, (int)hd);
+    t.v = (uint16_t*)cache->v + kv_run_off(t.km, (int64_t)layer * cache->n_kv_heads, (int)hd);
+    t.turns = turns;
+    t.len = len;
+    t.qd = (int)a->seg_rows[0];
+    t.kd = (int)a->seg_rows[1];
+    // quads of columns in one head, 8-byte stores
+    const bool fits = hd >= 8 && (hd & (hd - 1)) == 0 && t.km.stride % 4 == 0 && ((uintptr_t)q | (uintptr_t)cache->k | (uintptr_t)cache->v) % 8 == 0 &&
+                      (uintptr_t)turns % 16 == 0 && a->M < (int64_t)1 << 31 && t.qd % hd == 0 && t.kd % hd == 0;
+    while (fits && 1 << t.hd_log2 < hd) t.hd_log2++;
+    return gemm_with(a, fits ? &t : nullptr, done, st);
 }
 
 }  // namespace qie

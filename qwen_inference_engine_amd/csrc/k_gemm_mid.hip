@@ -90,6 +90,14 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
             src[i] = mid_wrow<EPI, BN>(p, nt, r - BM) + (int64_t)kb * mid::BK + cs * 8;
         }
     }
+    // kEpiQkv of small tiles: its operands are on their way before the first k-tile
+    constexpr bool EARLY = EPI == kEpiQkv && FH * FJ <= 8;
+    [[maybe_unused]] QkvOps<FH> ops[EARLY ? FJ : 1];
+    if constexpr (EARLY) {
+#pragma unroll
+        for (int j = 0; j < FJ; j++) qkv_load(p, m0 + wm * TM + wk * (FH * 16) + fr, nt * BN + wn * TN + 16 * j + 4 * g, ops[j]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
     auto stage = [&](int kt, int slot) {
         unsigned char* dst = smem + slot * SLOT + wave * 1024;
 #pragma unroll
@@ -253,6 +261,8 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
                 }
             }
         }
+    } else if constexpr (EPI == kEpiQkv) {
+        qkv_tail<FH, FJ, EARLY>(p, row0, nt * BN + wn * TN + 4 * g, res, ops);
     } else {
 #pragma unroll
         for (int j = 0; j < FJ; j++) {
@@ -334,6 +344,7 @@ int gemm_mid(const qie_linear_args* a, const GemmParams& q, float other_us, hipS
         if (g8_workspace(st, (int)cdiv(floats, 65536), (int)cut, &sk) == 0) sk.splitk = pl.splitk;
     }
     *launched = true;
+    if (p.qkv.q) return launch_mid<kEpiQkv>(p, pl, sk, st);
     switch (a->epilogue) {
         case QIE_EPI_SWIGLU: return launch_mid<QIE_EPI_SWIGLU>(p, pl, sk, st);
         case QIE_EPI_RESIDUAL: return launch_mid<QIE_EPI_RESIDUAL>(p, pl, sk, st);

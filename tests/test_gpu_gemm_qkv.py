@@ -1,0 +1,76 @@
+"""The QKV product whose epilogue turns q and k and writes the cache (gemm_qkv, what a prompt's layers call) against the product and
+qie_qkv_post: the same bits.  Short and tall tiles, split and whole, the 256x256 kernel, ragged rows, several prompts in a tile, heads of 64 and
+128, contiguous and paged; and a K that no kernel with that epilogue takes."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+import gpu_util as G
+from qwen_inference_engine_amd import _lib
+from qwen_inference_engine_amd._lib import KvCacheC, LinearArgsC
+
+pytestmark = pytest.mark.gpu
+SYMBOL = "_ZN3qie8gemm_qkvEPK15qie_linear_argsPK12qie_kv_cacheiiPKfPtP12ihipStream_tPb"
+
+
+# heads, key heads, head size, K, rows of a prompt, prompts, page
+@pytest.mark.parametrize("nq,nkv,hd,K,n,seqs,page,fused", [
+    (14, 2, 64, 896, 17, 1, 0, True), (14, 2, 64, 896, 113, 1, 128, True), (14, 2, 64, 896, 37, 5, 128, True),
+    (14, 2, 64, 896, 1501, 1, 0, True), (28, 4, 128, 3584, 63, 1, 128, True), (28, 4, 128, 3584, 301, 1, 0, True),
+    (28, 4, 128, 3584, 1030, 1, 128, True), (28, 4, 128, 512, 2100, 2, 256, True), (28, 4, 128, 512, 1363, 3, 0, True),
+    (3, 1, 8, 256, 65, 2, 0, True), (14, 2, 64, 928, 300, 1, 0, False)])
+def test_as_the_product_and_its_post_pass(qlib, nq, nkv, hd, K, n, seqs, page, fused):
+    M, QD, KD, ctx, layers, layer = n * seqs, nq * hd, nkv * hd, n + 3, 2, 1
+    N = QD + 2 * KD
+    g = torch.Generator("cuda").manual_seed(M + K)
+
+    def t(*shape, scale=1.0):
+        return (torch.randn(*shape, generator=g, device="cuda") * scale).bfloat16()
+    x, ws, bs = t(M, K), [t(r, K, scale=K ** -0.5) for r in (QD, KD, KD)], [t(r) for r in (QD, KD, KD)]
+    ang = torch.arange(ctx, device="cuda")[:, None] * 1e4 ** (-torch.arange(hd // 2, device="cuda") / (hd // 2))
+    cs, sn = ang.cos().float().contiguous(), ang.sin().float().contiguous()
+    turns = torch.stack([cs, sn], -1).contiguous()
+    pos = torch.arange(M, device="cuda", dtype=torch.int32) % n
+    pages = -(-ctx // page) if page else 0
+    table = (torch.randperm(seqs * pages, generator=g, device="cuda").int() + 1) if page else None
+
+    def cache():
+        c = KvCacheC()
+        shape = (seqs * pages + 1, layers, nkv, page, hd) if page else (seqs, layers, nkv, ctx, hd)
+        kv = [torch.full(shape, 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+        c.k, c.v, c.seq_stride = kv[0].data_ptr(), kv[1].data_ptr(), kv[0][0].numel()
+        c.n_layers, c.n_kv_heads, c.head_dim, c.max_ctx = layers, nkv, hd, ctx
+        if page:
+            c.block_table, c.page_tokens, c.max_pages = table.data_ptr(), page, pages
+        return c, kv
+
+    def args(y):
+        a = LinearArgsC()
+        a.x, a.ldx, a.M, a.K, a.N, a.y, a.ldy, a.epilogue = x.data_ptr(), K, M, K, N, y.data_ptr(), N, _lib.QIE_EPI_STORE
+        for i, (w, b) in enumerate(zip(ws, bs)):
+            a.w[i], a.bias[i], a.seg_rows[i] = w.data_ptr(), b.data_ptr(), w.shape[0]
+        return a
+    y, q = torch.zeros(M, N, dtype=torch.bfloat16, device="cuda"), torch.zeros(M, QD, dtype=torch.bfloat16, device="cuda")
+    c, kv = cache()
+    torch.cuda.synchronize()
+    G.check(qlib.qie_linear(C.byref(args(y)), None), "qie_linear")
+    G.check(qlib.qie_qkv_post(y.data_ptr(), M, pos.data_ptr(), n, None, None, cs.data_ptr(), sn.data_ptr(), nq, C.byref(c), layer, 1e-6,
+                              _lib.QIE_NUMERICS_REF, q.data_ptr(), None), "qie_qkv_post")
+    fn = getattr(C.CDLL(_lib.load()._name), SYMBOL)
+    fn.restype = C.c_int
+    fn.argtypes = [C.c_void_p, C.c_void_p, C.c_int32, C.c_int32] + [C.c_void_p] * 4
+    y2, q2, done = torch.zeros_like(y), torch.full_like(q, 7.0), C.c_bool()
+    c2, kv2 = cache()
+    torch.cuda.synchronize()
+    G.check(fn(C.byref(args(y2)), C.byref(c2), layer, n, turns.data_ptr(), q2.data_ptr(), None, C.byref(done)), "gemm_qkv")
+    torch.cuda.synchronize()
+    assert done.value == fused
+    if not fused:
+        assert torch.equal(y, y2) and (q2 == 7.0).all()
+        return
+    assert torch.equal(q, q2)
+    for a, b in zip(kv, kv2):   # untouched: the other layer, the rest of the context and the page that nobody holds
+        assert torch.equal(a, b)
+    assert np.isfinite(q2.float().sum().item())
