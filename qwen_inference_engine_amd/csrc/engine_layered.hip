@@ -1274,9 +1274,11 @@ static int enq_ff(qie_batch* b, int i, int T, hipStream_t on = nullptr) {
                                    s->sel, s->score, st));
     else
         QIE_TRY(lay::route_topk(y, L.w_router, L.router_b, m->f32, T, W, E, top, out_w ? 1 : 0, s->sel, s->score, st));
-    QIE_TRY(lay::moe_group(s->sel, n, ER, s->cnt, s->off, s->slot_of, st));
     const bool per_expert = !m->f32 && n >= kMoeSyncRows && W % 8 == 0 && ff % 8 == 0;
-    QIE_TRY(lay::moe_gather(y, in_score, s->slot_of, T, top, W, s->xg, per_expert ? s->xg_bf : nullptr, st));
+    const bool few = n <= 256 && !per_expert;
+    if (few) QIE_TRY(lay::moe_place(s->sel, T, top, ER, s->off, s->slot_of, y, in_score, W, s->xg, st));
+    else QIE_TRY(lay::moe_group(s->sel, n, ER, s->cnt, s->off, s->slot_of, st));
+    if (!few) QIE_TRY(lay::moe_gather(y, in_score, s->slot_of, T, top, W, s->xg, per_expert ? s->xg_bf : nullptr, st));
     if (per_expert) {
         // prompt-sized steps: the expert row ranges come to the host and every expert's rows go
         // through the MFMA kernels; the products are the grouped kernel's, in another order
@@ -1319,8 +1321,12 @@ static int enq_ff(qie_batch* b, int i, int T, hipStream_t on = nullptr) {
         QIE_TRY(join());
         return lay::moe_combine(s->yd, s->slot_of, out_score, T, top, W, s->ffo, st, id_sel, E, s->y);
     }
-    QIE_TRY(lin(e, s->xg, W, L.w_gu, W, s->gu, 2 * ff, n, 2 * ff, W, E, 0, (int64_t)2 * ff * W, 0, s->off));
-    QIE_TRY(lay::silu_mul(s->gu, s->act, nullptr, n, ff, st));
+    bool gated = false;   // gate, up and their product in one launch
+    QIE_TRY(lay::linear_gated({s->xg, W, L.w_gu, W, s->act, ff, n, ff, W, E, 0, (int64_t)2 * ff * W, 0, m->f32 ? 0 : 1, s->off, 0}, m->f32, e->stream, &gated));
+    if (!gated) {
+        QIE_TRY(lin(e, s->xg, W, L.w_gu, W, s->gu, 2 * ff, n, 2 * ff, W, E, 0, (int64_t)2 * ff * W, 0, s->off));
+        QIE_TRY(lay::silu_mul(s->gu, s->act, nullptr, n, ff, st));
+    }
     QIE_TRY(lin(e, s->act, ff, L.w_down, ff, s->yd, W, n, W, ff, E, 0, (int64_t)W * ff, 0, s->off));
     return lay::moe_combine(s->yd, s->slot_of, out_score, T, top, W, s->ffo, st, id_sel, E, s->y);
 }

@@ -38,6 +38,7 @@ struct LinearP {
     int mfma;   // bf16 weights, many rows: the direct MFMA kernel may take the product (batched / grouped forms)
 };
 int linear(const LinearP& p, bool w_f32, hipStream_t st);
+int linear_gated(const LinearP& p, bool w_f32, hipStream_t st, bool* done);
 // k_linear_f32.hip: fp32 operands, more than 16 rows, on the fp32 matrix cores; *done false: not its shape
 int linear_f32(const LinearP& p, hipStream_t st, bool* done);
 
@@ -596,6 +597,9 @@ int moe_group(const int32_t* sel, int n, int E, int32_t* cnt, int32_t* off, int3
 // score (may be null: 1) scales the gathered input rows / the combined output rows
 int moe_gather(const float* y, const float* score, const int32_t* slot_of, int T, int top, int W, float* xg, uint16_t* xg_bf,
                hipStream_t st);
+// moe_group and moe_gather of up to 256 entries
+int moe_place(const int32_t* sel, int T, int top, int E, int32_t* off, int32_t* slot_of, const float* y, const float* score, int W, float* xg,
+              hipStream_t st);
 // sel / n_real / y: a chosen expert >= n_real is an identity expert whose output is the row's input y
 int moe_combine(const float* yd, const int32_t* slot_of, const float* score, int T, int top, int W, float* f, hipStream_t st,
                 const int32_t* sel = nullptr, int n_real = 0, const float* y = nullptr);
