@@ -353,22 +353,22 @@ __device__ __forceinline__ float4 key4(const uint16_t* p) {
     return make_float4(bf_lo(u.x), bf_hi(u.x), bf_lo(u.y), bf_hi(u.y));
 }
 
-template <typename TC>
-__global__ __launch_bounds__(256) void gqa_attention_kernel(GqaAttnP p) {
-    constexpr int VC = 4 * GA_MAXV, KU = 4;
+template <typename TC, int NW>
+__global__ __launch_bounds__(64 * NW) void gqa_attention_kernel(GqaAttnP p) {
+    constexpr int VC = NW > 4 ? 4 : 4 * GA_MAXV, KU = 4, NT = 64 * NW;   // coordinates a lane: vdim <= 64 VC
     extern __shared__ __attribute__((aligned(16))) float sm[];
     const int dimp = (p.dim + 3) & ~3;
     float* q = sm;                 // [dim]
     float* sc = sm + dimp;         // [GA_CHUNK]
-    float* ob = sc + GA_CHUNK;     // [4][vdim]
-    __shared__ float red[4];
+    float* ob = sc + GA_CHUNK;     // [NW][vdim]
+    __shared__ float red[NW];
     __shared__ int64_t kbase[GA_CHUNK];   // a key's page, elements into the pool
     __shared__ int ktok[GA_CHUNK];        // its token in the page
     const int h = blockIdx.x, t = blockIdx.y, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int slot = p.row_slot[t], pos = p.row_pos[t];
     const int dim = p.dim, vdim = p.vdim, G = p.kv_heads, g = h / (p.heads / G), PT = p.cache.page_tokens;
     const float* qr = p.proj + (int64_t)t * p.ld + p.q_col + h * dim;
-    for (int i = tid; i < dim; i += 256) q[i] = qr[i];
+    for (int i = tid; i < dim; i += NT) q[i] = qr[i];
     const int lo = first_visible(p.mask, p.mask_size, pos);
     const float b1 = p.r1 ? p.r1[h] : 0.f, b2 = p.r1 ? p.r2[h] : 0.f;
     const float slope = p.slopes ? p.slopes[h] : 0.f;
@@ -393,11 +393,11 @@ __global__ __launch_bounds__(256) void gqa_attention_kernel(GqaAttnP p) {
             ktok[tid] = j % PT;
         }
         __syncthreads();
-        for (int jb = 0; jb < nk; jb += 16 * KU) {   // (uniform: every lane takes part in the sums over 16 lanes)
+        for (int jb = 0; jb < nk; jb += 4 * NW * KU) {   // (uniform: every lane takes part in the sums over 16 lanes)
             float s[KU];
 #pragma unroll
             for (int u = 0; u < KU; u++) {
-                const int jj = min(jb + 16 * u + gi, nk - 1);
+                const int jj = min(jb + 4 * NW * u + gi, nk - 1);
                 const TC* k = pool + kbase[jj] + p.k_off + ((int64_t)ktok[jj] * G + g) * dim;
                 s[u] = 0.f;
                 if (vec) {
@@ -414,7 +414,7 @@ __global__ __launch_bounds__(256) void gqa_attention_kernel(GqaAttnP p) {
                 const float v = group_sum<16>(s[u]);
                 s[0] = gl == u ? v : s[0];   // lane u of the group finishes its key u
             }
-            const int jj = jb + 16 * gl + gi;
+            const int jj = jb + 4 * NW * gl + gi;
             if (gl < KU && jj < nk) {
                 const int j = key_of(j0 + jj);
                 float v = s[0] * p.scale;
@@ -427,48 +427,58 @@ __global__ __launch_bounds__(256) void gqa_attention_kernel(GqaAttnP p) {
         __syncthreads();
         if (!sig) {   // (sigmoid weights are final: no running maximum, no normalisation)
             float mx = -INFINITY;
-            for (int jj = tid; jj < nk; jj += 256) mx = fmaxf(mx, sc[jj]);
+            for (int jj = tid; jj < nk; jj += NT) mx = fmaxf(mx, sc[jj]);
             mx = wmax(mx);
             if (lane == 0) red[wave] = mx;
             __syncthreads();
-            mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+            mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));   // (a chunk is 4 waves' keys)
             const float m_new = fmaxf(m_run, mx);
             const float alpha = expf(m_run - m_new);   // 0 on the first chunk
             __syncthreads();
             float ls = 0.f;
-            for (int jj = tid; jj < nk; jj += 256) {
+            for (int jj = tid; jj < nk; jj += NT) {
                 const float e = expf(sc[jj] - m_new);
                 sc[jj] = e;
                 ls += e;
             }
-            ls = bsum256(ls, red);
+            ls = wave_sum(ls);
+            if (lane == 0) red[wave] = ls;
+            __syncthreads();
+            ls = red[0] + red[1] + red[2] + red[3];
             l_run = l_run * alpha + ls;
             m_run = m_new;
 #pragma unroll
             for (int i = 0; i < VC; i++) acc[i] *= alpha;
         }
-        // a wave's keys: jj = wave, wave + 4, ...; a lane's coordinates r = lane + 64 c
+        // a wave's keys: jj = wave, wave + NW, ...; a lane's coordinates r = lane + 64 c
         auto value = [&](int jj, int r) {
             const int pt = ktok[jj];
             return ldc<TC>(pool + kbase[jj] + p.v_off, p.v_transposed ? ((int64_t)g * vdim + r) * PT + pt : ((int64_t)pt * G + g) * vdim + r);
         };
         int jj = wave;
-        for (; jj + 4 * (KU - 1) < nk; jj += 4 * KU)
+        for (; jj + NW * (KU - 1) < nk; jj += NW * KU)
 #pragma unroll
             for (int c = 0; c < VC; c++) {
                 if (64 * c >= vdim) break;   // uniform
                 const int r = min(lane + 64 * c, vdim - 1);
                 float v[KU];
 #pragma unroll
-                for (int u = 0; u < KU; u++) v[u] = value(jj + 4 * u, r);
+                for (int u = 0; u < KU; u++) v[u] = value(jj + NW * u, r);
 #pragma unroll
-                for (int u = 0; u < KU; u++) acc[c] = fmaf(sc[jj + 4 * u], v[u], acc[c]);
+                for (int u = 0; u < KU; u++) acc[c] = fmaf(sc[jj + NW * u], v[u], acc[c]);
             }
-        for (; jj < nk; jj += 4)
+        for (; jj < nk; jj += NW * (NW > 4 ? KU : 1))   // the rest: together where it is a large part, key by key
 #pragma unroll
             for (int c = 0; c < VC; c++) {
                 if (64 * c >= vdim) break;
-                acc[c] = fmaf(sc[jj], value(jj, min(lane + 64 * c, vdim - 1)), acc[c]);
+                const int r = min(lane + 64 * c, vdim - 1);
+                constexpr int U = NW > 4 ? KU : 1;
+                float v[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) v[u] = value(min(jj + NW * u, nk - 1), r);
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                    if (jj + NW * u < nk) acc[c] = fmaf(sc[jj + NW * u], v[u], acc[c]);
             }
     }
 #pragma unroll
@@ -478,10 +488,17 @@ __global__ __launch_bounds__(256) void gqa_attention_kernel(GqaAttnP p) {
     float inv = sig ? 1.0f : 1.0f / l_run;
     if (p.gate_col >= 0 && !p.gate_elem) inv *= 1.0f / (1.0f + expf(-p.proj[(int64_t)t * p.ld + p.gate_col + h]));
 #pragma unroll
-    for (int i = 0; i < GA_MAXV; i++) {
-        const int r = tid + i * 256;
+    for (int i = 0; i < GA_MAXV * 4 / NW; i++) {
+        const int r = tid + i * NT;
         if (r < vdim) {
-            float o = ((ob[r] + ob[vdim + r]) + (ob[2 * vdim + r] + ob[3 * vdim + r])) * inv;
+            float w[NW];
+#pragma unroll
+            for (int k = 0; k < NW; k++) w[k] = ob[k * vdim + r];
+#pragma unroll
+            for (int d = 1; d < NW; d *= 2)
+#pragma unroll
+                for (int k = 0; k < NW; k += 2 * d) w[k] += w[k + d];
+            float o = w[0] * inv;
             if (p.gate_col >= 0 && p.gate_elem) o *= 1.0f / (1.0f + expf(-p.proj[(int64_t)t * p.ld + p.gate_col + h * vdim + r]));
             ob[r] = o;
         }
@@ -490,7 +507,7 @@ __global__ __launch_bounds__(256) void gqa_attention_kernel(GqaAttnP p) {
     const float* vcs = p.rot_values ? p.vrope_cos + (int64_t)pos * (vdim / 2) : nullptr;
     const float* vsn = p.rot_values ? p.vrope_sin + (int64_t)pos * (vdim / 2) : nullptr;
     const int64_t o0 = (int64_t)t * p.ld_out + p.out_col + (int64_t)h * vdim;
-    for (int r = tid; r < vdim; r += 256) {
+    for (int r = tid; r < vdim; r += NT) {
         const float o = (p.rot_values ? turned(ob, r, vdim, p.rot_layout, vcs, vsn, -1.f) : ob[r]) * p.out_scale;
         if (p.out) p.out[o0 + r] = o;
         if (p.out_bf) p.out_bf[o0 + r] = f2bf(o);
@@ -503,11 +520,16 @@ int gqa_attention(const GqaAttnP& p, bool cache_f32, int T, hipStream_t st) {
     QIE_REQUIRE(p.mask_keep >= 0 && (p.mask_keep == 0 || p.mask == 1), "gqa attention: kept first keys go with the window mask");
     QIE_REQUIRE(p.heads % p.kv_heads == 0, "gqa attention: %d query heads over %d key heads", p.heads, p.kv_heads);
     QIE_REQUIRE((size_t)(p.dim + GA_CHUNK + p.vdim) * 4 <= 48 * 1024, "gqa attention: head size above the kernel's staging");
-    const size_t shm = (size_t)((p.dim + 3) / 4 * 4 + GA_CHUNK + 4 * p.vdim) * 4;
-    if (cache_f32)
-        hipLaunchKernelGGL(gqa_attention_kernel<float>, dim3(p.heads, T), dim3(256), shm, st, p);
-    else
-        hipLaunchKernelGGL(gqa_attention_kernel<uint16_t>, dim3(p.heads, T), dim3(256), shm, st, p);
+    // 16 waves a block where the blocks don't fill the chip (decode steps): a chunk's keys are scored in one trip and its values read in
+    // four.  us, Lugipel at width 1,024, fp32: 3 rows over 150 keys 16.2 -> 9.3
+    const bool wide = p.vdim <= 256 && p.dim <= 1024 && (int64_t)p.heads * T <= 2 * device_cu_count();
+    const int nw = wide ? 16 : 4;
+    const size_t shm = (size_t)((p.dim + 3) / 4 * 4 + GA_CHUNK + nw * p.vdim) * 4;
+    const dim3 grid(p.heads, T), block(64 * nw);
+    if (cache_f32 && wide) hipLaunchKernelGGL((gqa_attention_kernel<float, 16>), grid, block, shm, st, p);
+    else if (cache_f32) hipLaunchKernelGGL((gqa_attention_kernel<float, 4>), grid, block, shm, st, p);
+    else if (wide) hipLaunchKernelGGL((gqa_attention_kernel<uint16_t, 16>), grid, block, shm, st, p);
+    else hipLaunchKernelGGL((gqa_attention_kernel<uint16_t, 4>), grid, block, shm, st, p);
     QIE_LAUNCH_CHECK();
     return 0;
 }
