@@ -1234,7 +1234,8 @@ static int enq_mixer_out(qie_batch* b, int i, int T) {
 
 // feed-forward of layer i on its normed rows (s->y, in parallel blocks s->y2) -> ffo; where the layer's output product
 // takes the activations as well (cat_ff), they go beside the mixer's columns and the product is left to it
-static int enq_ff(qie_batch* b, int i, int T, hipStream_t on = nullptr) {
+// later: where the experts' sum may be left to (ffo is then not written)
+static int enq_ff(qie_batch* b, int i, int T, hipStream_t on = nullptr, lay::ExpertSum* later = nullptr) {
     const qie_engine* e = b->e;
     const LayeredModel* m = e->lm;
     const LayerDev& L = m->L[i];
@@ -1328,6 +1329,10 @@ static int enq_ff(qie_batch* b, int i, int T, hipStream_t on = nullptr) {
         QIE_TRY(lay::silu_mul(s->gu, s->act, nullptr, n, ff, st));
     }
     QIE_TRY(lin(e, s->act, ff, L.w_down, ff, s->yd, W, n, W, ff, E, 0, (int64_t)W * ff, 0, s->off));
+    if (later && W <= lay::kAddNormMax) {
+        *later = {s->yd, s->slot_of, out_score, id_sel, s->y, top, E};
+        return 0;
+    }
     return lay::moe_combine(s->yd, s->slot_of, out_score, T, top, W, s->ffo, st, id_sel, E, s->y);
 }
 
@@ -1850,7 +1855,7 @@ static int enq_run_prenorm(qie_batch* b, int r, int T, bool h_ready, bool* next_
     const bool canon = m->a.canon_taps > 0;
     // y: the sublayer result that updates the rows with the coefficients of sublayer q of this layer (null:
     // none); then the read-out with in_next (hyper-connections) normed with wn -> h (null wn: no read-out)
-    auto step = [&](const float* y, int q, const float* in_next, const float* wn, bool to_mixer, float* sum) -> int {
+    auto step = [&](const float* y, int q, const float* in_next, const float* wn, bool to_mixer, float* sum, const lay::ExpertSum& es = {}) -> int {
         float* h = to_mixer && canon ? s->x : s->y;
         uint16_t* h_bf = to_mixer && canon ? nullptr : s->y_bf;
         if (n > 0) {
@@ -1858,7 +1863,7 @@ static int enq_run_prenorm(qie_batch* b, int r, int T, bool h_ready, bool* next_
                                h, h_bf, sum, T, W};
             return lay::stream_step(p, st);
         }
-        return lay::add_norm(x, x, y, nullptr, nullptr, wn, h, h_bf, T, W, eps, st, w_one);
+        return lay::add_norm(x, x, es.yd ? nullptr : y, nullptr, nullptr, wn, h, h_bf, T, W, eps, st, w_one, 1, 0, es);
     };
     if (!h_ready) QIE_TRY(step(nullptr, 0, L.hc_in[0], L.n1, true, nullptr));
     if (canon) {
@@ -1889,8 +1894,9 @@ static int enq_run_prenorm(qie_batch* b, int r, int T, bool h_ready, bool* next_
     float* sum = n > 0 ? (s->keep_on && s->keep ? s->keep + (int64_t)r * plane : last ? s->x : nullptr) : nullptr;
     if (has_ff) {
         QIE_TRY(step(s->mix, 0, L.hc_in[1], L.n2, false, nullptr));
-        QIE_TRY(enq_ff(b, m->runs[r].layer, T));
-        QIE_TRY(step(s->ffo, 1, next_in, next_w, true, sum));
+        lay::ExpertSum es{};
+        QIE_TRY(enq_ff(b, m->runs[r].layer, T, nullptr, n > 0 ? nullptr : &es));
+        QIE_TRY(step(s->ffo, 1, next_in, next_w, true, sum, es));
     } else {
         QIE_TRY(step(s->mix, 0, next_in, next_w, true, sum));
     }
@@ -1927,8 +1933,9 @@ static int enq_run_sandwich(qie_batch* b, int r, int T, bool h_ready, bool* next
     const float* nx_add = fuse_next && m->runs[r + 1].add_embed ? x0 : nullptr;
     if (has_ff) {
         QIE_TRY(lay::add_norm(x, x, s->mix, L.n1b, nullptr, L.n2, s->y, s->y_bf, T, W, eps, st));
-        QIE_TRY(enq_ff(b, m->runs[r].layer, T));
-        QIE_TRY(lay::add_norm(x, x, s->ffo, L.n2b, nx_add, fuse_next ? N->n1 : nullptr, s->y, s->y_bf, T, W, eps, st));
+        lay::ExpertSum es{};
+        QIE_TRY(enq_ff(b, m->runs[r].layer, T, nullptr, &es));
+        QIE_TRY(lay::add_norm(x, x, es.yd ? nullptr : s->ffo, L.n2b, nx_add, fuse_next ? N->n1 : nullptr, s->y, s->y_bf, T, W, eps, st, 1.f, 1, 0, es));
     } else {
         QIE_TRY(lay::add_norm(x, x, s->mix, L.n1b, nx_add, fuse_next ? N->n1 : nullptr, s->y, s->y_bf, T, W, eps, st));
     }

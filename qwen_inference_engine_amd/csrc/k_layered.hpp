@@ -556,12 +556,22 @@ int rglru_step(const RgLruP& p, int T, int chain, hipStream_t st);
 int low_rank_log_sigmoid(const float* in, int64_t ld_in, int rank, const void* w, bool w_f32, const float* bias, float tau, int n, int T,
                          float* out, hipStream_t st);
 
+// What moe_combine would write, left to the add_norm that reads it (rows of up to kAddNormMax)
+struct ExpertSum {
+    const float* yd;   // null: none
+    const int32_t* slot_of;
+    const float* score;
+    const int32_t* sel;
+    const float* y;
+    int top, n_real;
+};
+constexpr int kAddNormMax = 4096;
 // Rows of W: x = xin + (wb ? rms(v) * (w_one + wb) : v) (when v) + add (when add); then (when wn)
 // h = rms(x) * (w_one + wn) with its bf16 image.  xin may be x.  w_one = 1: weight vectors stored
 // around zero; 0: plain weights.
-// copies > 1: h is written `copies` times, `plane` elements apart (the rows of several residual streams start equal).
+// m.yd: v is that sum.  copies > 1: h is written `copies` times, `plane` elements apart (the rows of several residual streams start equal).
 int add_norm(float* x, const float* xin, const float* v, const float* wb, const float* add, const float* wn, float* h, uint16_t* h_bf,
-             int T, int W, float eps, hipStream_t st, float w_one = 1.0f, int copies = 1, int64_t plane = 0);
+             int T, int W, float eps, hipStream_t st, float w_one = 1.0f, int copies = 1, int64_t plane = 0, const ExpertSum& m = {});
 
 // The producers below also write the bf16 image of their result when the *_bf pointer is set
 // (bf16 engines: the next product reads it; no separate rounding pass).

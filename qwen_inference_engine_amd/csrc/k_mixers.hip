@@ -444,7 +444,7 @@ __global__ __launch_bounds__(64 * NW) void gqa_attention_kernel(GqaAttnP p) {
             ls = wave_sum(ls);
             if (lane == 0) red[wave] = ls;
             __syncthreads();
-            ls = red[0] + red[1] + red[2] + red[3];
+            ls = (red[0] + red[1]) + (red[2] + red[3]);
             l_run = l_run * alpha + ls;
             m_run = m_new;
 #pragma unroll
@@ -1479,9 +1479,109 @@ __global__ __launch_bounds__(256) void add_norm_kernel(float* x, const float* xi
         if (h_bf) h_bf[r0 + i] = f2bf(o);
     }
 }
+// W <= 256 C: the same with the row and all operands in registers, asked for at once (the loops above go to memory four times, once to read
+// back what the thread has just stored).  m.yd: the branch is the routed experts' sum (moe_combine_kernel's, in its order; no launch and row
+// of its own).  us, 3 rows of 1,024: 4.6 -> 3.4, on the average of launches with the experts' sum (4.2 us before) and without.  Bits as there.
+template <int C>
+__global__ __launch_bounds__(256) void add_norm_reg_kernel(float* x, const float* xin, const float* v, const float* wb, const float* add,
+                                                           const float* wn, float* h, uint16_t* h_bf, int W, float eps, float w_one,
+                                                           int copies, int64_t plane, ExpertSum m) {
+    __shared__ float red[4];
+    const int64_t t = blockIdx.x, r0 = t * W;
+    float xv[C], vv[C], av[C], bv[C], nv[C];
+    int at[C];
+    bool in[C];
+    const bool branch = v || m.yd;
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        const int i = threadIdx.x + 256 * c;
+        in[c] = i < W;
+        at[c] = in[c] ? i : 0;
+        xv[c] = xin[r0 + at[c]];
+    }
+    if (v) {
+#pragma unroll
+        for (int c = 0; c < C; c++) vv[c] = v[r0 + at[c]];
+    }
+    if (add) {
+#pragma unroll
+        for (int c = 0; c < C; c++) av[c] = add[r0 + at[c]];
+    }
+    if (wb) {
+#pragma unroll
+        for (int c = 0; c < C; c++) bv[c] = wb[at[c]];
+    }
+    if (wn) {
+#pragma unroll
+        for (int c = 0; c < C; c++) nv[c] = wn[at[c]];
+    }
+    if (m.yd) {
+#pragma unroll
+        for (int c = 0; c < C; c++) vv[c] = 0.f;
+        for (int k0 = 0; k0 < m.top; k0 += 2) {
+            float o[2][C], sc[2];
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const int64_t e = t * m.top + min(k0 + k, m.top - 1);
+                const float* row = m.sel && m.sel[e] >= m.n_real ? m.y + r0 : m.yd + (int64_t)m.slot_of[e] * W;
+                sc[k] = m.score ? m.score[e] : 1.0f;
+#pragma unroll
+                for (int c = 0; c < C; c++) o[k][c] = row[at[c]];
+            }
+#pragma unroll
+            for (int k = 0; k < 2; k++)
+                if (k0 + k < m.top) {
+#pragma unroll
+                    for (int c = 0; c < C; c++) vv[c] = fmaf(sc[k], o[k][c], vv[c]);
+                }
+        }
+    }
+    float inv_v = 0.f;
+    if (branch && wb) {
+        float ss = 0.f;
+#pragma unroll
+        for (int c = 0; c < C; c++)
+            if (in[c]) ss += vv[c] * vv[c];
+        ss = bsum256(ss, red);
+        inv_v = 1.0f / sqrtf(ss / (float)W + eps);
+    }
+    float sx = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        if (!in[c]) continue;
+        float a = xv[c];
+        if (branch) a += wb ? vv[c] * inv_v * (w_one + bv[c]) : vv[c];
+        if (add) a += av[c];
+        if (branch || add || xin != x) x[r0 + at[c]] = a;
+        xv[c] = a;
+        sx += a * a;
+    }
+    if (!wn) return;
+    sx = bsum256(sx, red);
+    const float inv_x = 1.0f / sqrtf(sx / (float)W + eps);
+#pragma unroll
+    for (int c = 0; c < C; c++) {
+        if (!in[c]) continue;
+        const float o = xv[c] * inv_x * (w_one + nv[c]);
+        h[r0 + at[c]] = o;
+        for (int k = 1; k < copies; k++) h[k * plane + r0 + at[c]] = o;
+        if (h_bf) h_bf[r0 + at[c]] = f2bf(o);
+    }
+}
 int add_norm(float* x, const float* xin, const float* v, const float* wb, const float* add, const float* wn, float* h, uint16_t* h_bf,
-             int T, int W, float eps, hipStream_t st, float w_one, int copies, int64_t plane) {
-    QIE_REQUIRE(x && xin && (!wn || h), "add_norm: bad arguments");
+             int T, int W, float eps, hipStream_t st, float w_one, int copies, int64_t plane, const ExpertSum& m) {
+    QIE_REQUIRE(x && xin && (!wn || h) && !(v && m.yd), "add_norm: bad arguments");
+#define QIE_AN(C)                                                                                                                             \
+    if (W <= 256 * C) {                                                                                                                       \
+        hipLaunchKernelGGL(add_norm_reg_kernel<C>, dim3(T), dim3(256), 0, st, x, xin, v, wb, add, wn, h, h_bf, W, eps, w_one, copies, plane, m); \
+        QIE_LAUNCH_CHECK();                                                                                                                   \
+        return 0;                                                                                                                             \
+    }
+    QIE_AN(4)
+    QIE_AN(8)
+    QIE_AN(kAddNormMax / 256)
+#undef QIE_AN
+    QIE_REQUIRE(!m.yd, "add_norm: the experts' sum of a row of %d", W);
     hipLaunchKernelGGL(add_norm_kernel, dim3(T), dim3(256), 0, st, x, xin, v, wb, add, wn, h, h_bf, W, eps, w_one, copies, plane);
     QIE_LAUNCH_CHECK();
     return 0;
