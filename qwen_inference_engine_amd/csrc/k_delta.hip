@@ -293,9 +293,111 @@ __global__ __launch_bounds__(256) void delta_carry_kernel(DeltaCarryP p) {
     for (int r = r0; r < dim; r += 32) stp[(int64_t)r * vdim + col] = ss[r * DC_COLS + c];
 }
 
+// dim 64 and 128: M times 32 state columns on the fp32 matrix cores (v_mfma_f32_16x16x4f32, a lane's four k from one 16-byte load), the next
+// piece's M and local state on their way meanwhile.  A wave owns 16 RT rows of the state, which all waves read from LDS, transposed.  The form
+// above goes to memory for M inside its sums and reads all of it for 8 columns.  us, 16 heads of 128 x 128: 4 entries of 30 pieces in all
+// 160 -> 49, 5 entries of 9 pieces 94 -> 32.
+typedef float dc_f32x4 __attribute__((ext_vector_type(4)));
+template <int DIM>
+__global__ __launch_bounds__(256) void delta_carry_mfma_kernel(DeltaCarryP p) {
+    constexpr int RT = DIM / 64, KS = DIM / 16, CT = 2, LD = DIM + 4;   // row tiles a wave, 16-k steps, column tiles
+    __shared__ __attribute__((aligned(16))) float ss[2][16 * CT][LD];   // [column][row]
+    const int4 sp = p.spans[blockIdx.x];   // {first piece, pieces, slot, first position}
+    const int h = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, fr = lane & 15, g = lane >> 4;
+    const int vdim = p.vdim, H = p.H, row0 = wave * 16 * RT;
+    float* stp = p.state + (int64_t)sp.z * p.slot_stride + p.state_off + (int64_t)h * DIM * vdim;
+    int col[CT];
+    bool colv[CT];
+#pragma unroll
+    for (int j = 0; j < CT; j++) {
+        col[j] = blockIdx.z * 16 * CT + 16 * j + fr;
+        colv[j] = col[j] < vdim;
+        col[j] = colv[j] ? col[j] : vdim - 1;
+    }
+    auto at = [&](int i, int r, int j) { return (int64_t)(row0 + 16 * i + 4 * g + r) * vdim + col[j]; };
+    dc_f32x4 cur[RT][CT];
+#pragma unroll
+    for (int i = 0; i < RT; i++)
+#pragma unroll
+        for (int j = 0; j < CT; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) cur[i][j][r] = sp.w > 0 ? stp[at(i, r, j)] : 0.f;
+    struct Piece {
+        dc_f32x4 m[RT][KS], loc[RT][CT];
+    };
+    auto load = [&](Piece& q, int k) {
+        const int64_t ph = (int64_t)(sp.x + k) * H + h;
+        const float* mt = p.trans + ph * DIM * DIM;
+        const float* sl = p.s_loc + ph * DIM * vdim;
+#pragma unroll
+        for (int i = 0; i < RT; i++) {
+#pragma unroll
+            for (int kk = 0; kk < KS; kk++) q.m[i][kk] = *reinterpret_cast<const dc_f32x4*>(mt + (int64_t)(row0 + 16 * i + fr) * DIM + 16 * kk + 4 * g);
+#pragma unroll
+            for (int j = 0; j < CT; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) q.loc[i][j][r] = sl[at(i, r, j)];
+        }
+    };
+    auto step = [&](const Piece& q, Piece& next, int k) {
+        float* si = p.s_in + ((int64_t)(sp.x + k) * H + h) * DIM * vdim;
+        float (*s)[LD] = ss[k & 1];   // (written again two pieces on, behind the next piece's barrier)
+#pragma unroll
+        for (int i = 0; i < RT; i++)
+#pragma unroll
+            for (int j = 0; j < CT; j++) *reinterpret_cast<dc_f32x4*>(&s[16 * j + fr][row0 + 16 * i + 4 * g]) = cur[i][j];
+        if (k + 1 < sp.y) load(next, k + 1);
+#pragma unroll
+        for (int i = 0; i < RT; i++)
+#pragma unroll
+            for (int j = 0; j < CT; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (colv[j]) si[at(i, r, j)] = cur[i][j][r];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < RT; i++)
+#pragma unroll
+            for (int j = 0; j < CT; j++) cur[i][j] = q.loc[i][j];
+#pragma unroll
+        for (int kk = 0; kk < KS; kk++) {
+            dc_f32x4 b[CT];
+#pragma unroll
+            for (int j = 0; j < CT; j++) b[j] = *reinterpret_cast<const dc_f32x4*>(&s[16 * j + fr][16 * kk + 4 * g]);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int i = 0; i < RT; i++)
+#pragma unroll
+                    for (int j = 0; j < CT; j++) cur[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(q.m[i][kk][e], b[j][e], cur[i][j], 0, 0, 0);
+        }
+    };
+    Piece pa, pb;
+    if (sp.y > 0) load(pa, 0);
+    for (int k = 0; k < sp.y; k += 2) {   // uniform
+        step(pa, pb, k);
+        if (k + 1 < sp.y) step(pb, pa, k + 1);
+    }
+    if (!p.write_state) return;
+#pragma unroll
+    for (int i = 0; i < RT; i++)
+#pragma unroll
+        for (int j = 0; j < CT; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (colv[j]) stp[at(i, r, j)] = cur[i][j][r];
+}
+
 int delta_carry(const DeltaCarryP& p, hipStream_t st) {
     QIE_REQUIRE(p.spans && p.n_spans > 0 && p.s_loc && p.trans && p.s_in && p.state && p.dim > 0 && p.dim <= 512 && p.vdim > 0,
                 "delta_carry: bad arguments");
+    if ((p.dim == 64 || p.dim == 128) && (uintptr_t)p.trans % 16 == 0) {
+        const dim3 tiles((unsigned)p.n_spans, (unsigned)p.H, (unsigned)((p.vdim + 31) / 32));
+        if (p.dim == 64) hipLaunchKernelGGL(delta_carry_mfma_kernel<64>, tiles, dim3(256), 0, st, p);
+        else hipLaunchKernelGGL(delta_carry_mfma_kernel<128>, tiles, dim3(256), 0, st, p);
+        QIE_LAUNCH_CHECK();
+        return 0;
+    }
     const dim3 grid((unsigned)p.n_spans, (unsigned)p.H, (unsigned)((p.vdim + DC_COLS - 1) / DC_COLS));
     hipLaunchKernelGGL(delta_carry_kernel, grid, dim3(256), (size_t)p.dim * DC_COLS * 4, st, p);
     QIE_LAUNCH_CHECK();
