@@ -353,14 +353,17 @@ __device__ __forceinline__ float4 key4(const uint16_t* p) {
     return make_float4(bf_lo(u.x), bf_hi(u.x), bf_lo(u.y), bf_hi(u.y));
 }
 
-template <typename TC, int NW>
+// Values up to 256 wide (VC 4): a coordinate's sum is 16 sums, of every 16th key each, that meet in pairs, with 4 waves (4 sums a lane) as
+// with 16: a row's bits don't depend on how many rows there are.
+template <typename TC, int NW, int VC>
 __global__ __launch_bounds__(64 * NW) void gqa_attention_kernel(GqaAttnP p) {
-    constexpr int VC = NW > 4 ? 4 : 4 * GA_MAXV, KU = 4, NT = 64 * NW;   // coordinates a lane: vdim <= 64 VC
+    constexpr int KU = 4, NT = 64 * NW;
+    constexpr int NS = VC == 4 ? 16 / NW : 1, NP = NW * NS;   // sums a lane and coordinate, sums in all
     extern __shared__ __attribute__((aligned(16))) float sm[];
     const int dimp = (p.dim + 3) & ~3;
     float* q = sm;                 // [dim]
     float* sc = sm + dimp;         // [GA_CHUNK]
-    float* ob = sc + GA_CHUNK;     // [NW][vdim]
+    float* ob = sc + GA_CHUNK;     // [NP][vdim]
     __shared__ float red[NW];
     __shared__ int64_t kbase[GA_CHUNK];   // a key's page, elements into the pool
     __shared__ int ktok[GA_CHUNK];        // its token in the page
@@ -376,7 +379,7 @@ __global__ __launch_bounds__(64 * NW) void gqa_attention_kernel(GqaAttnP p) {
     const float pbh = sig ? p.pb[h] : 0.f;
     // a sink is a score without key or value: the running maximum and sum start from it
     float m_run = p.sink ? p.sink[h] : -INFINITY, l_run = p.sink ? 1.f : 0.f;
-    float acc[VC] = {};
+    float acc[NS][VC] = {};
     // the visible keys in order: the kept first ones that lie before the window, then the window's
     const int kept = min(p.mask_keep, lo), n_vis = kept + pos + 1 - lo;
     auto key_of = [&](int i) { return i < kept ? i : lo + i - kept; };
@@ -448,7 +451,9 @@ __global__ __launch_bounds__(64 * NW) void gqa_attention_kernel(GqaAttnP p) {
             l_run = l_run * alpha + ls;
             m_run = m_new;
 #pragma unroll
-            for (int i = 0; i < VC; i++) acc[i] *= alpha;
+            for (int n = 0; n < NS; n++)
+#pragma unroll
+                for (int i = 0; i < VC; i++) acc[n][i] *= alpha;
         }
         // a wave's keys: jj = wave, wave + NW, ...; a lane's coordinates r = lane + 64 c
         auto value = [&](int jj, int r) {
@@ -465,39 +470,41 @@ __global__ __launch_bounds__(64 * NW) void gqa_attention_kernel(GqaAttnP p) {
 #pragma unroll
                 for (int u = 0; u < KU; u++) v[u] = value(jj + NW * u, r);
 #pragma unroll
-                for (int u = 0; u < KU; u++) acc[c] = fmaf(sc[jj + NW * u], v[u], acc[c]);
+                for (int u = 0; u < KU; u++) acc[u % NS][c] = fmaf(sc[jj + NW * u], v[u], acc[u % NS][c]);
             }
-        for (; jj < nk; jj += NW * (NW > 4 ? KU : 1))   // the rest: together where it is a large part, key by key
+        for (; jj < nk; jj += NW * (VC == 4 ? KU : 1))   // the rest
 #pragma unroll
             for (int c = 0; c < VC; c++) {
                 if (64 * c >= vdim) break;
                 const int r = min(lane + 64 * c, vdim - 1);
-                constexpr int U = NW > 4 ? KU : 1;
+                constexpr int U = VC == 4 ? KU : 1;
                 float v[U];
 #pragma unroll
                 for (int u = 0; u < U; u++) v[u] = value(min(jj + NW * u, nk - 1), r);
 #pragma unroll
                 for (int u = 0; u < U; u++)
-                    if (jj + NW * u < nk) acc[c] = fmaf(sc[jj + NW * u], v[u], acc[c]);
+                    if (jj + NW * u < nk) acc[u % NS][c] = fmaf(sc[jj + NW * u], v[u], acc[u % NS][c]);
             }
     }
 #pragma unroll
-    for (int c = 0; c < VC; c++)
-        if (lane + 64 * c < vdim) ob[wave * vdim + lane + 64 * c] = acc[c];
+    for (int n = 0; n < NS; n++)
+#pragma unroll
+        for (int c = 0; c < VC; c++)
+            if (lane + 64 * c < vdim) ob[(wave + NW * n) * vdim + lane + 64 * c] = acc[n][c];
     __syncthreads();
     float inv = sig ? 1.0f : 1.0f / l_run;
     if (p.gate_col >= 0 && !p.gate_elem) inv *= 1.0f / (1.0f + expf(-p.proj[(int64_t)t * p.ld + p.gate_col + h]));
 #pragma unroll
-    for (int i = 0; i < GA_MAXV * 4 / NW; i++) {
+    for (int i = 0; i < (64 * VC + NT - 1) / NT; i++) {
         const int r = tid + i * NT;
         if (r < vdim) {
-            float w[NW];
+            float w[NP];
 #pragma unroll
-            for (int k = 0; k < NW; k++) w[k] = ob[k * vdim + r];
+            for (int k = 0; k < NP; k++) w[k] = ob[k * vdim + r];
 #pragma unroll
-            for (int d = 1; d < NW; d *= 2)
+            for (int d = 1; d < NP; d *= 2)
 #pragma unroll
-                for (int k = 0; k < NW; k += 2 * d) w[k] += w[k + d];
+                for (int k = 0; k < NP; k += 2 * d) w[k] += w[k + d];
             float o = w[0] * inv;
             if (p.gate_col >= 0 && p.gate_elem) o *= 1.0f / (1.0f + expf(-p.proj[(int64_t)t * p.ld + p.gate_col + h * vdim + r]));
             ob[r] = o;
@@ -521,15 +528,20 @@ int gqa_attention(const GqaAttnP& p, bool cache_f32, int T, hipStream_t st) {
     QIE_REQUIRE(p.heads % p.kv_heads == 0, "gqa attention: %d query heads over %d key heads", p.heads, p.kv_heads);
     QIE_REQUIRE((size_t)(p.dim + GA_CHUNK + p.vdim) * 4 <= 48 * 1024, "gqa attention: head size above the kernel's staging");
     // 16 waves a block where the blocks don't fill the chip (decode steps): a chunk's keys are scored in one trip and its values read in
-    // four.  us, Lugipel at width 1,024, fp32: 3 rows over 150 keys 16.2 -> 9.3
-    const bool wide = p.vdim <= 256 && p.dim <= 1024 && (int64_t)p.heads * T <= 2 * device_cu_count();
-    const int nw = wide ? 16 : 4;
-    const size_t shm = (size_t)((p.dim + 3) / 4 * 4 + GA_CHUNK + nw * p.vdim) * 4;
-    const dim3 grid(p.heads, T), block(64 * nw);
-    if (cache_f32 && wide) hipLaunchKernelGGL((gqa_attention_kernel<float, 16>), grid, block, shm, st, p);
-    else if (cache_f32) hipLaunchKernelGGL((gqa_attention_kernel<float, 4>), grid, block, shm, st, p);
-    else if (wide) hipLaunchKernelGGL((gqa_attention_kernel<uint16_t, 16>), grid, block, shm, st, p);
-    else hipLaunchKernelGGL((gqa_attention_kernel<uint16_t, 4>), grid, block, shm, st, p);
+    // four.  us, Lugipel at width 1,024, fp32: 3 rows over 150 keys 16.2 -> 9.1
+    const bool narrow = p.vdim <= 256 && p.dim <= 1024, wide = narrow && (int64_t)p.heads * T <= 2 * device_cu_count();
+    const size_t shm = (size_t)((p.dim + 3) / 4 * 4 + GA_CHUNK + (narrow ? 16 : 4) * p.vdim) * 4;
+    const dim3 grid(p.heads, T), block(wide ? 1024 : 256);
+#define QIE_GA(TC)                                                                                            \
+    if (wide) hipLaunchKernelGGL((gqa_attention_kernel<TC, 16, 4>), grid, block, shm, st, p);                 \
+    else if (narrow) hipLaunchKernelGGL((gqa_attention_kernel<TC, 4, 4>), grid, block, shm, st, p);           \
+    else hipLaunchKernelGGL((gqa_attention_kernel<TC, 4, 4 * GA_MAXV>), grid, block, shm, st, p)
+    if (cache_f32) {
+        QIE_GA(float);
+    } else {
+        QIE_GA(uint16_t);
+    }
+#undef QIE_GA
     QIE_LAUNCH_CHECK();
     return 0;
 }

@@ -1,7 +1,8 @@
 """The layered attention on exact rows (k_mixers.hip): blocks of 16 waves beside those of 4, against the numpy restatement."""
+import numpy as np
 import pytest
 
-from lugipel_oracle import attn
+from lugipel_oracle import attn, dense
 from test_gpu_lugipel import feed, model, rel  # noqa: F401
 
 pytestmark = pytest.mark.gpu
@@ -14,3 +15,13 @@ def test_attention_in_blocks_of_either_size(model):  # noqa: F811
     want = m.ref(toks)
     got = feed(m, 0, toks, [85, 86, 100, 60, 3, 1, 85])
     assert rel(got, want) < m.tol
+
+
+def test_bits_do_not_depend_on_the_blocks(model):  # noqa: F811
+    """Rows of more than 16 in a step, so that the products' kernels are the same: steps of either kind, one chunk of keys and two."""
+    m = model([attn(heads=6, kv_heads=3, dim=64, vdim=64, size=400, mlp=dense(1440)), attn(heads=6, kv_heads=2, dim=64, vdim=128, size=300, mlp=dense(1440))],
+              seed=4, width=512, vocab=503)
+    toks = m.tokens(420)
+    whole = m.batch.step([(0, toks)], range(420))
+    m.batch.release(0)
+    assert np.array_equal(feed(m, 0, toks, [85, 86, 100, 64, 85]), whole)
