@@ -839,7 +839,7 @@ static int dec8_launch(const Dec8Params& p, hipStream_t st) {
 }
 
 // ---------------------------------------------------------------------------
-// dec8s: long K (the down projection), plain rows: nobody else's sums.  The split-K form above shares a tile among ten workgroups that
+// dec8s: long K (the down projection), plain rows.  The split-K form above shares a tile among ten workgroups that
 // meet through memory: a ticket, a drain and a second trip behind every launch, 3.6 TB/s.  Here a workgroup of 8 waves owns whole
 // 16-row tiles and every wave streams the 128-k chunks of its own share of K by LDS-DMA through a ring of its own, X's rows beside
 // the weights' (they come from L2; all of them do not fit LDS), with no barrier until the waves' partial tiles meet in LDS.
@@ -1128,7 +1128,7 @@ static int dec8_epi(const Dec8Params& p, int epi, hipStream_t st) {
 
 // K slice shapes: (units per wave KU, waves KS) with KU * KS * 64 = K.  7 waves x 8 units at
 // K = 3,584 (14 x 4 measured the same for QKV and 0.45 µs slower for O at config 4).
-// Long K without such a shape (the down projection's 18,944 = 296 units): split-K over
+// Long K without such a shape (the down projection's 18,944 = 296 units), where dec8s_kernel does not take it: split-K over
 // parts of 8 waves x 4 units (10 parts at 18,944, the last one ragged; 128 VGPRs, two blocks
 // per CU), single-segment epilogues without a fused norm only (a norm needs the whole row in
 // one block).  Qwen2-7B, fp8, B = 8: the general skinny kernel 2,895 tok/s (down
