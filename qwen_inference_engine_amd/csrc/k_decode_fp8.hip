@@ -1148,7 +1148,7 @@ static bool dec8_shape(int64_t K, int* ku, int* ks) {
     return false;
 }
 static int dec8_split_parts(const qie_linear_args* a, int* ku) {
-    if (a->K % 64 != 0 || a->norm_w || a->epilogue == QIE_EPI_SWIGLU || a->seg_rows[1] > 0) return 0;
+    if (a->K % 64 != 0 || a->norm_w || a->epilogue == QIE_EPI_SWIGLU || a->seg_rows[0] != a->N) return 0;   // (weights, scales, bias of w[0] alone)
     if (a->N > (int64_t)kDec8MaxTiles * 16) return 0;   // the ticket array
     // (tiled weights can be read by this kernel only: the dev switch does not apply to them)
     if (!(a->flags & QIE_LINEAR_FP8_T16) && dev_env("QIE_DEC8_SPLIT", 1) == 0) return 0;
@@ -1221,8 +1221,7 @@ int dec8_linear(const qie_linear_args* a, hipStream_t st, bool* done) {
         p.seg_rows[0] = p.seg_rows[1] = p.seg_rows[2] = (int32_t)a->N;
         p.t01[0] = p.t01[1] = p.n_tiles;
     } else {
-        const int64_t r0 = a->seg_rows[0] > 0 ? a->seg_rows[0] : a->N;
-        const int64_t r1 = a->seg_rows[1];
+        const int64_t r0 = a->seg_rows[0], r1 = a->seg_rows[1];
         p.seg_rows[0] = (int32_t)r0;
         p.seg_rows[1] = (int32_t)(r1 > 0 ? r1 : 1);
         p.seg_rows[2] = (int32_t)std::max<int64_t>(1, a->N - r0 - r1);

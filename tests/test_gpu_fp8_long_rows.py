@@ -1,5 +1,7 @@
 """fp8 projections of long plain rows, up to 8 rows of X (k_decode_fp8.hip dec8s_kernel): uneven shares of K, a block's second tile, a ragged
 last tile, either layout of the weights, every epilogue, either number of X rows that a chunk carries."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -49,6 +51,46 @@ def test_long_rows(oracle, qlib, M, K, N, tiled):
     G.check(qlib.qie_keys_to_ids(G.p(keys), M, G.p(ids), None))
     for m in range(M):
         assert G.host(ids)[m] == oracle.argmax(np.ascontiguousarray(y[m, :N]))
+
+
+@pytest.mark.parametrize("tiled", [False, True])
+@pytest.mark.parametrize("M,K,r", [(2, 2176, (2048, 0, 1536)), (8, 2176, (2048, 0, 1536)), (2, 2176, (2048, 1024, 512)), (2, 2176, (0, 0, 3584)),
+                                   (8, 2176, (1024, 0, 512)), (2, 3584, (1024, 0, 512)), (2, 3584, (0, 0, 1536))])
+def test_weights_in_several_segments(oracle, qlib, M, K, r, tiled):
+    """Columns take weights, scales and biases of their own segment, whichever segments there are."""
+    N = sum(r)
+    x, res = rand_bf16(oracle, (M, K), seed=M), rand_bf16(oracle, (M, N), seed=5)
+    wf, b = rand_bf16(oracle, (N, K), 0.05, seed=N), rand_bf16(oracle, (N,), 0.1, seed=9)
+    at = np.concatenate([[0], np.cumsum(r)])
+    scale = np.repeat(np.float32([1.0, 2.0, 4.0]), r)   # segments of unlike size: unlike row scales
+    wf = oracle.f32_to_bf16(oracle.bf16_to_f32(wf) * scale[:, None])
+    parts = [_fp8_dev(qlib, wf[at[i]:at[i + 1]].copy()) if n else None for i, n in enumerate(r)]
+    dq = np.concatenate([p[1] for p in parts if p])
+    w = [(_tiled(qlib, p[0], n, K) if tiled else p[0]) if p else None for p, n in zip(parts, r)]
+    flags = _lib.QIE_LINEAR_FP8 | (_lib.QIE_LINEAR_FP8_T16 if tiled else 0)
+
+    def run(epi, biases):
+        y = G.dev(res.copy())
+        a = _lib.LinearArgsC()
+        dx = G.dev(x)
+        a.x, a.ldx, a.M, a.K, a.N, a.y, a.ldy, a.epilogue, a.flags = G.p(dx), K, M, K, N, G.p(y), N, epi, flags
+        a.w[0] = G.p(dx)   # (an empty first segment still has an address)
+        for i in range(3):
+            if r[i]:
+                a.w[i], a.seg_rows[i] = G.p(w[i]), r[i]
+            if r[i] and biases:
+                a.bias[i] = G.p(biases[i])
+        G.check(qlib.qie_linear(C.byref(a), None), "qie_linear")
+        return G.host_bf16(y)
+
+    size = _abs_scale(oracle, x, dq)
+    y = run(_lib.QIE_EPI_STORE, [G.dev(b[at[i]:at[i + 1]].copy()) if r[i] else None for i in range(3)])
+    G.assert_sum_close(y, oracle.matmul(x, dq, b), size, what="store")
+    got = oracle.bf16_to_f32(run(_lib.QIE_EPI_RESIDUAL, None)).astype(np.float64)
+    prod = oracle.bf16_to_f32(oracle.matmul(x, dq)).astype(np.float64)
+    want = oracle.bf16_to_f32(res) + prod
+    # a last bit of the product, and of the sum it goes into
+    assert (np.abs(got - want) <= np.maximum(2.0 ** -7 * (np.abs(prod) + np.abs(want)), 1e-5 * size)).all()
 
 
 def test_a_row_does_not_depend_on_its_neighbours(oracle, qlib):
