@@ -67,6 +67,7 @@ def test_weights_in_several_segments(oracle, qlib, M, K, r, tiled):
     parts = [_fp8_dev(qlib, wf[at[i]:at[i + 1]].copy()) if n else None for i, n in enumerate(r)]
     dq = np.concatenate([p[1] for p in parts if p])
     w = [(_tiled(qlib, p[0], n, K) if tiled else p[0]) if p else None for p, n in zip(parts, r)]
+    other = _fp8_dev(qlib, rand_bf16(oracle, (N, K), 1.0, seed=N + 1))[0]
     flags = _lib.QIE_LINEAR_FP8 | (_lib.QIE_LINEAR_FP8_T16 if tiled else 0)
 
     def run(epi, biases):
@@ -74,7 +75,7 @@ def test_weights_in_several_segments(oracle, qlib, M, K, r, tiled):
         a = _lib.LinearArgsC()
         dx = G.dev(x)
         a.x, a.ldx, a.M, a.K, a.N, a.y, a.ldy, a.epilogue, a.flags = G.p(dx), K, M, K, N, G.p(y), N, epi, flags
-        a.w[0] = G.p(dx)   # (an empty first segment still has an address)
+        a.w[0] = G.p(other)   # (an empty first segment still has an address, here of as many rows that are not to be read)
         for i in range(3):
             if r[i]:
                 a.w[i], a.seg_rows[i] = G.p(w[i]), r[i]
