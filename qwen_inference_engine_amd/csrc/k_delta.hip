@@ -295,7 +295,8 @@ __global__ __launch_bounds__(256) void delta_carry_kernel(DeltaCarryP p) {
 
 // dim 64 and 128: M times 32 state columns on the fp32 matrix cores (v_mfma_f32_16x16x4f32, a lane's four k from one 16-byte load), the next
 // piece's M and local state on their way meanwhile.  A wave owns 16 RT rows of the state, which all waves read from LDS, transposed.  The form
-// above goes to memory for M inside its sums and reads all of it for 8 columns.  us, 16 heads of 128 x 128: 4 entries of 30 pieces in all
+// above goes to memory for M inside its sums and reads all of it for 8 columns.  The products are summed from zero and join the local state in one
+// rounding, as there (in a chain from the local state the error was 3 to 11 times that).  us, 16 heads of 128 x 128: 4 entries of 30 pieces in all
 // 160 -> 49, 5 entries of 9 pieces 94 -> 32.
 typedef float dc_f32x4 __attribute__((ext_vector_type(4)));
 template <int DIM>
@@ -358,7 +359,7 @@ __global__ __launch_bounds__(256) void delta_carry_mfma_kernel(DeltaCarryP p) {
 #pragma unroll
         for (int i = 0; i < RT; i++)
 #pragma unroll
-            for (int j = 0; j < CT; j++) cur[i][j] = q.loc[i][j];
+            for (int j = 0; j < CT; j++) cur[i][j] = dc_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kk = 0; kk < KS; kk++) {
             dc_f32x4 b[CT];
@@ -371,6 +372,10 @@ __global__ __launch_bounds__(256) void delta_carry_mfma_kernel(DeltaCarryP p) {
 #pragma unroll
                     for (int j = 0; j < CT; j++) cur[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(q.m[i][kk][e], b[j][e], cur[i][j], 0, 0, 0);
         }
+#pragma unroll
+        for (int i = 0; i < RT; i++)
+#pragma unroll
+            for (int j = 0; j < CT; j++) cur[i][j] = cur[i][j] + q.loc[i][j];
     };
     Piece pa, pb;
     if (sp.y > 0) load(pa, 0);

@@ -49,3 +49,28 @@ def test_carry(qlib, dim, vdim, write):
         assert ((a.double() - b).abs() <= 1e-5 * (1 + b.abs())).all()
     if not write:
         assert torch.equal(got, state)
+
+
+@pytest.mark.parametrize("share", [1e-6, 1e-3, 1.0])
+@pytest.mark.parametrize("dim,vdim", [(64, 40), (128, 128), (96, 40)])
+def test_local_states_are_rounded_once(qlib, dim, vdim, share):
+    """A piece's products are summed by themselves and added to its local state in one rounding: a state of which little is left after a
+    piece (fast decay) costs the local state none of its bits."""
+    H, n = 2, 3
+    g = torch.Generator("cuda").manual_seed(dim)
+
+    def t(*shape):
+        return torch.randn(*shape, generator=g, device="cuda")
+    loc, trans, state = t(n, H, dim, vdim), share * dim ** -0.5 * t(n, H, dim, dim), t(1, H, dim, vdim)
+    sp, s_in, got = torch.tensor([(0, n, 0, 5)], dtype=torch.int32, device="cuda"), torch.zeros_like(loc), state.clone()
+    p = DeltaCarryP(sp.data_ptr(), 1, H, dim, vdim, loc.data_ptr(), trans.data_ptr(), s_in.data_ptr(), got.data_ptr(), H * dim * vdim, 0, 1)
+    torch.cuda.synchronize()
+    G.check(getattr(C.CDLL(_lib.load()._name), SYMBOL)(C.byref(p), None), "delta_carry")
+    torch.cuda.synchronize()
+    states = torch.cat([s_in, got])
+    assert torch.equal(states[0], state[0])
+    for k in range(n):   # each piece from the state that entered it
+        m, s = trans[k].double(), states[k].double()
+        want, size = torch.bmm(m, s) + loc[k].double(), torch.bmm(m.abs(), s.abs())
+        # dim fp32 roundings in the products' chain, each of at most their sum's size; one of the result
+        assert ((states[k + 1].double() - want).abs() <= 2.0 ** -24 * (1.001 * want.abs() + dim * size)).all()
