@@ -843,9 +843,11 @@ static int dec8_launch(const Dec8Params& p, hipStream_t st) {
 // meet through memory: a ticket, a drain and a second trip behind every launch, 3.6 TB/s.  Here a workgroup of 8 waves owns whole
 // 16-row tiles and every wave streams the 128-k chunks of its own share of K by LDS-DMA through a ring of its own, X's rows beside
 // the weights' (they come from L2; all of them do not fit LDS), with no barrier until the waves' partial tiles meet in LDS.
+// A wave's products are 8 sums (by chunk parity and 32-k step), which meet in pairs, as the waves' do: in one chain a wave, and the waves
+// in order, the result was up to 1.6 times as far from 64 bits as the split-K form's (9.6e-8 at K = 18,944; this one's 8.1e-8).
 // D = W Xᵀ: a lane ends with four neighbouring columns of one row.  XR: rows of X a chunk carries (X is as many bytes as the weights at
-// 8 rows, and they cost about 2 us).  us at 18,944 x 3,584, split-K form -> this one: 1 row 18.3 -> 13.5, 4 rows 19.2 -> 14.3, 8 rows
-// 19.7 -> 15.8 (weights read without the non-temporal hint: 14.7, -, 16.5); 16 rows 20.8 -> 22.7 and stay there.
+// 8 rows, and they cost about 2 us).  us at 18,944 x 3,584, split-K form -> this one: 1 row 18.5 -> 13.9, 4 rows 19.1 -> 14.7, 8 rows
+// 19.6 -> 16.9 (without the non-temporal hint on the weights 1.2 and 0.7 more); 16 rows 20.8 -> 22.7 and stay there.
 namespace d8s {
 constexpr int NW = 8;
 constexpr int CH = 128;         // k of a chunk
@@ -952,8 +954,8 @@ __global__ __launch_bounds__(512) void dec8s_kernel(Dec8Params p) {
     int done = 0, slot = 0;
     for (int it = 0; it < mine; it++) {
         const int tile = blockIdx.x + it * G;
-        d8_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        for (int c = 0; c < cnt; c++) {
+        d8_f32x4 even[4] = {}, odd[4] = {};
+        auto chunk = [&](d8_f32x4 (&acc)[4]) {
             // the oldest chunk has landed: R - 1 younger ones may fly (fewer at the end of the stream)
             if (done + R <= items) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(IPC * (R - 1)) : "memory");
             else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -972,15 +974,23 @@ __global__ __launch_bounds__(512) void dec8s_kernel(Dec8Params p) {
             for (int u = 0; u < 2; u++) {
                 const uint2 q0 = fp8x4_to_bf16x4(wf[u].x), q1 = fp8x4_to_bf16x4(wf[u].y);
                 const uint2 q2 = fp8x4_to_bf16x4(wf[u].z), q3 = fp8x4_to_bf16x4(wf[u].w);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(d8_bf16x8, d8_u32x4{q0.x, q0.y, q1.x, q1.y}), xf[2 * u], acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(d8_bf16x8, d8_u32x4{q2.x, q2.y, q3.x, q3.y}), xf[2 * u + 1], acc, 0, 0, 0);
+                acc[2 * u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(d8_bf16x8, d8_u32x4{q0.x, q0.y, q1.x, q1.y}), xf[2 * u], acc[2 * u], 0, 0, 0);
+                acc[2 * u + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(d8_bf16x8, d8_u32x4{q2.x, q2.y, q3.x, q3.y}), xf[2 * u + 1], acc[2 * u + 1], 0, 0, 0);
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the slot's reads are done
             __builtin_amdgcn_sched_barrier(0);
             if (done + R < items) issue(true);
             done++;
             slot = slot + 1 == R ? 0 : slot + 1;
+        };
+        for (int c = 0; c + 1 < cnt; c += 2) {
+            chunk(even);
+            chunk(odd);
         }
+        if (cnt & 1) chunk(even);
+#pragma unroll
+        for (int i = 0; i < 4; i++) even[i] = even[i] + odd[i];
+        const d8_f32x4 acc = (even[0] + even[1]) + (even[2] + even[3]);
         if (fr < 8) red[((it & 1) * d8s::NW + wave) * RS + rl] = acc;
         // one barrier a tile: a slot of `red` is written again two tiles on, behind the next tile's barrier, which the summing
         // wave reaches only after its reads.  (No vmcnt wait: the ring's loads stay in flight.)
@@ -989,9 +999,10 @@ __global__ __launch_bounds__(512) void dec8s_kernel(Dec8Params p) {
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
         if (wave != it % d8s::NW) continue;   // wave-uniform
-        d8_f32x4 v = red[(it & 1) * d8s::NW * RS + rl];
+        d8_f32x4 w[d8s::NW];
 #pragma unroll
-        for (int w = 1; w < d8s::NW; w++) v = v + red[((it & 1) * d8s::NW + w) * RS + rl];
+        for (int i = 0; i < d8s::NW; i++) w[i] = red[((it & 1) * d8s::NW + i) * RS + rl];
+        const d8_f32x4 v = ((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7]));
         if (it > 0) load_epi(tile, true);
         if (fr < M) {
             const int col = tile * 16 + 4 * g;

@@ -53,6 +53,22 @@ def test_long_rows(oracle, qlib, M, K, N, tiled):
         assert G.host(ids)[m] == oracle.argmax(np.ascontiguousarray(y[m, :N]))
 
 
+@pytest.mark.parametrize("K,N,bound", [(5120, 4096, 8.5e-8), (18944, 3584, 1.0e-7)])
+def test_sums_are_short(oracle, qlib, K, N, bound):
+    """The sums of a long row are many short ones that meet in pairs.  A rounding of a partial sum that holds the share s of the products
+    costs 0.41 * 2^-24 * sqrt(s) of the result on the average, and they add up in squares: 8 chains of K / 8,192 chunks a wave, 3 steps
+    of pairs there and 3 between the waves: 7 such units at K = 5,120, 11 at 18,944, 6.5e-8 and 8.1e-8; a chain over a wave's share has
+    14 and 42."""
+    M = 8
+    x = rand_bf16(oracle, (M, K), seed=1)
+    d, dq = _fp8_dev(qlib, rand_bf16(oracle, (N, K), 0.05, seed=2))
+    exact = oracle.bf16_to_f32(x).astype(np.float64) @ oracle.bf16_to_f32(dq).astype(np.float64).T
+    y = G.zeros((M, N), np.float32)
+    _linear(qlib, G.dev(x), [(_tiled(qlib, d, N, K), N)], [], M, K, N, y, _lib.QIE_EPI_F32, flags=_lib.QIE_LINEAR_FP8 | _lib.QIE_LINEAR_FP8_T16)
+    err = np.linalg.norm(G.host(y) - exact) / np.linalg.norm(exact)
+    assert err < bound
+
+
 @pytest.mark.parametrize("tiled", [False, True])
 @pytest.mark.parametrize("M,K,r", [(2, 2176, (2048, 0, 1536)), (8, 2176, (2048, 0, 1536)), (2, 2176, (2048, 1024, 512)), (2, 2176, (0, 0, 3584)),
                                    (8, 2176, (1024, 0, 512)), (2, 3584, (1024, 0, 512)), (2, 3584, (0, 0, 1536))])
