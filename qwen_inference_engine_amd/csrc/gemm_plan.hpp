@@ -81,6 +81,24 @@ inline int band_height(int n_mt, int bm, int bn, int at_once) {
     return (n_mt + bands - 1) / bands;
 }
 
+// ---------------------------------------------------------------- k_decode_fp8.hip, long rows
+namespace d8s {
+// Whole 16-row tiles a workgroup, one workgroup a CU (dec8s_kernel), or every tile split over `parts` of K.  Whole tiles read their weights
+// 10 to 35 % faster but go by rounds of the chip: not where they keep less than three quarters of it busy, nor where a last round is mostly
+// empty and K long, sooner with the 8 rows of X a chunk (M > 4) than with 4.  us, split / whole, M = 1 and 8: 17,408 x 4,608 (1.1 rounds)
+// 20.1 / 20.3 and 21.4 / 25.0, x 5,120 (1.25) 21.6 / 20.8 and 23.1 / 25.6, x 6,400 (1.6) 27.9 / 22.3 and 28.8 / 28.1; 9,728 x 4,608 14.0 / 15.1 at 8
+// rows; 5,120 x 5,120 9.9 / 8.6 and 10.6 / 10.3; 2,560 x 4,608 7.2 / 6.1 and 8.7 / 6.7.  The split form has at most 7 tiles a workgroup and two
+// workgroups a CU: from 14 sums a CU on they no longer run at once and it takes a third longer.
+inline bool whole_tiles(int64_t M, int64_t K, int64_t tiles, int64_t parts, int64_t cus) {
+    if (tiles * 4 < cus * 3) return false;
+    if (tiles <= cus || K <= 2560 || (K <= 5120 && tiles <= 2 * cus)) return true;
+    const int64_t rounds = (tiles + cus - 1) / cus;
+    const bool crowded = parts * tiles >= 14 * cus;
+    if (M <= 4) return crowded || 10 * rounds * cus <= 16 * tiles;
+    return 10 * rounds * cus <= (crowded ? 14 : tiles <= 2 * cus ? 13 : 12) * tiles;
+}
+}  // namespace d8s
+
 // ---------------------------------------------------------------- k_gemm_mid.hip
 namespace mid {
 constexpr int BK = 64;

@@ -26,6 +26,7 @@
 // Numerics: the dequantised products (e4m3 × 2^k is exact in bf16) accumulate in fp32 per
 // wave over its K slice, the KS slices are added in wave order, times the row scale; the
 // epilogues round exactly as the reference's separate kernels (bf16 after each op).
+#include "gemm_plan.hpp"
 #include "qie_common.hpp"
 #include "../../include/qie/qie_ops.h"
 
@@ -1057,10 +1058,9 @@ static int dec8s(const Dec8Params& p, int epi, hipStream_t st) {
         default: return dec8s_rows<QIE_EPI_STORE, T16>(p, st);
     }
 }
-// Where the tiles keep most CUs busy (below that the split-K form spreads K over the others), up to 8 rows.
-static bool dec8s_applies(const qie_linear_args* a) {
-    const int64_t tiles = (a->N + 15) / 16;
-    return a->M <= 8 && a->K % d8s::CH == 0 && a->K / d8s::CH >= d8s::NW && tiles * 4 >= device_cu_count() * 3 &&
+// Up to 8 rows, where whole tiles are the faster.  parts: of the split-K form.
+static bool dec8s_applies(const qie_linear_args* a, int parts) {
+    return a->M <= 8 && a->K % d8s::CH == 0 && a->K / d8s::CH >= d8s::NW && d8s::whole_tiles(a->M, a->K, (a->N + 15) / 16, parts, device_cu_count()) &&
            a->M * a->ldx < 1 << 30 && a->M * a->ldy < 1 << 29;   // 32-bit offsets
 }
 
@@ -1244,7 +1244,7 @@ int dec8_linear(const qie_linear_args* a, hipStream_t st, bool* done) {
     int ku = 0, ks = 0;
     if (!dec8_shape(a->K, &ku, &ks)) {
         p.parts = dec8_split_parts(a, &ku);
-        if (dec8s_applies(a)) return t16 ? dec8s<true>(p, a->epilogue, st) : dec8s<false>(p, a->epilogue, st);
+        if (dec8s_applies(a, p.parts)) return t16 ? dec8s<true>(p, a->epilogue, st) : dec8s<false>(p, a->epilogue, st);
         if (!dec8_workspace(st, &p)) {
             *done = false;
             return 0;
