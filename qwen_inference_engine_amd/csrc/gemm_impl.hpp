@@ -176,6 +176,6 @@ void g8_release(hipStream_t st);
 
 // k_gemm_mid.hip: the GEMM of a few dozen to about a thousand rows.  other_us: the expected time of the caller's kernel for
 // this shape; *launched = false: not a shape for this one, or the other is expected to be faster.
-int gemm_mid(const qie_linear_args* a, const GemmParams& q, float other_us, hipStream_t st, bool* launched);
+int gemm_mid(const qie_linear_args* a, const GemmParams& p, hipStream_t st, bool* launched);
 
 }  // namespace qie

@@ -64,7 +64,7 @@ QIE_PLAN_HD inline int quotient(int a, int b) {
 // Workgroup numbers run down bands of `gm` row tiles, column tile by column tile: the workgroups that an XCD runs at a time (32 CUs,
 // neighbours in number) cover about as many rows as columns, which is the least that its L2 has to fetch for them.  One band of all
 // row tiles fetched A anew for every column tile.  Qwen2-7B at 8,192 rows, one band / bands: gate and up 1,800 / 1,690 us, down
-// 950 / 885, QKV 263 / 256, O 234 / 228; Qwen2-0.5B down at 6,000 rows 68 / 60.  Up to 8 row tiles are one band as before.
+// 950 / 885, QKV 263 / 256, O 234 / 228 (256x256 tiles); Qwen2-0.5B down at 6,000 rows 68 / 60.
 QIE_PLAN_HD inline void banded(int wid, int n_mt, int n_nt, int gm, int* mt, int* nt) {
     const int band = gm * n_nt, b = quotient(wid, band), at = wid - b * band;
     const int h = n_mt - b * gm < gm ? n_mt - b * gm : gm, c = quotient(at, h);
@@ -72,8 +72,8 @@ QIE_PLAN_HD inline void banded(int wid, int n_mt, int n_nt, int gm, int* mt, int
     *nt = c;
 }
 
-// height of even bands, up to about twice as tall as wide (`at_once` tiles of bm x bn outputs): fewer bands read the weights less often,
-// and bands of 4 row tiles of 256 x 128 where 8 or 12 fit one band lost 4 %
+// height of even bands, up to about twice as tall as wide (`at_once` tiles of bm x bn outputs) and then as many as the row tiles hold whole, so
+// up to twice that: fewer bands read the weights less often, and bands of 4 row tiles of 256 x 128 where 8 or 12 fit one band lost 4 %
 inline int band_height(int n_mt, int bm, int bn, int at_once) {
     int h = 1;
     while ((h + 1) * (h + 1) * bm <= 2 * at_once * bn) h++;
@@ -99,6 +99,45 @@ inline bool whole_tiles(int64_t M, int64_t K, int64_t tiles, int64_t parts, int6
 }
 }  // namespace d8s
 
+// ---------------------------------------------------------------- k_gemm.hip, 256x256 kernel
+namespace g8p {
+// parts per tile: the fewest rounds of (tile, part) items over the CUs, in units of a tile
+// (112 tiles: 2 parts = one round of half tiles; 144 tiles: 3 parts, two rounds of thirds)
+// (short parts lose: QKV at 3 x 19 and O at 2 x 28 k-tiles measured 108 -> 112 and 71 -> 69 us,
+// the last arriver's serial slab read and the per-part pipeline fill eat the gain; down at
+// 2 x 148: 309 -> 247 us), so a part keeps >= 64 k-tiles (mink): split-K 2 for the O projection at 2,048 rows (112 tiles
+// -> 224, K = 3,584) ran 94-98 vs 84 us for the 256x128 kernel; QKV at 3 parts 114 vs 89
+inline int splitk(int64_t tiles, int64_t cus, int nk, int mink = 64) {
+    int best = 1;
+    double best_t = 1e30;
+    for (int s = 1; s <= 4 && nk / s >= mink; s++) {
+        const double t = (double)((tiles * s + cus - 1) / cus) / s;
+        if (t < best_t - 1e-9) {
+            best_t = t;
+            best = s;
+        }
+    }
+    return best;
+}
+// Parts per tile of a product of M rows and nk k-tiles of 64: 1 where the tiles fill the chip; 0: not its launch.  Unsplit, the tiles must
+// cover half the chip: QKV at 144 tiles 101.7 -> 87.8 us, but O at 112 tiles 78 -> 103 us (its 256x128 kernel fills 224 CUs).
+inline int parts(int64_t M, int64_t cols, int64_t K, int64_t cus, int mink = 64) {
+    if (M < 256 || K % 64 != 0 || K < 256) return 0;
+    const int64_t tiles = ((M + 255) / 256) * ((cols + 255) / 256);
+    if (tiles >= cus) return 1;
+    const int s = splitk(tiles, cus, (int)(K / 64), mink);
+    return s == 1 && 2 * tiles < cus ? 0 : s;
+}
+// expected time, us: 1.45 a k-tile and 5 a round of the chip (fitted as k_gemm_mid.hip's tiles; over 20 projections at 256 to 8,192 rows
+// the kernel now takes 2 % less on the average, 0.84 to 1.24 of this)
+inline float us(int64_t M, int64_t cols, int64_t K, int64_t cus) {
+    const int s = parts(M, cols, K, cus);
+    if (s == 0) return 1e30f;
+    const int64_t tiles = ((M + 255) / 256) * ((cols + 255) / 256), nk = K / 64;
+    return (float)((tiles * s + cus - 1) / cus) * (nk / (float)s * 1.45f + 5.f) + 5.f + (s > 1 ? 8.f * s : 0.f);
+}
+}  // namespace g8p
+
 // ---------------------------------------------------------------- k_gemm_mid.hip
 namespace mid {
 constexpr int BK = 64;
@@ -123,9 +162,9 @@ constexpr Tile TILES[] = {
 constexpr int N_TILES = sizeof(TILES) / sizeof(TILES[0]);
 // Tiles of 160 columns, numbered on from TILES: where the columns of 128-column tiles start a round of the chip that they hardly fill
 // (37,888 columns: 296 tiles, 237 of these), and so many rows of the workgroups' own (weights) that a tile of fewer columns loads more
-// for the same outputs.  Whole only.  Fitted to rounds that are nearly full.
+// for the same outputs.  Whole only.
 constexpr Tile WIDE[] = {
-    {128, 160, 4, 1, 3.f, 1.f, 14.3f, -1.3f, .69f}, {192, 160, 3, 1, 6.6f, 1.1f, 7.1f, 6.3f, .825f},
+    {128, 160, 4, 1, 3.f, 1.f, 11.7f, 0.f, .69f}, {192, 160, 3, 1, 6.6f, 1.1f, 7.1f, 6.3f, .825f},
     {256, 160, 3, 1, 8.8f, 1.29f, 0.f, 10.f, 1.f}, {320, 160, 2, 1, 9.6f, 1.56f, 0.f, 13.f, 1.17f},
 };
 constexpr int N_WIDE = sizeof(WIDE) / sizeof(WIDE[0]);
@@ -171,18 +210,36 @@ inline Plan plan(int64_t M, int64_t cols, int64_t K, int64_t cus) {
     return best;
 }
 
-// The plan among tiles of 160 columns.
+// The plan among tiles of 160 columns.  Which tiles it takes were measured against plan()'s and the 256x256 kernel on 20 projections (Qwen2-0.5B,
+// 1.5B and 7B, Qwen3-14B, and 2,048, 4,096 wide ones) at 72 to 8,192 rows.  Up to two rounds of the chip (320 rows: one): 0.72 to
+// 1.01 of their time, 0.88 on the average of the 73 shapes in 676 that it takes.  In more rounds each column tile's weights come as often as there
+// are row tiles and the others win: Qwen2-0.5B gate / up at 1,600 rows 47.5 us | 59.4 (128 x 160, 3.1 rounds), Qwen2-7B gate / up at 640 rows 166.7 | 179.1
+// (320 x 160, 1.9), Qwen3-14B down at 8,192 1,122 | 1,274 (256 x 160, 4), 5,120 718 | 792 (320 x 160, 2).  Except 320 rows x 160 over many row tiles
+// (2,000 rows on) whose A stays in the Infinity Cache: Qwen2-7B QKV at 8,192 rows 249.0 | 240.3, O at 6,000 175.5 | 167.5, Qwen3-14B QKV at 7,000 448 | 435.
 inline Plan plan_wide(int64_t M, int64_t cols, int64_t K, int64_t cus) {
     Plan best{-1, 0, 1, 0, 0, 1e30f};
     const int nk = (int)(K / BK);
+    const float floor_us = (float)cols * K * 2 / 5.3e6f + 4.f;   // as in plan()
     for (int c = 0; c < N_WIDE; c++) {
         const Tile& t = WIDE[c];
         const int64_t n_mt = (M + t.bm - 1) / t.bm, n_nt = (cols + t.bn - 1) / t.bn, tiles = n_mt * n_nt;
-        if (tiles > (1 << 22)) continue;
-        const float us = tiles <= cus ? t.a1 + nk * t.s1 : t.a2 + rounds(tiles / (float)cus) * (t.f2 + nk * t.s2);
+        const int64_t most = t.bm < 320 ? 2 : M >= 2048 && M * K * 2 <= 80000000 ? 4 : 1;   // rounds
+        if (tiles > most * cus) continue;
+        const float us = std::max(floor_us, tiles <= cus ? t.a1 + nk * t.s1 : t.a2 + rounds(tiles / (float)cus) * (t.f2 + nk * t.s2));
         if (us < best.us) best = {N_TILES + c, (int)tiles, 1, (int)n_mt, (int)n_nt, us};
     }
     return best;
+}
+
+// The tiles that take a product; tile -1: none, k_gemm.hip's kernels do.
+inline Plan choose(int64_t M, int64_t cols, int64_t K, int64_t cus) {
+    const Plan none{-1, 0, 1, 0, 0, 1e30f};
+    if (K % BK != 0) return none;   // (rows of x and weights are on the 16-byte grid of LDS-DMA: qie_linear)
+    const float other_us = g8p::us(M, cols, K, cus);
+    const Plan pl = plan(M, cols, K, cus), wide = plan_wide(M, cols, K, cus);
+    // (split plans of gate / up's many columns take 10 to 30 % longer than the fit says)
+    if (M > 64 && wide.tile >= 0 && wide.us < (pl.splitk > 1 ? 1.1f : 1.f) * pl.us && wide.us < .97f * other_us) return wide;
+    return pl.tile >= 0 && pl.us < .88f * other_us ? pl : none;   // 12 %: what the two fits are off by on long prompts
 }
 }  // namespace mid
 

@@ -1064,36 +1064,6 @@ static int launch_gemm8sk(int epi, const GemmParams& p, int n_mt, int tiles, hip
     return launch_gemm8sk_t<QIE_EPI_STORE>(p, n_mt, grid, sk, st);
 }
 
-// parts per tile: the fewest rounds of (tile, part) items over the CUs, in units of a tile
-// (112 tiles: 2 parts = one round of half tiles; 144 tiles: 3 parts, two rounds of thirds)
-// (short parts lose: QKV at 3 x 19 and O at 2 x 28 k-tiles measured 108 -> 112 and 71 -> 69 us,
-// the last arriver's serial slab read and the per-part pipeline fill eat the gain; down at
-// 2 x 148: 309 -> 247 us), so a part keeps >= 64 k-tiles
-static int g8_splitk(int64_t tiles, int64_t cus, int nk) {
-    int best = 1;
-    double best_t = 1e30;
-    // k-tiles per part at least QIE_GEMM8_SK_MINK (dev A/B; default 64: K >= 4,096 per part).
-    // Split-K 2 for the O projection at P = 2,048 (112 tiles -> 224, K = 3,584) ran
-    // 94-98 vs 84 µs for the 256x128 kernel; QKV at 3 parts 114 vs 89 — the slab round trip
-    // costs more than the idle CUs at this K
-    const int mink = std::max(4, dev_env("QIE_GEMM8_SK_MINK", 64));
-    for (int s = 1; s <= 4 && nk / s >= mink; s++) {
-        const double t = (double)((tiles * s + cus - 1) / cus) / s;
-        if (t < best_t - 1e-9) {
-            best_t = t;
-            best = s;
-        }
-    }
-    return best;
-}
-
-// expected time of gemm8_kernel, us: 1.45 a k-tile and 5 a round of the chip (fitted as k_gemm_mid.hip's tiles)
-static float g8_us(int64_t tiles, int64_t cus, int nk) {
-    const int s = tiles < cus ? g8_splitk(tiles, cus, nk) : 1;
-    if (s == 1 && 2 * tiles < cus) return 1e30f;   // not its launch (gemm() below)
-    return (float)cdiv(tiles * s, cus) * (nk / (float)s * 1.45f + 5.f) + 5.f + (s > 1 ? 8.f * s : 0.f);
-}
-
 template <int EPI, int BNT>
 static int launch_gemm_big_t(const GemmParams& p, int n_mt, int n_tiles, hipStream_t st) {
     const void* fn = (const void*)gemm_big_kernel<EPI, BNT>;
@@ -1566,7 +1536,7 @@ static int gemm_with(const qie_linear_args* a, const QkvTail* tail, bool* done, 
     QIE_REQUIRE(a->K % 8 == 0, "qie_linear: GEMM needs K %% 8 == 0");
     if (!(a->flags & QIE_LINEAR_FP8) && a->K % big::BK == 0 && a->ldx % 8 == 0) {
         // In this order:
-        //   1. K a multiple of 64: k_gemm_mid.hip, unless the next is expected to be faster (g8_us);
+        //   1. K a multiple of 64: k_gemm_mid.hip, unless the next is expected to be faster (mid::choose);
         //   2. K a multiple of 64 from 256 on, 256 rows: the phase-interleaved 256x256 kernel, whole where its tiles fill the chip,
         //      or half of it when K is too short to split; split over K otherwise;
         //   3. K an odd multiple of 32, or a split that gets no memory for its slabs, 256 rows: the LDS-DMA kernel, with 256x256 tiles
@@ -1587,7 +1557,7 @@ static int gemm_with(const qie_linear_args* a, const QkvTail* tail, bool* done, 
         if (dev_env("QIE_MID", 1) && force < 0 && !(a->flags & QIE_LINEAR_STREAMK)) {
             bool launched = false;
             if (tail) p.qkv = *tail;
-            const int rc = gemm_mid(a, p, g8ok && a->M >= big::BM ? g8_us(t256, cus, (int)(a->K / g8::BK)) : 1e30f, st, &launched);
+            const int rc = gemm_mid(a, p, st, &launched);
             if (done) *done = launched && tail;
             if (rc || launched) return rc;
         }
@@ -1604,11 +1574,9 @@ static int gemm_with(const qie_linear_args* a, const QkvTail* tail, bool* done, 
             return launch_gemm8(a->epilogue, p, (int)n_mt, (int)t256, sk, st);
         }
         if (g8ok && g8mode == 2 && force < 0 && a->M >= big::BM && t256 < cus) {
-            const int s = g8_splitk(t256, cus, (int)(a->K / g8::BK));
+            const int s = g8p::parts(a->M, cols, a->K, cus, std::max(4, dev_env("QIE_GEMM8_SK_MINK", 64)));   // (dev A/B: k-tiles a part)
             G8Split sk{1, nullptr, nullptr};
-            // unsplit, 256x256 tiles must still cover half the chip: QKV at 144 tiles 101.7 ->
-            // 87.8 us, but O at 112 tiles 78 -> 103 us (its 256x128 kernel fills 224 CUs)
-            if ((s == 1 && 2 * t256 >= cus) || (s > 1 && g8_workspace(st, (int)t256 * s, (int)t256, &sk) == 0 && (sk.splitk = s) > 1)) {
+            if (s == 1 || (s > 1 && g8_workspace(st, (int)t256 * s, (int)t256, &sk) == 0 && (sk.splitk = s) > 1)) {
                 if (done) *done = p.qkv.q != nullptr;
                 return launch_gemm8(a->epilogue, p, (int)n_mt, (int)t256, sk, st);
             }

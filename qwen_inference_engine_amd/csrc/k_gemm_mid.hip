@@ -325,18 +325,10 @@ int launch_mid(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, hipS
 }
 }  // namespace
 
-// other_us: what the caller's other kernel for this shape takes
-int gemm_mid(const qie_linear_args* a, const GemmParams& q, float other_us, hipStream_t st, bool* launched) {
+int gemm_mid(const qie_linear_args* a, const GemmParams& p, hipStream_t st, bool* launched) {
     *launched = false;
-    const GemmParams& p = q;
-    if (a->K % mid::BK != 0) return 0;   // (rows of x and weights are on the 16-byte grid of LDS-DMA: qie_linear)
-    const int64_t cols = a->epilogue == QIE_EPI_SWIGLU ? 2 * a->N : a->N;
-    mid::Plan pl = mid::plan(a->M, cols, a->K, device_cu_count());
-    const mid::Plan wide = mid::plan_wide(a->M, cols, a->K, device_cu_count());
-    // (split plans of gate / up's many columns take 10 to 30 % longer than the fit says)
-    const bool to_wide = a->M > 64 && wide.us < (pl.splitk > 1 ? 1.1f : 1.f) * pl.us && wide.us < 0.97f * other_us;
-    if (to_wide) pl = wide;
-    if (pl.tile < 0 || (!to_wide && pl.us >= 0.88f * other_us)) return 0;   // 12 %: what the two fits are off by on long prompts
+    const mid::Plan pl = mid::choose(a->M, a->epilogue == QIE_EPI_SWIGLU ? 2 * a->N : a->N, a->K, device_cu_count());
+    if (pl.tile < 0) return 0;
     G8Split sk{1, nullptr, nullptr};
     const int64_t cut = (int64_t)pl.n_mt * pl.n_nt - pl.whole;
     if (pl.splitk > 1 && cut > 0) {

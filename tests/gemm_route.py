@@ -1,0 +1,32 @@
+"""The GEMM dispatch's host rules (csrc/gemm_plan.hpp), compiled with the host compiler: which kernel and tile a product takes."""
+import os
+import subprocess
+import tempfile
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "qwen_inference_engine_amd", "csrc")
+
+DRIVER = r"""
+#include "gemm_plan.hpp"
+#include <cstdio>
+int main() {
+    long M, cols, K, cus;
+    while (std::scanf("%ld %ld %ld %ld", &M, &cols, &K, &cus) == 4) {
+        const qie::mid::Plan p = qie::mid::choose(M, cols, K, cus), w = qie::mid::plan_wide(M, cols, K, cus);
+        std::printf("%d %d %d %d %d %.9g\n", p.tile, p.n_mt * p.n_nt, p.splitk, qie::g8p::parts(M, cols, K, cus), w.tile, w.us);
+    }
+}
+"""
+
+
+def routes(cases, cus=256):
+    """For every (rows, weight rows, K): {tile (numbers of mid::TILES and mid::WIDE, -1: none of k_gemm_mid.hip's), tiles, splitk, parts
+    (of the 256x256 kernel, 0: not its launch; taken where tile is -1), wide (the best 160-column tile), wide_us}."""
+    with tempfile.TemporaryDirectory() as d:
+        src, exe = os.path.join(d, "drive.cpp"), os.path.join(d, "drive")
+        with open(src, "w") as f:
+            f.write(DRIVER)
+        subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, src, "-o", exe], check=True)
+        text = "\n".join("%d %d %d %d" % (*c, cus) for c in cases)
+        out = subprocess.run([exe], input=text, text=True, capture_output=True, check=True).stdout
+    names = ("tile", "tiles", "splitk", "parts", "wide", "wide_us")
+    return [dict(zip(names, [int(v) for v in line.split()[:5]] + [float(line.split()[5])])) for line in out.splitlines()]

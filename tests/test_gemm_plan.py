@@ -5,6 +5,7 @@ import subprocess
 
 import pytest
 
+from gemm_route import routes
 from test_gpu_gemm_mid import GROWS, PLANS
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "qwen_inference_engine_amd", "csrc")
@@ -76,6 +77,49 @@ def test_gemm_mid_plans_are_sound(plan):
     for (M, N, K, cus), (tile, whole, splitk, tiles) in zip(cases, plan(["m %d %d %d %d" % c for c in cases])):
         assert tile in range(8) and 1 <= splitk <= min(12, K // 64) and 0 <= whole <= tiles
         assert whole == tiles if splitk == 1 else whole < tiles and whole % cus == 0
+
+
+# rows, weight rows, K, us of the best of the other tiles and the 256x256 kernel, of the 160-column tiles 8 to 11
+MEASURED = [
+    (400, 9728, 896, 18.1, [16.9, 21.1, 24.8, 29.8]),
+    (1024, 9728, 896, 30.6, [30.8, 39.7, 26.3, 31.2]),
+    (1600, 9728, 896, 47.5, [59.4, 57.1, 48.0, 57.4]),
+    (3500, 9728, 896, 91.7, [105.2, 98.9, 96.7, 88.6]),
+    (100, 37888, 3584, 69.7, [57.5, 62.8, 71.6, 81.8]),
+    (300, 37888, 3584, 122.1, [122.3, 110.7, 129.8, 96.1]),
+    (512, 37888, 3584, 168.9, [173.9, 164.5, 135.5, 161.9]),
+    (640, 37888, 3584, 166.7, [215.4, 213.9, 193.0, 179.1]),
+    (960, 37888, 3584, 252.5, [328.6, 272.9, 261.0, 260.7]),
+    (640, 28672, 4096, 162.0, [192.0, 182.6, 213.0, 190.1]),
+    (640, 34816, 5120, 225.3, [304.4, 295.5, 266.5, 245.4]),
+    (4096, 4608, 3584, 159.1, [166.0, 156.0, 133.8, 155.4]),
+    (8192, 4608, 3584, 249.0, [331.3, 266.4, 254.2, 240.3]),
+    (6000, 3584, 3584, 175.5, [210.6, 168.2, 198.5, 167.5]),
+    (7000, 7168, 5120, 448.3, [546.7, 495.9, 460.0, 435.0]),
+    (6000, 3584, 18944, 771.5, [1003.8, 773.8, 917.7, 832.8]),
+    (5120, 5120, 17408, 717.9, [960.6, 959.8, 886.6, 791.8]),
+    (8192, 5120, 17408, 1121.6, [1566.4, 1467.3, 1274.1, 1598.9]),
+]
+
+
+def test_160_columns_where_they_are_no_slower():
+    """A product takes such a tile only where its time was at most 1 % above that of the kernels that it would take otherwise."""
+    got = routes([c[:3] for c in MEASURED])
+    for (M, N, K, other, wide), r in zip(MEASURED, got):
+        assert r["tile"] < 8 or wide[r["tile"] - 8] <= 1.012 * other, (M, N, K, r)
+    taken = [r["tile"] for r in got if r["tile"] >= 8]
+    assert len(taken) >= 8 and set(taken) == {8, 10, 11}
+
+
+def test_160_columns_have_sound_plans():
+    """Their times never fall below the weights' at the rate that they stream, however short K, and few rounds of the chip."""
+    r = random.Random(4)
+    cases = [(int(2 ** r.uniform(6, 17)), int(2 ** r.uniform(3, 17)), 64 * int(2 ** r.uniform(0, 9))) for _ in range(3000)] + [(50000, 4096, 64), (100000, 4096, 64), (100000, 4096, 128)]
+    for (M, N, K), p in zip(cases, routes(cases)):
+        if p["wide"] >= 0:
+            bm = (128, 192, 256, 320)[p["wide"] - 8]
+            rounds = -(-M // bm) * -(-N // 160) / 256
+            assert p["wide_us"] >= 2 * N * K / 5.3e6 + 3.99 and rounds <= (2 if bm < 320 else 1 if M < 2048 or 2 * M * K > 8e7 else 4)
 
 
 @pytest.mark.parametrize("seed", range(6))

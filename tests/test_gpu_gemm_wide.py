@@ -1,42 +1,26 @@
 """The GEMM's tiles of 160 columns (k_gemm_mid.hip) through qie_linear: shapes whose plan takes each of them, in one round of the chip
 and in more, with ragged rows and columns; every epilogue (a wave's slice has an odd number of fragments, and the waves' shares of a
 k-tile's rows differ); odd columns."""
-import ctypes as C
-import os
-import subprocess
-
 import numpy as np
 import pytest
 
 import gpu_util as G
+from gemm_route import routes
 from qwen_inference_engine_amd import _lib
 from test_gpu_gemm_mid import bf16, linear, products
 
-CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "qwen_inference_engine_amd", "csrc")
-# rows, columns, K -> tile
-SHAPES = [(100, 38002, 512, 8), (129, 37890, 1024, 9), (200, 37891, 1024, 10), (301, 37900, 1024, 11), (450, 37890, 512, 8), (450, 37890, 2048, 10)]
-
-DRIVER = r"""
-#include "gemm_plan.hpp"
-#include <cstdio>
-int main() {
-    long M, N, K;
-    while (std::scanf("%ld %ld %ld", &M, &N, &K) == 3) {
-        const qie::mid::Plan w = qie::mid::plan_wide(M, N, K, 256), p = qie::mid::plan(M, N, K, 256);
-        std::printf("%d %d %d %d %d\n", w.tile, w.whole, w.n_mt * w.n_nt, w.splitk, (int)(M > 64 && w.us < (p.splitk > 1 ? 1.1f : 1.f) * p.us));
-    }
-}
-"""
+# rows, columns, K -> tile: each in one round of the chip and in more
+SHAPES = [(100, 38002, 512, 8), (129, 37890, 1024, 9), (200, 37891, 1024, 10), (301, 37900, 1024, 11), (65, 58373, 1024, 8), (352, 32835, 512, 9),
+          (450, 37890, 2048, 10), (195, 49518, 512, 10), (2856, 6506, 1024, 11)]
+EPILOGUE_ROWS, EPILOGUE_K, EPILOGUE_N = [100, 129, 200, 301], 512, 37900
 
 
-def test_shapes_take_every_wide_tile(tmp_path):
-    (tmp_path / "drive.cpp").write_text(DRIVER)
-    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(tmp_path / "drive.cpp"), "-o", str(tmp_path / "drive")], check=True)
-    text = "\n".join("%d %d %d" % s[:3] for s in SHAPES)
-    out = subprocess.run([str(tmp_path / "drive")], input=text, text=True, capture_output=True, check=True).stdout
-    got = [[int(v) for v in line.split()] for line in out.splitlines()]
-    assert [g[0] for g in got] == [s[3] for s in SHAPES] and set(g[0] for g in got) == {8, 9, 10, 11}
-    assert all(g[1] == g[2] and g[3] == 1 and g[4] for g in got)
+def test_shapes_take_every_wide_tile():
+    got = routes([s[:3] for s in SHAPES])
+    assert [g["tile"] for g in got] == [s[3] for s in SHAPES]
+    assert {(g["tile"], g["tiles"] > 256) for g in got} == {(t, more) for t in (8, 9, 10, 11) for more in (False, True)}
+    got = routes([(M, n, EPILOGUE_K) for n in (EPILOGUE_N, EPILOGUE_N + 2) for M in EPILOGUE_ROWS])   # (odd SwiGLU: two weight rows more)
+    assert [g["tile"] for g in got] == 2 * [8, 9, 10, 11]
 
 
 @pytest.mark.gpu
@@ -51,10 +35,10 @@ def test_products(qlib, M, N, K, tile):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M", [100, 129, 200, 301])
+@pytest.mark.parametrize("M", EPILOGUE_ROWS)
 @pytest.mark.parametrize("epi", ["store", "residual", "swiglu", "swiglu odd"])
 def test_epilogues(qlib, oracle, M, epi):
-    K, N = 512, 37900
+    K, N = EPILOGUE_K, EPILOGUE_N
     x = bf16((M, K), 1.0, 3)
     if epi == "store":
         n = (30000, 5002, 2898)   # the bias changes inside a vector of four columns
