@@ -1,6 +1,8 @@
 // gemm_impl.hpp — what the prefill GEMMs share (k_gemm.hip, k_gemm_mid.hip): operands, LDS-DMA, the split-K workspace.
 #pragma once
 
+#include <type_traits>
+
 #include "qie_common.hpp"
 #include "../../include/qie/qie_ops.h"
 #include "split_pool.hpp"
@@ -14,7 +16,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // What follows a QKV projection of prompts laid end to end, each from position 0 on, without q / k norms and with rotary pairs
 // (2 i, 2 i + 1): q and k turned, q to its rows, k and v to the cache (qkv_post_kernel's results)
 struct QkvTail {
-    uint16_t* q;             // [M][qd]; null: no such tail
+    uint16_t* q;             // [M][qd]
     uint16_t *k, *v;         // the layer's first run
     const float* turns;      // [position][hd / 2][cos, sin]
     int len;                 // rows of a prompt
@@ -23,6 +25,11 @@ struct QkvTail {
     KvMap km;
 };
 constexpr int kEpiQkv = 4;   // the epilogue that does this: k_gemm.hip's 256x256 kernel and k_gemm_mid.hip's have it
+// The last argument of kernels with an epilogue EPI.  As part of every kernel's it moved what lies behind it (the grid's size) to a further line
+// of the argument segment: 0.3 us in each launch.
+struct NoTail {};
+template <int EPI>
+using TailOf = std::conditional_t<EPI == kEpiQkv, QkvTail, NoTail>;
 
 struct GemmParams {
     const uint16_t* A;
@@ -39,7 +46,6 @@ struct GemmParams {
     uint16_t* C;
     int64_t ldc;
     int vec = 0;         // rows of C take 4-element vector stores
-    QkvTail qkv{};
 };
 
 __device__ __forceinline__ void glds16(const void* src, void* lds) {
@@ -102,8 +108,7 @@ struct QkvOps {
     float4 turn[NI];
 };
 template <int NI>
-__device__ __forceinline__ void qkv_load(const GemmParams& p, int64_t row0, int64_t col, QkvOps<NI>& o) {
-    const QkvTail& t = p.qkv;
+__device__ __forceinline__ void qkv_load(const GemmParams& p, const QkvTail& t, int64_t row0, int64_t col, QkvOps<NI>& o) {
     const int hd = 1 << t.hd_log2, at = (int)(col < p.N ? col : p.N - 4);
     o.bias[0] = o.bias[1] = o.bias[2] = o.bias[3] = 0.f;
     quad_bias(p, at, o.bias);
@@ -118,10 +123,9 @@ __device__ __forceinline__ void qkv_load(const GemmParams& p, int64_t row0, int6
 // cost a launch.  A layer with this is shorter by: Qwen2-0.5B at 113 rows 2.6 us, Qwen2-7B at 301 rows 5.0, at 2,048 rows 6.3 (there the
 // epilogue takes some of it back: with the two tables apart, twice the loads, nothing was left), at 8,192 rows nothing.
 template <int NI, int NJ, bool EARLY>
-__device__ __forceinline__ void qkv_tail(const GemmParams& p, int64_t row0, int64_t col0, const f32x4 (&acc)[NI][NJ],
+__device__ __forceinline__ void qkv_tail(const GemmParams& p, const QkvTail& t, int64_t row0, int64_t col0, const f32x4 (&acc)[NI][NJ],
                                          const QkvOps<NI> (&early)[EARLY ? NJ : 1]) {
 #pragma clang fp contract(off)
-    const QkvTail& t = p.qkv;
     const int hd = 1 << t.hd_log2, turned = t.qd + t.kd;
     int64_t kv[NI];   // where the row's token lies in a run
 #pragma unroll
@@ -135,7 +139,7 @@ __device__ __forceinline__ void qkv_tail(const GemmParams& p, int64_t row0, int6
         const int64_t col = col0 + 16 * j;
         const int at = (int)(col < p.N ? col : p.N - 4);
         QkvOps<NI> late;
-        if constexpr (!EARLY) qkv_load(p, row0, col, late);
+        if constexpr (!EARLY) qkv_load(p, t, row0, col, late);
         const QkvOps<NI>& o = EARLY ? early[EARLY ? j : 0] : late;
         const int in_kv = at < t.qd ? 0 : at < turned ? at - t.qd : at - turned;
         uint16_t* run = (at < turned ? t.k : t.v) + kv_run_off(t.km, in_kv >> t.hd_log2, hd) + (in_kv & (hd - 1));
@@ -165,6 +169,8 @@ struct G8Split {
     float* slab;       // [tiles][splitk][256 * 256] fp32
     unsigned* cnt;     // [tiles], zero at rest
 };
+// (with four ints the arguments of the GEMM kernels: three lines of the segment, and the grid's size behind them in the third)
+static_assert(sizeof(GemmParams) + 4 * sizeof(int) + sizeof(G8Split) + 8 + 4 <= 192, "arguments of the GEMM kernels");
 
 // Slabs of 65,536 floats and zeroed tickets of stream `st`, grown on demand; non-zero: they would have to grow during a
 // graph capture, or there is no memory (the caller runs unsplit).  What a capture was given stays valid until g8_release.
@@ -176,6 +182,6 @@ void g8_release(hipStream_t st);
 
 // k_gemm_mid.hip: the GEMM of a few dozen to about a thousand rows.  other_us: the expected time of the caller's kernel for
 // this shape; *launched = false: not a shape for this one, or the other is expected to be faster.
-int gemm_mid(const qie_linear_args* a, const GemmParams& p, hipStream_t st, bool* launched);
+int gemm_mid(const qie_linear_args* a, const GemmParams& p, const QkvTail* tail, hipStream_t st, bool* launched);
 
 }  // namespace qie

@@ -436,7 +436,7 @@ constexpr int BUF = (BM + BN) * BK * 2;   // 64 KB: A rows [0, 256) then W rows,
 // in PART order (sc1 loads: cdna_hip_programming.md §5 'Projection GEMM' item 2), so the result
 // does not depend on arrival order, runs the epilogue and resets the ticket.
 template <int EPI>
-__global__ __launch_bounds__(512) void gemm8_kernel(GemmParams p, int n_mt, int n_nt, int gm, G8Split sk) {
+__global__ __launch_bounds__(512) void gemm8_kernel(GemmParams p, int n_mt, int n_nt, int gm, G8Split sk, TailOf<EPI> tail) {
 #pragma clang fp contract(off)
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -641,7 +641,7 @@ __global__ __launch_bounds__(512) void gemm8_kernel(GemmParams p, int n_mt, int 
         }
     } else if constexpr (EPI == kEpiQkv) {
         const QkvOps<8> none[1] = {};
-        qkv_tail<8, 4, false>(p, row0, nt * 256 + wn * 64 + 4 * g, acc, none);
+        qkv_tail<8, 4, false>(p, tail, row0, nt * 256 + wn * 64 + 4 * g, acc, none);
     } else {
         uint2 before[8][4];
         if constexpr (EPI == QIE_EPI_RESIDUAL) {   // all on their way at once: loads between the stores would each wait for memory
@@ -960,7 +960,7 @@ __global__ __launch_bounds__(512) void gemm8sk_kernel(GemmParams p, int n_mt, G8
 }
 
 template <int EPI>
-static int launch_gemm8_t(const GemmParams& p, int n_mt, int n_tiles, const G8Split& sk, hipStream_t st) {
+static int launch_gemm8_t(const GemmParams& p, int n_mt, int n_tiles, const G8Split& sk, hipStream_t st, const TailOf<EPI>& tail = {}) {
     const void* fn = (const void*)gemm8_kernel<EPI>;
     constexpr size_t shm = 2 * (size_t)g8::BUF;
     static bool raised = false;
@@ -969,12 +969,12 @@ static int launch_gemm8_t(const GemmParams& p, int n_mt, int n_tiles, const G8Sp
         raised = true;
     }
     hipLaunchKernelGGL((gemm8_kernel<EPI>), dim3((unsigned)(n_tiles * sk.splitk)), dim3(512), shm, st, p, n_mt,
-                       n_tiles / n_mt, band_height(n_mt, g8::BM, g8::BN, 32), sk);
+                       n_tiles / n_mt, band_height(n_mt, g8::BM, g8::BN, 32), sk, tail);
     QIE_LAUNCH_CHECK();
     return 0;
 }
-static int launch_gemm8(int epi, const GemmParams& p, int n_mt, int n_tiles, const G8Split& sk, hipStream_t st) {
-    if (p.qkv.q) return launch_gemm8_t<kEpiQkv>(p, n_mt, n_tiles, sk, st);
+static int launch_gemm8(int epi, const GemmParams& p, int n_mt, int n_tiles, const G8Split& sk, const QkvTail* tail, hipStream_t st) {
+    if (tail) return launch_gemm8_t<kEpiQkv>(p, n_mt, n_tiles, sk, st, *tail);
     if (epi == QIE_EPI_SWIGLU) return launch_gemm8_t<QIE_EPI_SWIGLU>(p, n_mt, n_tiles, sk, st);
     if (epi == QIE_EPI_RESIDUAL) return launch_gemm8_t<QIE_EPI_RESIDUAL>(p, n_mt, n_tiles, sk, st);
     if (epi == QIE_EPI_F32) return launch_gemm8_t<QIE_EPI_F32>(p, n_mt, n_tiles, sk, st);
@@ -1556,8 +1556,7 @@ static int gemm_with(const qie_linear_args* a, const QkvTail* tail, bool* done, 
         // (Qwen2-7B gate/up, us: 301 rows 161 with the 256x256 kernel, 97 with k_gemm_mid.hip; 700 rows 183 against 229)
         if (dev_env("QIE_MID", 1) && force < 0 && !(a->flags & QIE_LINEAR_STREAMK)) {
             bool launched = false;
-            if (tail) p.qkv = *tail;
-            const int rc = gemm_mid(a, p, st, &launched);
+            const int rc = gemm_mid(a, p, tail, st, &launched);
             if (done) *done = launched && tail;
             if (rc || launched) return rc;
         }
@@ -1570,15 +1569,15 @@ static int gemm_with(const qie_linear_args* a, const QkvTail* tail, bool* done, 
         }
         if (g8ok && g8mode != 0 && force != 2 && (force == 1 || (force < 0 && a->M >= big::BM && t256 >= cus))) {
             G8Split sk{1, nullptr, nullptr};
-            if (done) *done = p.qkv.q != nullptr;
-            return launch_gemm8(a->epilogue, p, (int)n_mt, (int)t256, sk, st);
+            if (done) *done = tail != nullptr;
+            return launch_gemm8(a->epilogue, p, (int)n_mt, (int)t256, sk, tail, st);
         }
         if (g8ok && g8mode == 2 && force < 0 && a->M >= big::BM && t256 < cus) {
             const int s = g8p::parts(a->M, cols, a->K, cus, std::max(4, dev_env("QIE_GEMM8_SK_MINK", 64)));   // (dev A/B: k-tiles a part)
             G8Split sk{1, nullptr, nullptr};
             if (s == 1 || (s > 1 && g8_workspace(st, (int)t256 * s, (int)t256, &sk) == 0 && (sk.splitk = s) > 1)) {
-                if (done) *done = p.qkv.q != nullptr;
-                return launch_gemm8(a->epilogue, p, (int)n_mt, (int)t256, sk, st);
+                if (done) *done = tail != nullptr;
+                return launch_gemm8(a->epilogue, p, (int)n_mt, (int)t256, sk, tail, st);
             }
         }
         if (force == 1 || (force < 0 && a->M >= big::BM && t256 >= cus))

@@ -47,7 +47,7 @@ __device__ __forceinline__ const uint16_t* mid_wrow(const GemmParams& p, int64_t
 }
 
 template <int EPI, int BM, int BN, int SLOTS>
-__global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, int n_nt, int gm, int whole, G8Split sk) {
+__global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, int n_nt, int gm, int whole, G8Split sk, TailOf<EPI> tail) {
 #pragma clang fp contract(off)
     constexpr int TM = BM / 2, TN = BN / 2, FI = TM / 16, FJ = TN / 16, FH = FI / 2;
     constexpr int SLOT = (BM + BN) * 128;      // A rows, then W rows, 128 B each
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
     [[maybe_unused]] QkvOps<FH> ops[EARLY ? FJ : 1];
     if constexpr (EARLY) {
 #pragma unroll
-        for (int j = 0; j < FJ; j++) qkv_load(p, m0 + wm * TM + wk * (FH * 16) + fr, nt * BN + wn * TN + 16 * j + 4 * g, ops[j]);
+        for (int j = 0; j < FJ; j++) qkv_load(p, tail, m0 + wm * TM + wk * (FH * 16) + fr, nt * BN + wn * TN + 16 * j + 4 * g, ops[j]);
         __builtin_amdgcn_sched_barrier(0);
     }
     auto stage = [&](int kt, int slot) {
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
             }
         }
     } else if constexpr (EPI == kEpiQkv) {
-        qkv_tail<FH, FJ, EARLY>(p, row0, nt * BN + wn * TN + 4 * g, res, ops);
+        qkv_tail<FH, FJ, EARLY>(p, tail, row0, nt * BN + wn * TN + 4 * g, res, ops);
     } else {
 #pragma unroll
         for (int j = 0; j < FJ; j++) {
@@ -291,7 +291,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
 // ---------------------------------------------------------------- the plan
 namespace {
 template <int EPI, int BM, int BN, int SLOTS>
-int launch_mid_t(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, hipStream_t st) {
+int launch_mid_t(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, const TailOf<EPI>& tail, hipStream_t st) {
     const void* fn = (const void*)gemm_mid_kernel<EPI, BM, BN, SLOTS>;
     constexpr size_t shm = (size_t)SLOTS * (BM + BN) * 128;
     static bool raised = false;
@@ -301,31 +301,31 @@ int launch_mid_t(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, hi
     }
     const int tiles = pl.n_mt * pl.n_nt, whole = sk.splitk > 1 ? pl.whole : tiles;
     hipLaunchKernelGGL((gemm_mid_kernel<EPI, BM, BN, SLOTS>), dim3((unsigned)(whole + (tiles - whole) * sk.splitk)), dim3(512), shm,
-                       st, p, pl.n_mt, pl.n_nt, band_height(pl.n_mt, BM, BN, 32 * mid::shape(pl.tile).per_cu), whole, sk);
+                       st, p, pl.n_mt, pl.n_nt, band_height(pl.n_mt, BM, BN, 32 * mid::shape(pl.tile).per_cu), whole, sk, tail);
     QIE_LAUNCH_CHECK();
     return 0;
 }
 
 template <int EPI>
-int launch_mid(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, hipStream_t st) {
+int launch_mid(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, hipStream_t st, const TailOf<EPI>& tail = {}) {
     switch (pl.tile) {
-        case 0: return launch_mid_t<EPI, 64, 64, 5>(p, pl, sk, st);
-        case 1: return launch_mid_t<EPI, 64, 128, 3>(p, pl, sk, st);
-        case 2: return launch_mid_t<EPI, 128, 64, 3>(p, pl, sk, st);
-        case 3: return launch_mid_t<EPI, 128, 128, 4>(p, pl, sk, st);
-        case 4: return launch_mid_t<EPI, 192, 128, 4>(p, pl, sk, st);
-        case 5: return launch_mid_t<EPI, 256, 128, 3>(p, pl, sk, st);
-        case 6: return launch_mid_t<EPI, 320, 64, 3>(p, pl, sk, st);
-        case 7: return launch_mid_t<EPI, 320, 128, 2>(p, pl, sk, st);
-        case 8: return launch_mid_t<EPI, 128, 160, 4>(p, pl, sk, st);
-        case 9: return launch_mid_t<EPI, 192, 160, 3>(p, pl, sk, st);
-        case 10: return launch_mid_t<EPI, 256, 160, 3>(p, pl, sk, st);
-        default: return launch_mid_t<EPI, 320, 160, 2>(p, pl, sk, st);
+        case 0: return launch_mid_t<EPI, 64, 64, 5>(p, pl, sk, tail, st);
+        case 1: return launch_mid_t<EPI, 64, 128, 3>(p, pl, sk, tail, st);
+        case 2: return launch_mid_t<EPI, 128, 64, 3>(p, pl, sk, tail, st);
+        case 3: return launch_mid_t<EPI, 128, 128, 4>(p, pl, sk, tail, st);
+        case 4: return launch_mid_t<EPI, 192, 128, 4>(p, pl, sk, tail, st);
+        case 5: return launch_mid_t<EPI, 256, 128, 3>(p, pl, sk, tail, st);
+        case 6: return launch_mid_t<EPI, 320, 64, 3>(p, pl, sk, tail, st);
+        case 7: return launch_mid_t<EPI, 320, 128, 2>(p, pl, sk, tail, st);
+        case 8: return launch_mid_t<EPI, 128, 160, 4>(p, pl, sk, tail, st);
+        case 9: return launch_mid_t<EPI, 192, 160, 3>(p, pl, sk, tail, st);
+        case 10: return launch_mid_t<EPI, 256, 160, 3>(p, pl, sk, tail, st);
+        default: return launch_mid_t<EPI, 320, 160, 2>(p, pl, sk, tail, st);
     }
 }
 }  // namespace
 
-int gemm_mid(const qie_linear_args* a, const GemmParams& p, hipStream_t st, bool* launched) {
+int gemm_mid(const qie_linear_args* a, const GemmParams& p, const QkvTail* tail, hipStream_t st, bool* launched) {
     *launched = false;
     const mid::Plan pl = mid::choose(a->M, a->epilogue == QIE_EPI_SWIGLU ? 2 * a->N : a->N, a->K, device_cu_count());
     if (pl.tile < 0) return 0;
@@ -336,7 +336,7 @@ int gemm_mid(const qie_linear_args* a, const GemmParams& p, hipStream_t st, bool
         if (g8_workspace(st, (int)cdiv(floats, 65536), (int)cut, &sk) == 0) sk.splitk = pl.splitk;
     }
     *launched = true;
-    if (p.qkv.q) return launch_mid<kEpiQkv>(p, pl, sk, st);
+    if (tail) return launch_mid<kEpiQkv>(p, pl, sk, st, *tail);
     switch (a->epilogue) {
         case QIE_EPI_SWIGLU: return launch_mid<QIE_EPI_SWIGLU>(p, pl, sk, st);
         case QIE_EPI_RESIDUAL: return launch_mid<QIE_EPI_RESIDUAL>(p, pl, sk, st);
