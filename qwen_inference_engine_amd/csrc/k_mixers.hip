@@ -916,7 +916,7 @@ __global__ __launch_bounds__(256) void gqa_attn_combine_kernel(GqaAttnMfmaP P, i
 #pragma unroll
         for (int k = 0; k < VPL; k++)
             if (in[k]) turn[wave][v[k]] = acc[k] * inv;
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
     }
     const int64_t o0 = (int64_t)row * a.ld_out + a.out_col + (int64_t)hh * vdim;
 #pragma unroll
