@@ -133,6 +133,9 @@ __global__ void set_state_kernel(int m, int32_t pos_v, int32_t step_v, int32_t t
         for (int64_t i = threadIdx.x; i < H8; i += blockDim.x) x_res[(int64_t)m * H8 + i] = E[(int64_t)tok * H8 + i];
 }
 
+// Ids that qie_decode fetches at once (longer calls copy row by row, which is little beside their steps): 64 KB of pinned memory at most,
+// whatever the contexts.
+int64_t ids_at_once(int32_t batch, int32_t max_ctx) { return std::min<int64_t>((int64_t)batch * max_ctx, 16384); }
 // ids of n_steps decode steps, [n_steps][B], to pinned host memory: sequence m's from history position at[m] on
 __global__ void fetch_ids_kernel(const int32_t* hist, int hist_stride, const int32_t* at, int B, int n_steps, int32_t* out) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1154,8 +1157,10 @@ static int batch_create(qie_engine* e, int32_t batch, int32_t max_ctx, int32_t p
         A((void**)&b->logits_full, batch * (int64_t)s.vocab * 2);
         A((void**)&b->gather_tmp, batch * (int64_t)s.vocab * 2);
     }
-    if (!rc && hipHostMalloc((void**)&b->h_ids, (size_t)batch * (max_ctx + 1) * 4, hipHostMallocDefault) != hipSuccess)
-        rc = fail(-2, "qie_batch_create: no pinned memory for the ids");
+    if (!rc && hipHostMalloc((void**)&b->h_ids, (size_t)(batch + ids_at_once(batch, max_ctx)) * 4, hipHostMallocDefault) != hipSuccess) {
+        b->h_ids = nullptr;   // (qie_decode does without)
+        (void)hipGetLastError();
+    }
     if (!rc) {
         hipMemsetAsync(b->dec_ws, 0, (size_t)dec_ws, e->stream);
         hipMemsetAsync(b->kc, 0, (size_t)n_runs * b->seq_stride * 2, e->stream);
@@ -1513,13 +1518,15 @@ int qie_decode(qie_batch* b, int32_t n_steps, const qie_sampling* smp, int32_t* 
     QIE_REQUIRE(b && n_steps >= 0, "qie_decode: bad arguments");
     QIE_TRY(prepare_steps(b, n_steps, "qie_decode"));
     const bool want = out_ids && n_steps > 0;
-    if (want)
-        for (int m = 0; m < b->B; m++) b->h_ids[m] = b->h_pos[m] + 1;   // (no call leaves a launch behind that reads or writes h_ids)
+    const bool at_once = want && b->h_ids && (int64_t)n_steps * b->B <= ids_at_once(b->B, b->max_ctx);
+    const std::vector<int32_t> p0 = b->h_pos;
+    if (at_once)
+        for (int m = 0; m < b->B; m++) b->h_ids[m] = p0[m] + 1;   // (no call leaves a launch behind that reads or writes h_ids)
     for (int i = 0; i < n_steps; i++) {
         QIE_TRY(launch_step(b, smp));
         for (int m = 0; m < b->B; m++) b->h_pos[m] += 1;
     }
-    if (want) {   // one launch behind the steps, and the wait that there is anyway (a copy and a wait a sequence took 15 us each)
+    if (at_once) {   // one launch behind the steps, and the wait that there is anyway (a copy and a wait a sequence take 15 us each)
         hipLaunchKernelGGL(fetch_ids_kernel, dim3((unsigned)cdiv(n_steps * b->B, 256)), dim3(256), 0, b->e->stream, b->d_hist, b->max_ctx, b->h_ids,
                            b->B, n_steps, b->h_ids + b->B);
         QIE_LAUNCH_CHECK();
@@ -1527,7 +1534,15 @@ int qie_decode(qie_batch* b, int32_t n_steps, const qie_sampling* smp, int32_t* 
     QIE_HIP(hipStreamSynchronize(b->e->stream));
     QIE_TRY(comm_check(b->e, "qie_decode"));
     QIE_TRY(pk_check(b));
-    if (want) memcpy(out_ids, b->h_ids + b->B, (size_t)n_steps * b->B * 4);
+    if (at_once) {
+        memcpy(out_ids, b->h_ids + b->B, (size_t)n_steps * b->B * 4);
+    } else if (want) {
+        std::vector<int32_t> row(n_steps);
+        for (int m = 0; m < b->B; m++) {
+            QIE_HIP(d2h(b->e, row.data(), b->d_hist + (int64_t)m * b->max_ctx + p0[m] + 1, (size_t)n_steps * 4));
+            for (int i = 0; i < n_steps; i++) out_ids[(int64_t)i * b->B + m] = row[i];
+        }
+    }
     return 0;
 }
 

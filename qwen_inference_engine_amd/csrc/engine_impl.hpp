@@ -89,7 +89,7 @@ struct qie_batch {
     uint16_t* gather_tmp = nullptr;   // [tp][B][V/tp]
     float* pf_part = nullptr;         // [pf_rows][H]
     std::vector<int32_t> h_pos;
-    int32_t* h_ids = nullptr;         // pinned: [B] first positions, then the ids of qie_decode [n_steps][B]
+    int32_t* h_ids = nullptr;         // pinned: [B] first positions, then the ids of qie_decode [n_steps][B], ids_at_once of them (null: none)
     // prefill scratch
     int64_t pf_rows = 0;
     uint16_t *pf_x = nullptr, *pf_hn = nullptr, *pf_qkv = nullptr, *pf_q = nullptr, *pf_att = nullptr,

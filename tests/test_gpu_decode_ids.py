@@ -29,3 +29,23 @@ def test_ids_equal_step_by_step(batch):
     assert b.decode(0).shape == (0, batch)
     b.close()
     eng.close()
+
+
+def test_more_ids_than_are_fetched_at_once():
+    """A call of more ids than the pinned room takes gives those of calls that fit it."""
+    import qwen_inference_engine_amd as q
+    from qwen_inference_engine_amd import spec as S, weights as W
+    spec = S.tiny("ids", n_layers=1, hidden=128, n_heads=2, n_kv_heads=1, head_dim=64, ffn=256, vocab=500)
+    eng = q.Engine(spec, device=0, max_ctx=2304).init_synthetic(W.SynthParams(seed=3, w_scale=0.08, norm_scale=0.25, bias_scale=0.05))
+    b = eng.batch(8, 2304)
+    for m in range(8):
+        b.prefill(m, list(range(5 + m)))
+    out = []
+    for parts in ((800, 800, 550), (2150,)):   # 17,200 ids in all
+        for m in range(8):
+            b.set_position(m, 5 + m, 7 + m)
+        out.append(np.concatenate([b.decode(n) for n in parts]))
+    assert np.array_equal(out[0], out[1])
+    assert b.history(7, 12 + 2151)[13:].tolist() == out[1][:, 7].tolist()
+    b.close()
+    eng.close()

@@ -204,3 +204,10 @@ def test_prefill_fp8_refused_where_it_cannot_hold(qlib, fp8, tiny_widths):
     rc = qlib.qie_engine_create(C.byref(sc), C.byref(opts), C.byref(h))
     assert rc == -22 and not h.value
     assert b"prefill_fp8" in qlib.qie_last_error()
+
+
+def test_ids_of_long_contexts_hold_little_pinned_memory(qlib):
+    """qie_decode's pinned ids: those of short contexts whole, a bounded number of long ones."""
+    room = C.CDLL(_lib.load()._name)._ZN3qie11ids_at_onceEii
+    room.restype = C.c_int64
+    assert room(1, 64) == 64 and room(8, 128) == 1024 and room(8, 1 << 20) == 16384
