@@ -990,7 +990,9 @@ int route_grouped(const float* y, const void* Wr, const float* corr, bool w_f32,
     QIE_REQUIRE(top >= 1 && top <= E && E <= 4096 && corr, "router: top %d of %d outputs", top, E);
     QIE_REQUIRE(groups >= 1 && E % groups == 0 && keep >= 1 && keep <= groups && top <= keep * (E / groups),
                 "router: %d groups of %d outputs, %d kept, top %d", groups, E, keep, top);
-    if (E <= 64) {
+    // Every lane of a wave takes part in each of the top x E steps of the choice: a thread does them beside other blocks' products where there are
+    // many rows.  us, that | lanes, 64 outputs: 512 rows, 64 chosen 278 | 207; 2,048 rows, 16 chosen 134 | 129, 32 216 | 229, 64 343 | 423
+    if (E <= 64 && (top <= 16 || T <= 512)) {
         const dim3 block(64 * (E < 16 ? E : 16));
         if (w_f32)
             hipLaunchKernelGGL(route_grouped_wave_kernel<float>, dim3(T), block, 0, st, y, (const float*)Wr, corr, W, E, top, groups, keep,

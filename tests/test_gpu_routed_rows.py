@@ -64,6 +64,20 @@ def test_router(qlib, E, top, groups, keep, f32):
     assert torch.allclose(score.double(), scale * chosen / chosen.sum(1, keepdim=True), rtol=2e-5)
 
 
+def test_router_of_many_rows(qlib):
+    """Many rows with many choices go to the kernel of one thread a row: the same bits."""
+    T, W, E, top = 513, 64, 64, 32
+    g = torch.Generator("cuda").manual_seed(2)
+    y, corr = torch.randn(T, W, generator=g, device="cuda"), 0.1 * torch.randn(E, generator=g, device="cuda")
+    w = torch.randn(E, W, generator=g, device="cuda") * W ** -0.5
+    got = []
+    for rows in (T, T - 1):
+        sel, score = torch.zeros(T, top, device="cuda", dtype=torch.int32), torch.zeros(T, top, device="cuda")
+        call("13route_groupedEPKfPKvS2_biiiiiifPiPfP12ihipStream_t", y, w, corr, C.c_bool(True), rows, W, E, top, 4, 3, C.c_float(1.5), sel, score, None)
+        got.append((sel[:T - 1], score[:T - 1]))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
 @pytest.mark.parametrize("f32", [True, False])
 @pytest.mark.parametrize("gated", [False, True])
 @pytest.mark.parametrize("K,counts", [(8, [1]), (504, [0, 3, 1]), (512, [2, 0, 0, 5]), (704, [17, 0, 15]), (1024, [1, 1, 0, 2, 2]), (1032, [3, 4])])
