@@ -95,7 +95,7 @@ inline bool whole_tiles(int64_t M, int64_t K, int64_t tiles, int64_t parts, int6
     const int64_t rounds = (tiles + cus - 1) / cus;
     const bool crowded = parts * tiles >= 14 * cus;
     if (M <= 4) return crowded || 10 * rounds * cus <= 16 * tiles;
-    return 10 * rounds * cus <= (crowded ? 14 : tiles <= 2 * cus ? 13 : 12) * tiles;
+    return 10 * rounds * cus <= (crowded || (K <= 10240 && tiles <= 2 * cus) ? 14 : tiles <= 2 * cus ? 13 : 12) * tiles;
 }
 }  // namespace d8s
 

@@ -923,8 +923,7 @@ __global__ __launch_bounds__(512) void dec8s_kernel(Dec8Params p) {
             wv = lane * 16;
             ws = (uint32_t)(tile * 16 * K);
         } else {
-            const int r = tile * 16 + fr;
-            wv = (uint32_t)((r < rows ? r : rows - 1) * K + 16 * g);
+            wv = (uint32_t)((tile * 16 + fr) * K + 16 * g);   // (rows are whole tiles: dec8_applies)
             ws = 0;
         }
     };
@@ -1010,7 +1009,6 @@ __global__ __launch_bounds__(512) void dec8s_kernel(Dec8Params p) {
             const uint32_t s4[4] = {sc.x, sc.y, sc.z, sc.w};
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                if (col + r >= p.N) continue;
                 const float c = v[r] * __uint_as_float(s4[r]);
                 const int64_t at = (int64_t)fr * p.ldy + col + r;
                 if constexpr (EPI == QIE_EPI_F32) {
