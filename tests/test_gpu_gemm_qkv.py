@@ -1,6 +1,6 @@
 """The QKV product whose epilogue turns q and k and writes the cache (gemm_qkv, what a prompt's layers call) against the product and
-qie_qkv_post: the same bits.  Short and tall tiles, split and whole, the 256x256 kernel, ragged rows, several prompts in a tile, heads of 64 and
-128, contiguous and paged; and a K that no kernel with that epilogue takes."""
+qie_qkv_post: the same bits.  Every tile of k_gemm_mid.hip and the 256x256 kernel, split and whole, ragged rows, several prompts in a tile, heads of
+8, 64 and 128, contiguous and paged; and a K that no kernel with that epilogue takes."""
 import ctypes as C
 
 import numpy as np
@@ -8,20 +8,36 @@ import pytest
 import torch
 
 import gpu_util as G
+from gemm_route import routes
 from qwen_inference_engine_amd import _lib
 from qwen_inference_engine_amd._lib import KvCacheC, LinearArgsC
 
-pytestmark = pytest.mark.gpu
 SYMBOL = "_ZN3qie8gemm_qkvEPK15qie_linear_argsPK12qie_kv_cacheiiPKfPtP12ihipStream_tPb"
 
 
-# heads, key heads, head size, K, rows of a prompt, prompts, page
-@pytest.mark.parametrize("nq,nkv,hd,K,n,seqs,page,fused", [
-    (14, 2, 64, 896, 17, 1, 0, True), (14, 2, 64, 896, 113, 1, 128, True), (14, 2, 64, 896, 37, 5, 128, True),
-    (14, 2, 64, 896, 1501, 1, 0, True), (28, 4, 128, 3584, 63, 1, 128, True), (28, 4, 128, 3584, 301, 1, 0, True),
-    (28, 4, 128, 3584, 1030, 1, 128, True), (28, 4, 128, 512, 2100, 2, 256, True), (28, 4, 128, 512, 1363, 3, 0, True),
-    (3, 1, 8, 256, 65, 2, 0, True), (14, 2, 64, 928, 300, 1, 0, False)])
-def test_as_the_product_and_its_post_pass(qlib, nq, nkv, hd, K, n, seqs, page, fused):
+# heads, key heads, head size, K, rows of a prompt, prompts, page, tile (k_gemm_mid.hip's, -1: the 256x256 kernel, None: one without this epilogue)
+CASES = [
+    (14, 2, 64, 896, 17, 1, 0, 0), (14, 2, 64, 896, 113, 1, 128, 0), (14, 2, 64, 896, 37, 5, 128, 0),
+    (14, 2, 64, 896, 1501, 1, 0, 1), (28, 4, 128, 3584, 63, 1, 128, 0), (28, 4, 128, 3584, 301, 1, 0, 2),
+    (28, 4, 128, 3584, 1030, 1, 128, 4), (28, 4, 128, 512, 2100, 2, 256, -1), (28, 4, 128, 512, 1363, 3, 0, -1),
+    (3, 1, 8, 256, 65, 2, 0, 0), (14, 2, 64, 928, 300, 1, 0, None), (28, 4, 128, 3584, 2500, 1, 0, -1), (28, 4, 128, 3584, 2048, 1, 128, 7),
+    (28, 4, 128, 3584, 1024, 8, 128, 11), (28, 4, 128, 3584, 4096, 1, 0, 10), (28, 4, 128, 3584, 1363, 1, 128, 5), (14, 2, 64, 896, 2300, 1, 0, 3),
+    (14, 2, 64, 896, 6000, 1, 0, 9), (16, 4, 128, 256, 1540, 1, 0, 6), (56, 8, 128, 256, 195, 1, 128, 8), (56, 8, 128, 4096, 67, 1, 0, 3),
+    (32, 8, 128, 16384, 500, 2, 128, -1)]
+
+
+def test_cases_take_every_kernel_with_the_epilogue():
+    got = routes([(c[4] * c[5], (c[0] + 2 * c[1]) * c[2], c[3]) for c in CASES])
+    for c, r in zip(CASES, got):
+        assert c[7] is None and c[3] % 64 != 0 or c[7] is not None and r["tile"] == c[7] and (c[7] >= 0 or r["parts"] >= 1), (c, r)
+    assert {r["tile"] for r in got} == set(range(-1, 12))
+    assert {r["parts"] for r, c in zip(got, CASES) if c[7] == -1} >= {1, 2}   # the 256x256 kernel whole and split
+    assert any(r["splitk"] > 1 for r in got)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nq,nkv,hd,K,n,seqs,page,tile", CASES)
+def test_as_the_product_and_its_post_pass(qlib, nq, nkv, hd, K, n, seqs, page, tile):
     M, QD, KD, ctx, layers, layer = n * seqs, nq * hd, nkv * hd, n + 3, 2, 1
     N = QD + 2 * KD
     g = torch.Generator("cuda").manual_seed(M + K)
@@ -66,8 +82,8 @@ def test_as_the_product_and_its_post_pass(qlib, nq, nkv, hd, K, n, seqs, page, f
     torch.cuda.synchronize()
     G.check(fn(C.byref(args(y2)), C.byref(c2), layer, n, turns.data_ptr(), q2.data_ptr(), None, C.byref(done)), "gemm_qkv")
     torch.cuda.synchronize()
-    assert done.value == fused
-    if not fused:
+    assert done.value == (tile is not None)
+    if tile is None:
         assert torch.equal(y, y2) and (q2 == 7.0).all()
         return
     assert torch.equal(q, q2)

@@ -42,6 +42,8 @@ def test_parts_meet(heads, kv, dim, vdim, layout, mask):
         b.close()
         eng.close()
     want, got = out["float32"], out["bfloat16"]
-    # bf16 rows and weights' products: half an ulp of 2^-9 each through one layer and the head, a few of them a logit
+    # A bf16 rounding is 2^-9 / sqrt(3) = 1.1e-3 of a value on the average; some ten of them stand one behind the other between the embedding and
+    # a logit (normed rows, q, k, v, weights of the softmax, heads, activations, the head's rows): 3.6e-3 of a row, three times that for the
+    # worst of thirty.  One wrong coordinate in the 128 to 1,152 of a row's heads is 4 to 12 % of its attention.
     err = np.sqrt(((got - want) ** 2).mean(axis=1)) / want.std()
-    assert err.max() < 5e-2
+    assert err.max() < 1.1e-2
