@@ -193,7 +193,8 @@ int qie_batch_logits(qie_batch* b, void* host_out);
 int qie_batch_positions(qie_batch* b, int32_t* host_pos);
 int qie_batch_history(qie_batch* b, int32_t seq, int32_t* host_ids, int32_t n);
 /* Rewind/set sequence `seq` to position pos with current token `token`
- * (KV rows >= pos are simply overwritten later). */
+ * (KV rows >= pos are simply overwritten later).  Queued on the engine's stream: returns without waiting for it,
+ * so a device error of its launch is reported by a later call. */
 int qie_batch_set_position(qie_batch* b, int32_t seq, int32_t pos, int32_t token);
 /* Decode structure of the batch's steps: 0 = five launches per layer (the reference path:
  * QKV GEMV, attention, O GEMV, gate/up GEMV, down GEMV, hipGraph-captured); 1 = the whole

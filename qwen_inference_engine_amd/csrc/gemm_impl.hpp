@@ -180,8 +180,8 @@ void g8_reserve(hipStream_t st);
 // Gives a stream's split-K memory back: before the engine that owns the stream destroys it, its batches' graphs gone.
 void g8_release(hipStream_t st);
 
-// k_gemm_mid.hip: the GEMM of a few dozen to about a thousand rows.  other_us: the expected time of the caller's kernel for
-// this shape; *launched = false: not a shape for this one, or the other is expected to be faster.
+// k_gemm_mid.hip: the GEMM of a few dozen to about a thousand rows, and of more where its tiles are the faster (mid::choose; *launched = false: not
+// such a shape).  tail: null, or what follows the product.
 int gemm_mid(const qie_linear_args* a, const GemmParams& p, const QkvTail* tail, hipStream_t st, bool* launched);
 
 }  // namespace qie

@@ -335,8 +335,8 @@ int gqa_post(const GqaPostP& p, bool cache_f32, int T, hipStream_t st) {
 // ------------------------------------------------------------------ attention, exact form
 // One block per (head, row): the visible keys go through in chunks of GA_CHUNK with a running
 // maximum and sum.  16 lanes score a key (16 bytes of it each at a time where its rows are on that
-// grid), four keys' loads in flight a lane; then the waves take every fourth key's value row, a lane
-// per coordinate, and their sums meet at the end.  (A wave per key and a thread per coordinate over
+// grid), four keys' loads in flight a lane; then each wave takes the value rows of every 4th (16 waves a block: every
+// 16th) key, a lane per coordinate, and the sums meet at the end.  (A wave per key and a thread per coordinate over
 // all keys, one load behind the other: 97 us for 3 rows of 16 heads over 160 keys of 64 in fp32.)
 constexpr int GA_CHUNK = 256;
 constexpr int GA_MAXV = 4;   // vdim <= 256 * GA_MAXV
