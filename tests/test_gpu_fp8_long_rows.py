@@ -72,7 +72,7 @@ def test_sums_are_short(oracle, qlib, K, N, bound):
 
 @pytest.mark.parametrize("tiled", [False, True])
 @pytest.mark.parametrize("M,K,r", [(2, 2176, (2048, 0, 1536)), (8, 2176, (2048, 0, 1536)), (2, 2176, (2048, 1024, 512)), (2, 2176, (0, 0, 3584)),
-                                   (8, 2176, (1024, 0, 512)), (2, 3584, (1024, 0, 512)), (2, 3584, (0, 0, 1536))])
+                                   (8, 2176, (1024, 0, 512)), (2, 3584, (1024, 0, 512)), (2, 3584, (0, 0, 1536)), (2, 3584, (0, 1536, 0))])
 def test_weights_in_several_segments(oracle, qlib, M, K, r, tiled):
     """Columns take weights, scales and biases of their own segment, whichever segments there are."""
     N = sum(r)
