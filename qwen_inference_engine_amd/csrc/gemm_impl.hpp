@@ -86,8 +86,15 @@ __device__ __forceinline__ uint2 quad_before(const uint16_t* src, bool vec, int6
         if (r < left) h[r] = src[r];
     return make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
 }
+__device__ __forceinline__ void sum_quad(uint2 x, f32x4 v, float (&o)[4]) {
+    o[0] = bf_lo(x.x) + rbf(v[0]);
+    o[1] = bf_hi(x.x) + rbf(v[1]);
+    o[2] = bf_lo(x.y) + rbf(v[2]);
+    o[3] = bf_hi(x.y) + rbf(v[3]);
+}
 __device__ __forceinline__ void add_quad(uint16_t* dst, uint2 x, f32x4 v, bool vec, int64_t left) {
-    const float o[4] = {bf_lo(x.x) + rbf(v[0]), bf_hi(x.x) + rbf(v[1]), bf_lo(x.y) + rbf(v[2]), bf_hi(x.y) + rbf(v[3])};
+    float o[4];
+    sum_quad(x, v, o);
     store_quad(dst, o, vec, left);
 }
 // biases of columns col .. col + 3 (zero where a segment has none)
@@ -162,6 +169,7 @@ __device__ __forceinline__ void qkv_tail(const GemmParams& p, const QkvTail& t, 
 }
 
 typedef unsigned int u32x4_g8 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2_g8 __attribute__((ext_vector_type(2)));
 
 // split-K workspace of one launch (gemm8_kernel has the protocol)
 struct G8Split {

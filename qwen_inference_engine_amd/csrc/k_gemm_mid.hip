@@ -12,11 +12,18 @@
 //     measured the same), so the time follows the rows of A and W that a CU stages for its outputs: tall tiles, and columns in tiles
 //     that fill rounds of the chip.  Qwen2-7B gate / up, 128 / 160 columns a tile: 113 rows 71 / 58 us, 200 rows 97 / 78, 301 rows 120 /
 //     97, 512 rows 171 / 143;
-//   * 8 waves as 2 (M) x 2 (N) x 2 (K halves of every k-tile): a wave's tile is half the block's in both directions, which
-//     reads LDS as often as four waves would, and two waves a SIMD cover each other's fragment reads.  The K halves meet in
-//     LDS once, behind the loop;
-//   * split-K over workgroups where the tiles do not fill the chip (fp32 slabs, the last arriver sums them in part order:
-//     gemm8_kernel's protocol, the result does not depend on arrival order);
+//   * 8 waves.  The two 32-deep halves of a k-tile are summed apart, either by waves 0 .. 3 and 4 .. 7 (2 x 2 of them over the tile; they meet
+//     in LDS behind the loop) or by every wave (4 x 2) in registers of its own, which needs no meeting: 320 x 160 spent 10 of 100 us on it.
+//     The sums are the same bits.  LDS gives 230 B a clock, so how often it is read does not decide;
+//   * in turns: waves 4 .. 7 run one barrier behind waves 0 .. 3, on every SIMD one wave's products run while the other's fragments are
+//     read.  Which form a tile has is what 184 shapes of 12 projections at 24 to 3,000 rows measured: 128 x 128 at K = 18,944, all eight in
+//     step with halves by wave 66.3 us, halves by register 67.4, in turns 69.5, in turns with halves by wave 63.1; at K = 896 13.1, 12.7,
+//     13.6, 14.1.  On the average of the 184 the products take 0.967 of what they took with halves by wave in step;
+//   * 320 rows: W of one k-tile more than A in flight (its lines come from HBM, A's mostly from L2, and a CU returns them in order): the
+//     staging alone 80 -> 69 us at 320 x 160;
+//   * split-K over workgroups where the tiles do not fill the chip (fp32 slabs, the last arriver sums them in part order: gemm8_kernel's
+//     protocol, the result does not depend on arrival order).  A wave's share of a tile meets by itself, with a ticket of its own: the
+//     shares' last arrivers are spread over the parts' CUs, and none waits for its workgroup (301 rows, O, 25.4 -> 22.9 us);
 //   * workgroups that share a weight tile are neighbours in one XCD, parts are the slowest index: an XCD's L2 holds one K
 //     range of A.
 #include "gemm_impl.hpp"
@@ -46,17 +53,18 @@ __device__ __forceinline__ const uint16_t* mid_wrow(const GemmParams& p, int64_t
     }
 }
 
-template <int EPI, int BM, int BN, int SLOTS>
+template <int EPI, int BM, int BN, int SA, int SW, int KW, bool TURNS>
 __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, int n_nt, int gm, int whole, G8Split sk, TailOf<EPI> tail) {
 #pragma clang fp contract(off)
-    constexpr int TM = BM / 2, TN = BN / 2, FI = TM / 16, FJ = TN / 16, FH = FI / 2;
-    constexpr int SLOT = (BM + BN) * 128;      // A rows, then W rows, 128 B each
-    // LDS-DMA instructions (8 rows each) per wave and k-tile; where the waves don't share them evenly, the first MORE have one more
-    constexpr int BLOCKS = (BM + BN) / 8, IPW = (BLOCKS + 7) / 8, MORE = BLOCKS % 8;
+    constexpr int HV = 2 / KW;   // halves of a k-tile that a wave has: KW 1, waves as 4 (M) x 2 (N), both; KW 2, 2 x 2 x the halves
+    constexpr int TM = BM / (4 / KW), TN = BN / 2, FI = TM / 16, FJ = TN / 16;   // a wave's tile
+    constexpr int A_SLOT = BM * 128, W_SLOT = BN * 128, W_BASE = SA * A_SLOT;
+    // LDS-DMA instructions (8 rows each) per wave and k-tile; where the waves don't share W's evenly, the first MORE have one more
+    constexpr int AIW = BM / 64, WIW = (BN / 8 + 7) / 8, MORE = BN / 8 % 8;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wk = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+    const int wk = KW == 2 ? wave >> 2 : 0, wm = KW == 2 ? (wave >> 1) & 1 : wave >> 1, wn = wave & 1;
     const int fr = lane & 15, g = lane >> 4;
     // workgroups [0, whole): a tile each; behind them the other tiles, splitk parts each.  Within either range the
     // bijective XCD remap keeps neighbours (the M tiles of a weight tile) on one XCD
@@ -70,178 +78,299 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
     banded(tile, n_mt, n_nt, gm, &mti, &nti);
     const int64_t mt = mti, nt = nti, m0 = mt * BM;
 
-    const int nk_all = (int)(p.K / mid::BK);
-    const int kb = (int)((int64_t)part * nk_all / parts);        // this part's k-tiles [kb, kb + nk)
-    const int nk = (int)((int64_t)(part + 1) * nk_all / parts) - kb;
+    const int nk_all = (int)(p.K >> 6);
+    const int kb = quotient(part * nk_all, parts), nk = quotient((part + 1) * nk_all, parts) - kb;   // this part's k-tiles [kb, kb + nk)
 
     // instruction i of this wave fills the slot's rows 8 b .. 8 b + 7, b = 8 i + wave: lane -> row 8 b + (lane >> 3),
     // LDS chunk lane & 7, which holds the source's chunk (lane & 7) ^ swz(row)
-    const uint16_t* src[IPW];
+    uint32_t a_off[AIW];   // bytes behind the tile's first row
+    const uint16_t* w_src[WIW];
+    const int r0 = 8 * wave + (lane >> 3), cs = ((lane & 7) ^ g8_swz(r0)) * 8;   // (64 rows on: the same chunk)
+    const int64_t k0 = (int64_t)kb * mid::BK + cs;
 #pragma unroll
-    for (int i = 0; i < IPW; i++) {
-        if (MORE && i == IPW - 1 && wave >= MORE) break;   // uniform
-        const int r = 8 * (8 * i + wave) + (lane >> 3);
-        const int cs = (lane & 7) ^ g8_swz(r);
-        if (r < BM) {   // uniform over the wave: BM is a multiple of 8
-            int64_t ar = m0 + r;
-            ar = ar < p.M ? ar : p.M - 1;   // rows past M: re-read row M - 1, never stored
-            src[i] = p.A + ar * p.lda + (int64_t)kb * mid::BK + cs * 8;
-        } else {
-            src[i] = mid_wrow<EPI, BN>(p, nt, r - BM) + (int64_t)kb * mid::BK + cs * 8;
-        }
+    for (int i = 0; i < AIW; i++) {
+        int64_t ar = m0 + r0 + 64 * i;
+        ar = ar < p.M ? ar : p.M - 1;   // rows past M: re-read row M - 1, never stored
+        a_off[i] = (uint32_t)(ar - m0) * (uint32_t)p.lda * 2 + (uint32_t)cs * 2;
     }
+#pragma unroll
+    for (int i = 0; i < WIW; i++) {
+        if (MORE && i == WIW - 1 && wave >= MORE) break;   // uniform
+        w_src[i] = mid_wrow<EPI, BN>(p, nt, r0 + 64 * i) + k0;
+    }
+    constexpr int FR = FI / KW;   // a wave's rows of the result, in fragments
+    const int wrow = wm * TM + wk * (FR * 16) + fr;
     // kEpiQkv of small tiles: its operands are on their way before the first k-tile
-    constexpr bool EARLY = EPI == kEpiQkv && FH * FJ <= 8;
-    [[maybe_unused]] QkvOps<FH> ops[EARLY ? FJ : 1];
+    const int64_t row0 = m0 + wrow;
+    constexpr bool EARLY = EPI == kEpiQkv && FR * FJ <= 8;
+    [[maybe_unused]] QkvOps<FR> ops[EARLY ? FJ : 1];
     if constexpr (EARLY) {
 #pragma unroll
-        for (int j = 0; j < FJ; j++) qkv_load(p, tail, m0 + wm * TM + wk * (FH * 16) + fr, nt * BN + wn * TN + 16 * j + 4 * g, ops[j]);
+        for (int j = 0; j < FJ; j++) qkv_load(p, tail, row0, nt * BN + wn * TN + 16 * j + 4 * g, ops[j]);
         __builtin_amdgcn_sched_barrier(0);
     }
-    auto stage = [&](int kt, int slot) {
-        unsigned char* dst = smem + slot * SLOT + wave * 1024;
+    const uint16_t* a_at = p.A + m0 * p.lda + (int64_t)kb * mid::BK;
+    auto stage_a = [&](int kt, int slot) {
 #pragma unroll
-        for (int i = 0; i < IPW; i++) {
-            if (MORE && i == IPW - 1 && wave >= MORE) break;
-            glds16(src[i] + (int64_t)kt * mid::BK, dst + i * 8192);
+        for (int i = 0; i < AIW; i++) glds16(reinterpret_cast<const unsigned char*>(a_at + (int64_t)kt * mid::BK) + a_off[i], smem + slot * A_SLOT + wave * 1024 + i * 8192);
+    };
+    auto stage_w = [&](int kt, int slot) {
+#pragma unroll
+        for (int i = 0; i < WIW; i++) {
+            if (MORE && i == WIW - 1 && wave >= MORE) break;
+            glds16(w_src[i] + (int64_t)kt * mid::BK, smem + W_BASE + slot * W_SLOT + wave * 1024 + i * 8192);
         }
     };
 
-    f32x4 acc[FI][FJ];
+    // sums of either half of every k-tile
+    f32x4 acc[HV][FI][FJ];
 #pragma unroll
-    for (int i = 0; i < FI; i++)
+    for (int s = 0; s < HV; s++)
 #pragma unroll
-        for (int j = 0; j < FJ; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < FI; i++)
+#pragma unroll
+            for (int j = 0; j < FJ; j++) acc[s][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    for (int t = 0; t < SLOTS - 1 && t < nk; t++) stage(t, t);
-    int slot = 0, fill = SLOTS - 1;
-    for (int t = 0; t < nk; t++) {
-        // k-tile t has landed (the SLOTS - 2 younger ones may still fly), and every wave is done with the slot of t - 1
-        if (t + SLOTS - 1 <= nk && (MORE == 0 || wave < MORE)) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(IPW * (SLOTS - 2)) : "memory");
-        else if (t + SLOTS - 1 <= nk) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((IPW - 1) * (SLOTS - 2)) : "memory");
+    // step t stages A of k-tile t + SA - 1, then W of t + SW - 1: the steps before the first
+#pragma unroll
+    for (int t = 1 - SW; t < 0; t++) {
+        if (t + SA - 1 >= 0 && t + SA - 1 < nk) stage_a(t + SA - 1, t + SA - 1);
+        if (t + SW - 1 < nk) stage_w(t + SW - 1, t + SW - 1);
+    }
+    constexpr int YOUNG = SA - 2, AHEAD_W = SW > SA ? 1 : 0;   // k-tiles, and W's of one more, that fly behind the one waited for
+    static_assert(SW >= SA, "A of a k-tile is staged no earlier than its W");
+    auto landed = [&](bool steady) {   // the k-tile after which `steady` steps were staged
+        if (steady && (MORE == 0 || wave < MORE)) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AIW + WIW) * YOUNG + WIW * AHEAD_W) : "memory");
+        else if (steady) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((AIW + WIW - 1) * YOUNG + (WIW - 1) * AHEAD_W) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    };
+    auto bar = [&]() {
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
-        if (t + SLOTS - 1 < nk) stage(t + SLOTS - 1, fill);
-        const unsigned char* buf = smem + slot * SLOT;
-        bf16x8 fa[FI], fb[FJ];
-        auto read_a = [&](int i) {
-            const int row = wm * TM + i * 16 + fr;
-            fa[i] = *reinterpret_cast<const bf16x8*>(buf + row * 128 + (((4 * wk + g) ^ g8_swz(row)) * 16));
-        };
+    };
+    auto frag = [&](const unsigned char* buf, int row, int s) {
+        return *reinterpret_cast<const bf16x8*>(buf + row * 128 + (((4 * s + g) ^ g8_swz(row)) * 16));
+    };
+    int sa = 0, sw = 0, fill_a = SA - 1, fill_w = SW - 1;
+    auto advance = [&]() {
+        sa = sa + 1 == SA ? 0 : sa + 1;
+        fill_a = fill_a + 1 == SA ? 0 : fill_a + 1;
+        sw = sw + 1 == SW ? 0 : sw + 1;
+        fill_w = fill_w + 1 == SW ? 0 : fill_w + 1;
+    };
+    if constexpr (TURNS) {
+        // Waves 4 .. 7 run one barrier behind waves 0 .. 3: on every SIMD one wave reads its fragments while the other's products run.
+        // A slot's reads end before the barrier behind them, so it is staged anew from the next step on.
+        constexpr int PH = FI * FJ * HV <= 32 ? 1 : HV, HS = HV / PH;   // phases a k-tile: both halves' fragments at once where registers hold them
+        const bool late = wave >= 4;
+        landed(SW - 1 <= nk);
+        bar();
+        if (late) bar();
+        for (int t = 0; t < nk; t++) {
+            const unsigned char *a_buf = smem + sa * A_SLOT, *w_buf = smem + W_BASE + sw * W_SLOT;
 #pragma unroll
-        for (int j = 0; j < FJ; j++) {
-            const int row = BM + wn * TN + j * 16 + fr;
-            fb[j] = *reinterpret_cast<const bf16x8*>(buf + row * 128 + (((4 * wk + g) ^ g8_swz(row)) * 16));
-        }
-        constexpr int AHEAD = BM >= 256 ? 2 : FI;   // tall tiles: two A fragments on their way while one is multiplied
+            for (int ph = 0; ph < PH; ph++) {
+                bf16x8 fa[HS][FI], fb[HS][FJ];
 #pragma unroll
-        for (int i = 0; i < AHEAD; i++) read_a(i);
+                for (int h = 0; h < HS; h++) {
 #pragma unroll
-        for (int i = 0; i < FI; i++) {
-            if (i + AHEAD < FI) read_a(i + AHEAD);
-            if (AHEAD < FI) __builtin_amdgcn_sched_barrier(0);
+                    for (int j = 0; j < FJ; j++) fb[h][j] = frag(w_buf, wn * TN + j * 16 + fr, wk + ph * HS + h);
 #pragma unroll
-            for (int j = 0; j < FJ; j++)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);   // W Aᵀ
-            if (AHEAD < FI) __builtin_amdgcn_sched_barrier(0);
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave's reads of the slot are done
-        __builtin_amdgcn_sched_barrier(0);
-        slot = slot + 1 == SLOTS ? 0 : slot + 1;
-        fill = fill + 1 == SLOTS ? 0 : fill + 1;
-    }
-
-    // ---------------- the two K halves: wave w and w ^ 4 hold the same tile; each keeps half of its rows
-    f32x4 res[FH][FJ];
-    {
-        f32x4* ex = reinterpret_cast<f32x4*>(smem);
-        constexpr int FIT = SLOTS * SLOT / (8 * FH * 1024), JN = FIT < FJ ? FIT : FJ;   // fragment columns the LDS takes at once
-        static_assert(JN >= 1, "exchange area");
-#pragma unroll
-        for (int j0 = 0; j0 < FJ; j0 += JN) {
-            __syncthreads();
-#pragma unroll
-            for (int i = 0; i < FH; i++)
-#pragma unroll
-                for (int j = j0; j < j0 + JN && j < FJ; j++) {
-                    if (wk == 0) {
-                        ex[((wave * FH + i) * JN + j - j0) * 64 + lane] = acc[FH + i][j];
-                        res[i][j] = acc[i][j];
-                    } else {
-                        ex[((wave * FH + i) * JN + j - j0) * 64 + lane] = acc[i][j];
-                        res[i][j] = acc[FH + i][j];
-                    }
+                    for (int i = 0; i < FI; i++) fa[h][i] = frag(a_buf, wm * TM + i * 16 + fr, wk + ph * HS + h);
                 }
-            __syncthreads();
+                __builtin_amdgcn_sched_barrier(0);
+                if (ph == 0) {
+                    if (t + SA - 1 < nk) stage_a(t + SA - 1, fill_a);
+                    if (t + SW - 1 < nk) stage_w(t + SW - 1, fill_w);
+                }
+                if (ph == PH - 1 && late && t + 1 < nk) landed(t + SW <= nk);
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                bar();
+                __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-            for (int i = 0; i < FH; i++)
+                for (int h = 0; h < HS; h++)
 #pragma unroll
-                for (int j = j0; j < j0 + JN && j < FJ; j++) res[i][j] = res[i][j] + ex[(((wave ^ 4) * FH + i) * JN + j - j0) * 64 + lane];
+                    for (int i = 0; i < FI; i++)
+#pragma unroll
+                        for (int j = 0; j < FJ; j++)
+                            acc[ph * HS + h][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[h][j], fa[h][i], acc[ph * HS + h][i][j], 0, 0, 0);   // W Aᵀ
+                __builtin_amdgcn_s_setprio(0);
+                __builtin_amdgcn_sched_barrier(0);
+                if (ph == PH - 1 && !late && t + 1 < nk) landed(t + SW <= nk);
+                bar();
+            }
+            advance();
+        }
+        if (!late) bar();
+    } else {
+        for (int t = 0; t < nk; t++) {
+            // k-tile t has landed (what was staged behind it may still fly), and every wave is done with the slots of t - 1
+            landed(t + SW - 1 <= nk);
+            bar();
+            if (t + SA - 1 < nk) stage_a(t + SA - 1, fill_a);
+            if (t + SW - 1 < nk) stage_w(t + SW - 1, fill_w);
+            const unsigned char *a_buf = smem + sa * A_SLOT, *w_buf = smem + W_BASE + sw * W_SLOT;
+            constexpr int HS = FI * FJ <= 10 ? HV : 1;      // halves whose fragments are read together
+            constexpr int AHEAD = FI * FJ > 20 ? 2 : FI;    // few registers left: two A fragments on their way while one is multiplied
+#pragma unroll
+            for (int s0 = 0; s0 < HV; s0 += HS) {
+                bf16x8 fa[HS][FI], fb[HS][FJ];
+#pragma unroll
+                for (int h = 0; h < HS; h++) {
+#pragma unroll
+                    for (int j = 0; j < FJ; j++) fb[h][j] = frag(w_buf, wn * TN + j * 16 + fr, wk + s0 + h);
+#pragma unroll
+                    for (int i = 0; i < AHEAD; i++) fa[h][i] = frag(a_buf, wm * TM + i * 16 + fr, wk + s0 + h);
+                }
+                if (HS == 2) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int h = 0; h < HS; h++)
+#pragma unroll
+                    for (int i = 0; i < FI; i++) {
+                        if (i + AHEAD < FI) fa[h][i + AHEAD] = frag(a_buf, wm * TM + (i + AHEAD) * 16 + fr, wk + s0 + h);
+                        if (AHEAD < FI) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int j = 0; j < FJ; j++)
+                            acc[s0 + h][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[h][j], fa[h][i], acc[s0 + h][i][j], 0, 0, 0);   // W Aᵀ
+                        if (AHEAD < FI) __builtin_amdgcn_sched_barrier(0);
+                    }
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave's reads of the slots are done
+            __builtin_amdgcn_sched_barrier(0);
+            advance();
+        }
+    }
+    f32x4 res[FR][FJ];
+    if constexpr (KW == 1) {
+#pragma unroll
+        for (int i = 0; i < FR; i++)
+#pragma unroll
+            for (int j = 0; j < FJ; j++) res[i][j] = acc[0][i][j] + acc[1][i][j];
+    } else {   // waves w and w ^ 4 hold the same tile; each keeps half of its rows
+        f32x4* ex = reinterpret_cast<f32x4*>(smem);
+        static_assert(8 * FR * FJ * 1024 <= (SA * BM + SW * BN) * 128, "exchange area");
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < FR; i++)
+#pragma unroll
+            for (int j = 0; j < FJ; j++) {
+                ex[((wave * FR + i) * FJ + j) * 64 + lane] = wk == 0 ? acc[0][FR + i][j] : acc[0][i][j];
+                res[i][j] = wk == 0 ? acc[0][i][j] : acc[0][FR + i][j];
+            }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < FR; i++)
+#pragma unroll
+            for (int j = 0; j < FJ; j++) res[i][j] = res[i][j] + ex[(((wave ^ 4) * FR + i) * FJ + j) * 64 + lane];
+    }
+
+    // The tile's part of C as a buffer: rows past M lie behind its end, and so do columns past N, moved there by `at`; loads from there give 0,
+    // stores do nothing.
+    constexpr int OUT_BN = EPI == QIE_EPI_SWIGLU ? BN / 2 : BN, SZ = EPI == QIE_EPI_F32 ? 4 : 2, OUTSIDE = 1 << 31;
+    const bool quads = p.vec != 0 && (p.N & 3) == 0;   // uniform
+    const int ld = (int)p.ldc * SZ, left = (int)(p.N - nt * OUT_BN < OUT_BN ? p.N - nt * OUT_BN : OUT_BN);   // bytes of a row; columns
+    const auto c_rs = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<unsigned char*>(p.C) + (m0 * p.ldc + nt * OUT_BN) * SZ, (short)0,
+                                                        ((int)(p.M - m0 < BM ? p.M - m0 : BM) - 1) * ld + left * SZ, 0x00020000);
+    const int c_row = wrow * ld;
+    auto at = [&](int i, int col) { return (col < left ? c_row + col * SZ : OUTSIDE) + i * 16 * ld; };
+    auto put = [&](int i, int col, int n, const float (&v)[4]) {   // columns col .. col + n - 1 of the tile
+        if (quads) {
+            if (n == 4) __builtin_amdgcn_raw_buffer_store_b64(u32x2_g8{pack2(v[0], v[1]), pack2(v[2], v[3])}, c_rs, at(i, col), 0, 0);
+            else __builtin_amdgcn_raw_buffer_store_b32(pack2(v[0], v[1]), c_rs, at(i, col), 0, 0);
+        } else {
+#pragma unroll
+            for (int r = 0; r < n; r++) __builtin_amdgcn_raw_buffer_store_b16(f2bf(v[r]), c_rs, at(i, col + r), 0, 0);
+        }
+    };
+    const int col0 = wn * TN + 4 * g;
+    // residuals: all on their way at once
+    [[maybe_unused]] uint2 before[FR][FJ];
+    if constexpr (EPI == QIE_EPI_RESIDUAL) {
+        if (quads) {
+#pragma unroll
+            for (int i = 0; i < FR; i++)
+#pragma unroll
+                for (int j = 0; j < FJ; j++)
+                    before[i][j] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(c_rs, at(i, col0 + 16 * j), 0, 0));
+        } else {
+#pragma unroll
+            for (int i = 0; i < FR; i++)
+#pragma unroll
+                for (int j = 0; j < FJ; j++) {
+                    uint32_t h[4];
+#pragma unroll
+                    for (int r = 0; r < 4; r++) h[r] = __builtin_amdgcn_raw_buffer_load_b16(c_rs, at(i, col0 + 16 * j + r), 0, 0);
+                    before[i][j] = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+                }
         }
     }
 
-    if (parts > 1) {   // uniform
+    constexpr bool SPLITS = BN != 160;   // (mid::WIDE: whole only)
+    if (SPLITS && parts > 1) {   // uniform.  A wave's share of the tile meets by itself: no wave waits for the others of its workgroup
         constexpr int SLAB = BM * BN;   // floats
         const int64_t tb = (int64_t)ct * parts;
+        const int slab_at = (wave * FR * FJ * 64 + lane) * 16;
         const auto rs = __builtin_amdgcn_make_buffer_rsrc(sk.slab + (tb + part) * SLAB, (short)0, SLAB * 4, 0x00020000);
 #pragma unroll
-        for (int i = 0; i < FH; i++)
+        for (int i = 0; i < FR; i++)
 #pragma unroll
             for (int j = 0; j < FJ; j++)
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_g8, res[i][j]), rs,
-                                                       (((wave * FH + i) * FJ + j) * 64 + lane) * 16, 0, 16);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every storing wave drains
-        __syncthreads();
-        int* flag = reinterpret_cast<int*>(smem);
-        if (tid == 0) {
-            const unsigned old = __hip_atomic_fetch_add(sk.cnt + ct, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            *flag = old == (unsigned)parts - 1 ? 1 : 0;
-        }
-        __syncthreads();
-        if (*flag == 0) return;   // uniform
-        // part order: independent of who arrived last; QN parts' loads in flight (one after the other cost 0.75 us each)
-        constexpr int QN = FH * FJ >= 16 ? 1 : 16 / (FH * FJ);
-        for (int q0 = 0; q0 < parts; q0 += QN) {
-            f32x4 v[QN][FH][FJ];
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_g8, res[i][j]), rs, slab_at + (i * FJ + j) * 1024, 0, 16);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // stored
+        unsigned* cnt = sk.cnt + ct * 8 + wave;
+        unsigned old = 0;
+        if (lane == 0) old = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        old = __builtin_amdgcn_readfirstlane(old);
+        if (old != (unsigned)parts - 1) return;   // uniform
+        asm volatile("" ::: "memory");
+        // part order, this part's own from its registers: independent of who arrived last; as many of the others' on their way as registers
+        // hold (small tiles: of two workgroups a CU)
+        constexpr int FLY = KW == 2 ? 16 : FR * FJ <= 16 ? 24 : 12, IG = FR * FJ <= 8 ? FR : 1, QN = FLY / (IG * FJ) < 6 ? FLY / (IG * FJ) : 6;   // fragments; rows of them; parts
 #pragma unroll
-            for (int u = 0; u < QN; u++) {
-                const int q = q0 + u < parts ? q0 + u : parts - 1;
-                const auto rq = __builtin_amdgcn_make_buffer_rsrc(sk.slab + (tb + q) * SLAB, (short)0, SLAB * 4, 0x00020000);
+        for (int i0 = 0; i0 < FR; i0 += IG) {
+            f32x4 sum[IG][FJ];
+            for (int q0 = 0; q0 < parts; q0 += QN) {
+                f32x4 v[QN][IG][FJ];
 #pragma unroll
-                for (int i = 0; i < FH; i++)
+                for (int u = 0; u < QN; u++) {
+                    if (q0 + u >= parts || q0 + u == part) continue;
+                    const auto rq = __builtin_amdgcn_make_buffer_rsrc(sk.slab + (tb + q0 + u) * SLAB, (short)0, SLAB * 4, 0x00020000);
 #pragma unroll
-                    for (int j = 0; j < FJ; j++)
-                        v[u][i][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                                   rq, (((wave * FH + i) * FJ + j) * 64 + lane) * 16, 0, 16));
+                    for (int i = 0; i < IG; i++)
+#pragma unroll
+                        for (int j = 0; j < FJ; j++)
+                            v[u][i][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rq, slab_at + ((i0 + i) * FJ + j) * 1024, 0, 16));
+                }
+#pragma unroll
+                for (int u = 0; u < QN; u++) {
+                    if (q0 + u >= parts) break;
+#pragma unroll
+                    for (int i = 0; i < IG; i++)
+#pragma unroll
+                        for (int j = 0; j < FJ; j++) {
+                            const f32x4 w = q0 + u == part ? res[i0 + i][j] : v[u][i][j];
+                            sum[i][j] = q0 + u == 0 ? w : sum[i][j] + w;
+                        }
+                }
             }
 #pragma unroll
-            for (int u = 0; u < QN; u++) {
-                if (q0 + u >= parts) break;
+            for (int i = 0; i < IG; i++)
 #pragma unroll
-                for (int i = 0; i < FH; i++)
-#pragma unroll
-                    for (int j = 0; j < FJ; j++) res[i][j] = q0 + u == 0 ? v[u][i][j] : res[i][j] + v[u][i][j];
-            }
+                for (int j = 0; j < FJ; j++) res[i0 + i][j] = sum[i][j];
         }
-        if (tid == 0) __hip_atomic_store(sk.cnt + ct, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (lane == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 
     // ---------------- epilogue.  D = W Aᵀ: a lane holds row m = lane & 15 and the columns 4 g .. 4 g + 3 of a fragment, one
     // 8- (fp32: 16-) byte store where C's rows allow it
-    const bool vec = p.vec != 0;
-    const int64_t row0 = m0 + wm * TM + wk * (FH * 16) + fr;
     if constexpr (EPI == QIE_EPI_SWIGLU) {
 #pragma unroll
         for (int m = 0; m < (FJ + 1) / 2; m++) {
             constexpr int PAIRS = FJ / 2;
             const int n = m < PAIRS ? 4 : 2;   // outputs
-            const int64_t col = nt * TN + (TN / 2) * wn + 16 * m + n * g;
 #pragma unroll
-            for (int i = 0; i < FH; i++) {
-                const int64_t row = row0 + i * 16;
-                if (row >= p.M) continue;
+            for (int i = 0; i < FR; i++) {
                 float h[4];
 #pragma unroll
                 for (int r = 0; r < n; r++) {
@@ -250,38 +379,30 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
                     const float uu = rbf(v[2 + (r & 1)]);
                     h[r] = uu * rbf(gg * (1.0f / (1.0f + expf(-gg))));
                 }
-                uint16_t* dst = p.C + row * p.ldc + col;
-                if (vec && col + n <= p.N) {
-                    if (n == 4) *reinterpret_cast<uint2*>(dst) = make_uint2(pack2(h[0], h[1]), pack2(h[2], h[3]));
-                    else *reinterpret_cast<uint32_t*>(dst) = pack2(h[0], h[1]);
-                } else {
-#pragma unroll
-                    for (int r = 0; r < n; r++)
-                        if (col + r < p.N) dst[r] = f2bf(h[r]);
-                }
+                put(i, (TN / 2) * wn + 16 * m + n * g, n, h);
             }
         }
     } else if constexpr (EPI == kEpiQkv) {
-        qkv_tail<FH, FJ, EARLY>(p, tail, row0, nt * BN + wn * TN + 4 * g, res, ops);
+        qkv_tail<FR, FJ, EARLY>(p, tail, row0, nt * BN + wn * TN + 4 * g, res, ops);
     } else {
 #pragma unroll
         for (int j = 0; j < FJ; j++) {
-            const int64_t col = nt * BN + wn * TN + j * 16 + 4 * g;
             float bias[4] = {0.f, 0.f, 0.f, 0.f};
-            if constexpr (EPI == QIE_EPI_STORE) quad_bias(p, col, bias);
+            if constexpr (EPI == QIE_EPI_STORE) quad_bias(p, nt * BN + col0 + 16 * j, bias);
 #pragma unroll
-            for (int i = 0; i < FH; i++) {
-                const int64_t row = row0 + i * 16;
-                if (row >= p.M) continue;
+            for (int i = 0; i < FR; i++) {
                 const f32x4 v = res[i][j];
                 if constexpr (EPI == QIE_EPI_F32) {
-                    store_quad_f32(reinterpret_cast<float*>(p.C) + row * p.ldc + col, v, vec, p.N - col);
-                } else if constexpr (EPI == QIE_EPI_RESIDUAL) {
-                    uint16_t* dst = p.C + row * p.ldc + col;
-                    add_quad(dst, quad_before(dst, vec, p.N - col), v, vec, p.N - col);
+                    if (quads) {
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_g8, v), c_rs, at(i, col0 + 16 * j), 0, 0);
+                    } else {
+#pragma unroll
+                        for (int r = 0; r < 4; r++) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[r]), c_rs, at(i, col0 + 16 * j + r), 0, 0);
+                    }
                 } else {
-                    const float o[4] = {v[0] + bias[0], v[1] + bias[1], v[2] + bias[2], v[3] + bias[3]};
-                    store_quad(p.C + row * p.ldc + col, o, vec, p.N - col);
+                    float o[4] = {v[0] + bias[0], v[1] + bias[1], v[2] + bias[2], v[3] + bias[3]};
+                    if constexpr (EPI == QIE_EPI_RESIDUAL) sum_quad(before[i][j], v, o);
+                    put(i, col0 + 16 * j, 4, o);
                 }
             }
         }
@@ -290,17 +411,17 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
 
 // ---------------------------------------------------------------- the plan
 namespace {
-template <int EPI, int BM, int BN, int SLOTS>
+template <int EPI, int BM, int BN, int SA, int SW, int KW, bool TURNS>
 int launch_mid_t(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, const TailOf<EPI>& tail, hipStream_t st) {
-    const void* fn = (const void*)gemm_mid_kernel<EPI, BM, BN, SLOTS>;
-    constexpr size_t shm = (size_t)SLOTS * (BM + BN) * 128;
+    const void* fn = (const void*)gemm_mid_kernel<EPI, BM, BN, SA, SW, KW, TURNS>;
+    constexpr size_t shm = (size_t)(SA * BM + SW * BN) * 128;
     static bool raised = false;
     if (!raised) {
         QIE_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
         raised = true;
     }
     const int tiles = pl.n_mt * pl.n_nt, whole = sk.splitk > 1 ? pl.whole : tiles;
-    hipLaunchKernelGGL((gemm_mid_kernel<EPI, BM, BN, SLOTS>), dim3((unsigned)(whole + (tiles - whole) * sk.splitk)), dim3(512), shm,
+    hipLaunchKernelGGL((gemm_mid_kernel<EPI, BM, BN, SA, SW, KW, TURNS>), dim3((unsigned)(whole + (tiles - whole) * sk.splitk)), dim3(512), shm,
                        st, p, pl.n_mt, pl.n_nt, band_height(pl.n_mt, BM, BN, 32 * mid::shape(pl.tile).per_cu), whole, sk, tail);
     QIE_LAUNCH_CHECK();
     return 0;
@@ -309,18 +430,20 @@ int launch_mid_t(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, co
 template <int EPI>
 int launch_mid(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, hipStream_t st, const TailOf<EPI>& tail = {}) {
     switch (pl.tile) {
-        case 0: return launch_mid_t<EPI, 64, 64, 5>(p, pl, sk, tail, st);
-        case 1: return launch_mid_t<EPI, 64, 128, 3>(p, pl, sk, tail, st);
-        case 2: return launch_mid_t<EPI, 128, 64, 3>(p, pl, sk, tail, st);
-        case 3: return launch_mid_t<EPI, 128, 128, 4>(p, pl, sk, tail, st);
-        case 4: return launch_mid_t<EPI, 192, 128, 4>(p, pl, sk, tail, st);
-        case 5: return launch_mid_t<EPI, 256, 128, 3>(p, pl, sk, tail, st);
-        case 6: return launch_mid_t<EPI, 320, 64, 3>(p, pl, sk, tail, st);
-        case 7: return launch_mid_t<EPI, 320, 128, 2>(p, pl, sk, tail, st);
-        case 8: return launch_mid_t<EPI, 128, 160, 4>(p, pl, sk, tail, st);
-        case 9: return launch_mid_t<EPI, 192, 160, 3>(p, pl, sk, tail, st);
-        case 10: return launch_mid_t<EPI, 256, 160, 3>(p, pl, sk, tail, st);
-        default: return launch_mid_t<EPI, 320, 160, 2>(p, pl, sk, tail, st);
+        case 0: return launch_mid_t<EPI, 64, 64, 5, 5, 2, false>(p, pl, sk, tail, st);
+        case 1: return launch_mid_t<EPI, 64, 128, 3, 3, 2, false>(p, pl, sk, tail, st);
+        case 2: return launch_mid_t<EPI, 128, 64, 3, 3, 2, false>(p, pl, sk, tail, st);
+        case 3:
+            if (p.K < 1792) return launch_mid_t<EPI, 128, 128, 4, 4, 1, false>(p, pl, sk, tail, st);
+            return launch_mid_t<EPI, 128, 128, 4, 4, 2, true>(p, pl, sk, tail, st);
+        case 4: return launch_mid_t<EPI, 192, 128, 4, 4, 2, true>(p, pl, sk, tail, st);
+        case 5: return launch_mid_t<EPI, 256, 128, 3, 3, 2, true>(p, pl, sk, tail, st);
+        case 6: return launch_mid_t<EPI, 320, 64, 3, 3, 1, false>(p, pl, sk, tail, st);
+        case 7: return launch_mid_t<EPI, 320, 128, 2, 4, 1, true>(p, pl, sk, tail, st);
+        case 8: return launch_mid_t<EPI, 128, 160, 4, 4, 1, true>(p, pl, sk, tail, st);
+        case 9: return launch_mid_t<EPI, 192, 160, 3, 3, 1, true>(p, pl, sk, tail, st);
+        case 10: return launch_mid_t<EPI, 256, 160, 3, 3, 1, true>(p, pl, sk, tail, st);
+        default: return launch_mid_t<EPI, 320, 160, 2, 3, 1, false>(p, pl, sk, tail, st);
     }
 }
 }  // namespace
@@ -328,12 +451,12 @@ int launch_mid(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, hipS
 int gemm_mid(const qie_linear_args* a, const GemmParams& p, const QkvTail* tail, hipStream_t st, bool* launched) {
     *launched = false;
     const mid::Plan pl = mid::choose(a->M, a->epilogue == QIE_EPI_SWIGLU ? 2 * a->N : a->N, a->K, device_cu_count());
-    if (pl.tile < 0) return 0;
+    if (pl.tile < 0 || a->ldy > 1 << 20) return 0;   // (a tile of C by 32-bit offsets)
     G8Split sk{1, nullptr, nullptr};
     const int64_t cut = (int64_t)pl.n_mt * pl.n_nt - pl.whole;
     if (pl.splitk > 1 && cut > 0) {
         const int64_t floats = cut * pl.splitk * mid::shape(pl.tile).bm * mid::shape(pl.tile).bn;
-        if (g8_workspace(st, (int)cdiv(floats, 65536), (int)cut, &sk) == 0) sk.splitk = pl.splitk;
+        if (g8_workspace(st, (int)cdiv(floats, 65536), (int)cut * 8, &sk) == 0) sk.splitk = pl.splitk;
     }
     *launched = true;
     if (tail) return launch_mid<kEpiQkv>(p, pl, sk, st, *tail);

@@ -1,0 +1,48 @@
+"""What every tile of k_gemm_mid.hip writes: its residual and SwiGLU epilogues, whole and split over K, by quads and by elements, against fp32
+products; nothing behind a row's columns or behind the last row.  128 x 128 in both of its forms (K on either side of 1,792)."""
+import numpy as np
+import pytest
+
+import gpu_util as G
+from gemm_route import routes
+from qwen_inference_engine_amd import _lib
+from test_gpu_gemm_mid import bf16, linear, products
+
+pytestmark = pytest.mark.gpu
+
+# rows, weight rows, K, tile, parts
+SHAPES = [(17, 72, 64, 0, 1), (33, 72, 2048, 0, 4), (17, 16500, 64, 1, 1), (64, 8200, 4096, 1, 3), (65, 8200, 1024, 2, 1), (129, 4000, 4096, 2, 2),
+          (301, 9728, 896, 3, 1), (128, 8200, 4096, 3, 3), (131, 11014, 3712, 4, 2), (210, 9278, 6464, 5, 3), (640, 4000, 4096, 6, 2),
+          (257, 8338, 11264, 7, 3), (127, 16500, 64, 8, 1), (640, 8200, 448, 9, 1)]
+
+
+def test_the_shapes_take_their_tiles():
+    assert [(r["tile"], r["splitk"]) for r in routes([s[:3] for s in SHAPES])] == [s[3:] for s in SHAPES]
+
+
+@pytest.mark.parametrize("M,rows,K,tile,parts", SHAPES)
+@pytest.mark.parametrize("odd", [0, 1])
+@pytest.mark.parametrize("epi", ["residual", "swiglu"])
+def test_writes_its_part_of_the_rows(qlib, oracle, M, rows, K, tile, parts, odd, epi):
+    N = rows // 2 if epi == "swiglu" else rows
+    N -= odd                      # odd: element by element
+    ld = N + (4 if not odd else 3)
+    x, y0 = bf16((M, K), 1.0, 11), bf16((M + 1, ld), 1.0, 12)
+    y = G.dev(y0)
+    if epi == "residual":
+        w = bf16((N, K), K ** -0.5, 13)
+        linear(G.dev(x), [G.dev(w)], [], M, K, N, y, _lib.QIE_EPI_RESIDUAL, ldy=ld)
+        acc, scale = products(x, w)
+        want = G.bf(y0)[:M, :N] + G.bf(oracle.f32_to_bf16(acc))
+        # bf16(res + bf16(acc)): an ulp of either rounding
+        tol = 2.0 ** -7 * (np.abs(acc) + np.abs(want)) + 1e-5 * scale
+    else:
+        wg, wu = bf16((N, K), 1.5 * K ** -0.5, 14), bf16((N, K), K ** -0.5, 15)
+        linear(G.dev(x), [G.dev(wg), G.dev(wu)], [], M, K, N, y, _lib.QIE_EPI_SWIGLU, ldy=ld)
+        (g, gs), (u, us) = products(x, wg), products(x, wu)
+        want = u / (1.0 + np.exp(-g)) * g
+        # |silu'| <= 1.1; three bf16 roundings (gate, silu, product) and one of the up sum
+        tol = 2.0 ** -7 * (np.abs(want) + 1.1 * np.abs(u) * np.abs(g)) + 1e-5 * (1.1 * np.abs(u) * gs + np.abs(g) * us)
+    got = G.host_bf16(y)
+    assert (np.abs(G.bf(got)[:M, :N] - want) <= tol).all()
+    assert np.array_equal(got[:M, N:], y0[:M, N:]) and np.array_equal(got[M], y0[M])
