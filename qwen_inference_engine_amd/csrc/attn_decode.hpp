@@ -3,6 +3,8 @@
 // (k_persist.hip) runs the SAME body (same arithmetic, bit-identical outputs) as one of its
 // roles.  Replaces selfattention (layers/src/self_attension.cu:10-149) for one query row.
 #pragma once
+#include <type_traits>
+
 #include "qie_common.hpp"
 #include "../../include/qie/qie_ops.h"
 
@@ -38,9 +40,9 @@ __device__ __forceinline__ void buf_lds16(__amdgpu_buffer_rsrc_t rs, uint16_t* l
 // ---------------------------------------------------------------------------
 // Fused decode attention: q-projection post-processing (qk-norm + RoPE) in the
 // prologue, KV append of the new token (qkv_post fused away), split-K over the context,
-// and the split combine done by the last arriving workgroup of each (row, kv head):
-// write-through (sc1) partials + ticket, one agent acquire in the combiner.
-// Grid: (nkv * nsplit_max, B); row m has one query token at position pos[m].
+// and the split combine done by the last arriving wave of each (row, kv head, wave's heads):
+// write-through (sc1) partials + ticket, sc1 loads in the combiner.
+// Grid: (nsplit_max, nkv, B); row m has one query token at position pos[m].
 struct DecodeAttnParams {
     const uint16_t* qkv;      // [B][(nq + 2 nkv) * HD] projection output (bias added)
     const int32_t* pos;
@@ -51,27 +53,22 @@ struct DecodeAttnParams {
     uint16_t* kc;
     uint16_t* vc;
     KvMap km;
-    int layer, nkv, nq, max_ctx, nsplit_max;
+    int layer, nkv, nq, G, max_ctx, nsplit_max;   // G = nq / nkv
     int splits_target;        // ~splits per (row, kv head) at long context
-    int dbg;                  // timing experiments only (QIE_DEC_DBG): 1 no combine,
-                              // 8/16 stop after prologue / P.V, 64 exit at once
-    int sc1;                  // combine reads the partials with sc1 loads instead of an acquire
+    int dbg;                  // timing experiments only (QIE_DEC_DBG): 1 no combine, 64 exit at once
     int pre_roped;            // q and the new k arrive rotated by the QKV projection's epilogue
                               // (REF numerics, no qk-norm): the prologue only moves them
     float eps;
     int numerics;
     float* part_o;            // [B][nq][nsplit_max][HD]
     float* part_ml;           // [B][nq][nsplit_max][2]
-    unsigned* counters;       // [B][nkv], zero at rest
+    unsigned* counters;       // [B][nkv][waves][kDecMTicket], zero at rest
     uint16_t* out;            // [B][nq * HD]
     // engine-maintained RoPE row of each sequence's CURRENT position (finalize / set_state
     // write it, tagged with the position; [B][rope_cur_stride(HD)]): the prologue's RoPE
-    // loads need no position, so with the speculative K / V step every load of the launch
-    // goes out at once.  Null (operator API) or a stale tag: the table row at pos.
+    // loads need no position, so they go out before it is known.  Null (operator API) or a stale tag: the table row at pos.
     const float* rc;
-    int pv3;                  // P.V with three bf16 parts of P (else two; dev A/B)
-    int spec_ok;              // the speculative K / V step may be issued (see fill_dec_params)
-    int ks;                   // keys per block step (host: picks the kernel instance)
+    int spec_ok;              // the speculative K loads may be issued (see fill_dec_params)
 };
 
 constexpr int kDecMaxSplits = 512;   // 64k keys per (row, kv head)
@@ -124,47 +121,42 @@ __device__ __forceinline__ void split_bf16x8(const float* e, uint4* parts) {
 }
 
 // ---------------------------------------------------------------------------
-// Decode attention on MFMA (default decode path).  The q heads of one kv head
-// (G <= 8, padded to 16) play the role of the 16 "query rows" of the prefill
-// kernel above, so GQA decode is a 16 x 32 x HD flash step per wave:
-//   S^T = K . Q^T : A = K rows straight from HBM into registers (lane: key l&15,
-//                   8 contiguous d), B = Q^T from LDS (bf16 after norm + RoPE);
-//   O  += P . V   : A = P from the S^T accumulators, split into bf16 hi + lo parts
-//                   (two MFMAs) so the fp32 probabilities keep ~16 mantissa bits;
-//                   B = V through a per-wave LDS slot read with ds_read_b64_tr_b16.
-// Block = (kv head, split) x 4 waves; a block step covers 128 keys (32 per wave);
-// waves run an online softmax, are merged in LDS, and the splits are merged by
-// the last-arriving block (release / acquire, as the VALU kernel).  The VALU
-// kernel spent ~7 us of ~11 in dot products and cross-lane reductions here.
-constexpr int kDecMStep = 128;      // keys per block step (4 waves x 32)
+// Decode attention on MFMA.  The q heads of one kv head (G <= 8, padded to 16) play the role of the 16 "query rows" of the prefill
+// kernel.  Workgroup = (split, kv head, row of the batch); a step covers 128 keys, 32 for each of four waves, and a wave goes through its
+// own keys without a look at the others':
+//   S^T = K . Q^T : A = K rows straight from memory into registers (lane: key l & 15, 8 contiguous d), B = Q^T from LDS (bf16 after
+//                   norm + RoPE).  D: lane = head l & 15, keys 16 t + 4 (l >> 4) + r of tiles t = 0, 1;
+//   O  += P . V   : those 8 probabilities of a lane are A's 8 k slots as they lie (k slot 8 g + 4 t + r is key 16 t + 4 g + r), in three
+//                   bf16 parts (hi, mid, lo: the 24 bits of the fp32 value, so every product is the fp32 product); B = the V rows in that
+//                   order, transposed by ds_read_b64_tr_b16 out of LDS that only this wave writes and reads.
+// The waves' (max, sum, O) meet in LDS once per split, the splits in memory, by the last-arriving workgroup.
+// What it waits for is memory and instruction latency, at one wave a SIMD (Qwen2-7B, 2,049 keys: 4 MB of K / V in 68 workgroups), so the
+// layout spares instructions and meetings.  With the scores of all 128 keys exponentiated and split by every wave, each for its slice of d,
+// a step had two barriers and took 1.7 us behind its loads, now 0.9; with one ticket a kv head, its workgroup alone read all splits back:
+// 2.7 us for 17, now 1.8 by four waves on CUs of their own.  A launch, by time stamps inside it, before / now: Qwen2-0.5B at 129 keys 5.5 / 4.0
+// us, 7 rows at 700 8.1 / 5.3, Qwen2-7B at 2,049 9.1 / 7.7, 4 rows at 1,500 9.9 / 7.3, 8 at 1,025 12.6 / 9.7, Qwen3-14B at 6,001 15.0 / 11.7.
+constexpr int kDecMStep = 128;      // keys per step
+constexpr int kDecMWaves = 4;       // waves that have keys
 constexpr int kDecMSplits = 32;     // default split target
+constexpr int kDecMTicket = 32;     // a ticket's words: 128 bytes (16 tickets in one line took 2 us of the 17 splits' adds)
 constexpr int kDecMOneSplit = 2;    // contexts of up to this many steps run as ONE split
 
-__host__ __device__ __forceinline__ int decm_chunk(int ctx, int target, int ks = kDecMStep) {
+__host__ __device__ __forceinline__ int decm_chunk(int ctx, int target) {
     // Short contexts: one block walks both steps instead of two one-step splits that pay
     // the publish + ticket + combine round trips (Qwen2-0.5B, ctx 129-256: 8.8 -> 7.4 us
     // per launch, 1,235 -> 1,271 tok/s).  Longer contexts want the CUs: a split's K/V comes
-    // through one CU, so at ctx 2k ten two-step splits took 13.1 us against 10.5 for twenty
-    // one-step ones — also with the second step's loads issued up front (13.6 vs 10.7,
-    // measured and dropped: that second register set halved the occupancy).
-    if (ctx <= kDecMOneSplit * ks) return kDecMOneSplit * ks;
-    const int per = ks * target;
-    const int steps = (ctx + per - 1) / per;
-    return ks * (steps < 1 ? 1 : steps);
+    // through one CU.
+    if (ctx <= kDecMOneSplit * kDecMStep) return kDecMOneSplit * kDecMStep;
+    const int per = kDecMStep * target;
+    return ctx <= per ? kDecMStep : kDecMStep * ((ctx + per - 1) / per);
+}
+// splits of a context: chunks of one or two steps without a division
+__host__ __device__ __forceinline__ int decm_splits(int ctx, int chunk) {
+    if (chunk == kDecMStep) return (ctx + kDecMStep - 1) / kDecMStep;
+    if (chunk == 2 * kDecMStep) return (ctx + 2 * kDecMStep - 1) / (2 * kDecMStep);
+    return (ctx + chunk - 1) / chunk;
 }
 
-
-// ---------------------------------------------------------------------------
-// Decode attention, MFMA: as the prefill kernel's 16-row flash step, but the 4 waves of
-// a block split the head dimension for P.V instead of the keys, so no cross-wave
-// softmax merge is needed:
-//   * S^T for the step's 128 keys: wave w computes keys 32w..32w+31 (2 MFMA tiles),
-//     writes the raw dots to LDS, one barrier, then EVERY wave holds all 128 scores;
-//   * each wave runs the (identical) online softmax over the 128 keys itself and
-//     accumulates O for ITS d-slice (HD/4 dims: 2 tiles at hd 128) over the 4 key
-//     blocks of 32 (P in natural key order, V slice via ds_read_b64_tr_b16);
-//   * the split's partial O leaves straight from the accumulators (the v1 kernel's
-//     LDS merge of 4 waves cost ~2.7 us of a 13.5 us launch).
 struct DecPro {
     uint4 raw, nraw;
     float4 c0, s0, c1, s1;
@@ -280,113 +272,132 @@ __device__ __forceinline__ void dec_pro_finish(const DecodeAttnParams& a, DecPro
     }
 }
 
-// Body of the decode attention for workgroup (bx, by); true when this workgroup wrote a
-// combined (row, kv head) output (its stores are write-through, sc1).
+// Body of the decode attention for split s of kv head g, batch row by.
 // Hooks of the body (X): the stand-alone kernel runs it with AttnNoHook — q / k / v rows from
 // a.qkv, outputs to a.out.  The persistent decode kernel (k_persist.hip) passes a hook whose
 // gather() fills the q / k / v row image (a.qkv points at it) from the projection's hand-off
-// granules AFTER this block's K / V loads are issued (they need no q), and whose out2 / out4
-// take the block's output values (to publish them as granules).  The arithmetic is the same.
+// granules AFTER this block's K / V loads are issued (they need no q), and whose out4
+// takes the block's output values (to publish them as granules).  The arithmetic is the same.
 struct AttnNoHook {
     static constexpr bool on = false;
     __device__ void gather() {}
-    __device__ void out1(int64_t, uint16_t) {}
     __device__ void out4(int64_t, unsigned long long) {}
 };
 
-template <int HD, bool PG, int NWA, bool PR, int KS, class X = AttnNoHook>
-__device__ __forceinline__ bool attn_decode_mfma2_body(const DecodeAttnParams& a, const int bx, const int by,
+template <int HD, bool PG, int NWA, bool PR, class X = AttnNoHook>
+__device__ __forceinline__ void attn_decode_mfma2_body(const DecodeAttnParams& a, const int g, const int s, const int by,
                                                        X* hook = nullptr) {
 #pragma clang fp contract(off)
+    constexpr int KS = kDecMStep;
     constexpr int LPT = HD / 8;          // prologue: lanes per head row
     constexpr int KSTEPS = HD / 32;      // MFMA k-steps over d for S
-    constexpr int CPR = HD / 8;          // 16-byte chunks per K row
-    constexpr int DW = HD / NWA;         // output dims per wave
-    constexpr int DTW = DW / 16;         // output d tiles per wave (2 at hd 128 x 4 waves, else 1)
-    constexpr int CPW = DW / 8;          // 16-byte chunks of a V row per wave
-    constexpr int VCH = KS * CPW / 64;   // V chunks per lane per step
-    constexpr int TPW = KS / (16 * NWA);  // 16-key S tiles per wave per step
+    constexpr int CPR = HD / 8;          // 16-byte chunks per row
+    constexpr int DT = HD / 16;          // output d tiles
+    constexpr int VCH = 32 * CPR / 64;   // V chunks per lane per step
     constexpr int NT = 64 * NWA;         // threads
-    static_assert(DTW >= 1 && TPW >= 1, "attn_decode: NWA too large for HD");
+    static_assert(NWA >= kDecMWaves, "attn_decode: four waves have keys");
     __shared__ __attribute__((aligned(16))) uint16_t q_s[16][HD];
     __shared__ __attribute__((aligned(16))) uint16_t kv_new[2][HD];
-    __shared__ __attribute__((aligned(16))) uint16_t v_s[NWA][KS * DW];
-    __shared__ __attribute__((aligned(16))) float s_s[16][KS + 4];
-    __shared__ int last_flag;
+    __shared__ __attribute__((aligned(16))) uint16_t v_s[kDecMWaves][32 * HD];   // V rows of a wave's keys; behind the steps its O
+    __shared__ __attribute__((aligned(16))) float2 ml_s[kDecMWaves][16];
 
     const int64_t m = by;
-    const int g = bx / a.nsplit_max, s = bx % a.nsplit_max;
-    const int G = a.nq / a.nkv;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int G = a.G;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int fr = lane & 15, gq = lane >> 4;
     const int grp = tid / LPT, dl = tid % LPT;
+    const bool keyed = wave < kDecMWaves;
     const int QKVD = (a.nq + 2 * a.nkv) * HD;
     const uint16_t* row = a.qkv + m * (int64_t)QKVD;
     const int64_t head_off = kv_run_off(a.km, (int64_t)a.layer * a.nkv + g, HD);
     uint16_t* kb = a.kc + head_off;
     uint16_t* vb = a.vc + head_off;
-    uint4 kf[TPW][KSTEPS], vr[VCH];
-    // step loads of keys [kb0, kb0 + 128), rows past `last` re-read row `last`
-    auto load_step_at = [&](int kb0, int last) {
-        // a 128-key step never straddles a page (chunks and pages are multiples of 128)
-        const int64_t so = kv_tok<PG>(a.km, m, kb0, HD);
+    // steps in flight; at head dim 128 one, in 250 registers: a second workgroup on the CU hides more than a second step (and the persistent
+    // kernel has no registers for it)
+    constexpr int SETS = X::on || HD == 128 ? 1 : 2;
+    uint4 kf[SETS][2][KSTEPS], vr[SETS][VCH];   // [step % SETS]
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, SETS - 1> odd{};
+    // loads of this wave's 32 of the `n` keys (128 at most count) that start at element `so` of a run; rows past them read as zeros
+    // (a 128-key step never straddles a page: chunks and pages are multiples of 128)
+    const int k_at = 32 * wave * HD * 2;
+    auto load_k = [&](auto x, int64_t so, int n) {
+        const auto rs = __builtin_amdgcn_make_buffer_rsrc(kb + so, (short)0, n * HD * 2, 0x00020000);
 #pragma unroll
-        for (int t = 0; t < TPW; t++) {
-            const int key = min(kb0 + 16 * TPW * wave + 16 * t + fr, last);
+        for (int t = 0; t < 2; t++)
 #pragma unroll
             for (int ks = 0; ks < KSTEPS; ks++)
-                kf[t][ks] = *reinterpret_cast<const uint4*>(kb + so + (int64_t)(key - kb0) * HD + 32 * ks + 8 * gq);
-        }
-#pragma unroll
-        for (int i = 0; i < VCH; i++) {
-            const int c = lane + 64 * i;
-            const int key = min(kb0 + c / CPW, last);
-            vr[i] = *reinterpret_cast<const uint4*>(vb + so + (int64_t)(key - kb0) * HD + wave * DW + (c % CPW) * 8);
-        }
+                kf[x][t][ks] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, k_at + (16 * t + fr) * HD * 2 + 16 * gq + 64 * ks, 0, 0));
     };
-    // Speculative step: the split of every context of 257 ..
+    auto load_v = [&](auto x, int64_t so, int n) {
+        const auto rs = __builtin_amdgcn_make_buffer_rsrc(vb + so, (short)0, n * HD * 2, 0x00020000);
+#pragma unroll
+        for (int i = 0; i < VCH; i++)
+            vr[x][i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, k_at + lane * 16 + i * 1024, 0, 0));
+    };
+    // Speculative step (contiguous cache): the split of every context of 257 ..
     // 128 * splits keys is keys [128 s, 128 s + 128) (decm_chunk's one-step rule), so its
-    // K / V loads go out with the position load instead of one HBM round trip behind it.
+    // K loads go out with the position load instead of one HBM round trip behind it.
     // The rotated q / k / v row goes out first (position-independent): vmcnt retires in
-    // order, and the prologue that waits for it must not wait behind the whole K / V step.
+    // order, and the prologue that waits for it must not wait behind the whole step.
     // Without the pre-rotation the same holds when the engine keeps the current position's
     // RoPE row (a.rc, tagged with the position): the prologue's loads then need no position
     // either, and a stale tag (a position set some other way) reloads the table row.
-    // (Paged, measured: the step's page from the block-table entry of (row,
-    // 128 s) needs no position either, but the speculative form ran config 4 at 3,563 vs
-    // 3,624 tok/s for the plain one — the table round trip still precedes the K / V loads.)
-    constexpr bool SPEC = !PG;
-    const bool spec = (PR || a.rc != nullptr) && a.spec_ok;   // uniform
+    // (Paged: the pages of a one-step and of a two-step split come with the position; the K / V loads themselves, issued
+    // ahead by them, made eight users slower: 3,563 tok/s against 3,624.)
+    const bool ahead = PR || a.rc != nullptr;   // uniform: the prologue's loads need no position
+    const bool spec = !PG && ahead && a.spec_ok;
     const int p = a.pos[m];
+    int page1 = 0, page2 = 0;
+    if constexpr (PG) {
+        const int32_t* tb = a.km.table + m * a.km.max_pages;
+        page1 = tb[min((KS * s) >> a.km.shift, a.km.max_pages - 1)];
+        page2 = tb[min((2 * KS * s) >> a.km.shift, a.km.max_pages - 1)];
+    }
     const float* rcm = a.rc ? a.rc + m * rope_cur_stride(HD) : a.cs;
     const int rtag = a.rc ? __float_as_int(rcm[0]) : -1;
     DecPro pr;
-    if (SPEC && spec) {
+    if (spec) {
         if constexpr (X::on) {   // the row is gathered after the K / V step is in flight
-            load_step_at(KS * s, a.max_ctx - 1);
+            if (keyed) load_k(even, kv_tok<false>(a.km, m, KS * s, HD), min(KS, a.max_ctx - KS * s));
             __builtin_amdgcn_sched_barrier(0);
             hook->gather();
             pr = dec_pro_issue<HD, PR>(a, row, g, G, grp, dl, rcm + 8, rcm + 8 + HD / 2, false);
         } else {
             pr = dec_pro_issue<HD, PR>(a, row, g, G, grp, dl, rcm + 8, rcm + 8 + HD / 2, false);
             __builtin_amdgcn_sched_barrier(0);
-            load_step_at(KS * s, a.max_ctx - 1);
+            if (keyed) load_k(even, kv_tok<false>(a.km, m, KS * s, HD), min(KS, a.max_ctx - KS * s));
             __builtin_amdgcn_sched_barrier(0);
         }
-    } else if constexpr (X::on) {
-        hook->gather();
+    } else {
+        if constexpr (X::on) hook->gather();
+        if (ahead) pr = dec_pro_issue<HD, PR>(a, row, g, G, grp, dl, rcm + 8, rcm + 8 + HD / 2, false);
     }
     const int ctx = p + 1;
-    const int chunk = decm_chunk(ctx, a.splits_target, KS);
-    const int nsplit = (ctx + chunk - 1) / chunk;
-    if (s >= nsplit || QIE_DBG(a.dbg & 64)) return false;
+    const int chunk = decm_chunk(ctx, a.splits_target);
+    const int nsplit = decm_splits(ctx, chunk);
+    if (s >= nsplit || QIE_DBG(a.dbg & 64)) return;
     const int t0 = s * chunk, t1 = min(ctx, t0 + chunk);
     const int nstep = (t1 - t0 + KS - 1) / KS;
     const bool has_new = (t1 == ctx);
-    auto load_step = [&](int st) { load_step_at(t0 + st * KS, t1 - 1); };
+    auto run_of = [&](int tok) -> int64_t {   // kv_tok of the first key of a step
+        if constexpr (PG) {
+            const int page = tok == KS * s ? page1 : tok == 2 * KS * s ? page2 : a.km.table[m * a.km.max_pages + (tok >> a.km.shift)];
+            return (int64_t)page * a.km.stride + (int64_t)(tok & ((1 << a.km.shift) - 1)) * HD;
+        } else {
+            return kv_tok<false>(a.km, m, tok, HD);
+        }
+    };
+    auto keys_of = [&](int st) { return min(KS, t1 - t0 - st * KS); };
+    auto load_step = [&](auto x, int st) {
+        const int64_t so = run_of(t0 + st * KS);
+        load_k(x, so, keys_of(st));
+        load_v(x, so, keys_of(st));
+    };
 
-    // ---------------- loads: prologue operands, then step 0's K tiles and V slice
-    if (SPEC && spec) {
+    // ---------------- loads: prologue operands, then the first step's K, and its V behind the prologue: a CU has some 40 KB of loads in
+    // flight, and a wave that has more to send waits
+    if (ahead) {
         pr.pro = pr.is_q || ((pr.is_k || pr.is_v) && has_new);
         if (!PR && rtag != p)   // uniform: the kept row is not this position's
             dec_rope_load<HD>(pr, dl, a.cs + (int64_t)p * (HD / 2), a.sn + (int64_t)p * (HD / 2));
@@ -398,297 +409,257 @@ __device__ __forceinline__ bool attn_decode_mfma2_body(const DecodeAttnParams& a
     // (uniform) the speculative step is this split's first step iff the split starts at key
     // KS s: one-step splits, and split 0 of every context (the one-split contexts of <= 2
     // steps, Qwen2-0.5B's ctx 129-256, re-issued the same loads behind the position: +1.2 us)
-    if (!(SPEC && spec) || t0 != KS * s) load_step(0);
-    if (SPEC && spec) {
-        // rows past the context hold whatever the cache has there: their scores are masked
-        // to -inf (P = 0), and their V rows are zeroed so that 0 * V stays 0 for any bits
-#pragma unroll
-        for (int i = 0; i < VCH; i++)
-            if (t0 + (lane + 64 * i) / CPW >= t1) vr[i] = make_uint4(0, 0, 0, 0);
-    }
+    // (rows past the context hold whatever the cache has there: their scores are masked to -inf)
+    const int64_t so0 = run_of(t0);
+    if (keyed && (!spec || t0 != KS * s)) load_k(even, so0, keys_of(0));
+    // (the new token's place is asked for by the splits that do not hold it too: p is in the row's pages)
     dec_pro_finish<HD, PR>(a, pr, dl, grp, kv_tok<PG>(a.km, m, p, HD), kb, vb, q_s, kv_new);
+    if (keyed) load_v(even, so0, keys_of(0));
+    if (SETS > 1 && keyed && nstep > 1) load_step(odd, 1);
     for (int idx = tid; idx < (16 - G) * CPR; idx += NT)   // padded q rows
         *reinterpret_cast<uint4*>(&q_s[G + idx / CPR][(idx % CPR) * 8]) = make_uint4(0, 0, 0, 0);
     __syncthreads();
-    if (QIE_DBG(a.dbg & 8)) {
-        if (tid == 0) a.out[m] = (uint16_t)(kf[0][0].x + vr[VCH - 1].y + kf[TPW - 1][KSTEPS - 1].z);
-        return false;
-    }
 
-    bf16x8_t qb[KSTEPS];
-    uint4 knew[KSTEPS];
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ks++) {
-        qb[ks] = *reinterpret_cast<const bf16x8_t*>(&q_s[fr][32 * ks + 8 * gq]);
-        knew[ks] = *reinterpret_cast<const uint4*>(&kv_new[0][32 * ks + 8 * gq]);
-    }
     const float scale = sqrtf((float)HD);
     // dot / scale as q = dot * (1 / scale) plus one FMA residual step (Markstein): the
     // correctly rounded quotient for every dot above 2^-100 in magnitude (k_decode_fp8.hip
     // d8_rms_pair), three VALU ops instead of the IEEE division sequence's ~10 with its
-    // serial latency — 8 quotients per lane per step on the step's critical path
+    // serial latency
     const float inv_scale = 1.0f / scale;
     auto qdiv = [&](float d) {
         const float q = d * inv_scale;
         if constexpr (HD == 64 || HD == 256) return q;   // sqrt(hd) a power of two: exact
         else return fmaf(fmaf(-q, scale, d), inv_scale, q);
     };
-    float m_run = -INFINITY, l_run = 0.f;
-    f32x4_t oacc[DTW];
+    const int nq = a.nq;
+    uint16_t* vw = &v_s[wave < kDecMWaves ? wave : 0][0];
+    if (keyed) {
+        bf16x8_t qb[KSTEPS];
 #pragma unroll
-    for (int d = 0; d < DTW; d++) oacc[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    uint16_t* vw = &v_s[wave][0];
-    const int q4 = fr >> 2, p4 = fr & 3;
-
-    for (int st = 0; st < nstep; st++) {
-        const int kb0 = t0 + st * KS;
-        // Only the step holding the new token takes its K / V rows from LDS, and only a step
-        // past the split's end masks scores (the last step of the last split; both uniform,
-        // scalar branches around in-place selects): the other steps carry no per-element
-        // compare / select.  (A whole second copy of the step body per case took the hd-128
-        // kernel from 216 to 298 registers.)
-        const bool hasp = p >= kb0 && p < kb0 + KS;
-        const bool full = kb0 + KS <= t1;
-        if (hasp) {
+        for (int ks = 0; ks < KSTEPS; ks++) qb[ks] = *reinterpret_cast<const bf16x8_t*>(&q_s[fr][32 * ks + 8 * gq]);
+        float m_run = -INFINITY, l_run = 0.f;
+        f32x4_t oacc[DT];
 #pragma unroll
-            for (int t = 0; t < TPW; t++) {
-                const bool nw = kb0 + 16 * TPW * wave + 16 * t + fr == p;
+        for (int d = 0; d < DT; d++) oacc[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        // element of row r, column c (a multiple of 4) of the V rows: 32-byte chunks of a row in turn, so that the 16 rows of a
+        // transposing read lie in different banks
+        auto v_at = [&](int r, int c) { return r * HD + (((c >> 4) ^ (HD == 128 ? r & 7 : (r >> 1) & 3)) << 4) + (c & 15); };
+        const int q4 = fr >> 2, p4 = fr & 3;
+        auto process = [&](auto x, int st) {
+            const int kb0 = t0 + st * KS, k0 = kb0 + 32 * wave;
+            // the new token's K / V rows from LDS (uniform: the wave that has it)
+            if (p >= k0 && p < k0 + 32) {
 #pragma unroll
-                for (int ks = 0; ks < KSTEPS; ks++) kf[t][ks] = sel4(nw, knew[ks], kf[t][ks]);
+                for (int ks = 0; ks < KSTEPS; ks++) {
+                    const uint4 kn = *reinterpret_cast<const uint4*>(&kv_new[0][32 * ks + 8 * gq]);
+#pragma unroll
+                    for (int t = 0; t < 2; t++) kf[x][t][ks] = sel4(k0 + 16 * t + fr == p, kn, kf[x][t][ks]);
+                }
+                const uint4 vn = *reinterpret_cast<const uint4*>(&kv_new[1][(lane % CPR) * 8]);   // (64 is a multiple of CPR)
+#pragma unroll
+                for (int i = 0; i < VCH; i++) vr[x][i] = sel4(k0 + (lane + 64 * i) / CPR == p, vn, vr[x][i]);
             }
+            // ---- S^T of this wave's 32 keys: lane = head fr, keys 16 t + 4 gq + r
+            f32x4_t sacc[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int ks = 0; ks < KSTEPS; ks++)
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+                    sacc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[x][t][ks]), qb[ks], sacc[t], 0, 0, 0);
 #pragma unroll
             for (int i = 0; i < VCH; i++) {
                 const int c = lane + 64 * i;
-                const int r = c / CPW, ch = c % CPW;
-                const uint4 vn = *reinterpret_cast<const uint4*>(&kv_new[1][wave * DW + ch * 8]);
-                vr[i] = sel4(kb0 + r == p, vn, vr[i]);
+                *reinterpret_cast<uint4*>(vw + v_at(c / CPR, (c % CPR) * 8)) = vr[x][i];
             }
-        }
-        // ---- S^T for this wave's 32 keys -> LDS (raw dots)
+            if (st + SETS < nstep) load_step(x, st + SETS);
+            // scores s = dot / sqrt(hd) (self_attension.cu); those past the split's end are no keys (uniform)
+            float e[8];
 #pragma unroll
-        for (int t = 0; t < TPW; t++) {
-            f32x4_t sacc = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int ks = 0; ks < KSTEPS; ks++)
-                sacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf[t][ks]), qb[ks], sacc, 0, 0, 0);
-            // C map: col = head fr, rows = keys 4 gq + r of the tile; scores s = dot / sqrt(hd)
-            // (self_attension.cu) divided once here, not by every wave that reads them
-            *reinterpret_cast<float4*>(&s_s[fr][16 * TPW * wave + 16 * t + 4 * gq]) =
-                make_float4(qdiv(sacc[0]), qdiv(sacc[1]), qdiv(sacc[2]), qdiv(sacc[3]));
-        }
-        // ---- this wave's V slice -> LDS (the new token's row from kv_new)
-#pragma unroll
-        for (int i = 0; i < VCH; i++) {
-            const int c = lane + 64 * i;
-            const int r = c / CPW, ch = c % CPW;
-            *reinterpret_cast<uint4*>(vw + r * DW + ch * 8) = vr[i];
-        }
-        if (st + 1 < nstep) load_step(st + 1);
-        __syncthreads();   // scores and V slices visible
-        // ---- online softmax over the step's 128 keys (every wave, identical); lane:
-        // head fr, keys 32 c + 8 gq + j (natural order, the P.V k slots)
-        float e[KS / 32][8];
-        float mt = -INFINITY;
-#pragma unroll
-        for (int c = 0; c < KS / 32; c++) {
-            const float4 lo = *reinterpret_cast<const float4*>(&s_s[fr][32 * c + 8 * gq]);
-            const float4 hi = *reinterpret_cast<const float4*>(&s_s[fr][32 * c + 8 * gq + 4]);
-            e[c][0] = lo.x; e[c][1] = lo.y; e[c][2] = lo.z; e[c][3] = lo.w;
-            e[c][4] = hi.x; e[c][5] = hi.y; e[c][6] = hi.z; e[c][7] = hi.w;
-        }
-        if (!full) {
-#pragma unroll
-            for (int c = 0; c < KS / 32; c++)
+            for (int j = 0; j < 8; j++) e[j] = qdiv(sacc[j / 4][j % 4]);
+            if (k0 + 32 > t1) {
 #pragma unroll
                 for (int j = 0; j < 8; j++)
-                    if (kb0 + 32 * c + 8 * gq + j >= t1) e[c][j] = -INFINITY;
-        }
-#pragma unroll
-        for (int c = 0; c < KS / 32; c++)
-#pragma unroll
-            for (int j = 0; j < 8; j++) mt = fmaxf(mt, e[c][j]);
-        mt = xor32_max(xor16_max(mt));
-        const float m_new = fmaxf(m_run, mt);
-        const float m_use = m_new == -INFINITY ? 0.f : m_new;
-        // __expf (v_exp_f32 on x * log2 e, ~2 ulp): every wave exponentiates all 128 scores,
-        // and the libm expf sequence was ~0.8 us of the step; the reference build itself
-        // compiles with -use_fast_math, i.e. the same approximation.
-        const float alpha = __expf(m_run - m_use);
-        float ls = 0.f;
-#pragma unroll
-        for (int c = 0; c < KS / 32; c++)
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                e[c][j] = __expf(e[c][j] - m_use);
-                ls += e[c][j];
+                    if (k0 + 16 * (j / 4) + 4 * gq + j % 4 >= t1) e[j] = -INFINITY;
             }
-        ls = xor32_sum(xor16_sum(ls));
-        l_run = l_run * alpha + ls;
-        m_run = m_new;
-        // bit-identical skip, as in the prefill kernel: step 0's O is zero, and alpha == 1
-        // exactly where no row's max grew (wave-uniform ballot)
-        if (st > 0 && __builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
-            float ar[4];
+            float mt = fmaxf(fmaxf(fmaxf(e[0], e[1]), fmaxf(e[2], e[3])), fmaxf(fmaxf(e[4], e[5]), fmaxf(e[6], e[7])));
+            mt = xor32_max(xor16_max(mt));
+            const float m_new = fmaxf(m_run, mt);
+            const float m_use = m_new == -INFINITY ? 0.f : m_new;
+            // __expf (v_exp_f32 on x * log2 e, ~2 ulp): the reference build itself
+            // compiles with -use_fast_math, i.e. the same approximation
+            const float alpha = __expf(m_run - m_use);
 #pragma unroll
-            for (int r = 0; r < 4; r++) ar[r] = __shfl(alpha, gq * 4 + r, 64);
+            for (int j = 0; j < 8; j++) e[j] = __expf(e[j] - m_use);
+            const float ls = xor32_sum(xor16_sum(((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]))));
+            l_run = l_run * alpha + ls;
+            m_run = m_new;
+            // bit-identical skip, as in the prefill kernel: step 0's O is zero, and alpha == 1
+            // exactly where no row's max grew (wave-uniform ballot)
+            if (st > 0 && __builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+                float ar[4];
 #pragma unroll
-            for (int d = 0; d < DTW; d++)
+                for (int r = 0; r < 4; r++) ar[r] = __shfl(alpha, gq * 4 + r, 64);
 #pragma unroll
-                for (int r = 0; r < 4; r++) oacc[d][r] *= ar[r];
-        }
-        // ---- O[:, slice] += P . V[:, slice], P = hi + mid + lo: three bf16 parts hold all
-        // 24 bits of the fp32 probability, so every P.V product is the reference's fp32
-        // product (self_attension.cu:127-135) — only the accumulation order differs
+                for (int d = 0; d < DT; d++)
 #pragma unroll
-        for (int c = 0; c < KS / 32; c++) {
+                    for (int r = 0; r < 4; r++) oacc[d][r] *= ar[r];
+            }
             uint4 pp[3];
-            split_bf16x8<3>(e[c], pp);
+            split_bf16x8<3>(e, pp);
             const bf16x8_t ph = __builtin_bit_cast(bf16x8_t, pp[0]), pm = __builtin_bit_cast(bf16x8_t, pp[1]),
                            pl = __builtin_bit_cast(bf16x8_t, pp[2]);
+            constexpr int DG = 4;   // tiles of d at a time
 #pragma unroll
-            for (int d = 0; d < DTW; d++) {
-                const uint16_t* a0 = vw + (32 * c + 8 * gq + q4) * DW + 16 * d + 4 * p4;
-                const i16x4_t v0 =
-                    __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) i16x4_t*)(a0));
+            for (int d0 = 0; d0 < DT; d0 += DG) {
+            bf16x8_t vt[DG];
+#pragma unroll
+            for (int dd = 0; dd < DG; dd++) {
+                const int d = d0 + dd;
+                const i16x4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (__attribute__((address_space(3))) i16x4_t*)(vw + v_at(4 * gq + q4, 16 * d + 4 * p4)));
                 const i16x4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                    (__attribute__((address_space(3))) i16x4_t*)(a0 + 4 * DW));
-                const bf16x8_t vb8 = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
-                oacc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ph, vb8, oacc[d], 0, 0, 0);
-                oacc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pm, vb8, oacc[d], 0, 0, 0);
-                if (!QIE_DBG(!a.pv3)) oacc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl, vb8, oacc[d], 0, 0, 0);
+                    (__attribute__((address_space(3))) i16x4_t*)(vw + v_at(16 + 4 * gq + q4, 16 * d + 4 * p4)));
+                vt[dd] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
             }
-        }
-        __syncthreads();   // scores / V slots free for the next step
-    }
-    if (QIE_DBG(a.dbg & 16)) {
-        if (tid == 0) a.out[m] = (uint16_t)(oacc[0][0] + m_run);
-        return false;
-    }
-
-    // ---------------- this wave's d-slice of the split result (rows = heads 4 gq + r)
-    const int nq = a.nq;
-    float lr[4];
 #pragma unroll
-    for (int r = 0; r < 4; r++) lr[r] = __shfl(l_run, gq * 4 + r, 64);
-    if (nsplit == 1) {
+            for (int dd = 0; dd < DG; dd++) oacc[d0 + dd] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ph, vt[dd], oacc[d0 + dd], 0, 0, 0);
+#pragma unroll
+            for (int dd = 0; dd < DG; dd++) oacc[d0 + dd] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pm, vt[dd], oacc[d0 + dd], 0, 0, 0);
+#pragma unroll
+            for (int dd = 0; dd < DG; dd++) oacc[d0 + dd] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl, vt[dd], oacc[d0 + dd], 0, 0, 0);
+            }
+        };
+        for (int st = 0; st < nstep; st += 2) {
+            process(even, st);
+            if (st + 1 < nstep) process(odd, st + 1);
+        }
+        // ---------------- the waves' results to LDS (O where this wave's V rows were: its own reads of them are done)
+        if (gq == 0) ml_s[wave][fr] = make_float2(m_run, l_run);
+        float* ow = reinterpret_cast<float*>(vw);   // [8 heads][HD]
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const int h = 4 * gq + r;
-            if (h >= G) continue;
+            if (h < G) {
 #pragma unroll
-            for (int d = 0; d < DTW; d++) {
-                const int64_t oi = m * (int64_t)nq * HD + (int64_t)(g * G + h) * HD + wave * DW + 16 * d + fr;
-                if constexpr (X::on) hook->out1(oi, f2bf(oacc[d][r] / lr[r]));
-                else a.out[oi] = f2bf(oacc[d][r] / lr[r]);
+                for (int d = 0; d < DT; d++) ow[h * HD + 16 * d + fr] = oacc[d][r];
             }
         }
-        return false;
-    }
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int h = 4 * gq + r;
-        if (h >= G) continue;
-        const int64_t pi = (m * nq + g * G + h) * (int64_t)a.nsplit_max + s;
-        // write-through (sc1) stores: published by the drain + ticket below, no release
-        // fence (cdna_hip_programming.md, in-launch split-K reduction)
-#pragma unroll
-        for (int d = 0; d < DTW; d++)
-            __hip_atomic_store(&a.part_o[pi * HD + wave * DW + 16 * d + fr], oacc[d][r], __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if (wave == 0 && gq == 0 && fr < G) {
-        const int64_t pi = (m * nq + g * G + fr) * (int64_t)a.nsplit_max + s;
-        __hip_atomic_store(&a.part_ml[pi * 2], m_run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(&a.part_ml[pi * 2 + 1], l_run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    // ---------------- publish this split; the last arriver combines (acquire)
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every storing wave drains
-    __syncthreads();
-    if (QIE_DBG(a.dbg & 1)) return false;
-    unsigned* cnt = a.counters + m * a.nkv + g;
-    if (tid == 0) {
-        const unsigned old = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        last_flag = (old == (unsigned)nsplit - 1) ? 1 : 0;
     }
     __syncthreads();
-    if (!last_flag || QIE_DBG(a.dbg & 128)) return false;   // (dev timing exit 128: ticket taken, no combine)
-    // Default: 16-B sc1 buffer loads on a uniform (SGPR) resource instead of the acquire:
-    // 9.79 -> 9.56 us per launch.  (Measured as well:
-    // 8-B agent-scope atomic loads at 11.4 vs 10.7 us, and 16-B sc1 loads at 73 us — that
-    // form put the resource in VGPRs, a waterfall loop per load.)
-    if (!a.sc1) {
-        if (tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-    }
-    // Per-thread online combine: thread (head gi, d4) loads the (m, l) of EVERY split of its
-    // head together with its 16-byte slice of every split's partial O (one batch of JB
-    // splits = one round trip; ctx <= JB * 128 keys in one), then merges them itself — no
-    // per-head wave pass, LDS weight table or barrier between the two load rounds.
-    constexpr int JB = KS == 64 ? 40 : (KS == 128 ? 24 : 16);   // splits per combine round trip
-    const bool has_item = tid < G * (HD / 4);
+    // ---------------- thread (head gi, 4 dims from 4 d4): the split's maximum, sum and O.  From here on every wave goes by itself: its
+    // heads have a ticket of their own, so that the last arrivers of a kv head's waves are spread over its splits' CUs
+    const int items = G * (HD / 4);
+    if (64 * wave >= items) return;   // uniform
+    const bool has_item = tid < items;
     const int gi = has_item ? tid / (HD / 4) : 0, d4 = tid % (HD / 4);
-    const int64_t hbase = (m * nq + g * G + gi) * (int64_t)a.nsplit_max;
-    const float4* src4 = reinterpret_cast<const float4*>(a.part_o) + hbase * (HD / 4) + d4;
-    const float2* ml2 = reinterpret_cast<const float2*>(a.part_ml) + hbase;
+    float2 wml[kDecMWaves];
+#pragma unroll
+    for (int w = 0; w < kDecMWaves; w++) wml[w] = ml_s[w][gi];
+    const float m_spl = fmaxf(fmaxf(wml[0].x, wml[1].x), fmaxf(wml[2].x, wml[3].x));   // finite: a split has a key
+    float l_spl = 0.f;
+    float4 o_spl = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int w = 0; w < kDecMWaves; w++) {
+        const float c = __expf(wml[w].x - m_spl);   // 0 for a wave without keys
+        const float4 o = reinterpret_cast<const float4*>(&v_s[w][0])[gi * (HD / 4) + d4];
+        l_spl = fmaf(wml[w].y, c, l_spl);
+        o_spl.x = fmaf(c, o.x, o_spl.x);
+        o_spl.y = fmaf(c, o.y, o_spl.y);
+        o_spl.z = fmaf(c, o.z, o_spl.z);
+        o_spl.w = fmaf(c, o.w, o_spl.w);
+    }
+    // divided (not multiplied by 1/l): the softmax normalisation's one rounding
+    auto result = [&](const float4& o, float l) {
+        return (unsigned long long)pack2(o.x / l, o.y / l) | ((unsigned long long)pack2(o.z / l, o.w / l) << 32);
+    };
+    const int64_t out_at = m * (int64_t)nq * HD + (int64_t)(g * G + gi) * HD + d4 * 4;
+    if (nsplit == 1) {
+        if (has_item) {
+            const unsigned long long pk = result(o_spl, l_spl);
+            if constexpr (X::on) hook->out4(out_at, pk);
+            else *reinterpret_cast<unsigned long long*>(a.out + out_at) = pk;
+        }
+        return;
+    }
+    // write-through (sc1) stores: published by the drain + ticket below, no release fence
+    const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc((void*)a.part_o, 0, 0x7fffffff, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc((void*)a.part_ml, 0, 0x7fffffff, 0x00020000);
+    const int hbase = (int)((m * nq + g * G + gi) * (int64_t)a.nsplit_max);
+    if (has_item) {
+        __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{__float_as_uint(o_spl.x), __float_as_uint(o_spl.y), __float_as_uint(o_spl.z), __float_as_uint(o_spl.w)},
+                                               ro, ((hbase + s) * (HD / 4) + d4) * 16, 0, 16);
+        if (d4 == 0) __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{__float_as_uint(m_spl), __float_as_uint(l_spl)}, rm, (hbase + s) * 8, 0, 16);
+    }
+    // ---------------- publish this split; the last arriver combines
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // stored
+    if (QIE_DBG(a.dbg & 1)) return;
+    unsigned* cnt = a.counters + ((m * a.nkv + g) * kDecMWaves + wave) * kDecMTicket;
+    unsigned old = 0;
+    if (lane == 0) old = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    old = __builtin_amdgcn_readfirstlane(old);
+    if (old != (unsigned)nsplit - 1) return;   // uniform
+    asm volatile("" ::: "memory");
+    // The splits of the head by 16-B sc1 buffer loads (L2 / memory side, never a stale L1 line) on a uniform resource: every partial
+    // was stored sc1 by a wave that drained (vmcnt 0) before its ticket add, and this wave's add came last.  (With an acquire fence instead 9.79 against 9.56 us per launch; 8-B agent-scope atomic loads 11.4 against 10.7.)
+    // A thread loads the (m, l) of EVERY split of its head together with its 16 bytes of their O, groups of four that exist in flight
+    // together (up to JB splits: one round trip), then merges them itself.
+    constexpr int JB = 24;
     float mx = -INFINITY, ls = 0.f;
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int j0 = 0; j0 < nsplit; j0 += JB) {
         float4 v[JB];
         float2 w[JB];
-        if (a.sc1) {
-            // sc1 loads (L2 / memory side, never a stale L1 line) in place of the acquire:
-            // every partial was stored sc1 by a wave that drained (vmcnt 0) before its
-            // workgroup's barrier and ticket add, and this workgroup's add came last
-            // (MI355X_MICROARCH.md hand-off table, row 1).  Buffer loads on a uniform
-            // resource: the resource stays in SGPRs.
-            const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc((void*)a.part_o, 0, 0x7fffffff, 0x00020000);
-            const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc((void*)a.part_ml, 0, 0x7fffffff, 0x00020000);
 #pragma unroll
-            for (int jj = 0; jj < JB; jj++) {
-                const int j = min(j0 + jj, nsplit - 1);
-                const u32x4_t q4 = __builtin_amdgcn_raw_buffer_load_b128(
-                    ro, (int)(((hbase + j) * (HD / 4) + d4) * 16), 0, 16);
-                const u32x2_t q2 = __builtin_amdgcn_raw_buffer_load_b64(rm, (int)((hbase + j) * 8), 0, 16);
-                v[jj] = make_float4(__uint_as_float(q4.x), __uint_as_float(q4.y), __uint_as_float(q4.z),
-                                    __uint_as_float(q4.w));
+        for (int b = 0; b < JB; b += 4) {
+            if (j0 + b >= nsplit) break;   // uniform
+#pragma unroll
+            for (int jj = b; jj < b + 4; jj++) {
+                const u32x2_t q2 = __builtin_amdgcn_raw_buffer_load_b64(rm, (hbase + min(j0 + jj, nsplit - 1)) * 8, 0, 16);
                 w[jj] = make_float2(__uint_as_float(q2.x), __uint_as_float(q2.y));
             }
-        } else {
+        }
 #pragma unroll
-            for (int jj = 0; jj < JB; jj++) {
-                const int j = min(j0 + jj, nsplit - 1);
-                v[jj] = src4[(int64_t)j * (HD / 4)];
-                w[jj] = ml2[j];
+        for (int b = 0; b < JB; b += 4) {
+            if (j0 + b >= nsplit) break;
+#pragma unroll
+            for (int jj = b; jj < b + 4; jj++) {
+                const u32x4_t q4 = __builtin_amdgcn_raw_buffer_load_b128(ro, ((hbase + min(j0 + jj, nsplit - 1)) * (HD / 4) + d4) * 16, 0, 16);
+                v[jj] = make_float4(__uint_as_float(q4.x), __uint_as_float(q4.y), __uint_as_float(q4.z), __uint_as_float(q4.w));
             }
         }
         float mb = mx;
 #pragma unroll
-        for (int jj = 0; jj < JB; jj++) mb = fmaxf(mb, j0 + jj < nsplit ? w[jj].x : -INFINITY);
+        for (int b = 0; b < JB; b += 4) {
+            if (j0 + b >= nsplit) break;
+#pragma unroll
+            for (int jj = b; jj < b + 4; jj++) mb = fmaxf(mb, j0 + jj < nsplit ? w[jj].x : -INFINITY);
+        }
         const float sc = __expf(mx - mb);   // 0 on the first batch (mx = -inf, mb finite)
         ls *= sc;
         acc.x *= sc; acc.y *= sc; acc.z *= sc; acc.w *= sc;
 #pragma unroll
-        for (int jj = 0; jj < JB; jj++) {
-            const float c = j0 + jj < nsplit ? __expf(w[jj].x - mb) : 0.f;
-            ls = fmaf(w[jj].y, c, ls);
-            acc.x = fmaf(c, v[jj].x, acc.x);
-            acc.y = fmaf(c, v[jj].y, acc.y);
-            acc.z = fmaf(c, v[jj].z, acc.z);
-            acc.w = fmaf(c, v[jj].w, acc.w);
+        for (int b = 0; b < JB; b += 4) {
+            if (j0 + b >= nsplit) break;
+#pragma unroll
+            for (int jj = b; jj < b + 4; jj++) {
+                const float c = j0 + jj < nsplit ? __expf(w[jj].x - mb) : 0.f;
+                ls = fmaf(w[jj].y, c, ls);
+                acc.x = fmaf(c, v[jj].x, acc.x);
+                acc.y = fmaf(c, v[jj].y, acc.y);
+                acc.z = fmaf(c, v[jj].z, acc.z);
+                acc.w = fmaf(c, v[jj].w, acc.w);
+            }
         }
         mx = mb;
     }
+    if (lane == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // (persistent kernel: who sees the output may take the next layer's ticket)
+    if constexpr (X::on) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (has_item) {
-        uint16_t* dst = a.out + m * (int64_t)nq * HD + (int64_t)(g * G + gi) * HD + d4 * 4;
-        // divided (not multiplied by 1/l): the softmax normalisation's one rounding
-        const unsigned long long pk = (unsigned long long)pack2(acc.x / ls, acc.y / ls) |
-                                      ((unsigned long long)pack2(acc.z / ls, acc.w / ls) << 32);
-        if constexpr (X::on) hook->out4(m * (int64_t)nq * HD + (int64_t)(g * G + gi) * HD + d4 * 4, pk);
-        else __hip_atomic_store(reinterpret_cast<unsigned long long*>(dst), pk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned long long pk = result(acc, ls);
+        if constexpr (X::on) hook->out4(out_at, pk);
+        else *reinterpret_cast<unsigned long long*>(a.out + out_at) = pk;
     }
-    if (tid == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return true;
 }
 
 }  // namespace qie

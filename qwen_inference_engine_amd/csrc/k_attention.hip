@@ -500,9 +500,9 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void attn_prefill_mfma2_kernel(Pre
 }
 
 
-template <int HD, bool PG, int NWA, bool PR, int KS = kDecMStep>
-__global__ __launch_bounds__(64 * NWA) void attn_decode_mfma2_kernel(DecodeAttnParams a) {
-    attn_decode_mfma2_body<HD, PG, NWA, PR, KS>(a, blockIdx.x, blockIdx.y);
+template <int HD, bool PG, bool PR>
+__global__ __launch_bounds__(64 * kDecMWaves) void attn_decode_mfma2_kernel(DecodeAttnParams a) {
+    attn_decode_mfma2_body<HD, PG, kDecMWaves, PR>(a, blockIdx.y, blockIdx.x, blockIdx.z);
 }
 
 
@@ -529,6 +529,8 @@ static int attn_nsplit(int64_t M, int32_t max_ctx) {
 static thread_local const float* g_rope_cur = nullptr;
 void set_decode_rope_cur(const float* rc) { g_rope_cur = rc; }
 
+static int64_t dec_counter_bytes(int64_t B, int32_t nkv) { return B * nkv * (kDecMWaves * kDecMTicket * 4); }
+
 static int fill_dec_params(DecodeAttnParams& a, const void* qkv, int64_t B, const int32_t* pos, const void* q_norm,
                            const void* k_norm, const float* rope_cos, const float* rope_sin, int32_t n_heads,
                            const qie_kv_cache* cache, int32_t layer, float eps, int32_t numerics, void* out, void* ws) {
@@ -544,48 +546,35 @@ static int fill_dec_params(DecodeAttnParams& a, const void* qkv, int64_t B, cons
     a.layer = layer;
     a.nkv = cache->n_kv_heads;
     a.nq = n_heads;
+    a.G = a.nq / a.nkv;
     a.max_ctx = cache->max_ctx;
     const int senv = std::min(dev_env("QIE_DEC_SPLITS", 0), kDecMaxSplits);
-    // split target: 32 (one-step splits up to 4k keys); at B >= 8, 8 — config 4 (B = 8, ctx
-    // 1,025-1,280) then runs two-step splits, half as many split blocks and combine inputs
-    // per row: 3,610 -> 3,637-3,645 tok/s same-box (at B = 1 the headline wants the CUs:
-    // targets 16 / 8 ran 349 / 340 vs 361 tok/s)
-    a.splits_target = senv > 0 ? senv : (B >= 8 ? 8 : kDecMSplits);
+    // split target: 32 (one-step splits up to 4k keys), from 8 rows on fewer where that would be more than two workgroups a CU: 8 at least
+    // (Qwen2-7B fp8, 8 rows at 1,025 keys: 9 one-step splits 2.33 ms a token, 5 of two steps 2.35)
+    const int two_a_cu = (int)(2 * device_cu_count() / (a.nkv * B));
+    a.splits_target = senv > 0 ? senv : B < 8 ? kDecMSplits : std::max(8, std::min(kDecMSplits, two_a_cu));
     a.dbg = dev_env("QIE_DEC_DBG", 0);
-    a.sc1 = dev_env("QIE_DEC_SC1", 1);   // 9.79 -> 9.56 us per launch (ctx 2.3k, Qwen2-7B)
-    // keys per block step (the launch picks the kernel instantiation with the same KS): 128.
-    // QIE_DEC_KS (dev A/B): 64 (hd 128, not pre-rotated), 256 (hd 64: ONE step where
-    // Qwen2-0.5B's config-2 contexts, 129-256 keys, walk two dependent 128-key steps in one
-    // block per kv head — measured equal, attention 7.94 vs 7.96 µs live, 1,446 vs 1,454 tok/s:
-    // the second step's chain is not what the launch waits on).
-    const int hd = cache->head_dim;
-    const int ks_env = dev_env("QIE_DEC_KS", 0);
-    // (a step never straddles a page: 256-key steps need pages of >= 256 tokens)
-    const bool ks256_ok = hd == 64 && (cache->block_table == nullptr || cache->page_tokens >= 256);
-    int ks = kDecMStep;
-    if (ks_env == 128 || (ks_env == 256 && ks256_ok) || (ks_env == 64 && hd == 128 && !(numerics & QIE_ATTN_PREROPED)))
-        ks = ks_env;
-    a.ks = ks;
-    a.nsplit_max = std::min(a.splits_target, (cache->max_ctx + ks - 1) / ks);
+    a.nsplit_max = std::min(a.splits_target, (cache->max_ctx + kDecMStep - 1) / kDecMStep);
     QIE_REQUIRE(a.nsplit_max <= kDecMaxSplits, "qie_attention_decode: max_ctx %d too long", cache->max_ctx);
     a.eps = eps;
     a.numerics = numerics & QIE_NUMERICS_MASK;
     a.pre_roped = (numerics & QIE_ATTN_PREROPED) != 0;
     QIE_REQUIRE(!a.pre_roped || (q_norm == nullptr && k_norm == nullptr && a.numerics == QIE_NUMERICS_REF),
                 "qie_attention_decode: QIE_ATTN_PREROPED needs REF numerics without qk-norm");
-    const int64_t cnt = ((B * a.nkv * 4 + 255) / 256) * 256;
+    const int64_t cnt = dec_counter_bytes(B, a.nkv);
     a.counters = (unsigned*)ws;
     a.part_o = (float*)((char*)ws + cnt);
     a.part_ml = a.part_o + B * n_heads * (int64_t)a.nsplit_max * cache->head_dim;
     a.out = (uint16_t*)out;
     a.rc = dev_env("QIE_DEC_ROPECUR", 1) ? g_rope_cur : nullptr;
-    a.pv3 = dev_env("QIE_DEC_PV3", 1);
     // The speculative step is issued before the position is known, so the grid's idle
     // splits (s >= this step's split count: the graph's grid is sized for max_ctx) load a
     // step too and drop it (config 4, max_ctx 1,344: 32-64 idle blocks of 352, 2-4 MB per
     // launch).  Measured, it still pays at B = 8 (3,478.6 vs 3,465.7 tok/s without it) as at
     // B = 1 (358.7 vs 357.2).  QIE_DEC_SPEC (dev A/B): 0 turns it off.
-    a.spec_ok = dev_env("QIE_DEC_SPEC", 1) != 0;
+    // Off where the cache is so long that contexts may have splits of several steps: then the step loaded is mostly not the split's
+    // first, and its 64 KB go through the CU ahead of the right ones (Qwen3-14B, 6,001 keys: 2 us of a launch).
+    a.spec_ok = dev_env("QIE_DEC_SPEC", 1) != 0 && a.max_ctx <= kDecMStep * a.splits_target;
     return 0;
 }
 
@@ -697,7 +686,7 @@ int64_t qie_attention_decode_workspace_bytes(int64_t B, int32_t n_heads, int32_t
                                              int32_t max_ctx) {
     // an upper bound for every splits_target <= kDecMaxSplits (nsplit_max in fill_dec_params)
     const int64_t ns = std::min<int64_t>(kDecMaxSplits, (max_ctx + 63) / 64);   // 64- or 128-key steps
-    const int64_t cnt = ((B * n_kv_heads * 4 + 255) / 256) * 256;
+    const int64_t cnt = dec_counter_bytes(B, n_kv_heads);
     return cnt + B * n_heads * ns * (head_dim + 2) * 4;
 }
 
@@ -714,26 +703,13 @@ int qie_attention_decode(const void* qkv, int64_t B, const int32_t* pos, const v
     DecodeAttnParams a;
     QIE_TRY(fill_dec_params(a, qkv, B, pos, q_norm, k_norm, rope_cos, rope_sin, n_heads, cache, layer, eps, numerics,
                             out, ws));
-    dim3 grid((unsigned)(a.nkv * a.nsplit_max), (unsigned)B);
-    const bool pg = a.km.table != nullptr;
-    // hd 128: 8 waves per workgroup (one 16-key S tile and a 16-dim P.V slice per wave);
-    // hd 64 keeps 4 (a 16-dim slice per wave is the MFMA tile's minimum)
-    // 4 waves per workgroup (8 at hd 128, one 16-key tile and a 16-dim P.V slice per wave,
-    // measured slower: 12.9 vs 9.8 us per launch at ctx 2.3k)
-    const bool pr = a.pre_roped != 0;
-    auto k2 = cache->head_dim == 128
-                  ? (pr ? (pg ? attn_decode_mfma2_kernel<128, true, 4, true> : attn_decode_mfma2_kernel<128, false, 4, true>)
-                        : (pg ? attn_decode_mfma2_kernel<128, true, 4, false> : attn_decode_mfma2_kernel<128, false, 4, false>))
-                  : (pr ? (pg ? attn_decode_mfma2_kernel<64, true, 4, true> : attn_decode_mfma2_kernel<64, false, 4, true>)
-                        : (pg ? attn_decode_mfma2_kernel<64, true, 4, false> : attn_decode_mfma2_kernel<64, false, 4, false>));
-    if (a.ks == 64 && cache->head_dim == 128 && !pr)   // 64-key steps (dev A/B)
-        k2 = pg ? attn_decode_mfma2_kernel<128, true, 4, false, 64> : attn_decode_mfma2_kernel<128, false, 4, false, 64>;
-    if (a.ks == 256 && cache->head_dim == 64)   // one 256-key step (short contexts at hd 64)
-        k2 = pr ? (pg ? attn_decode_mfma2_kernel<64, true, 4, true, 256> : attn_decode_mfma2_kernel<64, false, 4, true, 256>)
-                : (pg ? attn_decode_mfma2_kernel<64, true, 4, false, 256> : attn_decode_mfma2_kernel<64, false, 4, false, 256>);
-    QIE_REQUIRE(a.ks == 128 || (a.ks == 64 && cache->head_dim == 128 && !pr) || (a.ks == 256 && cache->head_dim == 64),
-                "qie_attention_decode: internal: no kernel for %d-key steps at hd %d", a.ks, cache->head_dim);
-    hipLaunchKernelGGL(k2, grid, dim3(256), 0, (hipStream_t)stream, a);
+    dim3 grid((unsigned)a.nsplit_max, (unsigned)a.nkv, (unsigned)B);
+    const bool pg = a.km.table != nullptr, pr = a.pre_roped != 0;
+    auto k2 = cache->head_dim == 128 ? (pr ? (pg ? attn_decode_mfma2_kernel<128, true, true> : attn_decode_mfma2_kernel<128, false, true>)
+                                           : (pg ? attn_decode_mfma2_kernel<128, true, false> : attn_decode_mfma2_kernel<128, false, false>))
+                                     : (pr ? (pg ? attn_decode_mfma2_kernel<64, true, true> : attn_decode_mfma2_kernel<64, false, true>)
+                                           : (pg ? attn_decode_mfma2_kernel<64, true, false> : attn_decode_mfma2_kernel<64, false, false>));
+    hipLaunchKernelGGL(k2, grid, dim3(64 * kDecMWaves), 0, (hipStream_t)stream, a);
     QIE_LAUNCH_CHECK();
     return 0;
 }

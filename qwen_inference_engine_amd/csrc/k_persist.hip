@@ -332,14 +332,13 @@ __device__ __forceinline__ void bar() {
 }
 
 // attention role hook (attn_decode.hpp): q / k / v row of kv head g from the QKV granules,
-// outputs into an LDS staging row
+// outputs published as granules
 template <int NT>
 struct AttnHook {
     static constexpr bool on = true;
     const unsigned long long* g_qkv;
     uint16_t* row;          // LDS image of the whole q|k|v row (the body reads a.qkv = row)
-    uint16_t* stage;        // LDS [G * hd]: this kv head's output
-    int64_t o0;             // output index of stage[0]
+    unsigned long long* g_att;   // the outputs' granules
     int g, G, hd, QD, KD;
     unsigned tag;
     const Params* p;
@@ -358,9 +357,9 @@ struct AttnHook {
         }
         __syncthreads();
     }
-    __device__ void out1(int64_t i, uint16_t v) { stage[i - o0] = v; }
-    __device__ void out4(int64_t i, unsigned long long v) {
-        *reinterpret_cast<unsigned long long*>(stage + (i - o0)) = v;
+    __device__ void out4(int64_t i, unsigned long long v) {   // outputs i .. i + 3: two granules
+        st_granule(g_att + i / 2, tag, (uint32_t)v);
+        st_granule(g_att + i / 2 + 1, tag, (uint32_t)(v >> 32));
     }
 };
 
@@ -385,7 +384,6 @@ __global__ __launch_bounds__(NW * 64, 1) void decode_layers_kernel(Params p) {
     uint16_t* nw = reinterpret_cast<uint16_t*>(q); q += al(H * 2);          // norm weights
     uint16_t* hb = reinterpret_cast<uint16_t*>(q); q += al((I > QKVD ? I : QKVD) * 2);   // h / q|k|v row image
     uint16_t* stage = reinterpret_cast<uint16_t*>(q); q += al(kStage * 2);
-    uint16_t* astage = reinterpret_cast<uint16_t*>(q); q += al(G * HD * 2);
     float* bias = reinterpret_cast<float*>(q); q += al(kMaxBias * 4);
     float* red = reinterpret_cast<float*>(q); q += 64;
     int* dead = reinterpret_cast<int*>(q);
@@ -396,8 +394,7 @@ __global__ __launch_bounds__(NW * 64, 1) void decode_layers_kernel(Params p) {
 
     // ---- attention jobs of this step: CUs [0, nA) = (kv head, split)
     const int pos = sld(p.pos);
-    const int chunk = decm_chunk(pos + 1, p.splits_target, kDecMStep);
-    const int nsplit = (pos + 1 + chunk - 1) / chunk;
+    const int nsplit = decm_splits(pos + 1, decm_chunk(pos + 1, p.splits_target));
     const int nA = p.nkv * nsplit;
     const bool att_cu = cu < nA;
     const int nO = ncu - nA;   // CUs owning O rows
@@ -534,8 +531,7 @@ __global__ __launch_bounds__(NW * 64, 1) void decode_layers_kernel(Params p) {
             AttnHook<kThreads> hk;
             hk.g_qkv = p.g_qkv;
             hk.row = hb;
-            hk.stage = astage;
-            hk.o0 = (int64_t)g * G * HD;
+            hk.g_att = p.g_att;
             hk.g = g;
             hk.G = G;
             hk.hd = HD;
@@ -544,16 +540,9 @@ __global__ __launch_bounds__(NW * 64, 1) void decode_layers_kernel(Params p) {
             hk.tag = tg;
             hk.p = &p;
             hk.dead = dead;
-            const bool comb = attn_decode_mfma2_body<HD, false, kWaves, false, kDecMStep, AttnHook<kThreads>>(
-                a, g * a.nsplit_max + s, 0, &hk);
-            // the combiner's ticket reset (and every partial store) is performed before anything
-            // this CU publishes later — the next layer's splits take tickets only after that
+            attn_decode_mfma2_body<HD, false, kWaves, false, AttnHook<kThreads>>(a, g, s, 0, &hk);
+            // every partial store is performed before anything this CU publishes later
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            if (comb || nsplit == 1) {
-                __syncthreads();
-                for (int i = tid; i < G * HD / 2; i += kThreads)
-                    st_granule(p.g_att + g * (G * HD / 2) + i, tg, reinterpret_cast<const uint32_t*>(astage)[i]);
-            }
             __syncthreads();
             ts(l, 3);
             if (*dead) return;
@@ -663,11 +652,11 @@ int decode_attn_params(DecodeAttnParams* a, const void* qkv, int64_t B, const in
                        const qie_kv_cache* cache, int32_t layer, float eps, int32_t numerics, void* out, void* ws);
 
 // ------------------------------------------------------------------ host side
-size_t persist_lds_bytes(int H, int I, int QD, int KD, int G, int hd) {
+size_t persist_lds_bytes(int H, int I, int QD, int KD) {
     auto al = [](size_t b) { return (b + 15) & ~(size_t)15; };
     const int QKVD = QD + 2 * KD;
     return al(H * 2) * 3 + al((size_t)(H > QD ? H : QD) * 2) + al((size_t)(I > QKVD ? I : QKVD) * 2) +
-           al(pk::kStage * 2) + al((size_t)G * hd * 2) + al(pk::kMaxBias * 4) + 64 + 16;
+           al(pk::kStage * 2) + al(pk::kMaxBias * 4) + 64 + 16;
 }
 
 // Which models / batches the persistent step covers (the launch path serves the rest):
@@ -699,7 +688,7 @@ bool persist_supported(const qie_model_spec& s, int B, int tp, bool fp8, bool pa
     const int per_cu = std::max({QKVD / 2 / ncu + 2, s.hidden / 2 / (ncu - s.n_kv_heads * nsplit_max) + 2,
                                  s.ffn / 2 / ncu + 2});
     if (2 * per_cu > pk::kStage || 2 * (QKVD / 2 / ncu + 2) > pk::kMaxBias) return no("per-CU ranges too large");
-    if (persist_lds_bytes(s.hidden, s.ffn, QD, KD, G, s.head_dim) + 48 * 1024 > 160 * 1024) return no("LDS");
+    if (persist_lds_bytes(s.hidden, s.ffn, QD, KD) + 48 * 1024 > 160 * 1024) return no("LDS");
     return true;
 }
 
@@ -715,7 +704,7 @@ int persist_attn_table(const qie_model_spec& s, const qie_layer_weights* h_layer
     for (int l = 0; l < s.n_layers; l++) {
         QIE_TRY(decode_attn_params(&t[l], qkv_scratch, 1, pos, h_layers[l].q_norm, h_layers[l].k_norm, rope_cos,
                                    rope_sin, s.n_heads, cache, l, s.rms_eps, s.numerics, (void*)qkv_scratch, dec_ws));
-        QIE_REQUIRE(t[l].ks == kDecMStep && !t[l].pre_roped && t[l].nsplit_max <= kDecMSplits,
+        QIE_REQUIRE(!t[l].pre_roped && t[l].nsplit_max <= kDecMSplits,
                     "persistent decode: unsupported attention step");
     }
     QIE_HIP(hipMemcpyAsync(d_attp, t.data(), sizeof(DecodeAttnParams) * t.size(), hipMemcpyHostToDevice, st));
@@ -753,7 +742,7 @@ int persist_decode_launch(const qie_model_spec& s, const qie_layer_weights* d_la
     p.ts = ts;
     p.pf_mask = (unsigned)dev_env("QIE_PK_PF_MASK", 0xFF);
     p.xw_even = dev_env("QIE_PK_XW", 100);
-    const size_t shm = persist_lds_bytes(p.H, p.I, p.QD, p.KD, p.nq / p.nkv, p.hd);
+    const size_t shm = persist_lds_bytes(p.H, p.I, p.QD, p.KD);
     const void* fn = s.head_dim == 128 ? (const void*)pk::decode_layers_kernel<128> : (const void*)pk::decode_layers_kernel<64>;
     static bool raised[2] = {false, false};
     bool& r = raised[s.head_dim == 128 ? 1 : 0];
