@@ -1016,7 +1016,7 @@ int g8_workspace(hipStream_t st, int slabs, int tiles, G8Split* out) {
 // (64 MB; growing step by step inside it took 0.3 to 1.1 ms).
 void g8_reserve(hipStream_t st) {
     G8Split ws;
-    (void)g8_workspace(st, device_cu_count(), 4096, &ws);   // no memory: a later launch asks again, or runs unsplit
+    (void)g8_workspace(st, device_cu_count(), 65536, &ws);   // no memory: a later launch asks again, or runs unsplit
 }
 
 void g8_release(hipStream_t st) {
