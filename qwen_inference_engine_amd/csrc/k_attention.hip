@@ -231,7 +231,7 @@ struct PrefillAttnParams {
 // Prefill kernel: each wave owns two 16-row query groups, so every K fragment
 // (S^T = K.Q^T) and every V fragment (O += P.V) read from LDS feeds up to two MFMAs.
 // Causal balance: the sequence's 16-row groups are paired (j, n-1-j) and wave j of the
-// grid gets pair j, so every wave (and every workgroup of 4 waves) has the same number of
+// grid gets pair j, so every wave (and every workgroup) has the same number of
 // (group, key tile) products; a workgroup stages K/V tiles up to its latest row and each
 // group skips the tiles past its own last position (the contiguous 128-row q tiles this
 // replaces left the workgroup with the last tile 16x the work of the first: 2x the
@@ -239,7 +239,7 @@ struct PrefillAttnParams {
 // (dot * log2(e) / sqrt(hd)) and are exponentiated with v_exp_f32: the reference build
 // compiles with -use_fast_math, i.e. __expf / __fdividef.
 template <int HD, bool PG, int NW>
-__global__ __launch_bounds__(64 * NW, 8 / NW) void attn_prefill_mfma2_kernel(PrefillAttnParams a) {
+__global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_prefill_mfma2_kernel(PrefillAttnParams a) {
     constexpr int KT = 64;
     constexpr int CPR = HD / 8;
     constexpr int KSTEPS = HD / 32;
@@ -516,6 +516,24 @@ __global__ void tr16_probe_kernel(int32_t* out) {
     for (int e = 0; e < 4; e++) out[threadIdx.x * 4 + e] = (uint16_t)v[e];
 }
 
+// Waves (pairs of 16-row groups) of a prefill attention workgroup; `npair` pairs for each of `heads` (sequence, head)s.  The same bits.
+// 2, and 4, while every workgroup has a CU of its own: a wave's chain of key tiles is what takes the time, and it runs faster the fewer waves
+// share the CU (Qwen2-7B, 301 rows: 8 waves 16.7 us, 4 12.5, 2 12.1; 900 rows, 420 workgroups of 2, 32.5, 25.8, 31.2).  Then 8 in one round of the
+// chip: half the K / V traffic of 4 (2,048 rows 60.4 against 64.1).  In more rounds two workgroups of 4 a CU take as long as one of 8 (5 % longer
+// over long prompts), and a last round of one a CU 0.78 of that: 2,500 rows 133 / 115 us, 4,096 210 / 220, 8 x 1,024 rows 135 / 125,
+// 8 x 301 34.6 / 26.6; Qwen3-14B 2,048 rows 114 / 100.
+static int prefill_attn_waves(int64_t npair, int64_t heads, int64_t rows, int64_t cus) {
+    const int env = dev_env("QIE_ATTN_PF_NW", 0);
+    if (env == 2 || env == 4 || env == 8) return env;
+    auto wgs = [&](int nw) { return (npair + nw - 1) / nw * heads; };
+    for (int nw : {2, 4, 8})
+        if (wgs(nw) <= cus) return nw;
+    const int64_t n4 = wgs(4), rest = n4 % (2 * cus);
+    const float two = rows < 1500 ? .98f : 1.05f, t8 = (float)((wgs(8) + cus - 1) / cus);
+    const float t4 = two * (float)(n4 / (2 * cus)) + (rest == 0 ? 0.f : rest <= cus ? .78f : two);
+    return t4 < t8 ? 4 : 8;
+}
+
 static int attn_nsplit(int64_t M, int32_t max_ctx) {
     int per = dev_env("QIE_ATTN_SPLIT_TOKENS", 0);
     if (per <= 0) per = M > 8 ? 512 : 64;
@@ -629,15 +647,14 @@ int qie_attention(const void* q, int64_t M, const int32_t* pos, int32_t rows_per
         const bool pg = pa.km.table != nullptr;
         // balanced causal split: ceil(ceil(R / 16) / 2) group pairs, NW per workgroup
         const int npair = ((rows_per_seq + 15) / 16 + 1) / 2;
-        // 8 waves (16 row groups) per workgroup: each staged K/V tile feeds twice the rows, half
-        // the LDS-DMA traffic of 4-wave workgroups (P = 2,048, 7B: 74.1-74.7 -> 69.9-70.7 us,
-        // bit-identical; tools/attn_nw_check.py).  Dev A/B: QIE_ATTN_PF_NW = 4.
-        const int nw = dev_env("QIE_ATTN_PF_NW", 8) == 4 ? 4 : 8;
+        const int nw = prefill_attn_waves(npair, n_heads * (M / rows_per_seq), rows_per_seq, device_cu_count());
         dim3 g2((unsigned)((npair + nw - 1) / nw), (unsigned)n_heads, (unsigned)(M / rows_per_seq));
-        auto k2 = nw == 8 ? (cache->head_dim == 128 ? (pg ? attn_prefill_mfma2_kernel<128, true, 8> : attn_prefill_mfma2_kernel<128, false, 8>)
-                                                    : (pg ? attn_prefill_mfma2_kernel<64, true, 8> : attn_prefill_mfma2_kernel<64, false, 8>))
-                          : (cache->head_dim == 128 ? (pg ? attn_prefill_mfma2_kernel<128, true, 4> : attn_prefill_mfma2_kernel<128, false, 4>)
-                                                    : (pg ? attn_prefill_mfma2_kernel<64, true, 4> : attn_prefill_mfma2_kernel<64, false, 4>));
+        auto pick = [&](auto w) {
+            constexpr int NW = decltype(w)::value;
+            return cache->head_dim == 128 ? (pg ? attn_prefill_mfma2_kernel<128, true, NW> : attn_prefill_mfma2_kernel<128, false, NW>)
+                                          : (pg ? attn_prefill_mfma2_kernel<64, true, NW> : attn_prefill_mfma2_kernel<64, false, NW>);
+        };
+        auto k2 = nw == 8 ? pick(std::integral_constant<int, 8>{}) : nw == 4 ? pick(std::integral_constant<int, 4>{}) : pick(std::integral_constant<int, 2>{});
         hipLaunchKernelGGL(k2, g2, dim3(64 * nw), shm, (hipStream_t)stream, pa);
         QIE_LAUNCH_CHECK();
         return 0;
