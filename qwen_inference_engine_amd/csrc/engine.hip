@@ -156,6 +156,49 @@ __global__ void copy_ids_kernel(const int32_t* src, int32_t* dst, int len, int64
     if (i < len) dst[blockIdx.y * dst_stride + i] = src[(int64_t)blockIdx.y * len + i];
 }
 
+// 16 bytes a thread, the last ones singly
+__global__ __launch_bounds__(256) void fetch_out_kernel(const uint4* src, uint4* dst, int64_t whole, int rest) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < whole) dst[i] = src[i];
+    if (blockIdx.x == 0 && (int)threadIdx.x < rest)
+        reinterpret_cast<unsigned char*>(dst + whole)[threadIdx.x] = reinterpret_cast<const unsigned char*>(src + whole)[threadIdx.x];
+}
+
+void make_out(qie_batch* b, size_t bytes) {
+    bytes = (bytes + 15) / 16 * 16;
+    if (bytes == 0 || bytes > (size_t)8 << 20) return;
+    if (hipHostMalloc((void**)&b->h_out, bytes, hipHostMallocDefault) == hipSuccess) {
+        b->h_out_cap = bytes;
+        memset(b->h_out, 0, bytes);   // the host's page tables too: a first fetch of 2.4 MB was 0.7 ms longer
+    } else {
+        b->h_out = nullptr;
+        (void)hipGetLastError();
+    }
+}
+
+// A copy into pageable memory waits for the stream, stages through memory of the runtime's and waits again.  Here one launch behind the
+// step's and one wait: a step of the Nukizen design at width 2,048, 5 rows of 32,000 logits, 335 -> 313 us, of the Lugipel design in fp32, 3
+// rows, 288 -> 265; qie_batch_logits of 8 rows of Qwen2-7B 152 -> 140, of 7 of Qwen2-0.5B 138 -> 119.
+int fetch_out(qie_batch* b, void* dst, const void* src, size_t bytes, int (*check)(qie_batch*)) {
+    hipStream_t st = b->e->stream;
+    const bool pinned = bytes <= b->h_out_cap && bytes > 0;
+    if (pinned) {
+        const int64_t whole = (int64_t)(bytes / 16);
+        hipLaunchKernelGGL(fetch_out_kernel, dim3((unsigned)std::max<int64_t>(1, cdiv(whole, 256))), dim3(256), 0, st, (const uint4*)src,
+                           (uint4*)b->h_out, whole, (int)(bytes % 16));
+        QIE_LAUNCH_CHECK();
+    }
+    QIE_HIP(hipStreamSynchronize(st));
+    if (check) QIE_TRY(check(b));
+    if (pinned) {
+        memcpy(dst, b->h_out, bytes);
+    } else if (bytes > 0) {
+        QIE_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
+        QIE_HIP(hipStreamSynchronize(st));
+    }
+    return 0;
+}
+
 int dmalloc(void** p, size_t bytes) {
     QIE_HIP(hipMalloc(p, bytes < 16 ? 16 : bytes));
     return 0;
@@ -1161,6 +1204,7 @@ static int batch_create(qie_engine* e, int32_t batch, int32_t max_ctx, int32_t p
         b->h_ids = nullptr;   // (qie_decode does without)
         (void)hipGetLastError();
     }
+    if (!rc) make_out(b, (size_t)batch * s.vocab * 2);
     if (!rc) {
         hipMemsetAsync(b->dec_ws, 0, (size_t)dec_ws, e->stream);
         hipMemsetAsync(b->kc, 0, (size_t)n_runs * b->seq_stride * 2, e->stream);
@@ -1254,6 +1298,7 @@ void qie_batch_destroy(qie_batch* b) {
     for (void* p : ps)
         if (p) hipFree(p);
     if (b->h_ids) hipHostFree(b->h_ids);
+    if (b->h_out) hipHostFree(b->h_out);
     delete b;
 }
 
@@ -1554,11 +1599,10 @@ int qie_batch_logits(qie_batch* b, void* host_out) {
         QIE_TRY(gather_logits(b, 0, b->B));
         src = b->logits_full;
     }
-    QIE_HIP(hipStreamSynchronize(b->e->stream));
-    QIE_TRY(comm_check(b->e, "qie_batch_logits"));
-    QIE_TRY(pk_check(b));
-    QIE_HIP(d2h(b->e, host_out, src, (size_t)b->B * b->e->spec.vocab * 2));
-    return 0;
+    return fetch_out(b, host_out, src, (size_t)b->B * b->e->spec.vocab * 2, [](qie_batch* q) {
+        QIE_TRY(comm_check(q->e, "qie_batch_logits"));
+        return pk_check(q);
+    });
 }
 
 int qie_batch_positions(qie_batch* b, int32_t* host_pos) {

@@ -2342,6 +2342,7 @@ int layered_batch_create(qie_engine* e, int32_t batch, int32_t max_ctx, int32_t 
     LayeredBatch* s = new LayeredBatch();
     b->e = e;
     b->lb = s;
+    make_out(b, (size_t)batch * m->a.vocab * 4);
     b->B = batch;
     b->max_ctx = max_ctx;
     b->page_tokens = page_tokens;
@@ -2952,10 +2953,8 @@ int qie_batch_step(qie_batch* b, int32_t n_entries, const int32_t* slots, const 
     s->last_T = (int)T;
     s->last_want = n_want;
     s->steps++;
-    if (host_logits && n_want > 0)
-        QIE_HIP(hipMemcpyAsync(host_logits, s->logits, (size_t)n_want * e->lm->a.vocab * 4, hipMemcpyDeviceToHost, st));
-    // the staging memory and the caller's array are free again after this
-    QIE_HIP(hipStreamSynchronize(st));
+    // the staging memory is free again after this, and the caller's array has the logits
+    QIE_TRY(fetch_out(b, host_logits, s->logits, host_logits ? (size_t)n_want * e->lm->a.vocab * 4 : 0));
     s->stage_busy = false;
     return 0;
 }
