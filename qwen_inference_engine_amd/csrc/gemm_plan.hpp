@@ -231,6 +231,36 @@ inline Plan plan_wide(int64_t M, int64_t cols, int64_t K, int64_t cus) {
     return best;
 }
 
+// The best of all tiles, the 256x256 kernel left aside
+inline Plan best(int64_t M, int64_t cols, int64_t K, int64_t cus) {
+    const Plan pl = plan(M, cols, K, cus), wide = plan_wide(M, cols, K, cus);
+    // (split plans of gate / up's many columns take 10 to 30 % longer than the fit says)
+    return M > 64 && wide.tile >= 0 && wide.us < (pl.splitk > 1 ? 1.1f : 1.f) * pl.us ? wide : pl;
+}
+
+// Columns that the 256x256 kernel takes of a product, whole rounds of the chip, with the rest to the tiles above in a launch behind it; 0: one
+// launch does all.  A last round of 256x256 tiles that fills little of the chip costs a whole one, and tiles of fewer columns fill it with what
+// is left.  us, one launch / two: Qwen2-7B gate / up 400 rows 145 / 134, 900 rows 264 / 234, 1,500 356 / 345, down 6,000 784 / 687; Qwen3-14B gate / up
+// 512 rows 198 / 162, 1,024 361 / 297, 2,048 609 / 573; Qwen2-0.5B gate / up 3,500 rows 93 / 78.
+inline int64_t columns_ahead(int64_t M, int64_t cols, int64_t K, int64_t cus) {
+    const int64_t n_mt = (M + 255) / 256, n_nt = (cols + 255) / 256;
+    if (K % BK != 0 || M < 256 || n_mt * n_nt <= cus) return 0;
+    const float whole = std::min(g8p::us(M, cols, K, cus), best(M, cols, K, cus).us);
+    float least = .97f * whole;   // (of 42 shapes the sum of the two fits was 5 % over the measured ratio on the average, 8 % at most)
+    int64_t ahead = 0;
+    const int64_t full = n_mt * n_nt / cus;
+    for (int64_t r = full; r >= 1 && r >= full - 1; r--) {
+        const int64_t c = r * cus / n_mt * 256;
+        if (c <= 0 || c >= cols) continue;
+        const float us = g8p::us(M, c, K, cus) + best(M, cols - c, K, cus).us;
+        if (us < least) {
+            least = us;
+            ahead = c;
+        }
+    }
+    return ahead;
+}
+
 // The tiles that take a product; tile -1: none, k_gemm.hip's kernels do.
 inline Plan choose(int64_t M, int64_t cols, int64_t K, int64_t cus) {
     const Plan none{-1, 0, 1, 0, 0, 1e30f};

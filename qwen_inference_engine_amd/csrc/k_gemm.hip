@@ -1536,6 +1536,8 @@ static int gemm_with(const qie_linear_args* a, const QkvTail* tail, bool* done, 
     QIE_REQUIRE(a->K % 8 == 0, "qie_linear: GEMM needs K %% 8 == 0");
     if (!(a->flags & QIE_LINEAR_FP8) && a->K % big::BK == 0 && a->ldx % 8 == 0) {
         // In this order:
+        //   0. more 256x256 tiles than CUs, one weight segment (SwiGLU: two): whole rounds of the phase-interleaved kernel for the first columns and
+        //      k_gemm_mid.hip's tiles for the rest, where mid::columns_ahead expects that to be the faster;
         //   1. K a multiple of 64: k_gemm_mid.hip, unless the next is expected to be faster (mid::choose);
         //   2. K a multiple of 64 from 256 on, 256 rows: the phase-interleaved 256x256 kernel, whole where its tiles fill the chip,
         //      or half of it when K is too short to split; split over K otherwise;
@@ -1553,6 +1555,22 @@ static int gemm_with(const qie_linear_args* a, const QkvTail* tail, bool* done, 
         // phase-interleaved 256x256 kernel (K a multiple of 64, >= 4 k-tiles): Qwen2-7B gate/up at 2,048
         // rows 612 -> 488 us, bit-identical to gemm_big; down split-K 2: 309 -> 247 us
         const bool g8ok = a->K % g8::BK == 0 && a->K >= 4 * g8::BK;
+        const bool one_segment = a->epilogue == QIE_EPI_SWIGLU || a->seg_rows[0] == a->N;
+        if (g8ok && force < 0 && !tail && one_segment && !(a->flags & QIE_LINEAR_STREAMK) && a->ldy <= 1 << 20 && dev_env("QIE_HYBRID", 1)) {
+            const int64_t ahead = mid::columns_ahead(a->M, cols, a->K, cus) / (a->epilogue == QIE_EPI_SWIGLU ? 2 : 1);   // outputs
+            if (ahead > 0) {
+                GemmParams first = p, rest = p;
+                first.N = first.n0 = first.n01 = ahead;
+                rest.N = rest.n0 = rest.n01 = a->N - ahead;
+                rest.w0 += ahead * a->K;
+                if (a->epilogue == QIE_EPI_SWIGLU) rest.w1 += ahead * a->K;
+                if (p.b0) rest.b0 += ahead;
+                rest.C += ahead * (a->epilogue == QIE_EPI_F32 ? 2 : 1);   // (ahead: a multiple of 128, so p.vec holds for both)
+                const int64_t n_nt = ahead * (a->epilogue == QIE_EPI_SWIGLU ? 2 : 1) / 256;
+                QIE_TRY(launch_gemm8(a->epilogue, first, (int)n_mt, (int)(n_mt * n_nt), G8Split{1, nullptr, nullptr}, nullptr, st));
+                return gemm_mid_rest(a->epilogue, rest, st);
+            }
+        }
         // (Qwen2-7B gate/up, us: 301 rows 161 with the 256x256 kernel, 97 with k_gemm_mid.hip; 700 rows 183 against 229)
         if (dev_env("QIE_MID", 1) && force < 0 && !(a->flags & QIE_LINEAR_STREAMK)) {
             bool launched = false;

@@ -450,24 +450,32 @@ int launch_mid(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, hipS
 }
 }  // namespace
 
-int gemm_mid(const qie_linear_args* a, const GemmParams& p, const QkvTail* tail, hipStream_t st, bool* launched) {
-    *launched = false;
-    const mid::Plan pl = mid::choose(a->M, a->epilogue == QIE_EPI_SWIGLU ? 2 * a->N : a->N, a->K, device_cu_count());
-    if (pl.tile < 0 || a->ldy > 1 << 20) return 0;   // (a tile of C by 32-bit offsets)
+static int run_mid(int epi, const GemmParams& p, const mid::Plan& pl, const QkvTail* tail, hipStream_t st) {
     G8Split sk{1, nullptr, nullptr};
     const int64_t cut = (int64_t)pl.n_mt * pl.n_nt - pl.whole;
     if (pl.splitk > 1 && cut > 0) {
         const int64_t floats = cut * pl.splitk * mid::shape(pl.tile).bm * mid::shape(pl.tile).bn;
         if (g8_workspace(st, (int)cdiv(floats, 65536), (int)cut * 8 * TICKET, &sk) == 0) sk.splitk = pl.splitk;
     }
-    *launched = true;
     if (tail) return launch_mid<kEpiQkv>(p, pl, sk, st, *tail);
-    switch (a->epilogue) {
+    switch (epi) {
         case QIE_EPI_SWIGLU: return launch_mid<QIE_EPI_SWIGLU>(p, pl, sk, st);
         case QIE_EPI_RESIDUAL: return launch_mid<QIE_EPI_RESIDUAL>(p, pl, sk, st);
         case QIE_EPI_F32: return launch_mid<QIE_EPI_F32>(p, pl, sk, st);
         default: return launch_mid<QIE_EPI_STORE>(p, pl, sk, st);
     }
+}
+
+int gemm_mid(const qie_linear_args* a, const GemmParams& p, const QkvTail* tail, hipStream_t st, bool* launched) {
+    *launched = false;
+    const mid::Plan pl = mid::choose(a->M, a->epilogue == QIE_EPI_SWIGLU ? 2 * a->N : a->N, a->K, device_cu_count());
+    if (pl.tile < 0 || a->ldy > 1 << 20) return 0;   // (a tile of C by 32-bit offsets)
+    *launched = true;
+    return run_mid(a->epilogue, p, pl, tail, st);
+}
+
+int gemm_mid_rest(int epi, const GemmParams& p, hipStream_t st) {
+    return run_mid(epi, p, mid::best(p.M, epi == QIE_EPI_SWIGLU ? 2 * p.N : p.N, p.K, device_cu_count()), nullptr, st);
 }
 
 }  // namespace qie

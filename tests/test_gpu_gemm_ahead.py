@@ -1,0 +1,82 @@
+"""Products in two launches, whole rounds of 256x256 tiles for the first columns and smaller tiles for the rest (gemm_plan.hpp columns_ahead): every
+epilogue, ragged columns, odd row strides, against fp32 products; and the rule itself on the host."""
+import os
+import random
+import subprocess
+
+import numpy as np
+import pytest
+
+import gpu_util as G
+from gemm_route import CSRC
+from qwen_inference_engine_amd import _lib
+from test_gpu_gemm_mid import bf16, linear, products
+
+DRIVER = r"""
+#include "gemm_plan.hpp"
+#include <cstdio>
+int main() {
+    long M, cols, K, cus;
+    while (std::scanf("%ld %ld %ld %ld", &M, &cols, &K, &cus) == 4) std::printf("%ld\n", (long)qie::mid::columns_ahead(M, cols, K, cus));
+}
+"""
+SHAPES = [(1030, 13500, 256), (700, 22004, 256), (511, 33001, 256), (2300, 7510, 256), (300, 43000, 768)]
+
+
+def ahead(tmp_path, cases):
+    (tmp_path / "d.cpp").write_text(DRIVER)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(tmp_path / "d.cpp"), "-o", str(tmp_path / "d")], check=True)
+    text = "\n".join("%d %d %d %d" % c for c in cases)
+    return [int(v) for v in subprocess.run([str(tmp_path / "d")], input=text, text=True, capture_output=True, check=True).stdout.split()]
+
+
+def test_the_rule_is_sound(tmp_path):
+    """What goes ahead is whole column tiles in whole rounds of the chip, and something is left."""
+    assert all(0 < a < N for (_, N, _), a in zip(SHAPES, ahead(tmp_path, [(*s, 256) for s in SHAPES])))
+    r = random.Random(4)
+    cases = [(r.randint(1, 9000), r.randint(8, 60000), 64 * r.randint(1, 300), r.choice([256, 304, 64])) for _ in range(3000)]
+    got = ahead(tmp_path, cases)
+    assert sum(a > 0 for a in got) > 100
+    for (M, cols, K, cus), a in zip(cases, got):
+        tiles = -(-M // 256) * (a // 256)
+        assert a == 0 or (a % 256 == 0 and a < cols and M >= 256 and K >= 256 and (tiles % cus == 0 or cus - tiles % cus < -(-M // 256))), (M, cols, K, cus, a)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,rows,K", SHAPES)
+@pytest.mark.parametrize("epi", ["f32", "store", "residual", "swiglu"])
+def test_two_launches(qlib, oracle, M, rows, K, epi):
+    N = rows // 2 if epi == "swiglu" else rows
+    ld = N + 3
+    x = bf16((M, K), 1.0, 21)
+    if epi == "swiglu":
+        wg, wu, y0 = bf16((N, K), 1.5 * K ** -0.5, 22), bf16((N, K), K ** -0.5, 23), bf16((M + 1, ld), 1.0, 24)
+        y = G.dev(y0)
+        linear(G.dev(x), [G.dev(wg), G.dev(wu)], [], M, K, N, y, _lib.QIE_EPI_SWIGLU, ldy=ld)
+        (g, gs), (u, us) = products(x, wg), products(x, wu)
+        want = u / (1.0 + np.exp(-g)) * g
+        # |silu'| <= 1.1; three bf16 roundings (gate, silu, product) and one of the up sum
+        tol = 2.0 ** -7 * (np.abs(want) + 1.1 * np.abs(u) * np.abs(g)) + 1e-5 * (1.1 * np.abs(u) * gs + np.abs(g) * us)
+    else:
+        w = bf16((N, K), K ** -0.5, 22)
+        acc, scale = products(x, w)
+        if epi == "f32":
+            y = G.zeros((M, N), np.float32)
+            linear(G.dev(x), [G.dev(w)], [], M, K, N, y, _lib.QIE_EPI_F32)
+            assert (np.abs(y.numpy() - acc) <= 1e-5 * scale).all()
+            return
+        y0 = bf16((M + 1, ld), 1.0, 24)
+        y = G.dev(y0)
+        if epi == "store":
+            b = bf16((N,), 0.5, 25)
+            linear(G.dev(x), [G.dev(w)], [G.dev(b)], M, K, N, y, _lib.QIE_EPI_STORE, ldy=ld)
+            want = acc + G.bf(b)
+            tol = 2.0 ** -8 * np.abs(want) + 1e-5 * scale
+        else:
+            linear(G.dev(x), [G.dev(w)], [], M, K, N, y, _lib.QIE_EPI_RESIDUAL, ldy=ld)
+            want = G.bf(y0)[:M, :N] + G.bf(oracle.f32_to_bf16(acc))
+            # bf16(res + bf16(acc)): an ulp of either rounding
+            tol = 2.0 ** -7 * (np.abs(acc) + np.abs(want)) + 1e-5 * scale
+    got = G.host_bf16(y)
+    assert (np.abs(G.bf(got)[:M, :N] - want) <= tol).all()
+    assert np.array_equal(got[:M, N:], y0[:M, N:]) and np.array_equal(got[M], y0[M])
