@@ -92,6 +92,7 @@ struct qie_batch {
     int32_t* h_ids = nullptr;         // pinned: [B] first positions, then the ids of qie_decode [n_steps][B], ids_at_once of them (null: none)
     unsigned char* h_out = nullptr;   // pinned: what goes back to the caller's pageable memory (fetch_out; null: none)
     size_t h_out_cap = 0;
+    unsigned char* h_pinned = nullptr;   // the allocation of both
     // prefill scratch
     int64_t pf_rows = 0;
     uint16_t *pf_x = nullptr, *pf_hn = nullptr, *pf_qkv = nullptr, *pf_q = nullptr, *pf_att = nullptr,
@@ -127,8 +128,8 @@ struct qie_batch {
 
 namespace qie {
 // hipMalloc of at least 16 bytes
-// Pinned memory for results of up to `bytes` (8 MB at most), made with the batch; none if there is none.
-void make_out(qie_batch* b, size_t bytes);
+// Pinned memory of a batch, made with it: for results of up to `bytes` (none above 8 MB), behind `ids` bytes for h_ids.
+void make_out(qie_batch* b, size_t bytes, size_t ids = 0);
 // `bytes` of device memory, 16-byte aligned, to the caller's: behind everything on the engine's stream, waited for.  check: run between the wait
 // and the copy into dst (what makes the results void).
 int fetch_out(qie_batch* b, void* dst, const void* src, size_t bytes, int (*check)(qie_batch*) = nullptr);
