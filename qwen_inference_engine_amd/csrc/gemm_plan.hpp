@@ -142,8 +142,12 @@ inline float us(int64_t M, int64_t cols, int64_t K, int64_t cus) {
 namespace mid {
 constexpr int BK = 64;
 
-// Times of a tile, us, fitted to the Qwen2-0.5B / 7B and Qwen3-14B projections at 20 to 2,048 rows (168 shapes; what the
-// rule below picks is 1 % over the best of all tiles, splits and the 256x256 kernel on the average, 17 % at most):
+// Times of a tile, us, fitted to the projections of Qwen2-0.5B / 1.5B / 7B, Qwen3-14B and of 4,096 columns at 17 to 2,300 rows (474
+// shapes, each measured on every tile with 1 to 8 segments; what the rule below picks is 1.6 % over the best of all of them on the
+// average and 17 % at most, with the constants fitted to 168 shapes before the kernel's ring and tickets changed 2.3 %).  Of 960
+// other shapes 156 went to another tile and took 0.97 of their time on the average: 1,536 -> 2 x 8,960 gate / up at 184 rows
+// 28.8 -> 24.1 us, 3,584 -> 4,608 at 489 36.4 -> 31.1, 17,408 -> 5,120 at 133 61.3 -> 53.5; the worst, 3,584 -> 3,584 at 214, 17.0
+// -> 18.6:
 // up to one workgroup a CU a1 + s1 per k-tile, more a2 + (rounds of the chip) * (f2 + s2 per k-tile).  A k-tile costs what its
 // lines take through one CU (about 50 GB/s where they come from HBM or another die, 120 GB/s from L2), not its matrix work,
 // which is why the tall tiles win as soon as the rows fill them.  The constants are an MI355X's, whole (256 CUs): `cus` moves
@@ -154,18 +158,18 @@ struct Tile {
     float a1, s1, a2, f2, s2;
 };
 constexpr Tile TILES[] = {
-    {64, 64, 5, 2, 3.2f, .285f, 5.f, .7f, .487f},   {64, 128, 3, 2, 2.6f, .475f, 5.4f, 1.1f, .74f},
-    {128, 64, 3, 2, 3.3f, .43f, 4.7f, 1.8f, .70f},  {128, 128, 4, 1, 5.9f, .54f, 7.5f, 3.9f, .575f},
-    {192, 128, 4, 1, 8.f, .65f, 5.f, 6.f, .72f},    {256, 128, 3, 1, 9.9f, .90f, 12.f, 2.5f, 1.037f},
-    {320, 64, 3, 1, 6.9f, .70f, 6.5f, 3.f, .787f},  {320, 128, 2, 1, 9.4f, 1.11f, 14.f, 2.f, 1.2f},
+    {64, 64, 5, 2, 3.16f, .285f, 4.93f, .68f, .487f}, {64, 128, 3, 2, 2.5f, .468f, 5.f, 1.05f, .71f},
+    {128, 64, 3, 2, 3.16f, .423f, 4.06f, 1.75f, .677f}, {128, 128, 4, 1, 5.38f, .539f, 4.43f, 2.78f, .554f},
+    {192, 128, 4, 1, 5.27f, .65f, 0.f, 6.45f, .693f}, {256, 128, 3, 1, 7.23f, .748f, 15.87f, .53f, .931f},
+    {320, 64, 3, 1, 4.68f, .711f, 5.22f, 2.82f, .769f}, {320, 128, 2, 1, 8.f, 1.041f, 12.67f, .28f, 1.196f},
 };
 constexpr int N_TILES = sizeof(TILES) / sizeof(TILES[0]);
 // Tiles of 160 columns, numbered on from TILES: where the columns of 128-column tiles start a round of the chip that they hardly fill
 // (37,888 columns: 296 tiles, 237 of these), and so many rows of the workgroups' own (weights) that a tile of fewer columns loads more
 // for the same outputs.  Whole only.
 constexpr Tile WIDE[] = {
-    {128, 160, 4, 1, 3.f, 1.f, 11.7f, 0.f, .69f}, {192, 160, 3, 1, 6.6f, 1.1f, 7.1f, 6.3f, .825f},
-    {256, 160, 3, 1, 8.8f, 1.29f, 0.f, 10.f, 1.f}, {320, 160, 2, 1, 9.6f, 1.56f, 0.f, 13.f, 1.17f},
+    {128, 160, 4, 1, 4.89f, .657f, 9.82f, .01f, .655f}, {192, 160, 3, 1, 6.33f, .776f, 3.01f, 4.56f, .829f},
+    {256, 160, 3, 1, 4.85f, 1.139f, 0.f, 8.74f, .922f}, {320, 160, 2, 1, 6.26f, 1.498f, 0.f, 10.73f, 1.137f},
 };
 constexpr int N_WIDE = sizeof(WIDE) / sizeof(WIDE[0]);
 inline const Tile& shape(int tile) { return tile < N_TILES ? TILES[tile] : WIDE[tile - N_TILES]; }
@@ -200,7 +204,7 @@ inline Plan plan(int64_t M, int64_t cols, int64_t K, int64_t cus) {
             } else {
                 if (cut == 0) break;
                 const float len = (float)((nk + s - 1) / s);
-                us = whole / room * (t.f2 + nk * t.s2) + 3.f * s * (t.bm * t.bn) / 16384.f + 1.f;
+                us = whole / room * (t.f2 + nk * t.s2) + 2.82f * s * (t.bm * t.bn) / 16384.f + .74f;
                 us += cut <= cus ? t.a1 + len * t.s1 : t.a2 + rounds(cut / room) * (t.f2 + len * t.s2);
             }
             us = std::max(us, floor_us);

@@ -20,7 +20,7 @@ int main() {
     while (std::scanf("%ld %ld %ld %ld", &M, &cols, &K, &cus) == 4) std::printf("%ld\n", (long)qie::mid::columns_ahead(M, cols, K, cus));
 }
 """
-SHAPES = [(1030, 13500, 256), (700, 22004, 256), (511, 33001, 256), (2300, 7510, 256), (300, 43000, 768)]
+SHAPES = [(1030, 13500, 768), (700, 22004, 512), (511, 33001, 256), (2300, 7510, 256), (345, 45029, 768)]
 
 
 def ahead(tmp_path, cases):
