@@ -175,8 +175,9 @@ typedef unsigned int u32x2_g8 __attribute__((ext_vector_type(2)));
 struct G8Split {
     int splitk;
     float* slab;       // [tiles][splitk][256 * 256] fp32
-    unsigned* cnt;     // [tiles], zero at rest
+    unsigned* cnt;     // tickets, zero at rest; a tile's eight waves' in lines of their own
 };
+constexpr int G8_TICKET = 16;   // words of a ticket: a line
 // (with four ints the arguments of the GEMM kernels: three lines of the segment, and the grid's size behind them in the third)
 static_assert(sizeof(GemmParams) + 4 * sizeof(int) + sizeof(G8Split) + 8 + 4 <= 192, "arguments of the GEMM kernels");
 

@@ -428,13 +428,70 @@ constexpr int BM = 256, BN = 256, BK = 64;
 constexpr int BUF = (BM + BN) * BK * 2;   // 64 KB: A rows [0, 256) then W rows, 128 B each
 }  // namespace g8
 
-// Split-K (tiles < CUs: Qwen2-7B O / down at 2,048 rows have 112 256x256 tiles, QKV 144): the
-// k-tiles of a tile are cut into `splitk` consecutive parts, one workgroup each (the remap
-// keeps a tile's parts on one XCD).  Every part stores its fp32 accumulators write-through
-// (sc1) into its slab [tile][part] (256 KB, each lane's 16-B accumulator quads in fragment
-// order), drains, and adds to the tile's ticket; the part whose add comes last sums the slabs
-// in PART order (sc1 loads: cdna_hip_programming.md §5 'Projection GEMM' item 2), so the result
-// does not depend on arrival order, runs the epilogue and resets the ticket.
+// Split-K (tiles < CUs: Qwen2-7B down at 2,048 rows has 112 256x256 tiles): the k-tiles of a tile are cut into `splitk`
+// consecutive parts, one workgroup each (the remap keeps a tile's parts on one XCD), and meet wave by wave: a wave stores its
+// share of the fp32 accumulators write-through (sc1) into its part's slab [tile][part] (256 KB, each lane's 16-B quads in fragment
+// order), drains, and adds to its ticket of the tile; the wave whose add comes last sums the parts in PART order (its own from
+// registers, the others by sc1 loads), so the result does not depend on arrival order, runs the epilogue and resets the ticket.
+// No wave waits for the others of its workgroup, and the sums are spread over the parts' CUs: 4 to 9 us, of one CU's reading of all
+// of a tile's slabs, are 2 to 4 % of the products that are cut (us before / now: Qwen2-7B down 2,016 rows 246 / 241, 1,344 rows in 3
+// parts 185 / 182, Qwen3-14B down 2,112 rows in 4 parts 429 / 413).
+template <class Acc>
+__device__ __forceinline__ bool sum_parts(const G8Split& sk, int tile, int part, int wave, int lane, Acc& acc) {
+    const int64_t tb = (int64_t)tile * sk.splitk;
+    const int at = (wave * 32 * 64 + lane) * 16;
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc(sk.slab + (tb + part) * 65536, (short)0, 65536 * 4, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_g8, acc[i][j]), rs, at + (i * 4 + j) * 1024, 0, 16);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // stored
+    unsigned* cnt = sk.cnt + (tile * 8 + wave) * G8_TICKET;
+    unsigned old = 0;
+    if (lane == 0) old = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    old = __builtin_amdgcn_readfirstlane(old);
+    if (old != (unsigned)sk.splitk - 1) return false;   // uniform
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i0 = 0; i0 < 8; i0 += 2) {   // (eight quads a wave on their way: 64 KB a CU, and what registers there are beside the accumulators)
+        const auto load = [&](int q, f32x4 (&v)[2][4]) {
+            const auto rq = __builtin_amdgcn_make_buffer_rsrc(sk.slab + (tb + q) * 65536, (short)0, 65536 * 4, 0x00020000);
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    v[i][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rq, at + ((i0 + i) * 4 + j) * 1024, 0, 16));
+        };
+        f32x4 v[2][4];
+        if (part > 0) {
+            load(0, v);
+            for (int q = 1; q < part; q++) {
+                f32x4 w[2][4];
+                load(q, w);
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) v[i][j] += w[i][j];
+            }
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[i0 + i][j] += v[i][j];
+        }
+        for (int q = part + 1; q < sk.splitk; q++) {
+            load(q, v);
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[i0 + i][j] += v[i][j];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (lane == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+}
+
 template <int EPI>
 __global__ __launch_bounds__(512) void gemm8_kernel(GemmParams p, int n_mt, int n_nt, int gm, G8Split sk, TailOf<EPI> tail) {
 #pragma clang fp contract(off)
@@ -580,42 +637,7 @@ __global__ __launch_bounds__(512) void gemm8_kernel(GemmParams p, int n_mt, int 
     }
     if (wm == 0) bar();   // balance the barrier count of the two wave groups
 
-    if (sk.splitk > 1) {   // uniform
-        // this wave's quads: slab float offset ((wave * 32 + i * 4 + j) * 64 + lane) * 4
-        const int64_t tb = (int64_t)tile * sk.splitk;
-        const auto rs = __builtin_amdgcn_make_buffer_rsrc(sk.slab + (tb + part) * 65536, (short)0, 65536 * 4, 0x00020000);
-#pragma unroll
-        for (int i = 0; i < 8; i++)
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_g8, acc[i][j]), rs,
-                                                       ((wave * 32 + i * 4 + j) * 64 + lane) * 16, 0, 16);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every storing wave drains
-        __syncthreads();
-        int* flag = reinterpret_cast<int*>(smem);   // the staging array is free (one LDS object)
-        if (tid == 0) {
-            const unsigned old = __hip_atomic_fetch_add(sk.cnt + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            *flag = old == (unsigned)sk.splitk - 1 ? 1 : 0;
-        }
-        __syncthreads();
-        if (*flag == 0) return;   // uniform
-#pragma unroll
-        for (int i = 0; i < 8; i++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int q = 0; q < sk.splitk; q++) {   // part order: independent of who arrived last
-            const auto rq = __builtin_amdgcn_make_buffer_rsrc(sk.slab + (tb + q) * 65536, (short)0, 65536 * 4, 0x00020000);
-#pragma unroll
-            for (int i = 0; i < 8; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const f32x4 v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                                  rq, ((wave * 32 + i * 4 + j) * 64 + lane) * 16, 0, 16));
-                    acc[i][j] = q == 0 ? v : acc[i][j] + v;
-                }
-        }
-        if (tid == 0) __hip_atomic_store(sk.cnt + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if (sk.splitk > 1 && !sum_parts(sk, tile, part, wave, lane, acc)) return;   // uniform
 
     // ---------------- epilogue.  D = W Aᵀ: a lane holds row lane & 15 and columns 4 g .. 4 g + 3 of a fragment, one 8- (fp32: 16-)
     // byte store where C's rows allow it
@@ -1337,41 +1359,7 @@ __global__ __launch_bounds__(512) void gemm8mx_kernel(MxParams p, int n_mt, G8Sp
     }
     if (wm == 0) bar();
 
-    if (sk.splitk > 1) {   // uniform (gemm8's split-K hand-off, part order)
-        const int64_t tb = (int64_t)tile * sk.splitk;
-        const auto rs = __builtin_amdgcn_make_buffer_rsrc(sk.slab + (tb + part) * 65536, (short)0, 65536 * 4, 0x00020000);
-#pragma unroll
-        for (int i = 0; i < 8; i++)
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_g8, acc[i][j]), rs,
-                                                       ((wave * 32 + i * 4 + j) * 64 + lane) * 16, 0, 16);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        int* flag = reinterpret_cast<int*>(smem);
-        if (tid == 0) {
-            const unsigned old = __hip_atomic_fetch_add(sk.cnt + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            *flag = old == (unsigned)sk.splitk - 1 ? 1 : 0;
-        }
-        __syncthreads();
-        if (*flag == 0) return;
-#pragma unroll
-        for (int i = 0; i < 8; i++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int q = 0; q < sk.splitk; q++) {
-            const auto rq = __builtin_amdgcn_make_buffer_rsrc(sk.slab + (tb + q) * 65536, (short)0, 65536 * 4, 0x00020000);
-#pragma unroll
-            for (int i = 0; i < 8; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const f32x4 v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                                  rq, ((wave * 32 + i * 4 + j) * 64 + lane) * 16, 0, 16));
-                    acc[i][j] = q == 0 ? v : acc[i][j] + v;
-                }
-        }
-        if (tid == 0) __hip_atomic_store(sk.cnt + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if (sk.splitk > 1 && !sum_parts(sk, tile, part, wave, lane, acc)) return;   // uniform
 
     // ---------------- epilogue (gemm8_kernel's)
     constexpr int NJ = 4;
@@ -1502,7 +1490,7 @@ static int gemm_mx(const qie_linear_args* a, hipStream_t st) {
                 best = s;
             }
         }
-        if (best > 1 && g8_workspace(st, (int)tiles * best, (int)tiles, &sk) == 0) sk.splitk = best;
+        if (best > 1 && g8_workspace(st, (int)tiles * best, (int)tiles * 8 * G8_TICKET, &sk) == 0) sk.splitk = best;
     }
     return t16 ? launch_gemm8mx<true>(a->epilogue, p, (int)n_mt, (int)tiles, sk, st)
                : launch_gemm8mx<false>(a->epilogue, p, (int)n_mt, (int)tiles, sk, st);
@@ -1593,7 +1581,7 @@ static int gemm_with(const qie_linear_args* a, const QkvTail* tail, bool* done, 
         if (g8ok && g8mode == 2 && force < 0 && a->M >= big::BM && t256 < cus) {
             const int s = g8p::parts(a->M, cols, a->K, cus, std::max(4, dev_env("QIE_GEMM8_SK_MINK", 64)));   // (dev A/B: k-tiles a part)
             G8Split sk{1, nullptr, nullptr};
-            if (s == 1 || (s > 1 && g8_workspace(st, (int)t256 * s, (int)t256, &sk) == 0 && (sk.splitk = s) > 1)) {
+            if (s == 1 || (s > 1 && g8_workspace(st, (int)t256 * s, (int)t256 * 8 * G8_TICKET, &sk) == 0 && (sk.splitk = s) > 1)) {
                 if (done) *done = tail != nullptr;
                 return launch_gemm8(a->epilogue, p, (int)n_mt, (int)t256, sk, tail, st);
             }

@@ -53,8 +53,6 @@ __device__ __forceinline__ const uint16_t* mid_wrow(const GemmParams& p, int64_t
     }
 }
 
-constexpr int TICKET = 16;   // words of a ticket: a line of its own
-
 template <int EPI, int BM, int BN, int SA, int SW, int KW, bool TURNS>
 __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, int n_nt, int gm, int whole, G8Split sk, TailOf<EPI> tail) {
 #pragma clang fp contract(off)
@@ -320,7 +318,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
             for (int j = 0; j < FJ; j++)
                 __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_g8, res[i][j]), rs, slab_at + (i * FJ + j) * 1024, 0, 16);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // stored
-        unsigned* cnt = sk.cnt + (ct * 8 + wave) * TICKET;
+        unsigned* cnt = sk.cnt + (ct * 8 + wave) * G8_TICKET;
         unsigned old = 0;
         if (lane == 0) old = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         old = __builtin_amdgcn_readfirstlane(old);
@@ -455,7 +453,7 @@ static int run_mid(int epi, const GemmParams& p, const mid::Plan& pl, const QkvT
     const int64_t cut = (int64_t)pl.n_mt * pl.n_nt - pl.whole;
     if (pl.splitk > 1 && cut > 0) {
         const int64_t floats = cut * pl.splitk * mid::shape(pl.tile).bm * mid::shape(pl.tile).bn;
-        if (g8_workspace(st, (int)cdiv(floats, 65536), (int)cut * 8 * TICKET, &sk) == 0) sk.splitk = pl.splitk;
+        if (g8_workspace(st, (int)cdiv(floats, 65536), (int)cut * 8 * G8_TICKET, &sk) == 0) sk.splitk = pl.splitk;
     }
     if (tail) return launch_mid<kEpiQkv>(p, pl, sk, st, *tail);
     switch (epi) {
