@@ -8,15 +8,13 @@
 //     selection order (value, then bitrev8(idx mod 256), then -idx; see
 //     qie_common.hpp sel_key) — greedy is a parallel max over keys (also fused
 //     into the lm_head GEMV epilogue, k_gemv.hip);
-//   * top-k = a radix selection per 4096-slice, one over the slices' winners, and a sort of
-//     the k that are left; the sorted keys reproduce the reference's k rounds exactly;
+//   * top-k = a radix selection per 4096-slice, sorted, and one pass over the slices' winners that
+//     leaves out what cannot be among the k; the sorted keys reproduce the reference's k rounds exactly;
 //   * softmax + draw in one wave: exponentials a lane each, sums in the reference's
 //     sequential order lane by lane, and a cuRAND-XORWOW restatement (curand_init(seed, 0, 0);
 //     curand_uniform).
 #include "qie_common.hpp"
 #include "../../include/qie/qie_ops.h"
-
-#include <algorithm>
 
 namespace qie {
 
@@ -51,29 +49,9 @@ __global__ void keys_to_ids_kernel(const unsigned long long* keys, int64_t M, in
     if (m < M) ids[m] = key_idx(keys[m]);
 }
 
-// Bitonic sort, descending, of n (power of two) keys in LDS.
-__device__ void bitonic_desc(unsigned long long* k, int n) {
-    for (int size = 2; size <= n; size <<= 1) {
-        for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            for (int j = threadIdx.x; j < n / 2; j += blockDim.x) {
-                const int i = (j / stride) * 2 * stride + (j % stride);
-                const int q = i + stride;
-                const bool desc = (i & size) == 0;
-                unsigned long long a = k[i], b = k[q];
-                if (desc ? (a < b) : (a > b)) {
-                    k[i] = b;
-                    k[q] = a;
-                }
-            }
-            __syncthreads();
-        }
-    }
-}
-
 // The k largest of a block's keys (KPT a thread, in registers), unordered, into out[0, k) (LDS or memory; zeros behind the
 // last where fewer than k keys are non-zero).  Radix selection from the top byte: a histogram of the keys that still share the
-// threshold's prefix, until the bin of the k-th holds just what is needed: three to six passes of about 1.5 us where the
-// bitonic sort of 4,096 keys makes 78.  (Bits 47..32 are the low half of a bf16's fp32 pattern: known from its sign.)
+// threshold's prefix, until the bin of the k-th holds just what is needed: three to six passes of about 1.5 us.  (Bits 47..32 are the low half of a bf16's fp32 pattern: known from its sign.)
 template <int KPT>
 __device__ void radix_top(const unsigned long long (&key)[KPT], int k, unsigned long long* out) {
     __shared__ unsigned hist[256];
@@ -136,6 +114,21 @@ __device__ void radix_top(const unsigned long long (&key)[KPT], int k, unsigned 
     __syncthreads();
 }
 
+// How many of keys[0, n) (LDS; a zero behind them where n is odd) are above `own`: its place among them in descending order, the
+// keys being distinct.  Two keys a read that serves the whole wave, no barriers: 0.5 us for 50 keys, where a bitonic sort of 64 in
+// LDS took 21 barriers, 4 us.
+__device__ __forceinline__ int rank_of(unsigned long long own, const unsigned long long* keys, int n) {
+    const ulonglong2* two = reinterpret_cast<const ulonglong2*>(keys);
+    int above = 0;
+#pragma unroll 8
+    for (int j = 0; j < (n + 1) / 2; j++) {
+        const ulonglong2 q = two[j];
+        above += (q.x > own) + (q.y > own);
+    }
+    return above;
+}
+
+// The k best of a slice, in descending order, zeros behind the last.
 __global__ __launch_bounds__(256) void topk_slice_kernel(const uint16_t* __restrict__ logits, int64_t V,
                                                          int64_t ld, int k,
                                                          unsigned long long* __restrict__ cand) {
@@ -155,8 +148,13 @@ __global__ __launch_bounds__(256) void topk_slice_kernel(const uint16_t* __restr
         const int64_t idx = base + threadIdx.x + 256 * i;
         key[i] = idx < V ? sel_key(bf2f(v[i]), (uint32_t)idx) : 0ull;
     }
-    // (at least k keys: k <= kMaxTopK <= kSlice)
-    radix_top<KPT>(key, k, cand + (m * gridDim.x + blockIdx.x) * (int64_t)k);
+    __shared__ __attribute__((aligned(16))) unsigned long long top[kMaxTopK + 2];
+    if (threadIdx.x == 0) top[k] = 0ull;
+    radix_top<KPT>(key, k, top);   // (at least k keys: k <= kMaxTopK <= kSlice; ends in a barrier)
+    const int i = threadIdx.x;
+    if (i >= k) return;
+    const unsigned long long own = top[i];   // (zeros stand behind the keys)
+    cand[(m * gridDim.x + blockIdx.x) * (int64_t)k + (own != 0ull ? rank_of(own, top, k) : i)] = own;
 }
 
 // cuRAND XORWOW, curand_init(seed, subsequence = 0, offset = 0) (no skip-ahead)
@@ -177,16 +175,24 @@ __device__ __forceinline__ float xorwow_uniform_first(uint64_t seed) {
 
 // One block per row: the k best of the slices' candidates, sorted, then temperature, softmax and one draw
 // (logit_decode.cu:225-272) by one wave that holds candidate i in lane i % 64: the exponentials side by side, the sums in the
-// reference's order.  k2: the power of two >= max(k, 2).
+// reference's order.
+// Bound by its steps' latencies.  Of `full` whole slices the least key in place ceil(k / full) has k keys at or above it, so what is
+// below it is left out first: of 151,936 logits and k = 50 some 250 of 1,900 candidates stay and are put in order at once, where a
+// radix selection makes four to six passes of 1.5 us.  It is still made where more than kFew stay (a few slices with all the best).
+// The running sums are made once: the total, the nucleus and the draw read them (were four chains of k additions).  us of a
+// call with its slices, 7 rows of 151,936 logits, k = 50: 30 to 35 -> 25; k = 256: 58 to 100 -> 42 to 56.
+constexpr int kFew = 768;
 template <int KPT>
 __global__ __launch_bounds__(256) void topk_merge_sample_kernel(const unsigned long long* __restrict__ cand,
-                                                                int nb, int k, int k2, float temperature,
+                                                                int nb, int full, int k, float temperature,
                                                                 float top_p, uint64_t seed,
                                                                 const int32_t* step, int32_t* ids) {
 #pragma clang fp contract(off)
     __shared__ unsigned long long sk[kMaxTopK];
+    __shared__ __attribute__((aligned(16))) unsigned long long few[kFew];
+    __shared__ int n_few;
     const int64_t m = blockIdx.x;
-    const int total = nb * k;
+    const int total = nb * k, lane = threadIdx.x & 63;
     unsigned long long key[KPT];
 #pragma unroll
     for (int i = 0; i < KPT; i++) {
@@ -194,12 +200,48 @@ __global__ __launch_bounds__(256) void topk_merge_sample_kernel(const unsigned l
         const unsigned long long c = cand[m * total + (j < total ? j : total - 1)];
         key[i] = j < total ? c : 0ull;
     }
-    for (int i = threadIdx.x; i < k2; i += 256) sk[i] = 0ull;
+    sk[threadIdx.x] = 0ull;
+    for (int i = threadIdx.x; i < kFew; i += 256) few[i] = 0ull;
+    if (threadIdx.x == 0) n_few = 0;
+    unsigned long long least = 0ull;   // complemented: the maximum's
+    if (full > 0) {
+        const int at = (k + full - 1) / full - 1;
+        for (int q = lane; q < full; q += 64) {
+            const unsigned long long c = ~cand[m * total + (int64_t)q * k + at];
+            least = c > least ? c : least;
+        }
+        least = ~wave_max(least);
+    }
     __syncthreads();
-    radix_top<KPT>(key, k, sk);
-    bitonic_desc(sk, k2);
+    int mine = 0;   // the wave's
+#pragma unroll
+    for (int i = 0; i < KPT; i++) mine += __popcll(__ballot(key[i] != 0ull && key[i] >= least));
+    int at = 0;
+    if (lane == 0) at = atomicAdd(&n_few, mine);
+    at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+    for (int i = 0; i < KPT; i++) {
+        const bool in = key[i] != 0ull && key[i] >= least;
+        const unsigned long long who = __ballot(in);
+        const int to = at + __popcll(who & ((1ull << lane) - 1ull));
+        if (in && to < kFew) few[to] = key[i];
+        at += __popcll(who);
+    }
+    __syncthreads();
+    int n_in = n_few;
+    if (n_in > kFew) {   // block-uniform
+        radix_top<KPT>(key, k, few);
+        if (threadIdx.x == 0) few[k] = 0ull;   // (k <= kMaxTopK < kFew)
+        n_in = k;
+        __syncthreads();
+    }
+    for (int i = threadIdx.x; i < n_in; i += 256) {
+        const unsigned long long own = few[i];
+        const int to = rank_of(own, few, n_in);
+        if (own != 0ull && to < k) sk[to] = own;
+    }
+    __syncthreads();
     if (threadIdx.x >= 64) return;
-    const int lane = threadIdx.x;
     constexpr int J = kMaxTopK / 64;
     int n = 0;
     float e[J];
@@ -216,40 +258,40 @@ __global__ __launch_bounds__(256) void topk_merge_sample_kernel(const unsigned l
         if (lane == 0) ids[m] = -1;
         return;
     }
-    auto at = [&](int i) {   // candidate i's weight (i uniform)
-        float v = e[0];
+    float upto[J], c = 0.0f;   // sums of the weights up to a candidate's, in order
 #pragma unroll
-        for (int j = 1; j < J; j++) v = i >= 64 * j ? e[j] : v;
+    for (int j = 0; j < J; j++) {
+        upto[j] = 0.0f;
+#pragma unroll 8
+        for (int l = 0; l < min(64, n - 64 * j); l++) {
+            c += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, e[j]), l));
+            if (lane == l) upto[j] = c;
+        }
+    }
+    auto sum_to = [&](int i) {   // i uniform
+        float v = upto[0];
+#pragma unroll
+        for (int j = 1; j < J; j++) v = i >= 64 * j ? upto[j] : v;
         return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), i & 63));
     };
-    float sum = 0.0f;
-    for (int i = 0; i < n; i++) sum += at(i);
-    if (top_p > 0.0f && top_p < 1.0f) {
-        float cum = 0.0f;
-        int keep = n;
-        for (int i = 0; i < n; i++) {
-            cum += at(i);
-            if (cum >= top_p * sum) { keep = i + 1; break; }
+    auto first = [&](auto holds, int none) {   // the first of n candidates whose running sum holds
+        int f = none;
+#pragma unroll
+        for (int j = J - 1; j >= 0; j--) {
+            const unsigned long long b = __ballot(64 * j + lane < n && holds(upto[j]));
+            if (b) f = 64 * j + __ffsll(b) - 1;
         }
-        n = keep;
-        sum = 0.0f;
-        for (int i = 0; i < n; i++) sum += at(i);
+        return f;
+    };
+    float sum = sum_to(n - 1);
+    if (top_p > 0.0f && top_p < 1.0f) {
+        n = first([&](float s) { return s >= top_p * sum; }, n - 1) + 1;
+        sum = sum_to(n - 1);
     }
     const uint64_t sd = seed + (step ? (uint64_t)(int64_t)step[m] : 0ull);
-    float u = xorwow_uniform_first(sd) * sum;
-    float cum = 0.0f;
-    int picked = n - 1;
-    for (int i = 0; i < n; i++) {
-        cum += at(i);
-        if (u <= cum) { picked = i; break; }
-    }
+    const float u = xorwow_uniform_first(sd) * sum;
+    const int picked = first([&](float s) { return u <= s; }, n - 1);
     if (lane == 0) ids[m] = key_idx(sk[picked]);
-}
-
-static int pow2_at_least(int x) {
-    int p = 1;
-    while (p < x) p <<= 1;
-    return p;
 }
 
 }  // namespace qie
@@ -299,7 +341,7 @@ int qie_sample(const void* logits, int64_t M, int64_t V, int64_t ld, const qie_s
     QIE_REQUIRE(total <= 64 * 256, "qie_sample: top-k of %d over %lld logits leaves %d candidates, more than %d", k, (long long)V, total, 64 * 256);
     const auto fn = total <= 8 * 256 ? topk_merge_sample_kernel<8> : total <= 40 * 256 ? topk_merge_sample_kernel<40>
                                                                                        : topk_merge_sample_kernel<64>;
-    hipLaunchKernelGGL(fn, dim3((unsigned)M), dim3(256), 0, st, cand, nb, k, std::max(2, pow2_at_least(k)),
+    hipLaunchKernelGGL(fn, dim3((unsigned)M), dim3(256), 0, st, cand, nb, (int)(V / kSlice), k,
                        s->temperature, s->top_p, (uint64_t)s->seed, step_dev, out_ids);
     QIE_LAUNCH_CHECK();
     return 0;

@@ -43,3 +43,16 @@ def test_masked_rows(qlib, oracle, V):
     assert sampled(qlib, lg, 50, 0.9, 0.95, 7, [0, 1, 2, 3]) == [oracle.sample(lg[m], 50, 0.9, 0.95, 7 + m) for m in range(4)]
     lg = np.full((1, V), 0xFF80, np.uint16)  # nothing to choose from
     assert sampled(qlib, lg, 50, 0.9, 0.95, 7, [0]) == [-1]
+
+
+@pytest.mark.parametrize("V,k", [(8192, 2), (20000, 50), (152064, 50), (152064, 256)])
+def test_where_the_best_are(qlib, oracle, V, k):
+    """Few candidates over the slices' bound and more than are put in order at once: the best spread out, at the end, in one slice, in every 4th."""
+    r = np.random.default_rng(V * k)
+    f = (r.standard_normal((4, V)) * 2).astype(np.float32)
+    f[1] = np.arange(V) * np.float32(30.0 / V)
+    f[2, 4096:8192] += 20.0
+    f[3, (np.arange(V) // 4096) % 4 != 0] -= 20.0
+    lg = oracle.f32_to_bf16(f)
+    for T, tp, seed in ((0.7, 0.9, 3), (2.5, 1.0, 4)):
+        assert sampled(qlib, lg, k, T, tp, seed, [0, 1, 2, 3]) == [oracle.sample(lg[m], k, T, tp, seed + m) for m in range(4)]
