@@ -1232,10 +1232,27 @@ static int enq_mixer_out(qie_batch* b, int i, int T) {
     return dense(b, s->ov, HV, L.wo, s->mix, m->a.width, T, m->a.width, (int)HV, s->ov_bf);
 }
 
+static int gate_of(const qie_layer_desc& d) {
+    return d.ff_act == QIE_ACT_GELU_TANH_GATED ? 1 : d.ff_act == QIE_ACT_CLAMPED_GATED ? 2 : d.ff_act == QIE_ACT_RELU_GATED ? 3 : 0;
+}
+
+// A feed-forward's gate and up product with the activation behind it in one launch, and the `plain` fp32 columns of proj before them, for the
+// few rows of a decode step: *done, the bf16 activations are where enq_ff's output product (or the layer's) reads them.
+static int gated_in(qie_batch* b, const LayerDev& L, const uint16_t* y_bf, const void* w, int plain, int T, hipStream_t st, bool* done) {
+    const LayeredModel* m = b->e->lm;
+    const qie_layer_desc& d = L.d;
+    LayeredBatch* s = b->lb;
+    *done = false;
+    const bool cat = L.cat_ff >= 0;
+    if (T > 16 || !y_bf || !s->ov_bf || !s->act_bf || d.ff_kind != QIE_FF_DENSE || d.ff_act == QIE_ACT_XIELU || !image_only(m, cat ? L.n_cat : d.ff)) return 0;
+    lay::GatedP p{y_bf, w, T, m->a.width, plain, d.ff, s->proj, L.n_in, cat ? s->ov_bf + L.cat_ff : s->act_bf, cat ? L.n_cat : d.ff, gate_of(d), d.ff_limit};
+    return dec_bf16_gated(p, st, done);
+}
+
 // feed-forward of layer i on its normed rows (s->y, in parallel blocks s->y2) -> ffo; where the layer's output product
 // takes the activations as well (cat_ff), they go beside the mixer's columns and the product is left to it
-// later: where the experts' sum may be left to (ffo is then not written)
-static int enq_ff(qie_batch* b, int i, int T, hipStream_t on = nullptr, lay::ExpertSum* later = nullptr) {
+// later: where the experts' sum may be left to (ffo is then not written); acted: the input product has made the activations (gated_in)
+static int enq_ff(qie_batch* b, int i, int T, hipStream_t on = nullptr, lay::ExpertSum* later = nullptr, bool acted = false) {
     const qie_engine* e = b->e;
     const LayeredModel* m = e->lm;
     const LayerDev& L = m->L[i];
@@ -1253,13 +1270,17 @@ static int enq_ff(qie_batch* b, int i, int T, hipStream_t on = nullptr, lay::Exp
     }
     if (d.ff_kind == QIE_FF_DENSE) {
         // one norm for both branches: the input product has made the gate and up columns as well
-        if (L.col_ff < 0) QIE_TRY(dense(b, y, W, L.w_gu, s->gu, 2 * ff, T, 2 * ff, W, y_bf, st));
-        const float* gu = L.col_ff < 0 ? s->gu : s->proj + L.col_ff;
-        const int64_t ld_gu = L.col_ff < 0 ? 2 * ff : L.n_in;
-        const int act = d.ff_act == QIE_ACT_GELU_TANH_GATED ? 1 : d.ff_act == QIE_ACT_CLAMPED_GATED ? 2 : d.ff_act == QIE_ACT_RELU_GATED ? 3 : 0;
-        if (L.cat_ff >= 0)
-            return lay::silu_mul(gu, image_only(m, L.n_cat) ? nullptr : s->ov + L.cat_ff, s->ov_bf ? s->ov_bf + L.cat_ff : nullptr, T, ff, st, act, d.ff_limit, L.n_cat, ld_gu);
-        QIE_TRY(lay::silu_mul(gu, image_only(m, ff) ? nullptr : s->act, s->act_bf, T, ff, st, act, d.ff_limit, 0, ld_gu));
+        if (!acted && L.col_ff < 0) QIE_TRY(gated_in(b, L, y_bf, L.w_gu, 0, T, st, &acted));
+        if (!acted) {
+            if (L.col_ff < 0) QIE_TRY(dense(b, y, W, L.w_gu, s->gu, 2 * ff, T, 2 * ff, W, y_bf, st));
+            const float* gu = L.col_ff < 0 ? s->gu : s->proj + L.col_ff;
+            const int64_t ld_gu = L.col_ff < 0 ? 2 * ff : L.n_in;
+            const bool cat = L.cat_ff >= 0;
+            float* a = image_only(m, cat ? L.n_cat : ff) ? nullptr : cat ? s->ov + L.cat_ff : s->act;
+            uint16_t* a_bf = !cat ? s->act_bf : s->ov_bf ? s->ov_bf + L.cat_ff : nullptr;
+            QIE_TRY(lay::silu_mul(gu, a, a_bf, T, ff, st, gate_of(d), d.ff_limit, cat ? L.n_cat : 0, ld_gu));
+        }
+        if (L.cat_ff >= 0) return 0;
         return dense(b, s->act, ff, L.w_down, s->ffo, W, T, W, ff, s->act_bf, st);
     }
     const int E = d.experts, top = d.top, n = T * top;
@@ -1383,11 +1404,13 @@ static int enq_in(qie_batch* b, int r, int T) {
     const LayeredModel* m = b->e->lm;
     const LayerDev& L = m->L[m->runs[r].layer];
     LayeredBatch* s = b->lb;
-    QIE_TRY(enq_proj(b, r, T));
+    bool acted = false;
+    if (L.col_ff >= 0) QIE_TRY(gated_in(b, L, s->y_bf, L.w_in, L.col_ff, T, b->e->stream, &acted));
+    if (!acted) QIE_TRY(enq_proj(b, r, T));
     if (L.col_ff < 0) return 0;
     s->ff_branch = T > kBranchRows;
     if (s->ff_branch) QIE_TRY(branch_fork(b, 0));
-    return enq_ff(b, m->runs[r].layer, T, s->ff_branch ? s->side[0] : nullptr);
+    return enq_ff(b, m->runs[r].layer, T, s->ff_branch ? s->side[0] : nullptr, nullptr, acted);
 }
 
 static int enq_gqa_post(qie_batch* b, int r, int T) {

@@ -186,7 +186,6 @@ __global__ __launch_bounds__(256) void linear_skinny_kernel(LinearP p) {
 // summed.  linear_skinny_kernel waits for memory at each 512 k and for each row.  GATED: a wave has column n of the gate and of the up
 // weights (N rows further on) and stores gated_act of the two.  us, 6 rows over 8 experts of fp32 weights (width 1,024, 704 inner): gate and up with
 // their gating launch 13.2 + 4.3 -> 7.8, down 10.1 -> 4.7.  Bits as there.
-__device__ __forceinline__ float gated_act(float g, float u, int act, float limit);
 template <typename TW, bool GATED>
 __global__ __launch_bounds__(256) void linear_short_kernel(LinearP p) {
     const int z = blockIdx.z, lane = threadIdx.x & 63;
@@ -683,17 +682,7 @@ int depth_mix(const float* stack, int64_t stride, const float* a, int n, float* 
 }
 
 // ------------------------------------------------------------------ gated activation
-// a[m, j] = silu(gu[m, j]) * gu[m, ff + j]
-// (act 1: the tanh form of gelu instead of silu, gelu(g) = g / 2 (1 + tanh(sqrt(2 / pi) (g + 0.044715 g^3)));
-// act 2: g sigmoid(1.702 g) (u + 1) with the gate cut at limit and u clamped to +-limit; act 3: max(g, 0) u)
-__device__ __forceinline__ float gated_act(float g, float u, int act, float limit) {
-    if (act == 3) return fmaxf(g, 0.f) * u;
-    if (act == 2) {
-        const float gc = fminf(g, limit), uc = fminf(fmaxf(u, -limit), limit);
-        return gc / (1.0f + expf(-1.702f * gc)) * (uc + 1.0f);
-    }
-    return (act == 1 ? 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g))) : g / (1.0f + expf(-g))) * u;
-}
+// a[m, j] = gated_act(gu[m, j], gu[m, ff + j])
 // V consecutive columns per thread (V = 4: ff and ld_a multiples of 4)
 template <int V>
 __global__ __launch_bounds__(256) void silu_mul_kernel(const float* gu, float* a, uint16_t* a_bf, int ff, uint32_t n, int act, float limit,

@@ -586,10 +586,34 @@ int postnorm_add(const float* x, const float* v, float* y, uint16_t* y_bf, int T
 int final_rows(const float* x, const int32_t* rows, float* out, uint16_t* out_bf, int n, int W, float gain, const float* w1p,
                float eps, hipStream_t st, float w_one = 1.0f);
 int depth_mix(const float* stack, int64_t stride, const float* a, int n, float* x, uint16_t* x_bf, int64_t count, hipStream_t st);
+// silu(g) u
+// (act 1: the tanh form of gelu instead of silu, gelu(g) = g / 2 (1 + tanh(sqrt(2 / pi) (g + 0.044715 g^3)));
+// act 2: g sigmoid(1.702 g) (u + 1) with the gate cut at limit and u clamped to +-limit; act 3: max(g, 0) u)
+__device__ __forceinline__ float gated_act(float g, float u, int act, float limit) {
+    if (act == 3) return fmaxf(g, 0.f) * u;
+    if (act == 2) {
+        const float gc = fminf(g, limit), uc = fminf(fmaxf(u, -limit), limit);
+        return gc / (1.0f + expf(-1.702f * gc)) * (uc + 1.0f);
+    }
+    return (act == 1 ? 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g))) : g / (1.0f + expf(-g))) * u;
+}
 // a[m * ld_a + j] = act(gu[m, j]) * gu[m, ff + j]; act 0: silu, 1: the tanh form of gelu, 2: g sigmoid(1.702 g) (u + 1)
 // with g = min(gu[m, j], limit), u = gu[m, ff + j] clamped to +-limit, 3: relu; ld_a 0: ff; ld_gu (rows of gu) 0: 2 ff
 int silu_mul(const float* gu, float* a, uint16_t* a_bf, int64_t M, int ff, hipStream_t st, int act = 0, float limit = 0.f,
              int64_t ld_a = 0, int64_t ld_gu = 0);
+// The product of a feed-forward's gate and up rows with the activation in its epilogue, for a few bf16 rows: h[m, j] = bf16(gated_act(x[m] .
+// gate_j, x[m] . up_j)); rows [0, plain) of the same weights go to y in fp32.  gate_j is row plain + j of w, up_j row plain + ff + j.
+struct GatedP {
+    const uint16_t* x;   // [M, K]
+    const void* w;       // [plain + 2 ff, K] bf16
+    int M, K, plain, ff;
+    float* y;
+    int64_t ldy;
+    uint16_t* h;
+    int64_t ldh;
+    int act;
+    float limit;
+};
 // x = c tanh(x / c) in place, n elements
 int softcap(float* x, int64_t n, float c, hipStream_t st);
 // a = ap u^2 + u / 2 where u > 0, else aq (exp(u) - 1 - u) + u / 2; n elements
@@ -619,4 +643,6 @@ int rows_to_bf16_strided(const float* x, int64_t ldx, uint16_t* y, int64_t ldy, 
 int bf16_to_f32(const uint16_t* x, float* y, int64_t n, hipStream_t st);
 
 }  // namespace lay
+
+int dec_bf16_gated(const lay::GatedP& p, hipStream_t st, bool* done);   // k_decode_bf16.hip
 }  // namespace qie

@@ -34,7 +34,7 @@ def main():
         variants += [("attn", 5, {})]
         for sp in ("8", "16", "24", "48"):
             variants.append(("attn", 5, {"QIE_DEC_SPLITS": sp}))
-        variants += [("attn", 5, {"QIE_DEC_DBG": d}) for d in ("1", "8", "16", "64")]
+        variants += [("attn", 5, {"QIE_DEC_DBG": d}) for d in ("1", "64")]
     if "gemv" in sets:
         for which in (0, 1, 2, 3, 4):
             variants.append((NAMES[which], which, {}))
