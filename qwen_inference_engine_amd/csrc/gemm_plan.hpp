@@ -144,10 +144,9 @@ constexpr int BK = 64;
 
 // Times of a tile, us, fitted to the projections of Qwen2-0.5B / 1.5B / 7B, Qwen3-14B and of 4,096 columns at 17 to 2,300 rows (474
 // shapes, each measured on every tile with 1 to 8 segments; what the rule below picks is 1.6 % over the best of all of them on the
-// average and 17 % at most, with the constants fitted to 168 shapes before the kernel's ring and tickets changed 2.3 %).  Of 960
-// other shapes 156 went to another tile and took 0.97 of their time on the average: 1,536 -> 2 x 8,960 gate / up at 184 rows
-// 28.8 -> 24.1 us, 3,584 -> 4,608 at 489 36.4 -> 31.1, 17,408 -> 5,120 at 133 61.3 -> 53.5; the worst, 3,584 -> 3,584 at 214, 17.0
-// -> 18.6:
+// average and 17 % at most, with the constants fitted to 168 shapes before the kernel's ring and tickets changed 2.3 %).  Of
+// 80 other shapes that went to another tile: 0.95 of their time on the average, 1.01 at most: 1,536 -> 2 x 8,960 gate / up at 184 rows 28.8 -> 24.1 us,
+// 3,584 -> 4,608 at 489 36.4 -> 31.1, 17,408 -> 5,120 at 133 61.3 -> 53.5; one known to lose is 3,584 -> 3,584 at 205 to 235 rows, 17.0 -> 18.6 at 214:
 // up to one workgroup a CU a1 + s1 per k-tile, more a2 + (rounds of the chip) * (f2 + s2 per k-tile).  A k-tile costs what its
 // lines take through one CU (about 50 GB/s where they come from HBM or another die, 120 GB/s from L2), not its matrix work,
 // which is why the tall tiles win as soon as the rows fill them.  The constants are an MI355X's, whole (256 CUs): `cus` moves
@@ -164,6 +163,16 @@ constexpr Tile TILES[] = {
     {320, 64, 3, 1, 4.68f, .711f, 5.22f, 2.82f, .769f}, {320, 128, 2, 1, 8.f, 1.041f, 12.67f, .28f, 1.196f},
 };
 constexpr int N_TILES = sizeof(TILES) / sizeof(TILES[0]);
+// Above the rows that were fitted the same tiles keep the times of an earlier fit: there the new ones took 0.98 on the average of 94 products but
+// 1.05 to 1.09 of Qwen2-7B down's at 6,784 rows (789 us -> 857), Qwen3-14B down's at 4,864 and Qwen2-0.5B QKV's at 4,384.
+constexpr int64_t FITTED_ROWS = 2304;
+constexpr Tile TALL_TILES[] = {
+    {64, 64, 5, 2, 3.2f, .285f, 5.f, .7f, .487f},   {64, 128, 3, 2, 2.6f, .475f, 5.4f, 1.1f, .74f},
+    {128, 64, 3, 2, 3.3f, .43f, 4.7f, 1.8f, .70f},  {128, 128, 4, 1, 5.9f, .54f, 7.5f, 3.9f, .575f},
+    {192, 128, 4, 1, 8.f, .65f, 5.f, 6.f, .72f},    {256, 128, 3, 1, 9.9f, .90f, 12.f, 2.5f, 1.037f},
+    {320, 64, 3, 1, 6.9f, .70f, 6.5f, 3.f, .787f},  {320, 128, 2, 1, 9.4f, 1.11f, 14.f, 2.f, 1.2f},
+};
+static_assert(sizeof(TALL_TILES) == sizeof(TILES), "one tile, one number");
 // Tiles of 160 columns, numbered on from TILES: where the columns of 128-column tiles start a round of the chip that they hardly fill
 // (37,888 columns: 296 tiles, 237 of these), and so many rows of the workgroups' own (weights) that a tile of fewer columns loads more
 // for the same outputs.  Whole only.
@@ -172,6 +181,11 @@ constexpr Tile WIDE[] = {
     {256, 160, 3, 1, 4.85f, 1.139f, 0.f, 8.74f, .922f}, {320, 160, 2, 1, 6.26f, 1.498f, 0.f, 10.73f, 1.137f},
 };
 constexpr int N_WIDE = sizeof(WIDE) / sizeof(WIDE[0]);
+constexpr Tile TALL_WIDE[] = {
+    {128, 160, 4, 1, 3.f, 1.f, 11.7f, 0.f, .69f}, {192, 160, 3, 1, 6.6f, 1.1f, 7.1f, 6.3f, .825f},
+    {256, 160, 3, 1, 8.8f, 1.29f, 0.f, 10.f, 1.f}, {320, 160, 2, 1, 9.6f, 1.56f, 0.f, 13.f, 1.17f},
+};
+static_assert(sizeof(TALL_WIDE) == sizeof(WIDE), "one tile, one number");
 inline const Tile& shape(int tile) { return tile < N_TILES ? TILES[tile] : WIDE[tile - N_TILES]; }
 
 struct Plan {
@@ -192,7 +206,7 @@ inline Plan plan(int64_t M, int64_t cols, int64_t K, int64_t cus) {
     const int nk = (int)(K / BK);
     const float floor_us = (float)cols * K * 2 / 5.3e6f + 4.f;   // the weights at the rate they stream here
     for (int c = 0; c < N_TILES; c++) {
-        const Tile& t = TILES[c];
+        const Tile& t = (M > FITTED_ROWS ? TALL_TILES : TILES)[c];
         const int64_t n_mt = (M + t.bm - 1) / t.bm, n_nt = (cols + t.bn - 1) / t.bn, tiles = n_mt * n_nt;
         if (tiles > (1 << 22)) continue;   // (of 32-bit workgroup counts)
         const float room = (float)(cus * t.per_cu);
@@ -204,7 +218,7 @@ inline Plan plan(int64_t M, int64_t cols, int64_t K, int64_t cus) {
             } else {
                 if (cut == 0) break;
                 const float len = (float)((nk + s - 1) / s);
-                us = whole / room * (t.f2 + nk * t.s2) + 2.82f * s * (t.bm * t.bn) / 16384.f + .74f;
+                us = whole / room * (t.f2 + nk * t.s2) + (M > FITTED_ROWS ? 3.f * s * (t.bm * t.bn) / 16384.f + 1.f : 2.82f * s * (t.bm * t.bn) / 16384.f + .74f);
                 us += cut <= cus ? t.a1 + len * t.s1 : t.a2 + rounds(cut / room) * (t.f2 + len * t.s2);
             }
             us = std::max(us, floor_us);
@@ -225,7 +239,7 @@ inline Plan plan_wide(int64_t M, int64_t cols, int64_t K, int64_t cus) {
     const int nk = (int)(K / BK);
     const float floor_us = (float)cols * K * 2 / 5.3e6f + 4.f;   // as in plan()
     for (int c = 0; c < N_WIDE; c++) {
-        const Tile& t = WIDE[c];
+        const Tile& t = (M > FITTED_ROWS ? TALL_WIDE : WIDE)[c];
         const int64_t n_mt = (M + t.bm - 1) / t.bm, n_nt = (cols + t.bn - 1) / t.bn, tiles = n_mt * n_nt;
         const int64_t most = t.bm < 320 ? 2 : M >= 2048 && M * K * 2 <= 80000000 ? 4 : 1;   // rounds
         if (tiles > most * cus) continue;
@@ -249,14 +263,17 @@ inline Plan best(int64_t M, int64_t cols, int64_t K, int64_t cus) {
 inline int64_t columns_ahead(int64_t M, int64_t cols, int64_t K, int64_t cus) {
     const int64_t n_mt = (M + 255) / 256, n_nt = (cols + 255) / 256;
     if (K % BK != 0 || M < 256 || n_mt * n_nt <= cus) return 0;
-    const float whole = std::min(g8p::us(M, cols, K, cus), best(M, cols, K, cus).us);
-    float least = .97f * whole;   // (of 42 shapes the sum of the two fits was 5 % over the measured ratio on the average, 8 % at most)
+    // (fitted rows: the tiles' times are 3 to 10 % short of the measured beside the 256x256 kernel's; without 1.06 of them Qwen3-14B gate / up at 2,048
+    // rows would leave 10,240 columns, 573 us, and not 2,048, 563)
+    const float more = M > FITTED_ROWS ? 1.f : 1.06f;
+    const float whole = std::min(g8p::us(M, cols, K, cus), more * best(M, cols, K, cus).us);
+    float least = .97f * whole;
     int64_t ahead = 0;
     const int64_t full = n_mt * n_nt / cus;
     for (int64_t r = full; r >= 1 && r >= full - 1; r--) {
         const int64_t c = r * cus / n_mt * 256;
         if (c <= 0 || c >= cols) continue;
-        const float us = g8p::us(M, c, K, cus) + best(M, cols - c, K, cus).us;
+        const float us = g8p::us(M, c, K, cus) + more * best(M, cols - c, K, cus).us;
         if (us < least) {
             least = us;
             ahead = c;
