@@ -146,8 +146,8 @@ constexpr int BK = 64;
 // shapes, each measured on every tile with 1 to 8 segments; what the rule below picks is 1.6 % over the best of all of them on the
 // average and 17 % at most, with the constants fitted to 168 shapes before the kernel's ring and tickets changed 2.3 %).  Of
 // 80 other shapes that went to another tile: 0.95 of their time on the average, 1.01 at most: 1,536 -> 2 x 8,960 gate / up at 184 rows 28.8 -> 24.1 us,
-// 3,584 -> 4,608 at 489 36.4 -> 31.1, 17,408 -> 5,120 at 133 61.3 -> 53.5; one known to lose is 3,584 -> 3,584 at 205 to 235 rows, 17.0 -> 18.6 at 214:
-// up to one workgroup a CU a1 + s1 per k-tile, more a2 + (rounds of the chip) * (f2 + s2 per k-tile).  A k-tile costs what its
+// 3,584 -> 4,608 at 489 36.4 -> 31.1, 17,408 -> 5,120 at 133 61.3 -> 53.5; one known to lose is 3,584 -> 3,584 at 205 to 235 rows, 17.0 -> 18.6 at 214.
+// Up to one workgroup a CU a1 + s1 per k-tile, more a2 + (rounds of the chip) * (f2 + s2 per k-tile).  A k-tile costs what its
 // lines take through one CU (about 50 GB/s where they come from HBM or another die, 120 GB/s from L2), not its matrix work,
 // which is why the tall tiles win as soon as the rows fill them.  The constants are an MI355X's, whole (256 CUs): `cus` moves
 // the rounds, but the slopes hold the bandwidth that 256 CUs share, so a part with fewer would still get a correct plan, not
