@@ -157,9 +157,11 @@ int qie_attention(const void* q, int64_t M, const int32_t* pos, int32_t rows_per
  * qkv rows [B][(nq + 2 nkv) hd] straight from the QKV projection; applies qk-norm
  * (q_norm/k_norm non-NULL) and RoPE at pos[m] to q and to the new k, appends the
  * new K/V row of sequence m at pos[m], and attends over [0, pos[m]].  Splits of 128
- * keys are combined in-launch by the last-arriving workgroup.  ws must hold
- * qie_attention_decode_workspace_bytes() and be ZEROED once before first use (it
- * is left zeroed by every call).
+ * keys are combined in-launch by the last-arriving waves.  ws must hold
+ * qie_attention_decode_workspace_bytes() and be ZEROED once before first use; every
+ * call leaves the part that has to be zero so.  Calls one after the other may share it,
+ * whatever their max_ctx, head_dim, n_heads and B, as long as it holds the largest of them and
+ * ceil(B * n_kv_heads / 1024) is the same for all.
  * numerics may carry QIE_ATTN_PREROPED (REF numerics, no qk-norm only): q and the new
  * k in qkv are already rotated (the engine's decode QKV projection applies RoPE in its
  * epilogue), so only the K/V append and the attention run here. */

@@ -547,7 +547,9 @@ static int attn_nsplit(int64_t M, int32_t max_ctx) {
 static thread_local const float* g_rope_cur = nullptr;
 void set_decode_rope_cur(const float* rc) { g_rope_cur = rc; }
 
-static int64_t dec_counter_bytes(int64_t B, int32_t nkv) { return B * nkv * (kDecMWaves * kDecMTicket * 4); }
+// Tickets at the front of the workspace, the splits' results behind them.  In steps of 1,024 pairs of row and kv head (512 KB): calls of fewer rows on a
+// workspace that served more keep its results where they were, not in the other rows' tickets.
+static int64_t dec_counter_bytes(int64_t B, int32_t nkv) { return (B * nkv + 1023) / 1024 * 1024 * (kDecMWaves * kDecMTicket * 4); }
 
 static int fill_dec_params(DecodeAttnParams& a, const void* qkv, int64_t B, const int32_t* pos, const void* q_norm,
                            const void* k_norm, const float* rope_cos, const float* rope_sin, int32_t n_heads,

@@ -66,3 +66,33 @@ def test_contexts_at_the_edges(qlib, hd, nq, nkv, paged, maxc, ctxs):
             want = attention(x[:nq], k, v, nq // nkv, hd)
             # one bf16 rounding of the result; sums of ctx products of 24-bit probabilities (2^-22 of the largest value)
             assert (np.abs(got[m] - want) <= 2.0 ** -8 * np.abs(want) + 2.0 ** -20 * np.abs(v).max()).all(), (ctx, np.abs(got[m] - want).max())
+
+
+@pytest.mark.parametrize("hd,nq,nkv,maxc", [(128, 28, 4, 1024), (64, 14, 2, 4352)])
+def test_calls_of_fewer_rows_share_a_workspace(qlib, hd, nq, nkv, maxc):
+    """8, 4, 1 and again 8 rows: the results of fewer rows' splits do not lie in the tickets of the others."""
+    rng = np.random.default_rng(hd)
+    B, ctxs = 8, [1024, 257, 700, 513, 900, 384, 1000, 640]
+    kc, vc = (bf16_words(rng, (B, 1, nkv, maxc, hd)) for _ in range(2))
+    dk, dv = G.dev(kc), G.dev(vc)
+    cache = _lib.KvCacheC()
+    cache.k, cache.v, cache.seq_stride, cache.n_layers, cache.n_kv_heads, cache.head_dim, cache.max_ctx = G.p(dk), G.p(dv), nkv * maxc * hd, 1, nkv, hd, maxc
+    ws, one = G.zeros_bytes(qlib.qie_attention_decode_workspace_bytes(B, nq, nkv, hd, maxc)), G.dev(np.ones((maxc, hd // 2), np.float32))
+    qkv = bf16_words(rng, (B, (nq + 2 * nkv) * hd))
+    dq, dp = G.dev(qkv), G.dev(np.array(ctxs, np.int32) - 1)
+    first = None
+    for rows in (8, 4, 1, 8, 3, 8):
+        out = G.zeros_bf16(B, nq * hd)
+        G.check(qlib.qie_attention_decode(G.p(dq), rows, G.p(dp), None, None, G.p(one), G.p(one), nq, C.byref(cache), 0, 1e-6, PREROPED, G.p(out),
+                                          G.p(ws), None))
+        got = G.bf(G.host_bf16(out)).reshape(B, nq, hd)
+        first = got if first is None else first
+        # (8 rows may have other splits than fewer: the same sums in another order, one bf16 rounding of each)
+        assert (np.abs(got[:rows] - first[:rows]) <= 2.0 ** -7 * np.abs(first[:rows]) + 2.0 ** -20 * 4.0).all(), rows
+        assert rows < 8 or np.array_equal(got, first)
+    for m, ctx in enumerate(ctxs):
+        x = G.bf(qkv[m]).astype(np.float64).reshape(-1, hd)
+        k, v = (G.bf(c[m, 0, :, :ctx]).astype(np.float64) for c in (kc, vc))
+        k[:, -1], v[:, -1] = x[nq:nq + nkv], x[nq + nkv:]
+        want = attention(x[:nq], k, v, nq // nkv, hd)
+        assert (np.abs(first[m] - want) <= 2.0 ** -8 * np.abs(want) + 2.0 ** -20 * np.abs(v).max()).all(), ctx
