@@ -188,6 +188,10 @@ constexpr Tile TALL_WIDE[] = {
 static_assert(sizeof(TALL_WIDE) == sizeof(WIDE), "one tile, one number");
 inline const Tile& shape(int tile) { return tile < N_TILES ? TILES[tile] : WIDE[tile - N_TILES]; }
 
+// Row strides (elements of x, and of y in up to 4 bytes) whose offsets inside a tile of 320 rows fit the kernel's 32 bits: unsigned for x, signed for
+// y, whose columns past the end lie at 2^31.
+inline bool strides_fit(int64_t ldx, int64_t ldy) { return ldx <= 1 << 22 && ldy <= 1 << 20; }
+
 struct Plan {
     int tile, whole, splitk, n_mt, n_nt;
     float us;

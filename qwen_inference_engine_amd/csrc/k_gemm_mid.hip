@@ -467,7 +467,7 @@ static int run_mid(int epi, const GemmParams& p, const mid::Plan& pl, const QkvT
 int gemm_mid(const qie_linear_args* a, const GemmParams& p, const QkvTail* tail, hipStream_t st, bool* launched) {
     *launched = false;
     const mid::Plan pl = mid::choose(a->M, a->epilogue == QIE_EPI_SWIGLU ? 2 * a->N : a->N, a->K, device_cu_count());
-    if (pl.tile < 0 || a->ldy > 1 << 20) return 0;   // (a tile of C by 32-bit offsets)
+    if (pl.tile < 0 || !mid::strides_fit(a->ldx, a->ldy)) return 0;
     *launched = true;
     return run_mid(a->epilogue, p, pl, tail, st);
 }

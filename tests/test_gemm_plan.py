@@ -14,7 +14,7 @@ DRIVER = r"""
 #include "gemm_plan.hpp"
 #include <cstdio>
 #include <vector>
-// "m M columns K cus": plan of k_gemm_mid.hip; "f M N K batch grouped cus": k_linear_f32.hip; "t M N K groups off[0] .. off[groups]": its row tiles' indices
+// "m M columns K cus": plan of k_gemm_mid.hip; "s ldx ldy": whether it takes such rows; "f M N K batch grouped cus": k_linear_f32.hip; "t M N K groups off[0] .. off[groups]": its row tiles' indices
 int main() {
     char op;
     while (std::scanf(" %c", &op) == 1) {
@@ -23,6 +23,9 @@ int main() {
             if (std::scanf("%ld %ld %ld %ld", &M, &N, &K, &cus) != 4) return 2;
             const qie::mid::Plan p = qie::mid::plan(M, N, K, cus);
             std::printf("%d %d %d %d\n", p.tile, p.whole, p.splitk, p.n_mt * p.n_nt);
+        } else if (op == 's') {
+            if (std::scanf("%ld %ld", &M, &N) != 2) return 2;
+            std::printf("%d\n", qie::mid::strides_fit(M, N) ? 1 : 0);
         } else if (op == 'f') {
             if (std::scanf("%ld %ld %ld %ld %ld %ld", &M, &N, &K, &batch, &x, &cus) != 6) return 2;
             const qie::lf::Plan p = qie::lf::plan(M, N, K, batch, x != 0, cus);
@@ -77,6 +80,17 @@ def test_gemm_mid_plans_are_sound(plan):
     for (M, N, K, cus), (tile, whole, splitk, tiles) in zip(cases, plan(["m %d %d %d %d" % c for c in cases])):
         assert tile in range(8) and 1 <= splitk <= min(12, K // 64) and 0 <= whole <= tiles
         assert whole == tiles if splitk == 1 else whole < tiles and whole % cus == 0
+
+
+def test_gemm_mid_offsets_fit(plan):
+    """Rows so far apart that a tile's offsets would wrap go to other kernels: 32 bits of bytes for x, 31 for y, of 4 bytes an element."""
+    rows, cols = 320, 160   # of the tallest and the widest tile
+    r = random.Random(6)
+    strides = [int(2 ** r.uniform(6, 40)) for _ in range(2000)] + [1 << 20, (1 << 20) + 8, 1 << 22, (1 << 22) + 8, 6731912, 6731920, 6731928, 7158280]
+    taken = [x for x, (t,) in zip(strides, plan([f"s {x} 64" for x in strides])) if t]
+    assert max(taken) >= 1 << 22 and all(((rows - 1) * x + 64) * 2 < 1 << 32 for x in taken)
+    taken = [y for y, (t,) in zip(strides, plan([f"s 64 {y}" for y in strides])) if t]
+    assert max(taken) >= 1 << 20 and all((rows * y + cols) * 4 < 1 << 31 for y in taken)
 
 
 # rows, weight rows, K, us of the best of the other tiles and the 256x256 kernel, of the 160-column tiles 8 to 11

@@ -123,3 +123,18 @@ def test_split_is_deterministic(qlib):
         linear(x, [w], [], M, K, N, y, _lib.QIE_EPI_F32)
         out.append(y.numpy())
     assert all(np.array_equal(out[0], o) for o in out[1:])
+
+
+@pytest.mark.parametrize("M,N,K", [(301, 1152, 896), (345, 45029, 768)])
+def test_rows_far_apart(qlib, M, N, K):
+    """Rows of x whose offsets inside a tile pass 32 bits (4.3 GB of 301 rows), of a product that k_gemm_mid.hip takes whole and of one that it takes
+    the last columns of: others do."""
+    ld = 7200000
+    x, w = bf16((M, K), 1.0, 1), bf16((N, K), K ** -0.5, 2)
+    far = G.DBuf((M - 1) * ld + K, np.uint16)
+    for m in range(M):
+        G.check(qlib.qie_memcpy_h2d(far.ptr + m * ld * 2, x[m].ctypes.data, K * 2))
+    y = G.zeros((M, N), np.float32)
+    linear(far, [G.dev(w)], [], M, K, N, y, _lib.QIE_EPI_F32, ldx=ld)
+    want, scale = products(x, w)
+    assert (np.abs(y.numpy() - want) <= 1e-5 * scale).all()
