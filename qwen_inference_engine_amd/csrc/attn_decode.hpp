@@ -471,6 +471,7 @@ __device__ __forceinline__ void attn_decode_mfma2_body(const DecodeAttnParams& a
                 const int c = lane + 64 * i;
                 *reinterpret_cast<uint4*>(vw + v_at(c / CPR, (c % CPR) * 8)) = vr[x][i];
             }
+            wave_lds_fence();   // (here: the reads below may go ahead of the exponentials)
             if (st + SETS < nstep) load_step(x, st + SETS);
             // scores s = dot / sqrt(hd) (self_attension.cu); those past the split's end are no keys (uniform)
             float e[8];
@@ -528,6 +529,7 @@ __device__ __forceinline__ void attn_decode_mfma2_body(const DecodeAttnParams& a
 #pragma unroll
             for (int dd = 0; dd < DG; dd++) oacc[d0 + dd] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl, vt[dd], oacc[d0 + dd], 0, 0, 0);
             }
+            wave_lds_fence();   // the next step's V, and O behind the last, go where these rows were
         };
         for (int st = 0; st < nstep; st += 2) {
             process(even, st);

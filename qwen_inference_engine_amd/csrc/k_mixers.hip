@@ -89,12 +89,6 @@ __device__ __forceinline__ int64_t page_base(const LatentCache& c, int slot, int
 // A wave per head and row (query, key, value heads alike; blockIdx.y spreads a row's heads over blocks when a step has
 // few rows), the head's coordinates staged in the wave's own LDS so that either pairing finds its partner: LDS
 // operations of one wave stay in order, so no block-wide barrier.
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 template <typename TC>
 __global__ __launch_bounds__(256) void gqa_post_kernel(GqaPostP p, int values) {
     extern __shared__ float sm[];

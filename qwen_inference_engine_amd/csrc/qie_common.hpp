@@ -188,6 +188,14 @@ __host__ __device__ __forceinline__ int64_t kv_run_off(const KvMap& k, int64_t l
     return lg * k.run * (int64_t)hd;
 }
 
+// Between a wave's writes to LDS of its own and its other lanes' reads of them, and between those reads and the next writes there: a wave's LDS
+// operations run in order, the compiler's need not.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ------------------------------------------------------ cross-lane reductions
 // __shfl_xor lowers to ds_bpermute_b32 (an LDS round trip, ~100 cycles); chains of
 // them serialised the decode attention.  These use DPP row ops (folded into the
