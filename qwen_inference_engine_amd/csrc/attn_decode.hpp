@@ -557,12 +557,13 @@ __device__ __forceinline__ void attn_decode_mfma2_body(const DecodeAttnParams& a
     float2 wml[kDecMWaves];
 #pragma unroll
     for (int w = 0; w < kDecMWaves; w++) wml[w] = ml_s[w][gi];
-    const float m_spl = fmaxf(fmaxf(wml[0].x, wml[1].x), fmaxf(wml[2].x, wml[3].x));   // finite: a split has a key
+    const float m_spl = fmaxf(fmaxf(wml[0].x, wml[1].x), fmaxf(wml[2].x, wml[3].x));
+    const float m_at = m_spl == -INFINITY ? 0.f : m_spl;   // (all keys of the split at -inf: its sum is 0, not NaN)
     float l_spl = 0.f;
     float4 o_spl = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (int w = 0; w < kDecMWaves; w++) {
-        const float c = __expf(wml[w].x - m_spl);   // 0 for a wave without keys
+        const float c = __expf(wml[w].x - m_at);   // 0 for a wave without keys
         const float4 o = reinterpret_cast<const float4*>(&v_s[w][0])[gi * (HD / 4) + d4];
         l_spl = fmaf(wml[w].y, c, l_spl);
         o_spl.x = fmaf(c, o.x, o_spl.x);
@@ -636,7 +637,8 @@ __device__ __forceinline__ void attn_decode_mfma2_body(const DecodeAttnParams& a
 #pragma unroll
             for (int jj = b; jj < b + 4; jj++) mb = fmaxf(mb, j0 + jj < nsplit ? w[jj].x : -INFINITY);
         }
-        const float sc = __expf(mx - mb);   // 0 on the first batch (mx = -inf, mb finite)
+        const float mu = mb == -INFINITY ? 0.f : mb;
+        const float sc = __expf(mx - mu);   // 0 on the first batch (mx = -inf)
         ls *= sc;
         acc.x *= sc; acc.y *= sc; acc.z *= sc; acc.w *= sc;
 #pragma unroll
@@ -644,7 +646,7 @@ __device__ __forceinline__ void attn_decode_mfma2_body(const DecodeAttnParams& a
             if (j0 + b >= nsplit) break;
 #pragma unroll
             for (int jj = b; jj < b + 4; jj++) {
-                const float c = j0 + jj < nsplit ? __expf(w[jj].x - mb) : 0.f;
+                const float c = j0 + jj < nsplit ? __expf(w[jj].x - mu) : 0.f;
                 ls = fmaf(w[jj].y, c, ls);
                 acc.x = fmaf(c, v[jj].x, acc.x);
                 acc.y = fmaf(c, v[jj].y, acc.y);

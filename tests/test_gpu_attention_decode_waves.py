@@ -96,3 +96,28 @@ def test_calls_of_fewer_rows_share_a_workspace(qlib, hd, nq, nkv, maxc):
         k[:, -1], v[:, -1] = x[nq:nq + nkv], x[nq + nkv:]
         want = attention(x[:nq], k, v, nq // nkv, hd)
         assert (np.abs(first[m] - want) <= 2.0 ** -8 * np.abs(want) + 2.0 ** -20 * np.abs(v).max()).all(), ctx
+
+
+@pytest.mark.parametrize("ctx,masked", [(200, (0, 64)), (700, (128, 384)), (700, (0, 640)), (4096, (0, 3328))])
+def test_keys_at_minus_infinity(qlib, ctx, masked):
+    """Scores of -inf (keys that hold it, against queries above zero there): a wave's keys, whole splits and every split of the merge's first round
+    trip count for nothing."""
+    hd, nq, nkv = 64, 14, 2
+    rng = np.random.default_rng(ctx)
+    kc, vc = (bf16_words(rng, (1, 1, nkv, ctx, hd)) for _ in range(2))
+    kc[..., masked[0]:masked[1], 0] = 0xFF80
+    qkv = bf16_words(rng, (1, (nq + 2 * nkv) * hd))
+    qkv.reshape(-1, hd)[:nq, 0] &= 0x7FFF
+    dk, dv = G.dev(kc), G.dev(vc)
+    cache = _lib.KvCacheC()
+    cache.k, cache.v, cache.seq_stride, cache.n_layers, cache.n_kv_heads, cache.head_dim, cache.max_ctx = G.p(dk), G.p(dv), nkv * ctx * hd, 1, nkv, hd, ctx
+    ws, out = G.zeros_bytes(qlib.qie_attention_decode_workspace_bytes(1, nq, nkv, hd, ctx)), G.zeros_bf16(1, nq * hd)
+    one = G.dev(np.ones((ctx, hd // 2), np.float32))
+    G.check(qlib.qie_attention_decode(G.p(G.dev(qkv)), 1, G.p(G.dev(np.array([ctx - 1], np.int32))), None, None, G.p(one), G.p(one), nq, C.byref(cache),
+                                      0, 1e-6, PREROPED, G.p(out), G.p(ws), None))
+    x = G.bf(qkv[0]).astype(np.float64).reshape(-1, hd)
+    k, v = (G.bf(c[0, 0]).astype(np.float64) for c in (kc, vc))
+    k[:, -1], v[:, -1] = x[nq:nq + nkv], x[nq + nkv:]
+    want = attention(x[:nq], k, v, nq // nkv, hd)
+    got = G.bf(G.host_bf16(out)).reshape(nq, hd)
+    assert (np.abs(got - want) <= 2.0 ** -8 * np.abs(want) + 2.0 ** -20 * np.abs(v).max()).all()
