@@ -306,7 +306,8 @@ __device__ __forceinline__ void attn_decode_mfma2_body(const DecodeAttnParams& a
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int fr = lane & 15, gq = lane >> 4;
     const int grp = tid / LPT, dl = tid % LPT;
-    const bool keyed = wave < kDecMWaves;
+    // (a constant where it is true of every wave: loads under a branch made the prologue wait for all of K, ahead of V)
+    const bool keyed = NWA == kDecMWaves || wave < kDecMWaves;
     const int QKVD = (a.nq + 2 * a.nkv) * HD;
     const uint16_t* row = a.qkv + m * (int64_t)QKVD;
     const int64_t head_off = kv_run_off(a.km, (int64_t)a.layer * a.nkv + g, HD);
@@ -343,16 +344,17 @@ __device__ __forceinline__ void attn_decode_mfma2_body(const DecodeAttnParams& a
     // Without the pre-rotation the same holds when the engine keeps the current position's
     // RoPE row (a.rc, tagged with the position): the prologue's loads then need no position
     // either, and a stale tag (a position set some other way) reloads the table row.
-    // (Paged: the pages of a one-step and of a two-step split come with the position; the K / V loads themselves, issued
+    // (Paged: the pages of a one-step and of a two-step split, one after the other 0.3 us of a launch each, come with the position; the K / V loads themselves, issued
     // ahead by them, made eight users slower: 3,563 tok/s against 3,624.)
     const bool ahead = PR || a.rc != nullptr;   // uniform: the prologue's loads need no position
     const bool spec = !PG && ahead && a.spec_ok;
     const int p = a.pos[m];
-    int page1 = 0, page2 = 0;
+    int page1 = 0, page2 = 0, page3 = 0;
     if constexpr (PG) {
         const int32_t* tb = a.km.table + m * a.km.max_pages;
         page1 = tb[min((KS * s) >> a.km.shift, a.km.max_pages - 1)];
         page2 = tb[min((2 * KS * s) >> a.km.shift, a.km.max_pages - 1)];
+        page3 = tb[min((2 * KS * s + KS) >> a.km.shift, a.km.max_pages - 1)];
     }
     const float* rcm = a.rc ? a.rc + m * rope_cur_stride(HD) : a.cs;
     const int rtag = a.rc ? __float_as_int(rcm[0]) : -1;
@@ -382,7 +384,8 @@ __device__ __forceinline__ void attn_decode_mfma2_body(const DecodeAttnParams& a
     const bool has_new = (t1 == ctx);
     auto run_of = [&](int tok) -> int64_t {   // kv_tok of the first key of a step
         if constexpr (PG) {
-            const int page = tok == KS * s ? page1 : tok == 2 * KS * s ? page2 : a.km.table[m * a.km.max_pages + (tok >> a.km.shift)];
+            int page = page1;
+            if (tok != KS * s) page = tok == 2 * KS * s ? page2 : tok == 2 * KS * s + KS ? page3 : a.km.table[m * a.km.max_pages + (tok >> a.km.shift)];
             return (int64_t)page * a.km.stride + (int64_t)(tok & ((1 << a.km.shift) - 1)) * HD;
         } else {
             return kv_tok<false>(a.km, m, tok, HD);
@@ -411,9 +414,9 @@ __device__ __forceinline__ void attn_decode_mfma2_body(const DecodeAttnParams& a
     // steps, Qwen2-0.5B's ctx 129-256, re-issued the same loads behind the position: +1.2 us)
     // (rows past the context hold whatever the cache has there: their scores are masked to -inf)
     const int64_t so0 = run_of(t0);
+    const int64_t new_at = has_new ? run_of(p & ~(KS - 1)) + (p & (KS - 1)) * HD : 0;   // the new token's place (a step's keys are in one page)
     if (keyed && (!spec || t0 != KS * s)) load_k(even, so0, keys_of(0));
-    // (the new token's place is asked for by the splits that do not hold it too: p is in the row's pages)
-    dec_pro_finish<HD, PR>(a, pr, dl, grp, kv_tok<PG>(a.km, m, p, HD), kb, vb, q_s, kv_new);
+    dec_pro_finish<HD, PR>(a, pr, dl, grp, new_at, kb, vb, q_s, kv_new);
     if (keyed) load_v(even, so0, keys_of(0));
     if (SETS > 1 && keyed && nstep > 1) load_step(odd, 1);
     for (int idx = tid; idx < (16 - G) * CPR; idx += NT)   // padded q rows

@@ -571,8 +571,8 @@ static int fill_dec_params(DecodeAttnParams& a, const void* qkv, int64_t B, cons
     const int senv = std::min(dev_env("QIE_DEC_SPLITS", 0), kDecMaxSplits);
     // split target: 32 (one-step splits up to 4k keys), from 8 rows on fewer where that would be more than two workgroups a CU: 8 at least
     // (Qwen2-7B fp8, 8 rows at 1,025 keys: 9 one-step splits 2.33 ms a token, 5 of two steps 2.35)
-    const int two_a_cu = (int)(2 * device_cu_count() / (a.nkv * B));
-    a.splits_target = senv > 0 ? senv : B < 8 ? kDecMSplits : std::max(8, std::min(kDecMSplits, two_a_cu));
+    auto two_a_cu = [&]() { return (int)(2 * device_cu_count() / (a.nkv * B)); };
+    a.splits_target = senv > 0 ? senv : B < 8 ? kDecMSplits : std::max(8, std::min(kDecMSplits, two_a_cu()));
     a.dbg = dev_env("QIE_DEC_DBG", 0);
     a.nsplit_max = std::min(a.splits_target, (cache->max_ctx + kDecMStep - 1) / kDecMStep);
     QIE_REQUIRE(a.nsplit_max <= kDecMaxSplits, "qie_attention_decode: max_ctx %d too long", cache->max_ctx);
