@@ -146,7 +146,7 @@ constexpr int BK = 64;
 // shapes, each measured on every tile with 1 to 8 segments; what the rule below picks is 1.6 % over the best of all of them on the
 // average and 17 % at most, with the constants fitted to 168 shapes before the kernel's ring and tickets changed 2.3 %).  Of
 // 80 other shapes that went to another tile: 0.95 of their time on the average, 1.01 at most: 1,536 -> 2 x 8,960 gate / up at 184 rows 28.8 -> 24.1 us,
-// 3,584 -> 4,608 at 489 36.4 -> 31.1, 17,408 -> 5,120 at 133 61.3 -> 53.5; one known to lose is 3,584 -> 3,584 at 205 to 235 rows, 17.0 -> 18.6 at 214.
+// 3,584 -> 4,608 at 489 36.4 -> 31.1, 17,408 -> 5,120 at 133 61.3 -> 53.5.
 // Up to one workgroup a CU a1 + s1 per k-tile, more a2 + (rounds of the chip) * (f2 + s2 per k-tile).  A k-tile costs what its
 // lines take through one CU (about 50 GB/s where they come from HBM or another die, 120 GB/s from L2), not its matrix work,
 // which is why the tall tiles win as soon as the rows fill them.  The constants are an MI355X's, whole (256 CUs): `cus` moves
@@ -219,6 +219,10 @@ inline Plan plan(int64_t M, int64_t cols, int64_t K, int64_t cus) {
             float us;
             if (s == 1) {
                 us = tiles <= cus ? t.a1 + nk * t.s1 : t.a2 + rounds(tiles / room) * (t.f2 + nk * t.s2);
+                // 64 x 64 on most CUs in one round, little of the last row tile filled: the rows that it lacks cost nothing, and the others' come the faster.
+                // us, split 128 x 64 / this: 3,584 -> 3,584 at 193 rows 18.1 / 16.4, 220 18.5 / 17.5, 230 18.8 / 18.2, 245 (.83 filled) 19.2 / 19.7; 2,560 ->
+                // 2,560 at 211 14.0 / 12.0; 5,120 -> 5,120 at 140 26.2 / 23.0, 166 27.6 / 27.3
+                if (c == 0 && M <= FITTED_ROWS && tiles <= cus && 2 * tiles > cus && 10 * ((M - 1) % t.bm + 1) <= 6 * t.bm) us *= .95f;
             } else {
                 if (cut == 0) break;
                 const float len = (float)((nk + s - 1) / s);

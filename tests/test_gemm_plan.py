@@ -93,6 +93,16 @@ def test_gemm_mid_offsets_fit(plan):
     assert max(taken) >= 1 << 20 and all((rows * y + cols) * 4 < 1 << 31 for y in taken)
 
 
+# rows, weight rows, K, us as 128 x 64 tiles in two parts of K and as whole 64 x 64 tiles
+SMALL = [(193, 3584, 3584, 18.1, 16.4), (220, 3584, 3584, 18.5, 17.5), (230, 3584, 3584, 18.8, 18.2), (245, 3584, 3584, 19.2, 19.7), (193, 2560, 2560, 13.8, 11.9),
+         (230, 2560, 2560, 13.9, 12.1), (129, 5120, 5120, 25.7, 22.1), (166, 5120, 5120, 27.6, 27.3)]
+
+
+def test_small_tiles_with_a_last_row_tile_hardly_filled():
+    for (M, N, K, split, whole), r in zip(SMALL, routes([c[:3] for c in SMALL])):
+        assert (r["tile"], r["splitk"]) == ((0, 1) if whole < split else (2, 2)), (M, N, K, r)
+
+
 # rows, weight rows, K, us of the best of the other tiles and the 256x256 kernel, of the 160-column tiles 8 to 11
 MEASURED = [
     (400, 9728, 896, 18.1, [16.9, 21.1, 24.8, 29.8]),
