@@ -18,7 +18,9 @@
 //   * in turns: waves 4 .. 7 run one barrier behind waves 0 .. 3, on every SIMD one wave's products run while the other's fragments are
 //     read.  Which form a tile has is what 184 shapes of 12 projections at 24 to 3,000 rows measured: 128 x 128 at K = 18,944, all eight in
 //     step with halves by wave 66.3 us, halves by register 67.4, in turns 69.5, in turns with halves by wave 63.1; at K = 896 13.1, 12.7,
-//     13.6, 14.1.  On the average of the 184 the products take 0.967 of what they took with halves by wave in step;
+//     13.6, 14.1.  192 and 256 x 128 in step with halves by register / in turns with halves by wave, us: 395 rows, K = 256, 8.7 / 10.6, 272 rows,
+//     896, 17.8 / 19.0, 830 rows, 2,048, 30.4 / 28.7; 217 rows, K = 512, 15.6 / 18.4, 250 rows, 1,536, 31.1 / 33.6, 667 rows, 3,584, 59.5 / 53.9.
+//     On the average of the 184 the products take 0.967 of what they took with halves by wave in step;
 //   * 320 rows: W of one k-tile more than A in flight (its lines come from HBM, A's mostly from L2, and a CU returns them in order): the
 //     staging alone 80 -> 69 us at 320 x 160;
 //   * split-K over workgroups where the tiles do not fill the chip (fp32 slabs, the last arriver sums them in part order: gemm8_kernel's
@@ -436,8 +438,12 @@ int launch_mid(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, hipS
         case 3:
             if (p.K < 1792) return launch_mid_t<EPI, 128, 128, 4, 4, 1, false>(p, pl, sk, tail, st);
             return launch_mid_t<EPI, 128, 128, 4, 4, 2, true>(p, pl, sk, tail, st);
-        case 4: return launch_mid_t<EPI, 192, 128, 4, 4, 2, true>(p, pl, sk, tail, st);
-        case 5: return launch_mid_t<EPI, 256, 128, 3, 3, 2, true>(p, pl, sk, tail, st);
+        case 4:
+            if (p.K < 1280) return launch_mid_t<EPI, 192, 128, 4, 4, 1, false>(p, pl, sk, tail, st);
+            return launch_mid_t<EPI, 192, 128, 4, 4, 2, true>(p, pl, sk, tail, st);
+        case 5:
+            if (p.K < 1792) return launch_mid_t<EPI, 256, 128, 3, 3, 1, false>(p, pl, sk, tail, st);
+            return launch_mid_t<EPI, 256, 128, 3, 3, 2, true>(p, pl, sk, tail, st);
         case 6: return launch_mid_t<EPI, 320, 64, 3, 3, 1, false>(p, pl, sk, tail, st);
         case 7: return launch_mid_t<EPI, 320, 128, 2, 4, 1, true>(p, pl, sk, tail, st);
         case 8: return launch_mid_t<EPI, 128, 160, 4, 4, 1, true>(p, pl, sk, tail, st);
