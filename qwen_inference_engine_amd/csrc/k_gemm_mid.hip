@@ -20,6 +20,7 @@
 //     step with halves by wave 66.3 us, halves by register 67.4, in turns 69.5, in turns with halves by wave 63.1; at K = 896 13.1, 12.7,
 //     13.6, 14.1.  192 and 256 x 128 in step with halves by register / in turns with halves by wave, us: 395 rows, K = 256, 8.7 / 10.6, 272 rows,
 //     896, 17.8 / 19.0, 830 rows, 2,048, 30.4 / 28.7; 217 rows, K = 512, 15.6 / 18.4, 250 rows, 1,536, 31.1 / 33.6, 667 rows, 3,584, 59.5 / 53.9.
+//     One row tile: 176 rows, 2,048, 36.2 / 38.2, 138 rows, 5,120, 70.3 / 73.9, 145 rows, 8,192, 116.9 / 108.7, in two parts of it 66.0 / 67.3;
 //     On the average of the 184 the products take 0.967 of what they took with halves by wave in step;
 //   * 320 rows: W of one k-tile more than A in flight (its lines come from HBM, A's mostly from L2, and a CU returns them in order): the
 //     staging alone 80 -> 69 us at 320 x 160;
@@ -431,6 +432,8 @@ int launch_mid_t(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, co
 
 template <int EPI>
 int launch_mid(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, hipStream_t st, const TailOf<EPI>& tail = {}) {
+    // one row tile, and a part of K that is not too long: what its workgroups wait for is their weights from memory, which the form in turns is no help to
+    const bool streams = pl.n_mt == 1 && p.K < 6144 * pl.splitk;
     switch (pl.tile) {
         case 0: return launch_mid_t<EPI, 64, 64, 5, 5, 2, false>(p, pl, sk, tail, st);
         case 1: return launch_mid_t<EPI, 64, 128, 3, 3, 2, false>(p, pl, sk, tail, st);
@@ -439,10 +442,10 @@ int launch_mid(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, hipS
             if (p.K < 1792) return launch_mid_t<EPI, 128, 128, 4, 4, 1, false>(p, pl, sk, tail, st);
             return launch_mid_t<EPI, 128, 128, 4, 4, 2, true>(p, pl, sk, tail, st);
         case 4:
-            if (p.K < 1280) return launch_mid_t<EPI, 192, 128, 4, 4, 1, false>(p, pl, sk, tail, st);
+            if (p.K < 1280 || streams) return launch_mid_t<EPI, 192, 128, 4, 4, 1, false>(p, pl, sk, tail, st);
             return launch_mid_t<EPI, 192, 128, 4, 4, 2, true>(p, pl, sk, tail, st);
         case 5:
-            if (p.K < 1792) return launch_mid_t<EPI, 256, 128, 3, 3, 1, false>(p, pl, sk, tail, st);
+            if (p.K < 1792 || streams) return launch_mid_t<EPI, 256, 128, 3, 3, 1, false>(p, pl, sk, tail, st);
             return launch_mid_t<EPI, 256, 128, 3, 3, 2, true>(p, pl, sk, tail, st);
         case 6: return launch_mid_t<EPI, 320, 64, 3, 3, 1, false>(p, pl, sk, tail, st);
         case 7: return launch_mid_t<EPI, 320, 128, 2, 4, 1, true>(p, pl, sk, tail, st);
