@@ -16,12 +16,12 @@
 //     in LDS behind the loop) or by every wave (4 x 2) in registers of its own, which needs no meeting: 320 x 160 spent 10 of 100 us on it.
 //     The sums are the same bits.  LDS gives 230 B a clock, so how often it is read does not decide;
 //   * in turns: waves 4 .. 7 run one barrier behind waves 0 .. 3, on every SIMD one wave's products run while the other's fragments are
-//     read.  Which form a tile has is what 184 shapes of 12 projections at 24 to 3,000 rows measured: 128 x 128 at K = 18,944, all eight in
-//     step with halves by wave 66.3 us, halves by register 67.4, in turns 69.5, in turns with halves by wave 63.1; at K = 896 13.1, 12.7,
-//     13.6, 14.1.  192 and 256 x 128 in step with halves by register / in turns with halves by wave, us: 395 rows, K = 256, 8.7 / 10.6, 272 rows,
-//     896, 17.8 / 19.0, 830 rows, 2,048, 30.4 / 28.7; 217 rows, K = 512, 15.6 / 18.4, 250 rows, 1,536, 31.1 / 33.6, 667 rows, 3,584, 59.5 / 53.9.
-//     One row tile: 176 rows, 2,048, 36.2 / 38.2, 138 rows, 5,120, 70.3 / 73.9, 145 rows, 8,192, 116.9 / 108.7, in two parts of it 66.0 / 67.3;
-//     On the average of the 184 the products take 0.967 of what they took with halves by wave in step;
+//     read.  Which form a tile has is what 184 shapes of 12 projections at 24 to 3,000 rows measured, and for 128, 192 and 256 x 128, that change
+//     it with the k-tiles of a part, 300 more.  Those three in step with halves by register / in turns with halves by wave, us: 128 rows a tile, 222
+//     rows, K = 1,792, 23.6 / 24.5, 232 rows, 3,072, 33.7 / 35.5, 336 rows, 4,096, 45.2 / 44.8, 885 rows, 2,048, 21.7 / 22.3, 846 rows, 3,584, 39.1 / 38.1,
+//     303 rows, 8,192, 80.9 / 78.2; 192, 395 rows, 256, 8.7 / 10.6, 272 rows, 896, 17.8 / 19.0, 830 rows, 2,048, 30.4 / 28.7; 256, 217 rows, 512, 15.6 / 18.4, 677 rows, 1,536, 31.1 / 31.3, 667 rows, 3,584,
+//     59.5 / 53.9.  One row tile: 104 rows, 2,048, 25.9 / 27.6, 72 rows, 5,120, 54.8 / 56.8, 176 rows, 2,048, 36.2 / 38.2, 138 rows, 5,120, 70.3 / 73.9,
+//     145 rows, 8,192, 116.9 / 108.7, in two parts of it 66.0 / 67.3;
 //   * 320 rows: W of one k-tile more than A in flight (its lines come from HBM, A's mostly from L2, and a CU returns them in order): the
 //     staging alone 80 -> 69 us at 320 x 160;
 //   * split-K over workgroups where the tiles do not fill the chip (fp32 slabs, the last arriver sums them in part order: gemm8_kernel's
@@ -439,7 +439,7 @@ int launch_mid(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, hipS
         case 1: return launch_mid_t<EPI, 64, 128, 3, 3, 2, false>(p, pl, sk, tail, st);
         case 2: return launch_mid_t<EPI, 128, 64, 3, 3, 2, false>(p, pl, sk, tail, st);
         case 3:
-            if (p.K < 1792) return launch_mid_t<EPI, 128, 128, 4, 4, 1, false>(p, pl, sk, tail, st);
+            if (p.K < (pl.n_mt <= 4 ? 4096 : 2304) * pl.splitk || streams) return launch_mid_t<EPI, 128, 128, 4, 4, 1, false>(p, pl, sk, tail, st);
             return launch_mid_t<EPI, 128, 128, 4, 4, 2, true>(p, pl, sk, tail, st);
         case 4:
             if (p.K < 1280 || streams) return launch_mid_t<EPI, 192, 128, 4, 4, 1, false>(p, pl, sk, tail, st);
