@@ -128,13 +128,15 @@ inline int parts(int64_t M, int64_t cols, int64_t K, int64_t cus, int mink = 64)
     const int s = splitk(tiles, cus, (int)(K / 64), mink);
     return s == 1 && 2 * tiles < cus ? 0 : s;
 }
-// expected time, us: 1.45 a k-tile and 5 a round of the chip (fitted as k_gemm_mid.hip's tiles; over 20 projections at 256 to 8,192 rows
-// the kernel now takes 2 % less on the average, 0.84 to 1.24 of this)
-inline float us(int64_t M, int64_t cols, int64_t K, int64_t cus) {
-    const int s = parts(M, cols, K, cus);
-    if (s == 0) return 1e30f;
+// expected time, us, of `s` parts a tile: 1.45 a k-tile and 5 a round of the chip (fitted as k_gemm_mid.hip's tiles; over 20 projections at 256 to
+// 8,192 rows the kernel now takes 2 % less on the average, 0.84 to 1.24 of this)
+inline float us_in(int64_t M, int64_t cols, int64_t K, int64_t cus, int s) {
     const int64_t tiles = ((M + 255) / 256) * ((cols + 255) / 256), nk = K / 64;
     return (float)((tiles * s + cus - 1) / cus) * (nk / (float)s * 1.45f + 5.f) + 5.f + (s > 1 ? 8.f * s : 0.f);
+}
+inline float us(int64_t M, int64_t cols, int64_t K, int64_t cus) {
+    const int s = parts(M, cols, K, cus);
+    return s == 0 ? 1e30f : us_in(M, cols, K, cus, s);
 }
 }  // namespace g8p
 
@@ -281,7 +283,7 @@ inline int64_t columns_ahead(int64_t M, int64_t cols, int64_t K, int64_t cus) {
     for (int64_t r = full; r >= 1 && r >= full - 1; r--) {
         const int64_t c = r * cus / n_mt * 256;
         if (c <= 0 || c >= cols) continue;
-        const float us = g8p::us(M, c, K, cus) + more * best(M, cols - c, K, cus).us;
+        const float us = g8p::us_in(M, c, K, cus, 1) + more * best(M, cols - c, K, cus).us;   // (the first launch is never split)
         if (us < least) {
             least = us;
             ahead = c;

@@ -42,6 +42,36 @@ def test_the_rule_is_sound(tmp_path):
         assert a == 0 or (a % 256 == 0 and a < cols and M >= 256 and K >= 256 and (tiles % cus == 0 or cus - tiles % cus < -(-M // 256))), (M, cols, K, cus, a)
 
 
+PRICES = r"""
+#include "gemm_plan.hpp"
+#include <cstdio>
+using namespace qie;
+int main() {
+    long M, cols, K, cus;
+    while (std::scanf("%ld %ld %ld %ld", &M, &cols, &K, &cus) == 4) {
+        const long a = (long)mid::columns_ahead(M, cols, K, cus), tiles = (M + 255) / 256 * (a / 256);
+        const float more = M > mid::FITTED_ROWS ? 1.f : 1.06f;
+        const float first = (tiles + cus - 1) / cus * (K / 64 * 1.45f + 5.f) + 5.f;   // unsplit
+        const float one = std::min(g8p::us(M, cols, K, cus), more * mid::best(M, cols, K, cus).us);
+        std::printf("%ld %.6g\n", a, a > 0 ? (first + more * mid::best(M, cols - a, K, cus).us) / one : 0.f);
+    }
+}
+"""
+
+
+def test_the_first_launch_is_priced_as_it_runs(tmp_path):
+    """Never split over K, also where its tiles are fewer than the CUs (many row tiles: a round of the chip is few columns)."""
+    r = random.Random(5)
+    cases = [(23808, 1024, 18944, 256), (23571, 622, 19648, 256)] + [(r.randint(256, 32000), r.randint(300, 9000), 64 * r.randint(8, 330), 256) for _ in range(2000)]
+    (tmp_path / "p.cpp").write_text(PRICES)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(tmp_path / "p.cpp"), "-o", str(tmp_path / "p")], check=True)
+    text = "\n".join("%d %d %d %d" % c for c in cases)
+    got = [line.split() for line in subprocess.run([str(tmp_path / "p")], input=text, text=True, capture_output=True, check=True).stdout.splitlines()]
+    assert sum(int(a) > 0 for a, _ in got) > 100
+    for c, (a, of_one) in zip(cases, got):
+        assert float(of_one) <= .9701, (c, a, of_one)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,rows,K", SHAPES)
 @pytest.mark.parametrize("epi", ["f32", "store", "residual", "swiglu"])
