@@ -272,7 +272,7 @@ inline Plan best(int64_t M, int64_t cols, int64_t K, int64_t cus) {
 // 512 rows 198 / 162, 1,024 361 / 297, 2,048 609 / 573; Qwen2-0.5B gate / up 3,500 rows 93 / 78.
 inline int64_t columns_ahead(int64_t M, int64_t cols, int64_t K, int64_t cus) {
     const int64_t n_mt = (M + 255) / 256, n_nt = (cols + 255) / 256;
-    if (K % BK != 0 || M < 256 || n_mt * n_nt <= cus) return 0;
+    if (K % BK != 0 || K < 256 || M < 256 || n_mt * n_nt <= cus) return 0;   // (no launch of the 256x256 kernel)
     // (fitted rows: the tiles' times are 3 to 10 % short of the measured beside the 256x256 kernel's; without 1.06 of them Qwen3-14B gate / up at 2,048
     // rows would leave 10,240 columns, 573 us, and not 2,048, 563)
     const float more = M > FITTED_ROWS ? 1.f : 1.06f;
