@@ -6,7 +6,7 @@ import subprocess
 import pytest
 
 from gemm_route import routes
-from test_gpu_gemm_mid import GROWS, PLANS
+from test_gpu_gemm_mid import GROWS, MORE, PLANS, SHAPES
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "qwen_inference_engine_amd", "csrc")
 
@@ -65,6 +65,15 @@ def test_gemm_mid_shapes_take_every_tile(plan):
     got = [(p[0], "whole" if p[2] == 1 else "split" if p[1] == 0 else "mixed") for p in plan([f"m {M} {N} {K} 256" for M, N, K, _, _ in PLANS])]
     assert got == [(t, kind) for _, _, _, t, kind in PLANS]
     assert set(got) == {(t, kind) for t in range(8) for kind in ("whole", "split", "mixed")}
+
+
+def test_gemm_mid_products_come_to_every_tile():
+    """What qie_linear does with the shapes that the GPU test multiplies, one segment each: every tile whole, split and both, but for two that are mixed
+    only where a tile of 160 columns is the better one."""
+    got = {(r["tile"], "whole" if r["splitk"] == 1 else "split" if r["whole"] == 0 else "mixed") for r in routes(SHAPES + MORE) if r["tile"] >= 0 and r["ahead"] == 0}
+    assert {g for g in got if g[0] < 8} == {(t, kind) for t in range(8) for kind in ("whole", "split", "mixed")} - {(2, "mixed"), (6, "mixed")}
+    (r,) = routes([GROWS])
+    assert 0 <= r["tile"] < 8 and r["splitk"] > 1 and r["ahead"] == 0
 
 
 def test_a_shape_whose_slabs_outgrow_the_reserve(plan):

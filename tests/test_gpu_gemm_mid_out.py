@@ -20,7 +20,7 @@ SHAPES = [(17, 72, 64, 0, 1), (33, 72, 2048, 0, 4), (17, 16500, 64, 1, 1), (64, 
 
 
 def test_the_shapes_take_their_tiles():
-    assert [(r["tile"], r["splitk"]) for r in routes([s[:3] for s in SHAPES])] == [s[3:] for s in SHAPES]
+    assert [(r["tile"], r["splitk"], r["ahead"]) for r in routes([s[:3] for s in SHAPES])] == [(*s[3:], 0) for s in SHAPES]
 
 
 @pytest.mark.parametrize("M,rows,K,tile,parts", SHAPES)

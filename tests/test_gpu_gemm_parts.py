@@ -13,7 +13,7 @@ SHAPES = [(599, 8376, 9280, 2), (782, 4636, 12416, 3), (385, 5660, 21952, 4)]
 
 
 def test_the_shapes_are_cut():
-    assert [(r["tile"], r["parts"]) for r in routes([s[:3] for s in SHAPES])] == [(-1, s[3]) for s in SHAPES]
+    assert [(r["tile"], r["parts"], r["ahead"]) for r in routes([s[:3] for s in SHAPES])] == [(-1, s[3], 0) for s in SHAPES]
 
 
 @pytest.mark.gpu
