@@ -268,13 +268,13 @@ inline Plan best(int64_t M, int64_t cols, int64_t K, int64_t cus) {
 
 // Columns that the 256x256 kernel takes of a product, whole rounds of the chip, with the rest to the tiles above in a launch behind it; 0: one
 // launch does all.  A last round of 256x256 tiles that fills little of the chip costs a whole one, and tiles of fewer columns fill it with what
-// is left.  us, one launch / two: Qwen2-7B gate / up 400 rows 145 / 134, 900 rows 264 / 234, 1,500 356 / 345, down 6,000 784 / 687; Qwen3-14B gate / up
-// 512 rows 198 / 162, 1,024 361 / 297, 2,048 609 / 573; Qwen2-0.5B gate / up 3,500 rows 93 / 78.
+// is left.  us, one launch / two: Qwen2-7B gate / up 400 rows 148 / 133, 900 rows 266 / 238, 1,500 360 / 344, down 6,000 793 / 677; Qwen3-14B gate / up
+// 512 rows 209 / 164, 1,024 365 / 305, 2,048 610 / 571; Qwen2-0.5B gate / up 3,500 rows 96 / 79.
 inline int64_t columns_ahead(int64_t M, int64_t cols, int64_t K, int64_t cus) {
     const int64_t n_mt = (M + 255) / 256, n_nt = (cols + 255) / 256;
     if (K % BK != 0 || K < 256 || M < 256 || n_mt * n_nt <= cus) return 0;   // (no launch of the 256x256 kernel)
     // (fitted rows: the tiles' times are 3 to 10 % short of the measured beside the 256x256 kernel's; without 1.06 of them Qwen3-14B gate / up at 2,048
-    // rows would leave 10,240 columns, 573 us, and not 2,048, 563)
+    // rows would leave 10,240 columns, which takes 2 % longer than 2,048)
     const float more = M > FITTED_ROWS ? 1.f : 1.06f;
     const float whole = std::min(g8p::us(M, cols, K, cus), more * best(M, cols, K, cus).us);
     float least = .97f * whole;
@@ -283,7 +283,11 @@ inline int64_t columns_ahead(int64_t M, int64_t cols, int64_t K, int64_t cus) {
     for (int64_t r = full; r >= 1 && r >= full - 1; r--) {
         const int64_t c = r * cus / n_mt * 256;
         if (c <= 0 || c >= cols) continue;
-        const float us = g8p::us_in(M, c, K, cus, 1) + more * best(M, cols - c, K, cus).us;   // (the first launch is never split)
+        const Plan rest = best(M, cols - c, K, cus);
+        // (320 x 128 tiles, whole, of long K: 1.2 to 1.35 a k-tile measured where the fit says 1.11.  Qwen3-14B down at 4,880 to 5,120 rows 748 in one launch,
+        // 775 in two, with such a rest; 14,336 -> 4,096 at 6,144 rows 615, 618)
+        const float slow = K > 8192 && rest.tile == 7 && rest.splitk == 1 ? 1.21f : 1.f;
+        const float us = g8p::us_in(M, c, K, cus, 1) + more * slow * rest.us;   // (the first launch is never split)
         if (us < least) {
             least = us;
             ahead = c;
