@@ -165,11 +165,12 @@ __global__ __launch_bounds__(256) void fetch_out_kernel(const uint4* src, uint4*
 }
 
 void make_out(qie_batch* b, size_t bytes, size_t ids) {
-    bytes = bytes > (size_t)8 << 20 ? 0 : (bytes + 15) / 16 * 16;
+    bytes = (std::min(bytes, (size_t)8 << 20) + 15) / 16 * 16;
     if (ids + bytes == 0) return;
     unsigned char* p = nullptr;
     if (hipHostMalloc((void**)&p, ids + bytes, hipHostMallocDefault) != hipSuccess) {   // (qie_decode and fetch_out do without)
         (void)hipGetLastError();
+        if (ids && bytes) make_out(b, 0, ids);
         return;
     }
     b->h_pinned = p;
@@ -193,11 +194,12 @@ int fetch_out(qie_batch* b, void* dst, const void* src, size_t bytes, int (*chec
                            (uint4*)b->h_out, whole, (int)(bytes % 16));
         QIE_LAUNCH_CHECK();
     }
+    const bool behind = !pinned && bytes > 0 && check;   // dst is written only when the check has passed
+    if (!pinned && bytes > 0 && !check) QIE_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
     QIE_HIP(hipStreamSynchronize(st));
     if (check) QIE_TRY(check(b));
-    if (pinned) {
-        memcpy(dst, b->h_out, bytes);
-    } else if (bytes > 0) {
+    if (pinned) memcpy(dst, b->h_out, bytes);
+    if (behind) {
         QIE_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
         QIE_HIP(hipStreamSynchronize(st));
     }

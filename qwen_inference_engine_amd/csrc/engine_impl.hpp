@@ -127,12 +127,12 @@ struct qie_batch {
 
 
 namespace qie {
-// hipMalloc of at least 16 bytes
-// Pinned memory of a batch, made with it: for results of up to `bytes` (none above 8 MB), behind `ids` bytes for h_ids.
+// Pinned memory of a batch, made with it: for results of up to `bytes` (8 MB of them), behind `ids` bytes for h_ids.
 void make_out(qie_batch* b, size_t bytes, size_t ids = 0);
 // `bytes` of device memory, 16-byte aligned, to the caller's: behind everything on the engine's stream, waited for.  check: run between the wait
 // and the copy into dst (what makes the results void).
 int fetch_out(qie_batch* b, void* dst, const void* src, size_t bytes, int (*check)(qie_batch*) = nullptr);
+// hipMalloc of at least 16 bytes
 int dmalloc(void** p, size_t bytes);
 // Page pool of a paged batch (host side, deterministic): take pages so that slot `seq` holds
 // positions [0, ntok) (all-or-nothing), return a slot's pages, upload the block table when it

@@ -43,3 +43,26 @@ def test_logits_of_an_odd_vocabulary():
     assert np.array_equal(three.logits(), np.repeat(want, 3, 0))
     for x in (one, three, eng):
         x.close()
+
+
+def test_slots_whose_logits_are_more_than_is_pinned():
+    """70 slots of 32,000 logits, 9 MB: a few rows by way of the pinned 8 MB, all of them past it."""
+    att = S.LatentAttention(4, 16, 8, 8, 32, 9, 8, 10000.0, 0.2, None)
+    spec = S.LayeredSpec("fetch", 64, 32000, 1e-5, (S.LayerSpec(att, S.FeedForward("dense", 96)),), True)
+    rng = np.random.default_rng(2)
+    tensors = {}
+    for n, s in spec.tensor_shapes().items():
+        v = np.ones(s, np.float32) if n.endswith(("norm1", "norm2", "final.norm", "dkv.norm")) else \
+            (rng.standard_normal(s) / np.sqrt(s[-1] if n != "embed" else 1.0)).astype(np.float32)
+        tensors[n] = (np.ascontiguousarray(v).view(np.uint32) >> 16).astype(np.uint16).reshape(s)
+    eng = q.Engine(spec, max_ctx=64, dtype="float32").load_tensors(tensors)
+    b = eng.batch(70, 64)
+    toks = [int(t) for t in rng.integers(0, 32000, 70)]
+    every = b.step([(m, [t]) for m, t in enumerate(toks)], range(70))
+    for m in (0, 41, 69):
+        b.release(m)
+        one = b.step([(m, [toks[m]])], [0])[0]
+        # (other kernels take the products of fewer rows: fp32 sums in another order)
+        assert one.any() and np.abs(one - every[m]).max() <= 1e-5 * np.abs(every).max()
+    b.close()
+    eng.close()
