@@ -704,7 +704,7 @@ int qie_debug_tr16_probe(int32_t* out_dev) {
 int64_t qie_attention_decode_workspace_bytes(int64_t B, int32_t n_heads, int32_t n_kv_heads, int32_t head_dim,
                                              int32_t max_ctx) {
     // an upper bound for every splits_target <= kDecMaxSplits (nsplit_max in fill_dec_params)
-    const int64_t ns = std::min<int64_t>(kDecMaxSplits, (max_ctx + 63) / 64);   // 64- or 128-key steps
+    const int64_t ns = std::min<int64_t>(kDecMaxSplits, ((int64_t)max_ctx + kDecMStep - 1) / kDecMStep);
     const int64_t cnt = dec_counter_bytes(B, n_kv_heads);
     return cnt + B * n_heads * ns * (head_dim + 2) * 4;
 }

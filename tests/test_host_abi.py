@@ -211,3 +211,10 @@ def test_ids_of_long_contexts_hold_little_pinned_memory(qlib):
     room = C.CDLL(_lib.load()._name)._ZN3qie11ids_at_onceEii
     room.restype = C.c_int64
     assert room(1, 64) == 64 and room(8, 128) == 1024 and room(8, 1 << 20) == 16384
+
+
+def test_decode_attention_workspace(qlib):
+    """Tickets of 512 bytes a row and kv head in multiples of 1,024 pairs, and the results of one split for each 128 keys, 512 at most."""
+    for B, nq, nkv, hd, ctx in ((1, 14, 2, 64, 1), (8, 28, 4, 128, 129), (8, 28, 4, 128, 4096), (64, 40, 8, 128, 32768), (1024, 8, 1, 64, 100000), (1025, 8, 1, 64, 256)):
+        splits = min(512, -(-ctx // 128))
+        assert qlib.qie_attention_decode_workspace_bytes(B, nq, nkv, hd, ctx) == -(-B * nkv // 1024) * 1024 * 512 + B * nq * splits * (hd + 2) * 4
