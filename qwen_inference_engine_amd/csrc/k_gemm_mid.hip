@@ -287,9 +287,9 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
         }
     };
     const int col0 = wn * TN + 4 * g;
-    // residuals: all on their way at once
+    // residuals: all on their way at once; ahead of the parts' sum where registers hold both
     [[maybe_unused]] uint2 before[FR][FJ];
-    if constexpr (EPI == QIE_EPI_RESIDUAL) {
+    [[maybe_unused]] auto load_before = [&]() {
         if (quads) {
 #pragma unroll
             for (int i = 0; i < FR; i++)
@@ -307,7 +307,9 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
                     before[i][j] = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
                 }
         }
-    }
+    };
+    constexpr bool BOTH = FR * FJ <= 16;
+    if constexpr (EPI == QIE_EPI_RESIDUAL && BOTH) load_before();
 
     constexpr bool SPLITS = BN != 160;   // (mid::WIDE: whole only)
     if (SPLITS && parts > 1) {   // uniform.  A wave's share of the tile meets by itself: no wave waits for the others of its workgroup
@@ -367,6 +369,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
 
     // ---------------- epilogue.  D = W Aᵀ: a lane holds row m = lane & 15 and the columns 4 g .. 4 g + 3 of a fragment, one
     // 8- (fp32: 16-) byte store where C's rows allow it
+    if constexpr (EPI == QIE_EPI_RESIDUAL && !BOTH) load_before();
     if constexpr (EPI == QIE_EPI_SWIGLU) {
 #pragma unroll
         for (int m = 0; m < (FJ + 1) / 2; m++) {
