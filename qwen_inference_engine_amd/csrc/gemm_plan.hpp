@@ -266,13 +266,26 @@ inline Plan best(int64_t M, int64_t cols, int64_t K, int64_t cus) {
     return M > 64 && wide.tile >= 0 && wide.us < (pl.splitk > 1 ? 1.1f : 1.f) * pl.us ? wide : pl;
 }
 
+// The tiles that take a product; tile -1: none, k_gemm.hip's kernels do.
+inline Plan choose(int64_t M, int64_t cols, int64_t K, int64_t cus) {
+    const Plan none{-1, 0, 1, 0, 0, 1e30f};
+    if (K % BK != 0) return none;   // (rows of x and weights are on the 16-byte grid of LDS-DMA: qie_linear)
+    const float other_us = g8p::us(M, cols, K, cus);
+    const Plan pl = plan(M, cols, K, cus), wide = plan_wide(M, cols, K, cus);
+    // (split plans of gate / up's many columns take 10 to 30 % longer than the fit says)
+    if (M > 64 && wide.tile >= 0 && wide.us < (pl.splitk > 1 ? 1.1f : 1.f) * pl.us && wide.us < .97f * other_us) return wide;
+    return pl.tile >= 0 && pl.us < .88f * other_us ? pl : none;   // 12 %: what the two fits are off by on long prompts
+}
 // Columns that the 256x256 kernel takes of a product, whole rounds of the chip, with the rest to the tiles above in a launch behind it; 0: one
 // launch does all.  A last round of 256x256 tiles that fills little of the chip costs a whole one, and tiles of fewer columns fill it with what
 // is left.  us, one launch / two: Qwen2-7B gate / up 400 rows 148 / 133, 900 rows 266 / 238, 1,500 360 / 344, down 6,000 793 / 677; Qwen3-14B gate / up
 // 512 rows 209 / 164, 1,024 365 / 305, 2,048 610 / 571; Qwen2-0.5B gate / up 3,500 rows 96 / 79.
-inline int64_t columns_ahead(int64_t M, int64_t cols, int64_t K, int64_t cus) {
+// f32: results in fp32.  The tiles sum the two halves of every k-tile apart, the 256x256 kernel in one chain: errors against 64 bits of 1.86e-7 and 2.69e-7
+// at K = 2,048.  bf16 results round either away; fp32 ones stay with the tiles that would take the whole product.
+inline int64_t columns_ahead(int64_t M, int64_t cols, int64_t K, int64_t cus, bool f32) {
     const int64_t n_mt = (M + 255) / 256, n_nt = (cols + 255) / 256;
     if (K % BK != 0 || K < 256 || M < 256 || n_mt * n_nt <= cus) return 0;   // (no launch of the 256x256 kernel)
+    if (f32 && choose(M, cols, K, cus).tile >= 0) return 0;
     // (fitted rows: the tiles' times are 3 to 10 % short of the measured beside the 256x256 kernel's; without 1.06 of them Qwen3-14B gate / up at 2,048
     // rows would leave 10,240 columns, which takes 2 % longer than 2,048)
     const float more = M > FITTED_ROWS ? 1.f : 1.06f;
@@ -296,16 +309,6 @@ inline int64_t columns_ahead(int64_t M, int64_t cols, int64_t K, int64_t cus) {
     return ahead;
 }
 
-// The tiles that take a product; tile -1: none, k_gemm.hip's kernels do.
-inline Plan choose(int64_t M, int64_t cols, int64_t K, int64_t cus) {
-    const Plan none{-1, 0, 1, 0, 0, 1e30f};
-    if (K % BK != 0) return none;   // (rows of x and weights are on the 16-byte grid of LDS-DMA: qie_linear)
-    const float other_us = g8p::us(M, cols, K, cus);
-    const Plan pl = plan(M, cols, K, cus), wide = plan_wide(M, cols, K, cus);
-    // (split plans of gate / up's many columns take 10 to 30 % longer than the fit says)
-    if (M > 64 && wide.tile >= 0 && wide.us < (pl.splitk > 1 ? 1.1f : 1.f) * pl.us && wide.us < .97f * other_us) return wide;
-    return pl.tile >= 0 && pl.us < .88f * other_us ? pl : none;   // 12 %: what the two fits are off by on long prompts
-}
 }  // namespace mid
 
 }  // namespace qie

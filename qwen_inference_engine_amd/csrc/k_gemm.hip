@@ -1545,7 +1545,7 @@ static int gemm_with(const qie_linear_args* a, const QkvTail* tail, bool* done, 
         const bool g8ok = a->K % g8::BK == 0 && a->K >= 4 * g8::BK;
         const bool one_segment = a->epilogue == QIE_EPI_SWIGLU || a->seg_rows[0] == a->N;
         if (g8ok && force < 0 && !tail && one_segment && !(a->flags & QIE_LINEAR_STREAMK) && mid::strides_fit(a->ldx, a->ldy) && dev_env("QIE_HYBRID", 1)) {
-            const int64_t ahead = mid::columns_ahead(a->M, cols, a->K, cus) / (a->epilogue == QIE_EPI_SWIGLU ? 2 : 1);   // outputs
+            const int64_t ahead = mid::columns_ahead(a->M, cols, a->K, cus, a->epilogue == QIE_EPI_F32) / (a->epilogue == QIE_EPI_SWIGLU ? 2 : 1);   // outputs
             if (ahead > 0) {
                 GemmParams first = p, rest = p;
                 first.N = first.n0 = first.n01 = ahead;

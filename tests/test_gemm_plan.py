@@ -70,9 +70,9 @@ def test_gemm_mid_shapes_take_every_tile(plan):
 def test_gemm_mid_products_come_to_every_tile():
     """What qie_linear does with the shapes that the GPU test multiplies, one segment each: every tile whole, split and both, but for two that are mixed
     only where a tile of 160 columns is the better one."""
-    got = {(r["tile"], "whole" if r["splitk"] == 1 else "split" if r["whole"] == 0 else "mixed") for r in routes(SHAPES + MORE) if r["tile"] >= 0 and r["ahead"] == 0}
+    got = {(r["tile"], "whole" if r["splitk"] == 1 else "split" if r["whole"] == 0 else "mixed") for r in routes(SHAPES + MORE, f32=True) if r["tile"] >= 0 and r["ahead"] == 0}
     assert {g for g in got if g[0] < 8} == {(t, kind) for t in range(8) for kind in ("whole", "split", "mixed")} - {(2, "mixed"), (6, "mixed")}
-    (r,) = routes([GROWS])
+    (r,) = routes([GROWS], f32=True)
     assert 0 <= r["tile"] < 8 and r["splitk"] > 1 and r["ahead"] == 0
 
 
@@ -155,6 +155,14 @@ MEASURED_AHEAD = [
     (1536, 16384, 2048, 109.7, 102.5), (3328, 16384, 2048, 225.7, 228.5), (6167, 16384, 2048, 402.9, 397.6), (9223, 16384, 2048, 603.1, 606.4),
     (2303, 32000, 3584, 460.3, 452.7), (3820, 32000, 3584, 740.0, 743.0), (5877, 32000, 3584, 1121.4, 1130.5), (8441, 32000, 3584, 1596.5, 1593.3),
 ]
+
+
+def test_fp32_results_stay_with_the_tiles():
+    """Products that one launch of k_gemm_mid.hip would take, whose sums are of two chains, keep them where the results are fp32."""
+    shapes = [c[:3] for c in MEASURED_AHEAD] + [(751, 22016, 2048), (978, 17920, 1536), (1586, 9728, 896)]
+    for x, bf, f32 in zip(shapes, routes(shapes), routes(shapes, f32=True)):
+        assert f32["ahead"] == (0 if f32["tile"] >= 0 else bf["ahead"]), x
+    assert any(bf["ahead"] and not f32["ahead"] for bf, f32 in zip(routes(shapes), routes(shapes, f32=True)))
 
 
 def test_two_launches_where_they_are_no_slower():

@@ -17,7 +17,7 @@ DRIVER = r"""
 #include <cstdio>
 int main() {
     long M, cols, K, cus;
-    while (std::scanf("%ld %ld %ld %ld", &M, &cols, &K, &cus) == 4) std::printf("%ld\n", (long)qie::mid::columns_ahead(M, cols, K, cus));
+    while (std::scanf("%ld %ld %ld %ld", &M, &cols, &K, &cus) == 4) std::printf("%ld\n", (long)qie::mid::columns_ahead(M, cols, K, cus, false));
 }
 """
 SHAPES = [(1030, 13500, 768), (700, 22004, 512), (511, 33001, 256), (2300, 7510, 256), (345, 45029, 768)]
@@ -54,7 +54,7 @@ using namespace qie;
 int main() {
     long M, cols, K, cus;
     while (std::scanf("%ld %ld %ld %ld", &M, &cols, &K, &cus) == 4) {
-        const long a = (long)mid::columns_ahead(M, cols, K, cus), tiles = (M + 255) / 256 * (a / 256);
+        const long a = (long)mid::columns_ahead(M, cols, K, cus, false), tiles = (M + 255) / 256 * (a / 256);
         const float more = M > mid::FITTED_ROWS ? 1.f : 1.06f;
         const float first = (tiles + cus - 1) / cus * (K / 64 * 1.45f + 5.f) + 5.f;   // unsplit
         const float one = std::min(g8p::us(M, cols, K, cus), more * mid::best(M, cols, K, cus).us);
@@ -115,3 +115,16 @@ def test_two_launches(qlib, oracle, M, rows, K, epi):
     got = G.host_bf16(y)
     assert (np.abs(G.bf(got)[:M, :N] - want) <= tol).all()
     assert np.array_equal(got[:M, N:], y0[:M, N:]) and np.array_equal(got[M], y0[M])
+
+
+@pytest.mark.gpu
+def test_fp32_results_keep_their_error(qlib):
+    """Of a product whose columns would go ahead with bf16 results.  An fp32 chain's error grows with the square root of its steps, so one chain over K errs
+    by sqrt(2) of what two over halves of it do: 1.55e-7 and 1.10e-7 of the result here, over 14 million of them.  The bound is their geometric mean."""
+    M, N, K = 1030, 13500, 768
+    x, w = bf16((M, K), 1.0, 41), bf16((N, K), K ** -0.5, 42)
+    y = G.zeros((M, N), np.float32)
+    linear(G.dev(x), [G.dev(w)], [], M, K, N, y, _lib.QIE_EPI_F32)
+    want = G.bf(x).astype(np.float64) @ G.bf(w).astype(np.float64).T
+    err = np.linalg.norm(y.numpy() - want) / np.linalg.norm(want)
+    assert err <= 1.31e-7, err
