@@ -129,12 +129,14 @@ __device__ __forceinline__ void split_bf16x8(const float* e, uint4* parts) {
 //   O  += P . V   : those 8 probabilities of a lane are A's 8 k slots as they lie (k slot 8 g + 4 t + r is key 16 t + 4 g + r), in three
 //                   bf16 parts (hi, mid, lo: the 24 bits of the fp32 value, so every product is the fp32 product); B = the V rows in that
 //                   order, transposed by ds_read_b64_tr_b16 out of LDS that only this wave writes and reads.
-// The waves' (max, sum, O) meet in LDS once per split, the splits in memory, by the last-arriving workgroup.
+// The waves' (max, sum, O) meet in LDS once per split, the splits in memory, by the last-arriving wave of a head's (tickets by wave).
 // What it waits for is memory and instruction latency, at one wave a SIMD (Qwen2-7B, 2,049 keys: 4 MB of K / V in 68 workgroups), so the
 // layout spares instructions and meetings.  With the scores of all 128 keys exponentiated and split by every wave, each for its slice of d,
 // a step had two barriers and took 1.7 us behind its loads, now 0.9; with one ticket a kv head, its workgroup alone read all splits back:
-// 2.7 us for 17, now 1.8 by four waves on CUs of their own.  A launch, by time stamps inside it, before / now: Qwen2-0.5B at 129 keys 5.5 / 4.0
-// us, 7 rows at 700 8.1 / 5.3, Qwen2-7B at 2,049 9.1 / 7.7, 4 rows at 1,500 9.9 / 7.3, 8 at 1,025 12.6 / 9.7, Qwen3-14B at 6,001 15.0 / 11.7.
+// 2.7 us for 17, now 1.8 by four waves on CUs of their own.  V goes out behind the prologue while K is on its way: 3 to 10 % of a launch over waiting
+// for K first (8 rows paged in 352 workgroups 2 % longer: some CUs have two, and one's V goes ahead of the other's K).  From launch to launch in a
+// graph, the form with barriers / now, us: Qwen2-0.5B at 129 keys 6.2 / 4.1, 7 rows at 700 8.5 / 5.3, Qwen2-7B at 2,049 9.2 / 7.3, 4 rows at 1,500 11.2 /
+// 7.6, 8 at 1,025 paged 11.9 / 9.2, Qwen3-14B at 6,001 14.3 / 10.0.
 constexpr int kDecMStep = 128;      // keys per step
 constexpr int kDecMWaves = 4;       // waves that have keys
 constexpr int kDecMSplits = 32;     // default split target
@@ -199,7 +201,7 @@ __device__ __forceinline__ DecPro dec_pro_issue(const DecodeAttnParams& a, const
 }
 
 // qk-norm + RoPE of the q heads and the new k, then q -> LDS (bf16), new k/v -> cache
-// and LDS.  Branch-free (only the stores are predicated), stores predicated, loads unconditional).
+// and LDS.  Branch-free: loads unconditional, only the stores predicated.
 template <int HD, bool PR>
 __device__ __forceinline__ void dec_pro_finish(const DecodeAttnParams& a, DecPro& d, int dl, int grp, int64_t poff,
                                                uint16_t* kb, uint16_t* vb, uint16_t (*q_s)[HD],
@@ -344,7 +346,7 @@ __device__ __forceinline__ void attn_decode_mfma2_body(const DecodeAttnParams& a
     // Without the pre-rotation the same holds when the engine keeps the current position's
     // RoPE row (a.rc, tagged with the position): the prologue's loads then need no position
     // either, and a stale tag (a position set some other way) reloads the table row.
-    // (Paged: the pages of a one-step and of a two-step split, one after the other 0.3 us of a launch each, come with the position; the K / V loads themselves, issued
+    // (Paged: the pages of a one-step and of a two-step split, 0.3 us of a launch each one after the other, come with the position; the K / V loads themselves, issued
     // ahead by them, made eight users slower: 3,563 tok/s against 3,624.)
     const bool ahead = PR || a.rc != nullptr;   // uniform: the prologue's loads need no position
     const bool spec = !PG && ahead && a.spec_ok;
@@ -431,7 +433,7 @@ __device__ __forceinline__ void attn_decode_mfma2_body(const DecodeAttnParams& a
     const float inv_scale = 1.0f / scale;
     auto qdiv = [&](float d) {
         const float q = d * inv_scale;
-        if constexpr (HD == 64 || HD == 256) return q;   // sqrt(hd) a power of two: exact
+        if constexpr (HD == 64) return q;   // sqrt(hd) a power of two: exact
         else return fmaf(fmaf(-q, scale, d), inv_scale, q);
     };
     const int nq = a.nq;

@@ -237,7 +237,7 @@ struct PrefillAttnParams {
 // replaces left the workgroup with the last tile 16x the work of the first: 2x the
 // makespan of the balanced split on 256 CUs).  Scores go to the log2 domain once
 // (dot * log2(e) / sqrt(hd)) and are exponentiated with v_exp_f32: the reference build
-// compiles with -use_fast_math (SURVEY §8(c)), i.e. __expf / __fdividef.
+// compiles with -use_fast_math, i.e. __expf / __fdividef.
 template <int HD, bool PG, int NW>
 __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_prefill_mfma2_kernel(PrefillAttnParams a) {
     constexpr int KT = 64;
@@ -427,7 +427,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_prefill_mfma2_k
                 // P = hi + lo: two bf16 parts carry 16 of the 24 mantissa bits of each fp32
                 // probability; the dropped remainder is < 2^-16 of p, a relative error per
                 // P.V product (<= 2^-17) below the fp32 summation-order spread of the
-                // reference's own sum over keys (DESIGN.md §4)
+                // reference's own sum over keys
                 bf16x8_t ph[QG], pl[QG];
 #pragma unroll
                 for (int q = 0; q < QG; q++) {

@@ -81,14 +81,14 @@ __device__ __forceinline__ void db_lds16(__amdgpu_buffer_rsrc_t rs, void* lds, u
 #endif
 }
 
+constexpr int kEpiGated = 5;   // after the QIE_EPI_ values: rows[0] rows as QIE_EPI_F32, then pairs of rows of w[1] and w[2] (lay::GatedP)
+
 // XM: 0 = X in LDS; 8, 16 = X's chunks (of 8 or 16 rows) through the ring.  NV: 16-byte vectors of a row per lane while X is
 // normed (K <= 512 NV), 0: not normed, its rows go to LDS as they are; R: ring slots a wave.
 // F32: rows of fp32 instead (p.K, p.ldx in 16-bit units; the fp32 epilogue, no norm): a 16-byte piece is 4 k, four
 // v_mfma_f32_16x16x4f32 instead of one v_mfma_f32_16x16x32_bf16.  Each of a chunk's 16 instructions has a sum of its own, and
 // these and the waves' meet in pairs: a sum is a chain of K / 128 terms at most, not of K / 8 (the Lugipel design at width 1,024,
 // decode steps against 64 bits: 4.5e-7 to 5.6e-7 of the logits with one chain a wave, 2.6e-7 to 3.4e-7 so; the column-per-wave kernel 3.4e-7 to 4.2e-7).
-constexpr int kEpiGated = 5;   // after the QIE_EPI_ values: rows[0] rows as QIE_EPI_F32, then pairs of rows of w[1] and w[2] (lay::GatedP)
-
 template <int EPI, int XM, int NV, int R, bool F32 = false>
 __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
 #pragma clang fp contract(off)
