@@ -69,7 +69,11 @@ struct DecodeAttnParams {
     // loads need no position, so they go out before it is known.  Null (operator API) or a stale tag: the table row at pos.
     const float* rc;
     int spec_ok;              // the speculative K loads may be issued (see fill_dec_params)
+    // Arguments of 192 bytes, whole lines of the segment that the host writes, take it 0.5 us a launch longer than of 200 (4.8 -> 5.3 us a call of
+    // qie_attention_decode; captured launches the same).  Behind what the kernel reads.
+    int64_t unused = 0;
 };
+static_assert(sizeof(DecodeAttnParams) % 64 != 0, "arguments of the decode attention");
 
 constexpr int kDecMaxSplits = 512;   // 64k keys per (row, kv head)
 
