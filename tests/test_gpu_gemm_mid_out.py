@@ -16,7 +16,8 @@ SHAPES = [(17, 72, 64, 0, 1), (33, 72, 2048, 0, 4), (17, 16500, 64, 1, 1), (64, 
           (301, 9728, 896, 3, 1), (128, 8200, 4096, 3, 3), (131, 11014, 3712, 4, 2), (210, 9278, 6464, 5, 3), (640, 4000, 4096, 6, 2),
           (257, 8338, 11264, 7, 3), (127, 16500, 64, 8, 1), (640, 8200, 448, 9, 1), (395, 10424, 256, 4, 1), (276, 15640, 1152, 4, 1),
           (439, 15744, 512, 5, 1), (213, 22912, 1536, 5, 1), (216, 12496, 5120, 3, 1), (467, 3512, 8192, 3, 2),
-          (104, 16500, 2048, 3, 1), (649, 7496, 1536, 4, 1), (1008, 7600, 2048, 5, 1)]
+          (104, 16500, 2048, 3, 1), (649, 7496, 1536, 4, 1), (1008, 7600, 2048, 5, 1), (393, 4688, 3072, 4, 2),
+          (469, 7088, 8192, 5, 2)]
 
 
 def test_the_shapes_take_their_tiles():
