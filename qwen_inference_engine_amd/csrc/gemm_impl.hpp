@@ -192,6 +192,8 @@ void g8_release(hipStream_t st);
 // k_gemm_mid.hip: the GEMM of a few dozen to about a thousand rows, and of more where its tiles are the faster (mid::choose; *launched = false: not
 // such a shape).  tail: null, or what follows the product.
 int gemm_mid(const qie_linear_args* a, const GemmParams& p, const QkvTail* tail, hipStream_t st, bool* launched);
+// k_gemm_few.hip: the GEMM of small products (few::choose; *launched = false: not such a shape)
+int gemm_few(const qie_linear_args* a, const GemmParams& p, const QkvTail* tail, hipStream_t st, bool* launched);
 // The same for the last columns of a product whose first the 256x256 kernel takes (mid::columns_ahead): always launched.
 int gemm_mid_rest(int epi, const GemmParams& p, hipStream_t st);
 

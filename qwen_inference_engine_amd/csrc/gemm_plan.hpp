@@ -2,6 +2,8 @@
 #pragma once
 
 #include <algorithm>
+#include <cmath>
+#include <cstddef>
 #include <cstdint>
 
 #if defined(__HIPCC__)
@@ -310,5 +312,62 @@ inline int64_t columns_ahead(int64_t M, int64_t cols, int64_t K, int64_t cus, bo
 }
 
 }  // namespace mid
+
+// ---------------------------------------------------------------- k_gemm_few.hip
+namespace few {
+// Times, us, fitted to 20 projections (Qwen2-0.5B / 1.5B / 7B, Qwen3-14B, 1,024 and 2,048 wide ones) at 17 to 1,300 rows, 4,900 launches: up to a workgroup
+// a CU a1 + s1 per k-tile of 64, more a2 + (rounds of the chip) * (f2 + s2 per k-tile), and what the weights take from memory, as the root of their
+// squares' sum; 6.3 % (rms) off.
+struct Time {
+    float a1, s1, a2, f2, s2;
+};
+struct Form {
+    int fi, fj, slots;   // fragments of 16 rows, of 16 columns; chunks of a wave's ring
+    Time t;
+};
+constexpr int WAVES = 4;
+constexpr Form FORMS[] = {
+    {2, 1, 4, {0.f, 0.0884f, 2.95f, 0.294f, 0.0711f}},
+    {2, 2, 2, {0.f, 0.128f, 1.03f, 1.31f, 0.186f}},
+    {2, 4, 2, {1.34f, 0.183f, 0.216f, 2.39f, 0.163f}},
+    {4, 2, 2, {1.05f, 0.175f, 0.504f, 2.48f, 0.15f}},
+    {4, 4, 2, {3.f, 0.226f, 1.47f, 3.15f, 0.212f}},
+};
+constexpr int N_FORMS = sizeof(FORMS) / sizeof(FORMS[0]);
+constexpr std::size_t lds(const Form& f) {   // the rings; behind the loop the waves' sums
+    const std::size_t ring = (std::size_t)WAVES * f.slots * 16 * (f.fi + f.fj) * 128, sums = (std::size_t)WAVES * f.fi * f.fj * 1024;
+    return ring > sums ? ring : sums;
+}
+
+inline float us_of(const Time& t, int64_t workgroups, int per_cu, int64_t nk, bool one_row_tile, int64_t cols, int64_t K, int64_t cus) {
+    const float work = workgroups <= cus ? t.a1 + nk * t.s1 : t.a2 + mid::rounds(workgroups / (float)(cus * per_cu)) * (t.f2 + nk * t.s2);
+    const float weights = (float)cols * K * 2e-6f / (one_row_tile ? 6.42f : 5.92f) + 3.91f;
+    return std::sqrt(work * work + weights * weights);
+}
+inline float us_in(const Form& f, int64_t M, int64_t cols, int64_t K, int64_t parts, int64_t cus) {
+    const int64_t n_mt = (M + 16 * f.fi - 1) / (16 * f.fi), tiles = n_mt * ((cols + 16 * f.fj - 1) / (16 * f.fj));
+    return us_of(f.t, tiles * parts, (int)(160 * 1024 / lds(f)), (K / 64 + parts - 1) / parts, n_mt == 1, cols, K, cus);
+}
+// what the other kernels are expected to take for a product
+inline float others(int64_t M, int64_t cols, int64_t K, int64_t cus) { return std::min(mid::best(M, cols, K, cus).us, g8p::us(M, cols, K, cus)); }
+
+struct Plan {
+    int form;   // -1: not its shape
+    float us;
+};
+// The form that takes a product.  Up to 512 rows, as fitted; gate and up up to 32 (beyond, x is read too often: Qwen2-7B at 64 rows 58.9 us | 60.7,
+// 1,536 -> 2 x 8,960 at 40 rows 18.1 | 20.1).  `ragged`: weight segments that are no multiples of 64 rows, which tiles would cross.
+inline Plan choose(int64_t M, int64_t cols, int64_t K, int64_t cus, bool gated, bool ragged) {
+    Plan best{-1, 1e30f};
+    if (K % 64 != 0 || ragged || M > (gated ? 32 : 512)) return best;
+    if (gated) return {(cols + 63) / 64 <= cus ? 2 : 1, 0.f};
+    for (int c = 0; c < N_FORMS; c++) {
+        if (16 * FORMS[c].fi >= 2 * M && FORMS[c].fi > 2) continue;
+        const float us = us_in(FORMS[c], M, cols, K, 1, cus);
+        if (us < best.us) best = {c, us};
+    }
+    return best.us < .97f * others(M, cols, K, cus) ? best : Plan{-1, 1e30f};
+}
+}  // namespace few
 
 }  // namespace qie

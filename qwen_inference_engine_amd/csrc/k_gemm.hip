@@ -1526,7 +1526,7 @@ static int gemm_with(const qie_linear_args* a, const QkvTail* tail, bool* done, 
         // In this order:
         //   0. more 256x256 tiles than CUs, one weight segment (SwiGLU: two): whole rounds of the phase-interleaved kernel for the first columns and
         //      k_gemm_mid.hip's tiles for the rest, where mid::columns_ahead expects that to be the faster;
-        //   1. K a multiple of 64: k_gemm_mid.hip, unless the next is expected to be faster (mid::choose);
+        //   1. K a multiple of 64: k_gemm_few.hip where it is expected to be the fastest (few::choose), else k_gemm_mid.hip, unless the next is (mid::choose);
         //   2. K a multiple of 64 from 256 on, 256 rows: the phase-interleaved 256x256 kernel, whole where its tiles fill the chip,
         //      or half of it when K is too short to split; split over K otherwise;
         //   3. K an odd multiple of 32, or a split that gets no memory for its slabs, 256 rows: the LDS-DMA kernel, with 256x256 tiles
@@ -1562,7 +1562,8 @@ static int gemm_with(const qie_linear_args* a, const QkvTail* tail, bool* done, 
         // (Qwen2-7B gate/up, us: 301 rows 161 with the 256x256 kernel, 97 with k_gemm_mid.hip; 700 rows 183 against 229)
         if (dev_env("QIE_MID", 1) && force < 0 && !(a->flags & QIE_LINEAR_STREAMK)) {
             bool launched = false;
-            const int rc = gemm_mid(a, p, tail, st, &launched);
+            int rc = dev_env("QIE_FEW", 1) ? gemm_few(a, p, tail, st, &launched) : 0;
+            if (!rc && !launched) rc = gemm_mid(a, p, tail, st, &launched);
             if (done) *done = launched && tail;
             if (rc || launched) return rc;
         }
