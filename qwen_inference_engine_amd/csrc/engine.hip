@@ -21,11 +21,14 @@
 #include <fstream>
 #include <vector>
 
+static int linear_check(const qie_linear_args* a);   // (qie_linear)
+
 namespace qie {
 int gemv(const qie_linear_args* a, hipStream_t st);
 int gemv_rope(const qie_linear_args* a, const int32_t* pos, const float* cs, const float* sn, int hd, int64_t rows,
               hipStream_t st);
 int gemm(const qie_linear_args* a, hipStream_t st);
+int gemm_add_norm(const qie_linear_args* a, const void* norm_w, float eps, int numerics, void* y, hipStream_t st);
 int gemm_qkv(const qie_linear_args* a, const qie_kv_cache* cache, int32_t layer, int32_t len, const float* turns, uint16_t* q,
              hipStream_t st, bool* done);
 bool dec8_applies(const qie_linear_args* a);
@@ -514,6 +517,20 @@ static int row_parallel(qie_batch* b, qie_linear_args& a, uint16_t* x, float* pa
     }
     QIE_TRY(qie_linear(&a, e->stream));
     return e->comm->allreduce_residual_bf16(part, x, n, e->stream);   // one kernel on the peer backend
+}
+
+// A prompt's row-parallel projection and the norm of its rows behind it (k_sum_norm.hip)
+static int row_parallel_norm(qie_batch* b, qie_linear_args& a, uint16_t* x, float* part, int64_t rows, const void* norm_w, uint16_t* y) {
+    qie_engine* e = b->e;
+    const qie_model_spec& s = e->spec;
+    if (use_comm(e)) {
+        QIE_TRY(row_parallel(b, a, x, part, rows));
+        return qie_rmsnorm(x, norm_w, y, rows, s.hidden, s.rms_eps, s.numerics, e->stream);
+    }
+    a.y = x;
+    a.epilogue = QIE_EPI_RESIDUAL;
+    QIE_TRY(::linear_check(&a));
+    return gemm_add_norm(&a, norm_w, s.rms_eps, s.numerics, y, e->stream);
 }
 
 // Batched rows (2 <= M <= 16) of the skinny MFMA kernel (shapes k_decode_bf16.hip and k_decode_fp8.hip do not take): RMSNorm the M rows once into b->xn
@@ -1308,8 +1325,6 @@ void qie_batch_destroy(qie_batch* b) {
     delete b;
 }
 
-static int linear_check(const qie_linear_args* a);
-
 // Prefill of n_seqs prompts of len ids each into slots seq0 .. seq0+n_seqs-1 (ids laid end
 // to end): every GEMM runs once over all n_seqs * len rows, attention and the KV append see
 // the prompts as sequences of rows_per_seq = len, and the head samples the n_seqs last rows
@@ -1403,7 +1418,7 @@ static int prefill_rows(qie_batch* b, int seq0, int n_seqs, const int32_t* ids, 
             continue;
         }
         const qie_layer_weights& L = pf16 ? e->layers_pf[l] : e->layers[l];
-        QIE_TRY(qie_rmsnorm(b->pf_x, L.attn_norm, b->pf_hn, n, H, s.rms_eps, s.numerics, st));
+        if (l == 0) QIE_TRY(qie_rmsnorm(b->pf_x, L.attn_norm, b->pf_hn, n, H, s.rms_eps, s.numerics, st));   // (else the layer before has)
         qie_linear_args a = pf_base();
         a.x = b->pf_hn; a.ldx = H;
         a.w[0] = L.wq; a.w[1] = L.wk; a.w[2] = L.wv;
@@ -1424,8 +1439,7 @@ static int prefill_rows(qie_batch* b, int seq0, int n_seqs, const int32_t* ids, 
         a = pf_base();
         a.x = b->pf_att; a.ldx = QD; a.w[0] = L.wo; a.seg_rows[0] = H;
         a.M = n; a.K = QD; a.N = H; a.ldy = H;
-        QIE_TRY(row_parallel(b, a, b->pf_x, b->pf_part, n));
-        QIE_TRY(qie_rmsnorm(b->pf_x, L.ffn_norm, b->pf_hn, n, H, s.rms_eps, s.numerics, st));
+        QIE_TRY(row_parallel_norm(b, a, b->pf_x, b->pf_part, n, L.ffn_norm, b->pf_hn));
         a = pf_base();
         a.x = b->pf_hn; a.ldx = H; a.w[0] = L.w_gate; a.w[1] = L.w_up; a.seg_rows[0] = I; a.seg_rows[1] = I;
         a.M = n; a.K = H; a.N = I; a.y = b->pf_h; a.ldy = I; a.epilogue = QIE_EPI_SWIGLU;
@@ -1433,7 +1447,8 @@ static int prefill_rows(qie_batch* b, int seq0, int n_seqs, const int32_t* ids, 
         a = pf_base();
         a.x = b->pf_h; a.ldx = I; a.w[0] = L.w_down; a.seg_rows[0] = H;
         a.M = n; a.K = I; a.N = H; a.ldy = H;
-        QIE_TRY(row_parallel(b, a, b->pf_x, b->pf_part, n));
+        if (l + 1 < s.n_layers) QIE_TRY(row_parallel_norm(b, a, b->pf_x, b->pf_part, n, e->layers[l + 1].attn_norm, b->pf_hn));
+        else QIE_TRY(row_parallel(b, a, b->pf_x, b->pf_part, n));
     }
     // position of each last prompt token; finalize advances it to len (the new token).
     for (int z = 0; z < n_seqs; z++) {

@@ -25,6 +25,7 @@ struct QkvTail {
     KvMap km;
 };
 constexpr int kEpiQkv = 4;   // the epilogue that does this: k_gemm.hip's 256x256 kernel and k_gemm_mid.hip's have it
+constexpr int kEpiParts = 6;   // k_gemm_mid.hip, k_gemm_few.hip: every part of K stores its own sums, fp32 rows [part][M][N], for k_sum_norm.hip
 // The last argument of kernels with an epilogue EPI.  As part of every kernel's it moved what lies behind it (the grid's size) to a further line
 // of the argument segment: 0.3 us in each launch.
 struct NoTail {};
@@ -194,6 +195,10 @@ void g8_release(hipStream_t st);
 int gemm_mid(const qie_linear_args* a, const GemmParams& p, const QkvTail* tail, hipStream_t st, bool* launched);
 // k_gemm_few.hip: the GEMM of small products (few::choose; *launched = false: not such a shape)
 int gemm_few(const qie_linear_args* a, const GemmParams& p, const QkvTail* tail, hipStream_t st, bool* launched);
+// One launch of a tile of k_gemm_mid.hip or a form of k_gemm_few.hip, every tile in sk.splitk parts of K whose sums go to sk.slab (kEpiParts).  N a
+// multiple of 4, parts below 2^31 bytes.
+int gemm_mid_parts(const GemmParams& p, int tile, const G8Split& sk, hipStream_t st);
+int gemm_few_parts(const GemmParams& p, int form, const G8Split& sk, hipStream_t st);
 // The same for the last columns of a product whose first the 256x256 kernel takes (mid::columns_ahead): always launched.
 int gemm_mid_rest(int epi, const GemmParams& p, hipStream_t st);
 

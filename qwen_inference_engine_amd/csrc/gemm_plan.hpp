@@ -313,7 +313,7 @@ inline int64_t columns_ahead(int64_t M, int64_t cols, int64_t K, int64_t cus, bo
 
 }  // namespace mid
 
-// ---------------------------------------------------------------- k_gemm_few.hip
+// ---------------------------------------------------------------- k_gemm_few.hip, and products in parts that the norm behind them adds up
 namespace few {
 // Times, us, fitted to 20 projections (Qwen2-0.5B / 1.5B / 7B, Qwen3-14B, 1,024 and 2,048 wide ones) at 17 to 1,300 rows, 4,900 launches: up to a workgroup
 // a CU a1 + s1 per k-tile of 64, more a2 + (rounds of the chip) * (f2 + s2 per k-tile), and what the weights take from memory, as the root of their
@@ -369,5 +369,54 @@ inline Plan choose(int64_t M, int64_t cols, int64_t K, int64_t cus, bool gated, 
     return best.us < .97f * others(M, cols, K, cus) ? best : Plan{-1, 1e30f};
 }
 }  // namespace few
+
+// Products with a residual and a norm behind them (O and down of a prompt's layer) in parts of K whose sums the norm's launch adds up: its blocks read
+// them on all CUs at once, where the last of a tile's workgroups reads the others' one after the other (3 us a part of 128 x 128 outputs).
+namespace apart {
+constexpr few::Time MID[] = {   // k_gemm_mid.hip's tiles, TILES and WIDE
+    {2.09f, 0.252f, 4.09f, 0.f, 0.381f}, {2.9f, 0.416f, 5.39f, 0.f, 0.566f}, {3.33f, 0.398f, 5.73f, 0.f, 0.517f},
+    {5.76f, 0.48f, 8.44f, 0.f, 0.497f}, {6.82f, 0.58f, 8.99f, 0.f, 0.613f}, {6.73f, 0.747f, 6.86f, 0.f, 0.781f},
+    {6.35f, 0.651f, 7.39f, 0.f, 0.629f}, {4.36f, 1.1f, 5.f, 0.f, 1.07f}, {6.17f, 0.566f, 9.87f, 0.f, 0.575f},
+    {5.87f, 0.701f, 8.14f, 0.f, 0.763f}, {4.97f, 0.944f, 7.55f, 0.f, 1.02f}, {3.12f, 1.28f, 3.59f, 2.23f, 1.29f},
+};
+static_assert(sizeof(MID) / sizeof(MID[0]) == mid::N_TILES + mid::N_WIDE, "one tile, one time");
+constexpr int64_t FLOATS = 16 << 20;   // of all parts: what a stream has from the start
+struct Plan {
+    int form, tile, parts;   // k_gemm_few.hip's form, or k_gemm_mid.hip's tile; both -1: one launch each for product and norm
+    float us;                // of both launches
+};
+// the norm's launch with `parts` to add; alone it takes 2.6 and 1.1 for a million values
+inline float sum_us(int64_t M, int64_t N, int64_t parts) { return 2.59f + 1.55e-6f * (float)(parts * M * N); }
+
+// Against product and norm apart, 157 of 190 shapes at 17 to 1,300 rows come here, in 0.85 of their time on the average (the best of all forms and parts: 0.84),
+// 0.70 to 1.03 but for Qwen3-14B down at 1,000 rows (172.7 us | 178.4 at the .95 that 900 rows and more had then).  us: Qwen2-7B down at 113 rows 46.1 | 38.3, 301
+// rows 68.0 | 59.4, O at 301 rows 27.0 | 24.1; Qwen3-14B down at 113 rows 55.8 | 46.1; Qwen2-0.5B down at 113 rows 13.0 | 10.6, O 9.2 | 6.6.  From 700 rows on the
+// parts' bytes take what they give, but where the tiles leave CUs idle (4,864 -> 896 at 800 rows 25.0 | 21.9).
+inline Plan choose(int64_t M, int64_t N, int64_t K, int64_t cus) {
+    Plan best{-1, -1, 1, 1e30f};
+    if (K % 64 != 0 || N % 8 != 0 || M <= 16 || M > 1024) return best;
+    for (int parts = 1; parts <= 16 && parts * M * N <= FLOATS; parts++) {
+        const float sum = sum_us(M, N, parts);
+        for (int c = 0; c < few::N_FORMS && M <= 640 && (parts == 1 || K / 64 >= 4 * parts); c++) {
+            const few::Form& f = few::FORMS[c];
+            if (f.fi > 2 && 16 * f.fi >= 2 * M) continue;
+            const int64_t tiles = ((M + 16 * f.fi - 1) / (16 * f.fi)) * ((N + 16 * f.fj - 1) / (16 * f.fj));
+            if (parts > 1 && tiles * parts > 3 * cus) continue;
+            const float us = few::us_in(f, M, N, K, parts, cus) + sum;
+            if (us < best.us) best = {c, -1, parts, us};
+        }
+        for (int c = 0; c < mid::N_TILES + mid::N_WIDE && parts > 1 && K / 64 >= 2 * parts; c++) {
+            const mid::Tile& t = mid::shape(c);
+            const int64_t n_mt = (M + t.bm - 1) / t.bm, tiles = n_mt * ((N + t.bn - 1) / t.bn);
+            if (t.bm - M >= 64 || tiles * parts > 2 * cus) continue;
+            const float us = few::us_of(MID[c], tiles * parts, t.per_cu, (K / 64 + parts - 1) / parts, n_mt == 1, N, K, cus) + sum;
+            if (us < best.us) best = {-1, c, parts, us};
+        }
+    }
+    const few::Plan whole = few::choose(M, N, K, cus, false, false);
+    const float now = std::min(whole.us, few::others(M, N, K, cus)) + 2.6f + 1.1e-6f * (float)(M * N);
+    return best.us < (M > 700 ? .9f : 1.03f) * now ? best : Plan{-1, -1, 1, 1e30f};
+}
+}  // namespace apart
 
 }  // namespace qie

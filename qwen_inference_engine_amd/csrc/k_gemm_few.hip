@@ -1,6 +1,6 @@
 // k_gemm_few.hip — MFMA bf16 GEMM for prompts whose tiles leave the chip's CUs mostly waiting: a wave has a share of K to itself.
 //
-//   C[M, N] = A[M, K] . W[N, K]^T, fp32 accumulation, the epilogues of k_gemm.hip
+//   C[M, N] = A[M, K] . W[N, K]^T, fp32 accumulation, the epilogues of k_gemm.hip, or the sums of parts of K
 //
 // k_gemm_mid.hip's workgroup walks K together, one barrier per 64 of it: 0.29 us a k-tile for 64 x 64 outputs however little of them there is
 // (Qwen2-0.5B's QKV at 24 rows 6.4 us, 6.2 with its weights already in L2; the launch alone 2.0).  What bounds such a launch is the bytes that one CU
@@ -33,7 +33,7 @@ __device__ __forceinline__ void few_lds16(__amdgpu_buffer_rsrc_t rs, void* lds, 
 
 // FI, FJ: fragments of 16 rows of A, of 16 weight rows (SwiGLU: gate and up in turn); SLOTS of a wave's ring; NT: weights that one row tile reads
 template <int EPI, int FI, int FJ, int SLOTS, bool NT>
-__global__ __launch_bounds__(64 * few::WAVES) void gemm_few_kernel(GemmParams p, int n_mt, int n_nt, TailOf<EPI> tail) {
+__global__ __launch_bounds__(64 * few::WAVES) void gemm_few_kernel(GemmParams p, int n_mt, int n_nt, int parts, float* slab, TailOf<EPI> tail) {
 #pragma clang fp contract(off)
     constexpr int NW = few::WAVES, BM = 16 * FI, BN = 16 * FJ;
     constexpr bool GATED = EPI == QIE_EPI_SWIGLU;
@@ -42,12 +42,13 @@ __global__ __launch_bounds__(64 * few::WAVES) void gemm_few_kernel(GemmParams p,
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int fr = lane & 15, g = lane >> 4;
-    // neighbours (the row tiles of a weight tile) on one XCD
+    // neighbours (the row tiles of a weight tile) on one XCD, parts slowest
     const int nwg = gridDim.x, orig = blockIdx.x, q8 = nwg >> 3, r8 = nwg & 7, xcd = orig & 7;
     const int wid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (orig >> 3);
-    const int nt = quotient(wid, n_mt), mt = wid - nt * n_mt;
+    const int tiles = n_mt * n_nt, part = quotient(wid, tiles), tile = wid - part * tiles, nt = quotient(tile, n_mt), mt = tile - nt * n_mt;
     const int64_t m0 = (int64_t)mt * BM, c0 = (int64_t)nt * (GATED ? BN / 2 : BN);
-    const int chunks = (int)(p.K >> 6), mine = chunks > wave ? (chunks - wave + NW - 1) / NW : 0;   // chunks wave + NW i of this wave
+    const int chunks = (int)(p.K >> 6), kb = quotient(part * chunks, parts), n = quotient((part + 1) * chunks, parts) - kb;
+    const int mine = n > wave ? (n - wave + NW - 1) / NW : 0;   // chunks kb + wave + NW i of this wave
 
     // A's and the weights' rows of the tile as buffers: rows past the end read zeros.  A tile lies in one weight segment (few::choose).
     const int rows = (int)(p.M - m0 < BM ? p.M - m0 : BM);
@@ -80,7 +81,7 @@ __global__ __launch_bounds__(64 * few::WAVES) void gemm_few_kernel(GemmParams p,
     const int a_8 = 8 * (int)p.lda * 2, w_8 = 8 * (int)p.K * 2;   // 8 rows on
     auto load = [&](int slot, int i) {
         const bool on = i < mine;   // uniform; off: nothing is read, so that every wait is a counted one
-        const int k = (wave + NW * i) * 128;
+        const int k = (kb + wave + NW * i) * 128;
         const auto ra = rsrc(a0, on ? a_bytes : 0u), r0 = rsrc(w0, on ? w_bytes : 0u), r1 = GATED ? rsrc(w1, on ? w_bytes : 0u) : r0;
         unsigned char* dst = ring + slot * SLOT;
 #pragma unroll
@@ -151,7 +152,9 @@ __global__ __launch_bounds__(64 * few::WAVES) void gemm_few_kernel(GemmParams p,
             if (row >= p.M || col >= p.N) continue;
             const int64_t to_go = p.N - col;
             uint16_t* dst = p.C + row * p.ldc + col;
-            if constexpr (EPI == QIE_EPI_F32) {
+            if constexpr (EPI == kEpiParts) {
+                *reinterpret_cast<f32x4*>(slab + ((int64_t)part * p.M + row) * p.N + col) = v[0];
+            } else if constexpr (EPI == QIE_EPI_F32) {
                 store_quad_f32(reinterpret_cast<float*>(p.C) + row * p.ldc + col, v[0], p.vec, to_go);
             } else if constexpr (GATED) {
                 float h[4];
@@ -175,7 +178,7 @@ __global__ __launch_bounds__(64 * few::WAVES) void gemm_few_kernel(GemmParams p,
 
 namespace {
 template <int EPI, int FORM, bool NT>
-int few_launch(const GemmParams& p, const TailOf<EPI>& tail, hipStream_t st) {
+int few_launch(const GemmParams& p, int parts, float* slab, const TailOf<EPI>& tail, hipStream_t st) {
     constexpr few::Form F = few::FORMS[FORM];
     constexpr size_t shm = few::lds(F);
     static_assert(shm <= 160 * 1024, "LDS");
@@ -185,27 +188,27 @@ int few_launch(const GemmParams& p, const TailOf<EPI>& tail, hipStream_t st) {
         raised = true;
     }
     const int n_mt = cdiv(p.M, 16 * F.fi), n_nt = cdiv(p.N, (EPI == QIE_EPI_SWIGLU ? 8 : 16) * F.fj);
-    hipLaunchKernelGGL((gemm_few_kernel<EPI, F.fi, F.fj, F.slots, NT>), dim3((unsigned)(n_mt * n_nt)), dim3(64 * few::WAVES), shm, st, p, n_mt, n_nt, tail);
+    hipLaunchKernelGGL((gemm_few_kernel<EPI, F.fi, F.fj, F.slots, NT>), dim3((unsigned)(n_mt * n_nt * parts)), dim3(64 * few::WAVES), shm, st, p, n_mt, n_nt, parts, slab, tail);
     QIE_LAUNCH_CHECK();
     return 0;
 }
 // weights with the non-temporal hint where one row tile reads them (Qwen2-7B gate / up at 24 rows 54.6 -> 48.8 us; where two do they come from memory twice)
 template <int EPI, int FORM>
-int few_one(const GemmParams& p, const TailOf<EPI>& tail, hipStream_t st) {
-    return p.M <= 16 * few::FORMS[FORM].fi ? few_launch<EPI, FORM, true>(p, tail, st) : few_launch<EPI, FORM, false>(p, tail, st);
+int few_one(const GemmParams& p, int parts, float* slab, const TailOf<EPI>& tail, hipStream_t st) {
+    return p.M <= 16 * few::FORMS[FORM].fi ? few_launch<EPI, FORM, true>(p, parts, slab, tail, st) : few_launch<EPI, FORM, false>(p, parts, slab, tail, st);
 }
 template <int EPI>
-int few_run(int form, const GemmParams& p, hipStream_t st, const TailOf<EPI>& tail = {}) {
+int few_run(int form, const GemmParams& p, int parts, float* slab, hipStream_t st, const TailOf<EPI>& tail = {}) {
     static_assert(few::N_FORMS == 5, "forms");
     if constexpr (EPI == QIE_EPI_SWIGLU) {   // (few::choose)
-        return form == 1 ? few_one<EPI, 1>(p, tail, st) : few_one<EPI, 2>(p, tail, st);
+        return form == 1 ? few_one<EPI, 1>(p, parts, slab, tail, st) : few_one<EPI, 2>(p, parts, slab, tail, st);
     } else {
         switch (form) {
-            case 0: return few_one<EPI, 0>(p, tail, st);
-            case 1: return few_one<EPI, 1>(p, tail, st);
-            case 2: return few_one<EPI, 2>(p, tail, st);
-            case 3: return few_one<EPI, 3>(p, tail, st);
-            default: return few_one<EPI, 4>(p, tail, st);
+            case 0: return few_one<EPI, 0>(p, parts, slab, tail, st);
+            case 1: return few_one<EPI, 1>(p, parts, slab, tail, st);
+            case 2: return few_one<EPI, 2>(p, parts, slab, tail, st);
+            case 3: return few_one<EPI, 3>(p, parts, slab, tail, st);
+            default: return few_one<EPI, 4>(p, parts, slab, tail, st);
         }
     }
 }
@@ -216,13 +219,15 @@ int gemm_few(const qie_linear_args* a, const GemmParams& p, const QkvTail* tail,
     const few::Plan pl = few::choose(a->M, gated ? 2 * a->N : a->N, a->K, device_cu_count(), gated, a->seg_rows[0] != a->N && (a->seg_rows[0] % 64 || a->seg_rows[1] % 64));
     *launched = pl.form >= 0 && mid::strides_fit(a->ldx, a->ldy);
     if (!*launched) return 0;
-    if (tail) return few_run<kEpiQkv>(pl.form, p, st, *tail);
+    if (tail) return few_run<kEpiQkv>(pl.form, p, 1, nullptr, st, *tail);
     switch (a->epilogue) {
-        case QIE_EPI_SWIGLU: return few_run<QIE_EPI_SWIGLU>(pl.form, p, st);
-        case QIE_EPI_RESIDUAL: return few_run<QIE_EPI_RESIDUAL>(pl.form, p, st);
-        case QIE_EPI_F32: return few_run<QIE_EPI_F32>(pl.form, p, st);
-        default: return few_run<QIE_EPI_STORE>(pl.form, p, st);
+        case QIE_EPI_SWIGLU: return few_run<QIE_EPI_SWIGLU>(pl.form, p, 1, nullptr, st);
+        case QIE_EPI_RESIDUAL: return few_run<QIE_EPI_RESIDUAL>(pl.form, p, 1, nullptr, st);
+        case QIE_EPI_F32: return few_run<QIE_EPI_F32>(pl.form, p, 1, nullptr, st);
+        default: return few_run<QIE_EPI_STORE>(pl.form, p, 1, nullptr, st);
     }
 }
+
+int gemm_few_parts(const GemmParams& p, int form, const G8Split& sk, hipStream_t st) { return few_run<kEpiParts>(form, p, sk.splitk, sk.slab, st); }
 
 }  // namespace qie

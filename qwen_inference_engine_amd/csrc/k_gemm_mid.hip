@@ -268,6 +268,19 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
             for (int j = 0; j < FJ; j++) res[i][j] = res[i][j] + ex[(((wave ^ 4) * FR + i) * FJ + j) * 64 + lane];
     }
 
+    if constexpr (EPI == kEpiParts) {   // rows past M lie behind the part's end, columns past N are moved there
+        const int ldp = (int)p.N * 4;
+        const auto rs = __builtin_amdgcn_make_buffer_rsrc(sk.slab + (int64_t)part * p.M * p.N, (short)0, (int)p.M * ldp, 0x00020000);
+#pragma unroll
+        for (int j = 0; j < FJ; j++) {
+            const int col = (int)nt * BN + wn * TN + 16 * j + 4 * g;
+#pragma unroll
+            for (int i = 0; i < FR; i++)
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_g8, res[i][j]), rs, col < p.N ? ((int)m0 + wrow + 16 * i) * ldp + col * 4 : 1 << 31, 0, 0);
+        }
+        return;
+    }
+
     // The tile's part of C as a buffer: rows past M lie behind its end, and so do columns past N, moved there by `at`; loads from there give 0,
     // stores do nothing.
     constexpr int OUT_BN = EPI == QIE_EPI_SWIGLU ? BN / 2 : BN, SZ = EPI == QIE_EPI_F32 ? 4 : 2, OUTSIDE = 1 << 31;
@@ -311,7 +324,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(GemmParams p, int n_mt, i
     constexpr bool BOTH = FR * FJ <= 16;
     if constexpr (EPI == QIE_EPI_RESIDUAL && BOTH) load_before();
 
-    constexpr bool SPLITS = BN != 160;   // (mid::WIDE: whole only)
+    constexpr bool SPLITS = BN != 160;   // (mid::WIDE: whole, or in parts that another launch adds up)
     if (SPLITS && parts > 1) {   // uniform.  A wave's share of the tile meets by itself: no wave waits for the others of its workgroup
         constexpr int SLAB = BM * BN;   // floats
         const int64_t tb = (int64_t)ct * parts;
@@ -426,7 +439,7 @@ int launch_mid_t(const GemmParams& p, const mid::Plan& pl, const G8Split& sk, co
         QIE_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
         raised = true;
     }
-    const int tiles = pl.n_mt * pl.n_nt, whole = sk.splitk > 1 ? pl.whole : tiles;
+    const int tiles = pl.n_mt * pl.n_nt, whole = EPI == kEpiParts ? 0 : sk.splitk > 1 ? pl.whole : tiles;
     hipLaunchKernelGGL((gemm_mid_kernel<EPI, BM, BN, SA, SW, KW, TURNS>), dim3((unsigned)(whole + (tiles - whole) * sk.splitk)), dim3(512), shm,
                        st, p, pl.n_mt, pl.n_nt, band_height(pl.n_mt, BM, BN, 32 * mid::shape(pl.tile).per_cu), whole, sk, tail);
     QIE_LAUNCH_CHECK();
@@ -482,6 +495,11 @@ int gemm_mid(const qie_linear_args* a, const GemmParams& p, const QkvTail* tail,
     if (pl.tile < 0 || !mid::strides_fit(a->ldx, a->ldy)) return 0;
     *launched = true;
     return run_mid(a->epilogue, p, pl, tail, st);
+}
+
+int gemm_mid_parts(const GemmParams& p, int tile, const G8Split& sk, hipStream_t st) {
+    mid::Plan pl{tile, 0, sk.splitk, (int)cdiv(p.M, mid::shape(tile).bm), (int)cdiv(p.N, mid::shape(tile).bn), 0.f};
+    return launch_mid<kEpiParts>(p, pl, sk, st);
 }
 
 int gemm_mid_rest(int epi, const GemmParams& p, hipStream_t st) {
