@@ -28,6 +28,8 @@ int gemv(const qie_linear_args* a, hipStream_t st);
 int gemv_rope(const qie_linear_args* a, const int32_t* pos, const float* cs, const float* sn, int hd, int64_t rows,
               hipStream_t st);
 int gemm(const qie_linear_args* a, hipStream_t st);
+int prompt_attention(const void* q, int64_t M, const int32_t* pos, int32_t rows_per_seq, const qie_kv_cache* cache, int32_t layer, int32_t n_heads, void* out, void* ws,
+                     hipStream_t st);
 int gemm_add_norm(const qie_linear_args* a, const void* norm_w, float eps, int numerics, void* y, hipStream_t st);
 int gemm_qkv(const qie_linear_args* a, const qie_kv_cache* cache, int32_t layer, int32_t len, const float* turns, uint16_t* q,
              hipStream_t st, bool* done);
@@ -1398,7 +1400,7 @@ static int prefill_rows(qie_batch* b, int seq0, int n_seqs, const int32_t* ids, 
             QIE_TRY(qie_linear(&a, st));
             QIE_TRY(qie_qkv_post(b->pf_qkv, n, b->pf_pos, len, L.q_norm, L.k_norm, e->rope_cos, e->rope_sin, sh.nq,
                                  &cache, l, s.rms_eps, s.numerics, b->pf_q, st));
-            QIE_TRY(qie_attention(b->pf_q, n, b->pf_pos, len, &cache, l, sh.nq, b->pf_att, b->pf_attn_ws, st));
+            QIE_TRY(prompt_attention(b->pf_q, n, b->pf_pos, len, &cache, l, sh.nq, b->pf_att, b->pf_attn_ws, st));
             a = lin_proj(e);
             QIE_TRY(mx_in(a, b->pf_att, QD));
             a.w[0] = L.wo; a.seg_rows[0] = H;
@@ -1435,7 +1437,7 @@ static int prefill_rows(qie_batch* b, int seq0, int n_seqs, const int32_t* ids, 
         if (!post)
             QIE_TRY(qie_qkv_post(b->pf_qkv, n, b->pf_pos, len, L.q_norm, L.k_norm, e->rope_cos, e->rope_sin, sh.nq,
                                  &cache, l, s.rms_eps, s.numerics, b->pf_q, st));
-        QIE_TRY(qie_attention(b->pf_q, n, b->pf_pos, len, &cache, l, sh.nq, b->pf_att, b->pf_attn_ws, st));
+        QIE_TRY(prompt_attention(b->pf_q, n, b->pf_pos, len, &cache, l, sh.nq, b->pf_att, b->pf_attn_ws, st));
         a = pf_base();
         a.x = b->pf_att; a.ldx = QD; a.w[0] = L.wo; a.seg_rows[0] = H;
         a.M = n; a.K = QD; a.N = H; a.ldy = H;

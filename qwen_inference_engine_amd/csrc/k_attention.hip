@@ -238,7 +238,10 @@ struct PrefillAttnParams {
 // makespan of the balanced split on 256 CUs).  Scores go to the log2 domain once
 // (dot * log2(e) / sqrt(hd)) and are exponentiated with v_exp_f32: the reference build
 // compiles with -use_fast_math, i.e. __expf / __fdividef.
-template <int HD, bool PG, int NW>
+//
+// NP: bf16 parts of a probability, 2 or (prompts of less than 32 rows) all 24 bits in 3.  Those prompts had the kernel of a row and a key head a
+// workgroup, which keeps probabilities in fp32: Qwen2-0.5B at 24 rows 13.3 us against 5.8.
+template <int HD, bool PG, int NW, int NP = 2>
 __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_prefill_mfma2_kernel(PrefillAttnParams a) {
     constexpr int KT = 64;
     constexpr int CPR = HD / 8;
@@ -428,17 +431,17 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_prefill_mfma2_k
                 // probability; the dropped remainder is < 2^-16 of p, a relative error per
                 // P.V product (<= 2^-17) below the fp32 summation-order spread of the
                 // reference's own sum over keys
-                bf16x8_t ph[QG], pl[QG];
+                bf16x8_t pb[QG][NP];
 #pragma unroll
                 for (int q = 0; q < QG; q++) {
                     if (!ON[q]) continue;
                     float e8[8];
 #pragma unroll
                     for (int jj = 0; jj < 8; jj++) e8[jj] = pv[q][2 * c + (jj >> 2)][jj & 3];
-                    uint4 pp[2];
-                    split_bf16x8<2>(e8, pp);
-                    ph[q] = __builtin_bit_cast(bf16x8_t, pp[0]);
-                    pl[q] = __builtin_bit_cast(bf16x8_t, pp[1]);
+                    uint4 pp[NP];
+                    split_bf16x8<NP>(e8, pp);
+#pragma unroll
+                    for (int k = 0; k < NP; k++) pb[q][k] = __builtin_bit_cast(bf16x8_t, pp[k]);
                 }
 #pragma unroll
                 for (int d = 0; d < DT; d++) {
@@ -454,8 +457,8 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_prefill_mfma2_k
 #pragma unroll
                     for (int q = 0; q < QG; q++) {
                         if (!ON[q]) continue;
-                        oacc[q][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ph[q], vb8, oacc[q][d], 0, 0, 0);
-                        oacc[q][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl[q], vb8, oacc[q][d], 0, 0, 0);
+#pragma unroll
+                        for (int k = 0; k < NP; k++) oacc[q][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pb[q][k], vb8, oacc[q][d], 0, 0, 0);
                     }
                 }
             }
@@ -619,9 +622,9 @@ int64_t qie_attention_workspace_bytes(int64_t M, int32_t n_heads, int32_t head_d
     return M * n_heads * (int64_t)ns * (head_dim + 2) * 4;
 }
 
-int qie_attention(const void* q, int64_t M, const int32_t* pos, int32_t rows_per_seq,
-                  const qie_kv_cache* cache, int32_t layer, int32_t n_heads, void* out, void* ws,
-                  void* stream) {
+// ordered: no row of a sequence comes before an earlier one (of 32 rows and more none does)
+static int attention(const void* q, int64_t M, const int32_t* pos, int32_t rows_per_seq, const qie_kv_cache* cache, int32_t layer, int32_t n_heads, void* out, void* ws,
+                     void* stream, bool ordered) {
     QIE_REQUIRE(q && pos && cache && cache->k && cache->v && out && M >= 0 && rows_per_seq > 0,
                 "qie_attention: bad arguments");
     QIE_REQUIRE(cache->head_dim == 64 || cache->head_dim == 128,
@@ -630,7 +633,7 @@ int qie_attention(const void* q, int64_t M, const int32_t* pos, int32_t rows_per
                 "qie_attention: n_heads/n_kv_heads must be an integer <= %d", kMaxGroup);
     QIE_REQUIRE(layer >= 0 && layer < cache->n_layers, "qie_attention: bad layer");
     if (M == 0) return 0;
-    if (rows_per_seq >= 32 && M % rows_per_seq == 0) {
+    if (rows_per_seq >= (ordered ? 2 : 32) && M % rows_per_seq == 0) {
         PrefillAttnParams pa;
         pa.q = (const uint16_t*)q;
         pa.pos = pos;
@@ -649,14 +652,17 @@ int qie_attention(const void* q, int64_t M, const int32_t* pos, int32_t rows_per
         const bool pg = pa.km.table != nullptr;
         // balanced causal split: ceil(ceil(R / 16) / 2) group pairs, NW per workgroup
         const int npair = ((rows_per_seq + 15) / 16 + 1) / 2;
-        const int nw = prefill_attn_waves(npair, n_heads * (M / rows_per_seq), rows_per_seq, device_cu_count());
+        const bool few = rows_per_seq < 32;
+        const int nw = few ? 2 : prefill_attn_waves(npair, n_heads * (M / rows_per_seq), rows_per_seq, device_cu_count());
         dim3 g2((unsigned)((npair + nw - 1) / nw), (unsigned)n_heads, (unsigned)(M / rows_per_seq));
         auto pick = [&](auto w) {
             constexpr int NW = decltype(w)::value;
             return cache->head_dim == 128 ? (pg ? attn_prefill_mfma2_kernel<128, true, NW> : attn_prefill_mfma2_kernel<128, false, NW>)
                                           : (pg ? attn_prefill_mfma2_kernel<64, true, NW> : attn_prefill_mfma2_kernel<64, false, NW>);
         };
-        auto k2 = nw == 8 ? pick(std::integral_constant<int, 8>{}) : nw == 4 ? pick(std::integral_constant<int, 4>{}) : pick(std::integral_constant<int, 2>{});
+        auto k2 = few ? (cache->head_dim == 128 ? (pg ? attn_prefill_mfma2_kernel<128, true, 2, 3> : attn_prefill_mfma2_kernel<128, false, 2, 3>)
+                                                : (pg ? attn_prefill_mfma2_kernel<64, true, 2, 3> : attn_prefill_mfma2_kernel<64, false, 2, 3>))
+                : nw == 8 ? pick(std::integral_constant<int, 8>{}) : nw == 4 ? pick(std::integral_constant<int, 4>{}) : pick(std::integral_constant<int, 2>{});
         hipLaunchKernelGGL(k2, g2, dim3(64 * nw), shm, (hipStream_t)stream, pa);
         QIE_LAUNCH_CHECK();
         return 0;
@@ -692,6 +698,12 @@ int qie_attention(const void* q, int64_t M, const int32_t* pos, int32_t rows_per
     }
     QIE_LAUNCH_CHECK();
     return 0;
+}
+
+int qie_attention(const void* q, int64_t M, const int32_t* pos, int32_t rows_per_seq,
+                  const qie_kv_cache* cache, int32_t layer, int32_t n_heads, void* out, void* ws,
+                  void* stream) {
+    return attention(q, M, pos, rows_per_seq, cache, layer, n_heads, out, ws, stream, false);
 }
 
 int qie_debug_tr16_probe(int32_t* out_dev) {
@@ -735,3 +747,12 @@ int qie_attention_decode(const void* qkv, int64_t B, const int32_t* pos, const v
 
 }  // extern "C"
 
+namespace qie {
+
+// qie_attention of prompts: rows of a sequence in the order of their positions
+int prompt_attention(const void* q, int64_t M, const int32_t* pos, int32_t rows_per_seq, const qie_kv_cache* cache, int32_t layer, int32_t n_heads, void* out, void* ws,
+                     hipStream_t st) {
+    return attention(q, M, pos, rows_per_seq, cache, layer, n_heads, out, ws, st, true);
+}
+
+}  // namespace qie
