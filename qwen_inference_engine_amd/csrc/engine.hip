@@ -568,6 +568,39 @@ static int dbg_snap(qie_batch* b, int slot) {
     return 0;
 }
 
+// Layer l behind its attention, for up to 16 rows: O and the feed-forward, into the residual rows x
+static int enqueue_layer_rest(qie_batch* b, int l, const uint16_t* att, uint16_t* x, uint16_t* h, float* part, int64_t rows) {
+    qie_engine* e = b->e;
+    const qie_model_spec& s = e->spec;
+    const qie_layer_weights& L = e->layers[l];
+    const int64_t H = s.hidden, QD = (int64_t)e->sh.nq * s.head_dim, I = e->sh.ffn;
+    qie_linear_args a = lin_proj(e);
+    a.x = att; a.ldx = QD;
+    a.w[0] = L.wo; a.seg_rows[0] = H;
+    a.M = rows; a.K = QD; a.N = H;
+    a.ldy = H;
+    QIE_TRY(row_parallel(b, a, x, part, rows));
+    QIE_TRY(dbg_snap(b, 2 * l + 1));
+
+    a = lin_proj(e);
+    a.x = x; a.ldx = H;
+    a.w[0] = L.w_gate; a.w[1] = L.w_up; a.seg_rows[0] = I; a.seg_rows[1] = I;
+    a.M = rows; a.K = H; a.N = I;
+    a.y = h; a.ldy = I;
+    a.epilogue = QIE_EPI_SWIGLU;
+    a.norm_w = L.ffn_norm; a.norm_eps = s.rms_eps; a.numerics = s.numerics;
+    QIE_TRY(prenorm(b, a, rows));
+    QIE_TRY(gemv(&a, e->stream));
+
+    a = lin_proj(e);
+    a.x = h; a.ldx = I;
+    a.w[0] = L.w_down; a.seg_rows[0] = H;
+    a.M = rows; a.K = I; a.N = H;
+    a.ldy = H;
+    QIE_TRY(row_parallel(b, a, x, part, rows));
+    return dbg_snap(b, 2 * l + 2);
+}
+
 static int enqueue_layer_decode(qie_batch* b, int l) {
     qie_engine* e = b->e;
     const qie_model_spec& s = e->spec;
@@ -597,31 +630,7 @@ static int enqueue_layer_decode(qie_batch* b, int l) {
                                          b->att, b->dec_ws, st);
     set_decode_rope_cur(nullptr);
     QIE_TRY(arc);
-    a = lin_proj(e);
-    a.x = b->att; a.ldx = QD;
-    a.w[0] = L.wo; a.seg_rows[0] = H;
-    a.M = B; a.K = QD; a.N = H;
-    a.ldy = H;
-    QIE_TRY(row_parallel(b, a, b->x_res, b->part, B));
-    QIE_TRY(dbg_snap(b, 2 * l + 1));
-
-    a = lin_proj(e);
-    a.x = b->x_res; a.ldx = H;
-    a.w[0] = L.w_gate; a.w[1] = L.w_up; a.seg_rows[0] = I; a.seg_rows[1] = I;
-    a.M = B; a.K = H; a.N = I;
-    a.y = b->h; a.ldy = I;
-    a.epilogue = QIE_EPI_SWIGLU;
-    a.norm_w = L.ffn_norm; a.norm_eps = s.rms_eps; a.numerics = s.numerics;
-    QIE_TRY(prenorm(b, a, B));
-    QIE_TRY(gemv(&a, st));
-
-    a = lin_proj(e);
-    a.x = b->h; a.ldx = I;
-    a.w[0] = L.w_down; a.seg_rows[0] = H;
-    a.M = B; a.K = I; a.N = H;
-    a.ldy = H;
-    QIE_TRY(row_parallel(b, a, b->x_res, b->part, B));
-    return dbg_snap(b, 2 * l + 2);
+    return enqueue_layer_rest(b, l, b->att, b->x_res, b->h, b->part, B);
 }
 
 static bool is_greedy(const qie_sampling* s) { return !s || s->top_k <= 1 || !(s->temperature > 0.f); }
@@ -720,20 +729,7 @@ static bool prefill_mx(const qie_engine* e) {
 }
 
 static int ensure_prefill_scratch(qie_batch* b, int64_t n) {
-    if (n <= b->pf_rows) {
-        // rows fit; the attention workspace is not monotone in n (<= 8 rows run the split
-        // kernel with partials, longer prompts need none), so size it for this n
-        const qie_model_spec& s = b->e->spec;
-        const int64_t ws = qie_attention_workspace_bytes(n, b->e->sh.nq, s.head_dim, b->max_ctx);
-        if (ws > b->pf_attn_ws_bytes) {
-            hipFree(b->pf_attn_ws);
-            b->pf_attn_ws = nullptr;
-            b->pf_attn_ws_bytes = 0;
-            QIE_TRY(dmalloc(&b->pf_attn_ws, (size_t)ws));
-            b->pf_attn_ws_bytes = ws;
-        }
-        return 0;
-    }
+    if (n <= b->pf_rows) return 0;
     const qie_model_spec& s = b->e->spec;
     const TpShard& sh = b->e->sh;
     const int64_t H = s.hidden, QD = (int64_t)sh.nq * s.head_dim, KD = (int64_t)sh.nkv * s.head_dim;
@@ -759,11 +755,8 @@ static int ensure_prefill_scratch(qie_batch* b, int64_t n) {
     }
     QIE_TRY(dmalloc((void**)&b->pf_pos, n * 4));
     QIE_TRY(dmalloc((void**)&b->pf_ids, n * 4));
-    b->pf_attn_ws = nullptr;
-    b->pf_attn_ws_bytes = 0;
-    int64_t ws = qie_attention_workspace_bytes(n, sh.nq, s.head_dim, b->max_ctx);
-    QIE_TRY(dmalloc(&b->pf_attn_ws, (size_t)ws));
-    b->pf_attn_ws_bytes = ws;
+    // attention of prompts needs a workspace only for one row of each: prompts of one token, and the last rows in the last layer
+    QIE_TRY(dmalloc(&b->pf_attn_ws, (size_t)qie_attention_workspace_bytes(b->B, sh.nq, s.head_dim, b->max_ctx)));
     b->pf_rows = n;
     return 0;
 }
@@ -1327,6 +1320,13 @@ void qie_batch_destroy(qie_batch* b) {
     delete b;
 }
 
+// the last of every `len` rows of x and q, one behind the other
+__global__ void last_rows_kernel(const uint4* __restrict__ x, uint4* __restrict__ xl, int64_t H8, const uint4* __restrict__ q, uint4* __restrict__ ql, int64_t Q8, int len) {
+    const int64_t z = blockIdx.x;
+    for (int64_t i = threadIdx.x; i < H8; i += blockDim.x) xl[z * H8 + i] = x[z * len * H8 + i];
+    for (int64_t i = threadIdx.x; i < Q8; i += blockDim.x) ql[z * Q8 + i] = q[z * len * Q8 + i];
+}
+
 // Prefill of n_seqs prompts of len ids each into slots seq0 .. seq0+n_seqs-1 (ids laid end
 // to end): every GEMM runs once over all n_seqs * len rows, attention and the KV append see
 // the prompts as sequences of rows_per_seq = len, and the head samples the n_seqs last rows
@@ -1387,6 +1387,16 @@ static int prefill_rows(qie_batch* b, int seq0, int n_seqs, const int32_t* ids, 
         a.flags |= QIE_LINEAR_ACT_FP8;
         return 0;
     };
+    // position of each last prompt token; finalize advances it to len (the new token).
+    for (int z = 0; z < n_seqs; z++) {
+        hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(64), 0, st, seq0 + z, len - 1, 0,
+                           ids[(int64_t)z * len + len - 1], b->d_pos, b->d_step, b->d_hist, b->max_ctx,
+                           (const uint4*)e->w.embed, (uint4*)b->x_res, (int64_t)H / 8, 0, rope_cur_args(b));
+        QIE_LAUNCH_CHECK();
+    }
+    // What follows the prompts is made of their last rows: behind the last layer's keys and values only those go on
+    const bool last_rows = !mx && len > 1;
+    const uint16_t* last = b->pf_x + (int64_t)(len - 1) * H;
     for (int l = 0; l < s.n_layers; l++) {
         if (mx) {   // every projection on fp8 codes x fp8 weights (e->layers: the fp8 arena)
             const qie_layer_weights& L = e->layers[l];
@@ -1437,6 +1447,26 @@ static int prefill_rows(qie_batch* b, int seq0, int n_seqs, const int32_t* ids, 
         if (!post)
             QIE_TRY(qie_qkv_post(b->pf_qkv, n, b->pf_pos, len, L.q_norm, L.k_norm, e->rope_cos, e->rope_sin, sh.nq,
                                  &cache, l, s.rms_eps, s.numerics, b->pf_q, st));
+        if (last_rows && l + 1 == s.n_layers) {
+            // (attention of a short prompt's rows takes less than the general kernel of its last: 301 rows 13 us | 25, 2,048 rows 70 | 33)
+            const bool all = len < 512;
+            if (all) QIE_TRY(prompt_attention(b->pf_q, n, b->pf_pos, len, &cache, l, sh.nq, b->pf_att, b->pf_attn_ws, st));
+            uint16_t* x = b->pf_x + (int64_t)(len - 1) * H;
+            const uint16_t* att = (all ? b->pf_att : b->pf_q) + (int64_t)(len - 1) * QD;
+            if (n_seqs > 1) {   // packed
+                hipLaunchKernelGGL(last_rows_kernel, dim3(n_seqs), dim3(256), 0, st, (const uint4*)x, (uint4*)b->pf_hn, H / 8, (const uint4*)att, (uint4*)b->pf_qkv, QD / 8, len);
+                QIE_LAUNCH_CHECK();
+                x = b->pf_hn;
+                att = b->pf_qkv;
+            }
+            if (!all) {
+                QIE_TRY(qie_attention(att, n_seqs, b->d_pos + seq0, 1, &cache, l, sh.nq, b->pf_att, b->pf_attn_ws, st));
+                att = b->pf_att;
+            }
+            QIE_TRY(enqueue_layer_rest(b, l, att, x, b->pf_h, b->pf_part, n_seqs));
+            last = x;
+            break;
+        }
         QIE_TRY(prompt_attention(b->pf_q, n, b->pf_pos, len, &cache, l, sh.nq, b->pf_att, b->pf_attn_ws, st));
         a = pf_base();
         a.x = b->pf_att; a.ldx = QD; a.w[0] = L.wo; a.seg_rows[0] = H;
@@ -1452,15 +1482,7 @@ static int prefill_rows(qie_batch* b, int seq0, int n_seqs, const int32_t* ids, 
         if (l + 1 < s.n_layers) QIE_TRY(row_parallel_norm(b, a, b->pf_x, b->pf_part, n, e->layers[l + 1].attn_norm, b->pf_hn));
         else QIE_TRY(row_parallel(b, a, b->pf_x, b->pf_part, n));
     }
-    // position of each last prompt token; finalize advances it to len (the new token).
-    for (int z = 0; z < n_seqs; z++) {
-        hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(64), 0, st, seq0 + z, len - 1, 0,
-                           ids[(int64_t)z * len + len - 1], b->d_pos, b->d_step, b->d_hist, b->max_ctx,
-                           (const uint4*)e->w.embed, (uint4*)b->x_res, (int64_t)H / 8, 0, rope_cur_args(b));
-        QIE_LAUNCH_CHECK();
-    }
-    const uint16_t* last = b->pf_x + (int64_t)(len - 1) * H;
-    if (n_seqs > 1) {   // the last rows, packed (the head's pre-norm reads contiguous rows)
+    if (n_seqs > 1 && !last_rows) {   // the last rows, packed (the head's pre-norm reads contiguous rows)
         QIE_HIP(hipMemcpy2DAsync(b->pf_hn, (size_t)H * 2, last, (size_t)len * H * 2, (size_t)H * 2, n_seqs,
                                  hipMemcpyDeviceToDevice, st));
         last = b->pf_hn;

@@ -100,7 +100,6 @@ struct qie_batch {
     int32_t *pf_pos = nullptr, *pf_ids = nullptr;
     uint8_t *pf_q8 = nullptr, *pf_e8 = nullptr;   // fp8 prefill (opts.prefill_fp8): codes [rows][max K], exps [rows]
     void* pf_attn_ws = nullptr;
-    int64_t pf_attn_ws_bytes = 0;   // the split workspace depends on n (short prompts split), not on n <= pf_rows
     // paged KV (qie_batch_create_paged): pool pages of page_tokens tokens, block table
     // [B][max_pages] on device and host, free list, pages held per slot
     int page_tokens = 0, max_pages = 0, n_pages = 0;
