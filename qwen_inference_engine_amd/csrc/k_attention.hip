@@ -241,13 +241,16 @@ struct PrefillAttnParams {
 //
 // NP: bf16 parts of a probability, 2 or (prompts of less than 32 rows) all 24 bits in 3.  Those prompts had the kernel of a row and a key head a
 // workgroup, which keeps probabilities in fp32: Qwen2-0.5B at 24 rows 13.3 us against 5.8.
-template <int HD, bool PG, int NW, int NP = 2>
-__global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_prefill_mfma2_kernel(PrefillAttnParams a) {
+//
+// QG: row groups of a wave.  2: a pair, so that every wave has the same work; some 220 registers, two waves a SIMD.  1: half the registers and twice the
+// waves, which hide each other's waits (a tile of a group takes 1,100 clocks of issue and 768 of matrix work, and 3,000 a wave with two waves a
+// SIMD); the latest groups, with the most keys, go first.  prefill_attn_plan has both sides.
+template <int HD, bool PG, int NW, int NP = 2, int QG = 2>
+__global__ __launch_bounds__(64 * NW, QG == 1 ? 4 : NW == 8 ? 1 : 2) void attn_prefill_mfma2_kernel(PrefillAttnParams a) {
     constexpr int KT = 64;
     constexpr int CPR = HD / 8;
     constexpr int KSTEPS = HD / 32;
     constexpr int DT = HD / 16;
-    constexpr int QG = 2;                  // 16-row query groups per wave
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     uint16_t* Ks = reinterpret_cast<uint16_t*>(smem);
     uint16_t* Vs = reinterpret_cast<uint16_t*>(smem + 2 * KT * HD * 2);
@@ -258,7 +261,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_prefill_mfma2_k
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int fr = lane & 15, g = lane >> 4;
-    const int h = blockIdx.y, seq = blockIdx.z;
+    const int blk = QG == 2 ? blockIdx.x : blockIdx.z, h = QG == 2 ? blockIdx.y : blockIdx.x, seq = QG == 2 ? blockIdx.z : blockIdx.y;
     const int R = a.rows_per_seq;
     const int ngr = (R + 15) / 16, npair = (ngr + 1) / 2;
     const int64_t row0 = (int64_t)seq * R;
@@ -266,14 +269,20 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_prefill_mfma2_k
     const int64_t head_off = kv_run_off(a.km, (int64_t)a.layer * a.nkv + kvh, HD);
     const uint16_t* kb = a.kc + head_off;
     const uint16_t* vb = a.vc + head_off;
-    // this wave's groups: pair j = (j, ngr-1-j); the workgroup's latest row is wave 0's
-    // second group (positions are non-decreasing within a sequence)
-    const int j = blockIdx.x * NW + wave;
-    const int grp[QG] = {j, ngr - 1 - j};
+    // this wave's groups: pair j = (j, ngr-1-j), or group ngr-1-j; the workgroup's latest row is wave 0's
+    // (last) group's (positions are non-decreasing within a sequence)
+    const int j = blk * NW + wave;
+    int grp[QG];
     bool gact[QG];
-    gact[0] = j < npair;
-    gact[1] = j < npair && grp[1] != j;
-    const int kmax = a.pos[row0 + min(16 * (ngr - 1 - (int)blockIdx.x * NW) + 15, R - 1)];
+    grp[QG - 1] = ngr - 1 - j;
+    if constexpr (QG == 2) {
+        grp[0] = j;
+        gact[0] = j < npair;
+        gact[1] = j < npair && grp[1] != j;
+    } else {
+        gact[0] = j < ngr;
+    }
+    const int kmax = a.pos[row0 + min(16 * (ngr - 1 - blk * NW) + 15, R - 1)];
     const int nkt = kmax / KT + 1;
 
     int qpos[QG], gpos[QG], gmin[QG];
@@ -349,7 +358,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_prefill_mfma2_k
     // s_and_saveexec / s_cbranch_execz / s_or_b64), and — unlike a three-way branch inside
     // one loop — the accumulators need no register copies where the cases meet.
     auto tile = [&](const int kt, const uint16_t* K, const uint16_t* Vt, auto q0c, auto q1c) {
-            constexpr bool ON[QG] = {decltype(q0c)::value, decltype(q1c)::value};
+            constexpr bool ON[2] = {decltype(q0c)::value, decltype(q1c)::value};
             f32x4_t sacc[QG][4];
 #pragma unroll
             for (int t = 0; t < 4; t++) {
@@ -477,10 +486,14 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : 2) void attn_prefill_mfma2_k
     };
     // tiles each group takes: kt * KT <= gpos (gpos = -1: none); gpos[1] >= gpos[0]
     const int nkt0 = gpos[0] >= 0 ? min(nkt, gpos[0] / KT + 1) : 0;
-    const int nkt1 = gpos[1] >= 0 ? min(nkt, gpos[1] / KT + 1) : 0;
-    if (nkt1 > 0) {
-        run(nkt0, std::true_type{}, std::true_type{});
-        run(nkt1, std::false_type{}, std::true_type{});
+    if constexpr (QG == 2) {
+        const int nkt1 = gpos[1] >= 0 ? min(nkt, gpos[1] / KT + 1) : 0;
+        if (nkt1 > 0) {
+            run(nkt0, std::true_type{}, std::true_type{});
+            run(nkt1, std::false_type{}, std::true_type{});
+        } else {
+            run(nkt0, std::true_type{}, std::false_type{});
+        }
     } else {
         run(nkt0, std::true_type{}, std::false_type{});
     }
@@ -519,22 +532,23 @@ __global__ void tr16_probe_kernel(int32_t* out) {
     for (int e = 0; e < 4; e++) out[threadIdx.x * 4 + e] = (uint16_t)v[e];
 }
 
-// Waves (pairs of 16-row groups) of a prefill attention workgroup; `npair` pairs for each of `heads` (sequence, head)s.  The same bits.
-// 2, and 4, while every workgroup has a CU of its own: a wave's chain of key tiles is what takes the time, and it runs faster the fewer waves
-// share the CU (Qwen2-7B, 301 rows: 8 waves 16.7 us, 4 12.5, 2 12.1; 900 rows, 420 workgroups of 2, 32.5, 25.8, 31.2).  Then 8 in one round of the
-// chip: half the K / V traffic of 4 (2,048 rows 60.4 against 64.1).  In more rounds two workgroups of 4 a CU take as long as one of 8 (5 % longer
-// over long prompts), and a last round of one a CU 0.78 of that: 2,500 rows 133 / 115 us, 4,096 210 / 220, 8 x 1,024 rows 135 / 125,
-// 8 x 301 34.6 / 26.6; Qwen3-14B 2,048 rows 114 / 100.
-static int prefill_attn_waves(int64_t npair, int64_t heads, int64_t rows, int64_t cus) {
-    const int env = dev_env("QIE_ATTN_PF_NW", 0);
-    if (env == 2 || env == 4 || env == 8) return env;
+// Waves of a prefill attention workgroup, and row groups of a wave, for `npair` pairs of 16-row groups of each of `heads` (sequence, head)s.  The same bits.
+// Pairs: 2 waves, and 4, while every workgroup has a CU of its own: a wave's chain of key tiles is what takes the time, and it runs faster the
+// fewer waves share the CU (Qwen2-7B, 301 rows: 8 waves 16.7 us, 4 12.5); then 8.
+// Where the pairs fill four fifths of the chip and no more than all of it, their even split is the faster form, us pairs | single groups: 28 heads of 128, 1,024 rows
+// 27.4 | 28.5, 2,048 60.0 | 63.1, 2,300 67.7 | 71.3, 2 x 1,000 35.6 | 38.2, 3 x 700 29.2 | 29.3; 14 heads of 64, 1,024 rows 18.1 | 18.8, 2,048 32.0 | 34.5 (from three
+// fifths in long prompts of head size 64: 1,500 rows 25.2 | 26.1; 2 x 330 9.4 | 8.7).  Elsewhere
+// single groups: 28 heads of 128, 40 rows 7.2 | 5.4, 420 15.6 | 14.5, 1,200 39.7 | 34.0, 2,600 118 | 88, 6,000 431 | 362, 8 x 1,024 122 | 121; 40 heads, 800 rows
+// 31.2 | 25.8, 2,048 99 | 76; 14 heads of 64, 113 rows 6.0 | 4.9, 2,600 51.2 | 44.1, 8,192 280 | 221, 3 x 2,500 97 | 72.  Their workgroups are of 4 waves; of 8 at head size 128 (32 KB of LDS for
+// a tile of keys, so two workgroups a CU) where the pairs would take more than the chip: 2,600 rows 93 | 88, 6,000 427 | 362, but 1,400 38.6 | 44.9.
+struct PrefillAttnPlan {
+    int waves, groups;
+};
+static PrefillAttnPlan prefill_attn_plan(int64_t npair, int64_t heads, int hd, int64_t cus) {
     auto wgs = [&](int nw) { return (npair + nw - 1) / nw * heads; };
-    for (int nw : {2, 4, 8})
-        if (wgs(nw) <= cus) return nw;
-    const int64_t n4 = wgs(4), rest = n4 % (2 * cus);
-    const float two = rows < 1500 ? .98f : 1.05f, t8 = (float)((wgs(8) + cus - 1) / cus);
-    const float t4 = two * (float)(n4 / (2 * cus)) + (rest == 0 ? 0.f : rest <= cus ? .78f : two);
-    return t4 < t8 ? 4 : 8;
+    const int nw = wgs(2) <= cus ? 2 : wgs(4) <= cus ? 4 : 8;
+    if (wgs(nw) <= cus && 5 * wgs(nw) > (hd == 64 && npair > 36 ? 3 : 4) * cus && (hd == 128 || nw < 8)) return {nw, 2};
+    return {hd == 128 && wgs(8) > cus ? 8 : 4, 1};
 }
 
 static int attn_nsplit(int64_t M, int32_t max_ctx) {
@@ -652,18 +666,26 @@ static int attention(const void* q, int64_t M, const int32_t* pos, int32_t rows_
         const bool pg = pa.km.table != nullptr;
         // balanced causal split: ceil(ceil(R / 16) / 2) group pairs, NW per workgroup
         const int npair = ((rows_per_seq + 15) / 16 + 1) / 2;
-        const bool few = rows_per_seq < 32;
-        const int nw = few ? 2 : prefill_attn_waves(npair, n_heads * (M / rows_per_seq), rows_per_seq, device_cu_count());
-        dim3 g2((unsigned)((npair + nw - 1) / nw), (unsigned)n_heads, (unsigned)(M / rows_per_seq));
-        auto pick = [&](auto w) {
-            constexpr int NW = decltype(w)::value;
-            return cache->head_dim == 128 ? (pg ? attn_prefill_mfma2_kernel<128, true, NW> : attn_prefill_mfma2_kernel<128, false, NW>)
-                                          : (pg ? attn_prefill_mfma2_kernel<64, true, NW> : attn_prefill_mfma2_kernel<64, false, NW>);
+        const PrefillAttnPlan pl = rows_per_seq < 32 ? PrefillAttnPlan{2, 2} : prefill_attn_plan(npair, n_heads * (M / rows_per_seq), cache->head_dim, device_cu_count());
+        const int ngr = (rows_per_seq + 15) / 16, nw = pl.waves;
+        auto launch = [&](auto size, auto w, auto parts, auto groups) {
+            constexpr int HD = decltype(size)::value, NW = decltype(w)::value, NP = decltype(parts)::value, QG = decltype(groups)::value;
+            const int seqs = (int)(M / rows_per_seq), blocks = ((QG == 2 ? npair : ngr) + NW - 1) / NW;
+            hipLaunchKernelGGL((pg ? attn_prefill_mfma2_kernel<HD, true, NW, NP, QG> : attn_prefill_mfma2_kernel<HD, false, NW, NP, QG>),
+                               QG == 2 ? dim3(blocks, n_heads, seqs) : dim3(n_heads, seqs, blocks), dim3(64 * NW), shm, (hipStream_t)stream, pa);
         };
-        auto k2 = few ? (cache->head_dim == 128 ? (pg ? attn_prefill_mfma2_kernel<128, true, 2, 3> : attn_prefill_mfma2_kernel<128, false, 2, 3>)
-                                                : (pg ? attn_prefill_mfma2_kernel<64, true, 2, 3> : attn_prefill_mfma2_kernel<64, false, 2, 3>))
-                : nw == 8 ? pick(std::integral_constant<int, 8>{}) : nw == 4 ? pick(std::integral_constant<int, 4>{}) : pick(std::integral_constant<int, 2>{});
-        hipLaunchKernelGGL(k2, g2, dim3(64 * nw), shm, (hipStream_t)stream, pa);
+        auto run = [&](auto size) {
+            constexpr bool wide = decltype(size)::value == 128;   // (of 64 never 8 waves)
+            constexpr std::integral_constant<int, 1> one{};
+            constexpr std::integral_constant<int, 2> two{};
+            constexpr std::integral_constant<int, 4> four{};
+            constexpr std::integral_constant<int, wide ? 8 : 4> most{};
+            if (rows_per_seq < 32) launch(size, two, std::integral_constant<int, 3>{}, two);
+            else if (pl.groups == 1) nw == 8 ? launch(size, most, two, one) : launch(size, four, two, one);
+            else nw == 8 ? launch(size, most, two, two) : nw == 4 ? launch(size, four, two, two) : launch(size, two, two, two);
+        };
+        if (cache->head_dim == 128) run(std::integral_constant<int, 128>{});
+        else run(std::integral_constant<int, 64>{});
         QIE_LAUNCH_CHECK();
         return 0;
     }
