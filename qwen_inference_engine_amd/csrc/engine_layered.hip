@@ -1448,20 +1448,43 @@ static int enq_gqa_post(qie_batch* b, int r, int T) {
     return lay::gqa_post(p, m->f32, T, e->stream);
 }
 
+// Parts of a step's keys in the matrix-core attention.  Up to 16 rows (steps that are captured: no rule on positions) as many as fill the chip, of two
+// 32-key blocks at least: a Nukizen decode step of 5 slots took 356 us with four blocks a part, 347 with two or one.
+// Steps of more rows: a wave's chain of blocks, or all waves' where that takes longer, against the parts' way through memory and the second pass.  us, 16 heads
+// of 128, whole | the parts that fill the chip: 4 prompts of 465 rows 34 | 50, 5 of 150 14 | 28, 11 of 40 9.5 | 25, one of 900 40 | 42; a step of
+// 4 tokens and a prompt of 310 rows 22 | 18, 16 in three parts.
+static int gqa_parts(const qie_batch* b, const lay::GqaAttnP& p, int T) {
+    const LayeredBatch* s = b->lb;
+    if (T <= 16) {
+        const int64_t waves = (int64_t)s->n_qgroups * p.heads;
+        const int max_blocks = (p.mask == QIE_MASK_CAUSAL ? b->max_ctx : std::min(b->max_ctx, p.mask_size + p.mask_keep)) / 32 + 2;
+        return (int)std::max<int64_t>(1, std::min<int64_t>({6144 / waves, max_blocks / 2, 32}));
+    }
+    int longest = 1;
+    int64_t all = 0;
+    for (const int4& g : s->h_qgroups) {   // {first row, rows, slot, first position}
+        const int b0 = lay::first_visible(p.mask, p.mask_size, g.w) >> 5, n = (g.w + g.y - 1) / 32 - b0 + 1 + std::min((p.mask_keep + 31) / 32, b0);
+        longest = std::max(longest, n);
+        all += n;
+    }
+    const float a_block = .15f + .0043f * (float)(p.dim + p.vdim), total = a_block * (float)all * (float)p.heads / 1024.f;
+    int best = 1;
+    float least = 1e30f;
+    for (int S = 1; S == 1 || (S <= 32 && 2 * S <= longest); S++) {
+        const float chain = a_block * (float)((longest + S - 1) / S), work = total * (1.f + .1f * (float)(S - 1));
+        const float us = std::max(chain, work) + .3f * std::min(chain, work) + (S > 1 ? 3.f + 2.2e-6f * (float)T * (float)(p.heads * p.vdim) * (float)S : 0.f);
+        if (us < least) least = us, best = S;
+    }
+    return dev_env("QIE_GQA_S", best);
+}
+
 static int enq_gqa_attention(qie_batch* b, int r, int T) {
     const qie_engine* e = b->e;
     LayeredBatch* s = b->lb;
     const lay::GqaAttnP p = gqa_attn_params(b, r);
     if (p.v_transposed && s->n_qgroups > 0) {
-        // enough key splits to fill the chip when the step has few rows (decoding)
         const int tiles = (p.heads + 3) / 4 * 4;
-        const int64_t waves = (int64_t)s->n_qgroups * p.heads;
-        const int max_blocks = (p.mask == QIE_MASK_CAUSAL ? b->max_ctx : std::min(b->max_ctx, p.mask_size + p.mask_keep)) / 32 + 2;
-        // (a wave walks its key blocks one after the other, each a trip to memory: prompts of a
-        // few thousand rows leave too few waves to hide them, so their keys are split as well.
-        // Two blocks a part: a Nukizen decode step of 5 slots took 356 us with four, 347 with two or one)
-        static const int split_waves = dev_env("QIE_GQA_SPLIT_WAVES", 6144);   // dev A/B knob: waves a launch aims for
-        const int S = (int)std::max<int64_t>(1, std::min<int64_t>({split_waves / waves, max_blocks / 2, 32}));
+        const int S = gqa_parts(b, p, T);
         const int64_t units = (int64_t)s->n_qgroups * tiles * S;
         if (S > 1 && units > s->gpart_cap) {
             hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;

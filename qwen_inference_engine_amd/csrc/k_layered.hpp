@@ -159,6 +159,13 @@ struct GqaPostP {
 };
 int gqa_post(const GqaPostP& p, bool cache_f32, int T, hipStream_t st);
 
+// First key that a row at `pos` sees under a mask (of GqaAttnP)
+__host__ __device__ inline int first_visible(int mask, int size, int pos) {
+    if (mask == 1) return pos - size + 1 > 0 ? pos - size + 1 : 0;
+    if (mask == 2) return pos / size * size;
+    return 0;
+}
+
 // Softmax attention of every (row, head) over the keys its mask lets it see (mask 0: all j <= i;
 // 1: the last mask_size and, of the earlier ones, the first mask_keep of the sequence; 2: those with
 // j / mask_size == i / mask_size); score = q.k * scale

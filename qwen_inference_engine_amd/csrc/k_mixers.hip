@@ -335,12 +335,6 @@ int gqa_post(const GqaPostP& p, bool cache_f32, int T, hipStream_t st) {
 constexpr int GA_CHUNK = 256;
 constexpr int GA_MAXV = 4;   // vdim <= 256 * GA_MAXV
 
-__device__ __forceinline__ int first_visible(int mask, int size, int pos) {
-    if (mask == 1) return max(0, pos - size + 1);
-    if (mask == 2) return pos / size * size;
-    return 0;
-}
-
 __device__ __forceinline__ float4 key4(const float* p) { return *reinterpret_cast<const float4*>(p); }
 __device__ __forceinline__ float4 key4(const uint16_t* p) {
     const uint2 u = *reinterpret_cast<const uint2*>(p);
@@ -551,14 +545,9 @@ typedef __bf16 gbf16x8_t __attribute__((ext_vector_type(8)));
 typedef float gf32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t gu32x4_t __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ float xg_max(float v) {   // over the 4 lanes n, n + 16, n + 32, n + 48
-    v = fmaxf(v, __shfl_xor(v, 16, 64));
-    return fmaxf(v, __shfl_xor(v, 32, 64));
-}
-__device__ __forceinline__ float xg_sum(float v) {
-    v += __shfl_xor(v, 16, 64);
-    return v + __shfl_xor(v, 32, 64);
-}
+// over the 4 lanes n, n + 16, n + 32, n + 48
+__device__ __forceinline__ float xg_max(float v) { return xor32_max(xor16_max(v)); }
+__device__ __forceinline__ float xg_sum(float v) { return xor32_sum(xor16_sum(v)); }
 
 // heads of one key head that a group of n_tok tokens packs into its 16 columns
 __host__ __device__ __forceinline__ int heads_per_token(int n_tok, int H, int G) {
@@ -636,17 +625,33 @@ __device__ __forceinline__ float gqa_out_factor(const GqaAttnP& a, float l, floa
     return f;
 }
 
+// 1 / d, its last bit right but for rare ties; 0 at infinity, NaN stays NaN (an IEEE division is 11 instructions)
+__device__ __forceinline__ float near_rcp(float d) {
+    const float r = __builtin_amdgcn_rcpf(d);
+    return d < 3e38f ? fmaf(fmaf(-d, r, 1.0f), r, r) : r;
+}
+
 // SHARE: the four waves of a workgroup are four heads of one key head (heads / kv_heads a
 // multiple of 4, one head per wave whatever the group's size): every 32-key K tile and V^T tile
 // is brought to LDS once per workgroup (next tile in registers meanwhile) and each wave takes
 // its fragments from there - a quarter of the cache traffic of four waves loading for themselves.
+// LDS has two of each tile where they take 64 KB at most, so that one barrier a block is enough: a wave writes tile i + 2 behind barrier i + 1,
+// which every wave reaches with tile i read.
+//
+// What bounds it is the instructions around the matrix products: 16 products of 16 clocks a block of 32 keys, and some 700 vector instructions of 4 before this
+// form.  Hence: visibility only in blocks that a column sees in part; the sums are scaled only when a maximum has moved (a factor of 1 changes no
+// bit); maxima cross lanes by permlane, the sums of weights once at the end; registers for two waves a SIMD, without which the sums' home is
+// another register file and every block moves them there and back.
+// us, 16 heads of 128 over 4, capped scores, with the parts that engine_layered.hip's gqa_parts takes: 11 prompts of 900 rows 272 -> 178, one 50 -> 38, 4 of
+// 465 59 -> 34, 11 of 40 24.5 -> 9.5; decode steps of 5 rows at 517 keys 12.2 -> 10.3, of 12 at 900 19.4 -> 15.6.
 template <int DK, int DV, bool SHARE>
-__global__ __launch_bounds__(256) void gqa_attn_mfma_kernel(GqaAttnMfmaP P) {
+__global__ __launch_bounds__(256, DV <= 12 && (SHARE ? DK + DV <= 16 : 20 * DK + 8 * DV <= 192) ? 2 : 1) void gqa_attn_mfma_kernel(GqaAttnMfmaP P) {
     const GqaAttnP& a = P.a;
     constexpr int dim = 32 * DK, vdim = 16 * DV;
     constexpr int KROW = dim + 8, VROW = 32 + 8;   // LDS rows padded by 16 bytes
-    __shared__ __align__(16) uint16_t lk[SHARE ? 32 * KROW : 8];
-    __shared__ __align__(16) uint16_t lv[SHARE ? vdim * VROW : 8];
+    constexpr int TILES = 2 * (32 * KROW + vdim * VROW) * 2 <= 65536 ? 2 : 1;
+    __shared__ __align__(16) uint16_t lk[SHARE ? TILES : 1][SHARE ? 32 * KROW : 8];
+    __shared__ __align__(16) uint16_t lv[SHARE ? TILES : 1][SHARE ? vdim * VROW : 8];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
     const int4 grp = P.groups[blockIdx.x];
     const int n_tok = grp.y, slot = grp.z, pos0 = grp.w;
@@ -657,9 +662,76 @@ __global__ __launch_bounds__(256) void gqa_attn_mfma_kernel(GqaAttnMfmaP P) {
     if (!SHARE && h0 >= H) return;
     const int tI = n / hpt, hh = h0 + n % hpt;
     const bool valid = active && tI < n_tok;
-    const int tC = valid ? tI : n_tok - 1;
+    const int tC = valid ? tI : n_tok - 1;   // (columns that are none: the last token's, not stored)
     const int qpos = pos0 + tC, row = grp.x + tC;
     const int kvh = h0 / (H / G);
+    const int lo_q = first_visible(a.mask, a.mask_size, qpos);
+    const int kmin = first_visible(a.mask, a.mask_size, pos0), kmax = pos0 + n_tok - 1, kmin_last = first_visible(a.mask, a.mask_size, kmax);
+    // 32-key blocks: those of the kept first keys that lie before the window's first block, then the window's
+    const int b0 = kmin >> 5, nk0 = min((a.mask_keep + 31) >> 5, b0), nb = nk0 + (kmax >> 5) - b0 + 1;
+    const int S = P.S, z = blockIdx.z;
+    const int bs = (int)((int64_t)nb * z / S), be = (int)((int64_t)nb * (z + 1) / S);
+    auto block_of = [&](int i) { return i < nk0 ? i : b0 + i - nk0; };
+    const int PT = a.cache.page_tokens;
+    const uint16_t* pool = (const uint16_t*)a.cache.pool;
+    const int32_t* tab = a.cache.table + (int64_t)slot * a.cache.max_pages;
+    // a block's page, looked up a block ahead of its loads, and its first token there
+    struct At {
+        int32_t page;
+        int tok0;
+    };
+    auto place = [&](int i) {
+        const int b = block_of(i < be ? i : be - 1), per = PT >> 5, q = b / per;
+        return At{tab[q], (b - q * per) << 5};
+    };
+    // K fragments of a 32-key block: two 16-key tiles x DK steps of 32 coordinates; the next
+    // block's are loaded while this block is scored, the block's V fragments before its softmax
+    uint4 kf[2][DK], kn[2][DK];
+    auto load_k = [&](At at, uint4 (&dst)[2][DK]) {
+        const uint16_t* page = pool + (int64_t)at.page * a.cache.page_stride + a.k_off;
+#pragma unroll
+        for (int tt = 0; tt < 2; tt++) {
+            const uint16_t* kr = page + ((int64_t)(at.tok0 + 16 * tt + n) * G + kvh) * dim + 8 * g;
+#pragma unroll
+            for (int ks = 0; ks < DK; ks++) dst[tt][ks] = *reinterpret_cast<const uint4*>(kr + 32 * ks);
+        }
+    };
+    // SHARE: a thread's 16-byte pieces of the workgroup's tiles (K: 32 keys x dim, V^T: vdim x 32 keys)
+    constexpr int NKP = (32 * dim / 8 + 255) / 256, NVP = (vdim * 4 + 255) / 256;
+    gu32x4_t gk[NKP], gv[NVP];   // (native vectors: arrays of the struct type end up in scratch memory)
+    auto fetch_tiles = [&](At at) {
+        const uint16_t* page = pool + (int64_t)at.page * a.cache.page_stride;
+#pragma unroll
+        for (int k = 0; k < NKP; k++) {
+            const int c = (int)threadIdx.x + 256 * k, key = c / (dim / 8), part = c % (dim / 8);
+            if (32 * dim / 8 % 256 == 0 || c < 32 * dim / 8)
+                gk[k] = *reinterpret_cast<const gu32x4_t*>(page + a.k_off + ((int64_t)(at.tok0 + key) * G + kvh) * dim + part * 8);
+        }
+#pragma unroll
+        for (int k = 0; k < NVP; k++) {
+            const int c = (int)threadIdx.x + 256 * k, r = c >> 2, part = c & 3;
+            if (vdim * 4 % 256 == 0 || c < vdim * 4) gv[k] = *reinterpret_cast<const gu32x4_t*>(page + a.v_off + ((int64_t)kvh * vdim + r) * PT + at.tok0 + part * 8);
+        }
+    };
+    auto store_tiles = [&](uint16_t* k_to, uint16_t* v_to) {
+#pragma unroll
+        for (int k = 0; k < NKP; k++) {
+            const int c = (int)threadIdx.x + 256 * k, key = c / (dim / 8), part = c % (dim / 8);
+            if (32 * dim / 8 % 256 == 0 || c < 32 * dim / 8) *reinterpret_cast<gu32x4_t*>(k_to + key * KROW + part * 8) = gk[k];
+        }
+#pragma unroll
+        for (int k = 0; k < NVP; k++) {
+            const int c = (int)threadIdx.x + 256 * k, r = c >> 2, part = c & 3;
+            if (vdim * 4 % 256 == 0 || c < vdim * 4) *reinterpret_cast<gu32x4_t*>(v_to + r * VROW + part * 8) = gv[k];
+        }
+    };
+    At here{0, 0}, ahead{0, 0};
+    if (bs < be) {
+        here = place(bs);
+        ahead = place(bs + 1);
+        if (SHARE) fetch_tiles(here);
+        else load_k(here, kf);
+    }
     // queries: B fragments (column n, k-slots 8g .. 8g + 7 of every 32 coordinates)
     gbf16x8_t qf[DK];
     {
@@ -673,100 +745,46 @@ __global__ __launch_bounds__(256) void gqa_attn_mfma_kernel(GqaAttnMfmaP P) {
             qf[ks] = __builtin_bit_cast(gbf16x8_t, u);
         }
     }
-    const int lo_q = first_visible(a.mask, a.mask_size, qpos);
-    const int kmin = first_visible(a.mask, a.mask_size, pos0), kmax = pos0 + n_tok - 1;
-    // 32-key blocks: those of the kept first keys that lie before the window's first block, then the window's
-    const int b0 = kmin >> 5, nk0 = min((a.mask_keep + 31) >> 5, b0), nb = nk0 + (kmax >> 5) - b0 + 1;
-    const int S = P.S, z = blockIdx.z;
-    const int bs = (int)((int64_t)nb * z / S), be = (int)((int64_t)nb * (z + 1) / S);
-    auto block_of = [&](int i) { return i < nk0 ? i : b0 + i - nk0; };
     const float b1 = a.r1 ? a.r1[hh] : 0.f, b2 = a.r1 ? a.r2[hh] : 0.f;
     const float slope = a.slopes ? a.slopes[hh] : 0.f;
     const float cap2 = a.softcap > 0.f ? 2.0f / a.softcap : 0.f;
     const bool sig = a.pb != nullptr;   // sigmoid weights: final as computed, no running maximum or sum
     const float pbh = sig ? a.pb[hh] : 0.f;
-    const int PT = a.cache.page_tokens;
-    const uint16_t* pool = (const uint16_t*)a.cache.pool;
-    const int32_t* tab = a.cache.table + (int64_t)slot * a.cache.max_pages;
-    float m_run = sig ? 0.f : -1e30f, l_run = sig ? 1.f : 0.f;
+    float m_run = sig ? 0.f : -1e30f, l_run = sig && g == 0 ? 1.f : 0.f;   // l_run: a lane's share of its column's sum
     gf32x4_t acc[DV];
 #pragma unroll
     for (int dv = 0; dv < DV; dv++) acc[dv] = gf32x4_t{0.f, 0.f, 0.f, 0.f};
-    // K fragments of a 32-key block: two 16-key tiles x DK steps of 32 coordinates; the next
-    // block's are loaded while this block is scored, the block's V fragments before its softmax
-    uint4 kf[2][DK], kn[2][DK];
-    auto load_k = [&](int kb, uint4 (&dst)[2][DK]) {
-        const int key0 = kb << 5;
-        const int64_t pb = (int64_t)tab[key0 / PT] * a.cache.page_stride;
-        const int tok0 = key0 % PT;
-#pragma unroll
-        for (int tt = 0; tt < 2; tt++) {
-            const uint16_t* kr = pool + pb + a.k_off + ((int64_t)(tok0 + 16 * tt + n) * G + kvh) * dim + 8 * g;
-#pragma unroll
-            for (int ks = 0; ks < DK; ks++) dst[tt][ks] = *reinterpret_cast<const uint4*>(kr + 32 * ks);
-        }
-    };
-    // SHARE: a thread's 16-byte pieces of the workgroup's tiles (K: 32 keys x dim, V^T: vdim x 32 keys)
-    constexpr int NKP = (32 * dim / 8 + 255) / 256, NVP = (vdim * 4 + 255) / 256;
-    gu32x4_t gk[NKP], gv[NVP];   // (native vectors: arrays of the struct type end up in scratch memory)
-    auto fetch_tiles = [&](int kb) {
-        const int key0 = kb << 5;
-        const int64_t pb = (int64_t)tab[key0 / PT] * a.cache.page_stride;
-        const int tok0 = key0 % PT;
-#pragma unroll
-        for (int k = 0; k < NKP; k++) {
-            const int c = (int)threadIdx.x + 256 * k, key = c / (dim / 8), part = c % (dim / 8);
-            if (c < 32 * dim / 8) gk[k] = *reinterpret_cast<const gu32x4_t*>(pool + pb + a.k_off + ((int64_t)(tok0 + key) * G + kvh) * dim + part * 8);
-        }
-#pragma unroll
-        for (int k = 0; k < NVP; k++) {
-            const int c = (int)threadIdx.x + 256 * k, r = c >> 2, part = c & 3;
-            if (c < vdim * 4) gv[k] = *reinterpret_cast<const gu32x4_t*>(pool + pb + a.v_off + ((int64_t)kvh * vdim + r) * PT + tok0 + part * 8);
-        }
-    };
-    auto store_tiles = [&]() {
-#pragma unroll
-        for (int k = 0; k < NKP; k++) {
-            const int c = (int)threadIdx.x + 256 * k, key = c / (dim / 8), part = c % (dim / 8);
-            if (c < 32 * dim / 8) *reinterpret_cast<gu32x4_t*>(lk + key * KROW + part * 8) = gk[k];
-        }
-#pragma unroll
-        for (int k = 0; k < NVP; k++) {
-            const int c = (int)threadIdx.x + 256 * k, r = c >> 2, part = c & 3;
-            if (c < vdim * 4) *reinterpret_cast<gu32x4_t*>(lv + r * VROW + part * 8) = gv[k];
-        }
-    };
-    if (bs < be) {
-        if (SHARE) fetch_tiles(block_of(bs));
-        else load_k(block_of(bs), kf);
-    }
     for (int kb = bs; kb < be; kb++) {
         const int key0 = block_of(kb) << 5;
-        const int64_t pb = (int64_t)tab[key0 / PT] * a.cache.page_stride;
-        const int tok0 = key0 % PT;
-        uint2 vf[DV][2];
+        gu32x4_t vf[DV];
         if (SHARE) {
-            __syncthreads();   // the previous tiles have been read
-            store_tiles();
+            uint16_t *k_tile = lk[TILES == 2 ? (kb - bs) & 1 : 0], *v_tile = lv[TILES == 2 ? (kb - bs) & 1 : 0];
+            if (TILES == 1) __syncthreads();   // the previous tiles have been read
+            store_tiles(k_tile, v_tile);
             __syncthreads();
-            if (kb + 1 < be) fetch_tiles(block_of(kb + 1));
+            if (kb + 1 < be) fetch_tiles(ahead);
+            ahead = place(kb + 2);
 #pragma unroll
             for (int tt = 0; tt < 2; tt++)
 #pragma unroll
-                for (int ks = 0; ks < DK; ks++) kf[tt][ks] = *reinterpret_cast<const uint4*>(lk + (16 * tt + n) * KROW + 32 * ks + 8 * g);
+                for (int ks = 0; ks < DK; ks++) kf[tt][ks] = *reinterpret_cast<const uint4*>(k_tile + (16 * tt + n) * KROW + 32 * ks + 8 * g);
 #pragma unroll
             for (int dv = 0; dv < DV; dv++) {
-                vf[dv][0] = *reinterpret_cast<const uint2*>(lv + (16 * dv + n) * VROW + 4 * g);
-                vf[dv][1] = *reinterpret_cast<const uint2*>(lv + (16 * dv + n) * VROW + 16 + 4 * g);
+                const uint2 v0 = *reinterpret_cast<const uint2*>(v_tile + (16 * dv + n) * VROW + 4 * g);
+                const uint2 v1 = *reinterpret_cast<const uint2*>(v_tile + (16 * dv + n) * VROW + 16 + 4 * g);
+                vf[dv] = gu32x4_t{v0.x, v0.y, v1.x, v1.y};
             }
         } else {
-            const uint16_t* vr = pool + pb + a.v_off + ((int64_t)kvh * vdim + n) * PT + tok0 + 4 * g;
+            const uint16_t* vr = pool + (int64_t)here.page * a.cache.page_stride + a.v_off + ((int64_t)kvh * vdim + n) * PT + here.tok0 + 4 * g;
 #pragma unroll
             for (int dv = 0; dv < DV; dv++) {
-                vf[dv][0] = *reinterpret_cast<const uint2*>(vr + (int64_t)16 * dv * PT);
-                vf[dv][1] = *reinterpret_cast<const uint2*>(vr + (int64_t)16 * dv * PT + 16);
+                const uint2 v0 = *reinterpret_cast<const uint2*>(vr + (int64_t)16 * dv * PT);
+                const uint2 v1 = *reinterpret_cast<const uint2*>(vr + (int64_t)16 * dv * PT + 16);
+                vf[dv] = gu32x4_t{v0.x, v0.y, v1.x, v1.y};
             }
-            if (kb + 1 < be) load_k(block_of(kb + 1), kn);
+            if (kb + 1 < be) load_k(ahead, kn);
+            here = ahead;
+            ahead = place(kb + 2);
         }
         gf32x4_t sacc[2];
 #pragma unroll
@@ -776,49 +794,64 @@ __global__ __launch_bounds__(256) void gqa_attn_mfma_kernel(GqaAttnMfmaP P) {
             for (int ks = 0; ks < DK; ks++)
                 sacc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gbf16x8_t, kf[tt][ks]), qf[ks], sacc[tt], 0, 0, 0);
         }
+        // key of score e: key0 + 4 g + step(e); `back`: how far it lies behind the column's token
+        auto step = [](int e) { return 16 * (e >> 2) + (e & 3); };
+        const int k4 = key0 + 4 * g, back = qpos - k4;
         float s[8];
-        bool vis[8];
-        float bm = -1e30f;
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-            const int kj = key0 + 16 * (e >> 2) + 4 * g + (e & 3);
-            vis[e] = valid && kj <= qpos && (kj >= lo_q || kj < a.mask_keep);
-            float x = sacc[e >> 2][e & 3] * a.scale;
-            if (a.softcap > 0.f) x = a.softcap * (1.0f - 2.0f / (1.0f + __expf(x * cap2)));   // c tanh(x / c)
-            if (a.r1) x -= b1 * __logf(1.0f + b2 * (float)max(qpos - kj, 0));
-            x -= slope * (float)max(qpos - kj, 0);
-            s[e] = vis[e] ? x : -1e30f;
-            bm = fmaxf(bm, s[e]);
+        for (int e = 0; e < 8; e++) s[e] = sacc[e >> 2][e & 3] * a.scale;
+        if (a.softcap > 0.f) {   // c tanh(x / c)
+#pragma unroll
+            for (int e = 0; e < 8; e++) s[e] = a.softcap * (1.0f - 2.0f * near_rcp(1.0f + __expf(s[e] * cap2)));
         }
-        float alpha = 1.0f, pv[8];
-        if (sig) {
+        if (a.r1) {
 #pragma unroll
-            for (int e = 0; e < 8; e++) pv[e] = vis[e] ? 1.0f / (1.0f + __expf(-(s[e] + pbh))) : 0.f;
-        } else {
-            bm = xg_max(bm);
-            const float m_new = fmaxf(m_run, bm);
-            alpha = __expf(m_run - m_new);
-            float ls = 0.f;
+            for (int e = 0; e < 8; e++) s[e] -= b1 * __logf(1.0f + b2 * (float)max(back - step(e), 0));
+        }
+        if (a.slopes) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) s[e] -= slope * (float)max(back - step(e), 0);
+        }
+        // every column sees every key of the block: uniform
+        const bool all = key0 + 31 <= pos0 && (key0 >= kmin_last || key0 + 31 < a.mask_keep);
+        uint32_t seen = 0xffu;
+        if (!all) {
+            seen = 0;
 #pragma unroll
             for (int e = 0; e < 8; e++) {
-                pv[e] = vis[e] ? __expf(s[e] - m_new) : 0.f;
-                ls += pv[e];
+                const bool vis = step(e) <= back && (k4 + step(e) >= lo_q || k4 + step(e) < a.mask_keep);
+                seen |= vis ? 1u << e : 0u;
+                s[e] = vis ? s[e] : -1e30f;
             }
-            ls = xg_sum(ls);
-            l_run = l_run * alpha + ls;
+        }
+        float pv[8];
+        if (sig) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) pv[e] = 1.0f / (1.0f + __expf(-(s[e] + pbh)));
+        } else {
+            const float bm = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
+            const float m_new = fmaxf(m_run, xg_max(bm));
+            const float alpha = __expf(m_run - m_new);
+#pragma unroll
+            for (int e = 0; e < 8; e++) pv[e] = __expf(s[e] - m_new);
+            if (__any(alpha != 1.0f)) {
+                l_run *= alpha;
+#pragma unroll
+                for (int dv = 0; dv < DV; dv++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) acc[dv][j] *= alpha;
+            }
             m_run = m_new;
         }
+        if (!all) {   // (where no key was seen yet the weights above are of -1e30 against itself)
+#pragma unroll
+            for (int e = 0; e < 8; e++) pv[e] = seen >> e & 1 ? pv[e] : 0.f;
+        }
+        if (!sig) l_run += ((pv[0] + pv[1]) + (pv[2] + pv[3])) + ((pv[4] + pv[5]) + (pv[6] + pv[7]));
         const uint4 pu = make_uint4(pack2(pv[0], pv[1]), pack2(pv[2], pv[3]), pack2(pv[4], pv[5]), pack2(pv[6], pv[7]));
         const gbf16x8_t pf = __builtin_bit_cast(gbf16x8_t, pu);
 #pragma unroll
-        for (int dv = 0; dv < DV; dv++) {
-            const uint4 vu = make_uint4(vf[dv][0].x, vf[dv][0].y, vf[dv][1].x, vf[dv][1].y);
-            if (!sig) {
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[dv][j] *= alpha;
-            }
-            acc[dv] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gbf16x8_t, vu), pf, acc[dv], 0, 0, 0);
-        }
+        for (int dv = 0; dv < DV; dv++) acc[dv] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gbf16x8_t, vf[dv]), pf, acc[dv], 0, 0, 0);
         if (!SHARE) {
 #pragma unroll
             for (int tt = 0; tt < 2; tt++)
@@ -826,6 +859,7 @@ __global__ __launch_bounds__(256) void gqa_attn_mfma_kernel(GqaAttnMfmaP P) {
                 for (int ks = 0; ks < DK; ks++) kf[tt][ks] = kn[tt][ks];
         }
     }
+    l_run = xg_sum(l_run);
     if (!active) return;
     if (S == 1) {
         if (valid) gqa_store<DV>(a, acc, gqa_out_factor(a, l_run, m_run, row, hh), row, hh, qpos, g);
