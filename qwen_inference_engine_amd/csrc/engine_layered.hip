@@ -1820,6 +1820,16 @@ static int enq_delta_gates(qie_batch* b, int r, int T) {
     return dense(b, s->proj + L.col_g1, L.n_in, L.w_g2, s->aux, (int64_t)c.heads * c.vdim, T, c.heads * c.vdim, L.rank_g);
 }
 
+// Entries of more than a few rows walk them in order (lay::delta_walk) where that takes less than pieces: 0.158 us a row of the longest entry, against
+// three launches, and all rows' columns twice.  us with the convolutions before, pieces | walk: 16 heads of 128, 20 rows 31 | 16, 300 rows 143 | 73,
+// 4 entries of 465 316 | 141, 11 of 900 1,430 | 650, one of 2,500 456 | 422; 16 heads of 64, 4 of 465 125 | 100, 11 of 900 439 | 273, but one of
+// 900 117 | 158, of 2,500 177 | 406.  (kLinStep: steps that are captured keep the side of it that their key names.)
+static bool delta_walks(const qie_delta_desc& c, int64_t ld, int64_t T, int max_count) {
+    if (max_count <= kLinStep || !lay::delta_walk_fits(c.dim, ld)) return false;
+    const float pieces = 60.f + 3.05e-7f * (float)c.heads * (float)c.dim * (float)(c.dim + c.vdim) * (float)T;
+    return max_count <= kScanLong || .158f * (float)max_count <= pieces;
+}
+
 static int enq_delta_scan(qie_batch* b, int r, int T, bool advance, hipStream_t st) {
     const qie_engine* e = b->e;
     const LayeredModel* m = e->lm;
@@ -1850,7 +1860,9 @@ static int enq_delta_scan(qie_batch* b, int r, int T, bool advance, hipStream_t 
     sp.state = s->state; sp.slot_stride = s->slot_state; sp.state_off = s->state_off[r];
     sp.read_state = 1; sp.write_state = advance ? 1 : 0;
     sp.out = s->olat;
-    if (s->max_count > kScanLong && s->s_loc && s->dw) {
+    if (delta_walks(c, C, s->step_T, s->max_count)) {
+        QIE_TRY(lay::delta_walk(sp, st));
+    } else if (s->max_count > kScanLong && s->s_loc && s->dw) {
         // long entries: pieces from zero states side by side (end states, transition matrices, transformed
         // queries), a carry over each entry's pieces, then the incoming states' share of every row
         const int64_t n = (int64_t)c.heads * c.dim * c.vdim;

@@ -23,6 +23,8 @@
 // rounding.
 #include "k_layered.hpp"
 
+#include <type_traits>
+
 namespace qie {
 namespace lay {
 
@@ -214,6 +216,161 @@ int delta_scan(const DeltaScanP& p, hipStream_t st) {
         default: QIE_DS(16); break;
     }
 #undef QIE_DS
+    QIE_LAUNCH_CHECK();
+    return 0;
+}
+
+// ------------------------------------------------------------------ entries of many rows, in order
+// The same walk with 8 state rows a lane instead of 32, so that a head's columns are four times as many waves and a row is short: a row's chain (two
+// products, a sum over LP lanes by DPP, u, one more product) of some 350 clocks is what bounds it, with one to four waves a SIMD (0.16 us a row; four entries of
+// 16 heads of 128 x 128 fill the chip with one); it needs no pieces, whose transition matrices are as many columns again, and no second pass.  A row's
+// output is made beside the next row's product: two sums over lanes side by side.  A lane's rows are 4 rg .. and 4 (LP + rg) ..: the reads of a row
+// out of LDS are contiguous.  Rows are staged 16 at a time, the next 16 on their way in registers; a lane keeps the
+// output of one row in LP and stores it then.  (delta_scan's form: three times as many LDS reads a product, and 16 lanes' sums through LDS.)  What both sides
+// take: engine_layered.hip, delta_walks.
+constexpr int DW_TT = 16;
+
+template <int LP, bool HEAD>
+__global__ __launch_bounds__(256) void delta_walk_kernel(DeltaScanP p) {
+    constexpr int dimP = 8 * LP, CPB = 256 / LP, Q4 = dimP / 4, NS = HEAD ? 2 : 3;   // q, k (, g): streams of staged rows
+    constexpr int NL = NS * DW_TT * Q4 / 256, NV = DW_TT * CPB / 256;
+    static_assert(LP == 8 || LP == 16, "whole threads");
+    __shared__ __attribute__((aligned(16))) float4 rows[2][NS][DW_TT][Q4];
+    __shared__ float vs[2][DW_TT][CPB];
+    __shared__ float2 bg[2][DW_TT];   // beta, (HEAD) the decay
+    const int h = blockIdx.x, tid = threadIdx.x, rg = tid % LP, lc = tid / LP, col = blockIdx.z * CPB + lc;
+    const int4 en = p.entries[blockIdx.y];   // {first packed row, rows, slot, first position}
+    const int dim = p.dim, vdim = p.vdim, G = p.G, H = p.H, gh = h / (H / G);
+    const bool colv = col < vdim;
+    const int64_t HV = (int64_t)H * vdim, HD = (int64_t)H * dim;
+    float* stp = p.state + (int64_t)en.z * p.slot_stride + p.state_off + (int64_t)h * dim * vdim + col;
+    const bool rd = (p.read_state == 2 || (p.read_state == 1 && en.w > 0)) && colv;
+    auto row_of = [&](int i) { return 4 * (i / 4 * LP + rg) + i % 4; };   // of the state
+    float S[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) S[i] = rd && row_of(i) < dim ? stp[(int64_t)row_of(i) * vdim] : 0.f;
+    float4 next[NL];
+    float vn[NV], bn = 0.f, gn = 0.f;
+    auto fetch = [&](int t0) {   // rows past the entry's end: its last
+#pragma unroll
+        for (int j = 0; j < NL; j++) {
+            const int c = tid + 256 * j, s = c / (DW_TT * Q4), tt = c / Q4 % DW_TT, r = 4 * (c % Q4);
+            const int64_t row = en.x + min(t0 + tt, en.y - 1);
+            const float* src = !HEAD && s == 2 ? p.g + row * HD + (int64_t)h * dim : p.qkv + row * p.ld_qkv + (s == 0 ? gh : G + gh) * dim;
+            next[j] = r < dim ? *reinterpret_cast<const float4*>(src + r) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+#pragma unroll
+        for (int j = 0; j < NV; j++) {
+            const int c = tid + 256 * j, cc = min((int)blockIdx.z * CPB + c % CPB, vdim - 1);
+            vn[j] = p.qkv[(en.x + min(t0 + c / CPB, en.y - 1)) * p.ld_qkv + 2 * G * dim + h * vdim + cc];
+        }
+        if (tid < DW_TT) {
+            const int64_t row = en.x + min(t0 + tid, en.y - 1);
+            bn = p.beta[row * p.ld_beta + h];
+            if (HEAD) gn = p.g[row * p.ld_g + h];
+        }
+    };
+    fetch(0);
+    int buf = 0;
+    for (int t0 = 0; t0 < en.y; t0 += DW_TT, buf ^= 1) {   // (written again two tiles on, behind the next tile's barrier)
+#pragma unroll
+        for (int j = 0; j < NL; j++) {
+            const int c = tid + 256 * j;
+            (&rows[buf][0][0][0])[c] = next[j];
+        }
+#pragma unroll
+        for (int j = 0; j < NV; j++) (&vs[buf][0][0])[tid + 256 * j] = vn[j];
+        if (tid < DW_TT) bg[buf][tid] = make_float2(bn, gn);
+        __syncthreads();
+        if (t0 + DW_TT < en.y) fetch(t0 + DW_TT);
+        struct Row {
+            float q[8], k[8], g[HEAD ? 1 : 8], v;
+            float2 w;
+        };
+        auto read = [&](int tr) {
+            Row x;
+            auto eight = [&](int s, float* to) {
+                const float4 a = rows[buf][s][tr][rg], b = rows[buf][s][tr][LP + rg];
+                to[0] = a.x; to[1] = a.y; to[2] = a.z; to[3] = a.w;
+                to[4] = b.x; to[5] = b.y; to[6] = b.z; to[7] = b.w;
+            };
+            eight(0, x.q);
+            eight(1, x.k);
+            if constexpr (!HEAD) eight(2, x.g);
+            x.w = bg[buf][tr];
+            x.v = vs[buf][tr][lc];
+            return x;
+        };
+        for (int b0 = 0; b0 < DW_TT && t0 + b0 < en.y; b0 += LP) {
+            const int nt = min(LP, en.y - t0 - b0);   // uniform
+            float kept = 0.f;
+            auto output = [&](const Row& x, float (&o)[4]) {   // S^T q, a lane's share
+#pragma unroll
+                for (int i = 0; i < 4; i++) o[i] = fmaf(x.q[i + 4], S[i + 4], x.q[i] * S[i]);
+            };
+            auto keep = [&](const float (&o)[4], int tt) {
+                const float sum = group_sum<LP>((o[0] + o[1]) + (o[2] + o[3]));
+                kept = rg == tt ? sum : kept;
+            };
+            auto walk = [&](const Row& x, const Row& before, int tt) {   // before (tt > 0): row tt - 1, whose output is made beside this row's product
+                float d[4], o[4];
+                if (tt > 0) output(before, o);
+#pragma unroll
+                for (int i = 0; i < 8; i++) S[i] *= HEAD ? x.w.y : x.g[HEAD ? 0 : i];
+#pragma unroll
+                for (int i = 0; i < 4; i++) d[i] = fmaf(x.k[i + 4], S[i + 4], x.k[i] * S[i]);
+                const float u = x.w.x * (x.v - group_sum<LP>((d[0] + d[1]) + (d[2] + d[3])));
+                if (tt > 0) keep(o, tt - 1);
+#pragma unroll
+                for (int i = 0; i < 8; i++) S[i] = fmaf(x.k[i], u, S[i]);
+            };
+            float o[4];
+            // the reads of a row are issued a row ahead (in a loop the compiler puts them back in front of their use: 0.22 us a row)
+            if (nt == LP) {
+                Row x[3];
+                x[0] = read(b0);
+#pragma unroll
+                for (int tt = 0; tt < LP; tt++) {
+                    if (tt + 1 < LP) x[(tt + 1) % 3] = read(b0 + tt + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    walk(x[tt % 3], x[(tt + 2) % 3], tt);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                output(x[(LP - 1) % 3], o);
+                keep(o, LP - 1);
+            } else {
+                for (int tt = 0; tt < nt; tt++) {
+                    const Row x = read(b0 + tt);
+                    walk(x, x, 0);
+                    output(x, o);
+                    keep(o, tt);
+                }
+            }
+            if (rg < nt && colv) p.out[(en.x + t0 + b0 + rg) * HV + (int64_t)h * vdim + col] = kept;
+        }
+    }
+    if (!p.write_state || !colv) return;
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+        if (row_of(i) < dim) stp[(int64_t)row_of(i) * vdim] = S[i];
+}
+
+bool delta_walk_fits(int dim, int64_t ld_qkv) { return dim <= 128 && dim % 8 == 0 && ld_qkv % 4 == 0; }
+
+int delta_walk(const DeltaScanP& p, hipStream_t st) {
+    QIE_REQUIRE(p.qkv && p.beta && p.g && p.entries && p.n_entries > 0 && p.state && p.out, "delta_walk: bad arguments");
+    QIE_REQUIRE(p.H > 0 && p.G > 0 && p.H % p.G == 0 && p.dim > 0 && p.vdim > 0 && delta_walk_fits(p.dim, p.ld_qkv) && !p.trans &&
+                    (uintptr_t)p.qkv % 16 == 0 && (p.ld_g > 0 || (uintptr_t)p.g % 16 == 0),
+                "delta_walk: %d heads over %d key heads of %d / %d", p.H, p.G, p.dim, p.vdim);
+    const bool head = p.ld_g > 0;
+    auto run = [&](auto lanes) {
+        constexpr int LP = decltype(lanes)::value, CPB = 256 / LP;
+        const dim3 grid((unsigned)p.H, (unsigned)p.n_entries, (unsigned)((p.vdim + CPB - 1) / CPB));
+        if (head) hipLaunchKernelGGL((delta_walk_kernel<LP, true>), grid, dim3(256), 0, st, p);
+        else hipLaunchKernelGGL((delta_walk_kernel<LP, false>), grid, dim3(256), 0, st, p);
+    };
+    if (p.dim > 64) run(std::integral_constant<int, 16>{});
+    else run(std::integral_constant<int, 8>{});
     QIE_LAUNCH_CHECK();
     return 0;
 }

@@ -442,6 +442,9 @@ struct DeltaScanP {
     float* w_out;
 };
 int delta_scan(const DeltaScanP& p, hipStream_t st);
+// The same for entries of many rows (dim a multiple of 8 up to 128, rows of qkv on 16 bytes, no pieces)
+bool delta_walk_fits(int dim, int64_t ld_qkv);
+int delta_walk(const DeltaScanP& p, hipStream_t st);
 // Walks every entry's pieces (spans {first piece, pieces, slot, first position}): s_in[c] = the state entering piece
 // c, from the slot's state (zero at position 0) through s <- M_c s + s_loc[c]; the slot's state = what leaves the
 // last piece (write_state).  s_loc, s_in [pieces][H][dim][vdim].
