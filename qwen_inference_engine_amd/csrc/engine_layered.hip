@@ -1475,7 +1475,7 @@ static int gqa_parts(const qie_batch* b, const lay::GqaAttnP& p, int T) {
         const float us = std::max(chain, work) + .3f * std::min(chain, work) + (S > 1 ? 3.f + 2.2e-6f * (float)T * (float)(p.heads * p.vdim) * (float)S : 0.f);
         if (us < least) least = us, best = S;
     }
-    return dev_env("QIE_GQA_S", best);
+    return best;
 }
 
 static int enq_gqa_attention(qie_batch* b, int r, int T) {

@@ -18,7 +18,7 @@ namespace qie {
 namespace lf {
 constexpr int BM = 64, BN = 64, BK = 32;
 constexpr int LEVELS = 4;           // of the tree of K segments: 16 at most
-constexpr int SLAB = 2 * BM * BN;   // floats of a part: both K halves
+constexpr int slab(int bm) { return 2 * bm * BN; }   // floats of a part: both K halves
 
 struct Plan {
     int n_nt, n_mt;      // tiles of N; tiles of M per group (of the most rows a group may have)
@@ -28,18 +28,26 @@ struct Plan {
 };
 
 // Index of the row tile from row m0 of group z (tile mt of the group) among those that exist.  Groups follow one another inside
-// [0, M): a later group's rows lie further on and its z is larger, so m0 / 64 + z is no other tile's, and below M / 64 + groups.
-QIE_PLAN_HD inline int64_t row_tile(bool grouped, int m0, int z, int mt, int n_mt) {
-    return grouped ? (int64_t)(m0 / BM) + z : (int64_t)z * n_mt + mt;
+// [0, M): a later group's rows lie further on and its z is larger, so m0 / bm + z is no other tile's, and below M / bm + groups.
+QIE_PLAN_HD inline int64_t row_tile(bool grouped, int m0, int z, int mt, int n_mt, int bm = BM) {
+    return grouped ? (int64_t)(m0 / bm) + z : (int64_t)z * n_mt + mt;
+}
+
+// Rows of a tile, the same bits: 32 where groups are small, whose last tiles are mostly padding (us, 64 | 32: eight experts of some 69 rows, 1,024 x
+// 1,408 and 704 x 1,024, 42 | 32 and 21 | 20; of some 25 rows 26 | 20 and 19.5 | 14.5), or where few tiles of 64 would be cut into more parts (102 rows
+// 1,024 x 1,024 12.5 | 10); else 64 (275 rows 1,024 x 3,072 45 | 53).
+inline int tile_rows(int64_t M, int64_t N, int64_t batch, bool grouped) {
+    if (grouped) return M < 128 * batch ? 32 : BM;
+    return M <= 224 && (M + BM - 1) / BM * ((N + BN - 1) / BN) * batch <= 128 ? 32 : BM;
 }
 
 // Segments of 8 k-tiles or more: of 4, their meetings cost a wave 5 % beside its products (a pass of the fp32 replay 4.08 ms, of 8
 // 4.04).  Workgroups a tile: until about 512 (two a CU) have work.  Grouped: rows spread over the groups.
 // (At most 1,024 parts have slabs then: 32 MB on 256 CUs.)
-inline Plan plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool grouped, int64_t cus) {
+inline Plan plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool grouped, int64_t cus, int bm = BM) {
     Plan p{};
     p.n_nt = (int)((N + BN - 1) / BN);
-    p.n_mt = (int)((M + BM - 1) / BM);
+    p.n_mt = (int)((M + bm - 1) / bm);
     p.row_tiles = grouped ? p.n_mt - 1 + batch : p.n_mt * batch;
     const int64_t busy = grouped ? std::max<int64_t>(batch, p.n_mt + batch / 2) : p.n_mt * batch;
     const int64_t want = 2 * cus / (busy * p.n_nt);

@@ -13,7 +13,7 @@
 // column group reads the same addresses), the next rows' values already in registers.  The state
 // is fp32 and lives with the slot; an entry that starts at position 0 starts from zero.
 //
-// Long entries run in pieces side by side.  A column s of S moves through a row as s <- A_t s + beta k v_c
+// Entries of more than a few rows walk them with fewer state rows a lane (delta_walk); where that would be longer (delta_walks), they run in pieces side by side.  A column s of S moves through a row as s <- A_t s + beta k v_c
 // with A_t = (I - beta k k^T) diag(g), the same A_t for every column, so over a piece s_end = M s_in + s_loc with
 // M = the product of the piece's A_t and s_loc the end state from zero.  A piece scanned from zero with dim extra
 // columns that start as the unit vectors and see v = 0 yields s_loc, M (those columns' end states) and, as those
