@@ -1448,14 +1448,14 @@ static int enq_gqa_post(qie_batch* b, int r, int T) {
     return lay::gqa_post(p, m->f32, T, e->stream);
 }
 
-// Parts of a step's keys in the matrix-core attention.  Up to 16 rows (steps that are captured: no rule on positions) as many as fill the chip, of two
-// 32-key blocks at least: a Nukizen decode step of 5 slots took 356 us with four blocks a part, 347 with two or one.
+// Parts of a step's keys in the matrix-core attention.  Up to 16 rows (steps that are captured: no rule on positions), and where every wave loads for itself
+// (head ratios off 4; 4 heads of 256 over 2, 8 prompts of 900 rows whole 283 us, in three parts 222), as many as fill the chip, of two 32-key blocks at least: a Nukizen decode step of 5 slots took 356 us with four blocks a part, 347 with two or one.
 // Steps of more rows: a wave's chain of blocks, or all waves' where that takes longer, against the parts' way through memory and the second pass.  us, 16 heads
 // of 128, whole | the parts that fill the chip: 4 prompts of 465 rows 34 | 50, 5 of 150 14 | 28, 11 of 40 9.5 | 25, one of 900 40 | 42; a step of
 // 4 tokens and a prompt of 310 rows 22 | 18, 16 in three parts.
 static int gqa_parts(const qie_batch* b, const lay::GqaAttnP& p, int T) {
     const LayeredBatch* s = b->lb;
-    if (T <= 16) {
+    if (T <= 16 || p.heads / p.kv_heads % 4 != 0) {
         const int64_t waves = (int64_t)s->n_qgroups * p.heads;
         const int max_blocks = (p.mask == QIE_MASK_CAUSAL ? b->max_ctx : std::min(b->max_ctx, p.mask_size + p.mask_keep)) / 32 + 2;
         return (int)std::max<int64_t>(1, std::min<int64_t>({6144 / waves, max_blocks / 2, 32}));

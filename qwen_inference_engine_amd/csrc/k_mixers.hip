@@ -545,9 +545,14 @@ typedef __bf16 gbf16x8_t __attribute__((ext_vector_type(8)));
 typedef float gf32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t gu32x4_t __attribute__((ext_vector_type(4)));
 
-// over the 4 lanes n, n + 16, n + 32, n + 48
-__device__ __forceinline__ float xg_max(float v) { return xor32_max(xor16_max(v)); }
-__device__ __forceinline__ float xg_sum(float v) { return xor32_sum(xor16_sum(v)); }
+__device__ __forceinline__ float xg_max(float v) {   // over the 4 lanes n, n + 16, n + 32, n + 48
+    v = fmaxf(v, __shfl_xor(v, 16, 64));
+    return fmaxf(v, __shfl_xor(v, 32, 64));
+}
+__device__ __forceinline__ float xg_sum(float v) {
+    v += __shfl_xor(v, 16, 64);
+    return v + __shfl_xor(v, 32, 64);
+}
 
 // heads of one key head that a group of n_tok tokens packs into its 16 columns
 __host__ __device__ __forceinline__ int heads_per_token(int n_tok, int H, int G) {
@@ -631,7 +636,7 @@ __device__ __forceinline__ float near_rcp(float d) {
     return d < 3e38f ? fmaf(fmaf(-d, r, 1.0f), r, r) : r;
 }
 
-// SHARE: the four waves of a workgroup are four heads of one key head (heads / kv_heads a
+// The four waves of a workgroup are four heads of one key head (heads / kv_heads a
 // multiple of 4, one head per wave whatever the group's size): every 32-key K tile and V^T tile
 // is brought to LDS once per workgroup (next tile in registers meanwhile) and each wave takes
 // its fragments from there - a quarter of the cache traffic of four waves loading for themselves.
@@ -644,27 +649,23 @@ __device__ __forceinline__ float near_rcp(float d) {
 // another register file and every block moves them there and back.
 // us, 16 heads of 128 over 4, capped scores, with the parts that engine_layered.hip's gqa_parts takes: 11 prompts of 900 rows 272 -> 178, one 50 -> 38, 4 of
 // 465 59 -> 34, 11 of 40 24.5 -> 9.5; decode steps of 5 rows at 517 keys 12.2 -> 10.3, of 12 at 900 19.4 -> 15.6.
-template <int DK, int DV, bool SHARE>
-__global__ __launch_bounds__(256, DV <= 12 && (SHARE ? DK + DV <= 16 : 20 * DK + 8 * DV <= 192) ? 2 : 1) void gqa_attn_mfma_kernel(GqaAttnMfmaP P) {
+template <int DK, int DV>
+__global__ __launch_bounds__(256, DV <= 12 && DK + DV <= 16 ? 2 : 1) void gqa_attn_mfma_kernel(GqaAttnMfmaP P) {
     const GqaAttnP& a = P.a;
     constexpr int dim = 32 * DK, vdim = 16 * DV;
     constexpr int KROW = dim + 8, VROW = 32 + 8;   // LDS rows padded by 16 bytes
     constexpr int TILES = 2 * (32 * KROW + vdim * VROW) * 2 <= 65536 ? 2 : 1;
-    __shared__ __align__(16) uint16_t lk[SHARE ? TILES : 1][SHARE ? 32 * KROW : 8];
-    __shared__ __align__(16) uint16_t lv[SHARE ? TILES : 1][SHARE ? vdim * VROW : 8];
+    __shared__ __align__(16) uint16_t lk[TILES][32 * KROW];
+    __shared__ __align__(16) uint16_t lv[TILES][vdim * VROW];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
     const int4 grp = P.groups[blockIdx.x];
     const int n_tok = grp.y, slot = grp.z, pos0 = grp.w;
     const int H = a.heads, G = a.kv_heads;
-    const int hpt = SHARE ? 1 : heads_per_token(n_tok, H, G);
-    const int tile = blockIdx.y * 4 + wave, h0 = SHARE ? min(tile, H - 1) : tile * hpt;
-    const bool active = SHARE ? tile < H : true;
-    if (!SHARE && h0 >= H) return;
-    const int tI = n / hpt, hh = h0 + n % hpt;
-    const bool valid = active && tI < n_tok;
-    const int tC = valid ? tI : n_tok - 1;   // (columns that are none: the last token's, not stored)
+    const int tile = blockIdx.y * 4 + wave, hh = min(tile, H - 1);
+    const bool active = tile < H, valid = active && n < n_tok;
+    const int tC = valid ? n : n_tok - 1;   // (columns that are none: the last token's, not stored)
     const int qpos = pos0 + tC, row = grp.x + tC;
-    const int kvh = h0 / (H / G);
+    const int kvh = hh / (H / G);
     const int lo_q = first_visible(a.mask, a.mask_size, qpos);
     const int kmin = first_visible(a.mask, a.mask_size, pos0), kmax = pos0 + n_tok - 1, kmin_last = first_visible(a.mask, a.mask_size, kmax);
     // 32-key blocks: those of the kept first keys that lie before the window's first block, then the window's
@@ -674,7 +675,8 @@ __global__ __launch_bounds__(256, DV <= 12 && (SHARE ? DK + DV <= 16 : 20 * DK +
     auto block_of = [&](int i) { return i < nk0 ? i : b0 + i - nk0; };
     const int PT = a.cache.page_tokens;
     const uint16_t* pool = (const uint16_t*)a.cache.pool;
-    const int32_t* tab = a.cache.table + (int64_t)slot * a.cache.max_pages;
+    // (constant for the launch)
+    const auto tab = (const __attribute__((address_space(4))) int32_t*)(uintptr_t)(a.cache.table + (int64_t)slot * a.cache.max_pages);
     // a block's page, looked up a block ahead of its loads, and its first token there
     struct At {
         int32_t page;
@@ -682,21 +684,9 @@ __global__ __launch_bounds__(256, DV <= 12 && (SHARE ? DK + DV <= 16 : 20 * DK +
     };
     auto place = [&](int i) {
         const int b = block_of(i < be ? i : be - 1), per = PT >> 5, q = b / per;
-        return At{tab[q], (b - q * per) << 5};
+        return At{tab[q], (b - q * per) << 5};   // (a scalar load: a vector one would stand between the tiles' loads)
     };
-    // K fragments of a 32-key block: two 16-key tiles x DK steps of 32 coordinates; the next
-    // block's are loaded while this block is scored, the block's V fragments before its softmax
-    uint4 kf[2][DK], kn[2][DK];
-    auto load_k = [&](At at, uint4 (&dst)[2][DK]) {
-        const uint16_t* page = pool + (int64_t)at.page * a.cache.page_stride + a.k_off;
-#pragma unroll
-        for (int tt = 0; tt < 2; tt++) {
-            const uint16_t* kr = page + ((int64_t)(at.tok0 + 16 * tt + n) * G + kvh) * dim + 8 * g;
-#pragma unroll
-            for (int ks = 0; ks < DK; ks++) dst[tt][ks] = *reinterpret_cast<const uint4*>(kr + 32 * ks);
-        }
-    };
-    // SHARE: a thread's 16-byte pieces of the workgroup's tiles (K: 32 keys x dim, V^T: vdim x 32 keys)
+    // a thread's 16-byte pieces of the workgroup's tiles (K: 32 keys x dim, V^T: vdim x 32 keys)
     constexpr int NKP = (32 * dim / 8 + 255) / 256, NVP = (vdim * 4 + 255) / 256;
     gu32x4_t gk[NKP], gv[NVP];   // (native vectors: arrays of the struct type end up in scratch memory)
     auto fetch_tiles = [&](At at) {
@@ -725,25 +715,26 @@ __global__ __launch_bounds__(256, DV <= 12 && (SHARE ? DK + DV <= 16 : 20 * DK +
             if (vdim * 4 % 256 == 0 || c < vdim * 4) *reinterpret_cast<gu32x4_t*>(v_to + r * VROW + part * 8) = gv[k];
         }
     };
-    At here{0, 0}, ahead{0, 0};
-    if (bs < be) {
-        here = place(bs);
-        ahead = place(bs + 1);
-        if (SHARE) fetch_tiles(here);
-        else load_k(here, kf);
-    }
-    // queries: B fragments (column n, k-slots 8g .. 8g + 7 of every 32 coordinates)
-    gbf16x8_t qf[DK];
+    // queries, on their way ahead of the first tiles: B fragments (column n, k-slots 8g .. 8g + 7 of every 32 coordinates)
+    float x[DK][8];
     {
         const float* qr = a.proj + (int64_t)row * a.ld + a.q_col + hh * dim + 8 * g;
 #pragma unroll
-        for (int ks = 0; ks < DK; ks++) {
-            float x[8];
+        for (int ks = 0; ks < DK; ks++)
 #pragma unroll
-            for (int i = 0; i < 8; i++) x[i] = qr[32 * ks + i];
-            const uint4 u = make_uint4(pack2(x[0], x[1]), pack2(x[2], x[3]), pack2(x[4], x[5]), pack2(x[6], x[7]));
-            qf[ks] = __builtin_bit_cast(gbf16x8_t, u);
-        }
+            for (int i = 0; i < 8; i++) x[ks][i] = qr[32 * ks + i];
+    }
+    At ahead{0, 0};
+    if (bs < be) {
+        const At here = place(bs);
+        ahead = place(bs + 1);
+        fetch_tiles(here);
+    }
+    gbf16x8_t qf[DK];
+#pragma unroll
+    for (int ks = 0; ks < DK; ks++) {
+        const uint4 u = make_uint4(pack2(x[ks][0], x[ks][1]), pack2(x[ks][2], x[ks][3]), pack2(x[ks][4], x[ks][5]), pack2(x[ks][6], x[ks][7]));
+        qf[ks] = __builtin_bit_cast(gbf16x8_t, u);
     }
     const float b1 = a.r1 ? a.r1[hh] : 0.f, b2 = a.r1 ? a.r2[hh] : 0.f;
     const float slope = a.slopes ? a.slopes[hh] : 0.f;
@@ -756,35 +747,23 @@ __global__ __launch_bounds__(256, DV <= 12 && (SHARE ? DK + DV <= 16 : 20 * DK +
     for (int dv = 0; dv < DV; dv++) acc[dv] = gf32x4_t{0.f, 0.f, 0.f, 0.f};
     for (int kb = bs; kb < be; kb++) {
         const int key0 = block_of(kb) << 5;
+        uint16_t *k_tile = lk[TILES == 2 ? (kb - bs) & 1 : 0], *v_tile = lv[TILES == 2 ? (kb - bs) & 1 : 0];
+        if (TILES == 1) __syncthreads();   // the previous tiles have been read
+        store_tiles(k_tile, v_tile);
+        __syncthreads();
+        if (kb + 1 < be) fetch_tiles(ahead);
+        ahead = place(kb + 2);
+        uint4 kf[2][DK];
         gu32x4_t vf[DV];
-        if (SHARE) {
-            uint16_t *k_tile = lk[TILES == 2 ? (kb - bs) & 1 : 0], *v_tile = lv[TILES == 2 ? (kb - bs) & 1 : 0];
-            if (TILES == 1) __syncthreads();   // the previous tiles have been read
-            store_tiles(k_tile, v_tile);
-            __syncthreads();
-            if (kb + 1 < be) fetch_tiles(ahead);
-            ahead = place(kb + 2);
 #pragma unroll
-            for (int tt = 0; tt < 2; tt++)
+        for (int tt = 0; tt < 2; tt++)
 #pragma unroll
-                for (int ks = 0; ks < DK; ks++) kf[tt][ks] = *reinterpret_cast<const uint4*>(k_tile + (16 * tt + n) * KROW + 32 * ks + 8 * g);
+            for (int ks = 0; ks < DK; ks++) kf[tt][ks] = *reinterpret_cast<const uint4*>(k_tile + (16 * tt + n) * KROW + 32 * ks + 8 * g);
 #pragma unroll
-            for (int dv = 0; dv < DV; dv++) {
-                const uint2 v0 = *reinterpret_cast<const uint2*>(v_tile + (16 * dv + n) * VROW + 4 * g);
-                const uint2 v1 = *reinterpret_cast<const uint2*>(v_tile + (16 * dv + n) * VROW + 16 + 4 * g);
-                vf[dv] = gu32x4_t{v0.x, v0.y, v1.x, v1.y};
-            }
-        } else {
-            const uint16_t* vr = pool + (int64_t)here.page * a.cache.page_stride + a.v_off + ((int64_t)kvh * vdim + n) * PT + here.tok0 + 4 * g;
-#pragma unroll
-            for (int dv = 0; dv < DV; dv++) {
-                const uint2 v0 = *reinterpret_cast<const uint2*>(vr + (int64_t)16 * dv * PT);
-                const uint2 v1 = *reinterpret_cast<const uint2*>(vr + (int64_t)16 * dv * PT + 16);
-                vf[dv] = gu32x4_t{v0.x, v0.y, v1.x, v1.y};
-            }
-            if (kb + 1 < be) load_k(ahead, kn);
-            here = ahead;
-            ahead = place(kb + 2);
+        for (int dv = 0; dv < DV; dv++) {
+            const uint2 v0 = *reinterpret_cast<const uint2*>(v_tile + (16 * dv + n) * VROW + 4 * g);
+            const uint2 v1 = *reinterpret_cast<const uint2*>(v_tile + (16 * dv + n) * VROW + 16 + 4 * g);
+            vf[dv] = gu32x4_t{v0.x, v0.y, v1.x, v1.y};
         }
         gf32x4_t sacc[2];
 #pragma unroll
@@ -830,7 +809,7 @@ __global__ __launch_bounds__(256, DV <= 12 && (SHARE ? DK + DV <= 16 : 20 * DK +
             for (int e = 0; e < 8; e++) pv[e] = 1.0f / (1.0f + __expf(-(s[e] + pbh)));
         } else {
             const float bm = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
-            const float m_new = fmaxf(m_run, xg_max(bm));
+            const float m_new = fmaxf(m_run, xor32_max(xor16_max(bm)));
             const float alpha = __expf(m_run - m_new);
 #pragma unroll
             for (int e = 0; e < 8; e++) pv[e] = __expf(s[e] - m_new);
@@ -852,15 +831,157 @@ __global__ __launch_bounds__(256, DV <= 12 && (SHARE ? DK + DV <= 16 : 20 * DK +
         const gbf16x8_t pf = __builtin_bit_cast(gbf16x8_t, pu);
 #pragma unroll
         for (int dv = 0; dv < DV; dv++) acc[dv] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gbf16x8_t, vf[dv]), pf, acc[dv], 0, 0, 0);
-        if (!SHARE) {
-#pragma unroll
-            for (int tt = 0; tt < 2; tt++)
-#pragma unroll
-                for (int ks = 0; ks < DK; ks++) kf[tt][ks] = kn[tt][ks];
-        }
     }
     l_run = xg_sum(l_run);
     if (!active) return;
+    if (S == 1) {
+        if (valid) gqa_store<DV>(a, acc, gqa_out_factor(a, l_run, m_run, row, hh), row, hh, qpos, g);
+        return;
+    }
+    const int64_t unit = ((int64_t)blockIdx.x * (gridDim.y * 4) + tile) * S + z;
+    if (!valid) return;   // (the second pass reads the columns that exist)
+    float* po = P.part_o + (unit * 16 + n) * vdim + 4 * g;
+#pragma unroll
+    for (int dv = 0; dv < DV; dv++) *reinterpret_cast<float4*>(po + 16 * dv) = make_float4(acc[dv][0], acc[dv][1], acc[dv][2], acc[dv][3]);
+    if (g == 0) {
+        P.part_ml[(unit * 16 + n) * 2] = m_run;
+        P.part_ml[(unit * 16 + n) * 2 + 1] = l_run;
+    }
+}
+
+// Other ratios: every wave loads its own fragments, groups of few tokens pack the heads of a key head into its columns.  (The form above with these loads
+// took 5 to 14 % longer in decode steps, which wait for loads more than for instructions: 16 heads of 128 over 8, 8 rows at 600 keys 20.5 us | 21.7; maxima by permlane alone 21.1.)
+template <int DK, int DV>
+__global__ __launch_bounds__(256) void gqa_attn_pack_kernel(GqaAttnMfmaP P) {
+    const GqaAttnP& a = P.a;
+    constexpr int dim = 32 * DK, vdim = 16 * DV;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+    const int4 grp = P.groups[blockIdx.x];
+    const int n_tok = grp.y, slot = grp.z, pos0 = grp.w;
+    const int H = a.heads, G = a.kv_heads;
+    const int hpt = heads_per_token(n_tok, H, G);
+    const int tile = blockIdx.y * 4 + wave, h0 = tile * hpt;
+    if (h0 >= H) return;
+    const int tI = n / hpt, hh = h0 + n % hpt;
+    const bool valid = tI < n_tok;
+    const int tC = valid ? tI : n_tok - 1;
+    const int qpos = pos0 + tC, row = grp.x + tC;
+    const int kvh = h0 / (H / G);
+    // queries: B fragments (column n, k-slots 8g .. 8g + 7 of every 32 coordinates)
+    gbf16x8_t qf[DK];
+    {
+        const float* qr = a.proj + (int64_t)row * a.ld + a.q_col + hh * dim + 8 * g;
+#pragma unroll
+        for (int ks = 0; ks < DK; ks++) {
+            float x[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) x[i] = qr[32 * ks + i];
+            const uint4 u = make_uint4(pack2(x[0], x[1]), pack2(x[2], x[3]), pack2(x[4], x[5]), pack2(x[6], x[7]));
+            qf[ks] = __builtin_bit_cast(gbf16x8_t, u);
+        }
+    }
+    const int lo_q = first_visible(a.mask, a.mask_size, qpos);
+    const int kmin = first_visible(a.mask, a.mask_size, pos0), kmax = pos0 + n_tok - 1;
+    // 32-key blocks: those of the kept first keys that lie before the window's first block, then the window's
+    const int b0 = kmin >> 5, nk0 = min((a.mask_keep + 31) >> 5, b0), nb = nk0 + (kmax >> 5) - b0 + 1;
+    const int S = P.S, z = blockIdx.z;
+    const int bs = (int)((int64_t)nb * z / S), be = (int)((int64_t)nb * (z + 1) / S);
+    auto block_of = [&](int i) { return i < nk0 ? i : b0 + i - nk0; };
+    const float b1 = a.r1 ? a.r1[hh] : 0.f, b2 = a.r1 ? a.r2[hh] : 0.f;
+    const float slope = a.slopes ? a.slopes[hh] : 0.f;
+    const float cap2 = a.softcap > 0.f ? 2.0f / a.softcap : 0.f;
+    const bool sig = a.pb != nullptr;   // sigmoid weights: final as computed, no running maximum or sum
+    const float pbh = sig ? a.pb[hh] : 0.f;
+    const int PT = a.cache.page_tokens;
+    const uint16_t* pool = (const uint16_t*)a.cache.pool;
+    const int32_t* tab = a.cache.table + (int64_t)slot * a.cache.max_pages;
+    float m_run = sig ? 0.f : -1e30f, l_run = sig ? 1.f : 0.f;
+    gf32x4_t acc[DV];
+#pragma unroll
+    for (int dv = 0; dv < DV; dv++) acc[dv] = gf32x4_t{0.f, 0.f, 0.f, 0.f};
+    // K fragments of a 32-key block: two 16-key tiles x DK steps of 32 coordinates; the next
+    // block's are loaded while this block is scored, the block's V fragments before its softmax
+    uint4 kf[2][DK], kn[2][DK];
+    auto load_k = [&](int kb, uint4 (&dst)[2][DK]) {
+        const int key0 = kb << 5;
+        const int64_t pb = (int64_t)tab[key0 / PT] * a.cache.page_stride;
+        const int tok0 = key0 % PT;
+#pragma unroll
+        for (int tt = 0; tt < 2; tt++) {
+            const uint16_t* kr = pool + pb + a.k_off + ((int64_t)(tok0 + 16 * tt + n) * G + kvh) * dim + 8 * g;
+#pragma unroll
+            for (int ks = 0; ks < DK; ks++) dst[tt][ks] = *reinterpret_cast<const uint4*>(kr + 32 * ks);
+        }
+    };
+    if (bs < be) load_k(block_of(bs), kf);
+    for (int kb = bs; kb < be; kb++) {
+        const int key0 = block_of(kb) << 5;
+        const int64_t pb = (int64_t)tab[key0 / PT] * a.cache.page_stride;
+        const int tok0 = key0 % PT;
+        uint2 vf[DV][2];
+        const uint16_t* vr = pool + pb + a.v_off + ((int64_t)kvh * vdim + n) * PT + tok0 + 4 * g;
+#pragma unroll
+        for (int dv = 0; dv < DV; dv++) {
+            vf[dv][0] = *reinterpret_cast<const uint2*>(vr + (int64_t)16 * dv * PT);
+            vf[dv][1] = *reinterpret_cast<const uint2*>(vr + (int64_t)16 * dv * PT + 16);
+        }
+        if (kb + 1 < be) load_k(block_of(kb + 1), kn);
+        gf32x4_t sacc[2];
+#pragma unroll
+        for (int tt = 0; tt < 2; tt++) {
+            sacc[tt] = gf32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < DK; ks++)
+                sacc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gbf16x8_t, kf[tt][ks]), qf[ks], sacc[tt], 0, 0, 0);
+        }
+        float s[8];
+        bool vis[8];
+        float bm = -1e30f;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const int kj = key0 + 16 * (e >> 2) + 4 * g + (e & 3);
+            vis[e] = valid && kj <= qpos && (kj >= lo_q || kj < a.mask_keep);
+            float x = sacc[e >> 2][e & 3] * a.scale;
+            if (a.softcap > 0.f) x = a.softcap * (1.0f - 2.0f / (1.0f + __expf(x * cap2)));   // c tanh(x / c)
+            if (a.r1) x -= b1 * __logf(1.0f + b2 * (float)max(qpos - kj, 0));
+            x -= slope * (float)max(qpos - kj, 0);
+            s[e] = vis[e] ? x : -1e30f;
+            bm = fmaxf(bm, s[e]);
+        }
+        float alpha = 1.0f, pv[8];
+        if (sig) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) pv[e] = vis[e] ? 1.0f / (1.0f + __expf(-(s[e] + pbh))) : 0.f;
+        } else {
+            bm = xg_max(bm);
+            const float m_new = fmaxf(m_run, bm);
+            alpha = __expf(m_run - m_new);
+            float ls = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                pv[e] = vis[e] ? __expf(s[e] - m_new) : 0.f;
+                ls += pv[e];
+            }
+            ls = xg_sum(ls);
+            l_run = l_run * alpha + ls;
+            m_run = m_new;
+        }
+        const uint4 pu = make_uint4(pack2(pv[0], pv[1]), pack2(pv[2], pv[3]), pack2(pv[4], pv[5]), pack2(pv[6], pv[7]));
+        const gbf16x8_t pf = __builtin_bit_cast(gbf16x8_t, pu);
+#pragma unroll
+        for (int dv = 0; dv < DV; dv++) {
+            const uint4 vu = make_uint4(vf[dv][0].x, vf[dv][0].y, vf[dv][1].x, vf[dv][1].y);
+            if (!sig) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[dv][j] *= alpha;
+            }
+            acc[dv] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gbf16x8_t, vu), pf, acc[dv], 0, 0, 0);
+        }
+#pragma unroll
+        for (int tt = 0; tt < 2; tt++)
+#pragma unroll
+            for (int ks = 0; ks < DK; ks++) kf[tt][ks] = kn[tt][ks];
+    }
     if (S == 1) {
         if (valid) gqa_store<DV>(a, acc, gqa_out_factor(a, l_run, m_run, row, hh), row, hh, qpos, g);
         return;
@@ -974,9 +1095,9 @@ bool gqa_attention_mfma_fits(int dim, int vdim, int page_tokens) {
 template <int DK, int DV>
 static void gqa_mfma_launch2(const GqaAttnMfmaP& p, dim3 grid, hipStream_t st) {
     if (p.pack)
-        hipLaunchKernelGGL((gqa_attn_mfma_kernel<DK, DV, false>), grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL((gqa_attn_pack_kernel<DK, DV>), grid, dim3(256), 0, st, p);
     else
-        hipLaunchKernelGGL((gqa_attn_mfma_kernel<DK, DV, true>), grid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL((gqa_attn_mfma_kernel<DK, DV>), grid, dim3(256), 0, st, p);
     if (p.S > 1) hipLaunchKernelGGL(gqa_attn_combine_kernel<DV>, dim3(grid.x, grid.y, 16), dim3(256), 0, st, p, (int)grid.y * 4);
 }
 template <int DK>
