@@ -23,11 +23,11 @@ namespace qie {
 
 // 16 bytes a lane into LDS: lane l at lds + 16 l.  NT: lines that one workgroup reads, once
 template <bool NT>
-__device__ __forceinline__ void few_lds16(__amdgpu_buffer_rsrc_t rs, void* lds, uint32_t voff, uint32_t soff) {
+__device__ __forceinline__ void few_lds16(__amdgpu_buffer_rsrc_t rs, void* lds, uint32_t voff) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(lds), 16, voff, soff, 0, NT ? 2 : 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(lds), 16, voff, 0, 0, NT ? 2 : 0);
 #else
-    (void)rs; (void)lds; (void)voff; (void)soff;
+    (void)rs; (void)lds; (void)voff;
 #endif
 }
 
@@ -50,15 +50,13 @@ __global__ __launch_bounds__(64 * few::WAVES) void gemm_few_kernel(GemmParams p,
     const int chunks = (int)(p.K >> 6), kb = quotient(part * chunks, parts), n = quotient((part + 1) * chunks, parts) - kb;
     const int mine = n > wave ? (n - wave + NW - 1) / NW : 0;   // chunks kb + wave + NW i of this wave
 
-    // A's and the weights' rows of the tile as buffers: rows past the end read zeros.  A tile lies in one weight segment (few::choose).
+    // A's and the weights' rows of the tile as buffers (few::bytes_from).  A tile lies in one weight segment (few::choose).
     const int rows = (int)(p.M - m0 < BM ? p.M - m0 : BM);
-    const uint32_t a_bytes = (uint32_t)(((int64_t)(rows - 1) * p.lda + p.K) * 2);
     const uint16_t* a0 = p.A + m0 * p.lda;
     const int64_t seg = GATED || c0 < p.n0 ? 0 : c0 < p.n01 ? p.n0 : p.n01, end = GATED ? p.N : c0 < p.n0 ? p.n0 : c0 < p.n01 ? p.n01 : p.N;
     const uint16_t* w0 = (GATED || c0 < p.n0 ? p.w0 : c0 < p.n01 ? p.w1 : p.w2) + (c0 - seg) * p.K;
     const uint16_t* w1 = GATED ? p.w1 + c0 * p.K : w0;
-    const int64_t left = end - c0 < (GATED ? BN / 2 : BN) ? end - c0 : (GATED ? BN / 2 : BN);
-    const uint32_t w_bytes = (uint32_t)left * (uint32_t)p.K * 2;
+    const int left = (int)(end - c0 < (GATED ? BN / 2 : BN) ? end - c0 : (GATED ? BN / 2 : BN));
     auto rsrc = [](const void* base, uint32_t bytes) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000); };
 
     // The fragments that this wave will sum, and what kEpiQkv loads for them ahead of the first chunk
@@ -77,18 +75,18 @@ __global__ __launch_bounds__(64 * few::WAVES) void gemm_few_kernel(GemmParams p,
     // (lane & 7) ^ swz(row); the swizzle of rows 8 on differs in one bit
     unsigned char* ring = smem + wave * (SLOTS * SLOT);
     const int dr = lane >> 3, piece[2] = {((lane & 7) ^ g8_swz(dr)) * 16, ((lane & 7) ^ g8_swz(dr + 8)) * 16};
-    const uint32_t a_row = (uint32_t)dr * (uint32_t)p.lda * 2, w_row = (uint32_t)dr * (uint32_t)p.K * 2;
-    const int a_8 = 8 * (int)p.lda * 2, w_8 = 8 * (int)p.K * 2;   // 8 rows on
     auto load = [&](int slot, int i) {
-        const bool on = i < mine;   // uniform; off: nothing is read, so that every wait is a counted one
-        const int k = (kb + wave + NW * i) * 128;
-        const auto ra = rsrc(a0, on ? a_bytes : 0u), r0 = rsrc(w0, on ? w_bytes : 0u), r1 = GATED ? rsrc(w1, on ? w_bytes : 0u) : r0;
+        const bool on = i < mine;   // uniform; off: buffers of no bytes, so that every wait is a counted one
+        const int64_t k = (int64_t)(kb + wave + NW * i) * 64;
+        const auto ra = rsrc(a0 + k, on ? few::bytes_from(rows, p.lda, p.K, k) : 0u);
+        const uint32_t w_bytes = on ? few::bytes_from(left, p.K, p.K, k) : 0u;
+        const auto r0 = rsrc(w0 + k, w_bytes), r1 = GATED ? rsrc(w1 + k, w_bytes) : r0;
         unsigned char* dst = ring + slot * SLOT;
 #pragma unroll
         for (int b = 0; b < BN / 8; b++)
-            few_lds16<NT>(GATED && (b & 2) ? r1 : r0, dst + b * 1024, w_row + piece[b & 1], k + (GATED ? b / 4 * 2 + (b & 1) : b) * w_8);
+            few_lds16<NT>(GATED && (b & 2) ? r1 : r0, dst + b * 1024, few::row_at(8 * (GATED ? b / 4 * 2 + (b & 1) : b) + dr, p.K) + piece[b & 1]);
 #pragma unroll
-        for (int b = 0; b < BM / 8; b++) few_lds16<false>(ra, dst + BN * 128 + b * 1024, a_row + piece[b & 1], k + b * a_8);
+        for (int b = 0; b < BM / 8; b++) few_lds16<false>(ra, dst + BN * 128 + b * 1024, few::row_at(8 * b + dr, p.lda) + piece[b & 1]);
     };
     f32x4 acc[FI][FJ];
 #pragma unroll
