@@ -21,6 +21,7 @@
 // fp32 or bf16 by the engine's compute type.  A row's result depends only on its own slot,
 // position and cache rows, never on what else the launch holds.
 #include "k_layered.hpp"
+#include "rcp.hpp"
 
 namespace qie {
 namespace lay {
@@ -630,11 +631,8 @@ __device__ __forceinline__ float gqa_out_factor(const GqaAttnP& a, float l, floa
     return f;
 }
 
-// 1 / d, its last bit right but for rare ties; 0 at infinity, NaN stays NaN (an IEEE division is 11 instructions)
-__device__ __forceinline__ float near_rcp(float d) {
-    const float r = __builtin_amdgcn_rcpf(d);
-    return d < 3e38f ? fmaf(fmaf(-d, r, 1.0f), r, r) : r;
-}
+// 1 / d for d >= 1 (rcp_from; an IEEE division is 11 instructions)
+__device__ __forceinline__ float fast_rcp(float d) { return rcp_from(d, __builtin_amdgcn_rcpf(d)); }
 
 // The four waves of a workgroup are four heads of one key head (heads / kv_heads a
 // multiple of 4, one head per wave whatever the group's size): every 32-key K tile and V^T tile
@@ -781,7 +779,7 @@ __global__ __launch_bounds__(256, DV <= 12 && DK + DV <= 16 ? 2 : 1) void gqa_at
         for (int e = 0; e < 8; e++) s[e] = sacc[e >> 2][e & 3] * a.scale;
         if (a.softcap > 0.f) {   // c tanh(x / c)
 #pragma unroll
-            for (int e = 0; e < 8; e++) s[e] = a.softcap * (1.0f - 2.0f * near_rcp(1.0f + __expf(s[e] * cap2)));
+            for (int e = 0; e < 8; e++) s[e] = a.softcap * (1.0f - 2.0f * fast_rcp(1.0f + __expf(s[e] * cap2)));
         }
         if (a.r1) {
 #pragma unroll
