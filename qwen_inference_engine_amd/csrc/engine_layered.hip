@@ -193,11 +193,11 @@ struct LayeredBatch {
     // lin_rows rows for the mixers of lay::linrec_walk
     PieceList pieces, lin[3];         // lin: pieces of 128, 256, 512 rows
     PieceList del[2];                 // delta rule: pieces of 128, 256 rows (64: pieces)
-    std::vector<int> del_units;       // (head, column tile) blocks of the model's delta rules, transition columns included
+    std::vector<std::pair<qie_delta_desc, int64_t>> deltas;   // the model's delta rules, and the stride of their rows of q, k, v
     int max_count = 0;
     int64_t step_T = 0;               // rows of the step being built
     bool ff_branch = false;           // parallel blocks: the layer's feed-forward is running on side[0]
-    bool has_scan = false, has_lin = false;   // layer runs of either kind
+    bool has_scan = false, has_lin = false;   // layer runs of either kind (delta rules: deltas)
     std::vector<int> lin_units;               // (head, column tile) blocks of the model's linear recurrences
     float *s_loc = nullptr, *s_in = nullptr, *s_decay = nullptr;
     int64_t scan_cap = 0;             // pieces the three buffers hold
@@ -2442,9 +2442,9 @@ int layered_batch_create(qie_engine* e, int32_t batch, int32_t max_ctx, int32_t 
         s->m_hd = std::max<int64_t>(s->m_hd, heads * dim);
     };
     auto delta_state = [&](int r, const qie_delta_desc& c) {
-        s->del_units.push_back(delta_units(c));
         // per slot the heads' states and the short convolutions' last inputs
         const int64_t C = 2 * (int64_t)c.kv_heads * c.dim + (int64_t)c.heads * c.vdim;
+        s->deltas.push_back({c, C});
         s->state_off[r] = s->slot_state;
         s->slot_state += (int64_t)c.heads * c.dim * c.vdim;
         s->conv_off[r] = s->slot_state;
@@ -2455,7 +2455,6 @@ int layered_batch_create(qie_engine* e, int32_t batch, int32_t max_ctx, int32_t 
         s->m_dw = std::max<int64_t>(s->m_dw, (int64_t)c.heads * c.dim);
         s->m_state = std::max<int64_t>(s->m_state, (int64_t)c.heads * c.dim * c.vdim);
         s->m_hd = std::max<int64_t>(s->m_hd, (int64_t)c.heads * c.dim * c.dim);
-        s->has_scan = true;
     };
     for (int r = 0; r < n_runs; r++) {
         const int i = m->runs[r].layer;
@@ -2987,11 +2986,13 @@ int qie_batch_step(qie_batch* b, int32_t n_entries, const int32_t* slots, const 
         s->step_T = T;
         s->max_count = 0;
         for (int i = 0; i < n_entries; i++) s->max_count = std::max(s->max_count, (int)counts[i]);
-        if (s->has_scan && s->max_count > kScanLong) QIE_TRY(build_pieces(b, s->pieces, kScanPiece));
-        for (int k = 0; k < 2 && s->max_count > kScanLong; k++) {
-            bool used = false;
-            for (int u : s->del_units) used = used || delta_list_of(T, s->max_count, u) == k + 1;
-            if (used) QIE_TRY(build_pieces(b, s->del[k], 128 << k));
+        if (s->max_count > kScanLong) {
+            bool used[3] = {s->has_scan, false, false};   // pieces of 64, 128, 256 rows.  Delta rules that walk need none
+            for (const auto& [c, ld] : s->deltas)
+                if (!delta_walks(c, ld, T, s->max_count)) used[delta_list_of(T, s->max_count, delta_units(c))] = true;
+            if (used[0]) QIE_TRY(build_pieces(b, s->pieces, kScanPiece));
+            for (int k = 0; k < 2; k++)
+                if (used[k + 1]) QIE_TRY(build_pieces(b, s->del[k], 128 << k));
         }
         for (int k = 0; k < 3 && s->has_lin; k++) {
             s->lin[k].rows = 128 << k;
