@@ -193,7 +193,12 @@ struct LayeredBatch {
     // lin_rows rows for the mixers of lay::linrec_walk
     PieceList pieces, lin[3];         // lin: pieces of 128, 256, 512 rows
     PieceList del[2];                 // delta rule: pieces of 128, 256 rows (64: pieces)
-    std::vector<std::pair<qie_delta_desc, int64_t>> deltas;   // the model's delta rules, and the stride of their rows of q, k, v
+    struct Delta {
+        qie_delta_desc c;
+        int64_t ld;       // of their rows of q, k, v
+        bool beside;      // an attention's other half
+    };
+    std::vector<Delta> deltas;        // the model's delta rules
     int max_count = 0;
     int64_t step_T = 0;               // rows of the step being built
     bool ff_branch = false;           // parallel blocks: the layer's feed-forward is running on side[0]
@@ -1820,14 +1825,19 @@ static int enq_delta_gates(qie_batch* b, int r, int T) {
     return dense(b, s->proj + L.col_g1, L.n_in, L.w_g2, s->aux, (int64_t)c.heads * c.vdim, T, c.heads * c.vdim, L.rank_g);
 }
 
-// Entries of more than a few rows walk them in order (lay::delta_walk) where that takes less than pieces: 0.158 us a row of the longest entry, against
+// Entries of more than a few rows walk them in order (lay::delta_walk) where that takes less than pieces: 0.16 us a row of the longest entry, against
 // three launches, and all rows' columns twice.  us with the convolutions before, pieces | walk: 16 heads of 128, 20 rows 31 | 16, 300 rows 143 | 73,
-// 4 entries of 465 316 | 141, 11 of 900 1,430 | 650, one of 2,500 456 | 422; 16 heads of 64, 4 of 465 125 | 100, 11 of 900 439 | 273, but one of
-// 900 117 | 158, of 2,500 177 | 406.  (kLinStep: steps that are captured keep the side of it that their key names.)
-static bool delta_walks(const qie_delta_desc& c, int64_t ld, int64_t T, int max_count) {
+// 4 entries of 465 316 | 132, 11 of 900 1,430 | 621, one of 2,500 453 | 420, 4,000 668 | 655, 6,000 848 | 989; 16 heads of 64, 4 of 465 123 | 98, one of
+// 500 108 | 94, 700 113 | 124, 900 119 | 154, 2,500 178 | 397.
+// Beside an attention and a feed-forward (`beside`) a row takes up to twice that, but pieces slow the others down: a chain of long entries is the
+// better one for longer, and a whole step of Nukizen is at most 3 % from the better form.  us a step, pieces | walk: 2k, 300 rows 700 | 628, 900 rows 1,055
+// | 964, 4 of 465 1,555 | 1,415, 11 of 900 6,900 | 5,970, one of 2,500 2,087 | 2,135, 4,000 3,120 | 2,910, 8,000 5,475 | 5,375, of 2,500 and 11 rows
+// 2,200 | 2,230; 1k, 300 rows 468 | 428, 900 570 | 604, 3 of 1,200 1,138 | 1,160, 6 of 900 1,550 | 1,460.
+// (kLinStep: steps that are captured keep the side of it that their key names.)
+static bool delta_walks(const qie_delta_desc& c, int64_t ld, int64_t T, int max_count, bool beside) {
     if (max_count <= kLinStep || !lay::delta_walk_fits(c.dim, ld)) return false;
-    const float pieces = 60.f + 3.05e-7f * (float)c.heads * (float)c.dim * (float)(c.dim + c.vdim) * (float)T;
-    return max_count <= kScanLong || .158f * (float)max_count <= pieces;
+    const float columns = (float)c.heads * (float)c.dim * (float)(c.dim + c.vdim) * (float)T, L = (float)max_count;
+    return max_count <= kScanLong || (beside ? .158f * L <= 60.f + 3.05e-7f * columns : 20.f + .16f * L <= 107.f + 2.6e-7f * columns);
 }
 
 static int enq_delta_scan(qie_batch* b, int r, int T, bool advance, hipStream_t st) {
@@ -1837,7 +1847,7 @@ static int enq_delta_scan(qie_batch* b, int r, int T, bool advance, hipStream_t 
     const qie_delta_desc& c = L.d.delta;
     LayeredBatch* s = b->lb;
     const int C = 2 * c.kv_heads * c.dim + c.heads * c.vdim;
-    const bool head = c.decay == QIE_DELTA_HEAD;
+    const bool head = c.decay == QIE_DELTA_HEAD, beside = L.d.mixer == QIE_MIXER_GQA_RECURRENT;
     lay::CausalConvP cv{};
     cv.in = s->proj; cv.ld_in = L.n_in; cv.col = L.col_d; cv.C = C; cv.taps = c.conv; cv.w = L.dl_conv;
     cv.row_slot = s->row_slot; cv.row_pos = s->row_pos; cv.row_k = s->row_k;
@@ -1860,7 +1870,7 @@ static int enq_delta_scan(qie_batch* b, int r, int T, bool advance, hipStream_t 
     sp.state = s->state; sp.slot_stride = s->slot_state; sp.state_off = s->state_off[r];
     sp.read_state = 1; sp.write_state = advance ? 1 : 0;
     sp.out = s->olat;
-    if (delta_walks(c, C, s->step_T, s->max_count)) {
+    if (delta_walks(c, C, s->step_T, s->max_count, beside)) {
         QIE_TRY(lay::delta_walk(sp, st));
     } else if (s->max_count > kScanLong && s->s_loc && s->dw) {
         // long entries: pieces from zero states side by side (end states, transition matrices, transformed
@@ -1882,7 +1892,6 @@ static int enq_delta_scan(qie_batch* b, int r, int T, bool advance, hipStream_t 
     } else {
         QIE_TRY(lay::delta_scan(sp, st));
     }
-    const bool beside = L.d.mixer == QIE_MIXER_GQA_RECURRENT;
     return lay::head_norm_rows(s->olat, nullptr, L.dl_norm, m->a.norm_eps, rec_out_scale(L.d), c.heads, c.vdim, T, ov_out(b, L), s->ov_bf,
                                L.n_cat, beside ? L.cat_rec : 0, st, head ? s->proj + L.col_g1 : s->aux, head ? L.n_in : 0, head ? 1 : 0);
 }
@@ -2441,10 +2450,10 @@ int layered_batch_create(qie_engine* e, int32_t batch, int32_t max_ctx, int32_t 
         s->m_state = std::max<int64_t>(s->m_state, heads * dim * vdim);
         s->m_hd = std::max<int64_t>(s->m_hd, heads * dim);
     };
-    auto delta_state = [&](int r, const qie_delta_desc& c) {
+    auto delta_state = [&](int r, const qie_delta_desc& c, bool beside) {
         // per slot the heads' states and the short convolutions' last inputs
         const int64_t C = 2 * (int64_t)c.kv_heads * c.dim + (int64_t)c.heads * c.vdim;
-        s->deltas.push_back({c, C});
+        s->deltas.push_back({c, C, beside});
         s->state_off[r] = s->slot_state;
         s->slot_state += (int64_t)c.heads * c.dim * c.vdim;
         s->conv_off[r] = s->slot_state;
@@ -2464,7 +2473,7 @@ int layered_batch_create(qie_engine* e, int32_t batch, int32_t max_ctx, int32_t 
             s->slot_state += (int64_t)(m->a.canon_taps - 1) * m->a.width;
         }
         if (d.mixer == QIE_MIXER_CHANNEL_DELTA) {
-            delta_state(r, d.delta);   // no cache rows
+            delta_state(r, d.delta, false);   // no cache rows
             s->m_in = std::max<int64_t>(s->m_in, m->L[i].n_in);
             s->m_hv = std::max<int64_t>(s->m_hv, m->L[i].n_cat);
             s->m_abf = std::max<int64_t>({s->m_abf, (int64_t)m->a.width, (int64_t)m->L[i].n_cat});
@@ -2523,7 +2532,7 @@ int layered_batch_create(qie_engine* e, int32_t batch, int32_t max_ctx, int32_t 
             }
             const int64_t rv = rec_cols(d);
             if (rv && d.rec.kind == QIE_REC_DELTA) {
-                delta_state(r, d.delta);
+                delta_state(r, d.delta, true);
             } else if (rv) {
                 s->state_off[r] = s->slot_state;
                 s->slot_state += (int64_t)d.rec.heads * d.rec.dim * d.rec.vdim;
@@ -2988,8 +2997,8 @@ int qie_batch_step(qie_batch* b, int32_t n_entries, const int32_t* slots, const 
         for (int i = 0; i < n_entries; i++) s->max_count = std::max(s->max_count, (int)counts[i]);
         if (s->max_count > kScanLong) {
             bool used[3] = {s->has_scan, false, false};   // pieces of 64, 128, 256 rows.  Delta rules that walk need none
-            for (const auto& [c, ld] : s->deltas)
-                if (!delta_walks(c, ld, T, s->max_count)) used[delta_list_of(T, s->max_count, delta_units(c))] = true;
+            for (const auto& d : s->deltas)
+                if (!delta_walks(d.c, d.ld, T, s->max_count, d.beside)) used[delta_list_of(T, s->max_count, delta_units(d.c))] = true;
             if (used[0]) QIE_TRY(build_pieces(b, s->pieces, kScanPiece));
             for (int k = 0; k < 2; k++)
                 if (used[k + 1]) QIE_TRY(build_pieces(b, s->del[k], 128 << k));
