@@ -402,10 +402,17 @@ struct Plan {
 // the norm's launch with `parts` to add; alone it takes 2.6 and 1.1 for a million values
 inline float sum_us(int64_t M, int64_t N, int64_t parts) { return 2.59f + 1.55e-6f * (float)(parts * M * N); }
 
-// Against product and norm apart, 157 of 190 shapes at 17 to 1,300 rows come here, in 0.85 of their time on the average (the best of all forms and parts: 0.84),
-// 0.70 to 1.03 but for Qwen3-14B down at 1,000 rows (172.7 us | 178.4 at the .95 that 900 rows and more had then).  us: Qwen2-7B down at 113 rows 46.1 | 38.3, 301
-// rows 68.0 | 59.4, O at 301 rows 27.0 | 24.1; Qwen3-14B down at 113 rows 55.8 | 46.1; Qwen2-0.5B down at 113 rows 13.0 | 10.6, O 9.2 | 6.6.  From 700 rows on the
-// parts' bytes take what they give, but where the tiles leave CUs idle (4,864 -> 896 at 800 rows 25.0 | 21.9).
+// us, apart | here: Qwen2-7B down at 113 rows 46.1 | 38.3, 301 rows 68.0 | 59.4, O at 301 rows 27.0 | 24.1; Qwen3-14B down at 113 rows 55.8 | 46.1;
+// Qwen2-0.5B down at 113 rows 13.0 | 10.6, O at 33 rows 6.6 | 6.2.  From 700 rows on the parts' bytes take what they give, but where the tiles leave CUs
+// idle (4,864 -> 896 at 800 rows 25.0 | 21.9).
+// How much of the expected time of product and norm apart a plan may take: the fit is some percent off either way, by sizes.  Of weights of 8M and more, and of
+// up to 64 rows, cut products take less than it says (5,120 x 17,408 at 113 rows 1.006 expected, 0.835 measured; 3,584 x 18,944 at 17 rows 0.994, 0.885).
+// Of smaller weights at more rows they take more where rows are multiples of 512 (1,024 x 2,816 at 400 rows 0.989, 1.133; 2,048 x 2,048 at 640 rows
+// 1.01, 1.081), else what it says or less (896 x 896 at 113 rows 1.006, 0.977).  Of 470 such plans, of 30 projections (256 to 5,120 wide) at 17 to 1,000
+// rows, 374 are taken so, in 0.93 of the time on the average; 5 take 2.5 % longer or more, 1.063 at worst.  (All up to 1.03: 44, 1.133 at worst.)
+inline float worth(int64_t M, int64_t N, int64_t K) {
+    return M > 700 ? .9f : M <= 64 || N * K >= 8 << 20 ? 1.03f : N % 512 != 0 ? 1.015f : .97f;
+}
 inline Plan choose(int64_t M, int64_t N, int64_t K, int64_t cus) {
     Plan best{-1, -1, 1, 1e30f};
     if (K % 64 != 0 || N % 8 != 0 || M <= 16 || M > 1024) return best;
@@ -429,7 +436,7 @@ inline Plan choose(int64_t M, int64_t N, int64_t K, int64_t cus) {
     }
     const few::Plan whole = few::choose(M, N, K, cus, false, false);
     const float now = std::min(whole.us, few::others(M, N, K, cus)) + 2.6f + 1.1e-6f * (float)(M * N);
-    return best.us < (M > 700 ? .9f : 1.03f) * now ? best : Plan{-1, -1, 1, 1e30f};
+    return best.us < worth(M, N, K) * now ? best : Plan{-1, -1, 1, 1e30f};
 }
 }  // namespace apart
 

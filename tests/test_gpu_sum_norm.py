@@ -50,6 +50,16 @@ def test_plans(tmp_path):
         assert (f >= 0) + (t >= 0) <= 1 and 1 <= p <= max(1, min(16, K // 64)) and p * M * N <= (16 << 20 if p > 1 else 1 << 40)
 
 
+# rows, columns, K, us apart and in the parts that the fit prefers or has on a level
+MEASURED = [(400, 1024, 2816, 11.2, 12.7), (640, 2048, 2048, 20.5, 22.1), (301, 2048, 2048, 13.5, 14.8), (512, 1024, 1024, 8.2, 9.0), (512, 512, 1536, 7.8, 8.4),
+            (301, 512, 2048, 7.8, 8.8), (17, 3584, 18944, 30.6, 27.1), (113, 5120, 17408, 55.1, 46.0), (80, 5120, 5120, 23.4, 22.0), (113, 896, 896, 6.73, 6.57)]
+
+
+def test_plans_that_measured_longer_are_not_taken(tmp_path):
+    for c, (f, t, _) in zip(MEASURED, plans(tmp_path, [c[:3] for c in MEASURED])):
+        assert (f >= 0 or t >= 0) == (c[4] < c[3]), c
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("numerics", [_lib.QIE_NUMERICS_REF, _lib.QIE_NUMERICS_HF])
 @pytest.mark.parametrize("M,N,K", SHAPES + APART_NOT[1:])
