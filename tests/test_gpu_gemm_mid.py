@@ -49,8 +49,8 @@ PLANS = [(17, 72, 64, 0, "whole"), (33, 72, 2048, 0, "split"), (17, 40000, 128, 
          (210, 9278, 6464, 5, "split"), (273, 38147, 1792, 6, "mixed"), (259, 12692, 64, 6, "whole"), (1064, 11882, 1728, 7, "mixed"),
          (257, 8338, 11264, 7, "split")]
 SHAPES = [p[:3] for p in PLANS]
-# Other tiles, or two launches, are the better choice for half of those; with these qie_linear comes to every tile in every way that is left
-MORE = [(129, 44169, 128), (72, 42624, 2048), (70, 16787, 320), (131, 42200, 2880), (130, 20894, 64), (193, 20859, 448), (261, 47014, 1536), (838, 28106, 64)]
+# Other tiles, k_gemm_few.hip or two launches are the better choice for half of those; with these qie_linear comes to every tile in every way that is left
+MORE = [(129, 44169, 128), (72, 42624, 2048), (70, 16787, 320), (131, 42200, 2880), (130, 20894, 64), (193, 20859, 448), (261, 47014, 1536), (838, 28106, 64), (33, 72, 12416)]
 GROWS = (130, 22370, 17472)   # partial tiles of more than the 64 MB that a stream has from the start
 
 

@@ -1,6 +1,6 @@
 """The QKV product whose epilogue turns q and k and writes the cache (gemm_qkv, what a prompt's layers call) against the product and
-qie_qkv_post: the same bits.  Every tile of k_gemm_mid.hip and the 256x256 kernel, split and whole, ragged rows, several prompts in a tile, heads of
-8, 64 and 128, contiguous and paged; and a K that no kernel with that epilogue takes."""
+qie_qkv_post: the same bits.  Every form of k_gemm_few.hip, every tile of k_gemm_mid.hip and the 256x256 kernel, split and whole, ragged rows, several prompts
+in a tile, heads of 8, 64 and 128, contiguous and paged; and a K that no kernel with that epilogue takes."""
 import ctypes as C
 
 import numpy as np
@@ -15,9 +15,13 @@ from qwen_inference_engine_amd._lib import KvCacheC, LinearArgsC
 SYMBOL = "_ZN3qie8gemm_qkvEPK15qie_linear_argsPK12qie_kv_cacheiiPKfPtP12ihipStream_tPb"
 
 
-# heads, key heads, head size, K, rows of a prompt, prompts, page, tile (k_gemm_mid.hip's, -1: the 256x256 kernel, None: one without this epilogue)
+# heads, key heads, head size, K, rows of a prompt, prompts, page, tile (k_gemm_mid.hip's, "few 0" ..: k_gemm_few.hip's forms, -1: the 256x256 kernel,
+# None: one without this epilogue)
 CASES = [
-    (14, 2, 64, 896, 17, 1, 0, 0), (14, 2, 64, 896, 113, 1, 128, 0), (14, 2, 64, 896, 37, 5, 128, 0),
+    (14, 2, 64, 896, 17, 1, 0, "few 0"), (14, 2, 64, 896, 113, 1, 128, "few 1"), (14, 2, 64, 896, 37, 5, 128, "few 1"),
+    (28, 4, 128, 3584, 71, 1, 128, "few 2"), (28, 4, 128, 3584, 31, 3, 0, "few 2"), (14, 2, 64, 896, 301, 1, 0, "few 3"),
+    (14, 2, 64, 896, 79, 5, 128, "few 3"), (28, 4, 128, 3584, 183, 1, 128, "few 4"), (28, 4, 128, 3584, 61, 3, 0, "few 4"),
+    (14, 2, 64, 896, 507, 1, 128, 0), (14, 2, 64, 256, 75, 4, 0, 0), (2, 1, 64, 2048, 601, 1, 128, 0), (2, 1, 64, 12288, 70, 3, 0, 0),
     (14, 2, 64, 896, 1501, 1, 0, 1), (28, 4, 128, 3584, 63, 1, 128, 0), (28, 4, 128, 3584, 301, 1, 0, 2),
     (28, 4, 128, 3584, 1030, 1, 128, 4), (28, 4, 128, 512, 2100, 2, 256, -1), (28, 4, 128, 512, 1363, 3, 0, -1),
     (3, 1, 8, 256, 65, 2, 0, 0), (14, 2, 64, 928, 300, 1, 0, None), (28, 4, 128, 3584, 2500, 1, 0, -1), (28, 4, 128, 3584, 2048, 1, 128, 7),
@@ -27,12 +31,15 @@ CASES = [
 
 
 def test_cases_take_every_kernel_with_the_epilogue():
-    got = routes([(c[4] * c[5], (c[0] + 2 * c[1]) * c[2], c[3]) for c in CASES])
+    got = routes([(c[4] * c[5], (c[0] + 2 * c[1]) * c[2], c[3], 0, c[0] * c[2] % 64 != 0 or c[1] * c[2] % 64 != 0) for c in CASES])
     for c, r in zip(CASES, got):
-        assert c[7] is None and c[3] % 64 != 0 or c[7] is not None and r["tile"] == c[7] and (c[7] >= 0 or r["parts"] >= 1), (c, r)
-    assert {r["tile"] for r in got} == set(range(-1, 12))
+        if c[7] is None:
+            assert c[3] % 64 != 0, c
+        else:
+            assert ("few %d" % r["few"] if r["few"] >= 0 else r["tile"]) == c[7] and (c[7] != -1 or r["parts"] >= 1), (c, r)
+    assert {r["tile"] for r in got} == set(range(-2, 12)) and {r["few"] for r in got} == set(range(-1, 5))
     assert {r["parts"] for r, c in zip(got, CASES) if c[7] == -1} >= {1, 2}   # the 256x256 kernel whole and split
-    assert any(r["splitk"] > 1 for r in got)
+    assert {r["splitk"] > 1 for r in got if r["tile"] == 0} == {False, True}
 
 
 @pytest.mark.gpu
