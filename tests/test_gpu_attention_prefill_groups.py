@@ -1,20 +1,29 @@
-"""Prefill attention by single row groups a wave, in workgroups of 4 and 8 (k_attention.hip prefill_attn_plan), beside the pairs: ragged rows, waves
-without a group, several sequences, pages, NaN in the cache behind the rows; against softmax attention in 64 bits."""
+"""Prefill attention by single row groups a wave, in workgroups of 4 and 8 waves, and by pairs of them in workgroups of 2, 4 and 8 (attn_plan.hpp): ragged
+rows, waves without a group or a pair, a middle group without a partner, several sequences, pages, NaN in the cache behind the rows; against softmax
+attention in 64 bits."""
 import ctypes as C
 
 import pytest
 import torch
 
 import gpu_util as G
+from attn_route import forms
 from qwen_inference_engine_amd import _lib
 
-pytestmark = pytest.mark.gpu
+# rows, sequences, heads, key heads, head size, page, (waves of a workgroup, groups of a wave)
+CASES = [(33, 1, 14, 2, 64, 0, (4, 1)), (65, 3, 14, 2, 64, 128, (4, 1)), (500, 8, 14, 2, 64, 128, (4, 1)), (49, 2, 7, 7, 128, 0, (4, 1)), (420, 1, 28, 4, 128, 128, (4, 1)),
+         (1210, 1, 28, 4, 128, 0, (4, 1)), (301, 8, 28, 4, 128, 0, (8, 1)), (1601, 1, 40, 8, 128, 128, (8, 1)),
+         (1100, 1, 14, 2, 64, 0, (2, 2)), (1030, 1, 14, 2, 64, 128, (2, 2)), (250, 4, 14, 2, 64, 128, (2, 2)), (1000, 1, 28, 4, 128, 0, (4, 2)), (1030, 1, 28, 4, 128, 128, (4, 2)),
+         (470, 2, 28, 4, 128, 0, (4, 2)), (1801, 1, 28, 4, 128, 128, (8, 2)), (2290, 1, 28, 4, 128, 0, (8, 2)), (950, 2, 28, 4, 128, 128, (8, 2)), (1000, 2, 28, 4, 128, 0, (8, 2))]
 
 
-# rows, sequences, heads, key heads, head size, page: single groups in 4 waves, in 8, pairs that fill the chip
-@pytest.mark.parametrize("R,B,nq,nkv,hd,page", [(33, 1, 14, 2, 64, 0), (65, 3, 14, 2, 64, 128), (1100, 1, 14, 2, 64, 0), (500, 8, 14, 2, 64, 128), (49, 2, 7, 7, 128, 0),
-                                                (420, 1, 28, 4, 128, 128), (1210, 1, 28, 4, 128, 0), (301, 8, 28, 4, 128, 0), (1601, 1, 40, 8, 128, 128), (1000, 1, 28, 4, 128, 0)])
-def test_single_groups(qlib, R, B, nq, nkv, hd, page):
+def test_cases_take_every_form():
+    assert forms([(c[0], c[1], c[2], c[4]) for c in CASES]) == [c[6] for c in CASES]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("R,B,nq,nkv,hd,page,form", CASES)
+def test_single_groups(qlib, R, B, nq, nkv, hd, page, form):
     g = torch.Generator().manual_seed(R + B)
     pages = -(-R // page) if page else 0
     room, M = page or R + 70, B * R

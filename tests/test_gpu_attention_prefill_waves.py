@@ -1,19 +1,25 @@
-"""Prefill attention in workgroups of 2, 4 and 8 waves (k_attention.hip prefill_attn_waves: by the rows, heads and sequences of a call): ragged
-rows, waves without a pair of row groups, NaN in the cache behind the rows, several sequences; against softmax attention in 64 bits."""
+"""Prefill attention of few rows and of many, one sequence and several (attn_plan.hpp: workgroups by the rows, heads and sequences of a call): ragged
+rows, waves without rows, NaN in the cache behind the rows; against softmax attention in 64 bits."""
 import ctypes as C
 
 import pytest
 import torch
 
 import gpu_util as G
+from attn_route import forms
 from qwen_inference_engine_amd import _lib
 
-pytestmark = pytest.mark.gpu
+# rows, sequences, heads, key heads, head size
+CASES = [(32, 1, 14, 2, 64), (113, 2, 14, 2, 64), (301, 1, 28, 4, 128), (449, 1, 7, 7, 128), (620, 1, 28, 4, 128), (1310, 1, 28, 4, 128), (301, 8, 28, 4, 128)]
 
 
-# rows, sequences, heads, key heads, head size: 2 waves for the first four, then 4, 8, and 4 in more than one round of the chip
-@pytest.mark.parametrize("R,B,nq,nkv,hd", [(32, 1, 14, 2, 64), (113, 2, 14, 2, 64), (301, 1, 28, 4, 128), (449, 1, 7, 7, 128), (620, 1, 28, 4, 128),
-                                           (1310, 1, 28, 4, 128), (301, 8, 28, 4, 128)])
+def test_forms():
+    """Single groups in 4 waves and, beyond one round of the chip, in 8 (pairs: test_gpu_attention_prefill_groups.py)."""
+    assert forms([(R, B, nq, hd) for R, B, nq, nkv, hd in CASES]) == [(4, 1)] * 6 + [(8, 1)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("R,B,nq,nkv,hd", CASES)
 def test_rows_of_every_workgroup(qlib, R, B, nq, nkv, hd):
     g = torch.Generator().manual_seed(R + B)
     room, M = R + 70, B * R
