@@ -26,16 +26,6 @@ __device__ __forceinline__ void dma16(const uint16_t* src, uint16_t* lds) {
                                      (__attribute__((address_space(3))) void*)(lds), 16, 0, 0);
 }
 
-// 16 bytes per lane from a buffer resource into LDS (buffer_load_dwordx4 … lds); `lds` is the
-// wave-instruction's 1-KiB base.  (The builtin exists for the device pass only: the host
-// pass, which emits the kernel's launch stub, must not instantiate it.)
-__device__ __forceinline__ void buf_lds16(__amdgpu_buffer_rsrc_t rs, uint16_t* lds, uint32_t voff) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(lds), 16, voff, 0, 0, 0);
-#else
-    (void)rs; (void)lds; (void)voff;
-#endif
-}
 
 // ---------------------------------------------------------------------------
 // Fused decode attention: q-projection post-processing (qk-norm + RoPE) in the

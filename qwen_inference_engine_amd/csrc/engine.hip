@@ -755,7 +755,8 @@ static int ensure_prefill_scratch(qie_batch* b, int64_t n) {
     }
     QIE_TRY(dmalloc((void**)&b->pf_pos, n * 4));
     QIE_TRY(dmalloc((void**)&b->pf_ids, n * 4));
-    // attention of prompts needs a workspace only for one row of each: prompts of one token, and the last rows in the last layer
+    // attention of prompts needs a workspace only for one row of each: prompts of one token, and the last rows in the last layer.  The bytes for
+    // all slots cover fewer rows as well: a batch has at most 8 (batch_create), and up to 8 rows the splits of a row are the same (attn_nsplit)
     QIE_TRY(dmalloc(&b->pf_attn_ws, (size_t)qie_attention_workspace_bytes(b->B, sh.nq, s.head_dim, b->max_ctx)));
     b->pf_rows = n;
     return 0;

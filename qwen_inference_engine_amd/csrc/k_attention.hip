@@ -329,8 +329,8 @@ __global__ __launch_bounds__(64 * NW, QG == 1 ? 4 : NW == 8 ? 1 : 2) void attn_p
 #pragma unroll
         for (int i = 0; i < IPW; i++) {
             const int inst = wave * IPW + i;
-            buf_lds16(rk, Ks + buf * KT * HD + inst * 512, koff[i]);
-            buf_lds16(rv, Vs + buf * KT * HD + inst * 512, voff[i]);
+            buffer_lds16(rk, Ks + buf * KT * HD + inst * 512, koff[i], 0);
+            buffer_lds16(rv, Vs + buf * KT * HD + inst * 512, voff[i], 0);
         }
     };
 

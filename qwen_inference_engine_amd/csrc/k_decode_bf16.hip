@@ -71,15 +71,6 @@ struct DecBfParams {
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t db_rsrc(const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
 }
-// 16 bytes a lane into LDS: lane l at lds + 16 l.  NT: lines that one workgroup reads, once
-template <bool NT = false>
-__device__ __forceinline__ void db_lds16(__amdgpu_buffer_rsrc_t rs, void* lds, uint32_t voff, uint32_t soff) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(lds), 16, voff, soff, 0, NT ? 2 : 0);
-#else
-    (void)rs; (void)lds; (void)voff; (void)soff;
-#endif
-}
 
 constexpr int kEpiGated = 5;   // after the QIE_EPI_ values: rows[0] rows as QIE_EPI_F32, then pairs of rows of w[1] and w[2] (lay::GatedP)
 
@@ -129,7 +120,7 @@ __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
     } else if constexpr (XM == 0) {
         for (int m = wave; m < M; m += db::NW) {
             const auto rx = db_rsrc(p.x + (int64_t)m * p.ldx, (uint32_t)K * 2);
-            for (int c = 0; c * 512 < K; c++) db_lds16(rx, xs + m * p.xstride + c * 1024, lane * 16, c * 1024);
+            for (int c = 0; c * 512 < K; c++) buffer_lds16(rx, xs + m * p.xstride + c * 1024, lane * 16, c * 1024);
         }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -208,10 +199,10 @@ __global__ __launch_bounds__(512) void dec_bf16_kernel(DecBfParams p) {
         const uint32_t k = (uint32_t)(c0 + n_c) * 256;
         const auto r0 = db_rsrc(wb0, on ? wbytes : 0u), r1 = EPI == QIE_EPI_SWIGLU || EPI == kEpiGated ? db_rsrc(wb1, on ? wbytes : 0u) : r0;
 #pragma unroll
-        for (int i = 0; i < 4; i++) db_lds16<true>(i < 2 ? r0 : r1, dst + i * 1024, wsrc[i], k);
+        for (int i = 0; i < 4; i++) buffer_lds16<true>(i < 2 ? r0 : r1, dst + i * 1024, wsrc[i], k);
         if constexpr (XM != 0) {
 #pragma unroll
-            for (int i = 0; i < XM / 4; i++) db_lds16(db_rsrc(p.x, on ? xbytes : 0u), dst + db::WCH + i * 1024, xsrc[i], k);
+            for (int i = 0; i < XM / 4; i++) buffer_lds16(db_rsrc(p.x, on ? xbytes : 0u), dst + db::WCH + i * 1024, xsrc[i], k);
         }
         n_slot = n_slot + 1 == R ? 0 : n_slot + 1;
         if (++n_c == cnt) {

@@ -857,15 +857,6 @@ constexpr int slots(int xr) { return xr == 8 ? 4 : 5; }   // of a wave's ring
 constexpr int lds(int xr) { return NW * slots(xr) * (WCH + xr * CH * 2) + 2 * NW * 512; }
 }  // namespace d8s
 
-// 16 bytes a lane into LDS: lane l at lds + 16 l.  NT: lines that nobody reads again
-template <bool NT>
-__device__ __forceinline__ void d8_lds16(__amdgpu_buffer_rsrc_t rs, void* lds, uint32_t voff, uint32_t soff) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(lds), 16, voff, soff, 0, NT ? 2 : 0);
-#else
-    (void)rs; (void)lds; (void)voff; (void)soff;
-#endif
-}
 
 template <int EPI, bool T16, int XR>
 __global__ __launch_bounds__(512) void dec8s_kernel(Dec8Params p) {
@@ -932,9 +923,9 @@ __global__ __launch_bounds__(512) void dec8s_kernel(Dec8Params p) {
         unsigned char* dst = ring + n_slot * SLOT;
         const int c = c0 + n_c;
 #pragma unroll
-        for (int u = 0; u < 2; u++) d8_lds16<true>(on ? rw : none, dst + u * 1024, wv, ws + (uint32_t)(2 * c + u) * (T16 ? 1024 : 64));
+        for (int u = 0; u < 2; u++) buffer_lds16<true>(on ? rw : none, dst + u * 1024, wv, ws + (uint32_t)(2 * c + u) * (T16 ? 1024 : 64));
 #pragma unroll
-        for (int i = 0; i < XR / 4; i++) d8_lds16<false>(on ? rx : none, dst + d8s::WCH + i * 1024, xsrc[i], (uint32_t)c * 256);
+        for (int i = 0; i < XR / 4; i++) buffer_lds16<false>(on ? rx : none, dst + d8s::WCH + i * 1024, xsrc[i], (uint32_t)c * 256);
         n_slot = n_slot + 1 == R ? 0 : n_slot + 1;
         if (++n_c == cnt) {
             n_c = 0;

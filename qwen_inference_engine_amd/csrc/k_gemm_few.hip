@@ -21,15 +21,6 @@
 
 namespace qie {
 
-// 16 bytes a lane into LDS: lane l at lds + 16 l.  NT: lines that one workgroup reads, once
-template <bool NT>
-__device__ __forceinline__ void few_lds16(__amdgpu_buffer_rsrc_t rs, void* lds, uint32_t voff) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(lds), 16, voff, 0, 0, NT ? 2 : 0);
-#else
-    (void)rs; (void)lds; (void)voff;
-#endif
-}
 
 // FI, FJ: fragments of 16 rows of A, of 16 weight rows (SwiGLU: gate and up in turn); SLOTS of a wave's ring; NT: weights that one row tile reads
 template <int EPI, int FI, int FJ, int SLOTS, bool NT>
@@ -84,9 +75,9 @@ __global__ __launch_bounds__(64 * few::WAVES) void gemm_few_kernel(GemmParams p,
         unsigned char* dst = ring + slot * SLOT;
 #pragma unroll
         for (int b = 0; b < BN / 8; b++)
-            few_lds16<NT>(GATED && (b & 2) ? r1 : r0, dst + b * 1024, few::row_at(8 * (GATED ? b / 4 * 2 + (b & 1) : b) + dr, p.K) + piece[b & 1]);
+            buffer_lds16<NT>(GATED && (b & 2) ? r1 : r0, dst + b * 1024, few::row_at(8 * (GATED ? b / 4 * 2 + (b & 1) : b) + dr, p.K) + piece[b & 1], 0);
 #pragma unroll
-        for (int b = 0; b < BM / 8; b++) few_lds16<false>(ra, dst + BN * 128 + b * 1024, few::row_at(8 * b + dr, p.lda) + piece[b & 1]);
+        for (int b = 0; b < BM / 8; b++) buffer_lds16<false>(ra, dst + BN * 128 + b * 1024, few::row_at(8 * b + dr, p.lda) + piece[b & 1], 0);
     };
     f32x4 acc[FI][FJ];
 #pragma unroll

@@ -63,6 +63,18 @@ inline int dev_env(const char*, int dflt) { return dflt; }
 #define QIE_DBG(expr) false
 #endif
 
+// ------------------------------------------------------------- loads into LDS
+// 16 bytes a lane from a buffer into LDS, lane l at lds + 16 l.  NT: lines that one workgroup reads, once.  Past the buffer's end: zeros, nothing is
+// read.  (The compiler's manual says that for voff; gfx950 counts soff as well, also where it alone lies behind the end.)
+template <bool NT = false>
+__device__ __forceinline__ void buffer_lds16(__amdgpu_buffer_rsrc_t rs, void* lds, uint32_t voff, uint32_t soff) {
+#if defined(__HIP_DEVICE_COMPILE__)   // (the builtin is the device pass's alone)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(lds), 16, voff, soff, 0, NT ? 2 : 0);
+#else
+    (void)rs; (void)lds; (void)voff; (void)soff;
+#endif
+}
+
 // ------------------------------------------------------------- bf16 helpers
 __device__ __forceinline__ float bf2f(uint32_t h16) { return __uint_as_float(h16 << 16); }
 __device__ __forceinline__ float bf_lo(uint32_t w) { return __uint_as_float(w << 16); }

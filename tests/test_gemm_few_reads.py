@@ -41,5 +41,5 @@ def test_rows_that_do_not_exist_are_not_read(tmp_path):
 
 def test_loads_have_no_scalar_offset():
     text = open(os.path.join(CSRC, "k_gemm_few.hip")).read()
-    calls = re.findall(r"raw_ptr_buffer_load_lds\((.*)\);", text)
-    assert calls and all(re.search(r", 16, voff, 0, 0, ", c) for c in calls), calls
+    calls = re.findall(r"buffer_lds16<.*;", text)
+    assert len(calls) == 2 and all(c.endswith(", 0);") for c in calls) and "raw_ptr_buffer_load_lds" not in text, calls
