@@ -11,8 +11,8 @@ from test_gpu_gemm_mid import bf16, linear, products
 
 pytestmark = pytest.mark.gpu
 
-# rows, weight rows, K, tile, parts
-SHAPES = [(17, 72, 64, 0, 1), (33, 72, 2048, 0, 4), (17, 16500, 64, 1, 1), (64, 8200, 4096, 1, 3), (65, 8200, 1024, 2, 1), (129, 4000, 4096, 2, 2),
+# rows, weight rows, K, tile, parts (gate and up of up to 32 rows: k_gemm_few.hip)
+SHAPES = [(17, 72, 64, 0, 1), (35, 104, 128, 0, 1), (33, 72, 12416, 0, 9), (17, 16500, 64, 1, 1), (35, 112, 192, 1, 1), (64, 8200, 4096, 1, 3), (65, 8200, 1024, 2, 1), (129, 4000, 4096, 2, 2),
           (301, 9728, 896, 3, 1), (128, 8200, 4096, 3, 3), (131, 11014, 3712, 4, 2), (210, 9278, 6464, 5, 3), (640, 4000, 4096, 6, 2),
           (257, 8338, 11264, 7, 3), (127, 16500, 64, 8, 1), (640, 8200, 448, 9, 1), (395, 10424, 256, 4, 1), (276, 15640, 1152, 4, 1),
           (439, 15744, 512, 5, 1), (213, 22912, 1536, 5, 1), (216, 12496, 5120, 3, 1), (467, 3512, 8192, 3, 2),
@@ -21,7 +21,9 @@ SHAPES = [(17, 72, 64, 0, 1), (33, 72, 2048, 0, 4), (17, 16500, 64, 1, 1), (64, 
 
 
 def test_the_shapes_take_their_tiles():
-    assert [(r["tile"], r["splitk"], r["ahead"]) for r in routes([s[:3] for s in SHAPES])] == [(*s[3:], 0) for s in SHAPES]
+    for gated in (0, 1):
+        got = [(r["tile"], r["splitk"], r["ahead"]) for r in routes([(*s[:3], gated, 0) for s in SHAPES])]
+        assert got == [(-2 if gated and s[0] <= 32 else s[3], s[4], 0) for s in SHAPES]
 
 
 @pytest.mark.parametrize("M,rows,K,tile,parts", SHAPES)
