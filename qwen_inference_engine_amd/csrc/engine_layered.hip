@@ -1829,7 +1829,7 @@ static int enq_delta_gates(qie_batch* b, int r, int T) {
 // three launches, and all rows' columns twice.  us with the convolutions before, pieces | walk: 16 heads of 128, 20 rows 31 | 16, 300 rows 143 | 73,
 // 4 entries of 465 316 | 132, 11 of 900 1,430 | 621, one of 2,500 453 | 420, 4,000 668 | 655, 6,000 848 | 989; 16 heads of 64, 4 of 465 123 | 98, one of
 // 500 108 | 94, 700 113 | 124, 900 119 | 154, 2,500 178 | 397.
-// Beside an attention and a feed-forward (`beside`) a row takes up to twice that, but pieces slow the others down: a chain of long entries is the
+// Beside an attention and a feed-forward (`beside`) a row takes up to 0.37, but pieces slow the others down: a chain of long entries is the
 // better one for longer, and a whole step of Nukizen is at most 3 % from the better form.  us a step, pieces | walk: 2k, 300 rows 700 | 628, 900 rows 1,055
 // | 964, 4 of 465 1,555 | 1,415, 11 of 900 6,900 | 5,970, one of 2,500 2,087 | 2,135, 4,000 3,120 | 2,910, 8,000 5,475 | 5,375, of 2,500 and 11 rows
 // 2,200 | 2,230; 1k, 300 rows 468 | 428, 900 570 | 604, 3 of 1,200 1,138 | 1,160, 6 of 900 1,550 | 1,460.
