@@ -347,10 +347,10 @@ constexpr std::size_t lds(const Form& f) {   // the rings; behind the loop the w
     return ring > sums ? ring : sums;
 }
 
-// A tile's rows as a buffer that begins at element k of the first of them: its bytes, and where row r begins.  A load past its end gives zeros and reads
-// nothing.  That check is documented for a lane's offset (the scalar offset beside it, says the compiler's manual, is left out; gfx950 was seen to
-// count it), so the lane's offset holds rows that do not exist away, and k lies in the buffer's base.
-QIE_PLAN_HD inline uint32_t bytes_from(int rows, int64_t ld, int64_t K, int64_t k) { return (uint32_t)(((int64_t)(rows - 1) * ld + K - k) * 2); }
+// A tile's rows as a buffer: its bytes, and where row r begins.  A load past its end gives zeros and reads nothing.  That check is documented for a
+// lane's offset (the scalar offset beside it, says the compiler's manual, is left out; gfx950 was seen to count it), so the lane's offset alone has to
+// hold rows that do not exist away: it has a row and a piece of 16 bytes, the scalar offset the k of a chunk, which lies in every row.
+QIE_PLAN_HD inline uint32_t bytes_of(int rows, int64_t ld, int64_t K) { return (uint32_t)(((int64_t)(rows - 1) * ld + K) * 2); }
 QIE_PLAN_HD inline uint32_t row_at(int r, int64_t ld) { return (uint32_t)r * (uint32_t)ld * 2; }
 
 inline float us_of(const Time& t, int64_t workgroups, int per_cu, int64_t nk, bool one_row_tile, int64_t cols, int64_t K, int64_t cus) {

@@ -41,7 +41,7 @@ __global__ __launch_bounds__(64 * few::WAVES) void gemm_few_kernel(GemmParams p,
     const int chunks = (int)(p.K >> 6), kb = quotient(part * chunks, parts), n = quotient((part + 1) * chunks, parts) - kb;
     const int mine = n > wave ? (n - wave + NW - 1) / NW : 0;   // chunks kb + wave + NW i of this wave
 
-    // A's and the weights' rows of the tile as buffers (few::bytes_from).  A tile lies in one weight segment (few::choose).
+    // A's and the weights' rows of the tile as buffers (few::bytes_of).  A tile lies in one weight segment (few::choose).
     const int rows = (int)(p.M - m0 < BM ? p.M - m0 : BM);
     const uint16_t* a0 = p.A + m0 * p.lda;
     const int64_t seg = GATED || c0 < p.n0 ? 0 : c0 < p.n01 ? p.n0 : p.n01, end = GATED ? p.N : c0 < p.n0 ? p.n0 : c0 < p.n01 ? p.n01 : p.N;
@@ -66,18 +66,21 @@ __global__ __launch_bounds__(64 * few::WAVES) void gemm_few_kernel(GemmParams p,
     // (lane & 7) ^ swz(row); the swizzle of rows 8 on differs in one bit
     unsigned char* ring = smem + wave * (SLOTS * SLOT);
     const int dr = lane >> 3, piece[2] = {((lane & 7) ^ g8_swz(dr)) * 16, ((lane & 7) ^ g8_swz(dr + 8)) * 16};
+    const uint32_t a_bytes = few::bytes_of(rows, p.lda, p.K), w_bytes = few::bytes_of(left, p.K, p.K);
+    uint32_t a_at[BM / 8], w_at[BN / 8];
+#pragma unroll
+    for (int b = 0; b < BM / 8; b++) a_at[b] = few::row_at(8 * b + dr, p.lda) + piece[b & 1];
+#pragma unroll
+    for (int b = 0; b < BN / 8; b++) w_at[b] = few::row_at(8 * (GATED ? b / 4 * 2 + (b & 1) : b) + dr, p.K) + piece[b & 1];
     auto load = [&](int slot, int i) {
         const bool on = i < mine;   // uniform; off: buffers of no bytes, so that every wait is a counted one
-        const int64_t k = (int64_t)(kb + wave + NW * i) * 64;
-        const auto ra = rsrc(a0 + k, on ? few::bytes_from(rows, p.lda, p.K, k) : 0u);
-        const uint32_t w_bytes = on ? few::bytes_from(left, p.K, p.K, k) : 0u;
-        const auto r0 = rsrc(w0 + k, w_bytes), r1 = GATED ? rsrc(w1 + k, w_bytes) : r0;
+        const int k = (kb + wave + NW * i) * 128;
+        const auto ra = rsrc(a0, on ? a_bytes : 0u), r0 = rsrc(w0, on ? w_bytes : 0u), r1 = GATED ? rsrc(w1, on ? w_bytes : 0u) : r0;
         unsigned char* dst = ring + slot * SLOT;
 #pragma unroll
-        for (int b = 0; b < BN / 8; b++)
-            buffer_lds16<NT>(GATED && (b & 2) ? r1 : r0, dst + b * 1024, few::row_at(8 * (GATED ? b / 4 * 2 + (b & 1) : b) + dr, p.K) + piece[b & 1], 0);
+        for (int b = 0; b < BN / 8; b++) buffer_lds16<NT>(GATED && (b & 2) ? r1 : r0, dst + b * 1024, w_at[b], k);
 #pragma unroll
-        for (int b = 0; b < BM / 8; b++) buffer_lds16<false>(ra, dst + BN * 128 + b * 1024, few::row_at(8 * b + dr, p.lda) + piece[b & 1], 0);
+        for (int b = 0; b < BM / 8; b++) buffer_lds16<false>(ra, dst + BN * 128 + b * 1024, a_at[b], k);
     };
     f32x4 acc[FI][FJ];
 #pragma unroll

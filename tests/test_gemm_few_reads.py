@@ -1,5 +1,5 @@
-"""CPU: which bytes of x and of the weights k_gemm_few.hip's loads may touch.  The hardware's range check is documented for a lane's offset alone, so a load
-has no scalar offset, and by few::bytes_from and few::row_at (csrc/gemm_plan.hpp) a lane's offset lies in the rows that exist or behind the buffer's end."""
+"""CPU: which bytes of x and of the weights k_gemm_few.hip's loads may touch.  The hardware's range check is documented for a lane's offset alone, so by
+few::bytes_of and few::row_at (csrc/gemm_plan.hpp) that offset lies in the rows that exist or behind the buffer's end; the scalar offset is a chunk's k."""
 import os
 import re
 import subprocess
@@ -13,12 +13,12 @@ DRIVER = r"""
 int main() {
     long rows, tile, ld, K, k;
     while (std::scanf("%ld %ld %ld %ld %ld", &rows, &tile, &ld, &K, &k) == 5) {
-        const long bytes = qie::few::bytes_from((int)rows, ld, K, k), tensor = ((rows - 1) * ld + K) * 2;
+        const long bytes = qie::few::bytes_of((int)rows, ld, K), tensor = ((rows - 1) * ld + K) * 2;
         long wrong = 0, read = 0;
         for (int r = 0; r < tile; r++)
             for (int piece = 0; piece < 8; piece++) {
                 const long at = (long)qie::few::row_at(r, ld) + 16 * piece, from = 2 * k + at;
-                const bool in = at + 16 <= bytes;
+                const bool in = at + 16 <= bytes;   // without k: what the check is documented to see
                 read += in;
                 wrong += in != (r < rows) || (in && (from != 2 * (r * ld + k) + 16 * piece || from + 16 > tensor)) || (!in && at < bytes);
             }
@@ -39,7 +39,7 @@ def test_rows_that_do_not_exist_are_not_read(tmp_path):
         assert [int(v) for v in line.split()] == [0, 8 * c[0]], c
 
 
-def test_loads_have_no_scalar_offset():
+def test_scalar_offsets_are_chunks():
     text = open(os.path.join(CSRC, "k_gemm_few.hip")).read()
     calls = re.findall(r"buffer_lds16<.*;", text)
-    assert len(calls) == 2 and all(c.endswith(", 0);") for c in calls) and "raw_ptr_buffer_load_lds" not in text, calls
+    assert len(calls) == 2 and all(re.search(r", [aw]_at\[b\], k\);$", c) for c in calls) and "raw_ptr_buffer_load_lds" not in text, calls
